@@ -4,13 +4,17 @@
 ``tinytorch::function::sdpAttention`` (reference src/Function/FuncNNLayer.h:298-302) and of
 ``FuncSDPAttention::forward`` (:231-266); the work itself is one call through the C ABI of include/ttsdpa.h.
 torch is only the owner of device memory and of the current stream here.
+
+Each entry point first hands its arguments to its native counterpart (csrc/torch_binding.cpp), which takes every call
+that is in order and returns None, with nothing enqueued, for the others: what follows here then makes the copies such a
+call needs or names what is wrong with it.
 """
 import ctypes
 import math
 
 import torch
 
-from . import _capi
+from . import _capi, _native
 
 _DTYPES = {torch.float32: _capi.F32, torch.float16: _capi.F16, torch.bfloat16: _capi.BF16}
 
@@ -113,6 +117,9 @@ def sdpAttention(query, key, value, isCausal=False, attnMask=None, dropoutP=0.0,
     blockTable (likewise not in the reference): int32 [B, n] on the device makes key/value page pools
     [pages,Hkv,pageSize,D]; key j of batch b is row j % pageSize of page blockTable[b, j // pageSize].
     """
+    out = _native.sdp_attention(query, key, value, isCausal, attnMask, dropoutP, scale, kvLens, causalAlign, blockTable)
+    if out is not None:
+        return out
     if dropoutP != 0.0:
         raise NotImplementedError("sdpAttention: dropoutP must be 0 on this path")
     if query.dim() != 4 or key.dim() != 4 or value.dim() != 4:
@@ -159,6 +166,9 @@ def sdpAttentionBackward(gradOut, query, key, value, out, isCausal=False, attnMa
     the shape of key / value: with grouped heads they sum over the query heads of a KV head; rows at or beyond
     kvLens[b] are zero.
     """
+    grads = _native.sdp_attention_backward(gradOut, query, key, value, out, isCausal, attnMask, scale, kvLens, causalAlign)
+    if grads is not None:
+        return grads
     if any(t.dim() != 4 for t in (gradOut, query, key, value, out)):
         raise ValueError("sdpAttentionBackward: expected 4-D tensors [B, H, N, D]")
     if not query.is_cuda:
@@ -196,6 +206,8 @@ def kvCacheAppend(kCache, vCache, kNew, vNew, positions, blockTable=None):
     blockTable: int32 [B, n] makes the caches page pools [pages,Hkv,pageSize,D]; row pos of batch b lands in row
     pos % pageSize of page blockTable[b, pos // pageSize], and the capacity per batch entry is n * pageSize.
     """
+    if _native.kv_cache_append(kCache, vCache, kNew, vNew, positions, blockTable):
+        return
     if kCache.dim() != 4 or kNew.dim() != 4 or vCache.shape != kCache.shape or vNew.shape != kNew.shape:
         raise ValueError("kvCacheAppend: expected caches [B,Hkv,Smax,D] and new rows [B,Hkv,Lnew,D]")
     B, Hkv, Smax, D = kCache.shape
@@ -262,6 +274,9 @@ def _launch(name, fn, device, *args):
 def rmsNorm(input, normalizedShape, weight=None, eps=1e-8):
     """input / sqrt(mean(input^2) + eps) * weight over the last axis (reference src/Function/FuncNNLayer.h:294-296;
     normalizedShape must be [input.shape[-1]] as in src/Operation/OpNNLayerCpu.h:183-184)."""
+    out = _native.rms_norm(input, normalizedShape, weight, eps)
+    if out is not None:
+        return out
     _check_rowwise("rmsNorm", input, weight)
     dim = input.shape[-1]
     if list(normalizedShape) != [dim]:
@@ -279,6 +294,8 @@ def rmsNorm(input, normalizedShape, weight=None, eps=1e-8):
 
 def fusedAddRmsNorm(input, residual, weight, eps):
     """In place: residual += input; input = rmsNorm(residual) * weight (reference src/Function/FuncFused.h:32-34)."""
+    if _native.fused_add_rms_norm(input, residual, weight, eps):
+        return
     _check_rowwise("fusedAddRmsNorm", input, residual, weight)
     if input.shape != residual.shape or not input.is_contiguous() or not residual.is_contiguous():
         raise ValueError("fusedAddRmsNorm: input and residual must be contiguous tensors of one shape")
@@ -293,6 +310,9 @@ def fusedAddRmsNorm(input, residual, weight, eps):
 
 def siluMul(x):
     """silu(x[..., :d]) * x[..., d:] with d = x.shape[-1] / 2 (reference src/Function/FuncFused.h:30)."""
+    out = _native.silu_mul(x)
+    if out is not None:
+        return out
     _check_rowwise("siluMul", x)
     if x.shape[-1] % 2 != 0:
         raise ValueError("siluMul: the last axis must be even")  # reference ASSERT, src/Operation/OpFusedCpu.h:17
@@ -306,6 +326,9 @@ def siluMul(x):
 
 
 def _softmax(name, x, dim, log):
+    out = _native.softmax(x, dim, log)
+    if out is not None:
+        return out
     _check_rowwise(name, x)
     if x.dim() == 0:
         raise ValueError("%s: expected at least one axis" % name)
@@ -334,6 +357,9 @@ def logSoftmax(x, dim=-1):
 
 
 def _softmax_backward(name, grad, output, dim, log):
+    out = _native.softmax_backward(grad, output, dim, log)
+    if out is not None:
+        return out
     _check_rowwise(name, grad, output)
     if grad.shape != output.shape or grad.dim() == 0:
         raise ValueError("%s: grad %s and output %s must have the same shape" % (name, tuple(grad.shape), tuple(output.shape)))
@@ -366,6 +392,9 @@ def logSoftmaxBackward(grad, output, dim=-1):
 def linear(input, weight, bias=None):
     """input [..., K] . weight [N, K]^T + bias [N] (reference src/Function/FuncNNLayer.h:270-272): fp32 accumulation
     starting from the bias, one rounding to the dtype of input."""
+    out = _native.linear(input, weight, bias)
+    if out is not None:
+        return out
     _check_rowwise("linear", input, weight, bias)
     if weight.dim() != 2 or input.dim() < 1 or input.shape[-1] != weight.shape[1]:
         raise ValueError("linear: input [..., K] and weight [N, K] do not match: %s, %s"
@@ -395,6 +424,9 @@ def matmul(a, b, transA=False, transB=False, bias=None):
     a column vector (their transpose flags are ignored, :63-72), and the added dimension is dropped from the result.
     For 2-D operands (False, True) is the linear layer; (False, False) and (True, False) are what
     FuncLinear::backward calls for the input and the weight gradient (reference src/Function/FuncNNLayer.h:20-33)."""
+    out = _native.matmul(a, b, transA, transB, bias)
+    if out is not None:
+        return out
     _check_rowwise("matmul", a, b, bias)
     if a.dim() == 0 or b.dim() == 0:
         raise ValueError("matmul: invalid shape")  # reference :54-57
