@@ -81,7 +81,7 @@ __device__ __forceinline__ void load_half_row(const float* row, int lh, float (&
 }
 
 // ---- kernel 1: dq, lse, delta -------------------------------------------------------------------------------------
-// MASKED: an attnMask (exclusive with CAUSAL) whose keys can be read four at a time, as in the forward kernel.
+// MASKED: an attnMask (exclusive with CAUSAL), as in the forward kernel.
 // PAD (both kernels): the tensors' head_dim f.D is a multiple of 4 below D.  The 16-byte chunks of a row beyond it are
 // taken as zeros (q, k: nothing added to a score; dout, v: nothing added to dP or delta; gradient columns beyond f.D are
 // not stored); everything else is the kernel for head_dim D.  No splits (their records are laid out for D).
@@ -218,6 +218,12 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dq_f32_kernel(
       const float* Vs = Ks + Lds::TILE;
 
       f32x16 s = score_product<D>(Ks + s_lane, qreg);  // S^T = K . Q^T
+      if (MASKED) {
+        int qi = qw0 + lq;
+        qi = qi < f.L ? qi : f.L - 1;
+        const long long mrow = b * f.ms[0] + h * f.ms[1] + qi * f.ms[2];
+        apply_attn_mask<float>(f, s, load_attn_mask<float>(f, mrow, kv0, lh, S), 1.f / f.scale);
+      }
       if ((CAUSAL && kv0 + BT - 1 > qw0 + coff) || kv0 + BT > S) {
         const int qi = qw0 + lq + coff;
 #pragma unroll
@@ -225,11 +231,6 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dq_f32_kernel(
           const int key = kv0 + 8 * (r >> 2) + 4 * lh + (r & 3);
           if (key >= S || (CAUSAL && key > qi)) s[r] = -INFINITY;
         }
-      }
-      if (MASKED) {
-        int qi = qw0 + lq;
-        qi = qi < f.L ? qi : f.L - 1;
-        apply_attn_mask<float, true>(f, s, b * f.ms[0] + h * f.ms[1] + qi * f.ms[2], kv0, lh, S, 1.f / f.scale);
       }
       float mloc = s[0];
 #pragma unroll

@@ -128,7 +128,7 @@ __device__ __forceinline__ vec8 regs_to_operand(const f32x16& acc, int t) {
 // ---- kernel 1: dq, lse, delta ----------------------------------------------------------------------------------------
 // BN: keys per streamed tile.  64 for head_dim 64; 32 for head_dim 128, which keeps a wavefront under 256 registers:
 // two wavefronts per SIMD (one's vector work overlaps the other's matrix work), accumulators in ordinary registers.
-// MASKED: an attnMask (exclusive with CAUSAL) whose keys can be read four at a time, as in the forward kernels.
+// MASKED: an attnMask (exclusive with CAUSAL), as in the forward kernels.
 // PAD (both register-staged kernels): the tensors' head_dim f.D is a multiple of 8 below D.  The 16-byte chunks of a row
 // beyond it are taken as zeros (q, k: nothing added to a score; dout, v: nothing added to dP or delta; the gradients'
 // columns beyond f.D are not stored); everything else is the kernel for head_dim D.  No splits (their records are laid
@@ -292,6 +292,14 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ks++) sacc[blk] = TR::mfma32(*(const vec8*)(krow + 16 * ks), qreg[ks], sacc[blk]);
       }
+      if (MASKED) {
+        int qi = qw0 + lq;
+        qi = qi < f.L ? qi : f.L - 1;
+        const long long mrow = b * f.ms[0] + h * f.ms[1] + qi * f.ms[2];
+#pragma unroll
+        for (int blk = 0; blk < NBLK; blk++)
+          apply_attn_mask<T>(f, sacc[blk], load_attn_mask<T>(f, mrow, kv0 + 32 * blk, lh, S), 1.f / f.scale);
+      }
       if ((CAUSAL && kv0 + BN - 1 > qw0 + coff) || kv0 + BN > S) {
         const int qi = qw0 + lq + coff;
 #pragma unroll
@@ -301,13 +309,6 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
             const int key = kv0 + 32 * blk + 8 * (r >> 2) + 4 * lh + (r & 3);
             if (key >= S || (CAUSAL && key > qi)) sacc[blk][r] = -INFINITY;
           }
-      }
-      if (MASKED) {
-        int qi = qw0 + lq;
-        qi = qi < f.L ? qi : f.L - 1;
-        const long long mrow = b * f.ms[0] + h * f.ms[1] + qi * f.ms[2];
-#pragma unroll
-        for (int blk = 0; blk < NBLK; blk++) apply_attn_mask<T, true>(f, sacc[blk], mrow, kv0 + 32 * blk, lh, S, 1.f / f.scale);
       }
       float mloc = sacc[0][0];
 #pragma unroll

@@ -129,16 +129,15 @@ __device__ __forceinline__ void store_from_float(_Float16* p, float x) { *p = (_
 // a lane holds one query row (mask row offset `mrow`, in elements) and, in register group rg, the four consecutive
 // keys kv0 + 8*rg + 4*lh .. +3.  Bool: hidden keys get -inf; additive: the bias joins the scaled score, i.e.
 // bias * inv_scale the raw score held here.  Element strides of 0 broadcast an axis.  Keys at or beyond S are left
-// alone (masked by the caller).  With a.mask_vec4 a group of four keys is one load.  VEC_ONLY: the caller guarantees
-// a.mask_vec4 and S % 4 == 0, and the element-wise path (and its registers) is left out.
-template <typename T, bool VEC_ONLY>
+// alone (masked by the caller).  With a.mask_vec4 a group of four keys is one load.  For the pipelined kernels' general
+// steps, which have few registers to spare.
+template <typename T>
 __device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, long long mrow, int kv0, int lh, int S,
                                                 float inv_scale) {
 #pragma unroll
   for (int rg = 0; rg < 4; rg++) {
     const int key0 = kv0 + 8 * rg + 4 * lh;
-    if (VEC_ONLY && key0 >= S) continue;
-    if (VEC_ONLY || (a.mask_vec4 && key0 + 3 < S)) {
+    if (a.mask_vec4 && key0 + 3 < S) {
       const long long at = mrow + key0;
       if (a.mask_kind == 1) {
         const uint32_t w = *(const uint32_t*)((const uint8_t*)a.mask + at);
@@ -165,6 +164,87 @@ __device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, long 
         }
       }
     }
+  }
+}
+
+// The same in two halves, so that a kernel can request a tile's mask ahead of the scores.  What is loaded: additive, the
+// block's 16 values; Bool, four bytes in each of the first four words.  With contiguous keys a group of four is one load
+// at whatever byte its row begins (rows of an odd length; global loads take any alignment), and the loads of a block
+// are in flight together; a group that runs past the last key is read from key S - 4 on and shifted.  Other masks are read
+// key by key.  S >= 1; values of keys at or beyond S are arbitrary: the caller hides those keys after the mask is applied.
+template <typename T>
+using MaskBlock = uint32_t __attribute__((ext_vector_type(4 * sizeof(T))));
+
+template <typename T>
+__device__ __forceinline__ MaskBlock<T> load_attn_mask(const KArgs& a, long long mrow, int kv0, int lh, int S) {
+  constexpr int WPG = sizeof(T);  // words per group of four keys, additive
+  typedef uint32_t loose32 __attribute__((aligned(1)));
+  typedef uint32_t looseg __attribute__((ext_vector_type(WPG), aligned(sizeof(T))));
+  MaskBlock<T> m = {};
+  if (a.ms[3] == 1 && kv0 + 32 <= S) {
+    const long long at = mrow + kv0 + 4 * lh;
+    if (a.mask_kind == 1) {
+      const uint8_t* p = (const uint8_t*)a.mask + at;
+#pragma unroll
+      for (int rg = 0; rg < 4; rg++) m[rg] = *(const loose32*)(p + 8 * rg);
+    } else {
+      const T* p = (const T*)a.mask + at;
+#pragma unroll
+      for (int rg = 0; rg < 4; rg++) {
+        const looseg w = *(const looseg*)(p + 8 * rg);
+#pragma unroll
+        for (int i = 0; i < WPG; i++) m[WPG * rg + i] = w[i];
+      }
+    }
+  } else if (a.ms[3] == 1 && S >= 4) {
+#pragma unroll
+    for (int rg = 0; rg < 4; rg++) {
+      const int key0 = kv0 + 8 * rg + 4 * lh;
+      const int past = key0 > S - 4 ? key0 - (S - 4) : 0;
+      if (a.mask_kind == 1) {
+        m[rg] = *(const loose32*)((const uint8_t*)a.mask + mrow + (key0 - past)) >> (8 * (past & 3));
+      } else {
+        looseg w = *(const looseg*)((const T*)a.mask + mrow + (key0 - past));
+        if constexpr (WPG == 2) {
+          if (past & 2) w = looseg{w[1], 0};
+          if (past & 1) w = looseg{(w[0] >> 16) | (w[1] << 16), w[1] >> 16};
+        } else {
+          if (past & 2) w = looseg{w[2], w[3], 0, 0};
+          if (past & 1) w = looseg{w[1], w[2], w[3], 0};
+        }
+#pragma unroll
+        for (int i = 0; i < WPG; i++) m[WPG * rg + i] = w[i];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int key = kv0 + 8 * (r >> 2) + 4 * lh + (r & 3);
+      const long long at = mrow + (key < S ? key : S - 1) * a.ms[3];
+      if (a.mask_kind == 1)
+        m[r >> 2] |= (uint32_t)((const uint8_t*)a.mask)[at] << (8 * (r & 3));
+      else if (WPG == 4)
+        m[r] = ((const uint32_t*)a.mask)[at];
+      else
+        m[r >> 1] |= (uint32_t)((const uint16_t*)a.mask)[at] << (16 * (r & 1));
+    }
+  }
+  return m;
+}
+
+// Bool: hidden keys get -inf; additive: the bias joins the scaled score.
+template <typename T>
+__device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, MaskBlock<T> m, float inv_scale) {
+  constexpr int WPG = sizeof(T);
+  if (a.mask_kind == 1) {
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+      if (((m[r >> 2] >> (8 * (r & 3))) & 0xffu) == 0) s[r] = -INFINITY;
+  } else {
+    typedef T vec16t __attribute__((ext_vector_type(16)));
+    const vec16t b = __builtin_bit_cast(vec16t, m);
+#pragma unroll
+    for (int r = 0; r < 16; r++) s[r] += (float)b[r] * inv_scale;
   }
 }
 

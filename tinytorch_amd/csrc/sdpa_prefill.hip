@@ -229,6 +229,22 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   const int k_lane = lq * K_PITCH + 8 * lh;                                              // elements
   const int v_lane = (4 * lh + ((lane & 15) >> 2)) * V_PITCH + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);  // elements
 
+  // the mask of a tile is requested while the tile before it is in its softmax and P.V (registers allow up to head_dim 96)
+  constexpr bool MASK_AHEAD = MASKED && D <= 96;
+  MaskBlock<T> mask[2];
+  long long mrow = 0;
+  float inv_scale = 0.f;
+  if (MASKED) {
+    const int qi = qw0 + lq;
+    mrow = b * a.ms[0] + h * a.ms[1] + (qi < a.L ? qi : a.L - 1) * a.ms[2];
+    inv_scale = 1.f / a.scale;
+  }
+  auto load_mask = [&](int kv0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int blk = 0; blk < 2; blk++) mask[blk] = load_attn_mask<T>(a, mrow, kv0 + 32 * blk, lh, S);
+  };
+  if (MASK_AHEAD && jt0 < jt1) load_mask(jt0 * BN);
+
   if (jt0 < jt1) {
     load_tile(jt0 * BN);
     store_tile(0);
@@ -262,6 +278,13 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
         }
       }
 
+      if (MASKED) {
+        if (!MASK_AHEAD) load_mask(kv0);
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) apply_attn_mask<T>(a, sacc[blk], mask[blk], inv_scale);
+        if (MASK_AHEAD && jt + 1 < jt1) load_mask(kv0 + BN);
+      }
+
       // ---- mask the diagonal / ragged tile -----------------------------------------------------------------------
       const bool need_mask = (CAUSAL && kv0 + BN - 1 > pos_lo + coff) || (kv0 + BN > S);
       if (need_mask) {
@@ -275,14 +298,6 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
             if (hidden) sacc[blk][r] = -INFINITY;
           }
       }
-      if (MASKED) {
-        int qi = qw0 + lq;
-        qi = qi < a.L ? qi : a.L - 1;
-        const long long mrow = b * a.ms[0] + h * a.ms[1] + qi * a.ms[2];
-#pragma unroll
-        for (int blk = 0; blk < 2; blk++) apply_attn_mask<T, true>(a, sacc[blk], mrow, kv0 + 32 * blk, lh, S, 1.f / a.scale);
-      }
-
       // ---- online softmax with a lazily raised maximum ---------------------------------------------------------------
       float psum = 0.f;
       f32x16 pr[2];

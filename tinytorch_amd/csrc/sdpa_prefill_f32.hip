@@ -183,6 +183,14 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
   const int k_lane = lq * K_PITCH + lh * (D / 2);  // floats
   const int v_lane = 4 * lh * V_PITCH + lq;        // floats; + (8*(t/4) + t%4) * V_PITCH + 32*db
 
+  long long mrow = 0;
+  float inv_scale = 0.f;
+  if (MASKED) {
+    const int qi = qw0 + lq;
+    mrow = b * a.ms[0] + h * a.ms[1] + (qi < a.L ? qi : a.L - 1) * a.ms[2];
+    inv_scale = 1.f / a.scale;
+  }
+
   if (jt0 < jt1) {
     load_tile(jt0 * BN);
     store_tile(0);
@@ -202,6 +210,9 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
       const float* Ks = smem + cur * Lds::STAGE;
       const float* Vs = Ks + BN * K_PITCH;
 
+      MaskBlock<float> mask = {};  // requested here, used behind the score products
+      if (MASKED) mask = load_attn_mask<float>(a, mrow, kv0, lh, S);
+
       // ---- S^T = K . Q^T, two accumulators over alternate k-steps ----------------------------------------------------
       f32x16 s0, s1;
 #pragma unroll
@@ -216,6 +227,8 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; r++) s[r] = s0[r] + s1[r];
 
+      if (MASKED) apply_attn_mask<float>(a, s, mask, inv_scale);
+
       // ---- mask the diagonal / ragged tile -----------------------------------------------------------------------------
       if ((CAUSAL && kv0 + BN - 1 > pos_lo + coff) || (kv0 + BN > S)) {
         const int qi = (a.pack_L ? (qw0 + lq) % a.pack_L : qw0 + lq) + coff;
@@ -225,11 +238,6 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
           bool hidden = key >= S || (CAUSAL && key > qi);
           if (hidden) s[r] = -INFINITY;
         }
-      }
-      if (MASKED) {
-        int qi = qw0 + lq;
-        qi = qi < a.L ? qi : a.L - 1;
-        apply_attn_mask<float, true>(a, s, b * a.ms[0] + h * a.ms[1] + qi * a.ms[2], kv0, lh, S, 1.f / a.scale);
       }
 
       // ---- online softmax with a lazily raised maximum -----------------------------------------------------------------

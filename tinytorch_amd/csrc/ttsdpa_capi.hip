@@ -103,14 +103,17 @@ bool fast_layout_ok(const ttsdpa_params* p, bool masks_ok = false, bool pages_ok
   return ptr_aligned(p->q, 16) && ptr_aligned(p->k, 16) && ptr_aligned(p->v, 16) && ptr_aligned(p->out, 16);
 }
 
-// The 4-wavefront and fp32 kernels read an attnMask four keys at a time: aligned groups, whole groups only.
-bool simple_mask_ok(const ttsdpa_params* p) {
-  return p->mask_kind == TTSDPA_MASK_NONE || (mask_vec4_ok(p) && p->S % 4 == 0 && !p->kv_len);
+// What the MFMA routes take: attnMasks readable four keys at a time (aligned groups, whole groups only).  The kernels
+// themselves apply any attnMask: any_mask = true in the tests below admits the others, which the general route hands
+// to them (a general-route call of 16 x 12 heads x 197 rows, head_dim 64, fp16, with a key-padding mask: 124 us on the
+// vector ALUs, 16 us there).
+bool simple_mask_ok(const ttsdpa_params* p, bool any_mask = false) {
+  return any_mask || p->mask_kind == TTSDPA_MASK_NONE || (mask_vec4_ok(p) && p->S % 4 == 0 && !p->kv_len);
 }
 
 // fp32 tensors the fp32 MFMA kernel can read and write with 16-byte accesses.
-bool f32_prefill_ok(const ttsdpa_params* p) {
-  if (p->dtype != TTSDPA_F32 || (p->block_table && p->page_size < kPrefillMinPage) || !simple_mask_ok(p)) return false;
+bool f32_prefill_ok(const ttsdpa_params* p, bool any_mask = false) {
+  if (p->dtype != TTSDPA_F32 || (p->block_table && p->page_size < kPrefillMinPage) || !simple_mask_ok(p, any_mask)) return false;
   if (p->D < 4 || p->D > 128 || p->D % 4 != 0) return false;  // 64 and 128; other multiples of 4 on the next one up with zero columns
   if (!(p->scale > 0.f) || !isfinite(p->scale) || p->S < 1 || p->L < 1) return false;
   if (!dense_last_ok(p->q_stride, 4) || !dense_last_ok(p->k_stride, 4) || !dense_last_ok(p->v_stride, 4) ||
@@ -221,8 +224,8 @@ SplitPlan plan_pipelined_splits(const ttsdpa_params* p) {
   return s;
 }
 
-bool prefill_ok(const ttsdpa_params* p) {
-  if (f32_prefill_ok(p)) return true;
+bool prefill_ok(const ttsdpa_params* p, bool any_mask = false) {
+  if (f32_prefill_ok(p, any_mask)) return true;
   // the pipelined head_dim-128 kernel takes any attnMask; the 4-wavefront kernel those it can read four keys at a time
   // head sizes between the 4-wavefront kernel's (32, 64, 96, 128, 192, 256) run on the next one up with zero columns
   const bool mfma_head_dim = p->D >= 8 && p->D <= 256 && p->D % 8 == 0;
@@ -230,7 +233,7 @@ bool prefill_ok(const ttsdpa_params* p) {
   // the 16-bit kernels address the rows of a K / V tile with 32-bit byte offsets (the fp32 kernel returned above does not)
   const bool tile_offsets_ok = p->k_stride[2] < (1 << 24) && p->v_stride[2] < (1 << 24);
   return fast_layout_ok(p, true, true) && mfma_head_dim && p->S >= 1 && p->L >= 1 && tile_offsets_ok &&
-         (pipelined_ok(p) || simple_mask_ok(p));
+         (pipelined_ok(p) || simple_mask_ok(p, any_mask));
 }
 
 bool decode_ok(const ttsdpa_params* p) {
@@ -287,10 +290,10 @@ int validate_backward(const ttsdpa_backward_params* p, BwdArgs* a) {
 
 // The MFMA backward kernels: 16-bit tensors they can read and write with 16-byte / 8-byte accesses, head_dim 64 or
 // 128, attnMasks the forward's 4-wavefront kernel takes (keys readable four at a time, no kv_len beside them).
-bool backward_mfma_ok(const ttsdpa_backward_params* p) {
+bool backward_mfma_ok(const ttsdpa_backward_params* p, bool any_mask = false) {
   const ttsdpa_params* f = &p->fwd;
   // head_dim 64 and 128; other multiples of 8 up to 128 on the register-staged kernels of the next one up (zero columns)
-  if (!fast_layout_ok(f, true) || !simple_mask_ok(f) || f->D < 8 || f->D > 128 || f->D % 8 != 0 || f->L < 1 || f->S < 1) return false;
+  if (!fast_layout_ok(f, true) || !simple_mask_ok(f, any_mask) || f->D < 8 || f->D > 128 || f->D % 8 != 0 || f->L < 1 || f->S < 1) return false;
   if (!dense_last_ok(p->dout_stride, 8) || !dense_last_ok(p->dq_stride, 8) || !dense_last_ok(p->dk_stride, 8) ||
       !dense_last_ok(p->dv_stride, 8))
     return false;
@@ -303,9 +306,9 @@ bool backward_mfma_ok(const ttsdpa_backward_params* p) {
 
 // The fp32 matrix-core backward kernels: fp32 tensors with 16-byte aligned rows, head_dim 64 or 128, attnMasks as for
 // the 16-bit pair.
-bool backward_f32_ok(const ttsdpa_backward_params* p) {
+bool backward_f32_ok(const ttsdpa_backward_params* p, bool any_mask = false) {
   const ttsdpa_params* f = &p->fwd;
-  if (f->dtype != TTSDPA_F32 || f->block_table || !simple_mask_ok(f) || f->D < 4 || f->D > 128 || f->D % 4 != 0) return false;
+  if (f->dtype != TTSDPA_F32 || f->block_table || !simple_mask_ok(f, any_mask) || f->D < 4 || f->D > 128 || f->D % 4 != 0) return false;
   if (!(f->scale > 0.f) || !isfinite(f->scale) || f->L < 1 || f->S < 1) return false;  // the row maximum is taken on unscaled scores
   if (!dense_last_ok(f->q_stride, 4) || !dense_last_ok(f->k_stride, 4) || !dense_last_ok(f->v_stride, 4) ||
       !dense_last_ok(f->o_stride, 4) || !dense_last_ok(p->dout_stride, 4) || !dense_last_ok(p->dq_stride, 4) ||
@@ -321,6 +324,11 @@ int pick_backward_route(const ttsdpa_backward_params* p) {
   return backward_mfma_ok(p) || backward_f32_ok(p) ? TTSDPA_ROUTE_PREFILL : TTSDPA_ROUTE_GENERAL;
 }
 
+// The matrix-core pairs run the call: the MFMA route, and of the general route what only its attnMask keeps off it.
+bool backward_on_mfma(const ttsdpa_backward_params* p) {
+  return pick_backward_route(p) != TTSDPA_ROUTE_NONE && (backward_mfma_ok(p, true) || backward_f32_ok(p, true));
+}
+
 size_t backward_stats_bytes(const ttsdpa_backward_params* p) {
   return (size_t)p->fwd.B * p->fwd.Hq * p->fwd.L * 2 * sizeof(float);
 }
@@ -328,7 +336,7 @@ size_t backward_stats_bytes(const ttsdpa_backward_params* p) {
 // Scratch layout: the statistics, then (matrix-core pairs with a split query stream) the partial dk / dv, 256-byte aligned.
 int dkv_splits_of(const ttsdpa_backward_params* p) {
   const ttsdpa_params* f = &p->fwd;
-  if (pick_backward_route(p) != TTSDPA_ROUTE_PREFILL) return 1;
+  if (!backward_on_mfma(p)) return 1;
   if (f->D != 64 && f->D != 128) return 1;  // the zero-column variants do not split (their records are laid out for 64 / 128)
   const int groups = f->dtype != TTSDPA_F32 && f->D == 128 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
   const int per_cu = f->D == 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
@@ -337,7 +345,7 @@ int dkv_splits_of(const ttsdpa_backward_params* p) {
 // ... then (matrix-core pairs whose dq kernel splits its key ranges) the partial dq records, 256-byte aligned.
 int dq_splits_of(const ttsdpa_backward_params* p) {
   const ttsdpa_params* f = &p->fwd;
-  if (pick_backward_route(p) != TTSDPA_ROUTE_PREFILL) return 1;
+  if (!backward_on_mfma(p)) return 1;
   if (f->D != 64 && f->D != 128) return 1;
   const int slots = f->dtype == TTSDPA_F32 && f->D == 128 ? 256 : 512;
   return backward_dq_splits(f->B, f->Hq, f->L, f->S, effective_causal(f) != TTSDPA_CAUSAL_NONE, slots);
@@ -461,12 +469,12 @@ int ttsdpa_general(const ttsdpa_params* p, void* stream) {
 }
 
 // ttsdpa_prefill with optional scratch: with it, a short-L call may divide its keys among workgroups.
-static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspace_bytes, void* stream) {
+static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspace_bytes, void* stream, bool any_mask = false) {
   KArgs a;
   int rc = validate(p, &a);
   if (rc != TTSDPA_OK) return rc;
   if (p->B == 0 || p->L == 0) return TTSDPA_OK;
-  if (!prefill_ok(p)) return TTSDPA_ERR_UNSUPPORTED;
+  if (!prefill_ok(p, any_mask)) return TTSDPA_ERR_UNSUPPORTED;
   if ((rc = check_grid((long long)a.B * a.Hq * ((a.L + 127) / 128))) != TTSDPA_OK) return rc;
   // head_dim 128 with enough rows to fill 256-row workgroups takes the software-pipelined kernel (its tile loads
   // address 64 rows with 32-bit byte offsets)
@@ -544,8 +552,11 @@ int ttsdpa_forward(const ttsdpa_params* p, void* workspace, size_t workspace_byt
     case TTSDPA_ROUTE_ZERO: return launch_zero(a, p->dtype, (hipStream_t)stream);
     case TTSDPA_ROUTE_DECODE: return ttsdpa_decode(p, workspace, workspace_bytes, stream);
     case TTSDPA_ROUTE_PREFILL: return prefill_impl(p, workspace, workspace_bytes, stream);
-    default: return ttsdpa_general(p, stream);
+    default: break;
   }
+  // the general route: what only its attnMask keeps off the MFMA kernels runs on them, the rest on the vector ALUs
+  if (p->mask_kind != TTSDPA_MASK_NONE && prefill_ok(p, true)) return prefill_impl(p, workspace, workspace_bytes, stream, true);
+  return ttsdpa_general(p, stream);
 }
 
 void ttsdpa_backward_params_init(ttsdpa_backward_params* p, int dtype, int B, int Hq, int Hkv, int L, int S, int D) {
@@ -585,7 +596,7 @@ int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t wor
   a.partial = a.dkv_splits > 1 ? (float*)((char*)workspace + backward_partial_offset(p)) : nullptr;
   a.dq_splits = dq_splits_of(p);
   a.dq_partial = a.dq_splits > 1 ? (float*)((char*)workspace + backward_dq_partial_offset(p)) : nullptr;
-  if (route == TTSDPA_ROUTE_PREFILL) {
+  if (backward_on_mfma(p)) {
     const long long g1 = (long long)a.f.B * a.f.Hq * ((a.f.L + 127) / 128) * a.dq_splits, g2 = (long long)a.f.B * a.f.Hkv * ((a.f.S + 127) / 128);
     if (check_grid(g1) != TTSDPA_OK || check_grid(g2) != TTSDPA_OK) return TTSDPA_ERR_SHAPE;
     if (p->fwd.dtype == TTSDPA_F32) return launch_backward_f32(a, (hipStream_t)stream);
