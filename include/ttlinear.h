@@ -23,7 +23,8 @@ enum ttlinear_route {
   TTLINEAR_ROUTE_NONE = 0,   /* empty output */
   TTLINEAR_ROUTE_MFMA = 1,   /* K a multiple of 64 (fp16/bf16) or 32 (fp32), 16-byte aligned rows, N a multiple of 4:
                                 MFMA kernel, fp32 accumulation (fp32 tensors: full fp32 products) */
-  TTLINEAR_ROUTE_GENERAL = 2 /* everything else (other K, unaligned rows): fp32 arithmetic on the vector ALUs */
+  TTLINEAR_ROUTE_GENERAL = 2 /* everything else (other K, unaligned rows): the streaming MFMA kernel, which takes any alignment; the
+                                vector ALUs only for contraction-major operands of fewer than 16 rows and for empty contractions */
 };
 
 /* out[m, n] = bias[n] + sum_k x[m, k] * w[n, k]   (m < M, n < N, k < K)
@@ -50,7 +51,7 @@ int ttlinear_plan(int dtype, const void* x, const void* w, const void* bias, con
  * row count a multiple of 8): no scratch is used then and workspace may be NULL.
  * workspace: ttlinear_matmul_workspace_bytes() bytes of device scratch, 256-byte aligned — for fp32 the MFMA route first
  * makes dense row-major copies of the operands that are stored contraction-major; with less (or NULL), or for shapes the
- * MFMA kernels do not take, the vector-ALU kernel reads the operands in place.  Same return codes as ttlinear_forward. */
+ * tiled kernels do not take, the general route reads the operands in place.  Same return codes as ttlinear_forward. */
 size_t ttlinear_matmul_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b);
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
                     int trans_a, int trans_b, int64_t lda, int64_t ldb, int64_t ldo, void* workspace,

@@ -15,27 +15,15 @@
 // Workgroups are numbered so that the 32 that run together on one XCD (workgroup i runs on XCD i % 8) form a 4 x 8
 // block of tiles: they share their x and w panels through that XCD's L2.
 //
-// linear_general_kernel: any element type and shape, fp32 arithmetic on the vector ALUs (64 x 64 tiles).
+// linear_general_kernel: any element type and shape, fp32 arithmetic on the vector ALUs (64 x 64 tiles); what neither this
+// file's matrix-core kernels nor the streaming one (linear_stream.hip) take.
 
 #include <type_traits>
 #include "../../include/ttlinear.h"
-#include "sdpa_common.h"
+#include "linear_args.h"
 
 namespace ttsdpa {
 namespace {
-
-struct LinArgs {
-  const void* x;
-  const void* w;
-  const void* bias;
-  void* out;
-  long long M, N, K, ldx, ldw, ldo;
-  // general kernel only: x is stored [K, M] (x(m,k) = x[k*ldx + m]) / w is stored [K, N] (w(n,k) = w[k*ldw + n])
-  int xt = 0, wt = 0;
-  // batch entries of one launch (linear_mfma_kernel: blockIdx.y, linear_general_kernel: blockIdx.z): entry e reads
-  // x + e*bsx, w + e*bsw and writes out + e*bso (elements; 0 = the operand is shared by all entries)
-  long long bsx = 0, bsw = 0, bso = 0;
-};
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
@@ -605,181 +593,6 @@ __global__ __launch_bounds__(256, 1) void linear256_kernel(LinArgs a) {
   }
 }
 
-// ---- few rows of x (a decode step's projections: M = the batch): the weight is read once at HBM speed ------------------
-// With M <= 64 the layer is a stream over w (N*K elements) against 64 rows of x that stay in L2: a workgroup owns 32
-// output columns and all rows of x; its four wavefronts take the 64-element k-blocks in turn (wavefront v: blocks v,
-// v+4, ...) and add their partial sums through LDS at the end.  Every wavefront has a ring of three k-blocks of its own in
-// LDS, filled by direct global->LDS loads (eight lanes fetch the 128 bytes of a row's k-block: whole cache lines) and
-// read back as MFMA operands, 16-byte chunk c of row r at slot c ^ ((r/2) % 8) (conflict-free b128 reads).  No
-// barriers inside the stream: a ring belongs to one wavefront.  out^T[n][m] accumulates with w as the A operand, so a
-// lane ends up with four consecutive n of one row m: 8-byte stores.
-template <int MB, int NB>
-struct Skinny {
-  static constexpr int WT = NB * 32 * 128;             // bytes of a weight tile: NB x 32 rows x 64 k
-  static constexpr int STG = WT + MB * 32 * 128;       // ... plus the x tile
-  static constexpr int NST = 4 * 3 * STG <= 160 * 1024 ? 3 : 2;  // k-blocks of a wavefront in LDS (what fits the CU's 160 KiB)
-  static constexpr int LPB = 4 * NB + 4 * MB;          // load instructions per k-block
-  static constexpr int LDS = 4 * NST * STG;
-  static_assert(LDS >= 3 * MB * NB * 16 * 64 * 4, "the partial sums of three wavefronts reuse the rings");
-};
-
-// MB = 32-row blocks of x: 1 (M <= 32) or 2 (M <= 64).  NB = 32-column blocks of the output a workgroup owns: every x
-// tile a wavefront fetches (from L2) serves NB weight tiles (from memory), so the bytes a CU takes in per weight byte
-// fall from 1 + MB to 1 + MB / NB.  At M = 64 the kernel with NB = 1 is bound by what the L2s deliver (three bytes per
-// weight byte).
-template <typename TR, int MB, int NB>
-__global__ __launch_bounds__(256) void linear_skinny_kernel(LinArgs a) {
-  typedef typename TR::elem T;
-  typedef typename TR::vec8 vec8;
-  typedef Skinny<MB, NB> SK;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lq = lane & 31, lh = lane >> 5;
-  const long long n0 = (long long)blockIdx.x * (32 * NB);
-  char* ring = smem + wave * SK::NST * SK::STG;
-  const unsigned ring_addr = (unsigned)(unsigned long)(lds_void_t*)ring;
-
-  auto dma16 = [&](const char* sbase, unsigned voff, unsigned lds_addr) __attribute__((always_inline)) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
-  };
-  // this lane's part of a load instruction: row 8i + lane/8 of a tile, slot lane%8
-  unsigned woff[NB][4], xoff[MB][4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int row = 8 * i + (lane >> 3);
-    const unsigned chunk = (unsigned)((lane & 7) ^ ((row >> 1) & 7));
-#pragma unroll
-    for (int nb = 0; nb < NB; nb++) {
-      const long long n = n0 + 32 * nb + row;  // columns past the end re-read the last weight row (not stored)
-      woff[nb][i] = (unsigned)(((n < a.N ? n - n0 : a.N - 1 - n0) * a.ldw + 8 * chunk) * 2);
-    }
-#pragma unroll
-    for (int mb = 0; mb < MB; mb++) {
-      const int m = 32 * mb + row;
-      xoff[mb][i] = (unsigned)(((m < a.M ? m : (int)(a.M - 1)) * a.ldx + 8 * chunk) * 2);
-    }
-  }
-  const char* wbase = (const char*)((const T*)a.w + n0 * a.ldw);
-  const char* xbase = (const char*)a.x;
-  auto issue = [&](long long kb, int stage) __attribute__((always_inline)) {
-    const unsigned at = ring_addr + stage * SK::STG;
-    const char* wk = wbase + kb * 128;
-    const char* xk = xbase + kb * 128;
-#pragma unroll
-    for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) dma16(wk, woff[nb][i], at + (32 * nb + 8 * i) * 128);
-#pragma unroll
-    for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) dma16(xk, xoff[mb][i], at + SK::WT + (32 * mb + 8 * i) * 128);
-  };
-  // operand (j): row lq, chunk 4*lh + j
-  unsigned rd[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) rd[j] = (unsigned)(lq * 128 + 16 * ((4 * lh + j) ^ ((lq >> 1) & 7)));
-
-  f32x16 acc[NB][MB];
-#pragma unroll
-  for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-    for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[nb][mb][r] = 0.f;
-  const long long nkb = a.K / 64;
-  const long long nb_ = nkb > wave ? (nkb - wave + 3) / 4 : 0;  // k-blocks of this wavefront: wave, wave + 4, ...
-  constexpr int AHEAD = SK::NST - 1;                             // k-blocks in flight beyond the one in use
-  for (int t = 0; t < AHEAD; t++)
-    if (nb_ > t) issue(wave + 4 * t, t);
-  int cur = 0;
-  for (long long t = 0; t < nb_; t++) {
-    const int nxt = cur == 0 ? SK::NST - 1 : cur - 1;  // (t + AHEAD) % NST
-    if (t + AHEAD < nb_) issue(wave + 4 * (t + AHEAD), nxt);
-    // block t has landed when only the loads of the blocks issued after it are outstanding
-    const long long later = nb_ - 1 - t < AHEAD ? nb_ - 1 - t : AHEAD;
-    if (later == 2) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * SK::LPB) : "memory");
-    } else if (later == 1) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SK::LPB) : "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    const char* wt = ring + cur * SK::STG;
-    const char* xt = wt + SK::WT;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      vec8 xv[MB];
-#pragma unroll
-      for (int mb = 0; mb < MB; mb++) xv[mb] = *(const vec8*)(xt + mb * 32 * 128 + rd[j]);
-#pragma unroll
-      for (int nb = 0; nb < NB; nb++) {
-        const vec8 wv = *(const vec8*)(wt + nb * 32 * 128 + rd[j]);
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++) acc[nb][mb] = TR::mfma32(wv, xv[mb], acc[nb][mb]);
-      }
-    }
-    cur = cur == SK::NST - 1 ? 0 : cur + 1;
-  }
-  __syncthreads();  // every ring is drained: the partial sums of wavefronts 1-3 take their place
-  float* part = (float*)smem;
-  if (wave > 0) {
-#pragma unroll
-    for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-      for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) part[((((wave - 1) * NB + nb) * MB + mb) * 16 + r) * 64 + lane] = acc[nb][mb][r];
-  }
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-    for (int mb = 0; mb < MB; mb++) {
-      const long long m = 32 * mb + lq;
-#pragma unroll
-      for (int rg = 0; rg < 4; rg++) {
-        const long long n = n0 + 32 * nb + 8 * rg + 4 * lh;
-        f32x4 v;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int r = 4 * rg + i;
-          float sum = acc[nb][mb][r];
-#pragma unroll
-          for (int w = 0; w < 3; w++) sum += part[(((w * NB + nb) * MB + mb) * 16 + r) * 64 + lane];
-          if (a.bias && n + i < a.N) sum += load_as_float((const T*)a.bias + n + i);
-          v[i] = sum;
-        }
-        if (m < a.M && n < a.N) {  // N is a multiple of 4 on this route: a group of four is inside or outside
-          *(typename TR::vec4*)((T*)a.out + m * a.ldo + n) = __builtin_convertvector(v, typename TR::vec4);
-        }
-      }
-    }
-}
-
-template <typename TR, int MB, int NB>
-int launch_skinny_mb(const LinArgs& a, hipStream_t stream) {
-  static hipError_t state[kMaxDevices];
-  static bool done[kMaxDevices];
-  constexpr int lds = Skinny<MB, NB>::LDS;
-  const hipError_t granted = grant_dynamic_lds((const void*)linear_skinny_kernel<TR, MB, NB>, lds, state, done);
-  if (granted != hipSuccess) return (int)granted;
-  const long long nwg = (a.N + 32 * NB - 1) / (32 * NB);
-  if (nwg > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
-  hipLaunchKernelGGL((linear_skinny_kernel<TR, MB, NB>), dim3((unsigned)nwg), dim3(256), lds, stream, a);
-  return (int)hipGetLastError();
-}
-
-// Two column blocks per workgroup once they still make a workgroup per CU (N >= 16384).  Weights beyond the last-level
-// cache, bf16, K = 4096: N = 28672 (an MLP's up projection) 3.9 -> 4.4 TB/s at M <= 8, 3.4 -> 4.3 at M = 32, 2.8 -> 3.5 at
-// M = 64; N = 6144 and 4096 (96 and 64 workgroups then) 3.0 -> 2.7 and 2.7 -> 2.4: those keep one block.
-template <typename TR>
-int launch_skinny(const LinArgs& a, hipStream_t stream) {
-  if (a.N >= 16384) return a.M <= 32 ? launch_skinny_mb<TR, 1, 2>(a, stream) : launch_skinny_mb<TR, 2, 2>(a, stream);
-  return a.M <= 32 ? launch_skinny_mb<TR, 1, 1>(a, stream) : launch_skinny_mb<TR, 2, 1>(a, stream);
-}
-
 // Any element type and shape: 64 x 64 output tile per workgroup, 4 x 4 outputs per lane, K in steps of 16 through LDS.
 template <typename T>
 __global__ __launch_bounds__(256) void linear_general_kernel(LinArgs a) {
@@ -984,8 +797,27 @@ int launch_mfma(const LinArgs& a, hipStream_t stream) {
   return big >= 256 ? launch_mfma_tile<TR, 256, 256, 4, 2>(a, stream) : launch_mfma_tile<TR, 128, 128, 4, 2>(a, stream);
 }
 
+// Microseconds of the tiled kernels, from measurements, against the streaming kernel's: a k-step of 128 bytes of a 128 x 128
+// tile takes 0.6 us (fp32 2.2) as long as every CU has one tile at most, and with more in proportion (128 .. 1000 x 4096
+// x 4096: 40 .. 45 us, 2000 rows 74; the 256 x 256 tiles are faster, but no product that fills the chip with them is
+// small enough for the other kernel).  k-major operands: 10 % more.
+double tiled_cost(const LinArgs& a, int dtype, unsigned entries) {
+  const double tiles = (double)((a.M + 127) / 128) * (double)((a.N + 127) / 128) * entries;
+  const double steps = a.K * (dtype == TTSDPA_F32 ? 4 : 2) / 128.0;
+  const double us = 3 + steps * (dtype == TTSDPA_F32 ? 2.2 : 0.6) * (tiles > 256 ? tiles / 256 : 1);
+  return a.xt || a.wt ? us * 1.1 : us;
+}
+
+bool streams(const LinArgs& a, int dtype, unsigned entries = 1) {
+  return stream_takes(a, dtype) && stream_cost(a, dtype, entries) < tiled_cost(a, dtype, entries);
+}
+
+// What the tiled kernels' layout does not allow: the streaming kernel, or where one of its operands is too narrow for that (a
+// k-major operand of fewer than 16 rows, an empty contraction) the vector ALUs.
 template <typename T>
 int launch_general_linear(const LinArgs& a, hipStream_t stream, unsigned entries = 1) {
+  const int dtype = sizeof(T) == 4 ? TTSDPA_F32 : std::is_same<T, _Float16>::value ? TTSDPA_F16 : TTSDPA_BF16;
+  if (stream_takes(a, dtype)) return launch_stream(a, dtype, stream, entries);
   dim3 grid((unsigned)((a.N + 63) / 64), (unsigned)((a.M + 63) / 64), entries);
   hipLaunchKernelGGL((linear_general_kernel<T>), grid, dim3(256), 0, stream, a);
   return (int)hipGetLastError();
@@ -1017,8 +849,7 @@ int ttlinear_forward(int dtype, const void* x, const void* w, const void* bias, 
   LinArgs a{x, w, bias, out, M, N, K, ldx, ldw, ldo};
   hipStream_t s = (hipStream_t)stream;
   if (route == TTLINEAR_ROUTE_MFMA) {
-    // a handful of rows (a decode step): stream the weight once instead of tiling for reuse
-    if (dtype != TTSDPA_F32 && M <= 64 && N >= 64) return dtype == TTSDPA_F16 ? launch_skinny<F16>(a, s) : launch_skinny<BF16>(a, s);
+    if (streams(a, dtype)) return launch_stream(a, dtype, s);
     return dtype == TTSDPA_F32 ? launch_mfma<F32>(a, s) : dtype == TTSDPA_F16 ? launch_mfma<F16>(a, s) : launch_mfma<BF16>(a, s);
   }
   switch (dtype) {
@@ -1063,9 +894,13 @@ int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, v
     };
     if (in_place(a, trans_a, M, lda) && in_place(b, !trans_b, N, ldb)) {
       LinArgs g{a, b, bias, out, M, N, K, lda, ldb, ldo, trans_a ? 1 : 0, trans_b ? 0 : 1};
+      if (streams(g, dtype)) return launch_stream(g, dtype, s);
       return dtype == TTSDPA_F16 ? launch_mfma_t<F16>(g, s) : launch_mfma_t<BF16>(g, s);
     }
   }
+
+  const LinArgs g{a, b, bias, out, M, N, K, lda, ldb, ldo, trans_a ? 1 : 0, trans_b ? 0 : 1};
+  if (dtype == TTSDPA_F32 && streams(g, dtype)) return launch_stream(g, dtype, s);
 
   // MFMA route: dense row-major copies of the operands that are stored contraction-major, then the x . w^T kernel
   const size_t need = ttlinear_matmul_workspace_bytes(dtype, M, N, K, trans_a, trans_b);
@@ -1094,7 +929,6 @@ int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, v
       return ttlinear_forward(dtype, x, w, bias, out, M, N, K, ldx, ldw, ldo, stream);
     }
   }
-  LinArgs g{a, b, bias, out, M, N, K, lda, ldb, ldo, trans_a ? 1 : 0, trans_b ? 0 : 1};
   switch (dtype) {
     case TTSDPA_F32: return launch_general_linear<float>(g, s);
     case TTSDPA_F16: return launch_general_linear<_Float16>(g, s);
@@ -1130,7 +964,7 @@ int ttlinear_matmul_batched(int dtype, const void* a, const void* b, const void*
   // One grid for all entries (the reference's strided-batched product, src/Operation/OpLinalg.cpp:113-150) when the
   // entries' offsets are a multiple of the entry index in both operands (no broadcast pattern that breaks the stride)
   // and an entry is small enough that a launch each would be launch-bound; x . w^T on the tiled matrix-core kernel when
-  // the layout allows, every other flag pair on the vector-ALU kernel, which reads the operands in place.
+  // the layout allows and its tiles are worth it, else on the general route, which reads the operands in place.
   if (entries > 1 && entries <= 65535 && M > 0 && N > 0 && K > 0 && a && b && out && (double)M * N * K <= (double)(1 << 27)) {
     long long sa = 0, sb = 0;
     offsets(1, &sa, &sb);
@@ -1148,7 +982,7 @@ int ttlinear_matmul_batched(int dtype, const void* a, const void* b, const void*
       int route = TTLINEAR_ROUTE_NONE;
       const long long kpc = 16 / (long long)esz;
       if (!trans_a && trans_b && check(dtype, a, b, out, M, N, K, lda, ldb, ldo, &route) == TTSDPA_OK && route == TTLINEAR_ROUTE_MFMA &&
-          sa % kpc == 0 && sb % kpc == 0 && out_batch_stride % 4 == 0 && !(dtype != TTSDPA_F32 && M <= 64 && N >= 64)) {
+          sa % kpc == 0 && sb % kpc == 0 && out_batch_stride % 4 == 0 && !streams(g, dtype, (unsigned)entries)) {
         g.xt = g.wt = 0;
         switch (dtype) {
           case TTSDPA_F32: return launch_mfma_tile<F32, 128, 128, 4, 2>(g, s, (unsigned)entries);

@@ -1,0 +1,26 @@
+// Argument block of the linear-layer kernels (linear.hip, linear_stream.hip).
+#pragma once
+
+#include "sdpa_common.h"
+
+namespace ttsdpa {
+
+struct LinArgs {
+  const void* x;
+  const void* w;
+  const void* bias;
+  void* out;
+  long long M, N, K, ldx, ldw, ldo;
+  // x is stored [K, M] (x(m,k) = x[k*ldx + m]) / w is stored [K, N] (w(n,k) = w[k*ldw + n])
+  int xt = 0, wt = 0;
+  // batch entries of one launch: entry e reads x + e*bsx, w + e*bsw and writes out + e*bso (elements; 0 = the operand is
+  // shared by all entries)
+  long long bsx = 0, bsw = 0, bso = 0;
+};
+
+// linear_stream.hip: products whose wavefronts divide the contraction among themselves, for any alignment of the operands.
+bool stream_takes(const LinArgs& a, int dtype);                             // sizes and strides are in its range
+double stream_cost(const LinArgs& a, int dtype, unsigned entries);          // estimated microseconds
+int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, unsigned entries = 1);
+
+}  // namespace ttsdpa

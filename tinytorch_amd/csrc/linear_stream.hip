@@ -1,0 +1,392 @@
+// Products whose wavefronts divide the contraction among themselves, for gfx950: few rows of x against a large weight
+// (a decode step's projections), small layers, and operands of any alignment and size (reference: op::matmul,
+// src/Operation/OpLinalg.cpp:52-276; device GEMM src/Operation/OpLinalgCuda.cuh:239-293).
+//
+//   out[m][n] = bias[n] + sum_k x(m,k) w(n,k)     x(m,k) = XT ? x[k*ldx + m] : x[m*ldx + k], w(n,k) likewise
+//
+// What bounds these shapes is latency and the bytes in flight, not the matrix pipe: a workgroup owns a small tile of the
+// output (16*MB rows of x by 16*NB of w) and its W wavefronts take the 128-byte pieces (units) of the contraction in turn,
+// each with a ring of P units of its own in registers; no barrier until the partial sums meet in LDS at the end.
+//   operands     a step of a unit is the 16 bytes that a lane supplies to v_mfma_f32_16x16x32 (16-bit: row l%16, k = 8(l/16)
+//                .. +7) or to four v_mfma_f32_16x16x4 (fp32: k = 4(l/16) + e in instruction e, the same pairing on both
+//                sides)
+//   loads        into registers, at any alignment, eight lanes to the 128 bytes of a row; then through a piece of LDS of the
+//                wavefront's own into operand order.  (Straight into operand order saves the LDS, but there 16 neighbouring
+//                lanes belong to 16 rows: a CU took in 16 bytes per clock, 24 x 2048 x 5632 ran 13 us instead of 7.4.)
+//   k-major      an operand stored [K, rows]: 16-bit loads 16 bytes along the rows and reads LDS transposed
+//                (ds_read_b64_tr_b16); fp32 loads its elements straight into operand order (64 contiguous bytes per k)
+//   edges        rows past the end re-read the last one (k-major: the last tile is moved back to end with the matrix).
+
+#include "linear_args.h"
+
+namespace ttsdpa {
+namespace {
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// 16 bytes at any element's address (rows may begin anywhere)
+typedef uint32_t loose16 __attribute__((ext_vector_type(4), aligned(2)));
+
+template <typename TR>
+struct Step {
+  typedef typename TR::elem elem;
+  typedef typename TR::vec8 frag;
+  static constexpr int KV = 8;  // consecutive k of a lane
+  static __device__ __forceinline__ f32x4 mma(frag a, frag b, f32x4 c) { return TR::mfma16(a, b, c); }
+};
+struct F32 {};
+template <>
+struct Step<F32> {
+  typedef float elem;
+  typedef f32x4 frag;
+  static constexpr int KV = 4;
+  static __device__ __forceinline__ f32x4 mma(frag a, frag b, f32x4 c) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+    return c;
+  }
+};
+
+// One operand of a tile: R blocks of 16 rows from `row0` on.  A unit of the contraction is 128 bytes of a row: 64 k of a
+// 16-bit type, 32 of fp32, two steps of 16 bytes per lane of an operand register.
+template <typename TR, bool KMAJOR, int R>
+struct Operand {
+  typedef Step<TR> S;
+  typedef typename S::elem T;
+  typedef typename S::frag frag;
+  static constexpr int KV = S::KV, KU = 8 * KV;             // k of a unit
+  static constexpr bool DIRECT = KMAJOR && KV == 4;         // fp32, k-major: no LDS
+  static constexpr int PITCH = 32 * R + 16;                 // 16-bit, k-major: bytes of a k-row in LDS (4 rows in different banks)
+  static constexpr int LDS = DIRECT ? 0 : KMAJOR ? KU * PITCH : 16 * R * 128;
+  static constexpr int NL = 2 * R;                        // 16-byte registers of a unit
+  static constexpr int CPR = KMAJOR ? 2 * R : 8, RPI = 64 / CPR;  // 16-byte chunks of a row as loaded, rows of one load instruction
+
+  const char* base;  // of the first row at k = 0
+  unsigned off[NL];  // bytes from base (+ the unit's advance) of what this lane loads
+  long long ld;      // bytes
+  int lane;
+
+  // `rows`: rows of the tile, at most 16 * R; those beyond re-read its last one
+  __device__ __forceinline__ void init(const void* p, long long row0, int rows, long long ld_elems, int lane_) {
+    lane = lane_;
+    ld = ld_elems * (long long)sizeof(T);
+    base = (const char*)p + (KMAJOR ? row0 * (long long)sizeof(T) : row0 * ld);
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+      if constexpr (DIRECT) {  // register i: block i / 2, step i % 2, k = 16 (i % 2) + 4 (lane / 16) + element
+        off[i] = (unsigned)((16 * (i & 1) + 4 * (lane >> 4)) * ld + (16 * (i >> 1) + (lane & 15)) * (long long)sizeof(T));
+      } else {
+        const int r = RPI * i + lane / CPR;
+        off[i] = (unsigned)((KMAJOR || r < rows ? r : rows - 1) * ld + 16 * (lane % CPR));
+      }
+    }
+  }
+
+  // k0: the unit's first k
+  __device__ __forceinline__ void load(u32x4 (&v)[NL], long long k0) const {
+    const char* at = base + k0 * (KMAJOR ? ld : (long long)sizeof(T));
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+      if constexpr (DIRECT) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[i][e] = *(const uint32_t*)(at + e * ld + off[i]);
+      } else {
+        v[i] = *(const loose16*)(at + off[i]);
+      }
+    }
+  }
+
+  // k of the first element that this lane loaded into register i, from the unit's first
+  __device__ __forceinline__ int k_of(int i) const {
+    return DIRECT ? 16 * (i & 1) + 4 * (lane >> 4) : KMAJOR ? RPI * i + lane / CPR : KV * (lane % CPR);
+  }
+
+  // zeros for the first `skip` k of the unit (the last unit of a contraction that is no whole number of units begins
+  // before the one in front of it ends)
+  __device__ __forceinline__ void clear(u32x4 (&v)[NL], int skip) const {
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+      const int gone = skip - k_of(i);
+      if constexpr (KMAJOR && !DIRECT) {
+        if (gone > 0) v[i] = u32x4{0u, 0u, 0u, 0u};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          if constexpr (KV == 4) v[i][e] = e < gone ? 0u : v[i][e];
+          else v[i][e] = 2 * e + 1 < gone ? 0u : 2 * e < gone ? v[i][e] & 0xffff0000u : v[i][e];
+        }
+      }
+    }
+  }
+
+  // a contraction of K < KU elements, then zeros
+  __device__ __forceinline__ void load_short(u32x4 (&v)[NL], int K) const {
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+      v[i] = u32x4{0u, 0u, 0u, 0u};
+      const int left = K - k_of(i);
+      if constexpr (KMAJOR && !DIRECT) {
+        if (left > 0) v[i] = *(const loose16*)(base + off[i]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < KV; e++)
+          if (e < left) {
+            const char* p = base + off[i] + (DIRECT ? e * ld : e * (long long)sizeof(T));
+            if constexpr (KV == 4) v[i][e] = *(const uint32_t*)p;
+            else v[i][e >> 1] |= (uint32_t)*(const uint16_t*)p << (16 * (e & 1));
+          }
+      }
+    }
+  }
+
+  // what was loaded, into the wavefront's piece of LDS (its LDS instructions run in order: no waits between the two)
+  __device__ __forceinline__ void stage(const u32x4 (&v)[NL], char* lds) const {
+    if constexpr (!DIRECT)
+#pragma unroll
+      for (int i = 0; i < NL; i++) {
+        const int r = RPI * i + lane / CPR, c = lane % CPR;
+        if constexpr (KMAJOR) *(u32x4*)(lds + r * PITCH + 16 * c) = v[i];
+        else *(u32x4*)(lds + r * 128 + 16 * (c ^ ((r >> 1) & 7))) = v[i];  // 16 rows of a chunk fall into different banks
+      }
+  }
+
+  // operand registers of step s (0 or 1) of the unit
+  __device__ __forceinline__ void frags(frag (&f)[R], const u32x4 (&v)[NL], const char* lds, int s) const {
+    const int r = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int b = 0; b < R; b++) {
+      if constexpr (DIRECT) {
+        f[b] = __builtin_bit_cast(frag, v[2 * b + s]);
+      } else if constexpr (KMAJOR) {
+        const char* from = lds + (32 * s + 8 * q + (r >> 2)) * PITCH + 8 * (r & 3) + 32 * b;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)from);
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(from + 4 * PITCH));
+        f[b] = __builtin_bit_cast(frag, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      } else {
+        f[b] = *(const frag*)(lds + (16 * b + r) * 128 + 16 * ((4 * s + q) ^ ((r >> 1) & 7)));
+      }
+    }
+  }
+};
+
+template <typename TR, bool XT, bool WT, int MB, int NB, int W>
+struct StreamLds {
+  static constexpr int STAGE = Operand<TR, XT, MB>::LDS + Operand<TR, WT, NB>::LDS;  // per wavefront
+  static constexpr int PITCH = 16 * NB + 4;                                            // floats of a row of partial sums
+  static constexpr int SUMS = 16 * MB * PITCH * 4;                                     // per wavefront
+  static constexpr int BYTES = W * (STAGE > SUMS ? STAGE : SUMS);
+};
+
+template <typename TR, bool XT, bool WT, int MB, int NB, int W, int P>
+__global__ __launch_bounds__(64 * W, W / 4) void linear_stream_kernel(LinArgs a) {
+  typedef Operand<TR, XT, MB> OX;
+  typedef Operand<TR, WT, NB> OW;
+  typedef StreamLds<TR, XT, WT, MB, NB, W> Lds;
+  typedef typename Step<TR>::elem T;
+  typedef typename Step<TR>::frag frag;
+  constexpr int TM = 16 * MB, TN = 16 * NB, KU = OX::KU;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+  // workgroup -> tile: an XCD (workgroup i runs on XCD i % 8) takes a contiguous band of tiles, rows of x fastest, so that
+  // the workgroups that read a piece of w run side by side
+  const int tiles_m = (int)((a.M + TM - 1) / TM), tiles_n = (int)((a.N + TN - 1) / TN);
+  const int band = (tiles_m * tiles_n + 7) / 8;
+  const int tile = (blockIdx.x & 7) * band + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= band || tile >= tiles_m * tiles_n) return;
+  long long m0 = (long long)(tile % tiles_m) * TM, n0 = (long long)(tile / tiles_m) * TN;
+  if (XT && m0 > a.M - TM) m0 = a.M - TM;  // k-major operands have at least a tile of rows (the host sees to it)
+  if (WT && n0 > a.N - TN) n0 = a.N - TN;
+
+  OX ox;
+  OW ow;
+  ox.init((const T*)a.x + (long long)blockIdx.y * a.bsx, m0, a.M - m0 < TM ? (int)(a.M - m0) : TM, a.ldx, lane);
+  ow.init((const T*)a.w + (long long)blockIdx.y * a.bsw, n0, a.N - n0 < TN ? (int)(a.N - n0) : TN, a.ldw, lane);
+  char* stage = smem + wave * Lds::STAGE;
+
+  f32x4 acc[NB][MB];
+#pragma unroll
+  for (int i = 0; i < NB; i++)
+#pragma unroll
+    for (int j = 0; j < MB; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  u32x4 xv[P][OX::NL], wv[P][OW::NL];
+  auto use = [&](int p) __attribute__((always_inline)) {
+    ow.stage(wv[p], stage + OX::LDS);
+    ox.stage(xv[p], stage);
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      frag xf[MB], wf[NB];
+      ow.frags(wf, wv[p], stage + OX::LDS, s);
+      ox.frags(xf, xv[p], stage, s);
+#pragma unroll
+      for (int i = 0; i < NB; i++)
+#pragma unroll
+        for (int j = 0; j < MB; j++) acc[i][j] = Step<TR>::mma(wf[i], xf[j], acc[i][j]);
+    }
+  };
+
+  // unit i of the contraction belongs to wavefront i % W; a last, incomplete one is read as the KU elements in front of
+  // the end, those of the unit before it as zeros
+  const int K = (int)a.K, units = (K + KU - 1) / KU;
+  const int n = units > wave ? (units - wave + W - 1) / W : 0;
+  const bool overlaps = K % KU != 0 && n > 0 && (n - 1) * W + wave == units - 1;  // this wavefront's last unit is that one
+  auto first_k = [&](int j) __attribute__((always_inline)) {
+    const int k = ((j < n ? j : n - 1) * W + wave) * KU;  // requests past the end repeat the last unit (never used)
+    return (long long)(k < K - KU ? k : K - KU);
+  };
+  if (K < KU) {
+    if (n > 0) {
+      ow.load_short(wv[0], K);
+      ox.load_short(xv[0], K);
+      use(0);
+    }
+  } else if (n > 0) {
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+      ow.load(wv[p], first_k(p));
+      ox.load(xv[p], first_k(p));
+    }
+    int j0 = 0;
+    for (; j0 + P < n; j0 += P)
+#pragma unroll
+      for (int p = 0; p < P; p++) {
+        use(p);
+        ow.load(wv[p], first_k(j0 + P + p));
+        ox.load(xv[p], first_k(j0 + P + p));
+      }
+#pragma unroll
+    for (int p = 0; p < P; p++)
+      if (j0 + p < n) {
+        if (overlaps && j0 + p == n - 1) {
+          ow.clear(wv[p], KU - K % KU);
+          ox.clear(xv[p], KU - K % KU);
+        }
+        use(p);
+      }
+  }
+
+  // partial sums: a lane holds rows m = 16j + l%16, columns n = 16i + 4(l/16) .. +3
+  __syncthreads();  // (the staging pieces of other wavefronts lie where the sums go)
+  float* sums = (float*)smem + wave * (Lds::SUMS / 4);
+#pragma unroll
+  for (int i = 0; i < NB; i++)
+#pragma unroll
+    for (int j = 0; j < MB; j++) *(f32x4*)(sums + (16 * j + (lane & 15)) * Lds::PITCH + 16 * i + 4 * (lane >> 4)) = acc[i][j];
+  __syncthreads();
+  const bool whole = (a.ldo & 3) == 0 && ((uintptr_t)a.out & (4 * sizeof(T) - 1)) == 0 && (a.bso & 3) == 0 && (n0 & 3) == 0;
+  for (int g = threadIdx.x; g < TM * (TN / 4); g += 64 * W) {
+    const int r = g / (TN / 4), c = 4 * (g % (TN / 4));
+    const long long m = m0 + r, col = n0 + c;
+    if (m >= a.M || col >= a.N) continue;
+    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; w++) v += *(const f32x4*)((const float*)smem + w * (Lds::SUMS / 4) + r * Lds::PITCH + c);
+    const int have = a.N - col < 4 ? (int)(a.N - col) : 4;
+    if (a.bias)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (e < have) v[e] += load_as_float((const T*)a.bias + col + e);
+    T* dst = (T*)a.out + (long long)blockIdx.y * a.bso + m * a.ldo + col;
+    if (whole && have == 4) {
+      typedef T out4 __attribute__((ext_vector_type(4)));
+      *(out4*)dst = __builtin_convertvector(v, out4);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (e < have) store_from_float(dst + e, v[e]);
+    }
+  }
+}
+
+template <typename TR, bool XT, bool WT, int MB, int NB, int W, int P>
+int launch_variant(const LinArgs& a, hipStream_t stream, unsigned entries) {
+  static hipError_t state[kMaxDevices];
+  static bool done[kMaxDevices];
+  constexpr int lds = StreamLds<TR, XT, WT, MB, NB, W>::BYTES;
+  const hipError_t granted = grant_dynamic_lds((const void*)linear_stream_kernel<TR, XT, WT, MB, NB, W, P>, lds, state, done);
+  if (granted != hipSuccess) return (int)granted;
+  const long long tiles = ((a.M + 16 * MB - 1) / (16 * MB)) * ((a.N + 16 * NB - 1) / (16 * NB));
+  if (tiles > 0x3fffffffLL) return -3;  // TTSDPA_ERR_SHAPE
+  hipLaunchKernelGGL((linear_stream_kernel<TR, XT, WT, MB, NB, W, P>), dim3((unsigned)((tiles + 7) / 8 * 8), entries), dim3(64 * W), lds, stream, a);
+  return (int)hipGetLastError();
+}
+
+}  // namespace
+
+namespace {
+
+// Microseconds of a product on tiles of 16*R rows of x by 16*R of w, from measurements (MI355X, 16-bit unless said):
+// 3 us of launch, latency and the meeting of the partial sums (2 more on the largest tile: a wavefront's sums are 16 KB);
+// then, for each round of the 256 CUs, half a microsecond and the operands of a tile at the 65 GB/s that a CU takes in
+// (it measured 60-75 over all shapes), or the tile's products where those take longer (fp32: 0.45 TFLOP/s of a CU's 0.61 on
+// the largest tile, 0.3 on the others).
+//   measured / this: 1000^3 on 16, 32, 64: 25 / 26, 12 / 13, 9.5 / 9.4; 24 x 2048 x 5632: 7.4 / 9, 10.5 / 13, 19 / 21;
+//   64 x 4096 x 4096: 17 / 20, 11 / 12, 21 / 22; fp32 1000^3: 42 / 43, 30 / 32, 25 / 24
+double stream_us(const LinArgs& a, int esz, int R, unsigned entries) {
+  const double tm = 16 * R, tn = 16 * R;
+  const double tiles = (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)) * entries;
+  const double rounds = tiles > 256 ? tiles / 256 : 1;
+  const double bytes = ((a.M < tm ? a.M : tm) + (a.N < tn ? a.N : tn)) * (double)a.K * esz;
+  const double flops = 2 * tm * tn * (double)a.K;
+  const double rate = esz == 2 ? 4e6 : R == 4 ? 0.45e6 : 0.3e6;
+  const double per = bytes / 65e3 > flops / rate ? bytes / 65e3 : flops / rate;
+  return (R == 4 ? 5 : 3) + rounds * (0.5 + per);
+}
+
+// Rows of a tile in blocks of 16: the cheapest of 1, 2 and 4 that a k-major operand has the rows for.
+int stream_rows(const LinArgs& a, int esz, unsigned entries, double* us) {
+  int best = 0;
+  for (int R = 1; R <= 4; R *= 2) {
+    if ((a.xt && a.M < 16 * R) || (a.wt && a.N < 16 * R)) break;
+    const double t = stream_us(a, esz, R, entries);
+    if (!best || t < *us) best = R, *us = t;
+  }
+  return best;
+}
+
+template <typename TR, bool XT, bool WT>
+int launch_rows(const LinArgs& a, int R, hipStream_t stream, unsigned entries) {
+  // eight wavefronts with a ring of as many units as their registers hold; on the largest tile four, which have twice the
+  // registers (eight measure the same with the bytes in flight that theirs allow, and spill)
+  if (R == 1) return launch_variant<TR, XT, WT, 1, 1, 8, 4>(a, stream, entries);
+  if (R == 2) return launch_variant<TR, XT, WT, 2, 2, 8, 2>(a, stream, entries);
+  return launch_variant<TR, XT, WT, 4, 4, 4, 1>(a, stream, entries);
+}
+
+template <typename TR>
+int launch_type(const LinArgs& a, int R, hipStream_t stream, unsigned entries) {
+  if (a.xt) return a.wt ? launch_rows<TR, true, true>(a, R, stream, entries) : launch_rows<TR, true, false>(a, R, stream, entries);
+  return a.wt ? launch_rows<TR, false, true>(a, R, stream, entries) : launch_rows<TR, false, false>(a, R, stream, entries);
+}
+
+}  // namespace
+
+bool stream_takes(const LinArgs& a, int dtype) {
+  // a tile's rows and a unit's k-rows are addressed with 32-bit byte offsets
+  const long long ld_max = 1ll << 24;
+  if (a.K < 1 || a.K > 0x3fffffffLL || a.ldx >= ld_max || a.ldw >= ld_max) return false;
+  double us;
+  return stream_rows(a, dtype == 0 ? 4 : 2, 1, &us) > 0;
+}
+
+double stream_cost(const LinArgs& a, int dtype, unsigned entries) {
+  double us = 0;
+  stream_rows(a, dtype == 0 ? 4 : 2, entries, &us);
+  return us;
+}
+
+int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, unsigned entries) {
+  double us;
+  const int R = stream_rows(a, dtype == 0 ? 4 : 2, entries, &us);
+  switch (dtype) {
+    case 0: return launch_type<F32>(a, R, stream, entries);
+    case 1: return launch_type<F16>(a, R, stream, entries);
+    default: return launch_type<BF16>(a, R, stream, entries);
+  }
+}
+
+}  // namespace ttsdpa
