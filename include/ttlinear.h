@@ -51,11 +51,22 @@ int ttlinear_plan(int dtype, const void* x, const void* w, const void* bias, con
  * row count a multiple of 8): no scratch is used then and workspace may be NULL.
  * workspace: ttlinear_matmul_workspace_bytes() bytes of device scratch, 256-byte aligned — for fp32 the MFMA route first
  * makes dense row-major copies of the operands that are stored contraction-major; with less (or NULL), or for shapes the
- * tiled kernels do not take, the general route reads the operands in place.  Same return codes as ttlinear_forward. */
+ * tiled kernels do not take, the general route reads the operands in place; and it lets products with few tiles divide their
+ * contraction among workgroups ((false, true) included: what ttlinear_forward cannot do).  Same return codes as ttlinear_forward. */
 size_t ttlinear_matmul_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b);
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
                     int trans_a, int trans_b, int64_t lda, int64_t ldb, int64_t ldo, void* workspace,
                     size_t workspace_bytes, void* stream);
+
+/* FuncLinear::backward (reference src/Function/FuncNNLayer.h:20-33) in one call: from the upstream gradient grad [M,N], the
+ * forward's x [M,K] and w [N,K] (row strides ldg, ldx, ldw in elements)
+ *   grad_x [M,K] = grad . w,   grad_w [N,K] = grad^T . x,   grad_b [N] = column sums of grad (NULL: not wanted),
+ * all dense, sums in fp32, one rounding of each result.  M, N, K > 0.  workspace: ttlinear_backward_workspace_bytes() bytes of
+ * device scratch, 256-byte aligned (TTSDPA_ERR_WORKSPACE with less).  Enqueues on `stream`. */
+size_t ttlinear_backward_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
+int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w, void* grad_x, void* grad_w, void* grad_b, int64_t M,
+                      int64_t N, int64_t K, int64_t ldg, int64_t ldx, int64_t ldw, void* workspace, size_t workspace_bytes,
+                      void* stream);
 
 /* op::matmul with batch dimensions (reference src/Operation/OpLinalg.cpp:107-223: leading dimensions of the two
  * operands broadcast against each other; its device path is a strided-batched or pointer-array GEMM, its CPU path a

@@ -74,3 +74,35 @@ def test_batched_entries():
     exp = a.double().cpu().numpy().swapaxes(-1, -2) @ b.double().cpu().numpy()
     got = matmul(a, b, True, False).double().cpu().numpy()
     assert np.abs(got - exp).max() <= 40 * 2.0 ** -24 * 35 * 4
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("M,K,N", [(1, 16, 16), (3, 17, 40), (64, 784, 500), (65, 130, 33), (200, 64, 1000), (1001, 515, 300),
+                                   (7, 5, 9), (2100, 136, 72)])
+def test_backward_of_a_layer(M, K, N, dtype):
+    """Both gradients and the bias's: one launch for small layers (tiles of 16, 32 and 64), separate kernels for operands too
+    narrow for it, column sums over several row ranges."""
+    from tinytorch_amd import linearBackward
+    print("layer backward M%d K%d N%d %s" % (M, K, N, dtype), flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    go, x, w = (torch.randn(*s, device="cuda", generator=g).to(TORCH_DTYPE[dtype]) for s in ((M, N), (M, K), (N, K)))
+    got = linearBackward(go, x, w)
+    god, xd, wd = (t.double().cpu().numpy() for t in (go, x, w))
+    ones = np.ones((M, 1))
+    for name, out, a, b in (("input", got[0], god, wd), ("weight", got[1], god.T, xd), ("bias", got[2][:, None], god.T, ones)):
+        exp, size, n = a @ b, np.abs(a) @ np.abs(b), a.shape[1]
+        err = np.abs(out.double().cpu().numpy() - exp)
+        assert (err <= EPS[dtype] * np.abs(exp) + (n + 2) * 2.0 ** -24 * size + 1e-30).all(), (name, err.max())
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("M,N", [(1, 1), (63, 127), (65, 129), (1500, 200), (5000, 70), (8192, 1030)])
+def test_column_sums(M, N, dtype):
+    """The bias's gradient where it has a kernel of its own (a layer with 8 inputs is too narrow for the joint launch)."""
+    from tinytorch_amd import linearBackward
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    go, x, w = (torch.randn(*s, device="cuda", generator=g).to(TORCH_DTYPE[dtype]) for s in ((M, N), (M, 8), (N, 8)))
+    got = linearBackward(go, x, w)[2].double().cpu().numpy()
+    god = go.double().cpu().numpy()
+    exp, size = god.sum(0), np.abs(god).sum(0)
+    assert (np.abs(got - exp) <= EPS[dtype] * np.abs(exp) + M * 2.0 ** -24 * size).all()

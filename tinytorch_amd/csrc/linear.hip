@@ -704,6 +704,80 @@ int launch_transpose(const void* src, void* dst, long long R, long long C, long 
   return (int)hipGetLastError();
 }
 
+// Column sums out[n] = sum_m x[m][n] in fp32 (the bias's gradient; reference op::sumOnDim behind src/Function/FuncNNLayer.h:30).
+// Bound by reading x: 1024 lanes take 16 (fp32: 8) columns of 16 bytes side by side and 64 rows at a time, so a column
+// block of 1000 rows is some 16 loads in flight per lane and the chip is filled with row ranges (blockIdx.y), whose
+// partial sums `part` [ranges][N] colsum_merge_kernel adds.  8192 x 6144 bf16: 16 + 3 us; the cast, the library
+// reduction and the cast back that it replaces took 44 + 47 + 5.
+template <typename T>
+__global__ __launch_bounds__(1024) void colsum_kernel(const T* x, long long M, long long N, long long ld, long long rows, T* out, float* part) {
+  constexpr int V = 16 / sizeof(T), LANES = 16;
+  typedef uint32_t loose16 __attribute__((ext_vector_type(4), aligned(2)));
+  __shared__ float sums[64][LANES * V + 1];
+  const int c = threadIdx.x % LANES, g = threadIdx.x / LANES;  // 16 bytes of columns, row group
+  const long long n0 = (long long)blockIdx.x * (LANES * V), n = n0 + V * c;
+  const long long m0 = blockIdx.y * rows, m1 = m0 + rows < M ? m0 + rows : M;
+  float acc[V];
+#pragma unroll
+  for (int e = 0; e < V; e++) acc[e] = 0.f;
+  if (n + V <= N) {
+    const T* p = x + n;
+#pragma unroll 8
+    for (long long m = m0 + g; m < m1; m += 64) {
+      typedef T vecT __attribute__((ext_vector_type(V)));
+      const vecT v = __builtin_bit_cast(vecT, (u32x4)*(const loose16*)(p + m * ld));
+#pragma unroll
+      for (int e = 0; e < V; e++) acc[e] += (float)v[e];
+    }
+  } else {
+    for (long long m = m0 + g; m < m1; m += 64)
+#pragma unroll
+      for (int e = 0; e < V; e++)
+        if (n + e < N) acc[e] += load_as_float(x + m * ld + n + e);
+  }
+#pragma unroll
+  for (int e = 0; e < V; e++) sums[g][V * c + e] = acc[e];
+  __syncthreads();
+  if (threadIdx.x < LANES * V && n0 + threadIdx.x < N) {
+    float v = 0.f;
+#pragma unroll 16
+    for (int i = 0; i < 64; i++) v += sums[i][threadIdx.x];
+    if (part) part[blockIdx.y * N + n0 + threadIdx.x] = v;
+    else store_from_float(out + n0 + threadIdx.x, v);
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void colsum_merge_kernel(const float* part, int ranges, long long N, T* out) {
+  const long long n = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (n >= N) return;
+  float v = 0.f;
+#pragma unroll 8
+  for (int i = 0; i < ranges; i++) v += part[i * N + n];
+  store_from_float(out + n, v);
+}
+
+// Row ranges: enough for two workgroups per CU, of no fewer than 1024 rows' worth of work each (16 loads per lane).
+int colsum_ranges(long long M, long long N, int dtype) {
+  const long long wide = dtype == TTSDPA_F32 ? 64 : 128, blocks = (N + wide - 1) / wide;
+  long long want = (512 + blocks - 1) / blocks;
+  const long long most = M / 512;
+  if (want > most) want = most;
+  return want > 1 ? (int)want : 1;
+}
+
+template <typename T>
+int launch_colsum(const void* x, long long M, long long N, long long ld, void* out, float* part, int ranges, hipStream_t stream) {
+  constexpr int wide = 16 * (16 / (int)sizeof(T));
+  const long long rows = (M + ranges - 1) / ranges;
+  if ((N + wide - 1) / wide > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
+  hipLaunchKernelGGL((colsum_kernel<T>), dim3((unsigned)((N + wide - 1) / wide), (unsigned)ranges), dim3(1024), 0, stream, (const T*)x, M, N, ld,
+                     rows, (T*)out, ranges > 1 ? part : nullptr);
+  if (ranges > 1)
+    hipLaunchKernelGGL((colsum_merge_kernel<T>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, part, ranges, N, (T*)out);
+  return (int)hipGetLastError();
+}
+
 bool aligned(const void* p, size_t n) { return ((uintptr_t)p % n) == 0; }
 
 int check(int dtype, const void* x, const void* w, const void* out, long long M, long long N, long long K, long long ldx,
@@ -800,24 +874,24 @@ int launch_mfma(const LinArgs& a, hipStream_t stream) {
 // Microseconds of the tiled kernels, from measurements, against the streaming kernel's: a k-step of 128 bytes of a 128 x 128
 // tile takes 0.6 us (fp32 2.2) as long as every CU has one tile at most, and with more in proportion (128 .. 1000 x 4096
 // x 4096: 40 .. 45 us, 2000 rows 74; the 256 x 256 tiles are faster, but no product that fills the chip with them is
-// small enough for the other kernel).  k-major operands: 10 % more.
+// small enough for the other kernel).  A k-major w alone, in place: 10 % more.
 double tiled_cost(const LinArgs& a, int dtype, unsigned entries) {
   const double tiles = (double)((a.M + 127) / 128) * (double)((a.N + 127) / 128) * entries;
   const double steps = a.K * (dtype == TTSDPA_F32 ? 4 : 2) / 128.0;
   const double us = 3 + steps * (dtype == TTSDPA_F32 ? 2.2 : 0.6) * (tiles > 256 ? tiles / 256 : 1);
-  return a.xt || a.wt ? us * 1.1 : us;
+  return a.wt && !a.xt ? us * 1.1 : us;
 }
 
-bool streams(const LinArgs& a, int dtype, unsigned entries = 1) {
-  return stream_takes(a, dtype) && stream_cost(a, dtype, entries) < tiled_cost(a, dtype, entries);
+bool streams(const LinArgs& a, int dtype, unsigned entries = 1, bool may_split = false) {
+  return stream_takes(a, dtype) && stream_cost(a, dtype, entries, may_split) < tiled_cost(a, dtype, entries);
 }
 
 // What the tiled kernels' layout does not allow: the streaming kernel, or where one of its operands is too narrow for that (a
 // k-major operand of fewer than 16 rows, an empty contraction) the vector ALUs.
 template <typename T>
-int launch_general_linear(const LinArgs& a, hipStream_t stream, unsigned entries = 1) {
+int launch_general_linear(const LinArgs& a, hipStream_t stream, unsigned entries = 1, void* scratch = nullptr, size_t scratch_bytes = 0) {
   const int dtype = sizeof(T) == 4 ? TTSDPA_F32 : std::is_same<T, _Float16>::value ? TTSDPA_F16 : TTSDPA_BF16;
-  if (stream_takes(a, dtype)) return launch_stream(a, dtype, stream, entries);
+  if (stream_takes(a, dtype)) return launch_stream(a, dtype, stream, entries, scratch, scratch_bytes);
   dim3 grid((unsigned)((a.N + 63) / 64), (unsigned)((a.M + 63) / 64), entries);
   hipLaunchKernelGGL((linear_general_kernel<T>), grid, dim3(256), 0, stream, a);
   return (int)hipGetLastError();
@@ -839,8 +913,9 @@ int ttlinear_plan(int dtype, const void* x, const void* w, const void* bias, con
   return rc;
 }
 
-int ttlinear_forward(int dtype, const void* x, const void* w, const void* bias, void* out, int64_t M, int64_t N,
-                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldo, void* stream) {
+// x . w^T + bias; scratch (optional): lets the streaming kernel divide the contraction among workgroups
+static int forward(int dtype, const void* x, const void* w, const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                   int64_t ldw, int64_t ldo, void* scratch, size_t scratch_bytes, void* stream) {
   int route = TTLINEAR_ROUTE_NONE;
   const int rc = check(dtype, x, w, out, M, N, K, ldx, ldw, ldo, &route);
   if (rc != TTSDPA_OK || route == TTLINEAR_ROUTE_NONE) return rc;
@@ -849,14 +924,19 @@ int ttlinear_forward(int dtype, const void* x, const void* w, const void* bias, 
   LinArgs a{x, w, bias, out, M, N, K, ldx, ldw, ldo};
   hipStream_t s = (hipStream_t)stream;
   if (route == TTLINEAR_ROUTE_MFMA) {
-    if (streams(a, dtype)) return launch_stream(a, dtype, s);
+    if (streams(a, dtype, 1, scratch)) return launch_stream(a, dtype, s, 1, scratch, scratch_bytes);
     return dtype == TTSDPA_F32 ? launch_mfma<F32>(a, s) : dtype == TTSDPA_F16 ? launch_mfma<F16>(a, s) : launch_mfma<BF16>(a, s);
   }
   switch (dtype) {
-    case TTSDPA_F32: return launch_general_linear<float>(a, s);
-    case TTSDPA_F16: return launch_general_linear<_Float16>(a, s);
-    default: return launch_general_linear<__bf16>(a, s);
+    case TTSDPA_F32: return launch_general_linear<float>(a, s, 1, scratch, scratch_bytes);
+    case TTSDPA_F16: return launch_general_linear<_Float16>(a, s, 1, scratch, scratch_bytes);
+    default: return launch_general_linear<__bf16>(a, s, 1, scratch, scratch_bytes);
   }
+}
+
+int ttlinear_forward(int dtype, const void* x, const void* w, const void* bias, void* out, int64_t M, int64_t N,
+                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldo, void* stream) {
+  return forward(dtype, x, w, bias, out, M, N, K, ldx, ldw, ldo, nullptr, 0, stream);
 }
 
 // Bytes of the dense transposed copies the MFMA route of ttlinear_matmul makes: a as [M, K] when it is stored [K, M],
@@ -866,15 +946,52 @@ static size_t matmul_copy_bytes(int dtype, int64_t rows, int64_t K) {
   return ((size_t)rows * (size_t)K * esz + 255) / 256 * 256;
 }
 
+// 16-bit operands that the matrix-core kernel reads in place, contraction-major or not (no copies, no scratch).
+static bool in_place_ok(const LinArgs& g, int dtype) {
+  if (dtype == TTSDPA_F32 || g.K < 1 || g.K % 64 != 0 || g.N % 4 != 0 || g.ldo % 4 != 0 || !aligned(g.out, 8)) return false;
+  auto operand_ok = [](const void* p, bool contraction_major, int64_t rows, int64_t ld) {
+    if (!aligned(p, 16) || ld % 8 != 0) return false;
+    // a tile's rows are addressed with 32-bit byte offsets: 64 k-rows of a contraction-major operand, 256 rows otherwise
+    return contraction_major ? (rows % 8 == 0 && ld < (1 << 24)) : ld < (1 << 21);
+  };
+  return operand_ok(g.x, g.xt, g.M, g.ldx) && operand_ok(g.w, g.wt, g.N, g.ldw);
+}
+
+// A product with a contraction-major operand goes to the streaming kernel when the tiled ones do not take it or are estimated
+// slower: 16-bit operands in place, or, given scratch, x . w^T on row-major copies (read and written at 4 TB/s, a launch each).
+static bool matmul_streams(const LinArgs& g, int dtype, bool scratch) {
+  if (!stream_takes(g, dtype)) return false;
+  double tiled = 0;
+  if (in_place_ok(g, dtype)) {
+    tiled = tiled_cost(g, dtype, 1);
+  } else if (scratch && g.K % (dtype == TTSDPA_F32 ? 32 : 64) == 0 && g.N % 4 == 0 && g.ldo % 4 == 0) {
+    LinArgs nt = g;
+    nt.xt = nt.wt = 0;
+    const double copied = ((g.xt ? g.M : 0) + (g.wt ? g.N : 0)) * (double)g.K * (dtype == TTSDPA_F32 ? 8 : 4);
+    tiled = tiled_cost(nt, dtype, 1) + copied / 4e6 + 2.5 * (g.xt + g.wt);
+  }
+  return tiled == 0 || stream_cost(g, dtype, 1, scratch) < tiled;
+}
+
+// Sizes and layout alone.
+static LinArgs flags_args(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
+  return LinArgs{nullptr, nullptr, nullptr, nullptr, M, N, K, trans_a ? M : K, trans_b ? K : N, N, trans_a ? 1 : 0, trans_b ? 0 : 1};
+}
+
 size_t ttlinear_matmul_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return (trans_a ? matmul_copy_bytes(dtype, M, K) : 0) + (!trans_b ? matmul_copy_bytes(dtype, N, K) : 0);
+  const size_t copies = (trans_a ? matmul_copy_bytes(dtype, M, K) : 0) + (!trans_b ? matmul_copy_bytes(dtype, N, K) : 0);
+  const size_t parts = stream_scratch(flags_args(M, N, K, trans_a, trans_b), dtype);
+  return parts > copies ? parts : copies;
 }
 
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
                     int trans_a, int trans_b, int64_t lda, int64_t ldb, int64_t ldo, void* workspace,
                     size_t workspace_bytes, void* stream) {
-  if (!trans_a && trans_b) return ttlinear_forward(dtype, a, b, bias, out, M, N, K, lda, ldb, ldo, stream);
+  const bool scratch_ok = workspace && aligned(workspace, 256);
+  if (!trans_a && trans_b)
+    return forward(dtype, a, b, bias, out, M, N, K, lda, ldb, ldo, scratch_ok ? workspace : nullptr, scratch_ok ? workspace_bytes : 0, stream);
+  if (!scratch_ok) workspace = nullptr, workspace_bytes = 0;
   if (dtype != TTSDPA_F32 && dtype != TTSDPA_F16 && dtype != TTSDPA_BF16) return TTSDPA_ERR_DTYPE;
   if (M < 0 || N < 0 || K < 0) return TTSDPA_ERR_SHAPE;
   if (M == 0 || N == 0) return TTSDPA_OK;
@@ -885,26 +1002,13 @@ int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, v
   if ((M + 63) / 64 > 65535 || (N + 63) / 64 > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
 
-  // 16-bit tensors: the matrix-core kernel that reads contraction-major operands in place (no copies, no scratch)
-  if (dtype != TTSDPA_F32 && K > 0 && K % 64 == 0 && N % 4 == 0 && ldo % 4 == 0 && aligned(out, 8)) {
-    auto in_place = [](const void* p, bool contraction_major, int64_t rows, int64_t ld) {
-      if (!aligned(p, 16) || ld % 8 != 0) return false;
-      // a tile's rows are addressed with 32-bit byte offsets: 64 k-rows of a contraction-major operand, 256 rows otherwise
-      return contraction_major ? (rows % 8 == 0 && ld < (1 << 24)) : ld < (1 << 21);
-    };
-    if (in_place(a, trans_a, M, lda) && in_place(b, !trans_b, N, ldb)) {
-      LinArgs g{a, b, bias, out, M, N, K, lda, ldb, ldo, trans_a ? 1 : 0, trans_b ? 0 : 1};
-      if (streams(g, dtype)) return launch_stream(g, dtype, s);
-      return dtype == TTSDPA_F16 ? launch_mfma_t<F16>(g, s) : launch_mfma_t<BF16>(g, s);
-    }
-  }
-
   const LinArgs g{a, b, bias, out, M, N, K, lda, ldb, ldo, trans_a ? 1 : 0, trans_b ? 0 : 1};
-  if (dtype == TTSDPA_F32 && streams(g, dtype)) return launch_stream(g, dtype, s);
+  if (K > 0 && matmul_streams(g, dtype, workspace)) return launch_stream(g, dtype, s, 1, workspace, workspace_bytes);
+  if (in_place_ok(g, dtype)) return dtype == TTSDPA_F16 ? launch_mfma_t<F16>(g, s) : launch_mfma_t<BF16>(g, s);
 
   // MFMA route: dense row-major copies of the operands that are stored contraction-major, then the x . w^T kernel
   const size_t need = ttlinear_matmul_workspace_bytes(dtype, M, N, K, trans_a, trans_b);
-  if (K > 0 && workspace && workspace_bytes >= need && aligned(workspace, 256)) {
+  if (K > 0 && workspace && workspace_bytes >= need) {
     const void* x = a;
     const void* w = b;
     long long ldx = lda, ldw = ldb;
@@ -930,9 +1034,9 @@ int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, v
     }
   }
   switch (dtype) {
-    case TTSDPA_F32: return launch_general_linear<float>(g, s);
-    case TTSDPA_F16: return launch_general_linear<_Float16>(g, s);
-    default: return launch_general_linear<__bf16>(g, s);
+    case TTSDPA_F32: return launch_general_linear<float>(g, s, 1, workspace, workspace_bytes);
+    case TTSDPA_F16: return launch_general_linear<_Float16>(g, s, 1, workspace, workspace_bytes);
+    default: return launch_general_linear<__bf16>(g, s, 1, workspace, workspace_bytes);
   }
 }
 
@@ -1012,6 +1116,57 @@ int ttlinear_matmul_batched(int dtype, const void* a, const void* b, const void*
     if (rc != 0) return rc;
   }
   return TTSDPA_OK;
+}
+
+size_t ttlinear_backward_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const size_t gi = ttlinear_matmul_workspace_bytes(dtype, M, K, N, 0, 0), gw = ttlinear_matmul_workspace_bytes(dtype, N, K, M, 1, 0);
+  const size_t gb = (size_t)colsum_ranges(M, N, dtype) * (size_t)N * sizeof(float);
+  const size_t pair = stream_pair_scratch(flags_args(N, K, M, 1, 0), flags_args(M, K, N, 0, 0), dtype);
+  size_t most = gi > gw ? gi : gw;  // one after the other on the same scratch
+  if (pair > most) most = pair;
+  return most > gb ? most : gb;
+}
+
+int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w, void* grad_x, void* grad_w, void* grad_b, int64_t M,
+                      int64_t N, int64_t K, int64_t ldg, int64_t ldx, int64_t ldw, void* workspace, size_t workspace_bytes,
+                      void* stream) {
+  if (dtype != TTSDPA_F32 && dtype != TTSDPA_F16 && dtype != TTSDPA_BF16) return TTSDPA_ERR_DTYPE;
+  if (M <= 0 || N <= 0 || K <= 0) return TTSDPA_ERR_SHAPE;
+  if (!grad || !x || !w || !grad_x || !grad_w) return TTSDPA_ERR_NULL;
+  if (ldg < N || ldx < K || ldw < K) return TTSDPA_ERR_STRIDE;
+  const size_t esz = dtype == TTSDPA_F32 ? 4 : 2;
+  if (!aligned(grad, esz) || !aligned(x, esz) || !aligned(w, esz) || !aligned(grad_x, esz) || !aligned(grad_w, esz) || !aligned(grad_b, esz))
+    return TTSDPA_ERR_STRIDE;
+  if (workspace_bytes < ttlinear_backward_workspace_bytes(dtype, M, N, K) || (workspace_bytes && (!workspace || !aligned(workspace, 256))))
+    return TTSDPA_ERR_WORKSPACE;
+  hipStream_t s = (hipStream_t)stream;
+  // grad_w [N,K] = grad^T . x, grad_x [M,K] = grad . w
+  LinArgs gw{grad, x, nullptr, grad_w, N, K, M, ldg, ldx, K, 1, 1};
+  const LinArgs gi{grad, w, nullptr, grad_x, M, K, N, ldg, ldw, K, 0, 1};
+  // Small layers: both products, and the column sums with the weight's, in one launch.  Where the two would be launched
+  // on the streaming kernel anyway and the launches saved (5 us, the column sums' among them) are worth more than what
+  // the common workgroup size may cost (64 x 784 x 500 fp32: 10 us in two launches and 5 for the column sums).
+  const bool gw_streams = matmul_streams(gw, dtype, true);
+  if (gw_streams && matmul_streams(gi, dtype, false) &&
+      stream_pair_cost(gw, gi, dtype) < stream_cost(gw, dtype, 1, true) + stream_cost(gi, dtype, 1, false) + 5) {
+    gw.rowsum = grad_b;
+    return launch_stream_pair(gw, gi, dtype, s, workspace);
+  }
+  int rc = ttlinear_matmul(dtype, grad, w, nullptr, grad_x, M, K, N, 0, 0, ldg, ldw, K, workspace, workspace_bytes, stream);
+  if (rc != 0) return rc;
+  if (gw_streams) {
+    gw.rowsum = grad_b;
+    return launch_stream(gw, dtype, s, 1, workspace, workspace_bytes);
+  }
+  rc = ttlinear_matmul(dtype, grad, x, nullptr, grad_w, N, K, M, 1, 0, ldg, ldx, K, workspace, workspace_bytes, stream);
+  if (rc != 0 || !grad_b) return rc;
+  const int ranges = colsum_ranges(M, N, dtype);
+  switch (dtype) {
+    case TTSDPA_F32: return launch_colsum<float>(grad, M, N, ldg, grad_b, (float*)workspace, ranges, s);
+    case TTSDPA_F16: return launch_colsum<_Float16>(grad, M, N, ldg, grad_b, (float*)workspace, ranges, s);
+    default: return launch_colsum<__bf16>(grad, M, N, ldg, grad_b, (float*)workspace, ranges, s);
+  }
 }
 
 }  // extern "C"

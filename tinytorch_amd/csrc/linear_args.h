@@ -16,11 +16,21 @@ struct LinArgs {
   // batch entries of one launch: entry e reads x + e*bsx, w + e*bsw and writes out + e*bso (elements; 0 = the operand is
   // shared by all entries)
   long long bsx = 0, bsw = 0, bso = 0;
+  // linear_stream.hip: the sums of x over the contraction ([M], or nullptr: not wanted; only with both operands k-major), and the division of the contraction
+  // among `splits` workgroups per tile, whose sums go to part ([splits][M*N + M] floats) to be added by another kernel
+  void* rowsum = nullptr;
+  int splits = 1;
+  float* part = nullptr;
 };
 
 // linear_stream.hip: products whose wavefronts divide the contraction among themselves, for any alignment of the operands.
 bool stream_takes(const LinArgs& a, int dtype);                             // sizes and strides are in its range
-double stream_cost(const LinArgs& a, int dtype, unsigned entries);          // estimated microseconds
-int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, unsigned entries = 1);
+double stream_cost(const LinArgs& a, int dtype, unsigned entries, bool may_split);  // estimated microseconds
+size_t stream_scratch(const LinArgs& a, int dtype);                         // bytes that let it divide the contraction
+int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, unsigned entries = 1, void* scratch = nullptr, size_t scratch_bytes = 0);
+// a layer's two backward products in one launch (gw: both operands k-major; gi: w k-major), each in the kernel's range
+double stream_pair_cost(const LinArgs& gw, const LinArgs& gi, int dtype);
+size_t stream_pair_scratch(const LinArgs& gw, const LinArgs& gi, int dtype);
+int launch_stream_pair(const LinArgs& gw, const LinArgs& gi, int dtype, hipStream_t stream, void* scratch);
 
 }  // namespace ttsdpa

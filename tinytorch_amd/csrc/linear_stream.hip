@@ -17,6 +17,7 @@
 //                (ds_read_b64_tr_b16); fp32 loads its elements straight into operand order (64 contiguous bytes per k)
 //   edges        rows past the end re-read the last one (k-major: the last tile is moved back to end with the matrix).
 
+#include "../../include/ttsdpa.h"
 #include "linear_args.h"
 
 namespace ttsdpa {
@@ -179,15 +180,16 @@ struct StreamLds {
   static constexpr int BYTES = W * (STAGE > SUMS ? STAGE : SUMS);
 };
 
-template <typename TR, bool XT, bool WT, int MB, int NB, int W, int P>
-__global__ __launch_bounds__(64 * W, W / 4) void linear_stream_kernel(LinArgs a) {
+// One tile of the product: workgroup `block` of those of entry `entry`.  ROWSUM: the workgroups of the first column of tiles
+// also write a.rowsum[m] = sum_k x(m,k) (a product with ones that rides along in the matrix pipe).
+template <typename TR, bool XT, bool WT, int MB, int NB, int W, int P, bool ROWSUM>
+__device__ __forceinline__ void stream_tile(const LinArgs& a, char* smem, int block, int entry) {
   typedef Operand<TR, XT, MB> OX;
   typedef Operand<TR, WT, NB> OW;
   typedef StreamLds<TR, XT, WT, MB, NB, W> Lds;
   typedef typename Step<TR>::elem T;
   typedef typename Step<TR>::frag frag;
   constexpr int TM = 16 * MB, TN = 16 * NB, KU = OX::KU;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
@@ -195,16 +197,18 @@ __global__ __launch_bounds__(64 * W, W / 4) void linear_stream_kernel(LinArgs a)
   // the workgroups that read a piece of w run side by side
   const int tiles_m = (int)((a.M + TM - 1) / TM), tiles_n = (int)((a.N + TN - 1) / TN);
   const int band = (tiles_m * tiles_n + 7) / 8;
-  const int tile = (blockIdx.x & 7) * band + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= band || tile >= tiles_m * tiles_n) return;
+  const int split = block / (8 * band);  // range of the contraction
+  block -= split * 8 * band;
+  const int tile = (block & 7) * band + (block >> 3);
+  if (tile >= tiles_m * tiles_n) return;
   long long m0 = (long long)(tile % tiles_m) * TM, n0 = (long long)(tile / tiles_m) * TN;
   if (XT && m0 > a.M - TM) m0 = a.M - TM;  // k-major operands have at least a tile of rows (the host sees to it)
   if (WT && n0 > a.N - TN) n0 = a.N - TN;
 
   OX ox;
   OW ow;
-  ox.init((const T*)a.x + (long long)blockIdx.y * a.bsx, m0, a.M - m0 < TM ? (int)(a.M - m0) : TM, a.ldx, lane);
-  ow.init((const T*)a.w + (long long)blockIdx.y * a.bsw, n0, a.N - n0 < TN ? (int)(a.N - n0) : TN, a.ldw, lane);
+  ox.init((const T*)a.x + (long long)entry * a.bsx, m0, a.M - m0 < TM ? (int)(a.M - m0) : TM, a.ldx, lane);
+  ow.init((const T*)a.w + (long long)entry * a.bsw, n0, a.N - n0 < TN ? (int)(a.N - n0) : TN, a.ldw, lane);
   char* stage = smem + wave * Lds::STAGE;
 
   f32x4 acc[NB][MB];
@@ -212,6 +216,17 @@ __global__ __launch_bounds__(64 * W, W / 4) void linear_stream_kernel(LinArgs a)
   for (int i = 0; i < NB; i++)
 #pragma unroll
     for (int j = 0; j < MB; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  f32x4 rowsum[ROWSUM ? MB : 1];
+  frag ones;
+  bool sums_rows = false;
+  if constexpr (ROWSUM) {
+    sums_rows = a.rowsum && tile < tiles_m;
+#pragma unroll
+    for (int j = 0; j < MB; j++) rowsum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < Step<TR>::KV; e++) ones[e] = (T)1.f;
+  }
 
   u32x4 xv[P][OX::NL], wv[P][OW::NL];
   auto use = [&](int p) __attribute__((always_inline)) {
@@ -226,16 +241,23 @@ __global__ __launch_bounds__(64 * W, W / 4) void linear_stream_kernel(LinArgs a)
       for (int i = 0; i < NB; i++)
 #pragma unroll
         for (int j = 0; j < MB; j++) acc[i][j] = Step<TR>::mma(wf[i], xf[j], acc[i][j]);
+      if constexpr (ROWSUM)
+        if (sums_rows)
+#pragma unroll
+          for (int j = 0; j < MB; j++) rowsum[j] = Step<TR>::mma(ones, xf[j], rowsum[j]);
     }
   };
 
   // unit i of the contraction belongs to wavefront i % W; a last, incomplete one is read as the KU elements in front of
   // the end, those of the unit before it as zeros
-  const int K = (int)a.K, units = (K + KU - 1) / KU;
+  const int K = (int)a.K, all_units = (K + KU - 1) / KU;
+  const int per_split = (all_units + a.splits - 1) / a.splits;
+  const int u0 = split * per_split;  // the split's units: u0 .. u0 + units - 1
+  const int units = all_units - u0 < per_split ? all_units - u0 : per_split;
   const int n = units > wave ? (units - wave + W - 1) / W : 0;
-  const bool overlaps = K % KU != 0 && n > 0 && (n - 1) * W + wave == units - 1;  // this wavefront's last unit is that one
+  const bool overlaps = K % KU != 0 && n > 0 && u0 + (n - 1) * W + wave == all_units - 1;  // this wavefront's last unit is that one
   auto first_k = [&](int j) __attribute__((always_inline)) {
-    const int k = ((j < n ? j : n - 1) * W + wave) * KU;  // requests past the end repeat the last unit (never used)
+    const int k = (u0 + (j < n ? j : n - 1) * W + wave) * KU;  // requests past the end repeat the last unit (never used)
     return (long long)(k < K - KU ? k : K - KU);
   };
   if (K < KU) {
@@ -276,7 +298,20 @@ __global__ __launch_bounds__(64 * W, W / 4) void linear_stream_kernel(LinArgs a)
   for (int i = 0; i < NB; i++)
 #pragma unroll
     for (int j = 0; j < MB; j++) *(f32x4*)(sums + (16 * j + (lane & 15)) * Lds::PITCH + 16 * i + 4 * (lane >> 4)) = acc[i][j];
+  if constexpr (ROWSUM)
+    if (sums_rows && lane < 16)  // (every row of the product with ones is the same)
+#pragma unroll
+      for (int j = 0; j < MB; j++) ((float*)(smem + Lds::BYTES))[wave * TM + 16 * j + lane] = rowsum[j][0];
   __syncthreads();
+  float* part = a.part ? a.part + split * (a.M * a.N + a.M) : nullptr;  // this split's sums: of the product, then of x's rows
+  if constexpr (ROWSUM)
+    if (sums_rows && threadIdx.x < TM && m0 + threadIdx.x < a.M) {
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; w++) v += ((const float*)(smem + Lds::BYTES))[w * TM + threadIdx.x];
+      if (part) part[a.M * a.N + m0 + threadIdx.x] = v;
+      else store_from_float((T*)a.rowsum + m0 + threadIdx.x, v);
+    }
   const bool whole = (a.ldo & 3) == 0 && ((uintptr_t)a.out & (4 * sizeof(T) - 1)) == 0 && (a.bso & 3) == 0 && (n0 & 3) == 0;
   for (int g = threadIdx.x; g < TM * (TN / 4); g += 64 * W) {
     const int r = g / (TN / 4), c = 4 * (g % (TN / 4));
@@ -286,11 +321,20 @@ __global__ __launch_bounds__(64 * W, W / 4) void linear_stream_kernel(LinArgs a)
 #pragma unroll
     for (int w = 0; w < W; w++) v += *(const f32x4*)((const float*)smem + w * (Lds::SUMS / 4) + r * Lds::PITCH + c);
     const int have = a.N - col < 4 ? (int)(a.N - col) : 4;
+    if (part) {
+      float* dst = part + m * a.N + col;
+      if (have == 4 && ((a.N | n0) & 3) == 0) *(f32x4*)dst = v;
+      else
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (e < have) dst[e] = v[e];
+      continue;
+    }
     if (a.bias)
 #pragma unroll
       for (int e = 0; e < 4; e++)
         if (e < have) v[e] += load_as_float((const T*)a.bias + col + e);
-    T* dst = (T*)a.out + (long long)blockIdx.y * a.bso + m * a.ldo + col;
+    T* dst = (T*)a.out + (long long)entry * a.bso + m * a.ldo + col;
     if (whole && have == 4) {
       typedef T out4 __attribute__((ext_vector_type(4)));
       *(out4*)dst = __builtin_convertvector(v, out4);
@@ -302,16 +346,96 @@ __global__ __launch_bounds__(64 * W, W / 4) void linear_stream_kernel(LinArgs a)
   }
 }
 
-template <typename TR, bool XT, bool WT, int MB, int NB, int W, int P>
-int launch_variant(const LinArgs& a, hipStream_t stream, unsigned entries) {
+// out = bias + the sum of the splits' partial products, and the same of the row sums.
+template <typename T>
+__global__ __launch_bounds__(256) void linear_merge_kernel(LinArgs a) {
+  const long long total = a.M * a.N + a.M;
+  const long long per = a.rowsum ? total : a.M * a.N;
+  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4; i < per; i += (long long)gridDim.x * 1024) {
+    if (i + 4 <= a.M * a.N && (a.N & 3) == 0 && (a.ldo & 3) == 0 && (total & 3) == 0) {
+      f32x4 v = *(const f32x4*)(a.part + i);
+#pragma unroll 4
+      for (int s = 1; s < a.splits; s++) v += *(const f32x4*)(a.part + s * total + i);
+      const long long m = i / a.N, n = i % a.N;
+      T* dst = (T*)a.out + m * a.ldo + n;
+#pragma unroll
+      for (int e = 0; e < 4; e++) store_from_float(dst + e, v[e] + (a.bias ? load_as_float((const T*)a.bias + n + e) : 0.f));
+    } else {
+      for (long long k = i; k < i + 4 && k < per; k++) {
+        float v = 0.f;
+#pragma unroll 4
+        for (int s = 0; s < a.splits; s++) v += a.part[s * total + k];
+        if (k >= a.M * a.N) store_from_float((T*)a.rowsum + (k - a.M * a.N), v);
+        else store_from_float((T*)a.out + k / a.N * a.ldo + k % a.N, v + (a.bias ? load_as_float((const T*)a.bias + k % a.N) : 0.f));
+      }
+    }
+  }
+}
+
+template <typename T>
+int launch_merge(const LinArgs& a, hipStream_t stream) {
+  const long long groups = (a.M * a.N + a.M + 1023) / 1024;
+  hipLaunchKernelGGL((linear_merge_kernel<T>), dim3((unsigned)(groups < 2048 ? groups : 2048)), dim3(256), 0, stream, a);
+  return (int)hipGetLastError();
+}
+
+int launch_merge_type(const LinArgs& a, int dtype, hipStream_t stream) {
+  return dtype == 0 ? launch_merge<float>(a, stream) : dtype == 1 ? launch_merge<_Float16>(a, stream) : launch_merge<__bf16>(a, stream);
+}
+
+// Wavefronts and units in flight of each by the tile's size in blocks of 16: eight with a ring of as many units as their registers
+// hold; on the largest tile four, which have twice the registers (eight measure the same, and spill).
+template <int R>
+struct Shape {
+  static constexpr int W = R == 4 ? 4 : 8, P = 4 / R;
+};
+
+template <typename TR, bool XT, bool WT, int R>
+__global__ __launch_bounds__(64 * Shape<R>::W, Shape<R>::W / 4) void linear_stream_kernel(LinArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  stream_tile<TR, XT, WT, R, R, Shape<R>::W, Shape<R>::P, XT && WT>(a, smem, blockIdx.x, blockIdx.y);  // row sums: a weight's gradient
+}
+
+// Both products of a linear layer's backward in one launch, the first `split` workgroups those of the weight's gradient
+// (grad^T . x, with grad's column sums: the bias's gradient), the others those of the input's (grad . w).
+template <typename TR, int RW, int RI>
+__global__ __launch_bounds__(64 * Shape<RW>::W, Shape<RW>::W / 4) void linear_stream_pair_kernel(LinArgs gw, LinArgs gi, int split) {
+  static_assert(Shape<RW>::W == Shape<RI>::W, "one workgroup size");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  if ((int)blockIdx.x < split) stream_tile<TR, true, true, RW, RW, Shape<RW>::W, Shape<RW>::P, true>(gw, smem, blockIdx.x, 0);
+  else stream_tile<TR, false, true, RI, RI, Shape<RI>::W, Shape<RI>::P, false>(gi, smem, blockIdx.x - split, 0);
+}
+
+template <int R>
+long long blocks_of(const LinArgs& a) {
+  const long long tiles = ((a.M + 16 * R - 1) / (16 * R)) * ((a.N + 16 * R - 1) / (16 * R));
+  return (tiles + 7) / 8 * 8 * a.splits;
+}
+
+template <typename TR, bool XT, bool WT, int R>
+int launch_kernel(const LinArgs& a, hipStream_t stream, unsigned entries) {
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  constexpr int lds = StreamLds<TR, XT, WT, MB, NB, W>::BYTES;
-  const hipError_t granted = grant_dynamic_lds((const void*)linear_stream_kernel<TR, XT, WT, MB, NB, W, P>, lds, state, done);
+  constexpr int lds = StreamLds<TR, XT, WT, R, R, Shape<R>::W>::BYTES + (XT && WT ? Shape<R>::W * 16 * R * 4 : 0);
+  const hipError_t granted = grant_dynamic_lds((const void*)linear_stream_kernel<TR, XT, WT, R>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long tiles = ((a.M + 16 * MB - 1) / (16 * MB)) * ((a.N + 16 * NB - 1) / (16 * NB));
-  if (tiles > 0x3fffffffLL) return -3;  // TTSDPA_ERR_SHAPE
-  hipLaunchKernelGGL((linear_stream_kernel<TR, XT, WT, MB, NB, W, P>), dim3((unsigned)((tiles + 7) / 8 * 8), entries), dim3(64 * W), lds, stream, a);
+  if (blocks_of<R>(a) > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
+  hipLaunchKernelGGL((linear_stream_kernel<TR, XT, WT, R>), dim3((unsigned)blocks_of<R>(a), entries), dim3(64 * Shape<R>::W), lds, stream, a);
+  return (int)hipGetLastError();
+}
+
+template <typename TR, int RW, int RI>
+int launch_pair_kernel(const LinArgs& gw, const LinArgs& gi, hipStream_t stream) {
+  static hipError_t state[kMaxDevices];
+  static bool done[kMaxDevices];
+  constexpr int W = Shape<RW>::W;
+  constexpr int lds_w = StreamLds<TR, true, true, RW, RW, W>::BYTES + W * 16 * RW * 4, lds_i = StreamLds<TR, false, true, RI, RI, W>::BYTES;
+  constexpr int lds = lds_w > lds_i ? lds_w : lds_i;
+  const hipError_t granted = grant_dynamic_lds((const void*)linear_stream_pair_kernel<TR, RW, RI>, lds, state, done);
+  if (granted != hipSuccess) return (int)granted;
+  const long long split = blocks_of<RW>(gw), all = split + blocks_of<RI>(gi);
+  if (all > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
+  hipLaunchKernelGGL((linear_stream_pair_kernel<TR, RW, RI>), dim3((unsigned)all), dim3(64 * W), lds, stream, gw, gi, (int)split);
   return (int)hipGetLastError();
 }
 
@@ -319,42 +443,53 @@ int launch_variant(const LinArgs& a, hipStream_t stream, unsigned entries) {
 
 namespace {
 
-// Microseconds of a product on tiles of 16*R rows of x by 16*R of w, from measurements (MI355X, 16-bit unless said):
-// 3 us of launch, latency and the meeting of the partial sums (2 more on the largest tile: a wavefront's sums are 16 KB);
-// then, for each round of the 256 CUs, half a microsecond and the operands of a tile at the 65 GB/s that a CU takes in
-// (it measured 60-75 over all shapes), or the tile's products where those take longer (fp32: 0.45 TFLOP/s of a CU's 0.61 on
-// the largest tile, 0.3 on the others).
+// Microseconds of a product on tiles of 16*R rows of x by 16*R of w, its contraction divided among S workgroups per tile, from
+// measurements (MI355X, 16-bit unless said): 3 us of launch, latency and the meeting of the partial sums (2 more on the
+// largest tile: a wavefront's sums are 16 KB); then, for each round of the 256 CUs, half a microsecond and the operands of
+// a tile at the 65 GB/s that a CU takes in (it measured 60-75 over all shapes; 16-bit k-major operands come in pieces of
+// 32*R bytes, which costs 2.6, 1.6 and 1.1 times that), or the tile's products where those take longer (fp32: 0.45 TFLOP/s
+// of a CU's 0.61 on the largest tile, 0.3 on the others).  With S > 1 another launch and the partial products written and
+// read.
 //   measured / this: 1000^3 on 16, 32, 64: 25 / 26, 12 / 13, 9.5 / 9.4; 24 x 2048 x 5632: 7.4 / 9, 10.5 / 13, 19 / 21;
-//   64 x 4096 x 4096: 17 / 20, 11 / 12, 21 / 22; fp32 1000^3: 42 / 43, 30 / 32, 25 / 24
-double stream_us(const LinArgs& a, int esz, int R, unsigned entries) {
+//   64 x 4096 x 4096: 17 / 20, 11 / 12, 21 / 22; fp32 1000^3: 42 / 43, 30 / 32, 25 / 24; both k-major, 500 x 500 x 8192:
+//   88 / 90, 29 / 29, 40 / 40
+double stream_us(const LinArgs& a, int esz, int R, int S, double entries) {
   const double tm = 16 * R, tn = 16 * R;
-  const double tiles = (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)) * entries;
+  const double tiles = (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)) * entries * S;
   const double rounds = tiles > 256 ? tiles / 256 : 1;
-  const double bytes = ((a.M < tm ? a.M : tm) + (a.N < tn ? a.N : tn)) * (double)a.K * esz;
-  const double flops = 2 * tm * tn * (double)a.K;
-  const double rate = esz == 2 ? 4e6 : R == 4 ? 0.45e6 : 0.3e6;
+  const double narrow = esz == 4 ? 1 : R == 1 ? 2.6 : R == 2 ? 1.6 : 1.1;
+  const double k = (double)a.K / S;
+  const double bytes = ((a.M < tm ? a.M : tm) * (a.xt ? narrow : 1) + (a.N < tn ? a.N : tn) * (a.wt ? narrow : 1)) * k * esz;
+  const double rate = esz == 2 ? 4e6 : R == 4 ? 0.45e6 : 0.3e6, flops = 2 * tm * tn * k;
   const double per = bytes / 65e3 > flops / rate ? bytes / 65e3 : flops / rate;
-  return (R == 4 ? 5 : 3) + rounds * (0.5 + per);
+  return (R == 4 ? 5 : 3) + rounds * (0.5 + per) + (S > 1 ? 3 + S * 8.0 * a.M * a.N / 4e6 : 0);
 }
 
-// Rows of a tile in blocks of 16: the cheapest of 1, 2 and 4 that a k-major operand has the rows for.
-int stream_rows(const LinArgs& a, int esz, unsigned entries, double* us) {
-  int best = 0;
-  for (int R = 1; R <= 4; R *= 2) {
+// The cheapest tile (rows in blocks of 16: 1, 2 or 4, as far as a k-major operand has them; R = 0: none) and, when the caller
+// has scratch for partial products, division of the contraction (no less than 512 of it per workgroup).
+struct StreamPlan {
+  int R, S;
+  double us;
+};
+StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split, int least = 1, int most = 4) {
+  StreamPlan best{0, 1, 0};
+  for (int R = least; R <= most; R *= 2) {
     if ((a.xt && a.M < 16 * R) || (a.wt && a.N < 16 * R)) break;
-    const double t = stream_us(a, esz, R, entries);
-    if (!best || t < *us) best = R, *us = t;
+    for (int S = 1; S <= 32 && (S == 1 || (may_split && a.K >= 512 * S)); S *= 2) {
+      const double t = stream_us(a, esz, R, S, entries);
+      if (!best.R || t < best.us) best = {R, S, t};
+    }
   }
   return best;
 }
 
+size_t part_bytes(const LinArgs& a, int S) { return S > 1 ? (size_t)S * (size_t)(a.M * a.N + a.M) * sizeof(float) : 0; }
+
 template <typename TR, bool XT, bool WT>
 int launch_rows(const LinArgs& a, int R, hipStream_t stream, unsigned entries) {
-  // eight wavefronts with a ring of as many units as their registers hold; on the largest tile four, which have twice the
-  // registers (eight measure the same with the bytes in flight that theirs allow, and spill)
-  if (R == 1) return launch_variant<TR, XT, WT, 1, 1, 8, 4>(a, stream, entries);
-  if (R == 2) return launch_variant<TR, XT, WT, 2, 2, 8, 2>(a, stream, entries);
-  return launch_variant<TR, XT, WT, 4, 4, 4, 1>(a, stream, entries);
+  if (R == 1) return launch_kernel<TR, XT, WT, 1>(a, stream, entries);
+  if (R == 2) return launch_kernel<TR, XT, WT, 2>(a, stream, entries);
+  return launch_kernel<TR, XT, WT, 4>(a, stream, entries);
 }
 
 template <typename TR>
@@ -363,30 +498,73 @@ int launch_type(const LinArgs& a, int R, hipStream_t stream, unsigned entries) {
   return a.wt ? launch_rows<TR, false, true>(a, R, stream, entries) : launch_rows<TR, false, false>(a, R, stream, entries);
 }
 
+template <typename TR>
+int launch_pair_type(const LinArgs& gw, const LinArgs& gi, int RW, int RI, hipStream_t stream) {
+  if (RW == 4) return launch_pair_kernel<TR, 4, 4>(gw, gi, stream);
+  if (RW == 2) return RI == 2 ? launch_pair_kernel<TR, 2, 2>(gw, gi, stream) : launch_pair_kernel<TR, 2, 1>(gw, gi, stream);
+  return RI == 2 ? launch_pair_kernel<TR, 1, 2>(gw, gi, stream) : launch_pair_kernel<TR, 1, 1>(gw, gi, stream);
+}
+
+// Tiles of the two products of a layer's backward: one workgroup size, so both of 64 rows or both of fewer.
+struct PairPlan {
+  StreamPlan gw, gi;
+};
+PairPlan plan_pair(const LinArgs& gw, const LinArgs& gi, int esz) {
+  const PairPlan few{plan_stream(gw, esz, 1, true, 1, 2), plan_stream(gi, esz, 1, false, 1, 2)};
+  const PairPlan many{plan_stream(gw, esz, 1, true, 4, 4), plan_stream(gi, esz, 1, false, 4, 4)};
+  return many.gw.R && many.gi.R && many.gw.us + many.gi.us < few.gw.us + few.gi.us ? many : few;
+}
+
 }  // namespace
 
 bool stream_takes(const LinArgs& a, int dtype) {
   // a tile's rows and a unit's k-rows are addressed with 32-bit byte offsets
   const long long ld_max = 1ll << 24;
   if (a.K < 1 || a.K > 0x3fffffffLL || a.ldx >= ld_max || a.ldw >= ld_max) return false;
-  double us;
-  return stream_rows(a, dtype == 0 ? 4 : 2, 1, &us) > 0;
+  return plan_stream(a, dtype == 0 ? 4 : 2, 1, false).R > 0;
 }
 
-double stream_cost(const LinArgs& a, int dtype, unsigned entries) {
-  double us = 0;
-  stream_rows(a, dtype == 0 ? 4 : 2, entries, &us);
-  return us;
+double stream_cost(const LinArgs& a, int dtype, unsigned entries, bool may_split) {
+  return plan_stream(a, dtype == 0 ? 4 : 2, entries, may_split).us;
 }
 
-int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, unsigned entries) {
-  double us;
-  const int R = stream_rows(a, dtype == 0 ? 4 : 2, entries, &us);
+size_t stream_scratch(const LinArgs& a, int dtype) { return part_bytes(a, plan_stream(a, dtype == 0 ? 4 : 2, 1, true).S); }
+
+int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, unsigned entries, void* scratch, size_t scratch_bytes) {
+  const int esz = dtype == 0 ? 4 : 2;
+  LinArgs a = args;
+  StreamPlan p = plan_stream(a, esz, entries, entries == 1 && scratch);
+  if (part_bytes(a, p.S) > scratch_bytes) p = plan_stream(a, esz, entries, false);
+  a.splits = p.S;
+  a.part = p.S > 1 ? (float*)scratch : nullptr;
+  int rc;
   switch (dtype) {
-    case 0: return launch_type<F32>(a, R, stream, entries);
-    case 1: return launch_type<F16>(a, R, stream, entries);
-    default: return launch_type<BF16>(a, R, stream, entries);
+    case 0: rc = launch_type<F32>(a, p.R, stream, entries); break;
+    case 1: rc = launch_type<F16>(a, p.R, stream, entries); break;
+    default: rc = launch_type<BF16>(a, p.R, stream, entries);
   }
+  return rc != 0 || p.S == 1 ? rc : launch_merge_type(a, dtype, stream);
+}
+
+double stream_pair_cost(const LinArgs& gw, const LinArgs& gi, int dtype) {
+  const PairPlan p = plan_pair(gw, gi, dtype == 0 ? 4 : 2);
+  return p.gw.us + p.gi.us - 3;  // one launch
+}
+
+size_t stream_pair_scratch(const LinArgs& gw, const LinArgs& gi, int dtype) { return part_bytes(gw, plan_pair(gw, gi, dtype == 0 ? 4 : 2).gw.S); }
+
+int launch_stream_pair(const LinArgs& gw_, const LinArgs& gi, int dtype, hipStream_t stream, void* scratch) {
+  const PairPlan p = plan_pair(gw_, gi, dtype == 0 ? 4 : 2);
+  LinArgs gw = gw_;
+  gw.splits = p.gw.S;
+  gw.part = p.gw.S > 1 ? (float*)scratch : nullptr;
+  int rc;
+  switch (dtype) {
+    case 0: rc = launch_pair_type<F32>(gw, gi, p.gw.R, p.gi.R, stream); break;
+    case 1: rc = launch_pair_type<F16>(gw, gi, p.gw.R, p.gi.R, stream); break;
+    default: rc = launch_pair_type<BF16>(gw, gi, p.gw.R, p.gi.R, stream);
+  }
+  return rc != 0 || p.gw.S == 1 ? rc : launch_merge_type(gw, dtype, stream);
 }
 
 }  // namespace ttsdpa

@@ -18,6 +18,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
+#include <initializer_list>
 
 #include "../../include/ttfused.h"
 #include "../../include/ttlinear.h"
@@ -80,6 +81,22 @@ PyObject* guarded(F&& f) {
   HANDLE_TH_ERRORS
   return f();
   END_HANDLE_TH_ERRORS
+}
+
+// A tuple of tensors, None for a nullptr.
+PyObject* tuple_of(std::initializer_list<const Tensor*> tensors) {
+  PyObject* all = PyTuple_New((Py_ssize_t)tensors.size());
+  if (!all) return nullptr;
+  Py_ssize_t i = 0;
+  for (const Tensor* t : tensors) {
+    PyObject* o = t ? THPVariable_Wrap(*t) : none();
+    if (!o) {
+      Py_DECREF(all);
+      return nullptr;
+    }
+    PyTuple_SET_ITEM(all, i++, o);
+  }
+  return all;
 }
 
 // ---- attention -------------------------------------------------------------------------------------------------------
@@ -220,18 +237,7 @@ PyObject* sdp_attention_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const size_t bytes = ttsdpa_backward_workspace_bytes(&bp);
     const Scratch ws(bytes, *q);
     if (ttsdpa_backward(&bp, ws.ptr, bytes, stream_of(*q)) != TTSDPA_OK) return none();
-    PyObject* grads = PyTuple_New(3);
-    if (!grads) return nullptr;
-    const Tensor* all[3] = {&gq, &gk, &gv};
-    for (int i = 0; i < 3; i++) {
-      PyObject* w = THPVariable_Wrap(*all[i]);
-      if (!w) {
-        Py_DECREF(grads);
-        return nullptr;
-      }
-      PyTuple_SET_ITEM(grads, i, w);
-    }
-    return grads;
+    return tuple_of({&gq, &gk, &gv});
   });
 }
 
@@ -420,8 +426,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::DimVector shape(x->sizes());
     shape.back() = N;
     const Tensor out = empty_like_shape(shape, *x);
-    if (ttlinear_forward(dt, x->data_ptr(), w->data_ptr(), b ? b->data_ptr() : nullptr, out.data_ptr(), M, N, K, ldx, ld_of(*w), N,
-                         stream_of(*x)) != TTSDPA_OK)
+    const size_t bytes = ttlinear_matmul_workspace_bytes(dt, M, N, K, 0, 1);
+    const Scratch ws(bytes, *x);
+    if (ttlinear_matmul(dt, x->data_ptr(), w->data_ptr(), b ? b->data_ptr() : nullptr, out.data_ptr(), M, N, K, 0, 1, ldx, ld_of(*w), N,
+                        ws.ptr, bytes, stream_of(*x)) != TTSDPA_OK)
       return none();
     return THPVariable_Wrap(out);
   });
@@ -453,11 +461,45 @@ PyObject* matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// (gradOut, input, weight, needBias) -> (gradInput, gradWeight, gradBias or None)
+PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  const Tensor *g, *x, *w;
+  if (n != 4 || !(g = tensor(a[0])) || !(x = tensor(a[1])) || !(w = tensor(a[2]))) return none();
+  const int need_bias = PyObject_IsTrue(a[3]);
+  if (need_bias < 0) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const int dt = dtype_of(*x);
+    if (dt < 0 || !on_current_gpu(*x) || !same_kind(*g, *x) || !same_kind(*w, *x) || !rows_ok(*w)) return none();
+    const int64_t N = w->size(0), K = w->size(1);
+    // rows: matrices as they lie, leading dimensions only where dense
+    auto rows = [](const Tensor& t, int64_t cols, int64_t* count, int64_t* ld) {
+      if (t.dim() < 1 || t.size(-1) != cols || cols < 1) return false;
+      *count = t.numel() / cols;
+      *ld = t.dim() == 2 && rows_ok(t) ? ld_of(t) : cols;
+      return (t.dim() == 2 && rows_ok(t)) || t.is_contiguous();
+    };
+    int64_t M, Mx, ldg, ldx;
+    if (!rows(*g, N, &M, &ldg) || !rows(*x, K, &Mx, &ldx) || M != Mx || M < 1) return none();
+    const Tensor gi = empty_like_shape(x->sizes(), *x), gw = empty_like_shape(w->sizes(), *w);
+    Tensor gb;
+    if (need_bias) {
+      const int64_t shape[1] = {N};
+      gb = empty_like_shape(shape, *x);
+    }
+    const size_t bytes = ttlinear_backward_workspace_bytes(dt, M, N, K);
+    const Scratch ws(bytes, *x);
+    if (ttlinear_backward(dt, g->data_ptr(), x->data_ptr(), w->data_ptr(), gi.data_ptr(), gw.data_ptr(), need_bias ? gb.data_ptr() : nullptr,
+                          M, N, K, ldg, ldx, ld_of(*w), ws.ptr, bytes, stream_of(*x)) != TTSDPA_OK)
+      return none();
+    return tuple_of({&gi, &gw, need_bias ? &gb : nullptr});
+  });
+}
+
 PyMethodDef methods[] = {
 #define TT_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
     TT_METHOD(sdp_attention), TT_METHOD(sdp_attention_backward), TT_METHOD(kv_cache_append), TT_METHOD(rms_norm),
     TT_METHOD(fused_add_rms_norm), TT_METHOD(silu_mul), TT_METHOD(softmax), TT_METHOD(softmax_backward), TT_METHOD(linear),
-    TT_METHOD(matmul), {nullptr, nullptr, 0, nullptr}};
+    TT_METHOD(matmul), TT_METHOD(linear_backward), {nullptr, nullptr, 0, nullptr}};
 #undef TT_METHOD
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Checked calls into libttsdpa.so for torch tensors.", -1, methods,

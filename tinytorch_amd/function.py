@@ -486,6 +486,9 @@ def matmul(a, b, transA=False, transB=False, bias=None):
 def linearBackward(gradOut, input, weight, needBias=True):
     """(gradInput, gradWeight, gradBias) of linear(input, weight, bias) — FuncLinear::backward (reference
     src/Function/FuncNNLayer.h:20-33): grad . weight, grad^T . input, and the column sums of grad."""
+    grads = _native.linear_backward(gradOut, input, weight, needBias)
+    if grads is not None:
+        return grads
     N, K = weight.shape
     g = gradOut.reshape(-1, N)
     x = input.reshape(-1, K)
