@@ -1,5 +1,4 @@
-// Split-KV attention for decode: a few query rows per KV head against a long, contiguous KV cache (fp16 / bf16,
-// head_dim 128 or 64).  Memory-bound: every K and V byte is read exactly once with 16-byte loads, whatever the number of
+// Split-KV attention for decode: a few query rows per KV head against a long, contiguous KV cache (head_dim 128 or 64).  Memory-bound: every K and V byte is read exactly once with 16-byte loads, whatever the number of
 // query heads sharing the KV head, instead of the reference's GEMM -> scale -> softmax -> GEMM chain over a
 // materialised score tensor (reference src/Function/FuncNNLayer.h:237-265).
 //
@@ -10,10 +9,10 @@
 // Per 32-key block and wavefront:
 //   scores  v_mfma_f32_16x16x32: A = the query rows (16 x 32 slice of head_dim, zero rows where unused), B = K^T taken
 //           straight from global memory: lane l supplies key l%16 and the 8 head_dim elements of group l/16, i.e. one
-//           16-byte load; head_dim/32 MFMAs cover the head.  Query row x sits at MFMA row 4*(x%4) + x/4, so the
+//           16-byte load; head_dim/32 MFMAs cover the head (fp32: 4 elements per load, four v_mfma_f32_16x16x4 each).  Query row x sits at MFMA row 4*(x%4) + x/4, so the
 //           result lane (key l%16, group l/16) holds rows l/16, l/16+4, ... in registers 0, 1, ...
 //   softmax running max per row (reduced over the 16 key lanes with DPP row rotations), exp2 with scale*log2e folded
-//   P.V     on the vector ALUs: with C = head_dim/8 chunks per row, lane l owns head_dim elements 8*(l%C) .. +7 of keys
+//   P.V     on the vector ALUs: with C 16-byte chunks per row, lane l owns the elements of chunk l%C of keys
 //           l/C, l/C + 64/C, ... (one 16-byte load per key, a wavefront load instruction covers 64/C whole V rows =
 //           1 KiB contiguous); the probabilities
 //           travel from the score lanes to the value lanes through a per-wavefront LDS patch.
@@ -28,6 +27,35 @@ namespace {
 
 constexpr int KB = 32;       // keys per wavefront block
 constexpr int NWAVE = 4;
+
+// What the kernel needs to know about the element type: 16 bytes of it as an MFMA operand, and as floats.
+template <typename TR>
+struct Dec {
+  typedef typename TR::elem elem;
+  typedef typename TR::vec8 chunk;
+  static __device__ __forceinline__ f32x4 mma(chunk q, chunk k, f32x4 c) { return TR::mfma16(q, k, c); }
+  static __device__ __forceinline__ void floats(u32x4 v, float (&f)[8]) {
+#pragma unroll
+    for (int w = 0; w < 4; w++) f[2 * w] = TR::lo(v[w]), f[2 * w + 1] = TR::hi(v[w]);
+  }
+};
+struct F32 {};
+template <>
+struct Dec<F32> {
+  typedef float elem;
+  typedef f32x4 chunk;
+  // four v_mfma_f32_16x16x4, instruction e contracting the lanes' e-th elements: the same head_dim elements on both sides
+  static __device__ __forceinline__ f32x4 mma(chunk q, chunk k, f32x4 c) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(q[e], k[e], c, 0, 0, 0);
+    return c;
+  }
+  static __device__ __forceinline__ void floats(u32x4 v, float (&f)[4]) {
+    const f32x4 x = __builtin_bit_cast(f32x4, v);
+#pragma unroll
+    for (int w = 0; w < 4; w++) f[w] = x[w];
+  }
+};
 
 // max over the 16 lanes of a DPP row (lanes 16*i .. 16*i+15), result in every lane of the row
 __device__ __forceinline__ float row16_max(float x) {
@@ -60,11 +88,12 @@ __device__ __forceinline__ void wave_lds_sync() {
 // unconditional); the split records keep the pitch DD + 2.
 template <typename TR, int R, int DD, bool PAGED, bool PAD>
 __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int chunk, float* __restrict__ ws) {
-  typedef typename TR::elem T;
-  typedef typename TR::vec8 vec8;
-  constexpr int NR = 4 * R;    // row slots
-  constexpr int KS = DD / 32;  // MFMAs along head_dim per 16 keys
-  constexpr int CH = DD / 8;   // 16-byte chunks of a V row = value lanes per key
+  typedef typename Dec<TR>::elem T;
+  typedef typename Dec<TR>::chunk chunk_t;
+  constexpr int E = 16 / sizeof(T);  // elements of a 16-byte chunk
+  constexpr int NR = 4 * R;          // row slots
+  constexpr int KS = DD / (4 * E);   // chunks of a key per score lane
+  constexpr int CH = DD / E;         // 16-byte chunks of a V row = value lanes per key
   constexpr int PH = 64 / CH;  // keys a wavefront V load covers (key phases)
 
   // per-wavefront patch: probabilities [KB keys][NR rows] + rescale factors [NR]; reused for the final merge
@@ -94,20 +123,20 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
   const T* kp = (const T*)a.k + b * a.ks[0] + hk * a.ks[1];
   const T* vp = (const T*)a.v + b * a.vs[0] + hk * a.vs[1];
 
-  // ---- query rows as MFMA A operands: lane l supplies MFMA row l%16, head_dim 32*ks + 8*(l/16) .. +7 --------------
-  vec8 qa[KS];
+  // ---- query rows as MFMA A operands: lane l supplies MFMA row l%16, head_dim 4*E*ks + E*(l/16) .. +E-1 -----------
+  chunk_t qa[KS];
   {
     int mrow = l16;                       // MFMA row
     int x = (mrow & 3) * 4 + (mrow >> 2); // query row stored there: row x sits at 4*(x%4) + x/4
     bool used = (mrow & 3) < R && x < rows;
     int xl = used ? x / a.G : 0, xg = used ? x % a.G : 0;
-    const T* qr = (const T*)a.q + b * a.qs[0] + (hk * a.G + xg) * a.qs[1] + xl * a.qs[2] + 8 * lg;
+    const T* qr = (const T*)a.q + b * a.qs[0] + (hk * a.G + xg) * a.qs[1] + xl * a.qs[2] + E * lg;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      const bool there = used && (!PAD || 32 * ks + 8 * lg < a.D);
-      vec8 t = *(const vec8*)(there ? qr + 32 * ks : qr - 8 * lg);
+      const bool there = used && (!PAD || 4 * E * ks + E * lg < a.D);
+      const chunk_t t = *(const chunk_t*)(there ? qr + 4 * E * ks : qr - E * lg);
 #pragma unroll
-      for (int i = 0; i < 8; i++) qa[ks][i] = there ? t[i] : (T)0.f;
+      for (int i = 0; i < E; i++) qa[ks][i] = there ? t[i] : (T)0.f;
     }
   }
 
@@ -115,11 +144,11 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
   float m_run[R], l_run[R];
 #pragma unroll
   for (int r = 0; r < R; r++) m_run[r] = -1e30f, l_run[r] = 0.f;
-  float acc[NR][8];
+  float acc[NR][E];
 #pragma unroll
   for (int x = 0; x < NR; x++)
 #pragma unroll
-    for (int i = 0; i < 8; i++) acc[x][i] = 0.f;
+    for (int i = 0; i < E; i++) acc[x][i] = 0.f;
   const float c = a.scale * kLog2e;
 
   const int s_begin = split * chunk;
@@ -160,14 +189,14 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
     for (int gi = 0; gi < 2; gi++) {
       int key = k0 + 16 * gi + l16;
       key = (key < S ? key : S - 1) - key0;
-      const T* kr = kpb + key * a.ks[2] + 8 * lg;
+      const T* kr = kpb + key * a.ks[2] + E * lg;
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) {
         if (!PAD) {
-          kreg[gi][ks] = __builtin_nontemporal_load((const u32x4*)(kr + 32 * ks));  // read once: keep it out of the caches
+          kreg[gi][ks] = __builtin_nontemporal_load((const u32x4*)(kr + 4 * E * ks));  // read once: keep it out of the caches
         } else {
-          const bool there = 32 * ks + 8 * lg < a.D;
-          const u32x4 t = __builtin_nontemporal_load((const u32x4*)(there ? kr + 32 * ks : kr - 8 * lg));
+          const bool there = 4 * E * ks + E * lg < a.D;
+          const u32x4 t = __builtin_nontemporal_load((const u32x4*)(there ? kr + 4 * E * ks : kr - E * lg));
           kreg[gi][ks] = there ? t : u32x4{0u, 0u, 0u, 0u};
         }
       }
@@ -177,7 +206,7 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
     for (int i = 0; i < KB / PH; i++) {
       int key = k0 + PH * i + vph;
       key = (key < S ? key : S - 1) - key0;
-      vreg[i] = __builtin_nontemporal_load((const u32x4*)(vpb + key * a.vs[2] + (PAD && 8 * vc >= a.D ? 0 : 8 * vc)));
+      vreg[i] = __builtin_nontemporal_load((const u32x4*)(vpb + key * a.vs[2] + (PAD && E * vc >= a.D ? 0 : E * vc)));
     }
 
     // ---- scores --------------------------------------------------------------------------------------------------------
@@ -187,7 +216,7 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
       sc[gi] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KS; ks++)
-        sc[gi] = TR::mfma16(qa[ks], __builtin_bit_cast(vec8, kreg[gi][ks]), sc[gi]);
+        sc[gi] = Dec<TR>::mma(qa[ks], __builtin_bit_cast(chunk_t, kreg[gi][ks]), sc[gi]);
       if (k0 + 16 * gi + l16 >= klim_min) {
 #pragma unroll
         for (int r = 0; r < 4; r++)
@@ -219,46 +248,41 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
 #pragma unroll
       for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int i = 0; i < 8; i++) acc[4 * r + j][i] *= al[j];
+        for (int i = 0; i < E; i++) acc[4 * r + j][i] *= al[j];
     }
 #pragma unroll
     for (int i = 0; i < KB / PH; i++) {
-      float vf[8];
-#pragma unroll
-      for (int w = 0; w < 4; w++) {
-        vf[2 * w] = TR::lo(vreg[i][w]);
-        vf[2 * w + 1] = TR::hi(vreg[i][w]);
-      }
+      float vf[E];
+      Dec<TR>::floats(vreg[i], vf);
 #pragma unroll
       for (int r = 0; r < R; r++) {
         f32x4 p = *(const f32x4*)(pl + (PH * i + vph) * NR + 4 * r);
 #pragma unroll
         for (int j = 0; j < 4; j++)
 #pragma unroll
-          for (int e = 0; e < 8; e++) acc[4 * r + j][e] = fmaf(p[j], vf[e], acc[4 * r + j][e]);
+          for (int e = 0; e < E; e++) acc[4 * r + j][e] = fmaf(p[j], vf[e], acc[4 * r + j][e]);
       }
     }
     wave_lds_sync();
   }
 
-  // ---- wavefront totals: sums over the 16 key lanes; accumulators over the 4 key phases ------------------------------------
+  // ---- wavefront totals: sums over the 16 key lanes; accumulators over the key phases ------------------------------------
 #pragma unroll
   for (int r = 0; r < R; r++) l_run[r] = row16_sum(l_run[r]);
 #pragma unroll
   for (int x = 0; x < NR; x++)
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < E; i++) {
       float t = acc[x][i];
-      if (CH <= 8) t += __shfl_xor(t, 8);
-      t += __shfl_xor(t, 16);
-      t += __shfl_xor(t, 32);
+#pragma unroll
+      for (int off = CH; off < 64; off *= 2) t += __shfl_xor(t, off);
       acc[x][i] = t;
     }
   if (vph == 0) {
 #pragma unroll
     for (int x = 0; x < NR; x++)
 #pragma unroll
-      for (int i = 0; i < 8; i++) Om[wave][x][8 * vc + i] = acc[x][i];
+      for (int i = 0; i < E; i++) Om[wave][x][E * vc + i] = acc[x][i];
   }
   if (l16 == 0) {
 #pragma unroll
@@ -338,7 +362,7 @@ __global__ __launch_bounds__(DD) void merge_kernel(KArgs a, int splits, const fl
 
 template <typename TR, int DD, bool PAD>
 int launch_decode_t(const KArgs& a, const DecodePlan& pl, float* ws, hipStream_t stream) {
-  typedef typename TR::elem T;
+  typedef typename Dec<TR>::elem T;
   dim3 grid((unsigned)((long long)a.B * a.Hkv * pl.splits)), block(256);
   int R = (pl.rows + 3) / 4;
 #define TT_DECODE(R_)                                                                                                      \
@@ -368,8 +392,17 @@ DecodePlan plan_decode(const KArgs& a) {
   long long pairs = (long long)a.B * a.Hkv;
   int max_splits = (a.S + 2 * round - 1) / (2 * round);
   if (max_splits < 1) max_splits = 1;
-  long long want = (2 * 256 + pairs - 1) / pairs;  // aim for >= 2 workgroups per CU
-  int splits = (int)(want < 1 ? 1 : want);
+  // Two workgroups per CU or a few more: the count, up to four per CU, that fills its last round best (a CU takes in its
+  // workgroups' keys at a rate of its own, so 2.25 per CU cost as much as 3: 24 sequences of 3000 keys on 4 KV heads, 96
+  // pairs, 37.7 us in 6 splits of the keys and 31 in 8), the smaller of two that are equally good.
+  int splits = 1;
+  double best = 0;
+  for (long long s = (500 + pairs - 1) / pairs; s == 1 || s * pairs <= 4 * 256; s++) {
+    const long long wgs = s * pairs, rounds = (wgs + 255) / 256;
+    const double fill = (double)wgs / (double)(rounds * 256) - 0.01 * rounds;
+    if (s > 1 && fill <= best) continue;
+    best = fill, splits = (int)s;
+  }
   if (splits > max_splits) splits = max_splits;
   if (splits > kMaxSplits) splits = kMaxSplits;
   int chunk = (a.S + splits - 1) / splits;
@@ -398,21 +431,28 @@ int launch_merge(const KArgs& a, int dtype, int splits, const float* ws, hipStre
   return (int)hipGetLastError();
 }
 
+namespace {
+
+// head_dim 64 and 128; any other whole number of 16-byte chunks up to 128: the kernel of the next size up, the missing
+// columns as zeros
+template <typename TR>
+int launch_decode_d(const KArgs& a, const DecodePlan& pl, float* ws, hipStream_t stream) {
+  constexpr int E = 16 / (int)sizeof(typename Dec<TR>::elem);
+  if (a.D % E != 0 || a.D < E || a.D > 128) return (int)hipErrorInvalidValue;  // (the callers keep to this)
+  if (a.D == 64) return launch_decode_t<TR, 64, false>(a, pl, ws, stream);
+  if (a.D == 128) return launch_decode_t<TR, 128, false>(a, pl, ws, stream);
+  return a.D < 64 ? launch_decode_t<TR, 64, true>(a, pl, ws, stream) : launch_decode_t<TR, 128, true>(a, pl, ws, stream);
+}
+
+}  // namespace
+
 int launch_decode(const KArgs& a, int dtype, void* workspace, hipStream_t stream) {
-  DecodePlan pl = plan_decode(a);
-  if (a.D == 64)
-    return dtype == 1 ? launch_decode_t<F16, 64, false>(a, pl, (float*)workspace, stream)
-                      : launch_decode_t<BF16, 64, false>(a, pl, (float*)workspace, stream);
-  if (a.D == 128)
-    return dtype == 1 ? launch_decode_t<F16, 128, false>(a, pl, (float*)workspace, stream)
-                      : launch_decode_t<BF16, 128, false>(a, pl, (float*)workspace, stream);
-  // any other multiple of 8 up to 128: the kernel of the next size up, the missing columns as zeros
-  if (a.D % 8 != 0 || a.D < 8 || a.D > 128) return (int)hipErrorInvalidValue;  // (the callers keep to this)
-  if (a.D < 64)
-    return dtype == 1 ? launch_decode_t<F16, 64, true>(a, pl, (float*)workspace, stream)
-                      : launch_decode_t<BF16, 64, true>(a, pl, (float*)workspace, stream);
-  return dtype == 1 ? launch_decode_t<F16, 128, true>(a, pl, (float*)workspace, stream)
-                    : launch_decode_t<BF16, 128, true>(a, pl, (float*)workspace, stream);
+  const DecodePlan pl = plan_decode(a);
+  switch (dtype) {
+    case 0: return launch_decode_d<F32>(a, pl, (float*)workspace, stream);
+    case 1: return launch_decode_d<F16>(a, pl, (float*)workspace, stream);
+    default: return launch_decode_d<BF16>(a, pl, (float*)workspace, stream);
+  }
 }
 
 }  // namespace ttsdpa

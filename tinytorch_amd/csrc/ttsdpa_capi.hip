@@ -246,6 +246,14 @@ bool decode_ok(const ttsdpa_params* p) {
   return (long long)p->L * (p->Hq / p->Hkv) <= kDecodeMaxRows;
 }
 
+// fp32 calls of the prefill route that the split-KV streaming kernel runs when it has its scratch: few query rows per KV head
+// (4 sequences of 1000 keys, 16 query heads on 4, head_dim 128, strided q: 145 us on the fp32 MFMA kernel's 128-row
+// tiles, which such a q keeps from sharing heads and splitting keys).
+bool f32_decode_ok(const ttsdpa_params* p) {
+  return f32_prefill_ok(p) && p->mask_kind == TTSDPA_MASK_NONE && effective_causal(p) != TTSDPA_CAUSAL_TOP_LEFT &&
+         (long long)p->L * (p->Hq / p->Hkv) <= kDecodeMaxRows;
+}
+
 int pick_route(const ttsdpa_params* p) {
   if (p->B == 0 || p->L == 0) return TTSDPA_ROUTE_NONE;
   if (p->S == 0) return TTSDPA_ROUTE_ZERO;
@@ -449,6 +457,10 @@ size_t ttsdpa_workspace_bytes(const ttsdpa_params* p) {
   // enough for ttsdpa_forward's route and for an explicit ttsdpa_decode of the same call
   size_t need = decode_ok(p) ? plan_decode(a).ws_bytes : 0;
   if (pick_route(p) == TTSDPA_ROUTE_PREFILL) {
+    if (f32_decode_ok(p)) {
+      const size_t decode = plan_decode(a).ws_bytes;
+      need = decode > need ? decode : need;
+    }
     if (pack_heads_ok(p)) pack_heads(&a);
     size_t split = plan_prefill_splits(p, a).ws_bytes;
     need = split > need ? split : need;
@@ -495,6 +507,12 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
     else
       a.kv_splits = 1, a.kv_chunk = 0, a.ws = nullptr;
     return launch_prefill_d64(a, p->dtype, (hipStream_t)stream);  // with splits: the kernel and the merge of its records
+  }
+  if (f32_decode_ok(p)) {
+    const DecodePlan pl = plan_decode(a);
+    if ((pl.ws_bytes == 0 || (workspace && workspace_bytes >= pl.ws_bytes && ptr_aligned(workspace, 16))) &&
+        check_grid((long long)a.B * a.Hkv * pl.splits) == TTSDPA_OK)
+      return launch_decode(a, p->dtype, workspace, (hipStream_t)stream);
   }
   auto launch = [&](const KArgs& k) {
     return p->dtype == TTSDPA_F32 ? launch_prefill_f32(k, (hipStream_t)stream) : launch_prefill(k, p->dtype, (hipStream_t)stream);
