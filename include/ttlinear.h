@@ -22,9 +22,10 @@ extern "C" {
 enum ttlinear_route {
   TTLINEAR_ROUTE_NONE = 0,   /* empty output */
   TTLINEAR_ROUTE_MFMA = 1,   /* K a multiple of 64 (fp16/bf16) or 32 (fp32), 16-byte aligned rows, N a multiple of 4:
-                                MFMA kernel, fp32 accumulation (fp32 tensors: full fp32 products) */
-  TTLINEAR_ROUTE_GENERAL = 2 /* everything else (other K, unaligned rows): the streaming MFMA kernel, which takes any alignment; the
-                                vector ALUs only for contraction-major operands of fewer than 16 rows and for empty contractions */
+                                a matrix-core kernel reads the operands as they lie, fp32 accumulation (fp32 tensors: full fp32 products) */
+  TTLINEAR_ROUTE_GENERAL = 2 /* everything else (other K, unaligned rows): the streaming MFMA kernel, which takes any alignment, or, given
+                                scratch (ttlinear_matmul), the tiled ones on copies in whole k-tiles where that is faster; the vector
+                                ALUs only for contraction-major operands of fewer than 16 rows and for empty contractions */
 };
 
 /* out[m, n] = bias[n] + sum_k x[m, k] * w[n, k]   (m < M, n < N, k < K)
@@ -46,13 +47,13 @@ int ttlinear_plan(int dtype, const void* x, const void* w, const void* bias, con
  * [N, K] with transB).  (false, true) is ttlinear_forward; FuncLinear::backward (reference
  * src/Function/FuncNNLayer.h:20-33) uses the other two that matter: (false, false) for the input gradient
  * dy[M, N] . w[N, K], and (true, false) for the weight gradient dy^T . x.  lda / ldb / ldo are row strides in elements.
- * fp16 / bf16 operands stored contraction-major are read in place by the matrix-core kernel (K a multiple of 64, N a
- * multiple of 4, 16-byte aligned operands with leading dimensions that are multiples of 8, a contraction-major operand's
- * row count a multiple of 8): no scratch is used then and workspace may be NULL.
- * workspace: ttlinear_matmul_workspace_bytes() bytes of device scratch, 256-byte aligned — for fp32 the MFMA route first
- * makes dense row-major copies of the operands that are stored contraction-major; with less (or NULL), or for shapes the
- * tiled kernels do not take, the general route reads the operands in place; and it lets products with few tiles divide their
- * contraction among workgroups ((false, true) included: what ttlinear_forward cannot do).  Same return codes as ttlinear_forward. */
+ * workspace: ttlinear_matmul_workspace_bytes() bytes of device scratch, 256-byte aligned (0 bytes: none is used).  Operands whose
+ * layout the tiled matrix-core kernels do not take (contraction-major, rows that are not whole k-tiles, unaligned rows) are
+ * copied there where product and copies together are faster than reading them in place, and products with few tiles divide
+ * their contraction among workgroups ((false, true) included: what ttlinear_forward cannot do).  With less (or NULL) the
+ * operands are read in place: 16-bit contraction-major ones by the tiled kernels (K a multiple of 64, N a multiple of 4,
+ * 16-byte aligned operands with leading dimensions that are multiples of 8, a contraction-major operand's row count a
+ * multiple of 8), others by the streaming kernel.  Same return codes as ttlinear_forward. */
 size_t ttlinear_matmul_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b);
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
                     int trans_a, int trans_b, int64_t lda, int64_t ldb, int64_t ldo, void* workspace,

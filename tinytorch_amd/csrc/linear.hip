@@ -4,7 +4,7 @@
 // linear_mfma_kernel (fp16 / bf16 on v_mfma_f32_32x32x16, fp32 on v_mfma_f32_32x32x2 with full fp32 products): a workgroup of 8 wavefronts owns a 256 x 256 tile of the output and walks K in
 // steps of 128 bytes (64 or 32 elements).  Both operands have K contiguous ("NT"), which is the layout v_mfma_f32_32x32x16 wants for both inputs:
 // a lane supplies 8 consecutive k of one row, so operand fragments are plain 16-byte LDS reads, no transposes.
-//   global -> LDS   global_load_lds_dwordx4, two stages of 64 KB (x tile 256 x 64, w tile 256 x 64); the 16-byte chunks
+//   global -> LDS   global_load_lds_dwordx4, two (or four) stages, of 64 KB for this tile (x tile 256 x 64, w tile 256 x 64); the 16-byte chunks
 //                   of a 128-byte LDS row are XOR-swizzled with half the row number so that the 32 rows a fragment read
 //                   touches spread over the banks; the loads for tile t+2 are requested while tile t's last k-step
 //                   runs, one barrier per tile
@@ -13,7 +13,7 @@
 //                   along its contiguous axis without a transpose
 //   accumulators    start from the bias (the reference writes the bias into C and accumulates onto it), fp32
 // Workgroups are numbered so that the 32 that run together on one XCD (workgroup i runs on XCD i % 8) form a 4 x 8
-// block of tiles: they share their x and w panels through that XCD's L2.
+// block of tiles: they share their x and w panels through that XCD's L2 (tile_of_block).
 //
 // linear_general_kernel: any element type and shape, fp32 arithmetic on the vector ALUs (64 x 64 tiles); what neither this
 // file's matrix-core kernels nor the streaming one (linear_stream.hip) take.
@@ -26,6 +26,8 @@ namespace ttsdpa {
 namespace {
 
 typedef __attribute__((address_space(3))) void lds_void_t;
+
+typedef uint32_t loose16 __attribute__((ext_vector_type(4), aligned(2)));  // 16 bytes at any element's address
 
 constexpr int ROWB = 128;  // bytes of an LDS row: 64 k of a 16-bit type, 32 k of fp32
 
@@ -41,6 +43,32 @@ struct Gemm {
   static __device__ __forceinline__ f32x16 mma(frag a, frag b, f32x16 c) { return TR::mfma32(a, b, c); }
   static __device__ __forceinline__ out4 cvt(f32x4 v) { return __builtin_convertvector(v, out4); }
 };
+// The tile of this workgroup.  Tiles are numbered down strips of four tile rows, column by column, and each XCD takes an
+// eighth of that sequence: every XCD has as many tiles, and any 32 in a row are a 4 x 8 block.  (Whole 4 x 8 blocks dealt to
+// the XCDs in turn gave one of them twice the work where there were nine: 1501 x 2501 x 1999 fp32, 240 tiles, 260 -> 156 us.)
+template <int TM, int TN>
+__device__ __forceinline__ bool tile_of_block(const LinArgs& a, int* tm, int* tn) {
+  const int tiles_m = (int)((a.M + TM - 1) / TM), tiles_n = (int)((a.N + TN - 1) / TN);
+  const int tiles = tiles_m * tiles_n, per = (tiles + 7) / 8;
+  const int slot = blockIdx.x >> 3, at = (int)(blockIdx.x & 7) * per + slot;
+  if (slot >= per || at >= tiles) return false;
+  const int strip = at / (4 * tiles_n), rest = at - strip * 4 * tiles_n;
+  const int high = tiles_m - 4 * strip < 4 ? tiles_m - 4 * strip : 4;
+  *tm = 4 * strip + rest % high;
+  *tn = rest / high;
+  return true;
+}
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N == 0 || N == 4 || N == 8 || N == 12 || N == 16, "add the matching wait");
+  if constexpr (N == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if constexpr (N == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  if constexpr (N == 12) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+  if constexpr (N == 16) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+}
+
 struct F32 {};
 template <>
 struct Gemm<F32> {
@@ -59,7 +87,9 @@ struct Gemm<F32> {
 // TM x TN: the workgroup's output tile, 256 x 256 (two stages of 64 KB) or 128 x 128 for problems with too few large
 // tiles to fill the chip.
 // WN x WM wavefronts share the tile: a wavefront's part is (TN/WN n) x (TM/WM m).
-template <typename TR, int TM, int TN, int WN, int WM>
+// ST: k-tiles in LDS.  Four (128 KB) where a CU has one 128 x 128 tile anyway: with two, each tile's loads were requested one tile's
+// work ahead and their latency was waited for; with several workgroups on a CU one computes while another waits.
+template <typename TR, int TM, int TN, int WN, int WM, int ST>
 __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a) {
   constexpr int NW = WN * WM;
   constexpr int XTILE = TM * ROWB;
@@ -78,16 +108,8 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane & 31, lh = lane >> 5;
 
-  // ---- workgroup -> tile: 4 x 8 tile blocks per XCD ---------------------------------------------------------------
-  const int tiles_m = (int)((a.M + TM - 1) / TM), tiles_n = (int)((a.N + TN - 1) / TN);
-  const int super_n = (tiles_n + 7) / 8;
-  const int nsuper = ((tiles_m + 3) / 4) * super_n;
-  const int slot = blockIdx.x >> 3;
-  const int super = (slot >> 5) * 8 + (blockIdx.x & 7);
-  if (super >= nsuper) return;
-  const int tm = (super / super_n) * 4 + ((slot & 31) >> 3);
-  const int tn = (super % super_n) * 8 + (slot & 7);
-  if (tm >= tiles_m || tn >= tiles_n) return;
+  int tm, tn;
+  if (!tile_of_block<TM, TN>(a, &tm, &tn)) return;
   const long long m0 = (long long)tm * TM, n0 = (long long)tn * TN;
 
   // ---- global -> LDS: wavefront w moves rows (TM/8)w .. of the x tile and (TN/8)w .. of the w tile, 8 rows (1 KB) per instruction
@@ -165,24 +187,19 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
       for (int j = 0; j < MJ; j++) acc[i][j] = G::mma(fw[buf][i], fx[buf][j], acc[i][j]);
   };
 
+  // Past the last tile it is requested again, into stages that nothing reads any more: the number of loads in flight behind
+  // every wait is the same.
   const int ntk = (int)(a.K / BK);
   if (ntk > 0) {
-    dma_tile(0, 0);
-    if (ntk > 1) {
-      dma_tile(1, 1);
-      // tile 0's loads; tile 1's XI + WI may still be in flight
-      if constexpr (XI + WI == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      static_assert(XI + WI == 8 || XI + WI == 4, "add the matching wait");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+#pragma unroll
+    for (int t = 0; t < ST; t++) dma_tile(t < ntk ? t : ntk - 1, t);
+    wait_loads<(ST - 1) * (XI + WI)>();  // tile 0's
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     load_frag(0, smem, 0);
   }
   for (int t = 0; t < ntk; t++) {
-    const char* st = smem + (t & 1) * STAGE;
+    const char* st = smem + (t % ST) * STAGE;
     load_frag(1, st, 1);
     mma(0);
     __builtin_amdgcn_sched_barrier(0);
@@ -192,16 +209,59 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
     load_frag(1, st, 3);
     mma(0);
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    wait_loads<(ST - 2) * (XI + WI)>();  // tile t+1's
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + 2 < ntk) dma_tile(t + 2, t & 1);
-    if (t + 1 < ntk) load_frag(0, smem + ((t + 1) & 1) * STAGE, 0);
+    dma_tile(t + ST < ntk ? t + ST : ntk - 1, t % ST);
+    if (t + 1 < ntk) load_frag(0, smem + ((t + 1) % ST) * STAGE, 0);
     mma(1);
     __builtin_amdgcn_sched_barrier(0);
   }
+  wait_loads<0>();  // none may write LDS that has passed to another workgroup
+
+  if constexpr (TM == 128 && TN == 128) {
+    // The tile leaves through LDS as whole rows, 16 bytes at any alignment a lane (four elements of a row each, as the
+    // accumulators lie, took 56 us for a 4095 x 4095 x 64 product's rows of odd length, 25 so): 16-byte chunk c of row r at slot c ^ (r % chunks).
+    constexpr int CH = TN * ESZ / 16;  // chunks of a row
+    __builtin_amdgcn_s_barrier();      // every wavefront has taken its last operands
+#pragma unroll
+    for (int j = 0; j < MJ; j++) {
+      const int row = (TM / WM) * wm + 32 * j + lq;
+#pragma unroll
+      for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int rg = 0; rg < 4; rg++) {
+          const int col = (TN / WN) * wn + 32 * i + 8 * rg + 4 * lh;
+          f32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * rg + e];
+          *(typename G::out4*)(smem + row * TN * ESZ + 16 * ((col / G::KPC) ^ (row & (CH - 1))) + (col % G::KPC) * ESZ) = G::cvt(v);
+        }
+    }
+    __syncthreads();
+    constexpr int PER = NW * 64 / CH;  // rows at a time
+#pragma unroll
+    for (int it = 0; it < TM / PER; it++) {
+      const int row = PER * it + tid / CH, c = tid % CH;
+      const u32x4 v = *(const u32x4*)(smem + row * TN * ESZ + 16 * (c ^ (row & (CH - 1))));
+      const long long m = m0 + row, n = n0 + c * G::KPC;
+      if (m >= a.M) continue;
+      T* dst = (T*)a.out + (long long)blockIdx.y * a.bso + m * a.ldo + n;
+      if (n + G::KPC <= a.N) {
+        *(loose16*)dst = v;
+      } else {
+        const vec8 o = __builtin_bit_cast(vec8, v);
+#pragma unroll
+        for (int e = 0; e < G::KPC; e++)
+          if (n + e < a.N) dst[e] = o[e];
+      }
+    }
+    return;
+  }
 
   // ---- store: register group rg of acc[i][j] is out[m = .. + 32j + lq][n = .. + 32i + 8rg + 4lh .. +3] ----------------------
+  const bool whole = ((a.N | a.ldo) & 3) == 0 && ((uintptr_t)a.out & (4 * ESZ - 1)) == 0;
 #pragma unroll
   for (int j = 0; j < MJ; j++) {
     const long long m = m0 + (TM / WM) * wm + 32 * j + lq;
@@ -212,11 +272,18 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
 #pragma unroll
       for (int rg = 0; rg < 4; rg++) {
         const long long n = n0 + (TN / WN) * wn + 32 * i + 8 * rg + 4 * lh;
-        if (n < a.N) {  // N is a multiple of 4 on this route
+        if (n < a.N) {
           f32x4 v;
 #pragma unroll
           for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * rg + e];
-          *(typename G::out4*)(orow + n) = G::cvt(v);
+          const typename G::out4 o = G::cvt(v);
+          if (whole) {
+            *(typename G::out4*)(orow + n) = o;
+          } else {  // rows that do not begin at, or end with, groups of four
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+              if (n + e < a.N) orow[n + e] = o[e];
+          }
         }
       }
   }
@@ -258,16 +325,8 @@ __global__ __launch_bounds__(512, 1) void linear_mfma_t_kernel(LinArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane & 31, lh = lane >> 5;
 
-  // workgroup -> tile: 4 x 8 tile blocks per XCD, as in linear_mfma_kernel
-  const int tiles_m = (int)((a.M + TM - 1) / TM), tiles_n = (int)((a.N + TN - 1) / TN);
-  const int super_n = (tiles_n + 7) / 8;
-  const int nsuper = ((tiles_m + 3) / 4) * super_n;
-  const int slot = blockIdx.x >> 3;
-  const int super = (slot >> 5) * 8 + (blockIdx.x & 7);
-  if (super >= nsuper) return;
-  const int tm = (super / super_n) * 4 + ((slot & 31) >> 3);
-  const int tn = (super % super_n) * 8 + (slot & 7);
-  if (tm >= tiles_m || tn >= tiles_n) return;
+  int tm, tn;
+  if (!tile_of_block<TM, TN>(a, &tm, &tn)) return;
   const long long m0 = (long long)tm * TM, n0 = (long long)tn * TN;
 
   // ---- global -> LDS -------------------------------------------------------------------------------------------------------
@@ -484,16 +543,8 @@ __global__ __launch_bounds__(256, 1) void linear256_kernel(LinArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
 
-  // workgroup -> tile: 4 x 8 tile blocks per XCD, as in linear_mfma_kernel
-  const int tiles_m = (int)((a.M + TM - 1) / TM), tiles_n = (int)((a.N + TN - 1) / TN);
-  const int super_n = (tiles_n + 7) / 8;
-  const int nsuper = ((tiles_m + 3) / 4) * super_n;
-  const int slot = blockIdx.x >> 3;
-  const int super = (slot >> 5) * 8 + (blockIdx.x & 7);
-  if (super >= nsuper) return;
-  const int tm = (super / super_n) * 4 + ((slot & 31) >> 3);
-  const int tn = (super % super_n) * 8 + (slot & 7);
-  if (tm >= tiles_m || tn >= tiles_n) return;
+  int tm, tn;
+  if (!tile_of_block<TM, TN>(a, &tm, &tn)) return;
   const long long m0 = (long long)tm * TM, n0 = (long long)tn * TN;
 
   // global -> LDS: wavefront v moves rows 64v .. 64v+63 of both tiles, 8 rows (1 KB) per instruction; lane l fills
@@ -585,9 +636,12 @@ __global__ __launch_bounds__(256, 1) void linear256_kernel(LinArgs a) {
     if (m < a.M) {
       T* dst = (T*)a.out + m * a.ldo + n;
       if (n + 8 <= a.N) {
-        *(u32x4*)dst = v;
-      } else if (n + 4 <= a.N) {  // N is a multiple of 4 on this route
-        *(u32x2*)dst = u32x2{v[0], v[1]};
+        *(loose16*)dst = v;  // rows of any length and alignment; aligned ones take the same instruction
+      } else {
+        const typename TR::vec8 o = __builtin_bit_cast(typename TR::vec8, v);
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          if (n + e < a.N) dst[e] = o[e];
       }
     }
   }
@@ -646,60 +700,115 @@ __global__ __launch_bounds__(256) void linear_general_kernel(LinArgs a) {
   }
 }
 
-// dst[c, r] = src[r, c] for src [R, C] with row stride ld; dst dense [C, R].  64 x 64 tiles through LDS, 16 bytes per
-// global access where the row lengths allow it (VECOK: ld and R multiples of 16 bytes, both pointers 16-byte aligned).
-template <typename T, bool VECOK>
-__global__ __launch_bounds__(256) void transpose_kernel(const T* src, T* dst, long long R, long long C, long long ld) {
+// Operands brought into the layout of the x . w^T kernels: dst dense rows of `ldd` elements (a multiple of a k-tile), the
+// elements past the operand's own zeros.  Bound by memory: 16-byte accesses on both sides whatever the source's alignment.
+template <typename T>
+__global__ __launch_bounds__(256) void pack_rows_kernel(const T* src, T* dst, long long R, long long C, long long ld, long long ldd) {
   constexpr int VEC = 16 / sizeof(T);
-  constexpr int PITCH = 64 + VEC;  // rows stay 16-byte aligned
   typedef T vecT __attribute__((ext_vector_type(VEC)));
-  __shared__ __attribute__((aligned(16))) T tile[64][PITCH];
-  const long long r0 = (long long)blockIdx.y * 64, c0 = (long long)blockIdx.x * 64;
-  constexpr int CPR = 64 / VEC;  // 16-byte chunks per tile row
+  const long long c = ((long long)blockIdx.x * 64 + (threadIdx.x & 63)) * VEC;
+  if (c >= ldd) return;
+  const long long r0 = (long long)blockIdx.y * 16 + (threadIdx.x >> 6);
 #pragma unroll
-  for (int i = 0; i < 64 * CPR / 256; i++) {
-    const int chunk = threadIdx.x + 256 * i;
-    const int row = chunk / CPR, cc = (chunk % CPR) * VEC;
-    const long long r = r0 + row, c = c0 + cc;
-    if (r >= R) continue;
-    if (VECOK && c + VEC <= C) {
-      *(vecT*)&tile[row][cc] = *(const vecT*)(src + r * ld + c);
+  for (int i = 0; i < 4; i++) {
+    const long long r = r0 + 4 * i;
+    if (r >= R) return;
+    const T* p = src + r * ld + c;
+    vecT v;
+    if (c + VEC <= C) {
+      v = __builtin_bit_cast(vecT, (u32x4)*(const loose16*)p);
     } else {
 #pragma unroll
-      for (int e = 0; e < VEC; e++)
-        if (c + e < C) tile[row][cc + e] = src[r * ld + c + e];
+      for (int e = 0; e < VEC; e++) v[e] = c + e < C ? p[e] : (T)0;
     }
+    *(vecT*)(dst + r * ldd + c) = v;
   }
-  __syncthreads();
+}
+
+// dst[c, r] = src[r, c] for src [R, C] with row stride ld; dst [C, ldd].  A workgroup takes 64 columns of kPackRows rows through
+// LDS in 64 x 64 tiles (pitch: two dwords more than the tile's row, so that the eight lanes that read down a column of
+// eight rows each fall into different banks).  SUMS: also the fp32 sums of its rows' columns, to part[blockIdx.y][C]
+// (colsum_merge_kernel adds them): the bias's gradient costs no reading of its own.  6144 x 4096 bf16: 20 us, 5.0 TB/s.
+constexpr int kPackRows = 256;
+
+template <typename T, bool SUMS>
+__global__ __launch_bounds__(256) void pack_transposed_kernel(const T* src, T* dst, long long R, long long C, long long ld, long long ldd, float* part) {
+  constexpr int VEC = 16 / sizeof(T);
+  constexpr int PITCH = 64 + 4 / (int)sizeof(T);
+  constexpr int CPR = 64 / VEC;  // 16-byte chunks per tile row
+  typedef T vecT __attribute__((ext_vector_type(VEC)));
+  __shared__ uint32_t tile_words[64 * PITCH * sizeof(T) / 4];
+  T* tile = (T*)tile_words;
+  const long long c0 = (long long)blockIdx.x * 64;
+  float sums[64 * CPR / 256];
 #pragma unroll
-  for (int i = 0; i < 64 * CPR / 256; i++) {
-    const int chunk = threadIdx.x + 256 * i;
-    const int orow = chunk / CPR, oc = (chunk % CPR) * VEC;  // output row = source column; first of VEC source rows
-    const long long c = c0 + orow, r = r0 + oc;
-    if (c >= C) continue;
-    if (VECOK && r + VEC <= R) {
+  for (int i = 0; i < 64 * CPR / 256; i++) sums[i] = 0.f;
+  for (int t = 0; t < kPackRows / 64; t++) {
+    const long long r0 = (long long)blockIdx.y * kPackRows + 64 * t;
+    if (r0 >= ldd) break;
+    if (t) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 64 * CPR / 256; i++) {
+      const int chunk = threadIdx.x + 256 * i;
+      const int row = chunk / CPR, cc = (chunk % CPR) * VEC;
+      const long long r = r0 + row, c = c0 + cc;
+      const T* p = src + r * ld + c;
+      u32x4 v = {0, 0, 0, 0};
+      if (r < R) {
+        if (c + VEC <= C) {
+          v = *(const loose16*)p;
+        } else {
+          vecT w;
+#pragma unroll
+          for (int e = 0; e < VEC; e++) w[e] = c + e < C ? p[e] : (T)0;
+          v = __builtin_bit_cast(u32x4, w);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) tile_words[(row * PITCH + cc) * (int)sizeof(T) / 4 + e] = v[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 64 * CPR / 256; i++) {
+      const int chunk = threadIdx.x + 256 * i;
+      const int orow = chunk / CPR, oc = (chunk % CPR) * VEC;  // output row = source column; first of VEC source rows
+      const long long c = c0 + orow, r = r0 + oc;
       vecT v;
 #pragma unroll
-      for (int e = 0; e < VEC; e++) v[e] = tile[oc + e][orow];
-      *(vecT*)(dst + c * R + r) = v;
-    } else {
+      for (int e = 0; e < VEC; e++) v[e] = tile[(oc + e) * PITCH + orow];
+      if constexpr (SUMS) {
 #pragma unroll
-      for (int e = 0; e < VEC; e++)
-        if (r + e < R) dst[c * R + r + e] = tile[oc + e][orow];
+        for (int e = 0; e < VEC; e++) sums[i] += (float)v[e];
+      }
+      if (c < C && r < ldd) *(vecT*)(dst + c * ldd + r) = v;
+    }
+  }
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int i = 0; i < 64 * CPR / 256; i++) {
+      float v = sums[i];
+#pragma unroll
+      for (int m = 1; m < CPR; m <<= 1) v += __shfl_xor(v, m);
+      const int chunk = threadIdx.x + 256 * i;
+      const long long c = c0 + chunk / CPR;
+      if (chunk % CPR == 0 && c < C) part[(long long)blockIdx.y * C + c] = v;
     }
   }
 }
 
+// A product's operand [rows, K] (kmajor: stored [K, rows]) to rows of kpad elements.
 template <typename T>
-int launch_transpose(const void* src, void* dst, long long R, long long C, long long ld, hipStream_t stream) {
-  if ((R + 63) / 64 > 65535 || (C + 63) / 64 > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
-  dim3 grid((unsigned)((C + 63) / 64), (unsigned)((R + 63) / 64));
-  constexpr long long VEC = 16 / sizeof(T);
-  const bool vecok = ld % VEC == 0 && R % VEC == 0 && ((uintptr_t)src % 16) == 0 && ((uintptr_t)dst % 16) == 0;
-  if (vecok) {
-    hipLaunchKernelGGL((transpose_kernel<T, true>), grid, dim3(256), 0, stream, (const T*)src, (T*)dst, R, C, ld);
+int launch_pack(const void* src, void* dst, long long rows, long long K, long long ld, long long kpad, bool kmajor, float* part, hipStream_t stream) {
+  if (kmajor) {
+    const dim3 grid((unsigned)((rows + 63) / 64), (unsigned)((kpad + kPackRows - 1) / kPackRows));
+    if (part)
+      hipLaunchKernelGGL((pack_transposed_kernel<T, true>), grid, dim3(256), 0, stream, (const T*)src, (T*)dst, K, rows, ld, kpad, part);
+    else
+      hipLaunchKernelGGL((pack_transposed_kernel<T, false>), grid, dim3(256), 0, stream, (const T*)src, (T*)dst, K, rows, ld, kpad, part);
   } else {
-    hipLaunchKernelGGL((transpose_kernel<T, false>), grid, dim3(256), 0, stream, (const T*)src, (T*)dst, R, C, ld);
+    constexpr int VEC = 16 / (int)sizeof(T);
+    const dim3 grid((unsigned)((kpad / VEC + 63) / 64), (unsigned)((rows + 15) / 16));
+    hipLaunchKernelGGL((pack_rows_kernel<T>), grid, dim3(256), 0, stream, (const T*)src, (T*)dst, rows, K, ld, kpad);
   }
   return (int)hipGetLastError();
 }
@@ -712,7 +821,6 @@ int launch_transpose(const void* src, void* dst, long long R, long long C, long 
 template <typename T>
 __global__ __launch_bounds__(1024) void colsum_kernel(const T* x, long long M, long long N, long long ld, long long rows, T* out, float* part) {
   constexpr int V = 16 / sizeof(T), LANES = 16;
-  typedef uint32_t loose16 __attribute__((ext_vector_type(4), aligned(2)));
   __shared__ float sums[64][LANES * V + 1];
   const int c = threadIdx.x % LANES, g = threadIdx.x / LANES;  // 16 bytes of columns, row group
   const long long n0 = (long long)blockIdx.x * (LANES * V), n = n0 + V * c;
@@ -747,14 +855,26 @@ __global__ __launch_bounds__(1024) void colsum_kernel(const T* x, long long M, l
   }
 }
 
+// 64 columns per workgroup, the ranges among its four wavefronts
 template <typename T>
 __global__ __launch_bounds__(256) void colsum_merge_kernel(const float* part, int ranges, long long N, T* out) {
-  const long long n = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (n >= N) return;
+  __shared__ float sums[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long long n = (long long)blockIdx.x * 64 + lane;
   float v = 0.f;
+  if (n < N) {
 #pragma unroll 8
-  for (int i = 0; i < ranges; i++) v += part[i * N + n];
-  store_from_float(out + n, v);
+    for (int i = wave; i < ranges; i += 4) v += part[i * N + n];
+  }
+  sums[wave][lane] = v;
+  __syncthreads();
+  if (wave == 0 && n < N) store_from_float(out + n, (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]));
+}
+
+template <typename T>
+int launch_colsum_merge(const float* part, int ranges, long long N, void* out, hipStream_t stream) {
+  hipLaunchKernelGGL((colsum_merge_kernel<T>), dim3((unsigned)((N + 63) / 64)), dim3(256), 0, stream, part, ranges, N, (T*)out);
+  return (int)hipGetLastError();
 }
 
 // Row ranges: enough for two workgroups per CU, of no fewer than 1024 rows' worth of work each (16 loads per lane).
@@ -773,9 +893,7 @@ int launch_colsum(const void* x, long long M, long long N, long long ld, void* o
   if ((N + wide - 1) / wide > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
   hipLaunchKernelGGL((colsum_kernel<T>), dim3((unsigned)((N + wide - 1) / wide), (unsigned)ranges), dim3(1024), 0, stream, (const T*)x, M, N, ld,
                      rows, (T*)out, ranges > 1 ? part : nullptr);
-  if (ranges > 1)
-    hipLaunchKernelGGL((colsum_merge_kernel<T>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, part, ranges, N, (T*)out);
-  return (int)hipGetLastError();
+  return ranges > 1 ? launch_colsum_merge<T>(part, ranges, N, out, stream) : (int)hipGetLastError();
 }
 
 bool aligned(const void* p, size_t n) { return ((uintptr_t)p % n) == 0; }
@@ -799,19 +917,31 @@ int check(int dtype, const void* x, const void* w, const void* out, long long M,
   return TTSDPA_OK;
 }
 
-template <typename TR, int TM, int TN, int WN, int WM>
-int launch_mfma_tile(const LinArgs& a, hipStream_t stream, unsigned entries = 1) {
-  constexpr int lds = 2 * (TM + TN) * ROWB;
+// Workgroups that tile_of_block spreads over the 8 XCDs (the kernels count in 32 bits).
+long long blocks_of_tiles(const LinArgs& a, int TM, int TN) {
+  const long long tiles = ((a.M + TM - 1) / TM) * ((a.N + TN - 1) / TN);
+  return (tiles + 7) / 8 * 8;
+}
+
+template <typename TR, int TM, int TN, int WN, int WM, int ST>
+int launch_mfma_stages(const LinArgs& a, hipStream_t stream, unsigned entries) {
+  constexpr int lds = ST * (TM + TN) * ROWB;
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  const hipError_t granted = grant_dynamic_lds((const void*)linear_mfma_kernel<TR, TM, TN, WN, WM>, lds, state, done);
+  const hipError_t granted = grant_dynamic_lds((const void*)linear_mfma_kernel<TR, TM, TN, WN, WM, ST>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long tiles_m = (a.M + TM - 1) / TM, tiles_n = (a.N + TN - 1) / TN;
-  const long long nsuper = ((tiles_m + 3) / 4) * ((tiles_n + 7) / 8);
-  const long long nwg = (nsuper + 7) / 8 * 8 * 32;
-  if (nwg > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
-  hipLaunchKernelGGL((linear_mfma_kernel<TR, TM, TN, WN, WM>), dim3((unsigned)nwg, entries), dim3(WN * WM * 64), lds, stream, a);
+  const long long nwg = blocks_of_tiles(a, TM, TN);
+  if (nwg > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
+  hipLaunchKernelGGL((linear_mfma_kernel<TR, TM, TN, WN, WM, ST>), dim3((unsigned)nwg, entries), dim3(WN * WM * 64), lds, stream, a);
   return (int)hipGetLastError();
+}
+
+// 128 x 128 tiles, one per CU at most: four k-tiles in LDS
+bool tile_per_cu(const LinArgs& a, unsigned entries) { return ((a.M + 127) / 128) * ((a.N + 127) / 128) * entries <= 256; }
+
+template <typename TR>
+int launch_small_tiles(const LinArgs& a, hipStream_t stream, unsigned entries = 1) {
+  return tile_per_cu(a, entries) ? launch_mfma_stages<TR, 128, 128, 4, 2, 4>(a, stream, entries) : launch_mfma_stages<TR, 128, 128, 4, 2, 2>(a, stream, entries);
 }
 
 template <typename TR, int T_, bool XT, bool WT>
@@ -821,22 +951,21 @@ int launch_mfma_t_tile(const LinArgs& a, hipStream_t stream) {
   static bool done[kMaxDevices];
   const hipError_t granted = grant_dynamic_lds((const void*)linear_mfma_t_kernel<TR, T_, T_, XT, WT>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long tiles_m = (a.M + T_ - 1) / T_, tiles_n = (a.N + T_ - 1) / T_;
-  const long long nsuper = ((tiles_m + 3) / 4) * ((tiles_n + 7) / 8);
-  const long long nwg = (nsuper + 7) / 8 * 8 * 32;
-  if (nwg > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
+  const long long nwg = blocks_of_tiles(a, T_, T_);
+  if (nwg > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
   hipLaunchKernelGGL((linear_mfma_t_kernel<TR, T_, T_, XT, WT>), dim3((unsigned)nwg), dim3(512), lds, stream, a);
   return (int)hipGetLastError();
 }
 
+// 256 x 256 tiles once they fill the chip, unless their last round over the 256 CUs would be under 85 % full: then four
+// times as many 128 x 128 tiles (weight gradient of the QKV projection, 384 large tiles: 878 -> 936 TFLOP/s; its input
+// gradient, 512 large tiles, runs 1063 against 795 on the small ones)
+bool large_in_place(long long n256) { return n256 >= 256 && n256 * 100 >= (n256 + 255) / 256 * 256 * 85; }
+
 // 16-bit operands read as they lie in memory (a.xt / a.wt: stored contraction-major)
 template <typename TR>
 int launch_mfma_t(const LinArgs& a, hipStream_t stream) {
-  // 256 x 256 tiles once they fill the chip, unless their last round over the 256 CUs would be under 85 % full: then four
-  // times as many 128 x 128 tiles (weight gradient of the QKV projection, 384 large tiles: 878 -> 936 TFLOP/s; its input
-  // gradient, 512 large tiles, runs 1063 against 795 on the small ones)
-  const long long n256 = ((a.M + 255) / 256) * ((a.N + 255) / 256);
-  const bool big = n256 >= 256 && n256 * 100 >= (n256 + 255) / 256 * 256 * 85;
+  const bool big = large_in_place(((a.M + 255) / 256) * ((a.N + 255) / 256));
   if (a.xt && a.wt) return big ? launch_mfma_t_tile<TR, 256, true, true>(a, stream) : launch_mfma_t_tile<TR, 128, true, true>(a, stream);
   if (a.xt) return big ? launch_mfma_t_tile<TR, 256, true, false>(a, stream) : launch_mfma_t_tile<TR, 128, true, false>(a, stream);
   return big ? launch_mfma_t_tile<TR, 256, false, true>(a, stream) : launch_mfma_t_tile<TR, 128, false, true>(a, stream);
@@ -849,41 +978,60 @@ int launch_linear256(const LinArgs& a, hipStream_t stream) {
   static bool done[kMaxDevices];
   const hipError_t granted = grant_dynamic_lds((const void*)linear256_kernel<TR>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long tiles_m = (a.M + 255) / 256, tiles_n = (a.N + 255) / 256;
-  const long long nsuper = ((tiles_m + 3) / 4) * ((tiles_n + 7) / 8);
-  const long long nwg = (nsuper + 7) / 8 * 8 * 32;
-  if (nwg > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
+  const long long nwg = blocks_of_tiles(a, 256, 256);
+  if (nwg > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
   hipLaunchKernelGGL((linear256_kernel<TR>), dim3((unsigned)nwg), dim3(256), lds, stream, a);
   return (int)hipGetLastError();
 }
 
+// Microseconds of the tiled kernels, from measurements, against each other's and the streaming kernel's.  A k-step of 128
+// bytes of a 128 x 128 tile takes 0.6 us (fp32 2.2) as long as every CU has one tile at most, and with more in proportion
+// (128 .. 1000 x 4096 x 4096: 35 .. 41 us, 2000 rows 74) or, where the matrix pipe bounds it (fp32), by whole rounds.
+double small_tiles_cost(const LinArgs& a, int dtype, unsigned entries) {
+  const double tiles = (double)((a.M + 127) / 128) * (double)((a.N + 127) / 128) * entries;
+  const double steps = a.K * (dtype == TTSDPA_F32 ? 4 : 2) / 128.0;
+  if (dtype == TTSDPA_F32) return 3 + steps * 2.2 * (double)(long long)((tiles + 255) / 256);
+  return 3 + steps * 0.6 * (tiles > 256 ? tiles / 256 : 1);
+}
+// 16-bit, 256 x 256: a round of the 256 CUs takes a k-step in 1.6 us, however many of them have a tile: 1999 x 6144 x 4096,
+// 192 tiles, 112 us on the small tiles and 96 on these, 1999 x 4096 x 4096, 128 tiles, 75 against 106.
+double large_tiles_cost(const LinArgs& a) {
+  const long long tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256);
+  return 4 + a.K / 64.0 * 1.6 * (double)((tiles + 255) / 256);
+}
+
+// x . w^T on rows of whole k-tiles
+double nt_cost(const LinArgs& a, int dtype, unsigned entries) {
+  const double us = small_tiles_cost(a, dtype, entries);
+  if (dtype == TTSDPA_F32 || entries > 1) return us;
+  const double large = large_tiles_cost(a);
+  return large < us ? large : us;
+}
+
 template <typename TR>
 int launch_mfma(const LinArgs& a, hipStream_t stream) {
-  // 256 x 256 tiles once they fill the 256 CUs; smaller problems get four times as many 128 x 128 tiles
-  const long long big = ((a.M + 255) / 256) * ((a.N + 255) / 256);
   // (four wavefronts with 128 x 128 each — accumulators in AGPRs, half the LDS operand reads — measured 2-10 % slower
   // than eight with 64 x 128: one wavefront per SIMD hides too little)
   if constexpr (!std::is_same<TR, F32>::value) {
-    // 16-bit tensors: the hand-ordered kernel
-    // and it stores 16 bytes at a time
-    if (big >= 256 && a.ldo % 8 == 0 && ((uintptr_t)a.out & 15) == 0) return launch_linear256<TR>(a, stream);
+    if (large_tiles_cost(a) < small_tiles_cost(a, TTSDPA_BF16, 1)) return launch_linear256<TR>(a, stream);  // the hand-ordered kernel
+    return launch_small_tiles<TR>(a, stream);
+  } else {
+    const long long big = ((a.M + 255) / 256) * ((a.N + 255) / 256);
+    return big >= 256 ? launch_mfma_stages<TR, 256, 256, 4, 2, 2>(a, stream, 1) : launch_small_tiles<TR>(a, stream);
   }
-  return big >= 256 ? launch_mfma_tile<TR, 256, 256, 4, 2>(a, stream) : launch_mfma_tile<TR, 128, 128, 4, 2>(a, stream);
 }
 
-// Microseconds of the tiled kernels, from measurements, against the streaming kernel's: a k-step of 128 bytes of a 128 x 128
-// tile takes 0.6 us (fp32 2.2) as long as every CU has one tile at most, and with more in proportion (128 .. 1000 x 4096
-// x 4096: 40 .. 45 us, 2000 rows 74; the 256 x 256 tiles are faster, but no product that fills the chip with them is
-// small enough for the other kernel).  A k-major w alone, in place: 10 % more.
-double tiled_cost(const LinArgs& a, int dtype, unsigned entries) {
-  const double tiles = (double)((a.M + 127) / 128) * (double)((a.N + 127) / 128) * entries;
-  const double steps = a.K * (dtype == TTSDPA_F32 ? 4 : 2) / 128.0;
-  const double us = 3 + steps * (dtype == TTSDPA_F32 ? 2.2 : 0.6) * (tiles > 256 ? tiles / 256 : 1);
-  return a.wt && !a.xt ? us * 1.1 : us;
+// What the kernels of contraction-major operands take in place: the small tiles 10 % more where only w is (a tile of the
+// other form takes both kinds of LDS read), the large ones 2.3 us a k-step (8192 x 4096 x 6144, 512 tiles: 443 us).
+double in_place_cost(const LinArgs& a, int dtype, unsigned entries) {
+  if (!a.xt && !a.wt) return nt_cost(a, dtype, entries);
+  const long long n256 = ((a.M + 255) / 256) * ((a.N + 255) / 256);
+  if (large_in_place(n256)) return 3 + a.K / 64.0 * 2.3 * (double)((n256 + 255) / 256);
+  return small_tiles_cost(a, dtype, entries) * (a.wt && !a.xt ? 1.1 : 1);
 }
 
 bool streams(const LinArgs& a, int dtype, unsigned entries = 1, bool may_split = false) {
-  return stream_takes(a, dtype) && stream_cost(a, dtype, entries, may_split) < tiled_cost(a, dtype, entries);
+  return stream_takes(a, dtype) && stream_cost(a, dtype, entries, may_split) < in_place_cost(a, dtype, entries);
 }
 
 // What the tiled kernels' layout does not allow: the streaming kernel, or where one of its operands is too narrow for that (a
@@ -913,40 +1061,7 @@ int ttlinear_plan(int dtype, const void* x, const void* w, const void* bias, con
   return rc;
 }
 
-// x . w^T + bias; scratch (optional): lets the streaming kernel divide the contraction among workgroups
-static int forward(int dtype, const void* x, const void* w, const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t ldx,
-                   int64_t ldw, int64_t ldo, void* scratch, size_t scratch_bytes, void* stream) {
-  int route = TTLINEAR_ROUTE_NONE;
-  const int rc = check(dtype, x, w, out, M, N, K, ldx, ldw, ldo, &route);
-  if (rc != TTSDPA_OK || route == TTLINEAR_ROUTE_NONE) return rc;
-  const size_t esz = dtype == TTSDPA_F32 ? 4 : 2;
-  if (bias && !aligned(bias, esz)) return TTSDPA_ERR_STRIDE;
-  LinArgs a{x, w, bias, out, M, N, K, ldx, ldw, ldo};
-  hipStream_t s = (hipStream_t)stream;
-  if (route == TTLINEAR_ROUTE_MFMA) {
-    if (streams(a, dtype, 1, scratch)) return launch_stream(a, dtype, s, 1, scratch, scratch_bytes);
-    return dtype == TTSDPA_F32 ? launch_mfma<F32>(a, s) : dtype == TTSDPA_F16 ? launch_mfma<F16>(a, s) : launch_mfma<BF16>(a, s);
-  }
-  switch (dtype) {
-    case TTSDPA_F32: return launch_general_linear<float>(a, s, 1, scratch, scratch_bytes);
-    case TTSDPA_F16: return launch_general_linear<_Float16>(a, s, 1, scratch, scratch_bytes);
-    default: return launch_general_linear<__bf16>(a, s, 1, scratch, scratch_bytes);
-  }
-}
-
-int ttlinear_forward(int dtype, const void* x, const void* w, const void* bias, void* out, int64_t M, int64_t N,
-                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldo, void* stream) {
-  return forward(dtype, x, w, bias, out, M, N, K, ldx, ldw, ldo, nullptr, 0, stream);
-}
-
-// Bytes of the dense transposed copies the MFMA route of ttlinear_matmul makes: a as [M, K] when it is stored [K, M],
-// b as [N, K] when it is stored [K, N]; each rounded up to 256 bytes.
-static size_t matmul_copy_bytes(int dtype, int64_t rows, int64_t K) {
-  const size_t esz = dtype == TTSDPA_F32 ? 4 : 2;
-  return ((size_t)rows * (size_t)K * esz + 255) / 256 * 256;
-}
-
-// 16-bit operands that the matrix-core kernel reads in place, contraction-major or not (no copies, no scratch).
+// 16-bit operands that a matrix-core kernel reads in place, one of them contraction-major at least (no copies, no scratch).
 static bool in_place_ok(const LinArgs& g, int dtype) {
   if (dtype == TTSDPA_F32 || g.K < 1 || g.K % 64 != 0 || g.N % 4 != 0 || g.ldo % 4 != 0 || !aligned(g.out, 8)) return false;
   auto operand_ok = [](const void* p, bool contraction_major, int64_t rows, int64_t ld) {
@@ -954,44 +1069,129 @@ static bool in_place_ok(const LinArgs& g, int dtype) {
     // a tile's rows are addressed with 32-bit byte offsets: 64 k-rows of a contraction-major operand, 256 rows otherwise
     return contraction_major ? (rows % 8 == 0 && ld < (1 << 24)) : ld < (1 << 21);
   };
-  return operand_ok(g.x, g.xt, g.M, g.ldx) && operand_ok(g.w, g.wt, g.N, g.ldw);
+  return (g.xt || g.wt) && operand_ok(g.x, g.xt, g.M, g.ldx) && operand_ok(g.w, g.wt, g.N, g.ldw);
 }
 
-// A product with a contraction-major operand goes to the streaming kernel when the tiled ones do not take it or are estimated
-// slower: 16-bit operands in place, or, given scratch, x . w^T on row-major copies (read and written at 4 TB/s, a launch each).
-static bool matmul_streams(const LinArgs& g, int dtype, bool scratch) {
-  if (!stream_takes(g, dtype)) return false;
-  double tiled = 0;
-  if (in_place_ok(g, dtype)) {
-    tiled = tiled_cost(g, dtype, 1);
-  } else if (scratch && g.K % (dtype == TTSDPA_F32 ? 32 : 64) == 0 && g.N % 4 == 0 && g.ldo % 4 == 0) {
-    LinArgs nt = g;
-    nt.xt = nt.wt = 0;
-    const double copied = ((g.xt ? g.M : 0) + (g.wt ? g.N : 0)) * (double)g.K * (dtype == TTSDPA_F32 ? 8 : 4);
-    tiled = tiled_cost(nt, dtype, 1) + copied / 4e6 + 2.5 * (g.xt + g.wt);
+// x . w^T on the tiled kernels, with copies of the operands whose layout they do not take (contraction-major, rows that are
+// not whole k-tiles, unaligned) in scratch: what the copies need and what the product is estimated to take with them.
+struct PackPlan {
+  bool ok, x, w;
+  long long kpad;
+  size_t xbytes, bytes;
+  double us;
+};
+
+static PackPlan plan_pack(const LinArgs& g, int dtype) {
+  const long long esz = dtype == TTSDPA_F32 ? 4 : 2, bk = ROWB / esz, kpc = 16 / esz;
+  PackPlan p{};
+  p.kpad = (g.K + bk - 1) / bk * bk;
+  auto as_it_is = [&](const void* ptr, int kmajor, long long ld) { return !kmajor && g.K == p.kpad && ld % kpc == 0 && aligned(ptr, 16); };
+  p.x = !as_it_is(g.x, g.xt, g.ldx);
+  p.w = !as_it_is(g.w, g.wt, g.ldw);
+  // rows of a tile are addressed with 32-bit byte offsets; grids
+  p.ok = g.K > 0 && p.kpad < (1 << 21) && (p.x || g.ldx < (1 << 21)) && (p.w || g.ldw < (1 << 21)) && (g.M + 15) / 16 <= 65535 &&
+         (!p.w || (g.N + 15) / 16 <= 65535);
+  if (!p.ok) return p;
+  auto bytes = [&](long long rows) { return ((size_t)rows * (size_t)p.kpad * (size_t)esz + 255) / 256 * 256; };
+  p.xbytes = p.x ? bytes(g.M) : 0;
+  p.bytes = p.xbytes + (p.w ? bytes(g.N) : 0);
+  LinArgs nt = g;
+  nt.K = p.kpad, nt.xt = nt.wt = 0;
+  p.us = nt_cost(nt, dtype, 1) + (double)p.bytes * 2 / 4e6 + 2.5 * (p.x + p.w);  // read and written at 4 TB/s, a launch each
+  return p;
+}
+
+// sums: the column sums of x's rows' parts, where x is packed from a contraction-major operand ([ranges][M])
+static int launch_packed(const LinArgs& g, const PackPlan& p, int dtype, hipStream_t s, char* scratch, float* sums) {
+  LinArgs nt = g;
+  nt.K = p.kpad, nt.xt = nt.wt = 0;
+  auto pack = [&](const void* src, void* dst, long long rows, long long ld, bool kmajor, float* part) {
+    switch (dtype) {
+      case TTSDPA_F32: return launch_pack<float>(src, dst, rows, g.K, ld, p.kpad, kmajor, part, s);
+      case TTSDPA_F16: return launch_pack<_Float16>(src, dst, rows, g.K, ld, p.kpad, kmajor, part, s);
+      default: return launch_pack<__bf16>(src, dst, rows, g.K, ld, p.kpad, kmajor, part, s);
+    }
+  };
+  if (p.x) {
+    const int rc = pack(g.x, scratch, g.M, g.ldx, g.xt, sums);
+    if (rc != 0) return rc;
+    nt.x = scratch, nt.ldx = p.kpad;
   }
-  return tiled == 0 || stream_cost(g, dtype, 1, scratch) < tiled;
+  if (p.w) {
+    const int rc = pack(g.w, scratch + p.xbytes, g.N, g.ldw, g.wt, nullptr);
+    if (rc != 0) return rc;
+    nt.w = scratch + p.xbytes, nt.ldw = p.kpad;
+  }
+  return dtype == TTSDPA_F32 ? launch_mfma<F32>(nt, s) : dtype == TTSDPA_F16 ? launch_mfma<F16>(nt, s) : launch_mfma<BF16>(nt, s);
 }
 
-// Sizes and layout alone.
+// How a product runs: the cheapest by estimate of the ways that take it.
+enum class Way { General, Stream, InPlace, Packed };
+
+static Way choose(const LinArgs& g, int dtype, bool scratch, size_t scratch_bytes, PackPlan* p, double* us = nullptr) {
+  Way way = Way::General;
+  double best = 1e30;
+  auto take = [&](Way w, double cost) {
+    if (cost < best) way = w, best = cost;
+  };
+  *p = plan_pack(g, dtype);
+  if (p->ok && p->bytes <= (scratch ? scratch_bytes : 0)) take(Way::Packed, p->us);
+  if (in_place_ok(g, dtype)) take(Way::InPlace, in_place_cost(g, dtype, 1));
+  if (stream_takes(g, dtype)) take(Way::Stream, stream_cost(g, dtype, 1, scratch));
+  if (us) *us = best;
+  return way;
+}
+
+static int product(const LinArgs& g, int dtype, void* scratch, size_t scratch_bytes, hipStream_t s) {
+  PackPlan p;
+  switch (choose(g, dtype, scratch, scratch_bytes, &p)) {
+    case Way::Stream: return launch_stream(g, dtype, s, 1, scratch, scratch_bytes);
+    case Way::InPlace: return dtype == TTSDPA_F16 ? launch_mfma_t<F16>(g, s) : launch_mfma_t<BF16>(g, s);
+    case Way::Packed: return launch_packed(g, p, dtype, s, (char*)scratch, nullptr);
+    default: break;
+  }
+  switch (dtype) {
+    case TTSDPA_F32: return launch_general_linear<float>(g, s, 1, scratch, scratch_bytes);
+    case TTSDPA_F16: return launch_general_linear<_Float16>(g, s, 1, scratch, scratch_bytes);
+    default: return launch_general_linear<__bf16>(g, s, 1, scratch, scratch_bytes);
+  }
+}
+
+// x . w^T + bias; scratch (optional): lets the streaming kernel divide the contraction among workgroups, and holds copies
+static int forward(int dtype, const void* x, const void* w, const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                   int64_t ldw, int64_t ldo, void* scratch, size_t scratch_bytes, void* stream) {
+  int route = TTLINEAR_ROUTE_NONE;
+  const int rc = check(dtype, x, w, out, M, N, K, ldx, ldw, ldo, &route);
+  if (rc != TTSDPA_OK || route == TTLINEAR_ROUTE_NONE) return rc;
+  if (bias && !aligned(bias, dtype == TTSDPA_F32 ? 4 : 2)) return TTSDPA_ERR_STRIDE;
+  return product(LinArgs{x, w, bias, out, M, N, K, ldx, ldw, ldo}, dtype, scratch, scratch_bytes, (hipStream_t)stream);
+}
+
+int ttlinear_forward(int dtype, const void* x, const void* w, const void* bias, void* out, int64_t M, int64_t N,
+                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldo, void* stream) {
+  return forward(dtype, x, w, bias, out, M, N, K, ldx, ldw, ldo, nullptr, 0, stream);
+}
+
+// Sizes and layout alone: dense operands on aligned addresses.
 static LinArgs flags_args(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
   return LinArgs{nullptr, nullptr, nullptr, nullptr, M, N, K, trans_a ? M : K, trans_b ? K : N, N, trans_a ? 1 : 0, trans_b ? 0 : 1};
 }
 
+// Room for the copies (where the product would be made on copies, or operands lie contraction-major) or the parts of a divided contraction.
 size_t ttlinear_matmul_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const size_t copies = (trans_a ? matmul_copy_bytes(dtype, M, K) : 0) + (!trans_b ? matmul_copy_bytes(dtype, N, K) : 0);
-  const size_t parts = stream_scratch(flags_args(M, N, K, trans_a, trans_b), dtype);
-  return parts > copies ? parts : copies;
+  const LinArgs g = flags_args(M, N, K, trans_a, trans_b);
+  PackPlan p;
+  const bool packed = choose(g, dtype, true, ~(size_t)0, &p) == Way::Packed;
+  const size_t parts = stream_scratch(g, dtype);
+  return packed && p.bytes > parts ? p.bytes : parts;
 }
 
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
                     int trans_a, int trans_b, int64_t lda, int64_t ldb, int64_t ldo, void* workspace,
                     size_t workspace_bytes, void* stream) {
-  const bool scratch_ok = workspace && aligned(workspace, 256);
-  if (!trans_a && trans_b)
-    return forward(dtype, a, b, bias, out, M, N, K, lda, ldb, ldo, scratch_ok ? workspace : nullptr, scratch_ok ? workspace_bytes : 0, stream);
-  if (!scratch_ok) workspace = nullptr, workspace_bytes = 0;
+  if (!workspace || !aligned(workspace, 256)) workspace = nullptr, workspace_bytes = 0;
+  if (!trans_a && trans_b) return forward(dtype, a, b, bias, out, M, N, K, lda, ldb, ldo, workspace, workspace_bytes, stream);
   if (dtype != TTSDPA_F32 && dtype != TTSDPA_F16 && dtype != TTSDPA_BF16) return TTSDPA_ERR_DTYPE;
   if (M < 0 || N < 0 || K < 0) return TTSDPA_ERR_SHAPE;
   if (M == 0 || N == 0) return TTSDPA_OK;
@@ -1000,44 +1200,8 @@ int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, v
   const size_t esz = dtype == TTSDPA_F32 ? 4 : 2;
   if (!aligned(a, esz) || !aligned(b, esz) || !aligned(out, esz) || (bias && !aligned(bias, esz))) return TTSDPA_ERR_STRIDE;
   if ((M + 63) / 64 > 65535 || (N + 63) / 64 > 0x7fffffffLL) return TTSDPA_ERR_SHAPE;
-  hipStream_t s = (hipStream_t)stream;
-
-  const LinArgs g{a, b, bias, out, M, N, K, lda, ldb, ldo, trans_a ? 1 : 0, trans_b ? 0 : 1};
-  if (K > 0 && matmul_streams(g, dtype, workspace)) return launch_stream(g, dtype, s, 1, workspace, workspace_bytes);
-  if (in_place_ok(g, dtype)) return dtype == TTSDPA_F16 ? launch_mfma_t<F16>(g, s) : launch_mfma_t<BF16>(g, s);
-
-  // MFMA route: dense row-major copies of the operands that are stored contraction-major, then the x . w^T kernel
-  const size_t need = ttlinear_matmul_workspace_bytes(dtype, M, N, K, trans_a, trans_b);
-  if (K > 0 && workspace && workspace_bytes >= need) {
-    const void* x = a;
-    const void* w = b;
-    long long ldx = lda, ldw = ldb;
-    char* ws = (char*)workspace;
-    int route = TTLINEAR_ROUTE_NONE;
-    const void* xprobe = trans_a ? (const void*)ws : a;
-    const void* wprobe = !trans_b ? (const void*)(ws + (trans_a ? matmul_copy_bytes(dtype, M, K) : 0)) : b;
-    if (check(dtype, xprobe, wprobe, out, M, N, K, trans_a ? K : lda, !trans_b ? K : ldb, ldo, &route) == TTSDPA_OK &&
-        route == TTLINEAR_ROUTE_MFMA) {
-      int rc = 0;
-      if (trans_a) {  // a is [K, M]
-        rc = dtype == TTSDPA_F32 ? launch_transpose<float>(a, ws, K, M, lda, s) : launch_transpose<uint16_t>(a, ws, K, M, lda, s);
-        if (rc != 0) return rc;
-        x = ws, ldx = K;
-        ws += matmul_copy_bytes(dtype, M, K);
-      }
-      if (!trans_b) {  // b is [K, N]
-        rc = dtype == TTSDPA_F32 ? launch_transpose<float>(b, ws, K, N, ldb, s) : launch_transpose<uint16_t>(b, ws, K, N, ldb, s);
-        if (rc != 0) return rc;
-        w = ws, ldw = K;
-      }
-      return ttlinear_forward(dtype, x, w, bias, out, M, N, K, ldx, ldw, ldo, stream);
-    }
-  }
-  switch (dtype) {
-    case TTSDPA_F32: return launch_general_linear<float>(g, s, 1, workspace, workspace_bytes);
-    case TTSDPA_F16: return launch_general_linear<_Float16>(g, s, 1, workspace, workspace_bytes);
-    default: return launch_general_linear<__bf16>(g, s, 1, workspace, workspace_bytes);
-  }
+  return product(LinArgs{a, b, bias, out, M, N, K, lda, ldb, ldo, trans_a ? 1 : 0, trans_b ? 0 : 1}, dtype, workspace, workspace_bytes,
+                 (hipStream_t)stream);
 }
 
 int ttlinear_matmul_batched(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N,
@@ -1089,9 +1253,9 @@ int ttlinear_matmul_batched(int dtype, const void* a, const void* b, const void*
           sa % kpc == 0 && sb % kpc == 0 && out_batch_stride % 4 == 0 && !streams(g, dtype, (unsigned)entries)) {
         g.xt = g.wt = 0;
         switch (dtype) {
-          case TTSDPA_F32: return launch_mfma_tile<F32, 128, 128, 4, 2>(g, s, (unsigned)entries);
-          case TTSDPA_F16: return launch_mfma_tile<F16, 128, 128, 4, 2>(g, s, (unsigned)entries);
-          default: return launch_mfma_tile<BF16, 128, 128, 4, 2>(g, s, (unsigned)entries);
+          case TTSDPA_F32: return launch_small_tiles<F32>(g, s, (unsigned)entries);
+          case TTSDPA_F16: return launch_small_tiles<F16>(g, s, (unsigned)entries);
+          default: return launch_small_tiles<BF16>(g, s, (unsigned)entries);
         }
       }
       switch (dtype) {
@@ -1118,11 +1282,18 @@ int ttlinear_matmul_batched(int dtype, const void* a, const void* b, const void*
   return TTSDPA_OK;
 }
 
+// Ranges of rows that a packed grad^T's column sums come in.
+static long long pack_ranges(long long kpad) { return (kpad + kPackRows - 1) / kPackRows; }
+
 size_t ttlinear_backward_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const size_t gi = ttlinear_matmul_workspace_bytes(dtype, M, K, N, 0, 0), gw = ttlinear_matmul_workspace_bytes(dtype, N, K, M, 1, 0);
+  const LinArgs g = flags_args(N, K, M, 1, 0);
+  const size_t gi = ttlinear_matmul_workspace_bytes(dtype, M, K, N, 0, 0);
+  size_t gw = ttlinear_matmul_workspace_bytes(dtype, N, K, M, 1, 0);
+  PackPlan p;
+  if (choose(g, dtype, true, ~(size_t)0, &p) == Way::Packed) gw = p.bytes + (size_t)pack_ranges(p.kpad) * (size_t)N * sizeof(float);
   const size_t gb = (size_t)colsum_ranges(M, N, dtype) * (size_t)N * sizeof(float);
-  const size_t pair = stream_pair_scratch(flags_args(N, K, M, 1, 0), flags_args(M, K, N, 0, 0), dtype);
+  const size_t pair = stream_pair_scratch(g, flags_args(M, K, N, 0, 0), dtype);
   size_t most = gi > gw ? gi : gw;  // one after the other on the same scratch
   if (pair > most) most = pair;
   return most > gb ? most : gb;
@@ -1146,20 +1317,37 @@ int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w,
   const LinArgs gi{grad, w, nullptr, grad_x, M, K, N, ldg, ldw, K, 0, 1};
   // Small layers: both products, and the column sums with the weight's, in one launch.  Where the two would be launched
   // on the streaming kernel anyway and the launches saved (5 us, the column sums' among them) are worth more than what
-  // the common workgroup size may cost (64 x 784 x 500 fp32: 10 us in two launches and 5 for the column sums).
-  const bool gw_streams = matmul_streams(gw, dtype, true);
-  if (gw_streams && matmul_streams(gi, dtype, false) &&
-      stream_pair_cost(gw, gi, dtype) < stream_cost(gw, dtype, 1, true) + stream_cost(gi, dtype, 1, false) + 5) {
+  // the common workgroup size may cost (64 x 784 x 500 fp32: 10 us in two launches and 5 for the column sums); fp32, which
+  // the products bound, wherever it is estimated faster (1501 x 1999 x 2501: 322 us, on tiles with copies 381).
+  PackPlan pw, pi;
+  double us_w, us_i;
+  const Way way_w = choose(gw, dtype, true, workspace_bytes, &pw, &us_w);
+  const Way way_i = choose(gi, dtype, true, workspace_bytes, &pi, &us_i);
+  const bool pair = way_w == Way::Stream && way_i == Way::Stream;
+  if ((pair || (dtype == TTSDPA_F32 && stream_takes(gw, dtype) && stream_takes(gi, dtype))) &&
+      stream_pair_cost(gw, gi, dtype) < us_w + us_i + 5) {
     gw.rowsum = grad_b;
     return launch_stream_pair(gw, gi, dtype, s, workspace);
   }
-  int rc = ttlinear_matmul(dtype, grad, w, nullptr, grad_x, M, K, N, 0, 0, ldg, ldw, K, workspace, workspace_bytes, stream);
+  int rc = product(gi, dtype, workspace, workspace_bytes, s);
   if (rc != 0) return rc;
-  if (gw_streams) {
+  if (way_w == Way::Stream) {
     gw.rowsum = grad_b;
     return launch_stream(gw, dtype, s, 1, workspace, workspace_bytes);
   }
-  rc = ttlinear_matmul(dtype, grad, x, nullptr, grad_w, N, K, M, 1, 0, ldg, ldx, K, workspace, workspace_bytes, stream);
+  const long long sums = pack_ranges(pw.kpad);
+  if (way_w == Way::Packed && pw.x && workspace_bytes >= pw.bytes + (size_t)sums * (size_t)N * sizeof(float)) {
+    // the column sums come with the transposed copy
+    float* part = grad_b ? (float*)((char*)workspace + pw.bytes) : nullptr;
+    rc = launch_packed(gw, pw, dtype, s, (char*)workspace, part);
+    if (rc != 0 || !grad_b) return rc;
+    switch (dtype) {
+      case TTSDPA_F32: return launch_colsum_merge<float>(part, (int)sums, N, grad_b, s);
+      case TTSDPA_F16: return launch_colsum_merge<_Float16>(part, (int)sums, N, grad_b, s);
+      default: return launch_colsum_merge<__bf16>(part, (int)sums, N, grad_b, s);
+    }
+  }
+  rc = product(gw, dtype, workspace, workspace_bytes, s);
   if (rc != 0 || !grad_b) return rc;
   const int ranges = colsum_ranges(M, N, dtype);
   switch (dtype) {

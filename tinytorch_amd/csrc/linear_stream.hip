@@ -446,9 +446,10 @@ namespace {
 // Microseconds of a product on tiles of 16*R rows of x by 16*R of w, its contraction divided among S workgroups per tile, from
 // measurements (MI355X, 16-bit unless said): 3 us of launch, latency and the meeting of the partial sums (2 more on the
 // largest tile: a wavefront's sums are 16 KB); then, for each round of the 256 CUs, half a microsecond and the operands of
-// a tile at the 65 GB/s that a CU takes in (it measured 60-75 over all shapes; 16-bit k-major operands come in pieces of
+// a tile at the 65 GB/s that a CU takes in (it measured 60-75 over all shapes that the L2s hold or that are read once: when
+// both operands are larger, all tiles together take theirs in at 8 TB/s, 1636 x 3775 x 2025 100 us; 16-bit k-major operands come in pieces of
 // 32*R bytes, which costs 2.6, 1.6 and 1.1 times that), or the tile's products where those take longer (fp32: 0.45 TFLOP/s
-// of a CU's 0.61 on the largest tile, 0.3 on the others).  With S > 1 another launch and the partial products written and
+// of a CU's 0.61 on the largest tile while a CU has one, 0.36 with more, 0.3 on the others).  With S > 1 another launch and the partial products written and
 // read.
 //   measured / this: 1000^3 on 16, 32, 64: 25 / 26, 12 / 13, 9.5 / 9.4; 24 x 2048 x 5632: 7.4 / 9, 10.5 / 13, 19 / 21;
 //   64 x 4096 x 4096: 17 / 20, 11 / 12, 21 / 22; fp32 1000^3: 42 / 43, 30 / 32, 25 / 24; both k-major, 500 x 500 x 8192:
@@ -460,9 +461,12 @@ double stream_us(const LinArgs& a, int esz, int R, int S, double entries) {
   const double narrow = esz == 4 ? 1 : R == 1 ? 2.6 : R == 2 ? 1.6 : 1.1;
   const double k = (double)a.K / S;
   const double bytes = ((a.M < tm ? a.M : tm) * (a.xt ? narrow : 1) + (a.N < tn ? a.N : tn) * (a.wt ? narrow : 1)) * k * esz;
-  const double rate = esz == 2 ? 4e6 : R == 4 ? 0.45e6 : 0.3e6, flops = 2 * tm * tn * k;
+  const double rate = esz == 2 ? 4e6 : R < 4 ? 0.3e6 : rounds > 1.5 ? 0.36e6 : 0.45e6, flops = 2 * tm * tn * k;
   const double per = bytes / 65e3 > flops / rate ? bytes / 65e3 : flops / rate;
-  return (R == 4 ? 5 : 3) + rounds * (0.5 + per) + (S > 1 ? 3 + S * 8.0 * a.M * a.N / 4e6 : 0);
+  const double few = (double)(a.M < a.N ? a.M : a.N) * a.K * esz, all = (double)(a.M + a.N) * a.K * esz;
+  const double missed = few > 2e6 && all > 8e6 ? tiles * bytes / 8e6 : 0;
+  const double work = rounds * (0.5 + per);
+  return (R == 4 ? 5 : 3) + (work > missed ? work : missed) + (S > 1 ? 3 + S * 8.0 * a.M * a.N / 4e6 : 0);
 }
 
 // The cheapest tile (rows in blocks of 16: 1, 2 or 4, as far as a k-major operand has them; R = 0: none) and, when the caller
