@@ -65,3 +65,20 @@ def test_split_keys_with_per_batch_key_counts():
         assert rc == 0
         assert (out.float() - whole.float()).abs().max().item() <= 1e-2
         assert sampled_rows_err(out, host, causal, [(0, 1), (2, 3)], align="bottom-right", kv_len=lens) <= TOL["bf16"]
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("L,S", [(300, 2100), (512, 4096), (1100, 3000), (2048, 2048)])
+def test_split_sums(L, S, D):
+    """The sums of a causal call's splits: relative error of the whole output against float64.  A split that ends before the diagonal
+    must not count the keys behind its own (32 too many of 512 is an error of 6 %, hidden from absolute bounds by the small
+    means of long rows); 1e-3 is twice the rounding of probabilities and results to fp16."""
+    host, dev = make_inputs(77 + L, 1, 4, 2, L, S, D, "f16", 0.8)
+    q, k, v = (t.double() for t in dev)
+    k, v = k.repeat_interleave(2, 1), v.repeat_interleave(2, 1)
+    hidden = torch.arange(S, device="cuda")[None] > torch.arange(L, device="cuda")[:, None] + (S - L)
+    p = torch.softmax((q @ k.transpose(-1, -2).contiguous() / D ** 0.5).masked_fill(hidden, float("-inf")), -1)
+    rc, got = call("forward", *dev, causal=True, align="bottom-right")
+    assert rc == 0 and workspace_bytes(*dev, causal=True, align="bottom-right") > 0
+    ref = p @ v
+    assert ((got.double() - ref).norm() / ref.norm()).item() <= 1e-3

@@ -426,6 +426,9 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
     int t = my_halves / 2;
     const int f = S >= 96 ? (S - 32) / BN : 0;
     t = f < t ? f : t;
+    // the causal predicate hides the half behind this wavefront's last one where the diagonal ends its keys; where the
+    // split does, that half is another workgroup's: the last tile's exponentials would count it (from a stale K tile)
+    if (SPLIT && BN * ntiles_kv <= qc0 + WM - 1) t = ntiles_kv - 1 < t ? ntiles_kv - 1 : t;
     nfast_all = t > nfast ? t : nfast;
   }
   if (MASKB ? S < 160 : a.mask_kind != 0) nfast = 0, nfast_all = 0;  // other attnMasks are applied in the general form of a step
