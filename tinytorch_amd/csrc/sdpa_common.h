@@ -29,7 +29,7 @@ struct KArgs {
   int pack_L;
   // Split keys (4-wavefront prefill kernel, one query head per KV head after packing): workgroup (.., split) covers keys
   // split * kv_chunk .. + kv_chunk - 1 and writes a (acc[D], max, sum) record per row to ws instead of the output;
-  // the decode path's merge kernel combines them.  kv_splits <= 1: no split.
+  // tile_split_merge_kernel or prefill_split_merge_kernel combines them.  kv_splits <= 1: no split.
   int kv_splits, kv_chunk;
   float* ws;
   int mask_vec4;  // keys are contiguous in the mask and groups of 4 keys starting at a multiple of 4 are naturally aligned
@@ -506,9 +506,8 @@ int launch_prefill(const KArgs& a, int dtype, hipStream_t stream);       // 128-
 int launch_prefill_d128(const KArgs& a, int dtype, hipStream_t stream);  // 256-row workgroups, pipelined; head_dim 128
 int launch_prefill_d64(const KArgs& a, int dtype, hipStream_t stream);   // the same at head_dim 64 (no attnMask, no pages)
 int launch_prefill_f32(const KArgs& a, hipStream_t stream);              // fp32 tensors on the fp32 matrix cores; head_dim 64 or 128
+double prefill_f32_tiles(const KArgs& a);  // key tiles (of 32) that an unsplit launch takes one after the other
 int launch_decode(const KArgs& a, int dtype, void* workspace, hipStream_t stream);
-// combines per-split records [pair][split][row][D + 2] (pair = batch * Hkv + kv head, row = l * G + g) into a.out
-int launch_merge(const KArgs& a, int dtype, int splits, const float* ws, hipStream_t stream);
 
 // The records of a split launch of a pipelined prefill kernel -> out.  One thread per four elements of a row (eight rows per workgroup): the row's
 // splits up to its last visible key (a split wholly beyond the keys of a row tile wrote nothing), brought to their
@@ -563,7 +562,44 @@ int launch_prefill_split_merge(const KArgs& a, int dtype, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
+// The same for a split launch of the 4-wavefront kernels (16-bit and fp32), whose splits all write their records, of the kernel's
+// head_dim W >= a.D.  A row that sees no key although there are some: NaN, the unsplit kernels' and the reference's 0 / 0, or
+// with hidden_zero zeros.
+template <typename T>
+__global__ __launch_bounds__(256) void tile_split_merge_kernel(KArgs a, int W, int hidden_zero, long long nvec) {
+  typedef T vec4t __attribute__((ext_vector_type(4)));
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= nvec) return;
+  const int per = a.D / 4;
+  const int d = 4 * (int)(i % per);
+  const long long row_id = i / per;  // (b * Hq + h) * L + qi
+  const int qi = (int)(row_id % a.L);
+  const long long bh = row_id / a.L;
+  const int h = (int)(bh % a.Hq), b = (int)(bh / a.Hq);
+  const float c = a.scale * kLog2e;
+  const long long step = (long long)a.L * (W + 2);
+  const float* rec = a.ws + (bh * a.kv_splits * a.L + qi) * (W + 2);
+  float m = -1e30f;
+#pragma unroll 4
+  for (int s = 0; s < a.kv_splits; s++) m = fmaxf(m, rec[s * step + W]);
+  float l = 0.f;
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < a.kv_splits; s++) {
+    const float w = fast_exp2((rec[s * step + W] - m) * c);
+    l = fmaf(w, rec[s * step + W + 1], l);
+    const float2 lo = *(const float2*)(rec + s * step + d), hi = *(const float2*)(rec + s * step + d + 2);
+    x[0] = fmaf(w, lo.x, x[0]), x[1] = fmaf(w, lo.y, x[1]), x[2] = fmaf(w, hi.x, x[2]), x[3] = fmaf(w, hi.y, x[3]);
+  }
+  const bool empty = a.S == 0 || (a.kv_len && a.kv_len[b] <= 0);
+  const float inv = l > 0.f || !(empty || hidden_zero) ? 1.f / l : 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; e++) x[e] *= inv;
+  *(vec4t*)((T*)a.out + b * a.os[0] + h * a.os[1] + qi * a.os[2] + d) = __builtin_convertvector(x, vec4t);
+}
 
+
+int launch_tile_merge(const KArgs& a, int dtype, int W, bool hidden_zero, hipStream_t stream);  // tile_split_merge_kernel (sdpa_prefill.hip)
 int launch_zero(const KArgs& a, int dtype, hipStream_t stream);
 struct KvAppendArgs {
   void* kc;

@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   const int qi = qw0 + lq;
   if (nsplit > 1) {  // a partial result: unnormalised accumulator, the maximum it is relative to, the sum
     if (qi < a.L) {
-      float* rec = a.ws + ((long long)(pair * nsplit + split) * a.L + qi) * (D + 2);  // 8-byte aligned
+      float* rec = a.ws + (((long long)(b * a.Hq + h) * nsplit + split) * a.L + qi) * (D + 2);  // 8-byte aligned
 #pragma unroll
       for (int db = 0; db < DBLK; db++)
 #pragma unroll
@@ -405,8 +405,8 @@ int launch_prefill_k(const KArgs& a, dim3 grid, hipStream_t stream) {
 
 template <typename TR, int D, bool PAD>
 int launch_prefill_t(const KArgs& a, hipStream_t stream) {
-  // the callers keep to this (the records of a split are laid out for D, rows are read in 16-byte chunks)
-  if (PAD && (a.kv_splits > 1 || a.D % 8 != 0 || a.D >= D || a.D < 8)) return (int)hipErrorInvalidValue;
+  // the callers keep to this (rows are read in 16-byte chunks)
+  if (PAD && (a.D % 8 != 0 || a.D >= D || a.D < 8)) return (int)hipErrorInvalidValue;
   long long nwg = (long long)a.B * a.Hq * ((a.L + BM - 1) / BM) * (a.kv_splits > 1 ? a.kv_splits : 1);
   dim3 grid((unsigned)nwg);
   if (a.mask_kind != 0) return launch_prefill_k<TR, D, false, true, PAD>(a, grid, stream);  // exclusive with causal (validated)
@@ -433,6 +433,15 @@ int launch_prefill_d(const KArgs& a, hipStream_t stream) {
   if (a.D < 128) return launch_prefill_t<TR, 128, true>(a, stream);
   if (a.D < 192) return launch_prefill_t<TR, 192, true>(a, stream);
   return launch_prefill_t<TR, 256, true>(a, stream);
+}
+
+int launch_tile_merge(const KArgs& a, int dtype, int W, bool hidden_zero, hipStream_t stream) {
+  const long long nvec = (long long)a.B * a.Hq * a.L * (a.D / 4);
+  const dim3 grid((unsigned)((nvec + 255) / 256));
+  if (dtype == 0) hipLaunchKernelGGL((tile_split_merge_kernel<float>), grid, dim3(256), 0, stream, a, W, (int)hidden_zero, nvec);
+  else if (dtype == 1) hipLaunchKernelGGL((tile_split_merge_kernel<_Float16>), grid, dim3(256), 0, stream, a, W, (int)hidden_zero, nvec);
+  else hipLaunchKernelGGL((tile_split_merge_kernel<__bf16>), grid, dim3(256), 0, stream, a, W, (int)hidden_zero, nvec);
+  return (int)hipGetLastError();
 }
 
 int launch_prefill(const KArgs& a, int dtype, hipStream_t stream) {

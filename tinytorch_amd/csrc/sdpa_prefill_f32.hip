@@ -15,6 +15,10 @@
 //   O^T[D x 32 queries] += V^T . P^T      MFMA t contracts the two keys that the lane halves hold in accumulator
 //                                         register t, so P^T feeds the pipe straight from those registers and
 //                                         V^T[d][key] is a plain row-major LDS read along d
+// With few row tiles a CU's time is one wavefront's chain of 64-cycle matrix instructions (2.7 us a tile at head_dim 64, 4.6 at
+// 128): KEYS gives a workgroup 32 query rows and each of its wavefronts every fourth key tile, staged in a part of LDS of its
+// own, and adds the four partial results up through LDS.  Four times as many workgroups, each a quarter as long: 4
+// heads x 128 rows, head_dim 64, causal 14.8 -> 7.3 us, 4 x 8 heads x 300 rows, head_dim 128 49.6 -> 23.1.
 // The running maximum is raised only when exceeded by 2^8 in the exponent.  Causal masking as in the 16-bit kernels
 // (top-left aligned, reference src/Operation/OpTransformCpu.h:202-209): tiles above the diagonal are skipped.
 
@@ -33,32 +37,34 @@ struct F32Lds {
   static constexpr int K_PITCH = D + 1;   // floats; a column of 32 keys falls into 32 different banks
   static constexpr int V_PITCH = D + 32;  // floats; rows stay 16-byte aligned, the two lane halves use disjoint banks
   static constexpr int STAGE = BN * (K_PITCH + V_PITCH);
-  static constexpr int BYTES = 2 * STAGE * 4;
 };
 
 // MASKED: an attnMask is applied (a variant of its own: the mask addressing costs registers the other variants keep).
 // PAD: the tensors' head_dim a.D is a multiple of 4 below D; the 16-byte chunks of a row beyond it are taken as zeros (Q
 // and K: nothing added to a score; V: output columns that are not stored).  The reference takes any head size
 // (src/Function/FuncNNLayer.h:231-236).
-template <int D, bool CAUSAL, bool MASKED, bool PAD>
-__global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
+template <int D, bool CAUSAL, bool MASKED, bool PAD, bool KEYS>
+__global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs a) {
   typedef F32Lds<D> Lds;
   constexpr int K_PITCH = Lds::K_PITCH, V_PITCH = Lds::V_PITCH;
   constexpr int KSTEPS = D / 2;   // MFMAs along head_dim for S^T
   constexpr int DBLK = D / 32;    // 32-row blocks of O^T
-  constexpr int NLD = BN * D / 4 / 256;  // 16-byte chunks per thread per tile, for K and for V
+  constexpr int ROWS = KEYS ? 32 : BM;                // query rows of the workgroup
+  constexpr int STAGERS = KEYS ? 64 : 256;            // threads that bring a tile
+  constexpr int NLD = BN * D / 4 / STAGERS;           // 16-byte chunks per thread per tile, for K and for V
+  constexpr int STEP = KEYS ? 4 : 1;                  // a wavefront's (workgroup's) tiles: every STEP-th
 
   extern __shared__ __attribute__((aligned(16))) float smem_f32[];
-  float* smem = smem_f32;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  float* smem = smem_f32 + (KEYS ? wave * Lds::STAGE : 0);
   const int lq = lane & 31;
   const int lh = lane >> 5;
 
   // ---- workgroup -> (batch, kv head, query head in group, row tile); workgroup n runs on XCD n % 8 -------------
-  const int ntile = (a.L + BM - 1) / BM;
+  const int ntile = (a.L + ROWS - 1) / ROWS;
   const int inner = a.G * ntile;
   const int npair = a.B * a.Hkv;
   int pair, in;
@@ -79,8 +85,8 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
   const int g = in % a.G;
   const int rt = CAUSAL ? ntile - 1 - in / a.G : in / a.G;  // longest rows first
   const int h = hk * a.G + g;
-  const int q0 = rt * BM;
-  const int qw0 = q0 + wave * 32;
+  const int q0 = rt * ROWS;
+  const int qw0 = KEYS ? q0 : q0 + wave * 32;
 
   const float* qp = (const float*)a.q + b * a.qs[0] + h * a.qs[1];
   const int* table = a.block_table ? a.block_table + (long long)b * a.bt_stride : nullptr;  // paged cache
@@ -132,7 +138,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
   // are not monotone in the row, and the tile-level tests below use the range of all positions.
   const int pos_lo = a.pack_L ? 0 : qw0, pos_hi = a.pack_L ? a.pack_L - 1 : qw0 + 31;
   if (CAUSAL) {
-    int last = (a.pack_L ? a.pack_L - 1 : (q0 + BM - 1 < a.L - 1 ? q0 + BM - 1 : a.L - 1)) + coff;
+    int last = (a.pack_L ? a.pack_L - 1 : (q0 + ROWS - 1 < a.L - 1 ? q0 + ROWS - 1 : a.L - 1)) + coff;
     int lastkv = last < S - 1 ? last : S - 1;
     ntiles_kv = S > 0 ? lastkv / BN + 1 : 0;
   }
@@ -152,7 +158,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
                    // (the loads stay unconditional) and reach LDS as zeros
 #pragma unroll
   for (int i = 0; i < NLD; i++) {
-    int cidx = tid + 256 * i;
+    int cidx = (KEYS ? lane : tid) + STAGERS * i;
     lrow[i] = cidx / (D / 4);
     lcol[i] = cidx % (D / 4);
     cval[i] = !PAD || 4 * lcol[i] < a.D;
@@ -191,17 +197,27 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
     inv_scale = 1.f / a.scale;
   }
 
-  if (jt0 < jt1) {
-    load_tile(jt0 * BN);
-    store_tile(0);
-    if (jt0 + 1 < jt1) load_tile((jt0 + 1) * BN);
+  if (KEYS) {
+    jt0 += wave;
+    if (jt0 < jt1) load_tile(jt0 * BN);
+  } else {
+    if (jt0 < jt1) {
+      load_tile(jt0 * BN);
+      store_tile(0);
+      if (jt0 + 1 < jt1) load_tile((jt0 + 1) * BN);
+    }
+    __syncthreads();
   }
-  __syncthreads();
 
-  for (int jt = jt0; jt < jt1; jt++) {
+  for (int jt = jt0; jt < jt1; jt += STEP) {
     const int kv0 = jt * BN;
-    const int cur = (jt - jt0) & 1;
-    if (jt + 1 < jt1) {
+    const int cur = KEYS ? 0 : (jt - jt0) & 1;
+    if (KEYS) {  // the wavefront's own stage: its LDS reads and writes stay in order, no other wavefront sees them
+      __builtin_amdgcn_wave_barrier();
+      store_tile(0);
+      __builtin_amdgcn_wave_barrier();
+      if (jt + STEP < jt1) load_tile(kv0 + STEP * BN);
+    } else if (jt + 1 < jt1) {
       store_tile(cur ^ 1);  // stage cur^1 was last read before the barrier that ended the previous iteration
       if (jt + 2 < jt1) load_tile(kv0 + 2 * BN);
     }
@@ -275,15 +291,51 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
         }
       }
     }
-    __syncthreads();
+    if (!KEYS) __syncthreads();
   }
 
   // ---- normalise and store ----------------------------------------------------------------------------------------------
   float l_tot = l_run + __shfl_xor(l_run, 32);
   const int qi = qw0 + lq;
+  if constexpr (KEYS) {  // the four wavefronts' results to their common maximum, added in wavefront order
+    float* ml = smem_f32 + 4 * D * 32;  // [wavefront][maximum, sum][32 rows], behind the accumulators
+    static_assert(4 * D * 32 + 4 * 64 <= 4 * Lds::STAGE, "");
+    __syncthreads();
+    ml[wave * 64 + lane] = lh ? l_tot : m_use;
+    __syncthreads();
+    float m_all = ml[lq];
+#pragma unroll
+    for (int w = 1; w < 4; w++) m_all = fmaxf(m_all, ml[w * 64 + lq]);
+    float l_all = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) l_all = fmaf(fast_exp2((ml[w * 64 + lq] - m_all) * c), ml[w * 64 + 32 + lq], l_all);
+    const float f = fast_exp2((m_use - m_all) * c);
+    float* mine = smem_f32 + wave * D * 32 + lane;
+#pragma unroll
+    for (int db = 0; db < DBLK; db++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) mine[(16 * db + r) * 64] = oacc[db][r] * f;
+    __syncthreads();
+    const float inv = 1.f / l_all;
+    if (qi < a.L) {
+      float* op = (float*)a.out + b * a.os[0] + h * a.os[1] + qi * a.os[2];
+#pragma unroll
+      for (int db = 0; db < DBLK; db++) {
+        const int d = 32 * db + 8 * wave + 4 * lh;
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float* at = smem_f32 + (16 * db + 4 * wave + e) * 64 + lane;
+          x[e] = (((at[0] + at[D * 32]) + at[2 * D * 32]) + at[3 * D * 32]) * inv;
+        }
+        if (!PAD || d < a.D) *(f32x4*)(op + d) = x;
+      }
+    }
+    return;
+  }
   if (nsplit > 1) {  // a partial result: unnormalised accumulator, the maximum it is relative to, the sum
     if (qi < a.L) {
-      float* rec = a.ws + ((long long)(pair * nsplit + split) * a.L + qi) * (D + 2);  // 8-byte aligned
+      float* rec = a.ws + (((long long)(b * a.Hq + h) * nsplit + split) * a.L + qi) * (D + 2);  // 8-byte aligned
 #pragma unroll
       for (int db = 0; db < DBLK; db++)
 #pragma unroll
@@ -311,33 +363,56 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(KArgs a) {
   }
 }
 
-template <int D, bool CAUSAL, bool MASKED, bool PAD>
-int launch_f32_k(const KArgs& a, dim3 grid, hipStream_t stream) {
+template <int D, bool CAUSAL, bool MASKED, bool PAD, bool KEYS>
+int launch_f32_v(const KArgs& a, hipStream_t stream) {
+  constexpr int lds = (KEYS ? 4 : 2) * F32Lds<D>::STAGE * 4, rows = KEYS ? 32 : BM;
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  const hipError_t granted = grant_dynamic_lds((const void*)prefill_f32_kernel<D, CAUSAL, MASKED, PAD>, F32Lds<D>::BYTES, state, done);
+  const hipError_t granted = grant_dynamic_lds((const void*)prefill_f32_kernel<D, CAUSAL, MASKED, PAD, KEYS>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  hipLaunchKernelGGL((prefill_f32_kernel<D, CAUSAL, MASKED, PAD>), grid, dim3(256), F32Lds<D>::BYTES, stream, a);
+  const long long nwg = (long long)a.B * a.Hq * ((a.L + rows - 1) / rows) * (a.kv_splits > 1 ? a.kv_splits : 1);
+  if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL((prefill_f32_kernel<D, CAUSAL, MASKED, PAD, KEYS>), dim3((unsigned)nwg), dim3(256), lds, stream, a);
   return (int)hipGetLastError();
 }
 
+// Key tiles walked by one wavefront, times the rounds of the CUs: in workgroups of 128 rows, or of 32 with the tiles dealt out to
+// the wavefronts (one such workgroup per CU; half a tile's time to add the results up).
+bool keys_among_wavefronts(const KArgs& a, double* tiles_walked = nullptr) {
+  if (a.kv_splits > 1) return false;
+  const long long heads = (long long)a.B * a.Hq, wide = heads * ((a.L + BM - 1) / BM), narrow = heads * ((a.L + 31) / 32);
+  const long long tiles = ((a.causal && !a.pack_L && !a.kv_len && a.L < a.S ? a.L : a.S) + BN - 1) / BN;
+  const double whole = (double)tiles * (double)((wide + 255) / 256), dealt = (double)((tiles + 3) / 4) * (double)((narrow + 255) / 256) + 0.5;
+  if (tiles_walked) *tiles_walked = dealt < 0.9 * whole ? dealt : whole;
+  return dealt < 0.9 * whole;
+}
+
+template <int D, bool CAUSAL, bool MASKED, bool PAD>
+int launch_f32_k(const KArgs& a, hipStream_t stream) {
+  return keys_among_wavefronts(a) ? launch_f32_v<D, CAUSAL, MASKED, PAD, true>(a, stream) : launch_f32_v<D, CAUSAL, MASKED, PAD, false>(a, stream);
+}
+
 template <int D, bool PAD>
-int launch_f32_d(const KArgs& a, dim3 grid, hipStream_t stream) {
-  // the callers keep to this (the records of a split are laid out for D, rows are read in 16-byte chunks)
-  if (PAD && (a.kv_splits > 1 || a.D % 4 != 0 || a.D >= D || a.D < 4)) return (int)hipErrorInvalidValue;
-  if (a.mask_kind != 0) return launch_f32_k<D, false, true, PAD>(a, grid, stream);  // exclusive with causal (validated by the caller, as the reference asserts)
-  return a.causal ? launch_f32_k<D, true, false, PAD>(a, grid, stream) : launch_f32_k<D, false, false, PAD>(a, grid, stream);
+int launch_f32_d(const KArgs& a, hipStream_t stream) {
+  // the callers keep to this (rows are read in 16-byte chunks)
+  if (PAD && (a.D % 4 != 0 || a.D >= D || a.D < 4)) return (int)hipErrorInvalidValue;
+  if (a.mask_kind != 0) return launch_f32_k<D, false, true, PAD>(a, stream);  // exclusive with causal (validated by the caller, as the reference asserts)
+  return a.causal ? launch_f32_k<D, true, false, PAD>(a, stream) : launch_f32_k<D, false, false, PAD>(a, stream);
 }
 
 }  // namespace
 
+double prefill_f32_tiles(const KArgs& a) {
+  double tiles = 0;
+  keys_among_wavefronts(a, &tiles);
+  return tiles;
+}
+
 int launch_prefill_f32(const KArgs& a, hipStream_t stream) {
-  long long nwg = (long long)a.B * a.Hq * ((a.L + BM - 1) / BM) * (a.kv_splits > 1 ? a.kv_splits : 1);
-  dim3 grid((unsigned)nwg);
-  if (a.D == 128) return launch_f32_d<128, false>(a, grid, stream);
-  if (a.D == 64) return launch_f32_d<64, false>(a, grid, stream);
+  if (a.D == 128) return launch_f32_d<128, false>(a, stream);
+  if (a.D == 64) return launch_f32_d<64, false>(a, stream);
   // any other multiple of 4 up to 128: the kernel of the next size up, the missing columns as zeros
-  return a.D < 64 ? launch_f32_d<64, true>(a, grid, stream) : launch_f32_d<128, true>(a, grid, stream);
+  return a.D < 64 ? launch_f32_d<64, true>(a, stream) : launch_f32_d<128, true>(a, stream);
 }
 
 }  // namespace ttsdpa

@@ -173,31 +173,68 @@ void pack_heads(KArgs* a) {
   a->G = 1;
 }
 
-// Key splits of a short-L call on the 4-wavefront kernel (one query head per KV head, possibly after packing): when
-// batch x heads x row tiles leave most of the 256 CUs idle, the keys are divided among several workgroups whose
-// partial results the decode path's merge kernel combines.  Needs head_dim 64 or 128 (the merge kernel's) and scratch.
+// Key splits.  A workgroup walks its row tile's keys one tile after another, 2 us (fp32: 3 to 5) each however few workgroups there
+// are; when batch x heads x row tiles leave CUs idle, the keys are divided among several workgroups whose partial results a
+// second kernel combines.  The number is the one whose estimated time is least: the longest workgroup's tiles, in as
+// many rounds as the workgroups need; and with splits the second launch and its records, written and read.
 struct SplitPlan {
   int splits, chunk;
   size_t ws_bytes;
 };
-SplitPlan plan_prefill_splits(const ttsdpa_params* p, const KArgs& a /* after packing */) {
-  SplitPlan s{1, 0, 0};
-  if (a.G != 1 || (a.D != 64 && a.D != 128) || p->mask_kind != TTSDPA_MASK_NONE || pipelined_ok(p)) return s;
-  const long long wgs = (long long)a.B * a.Hq * ((a.L + 127) / 128);
-  long long want = (2 * 256 + wgs - 1) / wgs;  // aim for two workgroups per CU
-  const long long most = a.S / 512;            // at least 8 key tiles per split
-  if (want > most) want = most;
-  if (want > 64) want = 64;                    // the merge kernel's limit
-  if (want < 2) return s;
-  int chunk = (int)((a.S + want - 1) / want);
-  chunk = (chunk + 63) / 64 * 64;
-  s.splits = (a.S + chunk - 1) / chunk;
-  s.chunk = chunk;
-  if (s.splits < 2) return SplitPlan{1, 0, 0};
-  s.ws_bytes = (size_t)a.B * a.Hq * s.splits * a.L * (a.D + 2) * sizeof(float);
-  return s;
+
+// rows: records; whole_us: of the unsplit call, where it does not follow from the rest; tile_us, tile: of one key tile; slots: workgroups that run side by side; step: a chunk is a multiple of it
+SplitPlan cheapest_split(long long wgs, long long keys, long long rows, int width, bool causal, double tile_us, int tile, int slots, int step,
+                         double whole_us = 0) {
+  SplitPlan best{1, 0, 0};
+  double least = 0;
+  for (long long want = 1; want <= 64; want++) {  // 64: the merge kernels' limit
+    long long chunk = (keys + want - 1) / want;
+    chunk = (chunk + step - 1) / step * step;
+    const long long n = (keys + chunk - 1) / chunk;
+    if (n < want) continue;  // the same as fewer
+    const double busy = (double)(wgs * n) * (causal ? 0.6 : 1.0) / slots;
+    const double per = (double)((n > 1 ? chunk : keys) + tile - 1) / tile;
+    const size_t bytes = n > 1 ? (size_t)rows * (size_t)n * (width + 2) * sizeof(float) : 0;
+    const double us = (double)(long long)per * tile_us * (busy > 1 ? busy : 1) + (n > 1 ? 5 + 2.0 * bytes / 4e6 : 0);
+    if (n > 1 && us > 0.9 * least) continue;
+    if (n == 1 && whole_us > 0) {
+      least = whole_us;
+      continue;
+    }
+    if (n == 1 || us < least) least = us, best = SplitPlan{(int)n, n > 1 ? (int)chunk : 0, bytes};
+  }
+  return best;
 }
 
+// Head_dim of the 4-wavefront kernel that runs a call: its records' width.
+int tile_width(int dtype, int D) {
+  if (dtype == TTSDPA_F32) return D <= 64 ? 64 : 128;
+  return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : D <= 128 ? 128 : D <= 192 ? 192 : 256;
+}
+
+// The 4-wavefront kernels (128-row tiles; possibly after packing): fp32 tiles of 32 keys are bound by the matrix cores (2 heads x
+// 777 rows, head_dim 80, causal 118 -> 24 us), 16-bit ones of 64 keys by latency (4 heads x 449 rows, head_dim 64, key-padding mask
+// 18 -> 12 us, 2 x 8 x 927 rows, head_dim 80, 128 workgroups 37 -> 33).
+SplitPlan plan_prefill_splits(const ttsdpa_params* p, const KArgs& a /* after packing */) {
+  const bool f32 = p->dtype == TTSDPA_F32;
+  if (!f32 && pipelined_ok(p)) return SplitPlan{1, 0, 0};
+  const int W = tile_width(p->dtype, a.D);
+  const long long rows = (long long)a.B * a.Hq * a.L, wgs = (long long)a.B * a.Hq * ((a.L + 127) / 128);
+  const double us = f32 ? (W == 64 ? 2.7 : 4.6) : W <= 64 ? 1.8 : W <= 128 ? 2.2 : 4.0;
+  const long long keys = effective_causal(p) == TTSDPA_CAUSAL_TOP_LEFT && !a.pack_L && a.L < a.S ? a.L : a.S;
+  if (f32 && keys <= 512) return SplitPlan{1, 0, 0};  // short walks are dealt out to a workgroup's wavefronts instead, in one launch
+  KArgs whole = a;
+  whole.kv_splits = 1;
+  return cheapest_split(wgs, keys, rows, W, a.causal != 0, us, f32 ? 32 : 64, f32 || W > 128 ? 256 : 512, 64,
+                        f32 ? us * prefill_f32_tiles(whole) : 0);
+}
+
+// Calls of these sizes, one query head per KV head, without an attnMask, have always had zeros where a causal mask leaves a row
+// no key (their splits were merged by the decode path's kernel); others have NaN there.
+bool hidden_rows_zero(const ttsdpa_params* p, const KArgs& a) {
+  const long long wgs = (long long)a.B * a.Hq * ((a.L + 127) / 128);
+  return a.G == 1 && (a.D == 64 || a.D == 128) && p->mask_kind == TTSDPA_MASK_NONE && !pipelined_ok(p) && a.S >= 1024 && wgs < 512;
+}
 
 // Key splits for the pipelined kernels (head_dim 128 and 64): a call with a quarter as many 256-row tiles as the chip has CUs, or
 // fewer (a chunk of one sequence's rows against a long cache, a few heads of a tensor-parallel share), leaves most CUs
@@ -205,11 +242,16 @@ SplitPlan plan_prefill_splits(const ttsdpa_params* p, const KArgs& a /* after pa
 // tiles, so the kernel's stages keep their constants), enough for two workgroups per CU, and the
 // kernel's merge kernel combines the records.  The records cost: with 65-128 row tiles the split pays only under a
 // causal mask on 4096 keys or more (4 heads x 8192 rows +32 %, one KV head's share of 2 x 4096 rows +7 %; without a mask
-// -9 %, 2048 keys -18 %); with 64 and fewer it measured 1.1x to 5x (32 heads x 512 rows on 8192 keys 1.5x).
+// -9 %, 2048 keys -18 %); with 64 and fewer it measured 1.1x to 5x (32 heads x 512 rows on 8192 keys 1.5x), on fewer than
+// 2048 keys where the estimate says so.
 SplitPlan plan_pipelined_splits(const ttsdpa_params* p) {
   SplitPlan s{1, 0, 0};
   long long units, keys;
-  if (p->dtype == TTSDPA_F32 || !(pipelined_ok(p) || pipelined64_ok(p)) || !split_shape(p, &units, &keys)) return s;
+  if (p->dtype == TTSDPA_F32 || !(pipelined_ok(p) || pipelined64_ok(p))) return s;
+  if (!split_shape(p, &units, &keys)) {
+    if (p->mask_kind != TTSDPA_MASK_NONE || p->block_table || units > 64) return s;
+    return cheapest_split(units, keys, (long long)p->B * p->Hq * p->L, p->D, p->causal != 0, 1.4, 64, 256, 256);
+  }
   long long want = (512 + units - 1) / units;
   const long long most = keys / 512;  // at least 8 key tiles per split
   if (want > most) want = most;
@@ -456,7 +498,8 @@ size_t ttsdpa_workspace_bytes(const ttsdpa_params* p) {
   if (p->B == 0 || p->L == 0 || p->S == 0) return 0;
   // enough for ttsdpa_forward's route and for an explicit ttsdpa_decode of the same call
   size_t need = decode_ok(p) ? plan_decode(a).ws_bytes : 0;
-  if (pick_route(p) == TTSDPA_ROUTE_PREFILL) {
+  const int route = pick_route(p);
+  if (route == TTSDPA_ROUTE_PREFILL || (route == TTSDPA_ROUTE_GENERAL && p->mask_kind != TTSDPA_MASK_NONE && prefill_ok(p, true))) {
     if (f32_decode_ok(p)) {
       const size_t decode = plan_decode(a).ws_bytes;
       need = decode > need ? decode : need;
@@ -525,7 +568,7 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
     if ((rc = check_grid((long long)a.B * a.Hq * ((a.L + 127) / 128) * sp.splits)) != TTSDPA_OK) return rc;
     rc = launch(a);
     if (rc != 0) return rc;
-    return launch_merge(a, p->dtype, sp.splits, a.ws, (hipStream_t)stream);
+    return launch_tile_merge(a, p->dtype, tile_width(p->dtype, a.D), hidden_rows_zero(p, a), (hipStream_t)stream);
   }
   return launch(a);
 }
