@@ -84,7 +84,7 @@ __device__ __forceinline__ void load_half_row(const float* row, int lh, float (&
 // MASKED: an attnMask (exclusive with CAUSAL), as in the forward kernel.
 // PAD (both kernels): the tensors' head_dim f.D is a multiple of 4 below D.  The 16-byte chunks of a row beyond it are
 // taken as zeros (q, k: nothing added to a score; dout, v: nothing added to dP or delta; gradient columns beyond f.D are
-// not stored); everything else is the kernel for head_dim D.  No splits (their records are laid out for D).
+// not stored, records of splits hold f.D of them); everything else is the kernel for head_dim D.
 template <int D, bool CAUSAL, bool MASKED, bool PAD>
 __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dq_f32_kernel(BwdArgs a) {
   typedef BwdF32Lds<D> Lds;
@@ -327,8 +327,8 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED ? 1 : 2)) void backward_dkv_
   float* dkp = (float*)a.dk + b * a.dks[0] + hk * a.dks[1] + key * a.dks[2];
   float* dvp = (float*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + key * a.dvs[2];
   if (nsplit > 1) {  // partial sums: dense [split][dk | dv][B][Hkv][S][D]
-    const long long plane = (long long)f.B * f.Hkv * f.S * D;
-    dkp = a.partial + 2 * split * plane + (((long long)b * f.Hkv + hk) * f.S + key) * D;
+    const long long plane = (long long)f.B * f.Hkv * f.S * have;
+    dkp = a.partial + 2 * split * plane + (((long long)b * f.Hkv + hk) * f.S + key) * have;
     dvp = dkp + plane;
   }
   if (k0 >= S) {  // keys no query row attends to (at or beyond the batch entry's key count): zeros
@@ -500,8 +500,8 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED ? 1 : 2)) void backward_dkv_
 template <int D, bool CAUSAL, bool MASKED, bool PAD>
 int launch_k(const BwdArgs& args, hipStream_t stream) {
   BwdArgs a = args;
-  // the callers keep to this (the records of a split are laid out for D, rows are read in 16-byte chunks)
-  if (PAD && (a.dkv_splits > 1 || a.dq_splits > 1 || a.f.D % 4 != 0 || a.f.D >= D || a.f.D < 4)) return (int)hipErrorInvalidValue;
+  // the callers keep to this (rows are read in 16-byte chunks)
+  if (PAD && (a.f.D % 4 != 0 || a.f.D >= D || a.f.D < 4)) return (int)hipErrorInvalidValue;
   static hipError_t state1[kMaxDevices], state2[kMaxDevices];
   static bool done1[kMaxDevices], done2[kMaxDevices];
   hipError_t e = grant_dynamic_lds((const void*)backward_dq_f32_kernel<D, CAUSAL, MASKED, PAD>, BwdF32Lds<D>::BYTES, state1, done1);

@@ -70,15 +70,16 @@ __device__ __forceinline__ vec8 transposed_operand(const void* lane_base, int by
 // A lane's share of the dk / dv rows of key `key` (accumulator layout: registers 4rg .. 4rg+3 of block db are elements
 // 32db + 8rg + 4lh .. +3) goes to the gradient tensors, or — when the key block's query stream is split over several
 // workgroups — as fp32 to this split's partial sums, dense [split][dk | dv][B][Hkv][S][D].
-// PAD: the tensors' head_dim a.f.D is a multiple of 8 below D; only its columns are written (no splits then).
+// PAD: the tensors' head_dim a.f.D is a multiple of 8 below D; only its columns are written.
 template <typename TR, int D, bool PAD = false>
 __device__ __forceinline__ void store_key_grads(const BwdArgs& a, int split, int b, int hk, int key, int lh,
                                                 const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32], float scale) {
   typedef typename TR::elem T;
   if (key >= a.f.S) return;
   if (a.dkv_splits > 1) {
-    const long long plane = (long long)a.f.B * a.f.Hkv * a.f.S * D;
-    float* dkp = a.partial + 2 * split * plane + (((long long)b * a.f.Hkv + hk) * a.f.S + key) * D;
+    const int have = PAD ? a.f.D : D;
+    const long long plane = (long long)a.f.B * a.f.Hkv * a.f.S * have;
+    float* dkp = a.partial + 2 * split * plane + (((long long)b * a.f.Hkv + hk) * a.f.S + key) * have;
 #pragma unroll
     for (int db = 0; db < D / 32; db++)
 #pragma unroll
@@ -86,6 +87,7 @@ __device__ __forceinline__ void store_key_grads(const BwdArgs& a, int split, int
         f32x4 x, y;
 #pragma unroll
         for (int i = 0; i < 4; i++) x[i] = dkacc[db][4 * rg + i] * scale, y[i] = dvacc[db][4 * rg + i];
+        if (PAD && 32 * db + 8 * rg + 4 * lh >= have) continue;
         *(f32x4*)(dkp + 32 * db + 8 * rg + 4 * lh) = x;
         *(f32x4*)(dkp + plane + 32 * db + 8 * rg + 4 * lh) = y;
       }
@@ -131,8 +133,8 @@ __device__ __forceinline__ vec8 regs_to_operand(const f32x16& acc, int t) {
 // MASKED: an attnMask (exclusive with CAUSAL), as in the forward kernels.
 // PAD (both register-staged kernels): the tensors' head_dim f.D is a multiple of 8 below D.  The 16-byte chunks of a row
 // beyond it are taken as zeros (q, k: nothing added to a score; dout, v: nothing added to dP or delta; the gradients'
-// columns beyond f.D are not stored); everything else is the kernel for head_dim D.  No splits (their records are laid
-// out for D).
+// columns beyond f.D are not stored); everything else is the kernel for head_dim D (records of splits hold f.D
+// columns).
 template <typename TR, int D, bool CAUSAL, bool MASKED, bool PAD>
 __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
   constexpr int BN = DqTile<D>::BN;
@@ -1096,8 +1098,8 @@ __global__ __launch_bounds__(256, 2) void backward_dq128_kernel(BwdArgs a) {
 template <typename TR, int D, bool CAUSAL, bool MASKED, bool PAD>
 int launch_k(const BwdArgs& args, hipStream_t stream) {
   BwdArgs a = args;
-  // the callers keep to this (the records of a split are laid out for D, rows are read in 16-byte chunks)
-  if (PAD && (a.dkv_splits > 1 || a.dq_splits > 1 || a.f.D % 8 != 0 || a.f.D >= D || a.f.D < 8)) return (int)hipErrorInvalidValue;
+  // the callers keep to this (rows are read in 16-byte chunks)
+  if (PAD && (a.f.D % 8 != 0 || a.f.D >= D || a.f.D < 8)) return (int)hipErrorInvalidValue;
   typedef BwdLds<D> Lds;
   // with an attnMask, head_dim 128 takes the register-staged dk/dv kernel: the mask's 16 values per tile do not fit the
   // 256 registers of the direct-to-LDS one

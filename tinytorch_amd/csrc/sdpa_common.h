@@ -274,6 +274,22 @@ struct BwdArgs {
   int dkv_round;
 };
 
+// Splits of a backward launch that would leave half of the chip idle with `n`: its workgroups walk their streams tile by tile,
+// tile_us each, however few they are.  The number, up to 16, whose longest stream, second launch and partial records (record_us
+// for each split, written and read) take least by estimate: bf16 2 x 4 heads on 1 x 199 rows, head_dim 128: whole backward 50 -> 37 us;
+// fp32 8 heads on 1 x 2000 x 2000, head_dim 64: 665 -> 257.
+inline int cheapest_backward_splits(int n, long long wgs, long long tiles, long long slots, double tile_us, double record_us) {
+  if (wgs * n * 2 > slots) return n;
+  auto us = [&](int k) {
+    const double rounds = wgs * k > slots ? (double)(wgs * k) / (double)slots : 1.0;
+    return (double)((tiles + k - 1) / k) * tile_us * rounds + (k > 1 ? 4.5 + k * record_us : 0.0);
+  };
+  int best = n;
+  for (int k = n + 1; k <= 16; k++)
+    if (us(k) < 0.9 * us(best)) best = k;
+  return best;
+}
+
 // Workgroups that share a key block in the matrix-core dk/dv kernels (1: none, the kernel writes dk / dv itself).
 // A dk/dv workgroup owns 128 keys and about one runs per CU at a time; under a causal mask its length varies
 // 1 : (number of key blocks), and below about four workgroups per CU the longest ones set the time.  Without a causal
@@ -283,7 +299,7 @@ struct BwdArgs {
 // workgroups of a causal call further measured 4 % slower, 256 of them 7-21 % faster).
 // `per_cu`: workgroups of the kernel that fit a CU (2 at head_dim 64 without an attnMask, else 1): head_dim 64, 256 equal
 // workgroups without a causal mask: two splits +28 %; causal with 512: four splits instead of two -2 to -5 %.
-inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, bool causal, int groups, int per_cu) {
+inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, int D, bool causal, int groups, int per_cu, bool f32) {
   const long long wgs = (long long)B * Hkv * ((S + 127) / 128) * groups;
   const long long tiles = (long long)(Hq / Hkv) * ((L + 31) / 32) / groups;  // the longest query stream, in 32-row tiles
   // causal: two rounds of the workgroups a CU holds at a time (one for the 8-wavefront head_dim-128 kernel, whose two
@@ -292,8 +308,9 @@ inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, bool causal
   // third kernel for the partial sums; 256 of them (2048 x 2048) two splits 76.5, four 74.1 TFLOP/s.
   const long long enough = causal ? 512LL * per_cu * groups : 256 * per_cu;
   int n = 1;
-  while (n < 4 && wgs * n < enough && tiles >= 16 * n) n *= 2;
-  return n;
+  while (n < 4 && wgs * n < enough && tiles >= 16 * n && (D == 64 || D == 128)) n *= 2;  // (measured for these two sizes)
+  const double record_us = (double)B * Hkv * S * D * 16 / 4e6, tile_us = f32 ? (D <= 64 ? 5.0 : 10.0) : D <= 64 ? 1.15 : 2.0;
+  return cheapest_backward_splits(n, wgs / groups, tiles, 256 * per_cu, tile_us, record_us);
 }
 
 // Workgroups that share a 128-row query block in the matrix-core dq kernels (1: none, the kernel writes dq itself).
@@ -304,14 +321,15 @@ inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, bool causal
 // without a mask +22 %; 512 causal workgroups split in two measured 5 % slower: the partial records cost more than the
 // uneven end).  A split must still get a few hundred keys.
 // `slots`: workgroups of the kernel the chip holds at a time (512; 256 for the fp32 kernel at head_dim 128).
-inline int backward_dq_splits(int B, int Hq, int L, int S, bool causal, int slots) {
+inline int backward_dq_splits(int B, int Hq, int L, int S, int D, bool causal, int slots, bool f32) {
   const long long wgs = (long long)B * Hq * ((L + 127) / 128);
   const long long tiles = (S + 31) / 32;  // the longest key range, in 32-key tiles
   if (wgs >= slots) return 1;
   const long long enough = causal ? 2 * slots : slots;
   int n = 1;
-  while (n < 8 && wgs * n < enough && tiles >= 16 * n) n *= 2;
-  return n;
+  while (n < 8 && wgs * n < enough && tiles >= 16 * n && (D == 64 || D == 128)) n *= 2;
+  const double record_us = (double)B * Hq * L * D * 8 / 4e6, tile_us = f32 ? (D <= 64 ? 4.0 : 8.0) : D <= 64 ? 0.9 : 1.4;
+  return cheapest_backward_splits(n, wgs, tiles, slots, tile_us, record_us);
 }
 
 // Workgroup id of a dk/dv launch with split query streams -> (key-block workgroup n, split).  The hardware hands
@@ -364,7 +382,8 @@ template <int D>
 __device__ __forceinline__ void store_dq_partial(const BwdArgs& a, int piece, long long row_id, int lh, const f32x16 (&dqacc)[D / 32],
                                                  float mc, float l_tot, float delta) {
   const long long rows = (long long)a.f.B * a.f.Hq * a.f.L;
-  float* dst = a.dq_partial + (piece * rows + row_id) * D;
+  const int have = a.f.D;  // D, or fewer (the zero-column kernels)
+  float* dst = a.dq_partial + (piece * rows + row_id) * have;
 #pragma unroll
   for (int db = 0; db < D / 32; db++)
 #pragma unroll
@@ -372,10 +391,10 @@ __device__ __forceinline__ void store_dq_partial(const BwdArgs& a, int piece, lo
       f32x4 x;
 #pragma unroll
       for (int i = 0; i < 4; i++) x[i] = dqacc[db][4 * rg + i];
-      *(f32x4*)(dst + 32 * db + 8 * rg + 4 * lh) = x;
+      if (32 * db + 8 * rg + 4 * lh < have) *(f32x4*)(dst + 32 * db + 8 * rg + 4 * lh) = x;
     }
   if (lh == 0) {
-    float* ml = a.dq_partial + a.dq_splits * rows * D;
+    float* ml = a.dq_partial + a.dq_splits * rows * have;
     *(float2*)(ml + 2 * (piece * rows + row_id)) = make_float2(mc, l_tot);
     if (piece == 0) a.stats[2 * row_id + 1] = delta;
   }

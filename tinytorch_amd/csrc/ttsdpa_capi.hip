@@ -304,7 +304,7 @@ int pick_route(const ttsdpa_params* p) {
     // 9-16 rows per KV head: the streaming kernel does P.V on the vector ALUs and measures 5.5 TB/s there; the
     // 4-wavefront MFMA kernel with packed heads and split keys 5.85 TB/s, when the call allows it
     const long long rows = (long long)p->L * (p->Hq / p->Hkv);
-    // (head_dim 64 / 128: the zero-column variants of that kernel do not split their keys)
+    // (measured at head_dim 64 / 128; the sizes between keep to the streaming kernel)
     if (rows > 8 && (p->D == 64 || p->D == 128) && prefill_ok(p) && !pipelined_ok(p) && (p->Hq == p->Hkv || pack_heads_ok(p)))
       return TTSDPA_ROUTE_PREFILL;
     return TTSDPA_ROUTE_DECODE;
@@ -387,18 +387,16 @@ size_t backward_stats_bytes(const ttsdpa_backward_params* p) {
 int dkv_splits_of(const ttsdpa_backward_params* p) {
   const ttsdpa_params* f = &p->fwd;
   if (!backward_on_mfma(p)) return 1;
-  if (f->D != 64 && f->D != 128) return 1;  // the zero-column variants do not split (their records are laid out for 64 / 128)
   const int groups = f->dtype != TTSDPA_F32 && f->D == 128 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
-  const int per_cu = f->D == 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
-  return backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, effective_causal(f) != TTSDPA_CAUSAL_NONE, groups, per_cu);
+  const int per_cu = f->D <= 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
+  return backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, groups, per_cu, f->dtype == TTSDPA_F32);
 }
 // ... then (matrix-core pairs whose dq kernel splits its key ranges) the partial dq records, 256-byte aligned.
 int dq_splits_of(const ttsdpa_backward_params* p) {
   const ttsdpa_params* f = &p->fwd;
   if (!backward_on_mfma(p)) return 1;
-  if (f->D != 64 && f->D != 128) return 1;
-  const int slots = f->dtype == TTSDPA_F32 && f->D == 128 ? 256 : 512;
-  return backward_dq_splits(f->B, f->Hq, f->L, f->S, effective_causal(f) != TTSDPA_CAUSAL_NONE, slots);
+  const int slots = f->dtype == TTSDPA_F32 && f->D > 64 ? 256 : 512;
+  return backward_dq_splits(f->B, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, slots, f->dtype == TTSDPA_F32);
 }
 size_t backward_partial_offset(const ttsdpa_backward_params* p) { return (backward_stats_bytes(p) + 255) & ~(size_t)255; }
 size_t backward_dq_partial_offset(const ttsdpa_backward_params* p) {
