@@ -108,9 +108,10 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
   const int vc = lane % CH;   // value lanes: 16-byte chunk of the row
   const int vph = lane / CH;  // value lanes: key phase
 
-  int n = blockIdx.x;
-  const int split = n % splits;
-  n /= splits;
+  // Workgroup i runs on XCD i % 8: the splits of neighbouring pairs begin at different XCDs, so that sequences too short for
+  // all of theirs do not leave the same XCDs idle.
+  int n = blockIdx.x / splits;
+  const int split = (int)((blockIdx.x + n) % splits);
   const int hk = n % a.Hkv;
   const int b = n / a.Hkv;
   const int rows = a.L * a.G;  // query rows sharing this KV head, row x = (l, g) = (x / G, x % G)
@@ -118,6 +119,10 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
   if (a.kv_len) {
     int len = a.kv_len[b];
     S = len < 0 ? 0 : (len < S ? len : S);
+    // a sequence's own keys over all of its splits (24 sequences of 1000 .. 3000 keys, 4 KV heads: with the longest one's
+    // chunk 32.3 us, the short ones' work on the first splits' XCDs; 25.8 so)
+    const int own = (S + splits * NWAVE * KB - 1) / (splits * NWAVE * KB) * (NWAVE * KB);
+    chunk = own < chunk ? own : chunk;
   }
 
   const T* kp = (const T*)a.k + b * a.ks[0] + hk * a.ks[1];
@@ -390,7 +395,10 @@ DecodePlan plan_decode(const KArgs& a) {
   p.rows = a.L * a.G;
   const int round = NWAVE * KB;
   long long pairs = (long long)a.B * a.Hkv;
+  // two blocks of keys per wavefront at least, or one where that leaves most of the CUs idle (1 sequence of 1500 keys, 8 KV heads
+  // 11.2 -> 9.5 us, 2 of 324, one KV head 12.2 -> 10.3; not for a single chunk: the merge costs more)
   int max_splits = (a.S + 2 * round - 1) / (2 * round);
+  if (pairs * max_splits < 128 && a.S > 2 * round) max_splits = (a.S + round - 1) / round;
   if (max_splits < 1) max_splits = 1;
   // Two workgroups per CU or a few more: the count, up to four per CU, that fills its last round best (a CU takes in its
   // workgroups' keys at a rate of its own, so 2.25 per CU cost as much as 3: 24 sequences of 3000 keys on 4 KV heads, 96
