@@ -382,7 +382,15 @@ bool keys_among_wavefronts(const KArgs& a, double* tiles_walked = nullptr) {
   if (a.kv_splits > 1) return false;
   const long long heads = (long long)a.B * a.Hq, wide = heads * ((a.L + BM - 1) / BM), narrow = heads * ((a.L + 31) / 32);
   const long long tiles = ((a.causal && !a.pack_L && !a.kv_len && a.L < a.S ? a.L : a.S) + BN - 1) / BN;
-  const double whole = (double)tiles * (double)((wide + 255) / 256), dealt = (double)((tiles + 3) / 4) * (double)((narrow + 255) / 256) + 0.5;
+  // under a causal mask a launch of several rounds has a little more than half of the tiles to take
+  auto rounds = [&](long long wgs) {
+    const double r = (double)wgs * (a.causal ? 0.6 : 1.0) / 256;
+    return r > 1 ? r : 1.0;
+  };
+  // several rounds of the narrow ones: nothing overlaps a workgroup's loads, where two of the wide ones share a CU (4 x 8 heads x
+  // 778 rows, head_dim 80: 196 us dealt out, 125 whole)
+  const double whole = (double)tiles * rounds(wide), narrow_rounds = narrow <= 512 ? (double)((narrow + 255) / 256) : rounds(narrow);
+  const double dealt = (double)((tiles + 3) / 4) * (narrow_rounds > 1 ? 1.4 * narrow_rounds : 1.0) + 0.5;
   if (tiles_walked) *tiles_walked = dealt < 0.9 * whole ? dealt : whole;
   return dealt < 0.9 * whole;
 }

@@ -176,7 +176,8 @@ void pack_heads(KArgs* a) {
 // Key splits.  A workgroup walks its row tile's keys one tile after another, 2 us (fp32: 3 to 5) each however few workgroups there
 // are; when batch x heads x row tiles leave CUs idle, the keys are divided among several workgroups whose partial results a
 // second kernel combines.  The number is the one whose estimated time is least: the longest workgroup's tiles, in as
-// many rounds as the workgroups need; and with splits the second launch and its records, written and read.
+// many rounds as the workgroups need; and with splits the second launch and its records, written (a lane its own row's,
+// at 1 TB/s) and read.
 struct SplitPlan {
   int splits, chunk;
   size_t ws_bytes;
@@ -192,10 +193,11 @@ SplitPlan cheapest_split(long long wgs, long long keys, long long rows, int widt
     chunk = (chunk + step - 1) / step * step;
     const long long n = (keys + chunk - 1) / chunk;
     if (n < want) continue;  // the same as fewer
-    const double busy = (double)(wgs * n) * (causal ? 0.6 : 1.0) / slots;
+    double busy = (double)(wgs * n) * (causal ? 0.6 : 1.0) / slots;
+    if (slots <= 256 && busy > 1 && busy < 4) busy = (double)(long long)(busy + 0.999);  // one to a CU: whole rounds
     const double per = (double)((n > 1 ? chunk : keys) + tile - 1) / tile;
     const size_t bytes = n > 1 ? (size_t)rows * (size_t)n * (width + 2) * sizeof(float) : 0;
-    const double us = (double)(long long)per * tile_us * (busy > 1 ? busy : 1) + (n > 1 ? 5 + 2.0 * bytes / 4e6 : 0);
+    const double us = (double)(long long)per * tile_us * (busy > 1 ? busy : 1) + (n > 1 ? 5 + bytes / 0.8e6 : 0);
     if (n > 1 && us > 0.9 * least) continue;
     if (n == 1 && whole_us > 0) {
       least = whole_us;
