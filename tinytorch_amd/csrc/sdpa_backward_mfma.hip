@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
   const float l_tot = l_run + __shfl_xor(l_run, 32);
   const int qi = qw0 + lq;
   if (a.dq_splits > 1) {
-    if (qi < f.L) store_dq_partial<D>(a, piece, ((long long)b * f.Hq + h) * f.L + qi, lh, dqacc, m_use * c, l_tot, delta);
+    if (qi < f.L) store_dq_partial<D, PAD>(a, piece, ((long long)b * f.Hq + h) * f.L + qi, lh, dqacc, m_use * c, l_tot, delta);
     return;
   }
   if (qi < f.L) {

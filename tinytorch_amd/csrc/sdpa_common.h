@@ -276,7 +276,7 @@ struct BwdArgs {
 
 // Splits of a backward launch that would leave half of the chip idle with `n`: its workgroups walk their streams tile by tile,
 // tile_us each, however few they are.  The number, up to 16, whose longest stream, second launch and partial records (record_us
-// for each split, written and read) take least by estimate: bf16 2 x 4 heads on 1 x 199 rows, head_dim 128: whole backward 50 -> 37 us;
+// for each split, written and read at 2 TB/s) take least by estimate: bf16 2 x 4 heads on 1 x 199 rows, head_dim 128: whole backward 50 -> 37 us;
 // fp32 8 heads on 1 x 2000 x 2000, head_dim 64: 665 -> 257.
 inline int cheapest_backward_splits(int n, long long wgs, long long tiles, long long slots, double tile_us, double record_us) {
   if (wgs * n * 2 > slots) return n;
@@ -309,7 +309,7 @@ inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, int D, bool
   const long long enough = causal ? 512LL * per_cu * groups : 256 * per_cu;
   int n = 1;
   while (n < 4 && wgs * n < enough && tiles >= 16 * n && (D == 64 || D == 128)) n *= 2;  // (measured for these two sizes)
-  const double record_us = (double)B * Hkv * S * D * 16 / 4e6, tile_us = f32 ? (D <= 64 ? 5.0 : 10.0) : D <= 64 ? 1.15 : 2.0;
+  const double record_us = (double)B * Hkv * S * D * 16 / 2e6, tile_us = f32 ? (D <= 64 ? 5.0 : 10.0) : D <= 64 ? 1.15 : 2.0;
   return cheapest_backward_splits(n, wgs / groups, tiles, 256 * per_cu, tile_us, record_us);
 }
 
@@ -328,7 +328,7 @@ inline int backward_dq_splits(int B, int Hq, int L, int S, int D, bool causal, i
   const long long enough = causal ? 2 * slots : slots;
   int n = 1;
   while (n < 8 && wgs * n < enough && tiles >= 16 * n && (D == 64 || D == 128)) n *= 2;
-  const double record_us = (double)B * Hq * L * D * 8 / 4e6, tile_us = f32 ? (D <= 64 ? 4.0 : 8.0) : D <= 64 ? 0.9 : 1.4;
+  const double record_us = (double)B * Hq * L * D * 8 / 2e6, tile_us = f32 ? (D <= 64 ? 4.0 : 8.0) : D <= 64 ? 0.9 : 1.4;
   return cheapest_backward_splits(n, wgs, tiles, slots, tile_us, record_us);
 }
 
@@ -378,11 +378,11 @@ int launch_backward_dkv_sum(const BwdArgs& a, hipStream_t stream) {
 // A lane's share of a query row's unnormalised dq sums (accumulator layout of the 32 x 32 matrix instructions: registers 4rg .. 4rg+3 of block db are
 // elements 32db + 8rg + 4lh .. +3) and the row's (maximum in log2
 // units, sum of exponentials) as this split's partial record; split 0 also leaves delta for the dk/dv kernel.
-template <int D>
+template <int D, bool PAD = false>
 __device__ __forceinline__ void store_dq_partial(const BwdArgs& a, int piece, long long row_id, int lh, const f32x16 (&dqacc)[D / 32],
                                                  float mc, float l_tot, float delta) {
   const long long rows = (long long)a.f.B * a.f.Hq * a.f.L;
-  const int have = a.f.D;  // D, or fewer (the zero-column kernels)
+  const int have = PAD ? a.f.D : D;
   float* dst = a.dq_partial + (piece * rows + row_id) * have;
 #pragma unroll
   for (int db = 0; db < D / 32; db++)
@@ -391,7 +391,7 @@ __device__ __forceinline__ void store_dq_partial(const BwdArgs& a, int piece, lo
       f32x4 x;
 #pragma unroll
       for (int i = 0; i < 4; i++) x[i] = dqacc[db][4 * rg + i];
-      if (32 * db + 8 * rg + 4 * lh < have) *(f32x4*)(dst + 32 * db + 8 * rg + 4 * lh) = x;
+      if (!PAD || 32 * db + 8 * rg + 4 * lh < have) *(f32x4*)(dst + 32 * db + 8 * rg + 4 * lh) = x;
     }
   if (lh == 0) {
     float* ml = a.dq_partial + a.dq_splits * rows * have;
