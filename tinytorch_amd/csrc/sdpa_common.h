@@ -272,11 +272,13 @@ struct BwdArgs {
   // dk/dv kernels under a causal mask: workgroups of an XCD that run together (CUs per XCD x workgroups per CU), or 0.
   // The workgroups of every second such round walk their query tiles upwards (dkv_walks_up).
   int dkv_round;
+  // fp32 pair: the tiles of 32 rows' (keys') streams are dealt out to a workgroup's wavefronts (no splits then)
+  bool dq_dealt = false, dkv_dealt = false;
 };
 
 // Splits of a backward launch that would leave half of the chip idle with `n`: its workgroups walk their streams tile by tile,
 // tile_us each, however few they are.  The number, up to 16, whose longest stream, second launch and partial records (record_us
-// for each split, written and read at 2 TB/s) take least by estimate: bf16 2 x 4 heads on 1 x 199 rows, head_dim 128: whole backward 50 -> 37 us;
+// for each split, written and read at 2 TB/s, in fp32, whose tiles hide half of it, 4) take least by estimate: bf16 2 x 4 heads on 1 x 199 rows, head_dim 128: whole backward 50 -> 37 us;
 // fp32 8 heads on 1 x 2000 x 2000, head_dim 64: 665 -> 257.
 inline int cheapest_backward_splits(int n, long long wgs, long long tiles, long long slots, double tile_us, double record_us) {
   if (wgs * n * 2 > slots) return n;
@@ -290,6 +292,14 @@ inline int cheapest_backward_splits(int n, long long wgs, long long tiles, long 
   return best;
 }
 
+// fp32: whether dealing a stream's tiles out to the four wavefronts of workgroups of 32 rows is shorter than n splits (`narrow`: such
+// workgroups; one to a CU).
+inline bool backward_tiles_dealt(int n, long long narrow, long long tiles, double tile_us, double record_us) {
+  if (narrow > 256) return false;
+  const double dealt = ((double)((tiles + 3) / 4) + 0.5) * tile_us, split = (double)((tiles + n - 1) / n) * tile_us + (n > 1 ? 4.5 + n * record_us : 0.0);
+  return dealt < 0.95 * split;
+}
+
 // Workgroups that share a key block in the matrix-core dk/dv kernels (1: none, the kernel writes dk / dv itself).
 // A dk/dv workgroup owns 128 keys and about one runs per CU at a time; under a causal mask its length varies
 // 1 : (number of key blocks), and below about four workgroups per CU the longest ones set the time.  Without a causal
@@ -299,7 +309,7 @@ inline int cheapest_backward_splits(int n, long long wgs, long long tiles, long 
 // workgroups of a causal call further measured 4 % slower, 256 of them 7-21 % faster).
 // `per_cu`: workgroups of the kernel that fit a CU (2 at head_dim 64 without an attnMask, else 1): head_dim 64, 256 equal
 // workgroups without a causal mask: two splits +28 %; causal with 512: four splits instead of two -2 to -5 %.
-inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, int D, bool causal, int groups, int per_cu, bool f32) {
+inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, int D, bool causal, int groups, int per_cu, bool f32, bool* dealt) {
   const long long wgs = (long long)B * Hkv * ((S + 127) / 128) * groups;
   const long long tiles = (long long)(Hq / Hkv) * ((L + 31) / 32) / groups;  // the longest query stream, in 32-row tiles
   // causal: two rounds of the workgroups a CU holds at a time (one for the 8-wavefront head_dim-128 kernel, whose two
@@ -309,8 +319,10 @@ inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, int D, bool
   const long long enough = causal ? 512LL * per_cu * groups : 256 * per_cu;
   int n = 1;
   while (n < 4 && wgs * n < enough && tiles >= 16 * n && (D == 64 || D == 128)) n *= 2;  // (measured for these two sizes)
-  const double record_us = (double)B * Hkv * S * D * 16 / 2e6, tile_us = f32 ? (D <= 64 ? 5.0 : 10.0) : D <= 64 ? 1.15 : 2.0;
-  return cheapest_backward_splits(n, wgs / groups, tiles, 256 * per_cu, tile_us, record_us);
+  const double record_us = (double)B * Hkv * S * D * 16 / (f32 ? 4e6 : 2e6), tile_us = f32 ? (D <= 64 ? 5.0 : 10.0) : D <= 64 ? 1.15 : 2.0;
+  n = cheapest_backward_splits(n, wgs / groups, tiles, 256 * per_cu, tile_us, record_us);
+  *dealt = f32 && backward_tiles_dealt(n, (long long)B * Hkv * ((S + 31) / 32), tiles, tile_us, record_us);
+  return *dealt ? 1 : n;
 }
 
 // Workgroups that share a 128-row query block in the matrix-core dq kernels (1: none, the kernel writes dq itself).
@@ -321,15 +333,18 @@ inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, int D, bool
 // without a mask +22 %; 512 causal workgroups split in two measured 5 % slower: the partial records cost more than the
 // uneven end).  A split must still get a few hundred keys.
 // `slots`: workgroups of the kernel the chip holds at a time (512; 256 for the fp32 kernel at head_dim 128).
-inline int backward_dq_splits(int B, int Hq, int L, int S, int D, bool causal, int slots, bool f32) {
+inline int backward_dq_splits(int B, int Hq, int L, int S, int D, bool causal, int slots, bool f32, bool* dealt) {
+  *dealt = false;
   const long long wgs = (long long)B * Hq * ((L + 127) / 128);
   const long long tiles = (S + 31) / 32;  // the longest key range, in 32-key tiles
   if (wgs >= slots) return 1;
   const long long enough = causal ? 2 * slots : slots;
   int n = 1;
   while (n < 8 && wgs * n < enough && tiles >= 16 * n && (D == 64 || D == 128)) n *= 2;
-  const double record_us = (double)B * Hq * L * D * 8 / 2e6, tile_us = f32 ? (D <= 64 ? 4.0 : 8.0) : D <= 64 ? 0.9 : 1.4;
-  return cheapest_backward_splits(n, wgs, tiles, slots, tile_us, record_us);
+  const double record_us = (double)B * Hq * L * D * 8 / (f32 ? 4e6 : 2e6), tile_us = f32 ? (D <= 64 ? 4.0 : 8.0) : D <= 64 ? 0.9 : 1.4;
+  n = cheapest_backward_splits(n, wgs, tiles, slots, tile_us, record_us);
+  *dealt = f32 && backward_tiles_dealt(n, (long long)B * Hq * ((L + 31) / 32), tiles, tile_us, record_us);
+  return *dealt ? 1 : n;
 }
 
 // Workgroup id of a dk/dv launch with split query streams -> (key-block workgroup n, split).  The hardware hands

@@ -386,19 +386,25 @@ size_t backward_stats_bytes(const ttsdpa_backward_params* p) {
 }
 
 // Scratch layout: the statistics, then (matrix-core pairs with a split query stream) the partial dk / dv, 256-byte aligned.
-int dkv_splits_of(const ttsdpa_backward_params* p) {
+int dkv_splits_of(const ttsdpa_backward_params* p, bool* dealt = nullptr) {
   const ttsdpa_params* f = &p->fwd;
+  bool unused;
+  if (!dealt) dealt = &unused;
+  *dealt = false;
   if (!backward_on_mfma(p)) return 1;
   const int groups = f->dtype != TTSDPA_F32 && f->D == 128 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
   const int per_cu = f->D <= 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
-  return backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, groups, per_cu, f->dtype == TTSDPA_F32);
+  return backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, groups, per_cu, f->dtype == TTSDPA_F32, dealt);
 }
 // ... then (matrix-core pairs whose dq kernel splits its key ranges) the partial dq records, 256-byte aligned.
-int dq_splits_of(const ttsdpa_backward_params* p) {
+int dq_splits_of(const ttsdpa_backward_params* p, bool* dealt = nullptr) {
   const ttsdpa_params* f = &p->fwd;
+  bool unused;
+  if (!dealt) dealt = &unused;
+  *dealt = false;
   if (!backward_on_mfma(p)) return 1;
   const int slots = f->dtype == TTSDPA_F32 && f->D > 64 ? 256 : 512;
-  return backward_dq_splits(f->B, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, slots, f->dtype == TTSDPA_F32);
+  return backward_dq_splits(f->B, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, slots, f->dtype == TTSDPA_F32, dealt);
 }
 size_t backward_partial_offset(const ttsdpa_backward_params* p) { return (backward_stats_bytes(p) + 255) & ~(size_t)255; }
 size_t backward_dq_partial_offset(const ttsdpa_backward_params* p) {
@@ -653,9 +659,9 @@ int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t wor
   const size_t need = backward_scratch_bytes(p);
   if (need > 0 && (!workspace || workspace_bytes < need || !ptr_aligned(workspace, 16))) return TTSDPA_ERR_WORKSPACE;
   a.stats = (float*)workspace;
-  a.dkv_splits = dkv_splits_of(p);
+  a.dkv_splits = dkv_splits_of(p, &a.dkv_dealt);
   a.partial = a.dkv_splits > 1 ? (float*)((char*)workspace + backward_partial_offset(p)) : nullptr;
-  a.dq_splits = dq_splits_of(p);
+  a.dq_splits = dq_splits_of(p, &a.dq_dealt);
   a.dq_partial = a.dq_splits > 1 ? (float*)((char*)workspace + backward_dq_partial_offset(p)) : nullptr;
   if (backward_on_mfma(p)) {
     const long long g1 = (long long)a.f.B * a.f.Hq * ((a.f.L + 127) / 128) * a.dq_splits, g2 = (long long)a.f.B * a.f.Hkv * ((a.f.S + 127) / 128);
