@@ -480,7 +480,7 @@ StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split
   for (int R = least; R <= most; R *= 2) {
     if ((a.xt && a.M < 16 * R) || (a.wt && a.N < 16 * R)) break;
     // half of a 64 square tile idle: its few workgroups stream a weight slower than the estimate, which has every round full (12 x
-    // 5120 x 34944: 87 us in 64-row tiles, 65 in 32-row ones; 4096 x 28672 54 and 43)
+    // 5120 x 34944: 87 us in 64-row tiles, 69 in 32-row ones; 12 x 4096 x 28672 54 and 45)
     if (R == 4 && R > least && (a.M <= 32 || a.N <= 32)) break;
     for (int S = 1; S <= 32 && (S == 1 || (may_split && a.K >= 512 * S)); S *= 2) {
       const double t = stream_us(a, esz, R, S, entries);
