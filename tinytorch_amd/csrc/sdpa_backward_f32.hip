@@ -42,7 +42,7 @@ template <int D>
 struct BwdF32Lds {
   static constexpr int PITCH = D + 1;                 // floats per tile row
   static constexpr int TILE = BT * PITCH;             // K or V (kernel 1), Q or dout (kernel 2)
-  static constexpr int STAGE = 2 * TILE + 2 * BT;     // two tiles and, in kernel 2, (lse2, delta) per query row
+  static constexpr int STAGE = 2 * TILE + 3 * BT;     // two tiles and, in kernel 2, (statistic, delta) and log_sums per query row
   static constexpr int BYTES = 2 * STAGE * 4;         // double-buffered
 };
 
@@ -142,9 +142,9 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
   f32x16 dqacc[DBLK];
 #pragma unroll
   for (int i = 0; i < DBLK; i++) dqacc[i] = zero16();
-  const float c = f.scale * kLog2e;
+  const float c = MASKED ? scores_unit(f) : f.scale * kLog2e;
   const float lazy = kLazyExp / c;
-  float m_use = -1e30f, mc = m_use * c, l_run = 0.f;
+  float m_use = MASKED ? -FLT_MAX : -1e30f, mc = m_use * c, l_run = 0.f;
 
   const int S = keys_of_batch(f, b);
   if (S == 0) {  // no keys (an empty cache entry): the output did not depend on q
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
         int qi = qw0 + lq;
         qi = qi < f.L ? qi : f.L - 1;
         const long long mrow = b * f.ms[0] + h * f.ms[1] + qi * f.ms[2];
-        apply_attn_mask<float>(f, s, load_attn_mask<float>(f, mrow, kv0, lh, S), 1.f / f.scale);
+        apply_attn_mask<float>(f, s, load_attn_mask<float>(f, mrow, kv0, lh, S));
       }
       if ((CAUSAL && kv0 + BT - 1 > qw0 + coff) || kv0 + BT > S) {
         const int qi = qw0 + lq + coff;
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
       float psum = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        const float p = fast_exp2(fmaf(s[r], c, -mc));  // relative to m_use; normalised at the end
+        const float p = fast_exp2(MASKED ? (s[r] - m_use) * c : fmaf(s[r], c, -mc));  // relative to m_use; normalised at the end
         psum += p;
         s[r] = p * (dp[r] - delta);
       }
@@ -303,7 +303,10 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
     if (qi < f.L) {
       const long long row_id = ((long long)b * f.Hq + h) * f.L + qi;
       const bool seen = l_all > 0.f;
-      if (wave == 0 && lh == 0) *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_all * c + __log2f(l_all) : 1e30f, delta);
+      if (wave == 0 && lh == 0) {
+        *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_all * c + __log2f(l_all) : 1e30f, delta);
+        if (MASKED) store_masked_stat(a, row_id, seen, m_all, l_all);
+      }
       const float w = seen ? f.scale / l_all : 0.f;
       float* dqp = (float*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
 #pragma unroll
@@ -321,7 +324,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
     return;
   }
   if (a.dq_splits > 1) {
-    if (qi < f.L) store_dq_partial<D, PAD>(a, piece, ((long long)b * f.Hq + h) * f.L + qi, lh, dqacc, m_use * c, l_tot, delta);
+    if (qi < f.L) store_dq_partial<D, PAD>(a, piece, ((long long)b * f.Hq + h) * f.L + qi, lh, dqacc, MASKED ? m_use : m_use * c, l_tot, delta);
     return;
   }
   if (qi < f.L) {
@@ -329,7 +332,10 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
     // log2 of the row's sum of exponentials, the unit the second kernel's exp2 wants
     // a row whose keys are all hidden (possible with an attnMask): dq = 0, and a statistic that gives it weight 0 below
     const bool seen = l_tot > 0.f;
-    if (lh == 0) *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_use * c + __log2f(l_tot) : 1e30f, delta);
+    if (lh == 0) {
+      *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_use * c + __log2f(l_tot) : 1e30f, delta);
+      if (MASKED) store_masked_stat(a, row_id, seen, m_use, l_tot);
+    }
     const float w = seen ? f.scale / l_tot : 0.f;
     float* dqp = (float*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
 #pragma unroll
@@ -402,7 +408,8 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
   f32x16 dkacc[DBLK], dvacc[DBLK];
 #pragma unroll
   for (int i = 0; i < DBLK; i++) dkacc[i] = zero16(), dvacc[i] = zero16();
-  const float c = f.scale * kLog2e;
+  const float c = MASKED ? scores_unit(f) : f.scale * kLog2e;
+  const float raw = f.mask_kind == 2 ? f.scale : 1.f;  // a raw product's part in a score (scores_unit)
 
   // Query tiles it0 .. ntq-1 of each of the G heads see keys of this workgroup; taken from the last tile down, the heads
   // of a tile one after the other, so that the key blocks of a (batch, kv head) — which share an XCD — walk in step and
@@ -417,6 +424,7 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
 
   f32x4 qst[NLD], gst[NLD];
   float2 sst = make_float2(0.f, 0.f);
+  float slog = 0.f;
   int lrow[NLD], lcol[NLD], gcol[NLD];
   bool cval[NLD];  // PAD: as in the dq kernel
 #pragma unroll
@@ -441,7 +449,9 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
     }
     if ((DEAL ? lane : tid) < BT) {
       const int row = i0 + (DEAL ? lane : tid);
-      sst = row < f.L ? *(const float2*)(a.stats + 2 * (((long long)b * f.Hq + h) * f.L + row)) : make_float2(1e30f, 0.f);
+      const long long row_id = ((long long)b * f.Hq + h) * f.L + row;
+      sst = row < f.L ? *(const float2*)(a.stats + 2 * row_id) : make_float2(MASKED ? FLT_MAX : 1e30f, 0.f);
+      if (MASKED) slog = row < f.L ? a.log_sums[row_id] : 1e30f;
     }
   };
   auto store_tile = [&](int stage) {
@@ -454,7 +464,10 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
         Qs[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? qst[i][e] : 0.f;
         Gs[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? gst[i][e] : 0.f;
       }
-    if ((DEAL ? lane : tid) < BT) *(float2*)(Gs + Lds::TILE + 2 * (DEAL ? lane : tid)) = sst;
+    if ((DEAL ? lane : tid) < BT) {
+      *(float2*)(Gs + Lds::TILE + 2 * (DEAL ? lane : tid)) = sst;
+      if (MASKED) Gs[Lds::TILE + 2 * BT + (DEAL ? lane : tid)] = slog;
+    }
   };
   const int s_lane = lq * PITCH + lh * (D / 2);
   const int g_lane = 4 * lh * PITCH + lq;
@@ -489,31 +502,35 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
 
       f32x16 s = score_product<D>(Qs + s_lane, kreg);   // S = Q . K^T
       f32x16 dp = score_product<D>(Gs + s_lane, vreg);  // dP = dout . V^T
-      // only tiles on the diagonal, and the last key block, hide anything (rows past L carry lse = 1e30: weight 0)
+      // only tiles on the diagonal, and the last key block, hide anything (rows past L carry a statistic of weight 0)
       const bool need_mask = (CAUSAL && kw0 + 31 > i0 + coff) || kw0 + 32 > S;
 #pragma unroll
       for (int rg = 0; rg < 4; rg++) {
-        const f32x4 s0 = *(const f32x4*)(st + 2 * (8 * rg + 4 * lh));      // (lse2, delta) of rows 8rg+4lh+0, +1
+        const f32x4 s0 = *(const f32x4*)(st + 2 * (8 * rg + 4 * lh));      // (statistic, delta) of rows 8rg+4lh+0, +1
         const f32x4 s1 = *(const f32x4*)(st + 2 * (8 * rg + 4 * lh) + 4);  // ... +2, +3
-        const float lse2[4] = {s0[0], s0[2], s1[0], s1[2]};
+        f32x4 logs = {0.f, 0.f, 0.f, 0.f};
+        if (MASKED) logs = *(const f32x4*)(st + 2 * BT + 8 * rg + 4 * lh);
+        const float stat[4] = {s0[0], s0[2], s1[0], s1[2]};  // log2 of the row's sum, or with an attnMask its maximum
         const float dl[4] = {s0[1], s0[3], s1[1], s1[3]};
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const int r = 4 * rg + e;
-          float bias2 = 0.f;  // attnMask: the additive bias in log2 units, or -inf for a hidden key
+          float bias = 0.f;  // attnMask: the additive bias, or -inf for a hidden key
           if (MASKED) {
             int qrow = i0 + 8 * rg + 4 * lh + e;
             qrow = qrow < f.L ? qrow : f.L - 1;
             const long long at = b * f.ms[0] + h_of_tile * f.ms[1] + qrow * f.ms[2] + (key < S ? key : S - 1) * f.ms[3];
             if (f.mask_kind == 1) {
-              bias2 = ((const uint8_t*)f.mask)[at] == 0 ? -INFINITY : 0.f;
+              bias = ((const uint8_t*)f.mask)[at] == 0 ? -INFINITY : 0.f;
             } else {
-              bias2 = ((const float*)f.mask)[at] * kLog2e;
+              bias = ((const float*)f.mask)[at];
             }
           }
-          const float p = fast_exp2(fmaf(s[r], c, bias2 - lse2[e]));
-          s[r] = p;
-          dp[r] = p * (dp[r] - dl[e]);
+          // with an attnMask: the score as the dq kernel has it; a hidden key weighs nothing, whatever its k and v hold
+          const bool hidden = MASKED && bias == -INFINITY;
+          const float p = fast_exp2(MASKED ? fmaf(fmaf(s[r], raw, bias) - stat[e], c, -logs[e]) : fmaf(s[r], c, -stat[e]));
+          s[r] = hidden ? 0.f : p;
+          dp[r] = hidden ? 0.f : p * (dp[r] - dl[e]);
         }
       }
       if (need_mask) {

@@ -12,7 +12,7 @@
 // dk and dv sum over the query heads that share a KV head.
 //
 // Two kernels per call, no atomics (a fixed summation order: results are reproducible):
-//   1. per block of query rows: lse_i and delta_i (kept in scratch for the second kernel) and dq_i, the keys and
+//   1. per block of query rows: lse_i (as maximum and log of the sum relative to it) and delta_i (kept in scratch for the second kernel) and dq_i, the keys and
 //      values streamed through LDS as fp32 tiles, the softmax statistics built online;
 //   2. per block of keys: dk_j and dv_j over all query rows and the heads of the group, the query and dout rows
 //      streamed the same way.
@@ -153,10 +153,11 @@ __global__ __launch_bounds__(256) void backward_dq_tiled_kernel(BwdArgs a) {
     }
   }
   if (row < f.L) {
-    const bool seen = l > 0.f;  // a row whose keys are all hidden: dq = 0, and the dk/dv kernel skips it (lse = -inf)
+    const bool seen = l > 0.f;  // a row whose keys are all hidden: dq = 0, and the dk/dv kernel skips it (maximum -inf)
     if (sub == 0) {
       const long long row_id = ((long long)b * f.Hq + h) * f.L + row;
-      a.stats[2 * row_id] = seen ? m + __logf(l) : -INFINITY;
+      a.stats[2 * row_id] = seen ? m : -INFINITY;
+      a.log_sums[row_id] = seen ? __logf(l) : 0.f;
       a.stats[2 * row_id + 1] = delta;
     }
     const float wgt = seen ? f.scale / l : 0.f;
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(256) void backward_dkv_tiled_kernel(BwdArgs a) {
   constexpr int kRows = Tiled<LPR>::kRows, kTile = Tiled<LPR>::kTile;
   __shared__ float Qs[kTile][DP];
   __shared__ float Gs[kTile][DP];
-  __shared__ float Ls[kTile], Ds[kTile];
+  __shared__ float Ms[kTile], Ls[kTile], Ds[kTile];
   const KArgs& f = a.f;
   const int tid = threadIdx.x, sub = tid & (LPR - 1);
   const long long npair = (long long)f.B * f.Hkv;  // order as in the dq kernel: the first key blocks are the longest
@@ -204,6 +205,7 @@ __global__ __launch_bounds__(256) void backward_dkv_tiled_kernel(BwdArgs a) {
       const T* qp = (const T*)f.q + b * f.qs[0] + h * f.qs[1];
       const T* gp = (const T*)a.dout + b * a.dos[0] + h * a.dos[1];
       const float* st = a.stats + 2 * (((long long)b * f.Hq + h) * f.L);
+      const float* logs = a.log_sums + ((long long)b * f.Hq + h) * f.L;
       for (int i0 = ifirst & ~(kTile - 1); i0 < f.L; i0 += kTile) {
         __syncthreads();
         for (int e = tid; e < kTile * DP; e += 256) {
@@ -214,7 +216,8 @@ __global__ __launch_bounds__(256) void backward_dkv_tiled_kernel(BwdArgs a) {
         }
         if (tid < kTile) {
           const int i = i0 + tid;
-          Ls[tid] = i < f.L ? st[2 * i] : -INFINITY;  // rows past the end weigh nothing
+          Ms[tid] = i < f.L ? st[2 * i] : -INFINITY;  // rows past the end weigh nothing
+          Ls[tid] = i < f.L ? logs[i] : 0.f;
           Ds[tid] = i < f.L ? st[2 * i + 1] : 0.f;
         }
         __syncthreads();
@@ -228,13 +231,13 @@ __global__ __launch_bounds__(256) void backward_dkv_tiled_kernel(BwdArgs a) {
             pd = fmaf(Gs[ii][LPR * t + sub], vreg[t], pd);
           }
           const float sdot = group_sum<LPR>(ps), ddot = group_sum<LPR>(pd);
-          const float lse = Ls[ii];
+          const float m = Ms[ii];
           float p = 0.f, ds = 0.f;
-          if (key < S && lse > -INFINITY) {
+          if (key < S && m > -INFINITY) {
             const long long mrow = b * f.ms[0] + h * f.ms[1] + i * f.ms[2];
             const float x = biased_score<T>(f, sdot, i, key, coff, mrow);
             if (x > -INFINITY) {
-              p = __expf(x - lse);
+              p = __expf((x - m) - Ls[ii]);
               ds = p * (ddot - Ds[ii]) * f.scale;
             }
           }

@@ -43,7 +43,7 @@ struct BwdLds {
   static constexpr int RP = D + 8;    // row pitch (elements) of a tile read as a row-major operand (ds_read_b128)
   static constexpr int TP = D + 32;   // row pitch of a tile read as a transposed operand (ds_read_b64_tr_b16)
   static constexpr int KV_STAGE = BQ * (2 * RP + 2 * TP);   // Q and dout, each in both layouts
-  static constexpr int KV_STATS = 2 * BQ;                   // floats per stage: (lse, delta) per query row
+  static constexpr int KV_STATS = 3 * BQ;                   // floats per stage: (statistic, delta) and log_sums per query row
   static constexpr int KV_BYTES = 2 * KV_STAGE * 2 + 2 * KV_STATS * 4;
 };
 
@@ -202,9 +202,9 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
   for (int i = 0; i < DBLK; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) dqacc[i][r] = 0.f;
-  const float c = f.scale * kLog2e;
+  const float c = MASKED ? scores_unit(f) : f.scale * kLog2e;
   const float lazy = kLazyExp / c;
-  float m_use = -1e30f, mc = m_use * c, l_run = 0.f;
+  float m_use = MASKED ? -FLT_MAX : -1e30f, mc = m_use * c, l_run = 0.f;
 
   const int S = keys_of_batch(f, b);
   if (S == 0) {  // no keys (an empty cache entry): the output did not depend on q
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
         const long long mrow = b * f.ms[0] + h * f.ms[1] + qi * f.ms[2];
 #pragma unroll
         for (int blk = 0; blk < NBLK; blk++)
-          apply_attn_mask<T>(f, sacc[blk], load_attn_mask<T>(f, mrow, kv0 + 32 * blk, lh, S), 1.f / f.scale);
+          apply_attn_mask<T>(f, sacc[blk], load_attn_mask<T>(f, mrow, kv0 + 32 * blk, lh, S));
       }
       if ((CAUSAL && kv0 + BN - 1 > qw0 + coff) || kv0 + BN > S) {
         const int qi = qw0 + lq + coff;
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
       for (int blk = 0; blk < NBLK; blk++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-          const float p = fast_exp2(fmaf(sacc[blk][r], c, -mc));  // relative to m_use; normalised at the end
+          const float p = fast_exp2(MASKED ? (sacc[blk][r] - m_use) * c : fmaf(sacc[blk][r], c, -mc));  // relative to m_use; normalised at the end
           psum += p;
           sacc[blk][r] = p * (dpacc[blk][r] - delta);
         }
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
   const float l_tot = l_run + __shfl_xor(l_run, 32);
   const int qi = qw0 + lq;
   if (a.dq_splits > 1) {
-    if (qi < f.L) store_dq_partial<D, PAD>(a, piece, ((long long)b * f.Hq + h) * f.L + qi, lh, dqacc, m_use * c, l_tot, delta);
+    if (qi < f.L) store_dq_partial<D, PAD>(a, piece, ((long long)b * f.Hq + h) * f.L + qi, lh, dqacc, MASKED ? m_use : m_use * c, l_tot, delta);
     return;
   }
   if (qi < f.L) {
@@ -376,7 +376,10 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
     // log2 of the row's sum of exponentials, the unit the second kernel's exp2 wants
     // a row whose keys are all hidden (possible with an attnMask): dq = 0, and a statistic that gives it weight 0 below
     const bool seen = l_tot > 0.f;
-    if (lh == 0) *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_use * c + __log2f(l_tot) : 1e30f, delta);
+    if (lh == 0) {
+      *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_use * c + __log2f(l_tot) : 1e30f, delta);
+      if (MASKED) store_masked_stat(a, row_id, seen, m_use, l_tot);
+    }
     const float w = seen ? f.scale / l_tot : 0.f;
     T* dqp = (T*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
 #pragma unroll
@@ -451,7 +454,8 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dkv_mfma_kerne
   for (int i = 0; i < DBLK; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) dkacc[i][r] = 0.f, dvacc[i][r] = 0.f;
-  const float c = f.scale * kLog2e;
+  const float c = MASKED ? scores_unit(f) : f.scale * kLog2e;
+  const float raw = f.mask_kind == 2 ? f.scale : 1.f;  // a raw product's part in a score (scores_unit)
 
   // Query tiles it0 .. ntq-1 of each of the G heads see keys of this workgroup.  They are taken from the last tile down,
   // the heads of a tile one after the other: every key block of a (batch, kv head) then starts at the same tile and walks
@@ -467,6 +471,7 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dkv_mfma_kerne
 
   u32x4 qst[NLD], gst[NLD];
   float2 sst = make_float2(0.f, 0.f);
+  float slog = 0.f;
   int lrow[NLD], lcol[NLD], gcol[NLD];
   bool cval[NLD];  // PAD: as in the dq kernel
 #pragma unroll
@@ -492,7 +497,9 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dkv_mfma_kerne
     }
     if (tid < BQ) {
       const int row = i0 + tid;
-      sst = row < f.L ? *(const float2*)(a.stats + 2 * (((long long)b * f.Hq + h) * f.L + row)) : make_float2(1e30f, 0.f);
+      const long long row_id = ((long long)b * f.Hq + h) * f.L + row;
+      sst = row < f.L ? *(const float2*)(a.stats + 2 * row_id) : make_float2(MASKED ? FLT_MAX : 1e30f, 0.f);
+      if (MASKED) slog = row < f.L ? a.log_sums[row_id] : 1e30f;
     }
   };
   auto store_tile = [&](int stage) {
@@ -507,7 +514,10 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dkv_mfma_kerne
       *(u32x4*)(Gr + lrow[i] * RP + 8 * lcol[i]) = cval[i] ? gst[i] : zero4;
       *(u32x4*)(Gt + lrow[i] * TP + 8 * lcol[i]) = cval[i] ? gst[i] : zero4;
     }
-    if (tid < BQ) *(float2*)(sstats + stage * Lds::KV_STATS + 2 * tid) = sst;
+    if (tid < BQ) {
+      *(float2*)(sstats + stage * Lds::KV_STATS + 2 * tid) = sst;
+      if (MASKED) sstats[stage * Lds::KV_STATS + 2 * BQ + tid] = slog;
+    }
   };
   const int r_lane = lq * RP + 8 * lh;
   const int t_lane = (4 * lh + ((lane & 15) >> 2)) * TP + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
@@ -543,31 +553,35 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dkv_mfma_kerne
       for (int ks = 0; ks < KSTEPS; ks++) dpacc = TR::mfma32(*(const vec8*)(Gr + r_lane + 16 * ks), vreg[ks], dpacc);
 
       const int key = kw0 + lq;
-      // only tiles on the diagonal, and the last key block, hide anything (rows past L carry lse = 1e30: weight 0)
+      // only tiles on the diagonal, and the last key block, hide anything (rows past L carry a statistic of weight 0)
       const bool need_mask = (CAUSAL && kw0 + 31 > i0 + coff) || kw0 + 32 > S;
 #pragma unroll
       for (int rg = 0; rg < 4; rg++) {
-        const f32x4 s0 = *(const f32x4*)(st + 2 * (8 * rg + 4 * lh));      // (lse2, delta) of rows 8rg+4lh+0, +1
+        const f32x4 s0 = *(const f32x4*)(st + 2 * (8 * rg + 4 * lh));      // (statistic, delta) of rows 8rg+4lh+0, +1
         const f32x4 s1 = *(const f32x4*)(st + 2 * (8 * rg + 4 * lh) + 4);  // ... +2, +3
-        const float lse2[4] = {s0[0], s0[2], s1[0], s1[2]};
+        f32x4 logs = {0.f, 0.f, 0.f, 0.f};
+        if (MASKED) logs = *(const f32x4*)(st + 2 * BQ + 8 * rg + 4 * lh);
+        const float stat[4] = {s0[0], s0[2], s1[0], s1[2]};  // log2 of the row's sum, or with an attnMask its maximum
         const float dl[4] = {s0[1], s0[3], s1[1], s1[3]};
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const int r = 4 * rg + e;
-          float bias2 = 0.f;  // attnMask: the additive bias in log2 units, or -inf for a hidden key
+          float bias = 0.f;  // attnMask: the additive bias, or -inf for a hidden key
           if (MASKED) {
             int qrow = i0 + 8 * rg + 4 * lh + e;
             qrow = qrow < f.L ? qrow : f.L - 1;
             const long long at = b * f.ms[0] + h_of_tile * f.ms[1] + qrow * f.ms[2] + (key < S ? key : S - 1) * f.ms[3];
             if (f.mask_kind == 1) {
-              bias2 = ((const uint8_t*)f.mask)[at] == 0 ? -INFINITY : 0.f;
+              bias = ((const uint8_t*)f.mask)[at] == 0 ? -INFINITY : 0.f;
             } else {
-              bias2 = (float)((const T*)f.mask)[at] * kLog2e;
+              bias = (float)((const T*)f.mask)[at];
             }
           }
-          const float p = fast_exp2(fmaf(sacc[r], c, bias2 - lse2[e]));
-          sacc[r] = p;
-          dpacc[r] = p * (dpacc[r] - dl[e]);
+          // with an attnMask: the score as the dq kernel has it; a hidden key weighs nothing, whatever its k and v hold
+          const bool hidden = MASKED && bias == -INFINITY;
+          const float p = fast_exp2(MASKED ? fmaf(fmaf(sacc[r], raw, bias) - stat[e], c, -logs[e]) : fmaf(sacc[r], c, -stat[e]));
+          sacc[r] = hidden ? 0.f : p;
+          dpacc[r] = hidden ? 0.f : p * (dpacc[r] - dl[e]);
         }
       }
       if (need_mask) {

@@ -1,6 +1,7 @@
 // Shared device-side definitions for the gfx950 attention kernels.
 #pragma once
 
+#include <float.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -125,15 +126,22 @@ __device__ __forceinline__ void store_from_float(float* p, float x) { *p = x; }
 __device__ __forceinline__ void store_from_float(__bf16* p, float x) { *p = (__bf16)x; }
 __device__ __forceinline__ void store_from_float(_Float16* p, float x) { *p = (_Float16)x; }
 
+// The scores of a call with an attnMask, and what turns a difference of two of them into a power of two (scores_unit).  Bool:
+// raw products, hidden keys at -inf.  Additive: score = raw * scale + bias, an fp32 number as in the reference's chain
+// (src/Function/FuncNNLayer.h:237,249-260), whatever the bias: every finite value of the type is a key that counts.  A row may
+// therefore lie at the lowest value altogether, and a kernel's maximum starts at -FLT_MAX (hidden keys only: -inf - -FLT_MAX
+// gives weight 0) and is subtracted before anything is multiplied: with the bias divided by the scale and
+// exp2(fma(s, c, -m*c)), rows at fp32's lowest value were NaN (an overflow; every weight 0 against a start at -1e30), and at
+// -1e9 the rounding of m*c alone is a factor of 2^+-64.
+__device__ __forceinline__ float scores_unit(const KArgs& a) { return a.mask_kind == 2 ? kLog2e : a.scale * kLog2e; }
+
 // attnMask applied to the 32 x 32 score block of an MFMA accumulator (reference src/Function/FuncNNLayer.h:249-260):
 // a lane holds one query row (mask row offset `mrow`, in elements) and, in register group rg, the four consecutive
-// keys kv0 + 8*rg + 4*lh .. +3.  Bool: hidden keys get -inf; additive: the bias joins the scaled score, i.e.
-// bias * inv_scale the raw score held here.  Element strides of 0 broadcast an axis.  Keys at or beyond S are left
+// keys kv0 + 8*rg + 4*lh .. +3.  Element strides of 0 broadcast an axis.  Keys at or beyond S are left
 // alone (masked by the caller).  With a.mask_vec4 a group of four keys is one load.  For the pipelined kernels' general
 // steps, which have few registers to spare.
 template <typename T>
-__device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, long long mrow, int kv0, int lh, int S,
-                                                float inv_scale) {
+__device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, long long mrow, int kv0, int lh, int S) {
 #pragma unroll
   for (int rg = 0; rg < 4; rg++) {
     const int key0 = kv0 + 8 * rg + 4 * lh;
@@ -148,7 +156,7 @@ __device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, long 
         typedef T vec4t __attribute__((ext_vector_type(4)));
         const vec4t w = *(const vec4t*)((const T*)a.mask + at);
 #pragma unroll
-        for (int e = 0; e < 4; e++) s[4 * rg + e] += (float)w[e] * inv_scale;
+        for (int e = 0; e < 4; e++) s[4 * rg + e] = fmaf(s[4 * rg + e], a.scale, (float)w[e]);
       }
     } else {
 #pragma unroll
@@ -159,7 +167,7 @@ __device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, long 
           if (a.mask_kind == 1) {
             if (((const uint8_t*)a.mask)[at] == 0) s[4 * rg + e] = -INFINITY;
           } else {
-            s[4 * rg + e] += (float)((const T*)a.mask)[at] * inv_scale;
+            s[4 * rg + e] = fmaf(s[4 * rg + e], a.scale, (float)((const T*)a.mask)[at]);
           }
         }
       }
@@ -232,9 +240,8 @@ __device__ __forceinline__ MaskBlock<T> load_attn_mask(const KArgs& a, long long
   return m;
 }
 
-// Bool: hidden keys get -inf; additive: the bias joins the scaled score.
 template <typename T>
-__device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, MaskBlock<T> m, float inv_scale) {
+__device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, MaskBlock<T> m) {
   constexpr int WPG = sizeof(T);
   if (a.mask_kind == 1) {
 #pragma unroll
@@ -244,14 +251,17 @@ __device__ __forceinline__ void apply_attn_mask(const KArgs& a, f32x16& s, MaskB
     typedef T vec16t __attribute__((ext_vector_type(16)));
     const vec16t b = __builtin_bit_cast(vec16t, m);
 #pragma unroll
-    for (int r = 0; r < 16; r++) s[r] += (float)b[r] * inv_scale;
+    for (int r = 0; r < 16; r++) s[r] = fmaf(s[r], a.scale, (float)b[r]);
   }
 }
 
 // Backward call: the forward's arguments (f.out holds the forward's result, an input here) plus the upstream gradient
-// and the three gradients to write.  stats is scratch [B,Hq,L,2] floats: per query row the log of the sum of
-// exponentials of its scaled, biased scores (natural log in the vector-ALU kernels, log2 in the MFMA kernels: the two
-// kernels of a call are always of one family), and delta = dout . out.
+// and the three gradients to write.  stats is scratch [B,Hq,L,2] floats: per query row a statistic of its scores and delta =
+// dout . out.  Without an attnMask, in the MFMA kernels, the statistic is log2 of the sum of exponentials of the scaled
+// scores.  With one, and in the vector-ALU kernels, it is the row's maximum, in the scores' own units (scores_unit), and
+// log_sums ([B,Hq,L]) has the log of the sum relative to that maximum (log2 in the MFMA kernels, natural in the others; the
+// two kernels of a call are always of one family): next to a maximum of -1e9 the sum's logarithm is lost to rounding, and
+// such a row's weights were 1 each instead of 1 / keys.
 struct BwdArgs {
   KArgs f;
   const void* dout;
@@ -260,13 +270,15 @@ struct BwdArgs {
   void* dv;
   long long dos[3], dqs[3], dks[3], dvs[3];  // element strides: batch, head, sequence
   float* stats;
+  float* log_sums = nullptr;
   // matrix-core pairs only: with dkv_splits > 1 the query stream of every key block is dealt out to that many
   // workgroups, which leave partial dk / dv in `partial` ([split][dk | dv][B][Hkv][S][D] floats) for a third kernel to add.
   float* partial;
   int dkv_splits;
   // matrix-core pairs only: with dq_splits > 1 the key range of every 128-row query block is dealt out to that many
   // workgroups of the dq kernel, which leave their unnormalised fp32 sums in `dq_partial` ([split][B][Hq][L][D] floats,
-  // then [split][B][Hq][L] pairs (maximum in log2 units, sum of exponentials)) for backward_dq_merge_kernel.
+  // then [split][B][Hq][L] pairs (maximum in log2 units, or with an attnMask the scores' own; sum of exponentials)) for
+  // backward_dq_merge_kernel.
   float* dq_partial;
   int dq_splits;
   // dk/dv kernels under a causal mask: workgroups of an XCD that run together (CUs per XCD x workgroups per CU), or 0.
@@ -391,11 +403,11 @@ int launch_backward_dkv_sum(const BwdArgs& a, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 // A lane's share of a query row's unnormalised dq sums (accumulator layout of the 32 x 32 matrix instructions: registers 4rg .. 4rg+3 of block db are
-// elements 32db + 8rg + 4lh .. +3) and the row's (maximum in log2
-// units, sum of exponentials) as this split's partial record; split 0 also leaves delta for the dk/dv kernel.
+// elements 32db + 8rg + 4lh .. +3) and the row's (maximum, sum of exponentials) as this split's partial record; split 0 also
+// leaves delta for the dk/dv kernel.
 template <int D, bool PAD = false>
 __device__ __forceinline__ void store_dq_partial(const BwdArgs& a, int piece, long long row_id, int lh, const f32x16 (&dqacc)[D / 32],
-                                                 float mc, float l_tot, float delta) {
+                                                 float m, float l_tot, float delta) {
   const long long rows = (long long)a.f.B * a.f.Hq * a.f.L;
   const int have = PAD ? a.f.D : D;
   float* dst = a.dq_partial + (piece * rows + row_id) * have;
@@ -410,9 +422,16 @@ __device__ __forceinline__ void store_dq_partial(const BwdArgs& a, int piece, lo
     }
   if (lh == 0) {
     float* ml = a.dq_partial + a.dq_splits * rows * have;
-    *(float2*)(ml + 2 * (piece * rows + row_id)) = make_float2(mc, l_tot);
+    *(float2*)(ml + 2 * (piece * rows + row_id)) = make_float2(m, l_tot);
     if (piece == 0) a.stats[2 * row_id + 1] = delta;
   }
+}
+
+// A row's statistics in a call with an attnMask (matrix-core pairs); a row whose keys are all hidden gets a maximum and a
+// logarithm that give it weight 0 in the dk/dv kernel.
+__device__ __forceinline__ void store_masked_stat(const BwdArgs& a, long long row_id, bool seen, float m, float l) {
+  a.stats[2 * row_id] = seen ? m : FLT_MAX;
+  a.log_sums[row_id] = seen ? __log2f(l) : 1e30f;
 }
 
 // dq of a call whose key ranges were split: the splits' sums brought to the common maximum, added in a fixed order (split
@@ -442,12 +461,13 @@ __global__ __launch_bounds__(256) void backward_dq_merge_kernel(BwdArgs a, long 
     *out = __builtin_convertvector(x, vec4t);
     return;
   }
+  const float unit = f.mask_kind != 0 ? scores_unit(f) : 1.f;
   float m = -INFINITY;
   for (int s = 0; s < a.dq_splits; s++) m = fmaxf(m, ml[2 * (s * rows + row_id)]);
   float l = 0.f;
   for (int s = 0; s < a.dq_splits; s++) {
     const float2 st = *(const float2*)(ml + 2 * (s * rows + row_id));
-    const float w = fast_exp2(st.x - m);
+    const float w = fast_exp2((st.x - m) * unit);
     l += st.y * w;
     x += *(const f32x4*)(a.dq_partial + (s * rows + row_id) * f.D + d) * w;
   }
@@ -457,7 +477,10 @@ __global__ __launch_bounds__(256) void backward_dq_merge_kernel(BwdArgs a, long 
 #pragma unroll
   for (int e = 0; e < 4; e++) x[e] = seen ? x[e] * w : 0.f;
   *out = __builtin_convertvector(x, vec4t);
-  if (d == 0) a.stats[2 * row_id] = seen ? m + __log2f(l) : 1e30f;
+  if (d == 0) {
+    if (f.mask_kind != 0) store_masked_stat(a, row_id, seen, m, l);
+    else a.stats[2 * row_id] = seen ? m + __log2f(l) : 1e30f;
+  }
 }
 template <typename T>
 int launch_backward_dq_merge(const BwdArgs& a, hipStream_t stream) {
@@ -610,10 +633,10 @@ __global__ __launch_bounds__(256) void tile_split_merge_kernel(KArgs a, int W, i
   const int qi = (int)(row_id % a.L);
   const long long bh = row_id / a.L;
   const int h = (int)(bh % a.Hq), b = (int)(bh / a.Hq);
-  const float c = a.scale * kLog2e;
+  const float c = scores_unit(a);
   const long long step = (long long)a.L * (W + 2);
   const float* rec = a.ws + (bh * a.kv_splits * a.L + qi) * (W + 2);
-  float m = -1e30f;
+  float m = -FLT_MAX;
 #pragma unroll 4
   for (int s = 0; s < a.kv_splits; s++) m = fmaxf(m, rec[s * step + W]);
   float l = 0.f;

@@ -19,7 +19,7 @@
 //                                                 accumulator registers (the V side applies the same permutation
 //                                                 of the contraction index, see v_operand)
 // The maximum m the exponentials are taken against is raised lazily: a lane's 32 probabilities of a tile are summed
-// anyway, and only when such a sum leaves [0, 1024] (which includes the first tile of a row, taken against -1e30) is
+// anyway, and only when such a sum leaves [0, 1024] (which includes the first tile of a row, taken against -1e30 or lower) is
 // the true row maximum formed, sum and accumulator rescaled and the tile's exponentials redone.  No per-tile row
 // maximum: at small head sizes the vector ALUs, not the matrix pipe, bound this kernel (a score costs the same vector
 // work whatever head_dim is).
@@ -137,9 +137,10 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   for (int i = 0; i < DBLK; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) oacc[i][r] = 0.f;
-  const float c = a.scale * kLog2e;
-  float m_use = -1e30f;  // maximum the exponentials are taken against (raw scores); finite: no inf - inf
+  const float c = MASKED ? scores_unit(a) : a.scale * kLog2e;
+  float m_use = MASKED ? -FLT_MAX : -1e30f;  // maximum the exponentials are taken against; finite: no inf - inf
   float mc = m_use * c;
+  auto weight = [&](float s) __attribute__((always_inline)) { return fast_exp2(MASKED ? (s - m_use) * c : fmaf(s, c, -mc)); };
   float l_run = 0.f;     // this lane's share of the running row sum
 
   int S = a.S;  // keys of this batch entry: all of them, or the filled prefix of a cache / the unpadded length
@@ -233,11 +234,9 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   constexpr bool MASK_AHEAD = MASKED && D <= 96;
   MaskBlock<T> mask[2];
   long long mrow = 0;
-  float inv_scale = 0.f;
   if (MASKED) {
     const int qi = qw0 + lq;
     mrow = b * a.ms[0] + h * a.ms[1] + (qi < a.L ? qi : a.L - 1) * a.ms[2];
-    inv_scale = 1.f / a.scale;
   }
   auto load_mask = [&](int kv0) __attribute__((always_inline)) {
 #pragma unroll
@@ -281,7 +280,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
       if (MASKED) {
         if (!MASK_AHEAD) load_mask(kv0);
 #pragma unroll
-        for (int blk = 0; blk < 2; blk++) apply_attn_mask<T>(a, sacc[blk], mask[blk], inv_scale);
+        for (int blk = 0; blk < 2; blk++) apply_attn_mask<T>(a, sacc[blk], mask[blk]);
         if (MASK_AHEAD && jt + 1 < jt1) load_mask(kv0 + BN);
       }
 
@@ -305,7 +304,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
       for (int blk = 0; blk < 2; blk++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-          pr[blk][r] = fast_exp2(fmaf(sacc[blk][r], c, -mc));
+          pr[blk][r] = weight(sacc[blk][r]);
           psum += pr[blk][r];
         }
       if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(psum <= kSumLimit)) != 0, 0)) {  // some row of the wavefront outgrew its maximum
@@ -329,7 +328,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
           for (int r = 0; r < 16; r++) {
-            pr[blk][r] = fast_exp2(fmaf(sacc[blk][r], c, -mc));
+            pr[blk][r] = weight(sacc[blk][r]);
             psum += pr[blk][r];
           }
       }

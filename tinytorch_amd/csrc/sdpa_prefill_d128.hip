@@ -45,12 +45,13 @@
 // general form.  The eight row groups of a workgroup reach the diagonal in eight different tiles, and with the
 // general form on every one of them each of the workgroup's last five tiles waited for one wavefront in that form.
 // Under a causal mask a workgroup takes a row tile and its mirror (equal work for every workgroup), the long one first.
-// A Bool attnMask whose keys can be read four at a time (variant MASKB; the reference's masked fill, src/Function/FuncNNLayer.h:249-255)
+// A Bool attnMask whose keys can be read four at a time (variant kStreamed; the reference's masked fill, src/Function/FuncNNLayer.h:249-255)
 // stays in the pipelined form as well.  A wavefront's mask bytes of a tile (32 rows x 64 keys) come into LDS by direct loads two
 // tiles ahead, as whole 64-byte row segments (a ring of two tiles per wavefront in the area the output later leaves through,
 // idle during the loop); a step reads the lane's four dwords of the half after next from there, and its streams keep a
-// probability iff its byte is set (a byte compare through SDWA and a select per score).  Other masks (additive: a ring of 32
-// registers would be needed beside the 200 the pipelined form pins; other layouts) take the general form of a step.
+// probability iff its byte is set (a byte compare through SDWA and a select per score).  Other masks (variant kStepped; additive: a
+// ring of 32 registers would be needed beside the 200 the pipelined form pins; other layouts) take the general form of a step,
+// a variant of its own: its scores and weights are those of scores_unit (sdpa_common.h).
 // Grouped-query attention: kv head = query head / (Hq/Hkv), resolved in the kernel; the workgroup order puts the
 // query heads and row tiles that share a KV head on the same XCD so its L2 holds that K/V once.
 
@@ -89,11 +90,14 @@ __device__ __forceinline__ int swz(int row) { return ((row & 3) << 2) | ((row >>
 // SPLIT (launches with fewer row tiles than the chip needs): a workgroup takes key tiles kt0 .. kt0 + kv_chunk/64 - 1 of
 // its row tile (kt0 a multiple of 4, so the stages keep their constants) and leaves (unnormalised accumulator, maximum,
 // sum) records in a.ws for the merge kernel of the decode path; row tiles are single (no mirror pairs).
-// MASKB (calls without a causal mask, pages or splits): a.mask is a Bool mask with unit key stride, dword-aligned rows and
-// row offsets below 2^32; the steady state applies it in the streams.
-template <typename TR, bool CAUSAL, bool PAGED, bool SPLIT, bool MASKB = false>
+// kStreamed (calls without a causal mask, pages or splits): a.mask is a Bool mask with unit key stride, dword-aligned rows and
+// row offsets below 2^32; the steady state applies it in the streams.  kStepped: any other mask, without a causal mask or splits.
+enum MaskForm { kNoMask, kStreamed, kStepped };
+template <typename TR, bool CAUSAL, bool PAGED, bool SPLIT, MaskForm MASK = kNoMask>
 __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
+  constexpr bool MASKB = MASK == kStreamed, MASKS = MASK == kStepped;
   static_assert(!MASKB || (!CAUSAL && !PAGED && !SPLIT), "the Bool-mask streams exist for the plain variant only");
+  static_assert(!MASKS || (!CAUSAL && !SPLIT), "an attnMask excludes a causal one, and masked calls are not split");
   typedef typename TR::elem T;
   typedef typename TR::vec8 vec8;
 
@@ -316,7 +320,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
     if (kt0 + 2 < ntiles_kv) dma_v(kt0 + 2, 2);
   };
   issue_tiles(0);
-  // ---- Bool attnMask in the streams (MASKB) -------------------------------------------------------------------------------
+  // ---- Bool attnMask in the streams (kStreamed) -------------------------------------------------------------------------------
   // Ring in LDS: two tiles of 2 KiB per wavefront behind the K/V stages.  Load i of a tile (two per tile) brings the 64-byte
   // segments of rows 16i .. 16i+15 of the wavefront, 16 bytes per lane: lane l the chunk l/16 of row 16i + l%16, which lands at
   // 1024 i + 16 l, i.e. chunk c of row q at 1024 (q/16) + 256 c + 16 (q%16).  A lane (row q, h = lane/32) needs dwords g = 0..3 of
@@ -431,7 +435,9 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
     if (SPLIT && BN * ntiles_kv <= qc0 + WM - 1) t = ntiles_kv - 1 < t ? ntiles_kv - 1 : t;
     nfast_all = t > nfast ? t : nfast;
   }
-  if (MASKB ? S < 160 : a.mask_kind != 0) nfast = 0, nfast_all = 0;  // other attnMasks are applied in the general form of a step
+  // kStepped: always 0, and a run-time test all the same: with the streams left out of this variant the compiler keeps the general
+  // form's values elsewhere and spills 400 bytes per lane (8 x 12 heads x 776 rows, additive mask: 490 us against 134)
+  if (MASKS ? a.mask_kind != 0 : MASKB && S < 160) nfast = 0, nfast_all = 0;
   // The fast form requests its tiles without the ragged-tile case: iteration j sends for K(j+4) and V(j+3), which have to
   // be whole tiles.
   if (!PAGED && (S % BN) != 0) {
@@ -457,11 +463,11 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
   for (int db = 0; db < 4; db++)
 #pragma unroll
     for (int r = 0; r < 16; r++) oacc[db][r] = 0.f;
-  const float c = a.scale * kLog2e;
+  const float c = MASKS ? scores_unit(a) : a.scale * kLog2e;
   // the same, in a scalar register (causal step statements: their predicate operands take the freed vector register)
   const float c_s = CAUSAL ? __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, c))) : 0.f;
-  float m_use = -1e30f;  // maximum the exponentials are taken against (raw scores)
-  float mc = -1e30f * c;
+  float m_use = MASKS ? -FLT_MAX : -1e30f;  // maximum the exponentials are taken against (raw scores)
+  float mc = m_use * c;
   float l_run = 0.f;
 
   // S^T of one half tile (32 keys); kh = LDS address of the half's first K row
@@ -488,7 +494,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
   auto user_mask_half = [&](f32x16& s, int kv0) __attribute__((always_inline)) {
     int qi = qw0 + lq;
     qi = qi < a.L ? qi : a.L - 1;
-    apply_attn_mask<T>(a, s, b * a.ms[0] + h * a.ms[1] + qi * a.ms[2], kv0, lh, S, 1.f / a.scale);
+    apply_attn_mask<T>(a, s, b * a.ms[0] + h * a.ms[1] + qi * a.ms[2], kv0, lh, S);
   };
 
   auto row_max = [&](const f32x16& s) __attribute__((always_inline)) {
@@ -512,7 +518,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
       f32x8 x;
 #pragma unroll
       for (int i = 0; i < 8; i++) {
-        x[i] = fast_exp2(fmaf(s[8 * t + i], c, -mc));
+        x[i] = fast_exp2(MASKS ? (s[8 * t + i] - m_use) * c : fmaf(s[8 * t + i], c, -mc));
         psum += x[i];
       }
       pb[t] = __builtin_convertvector(x, vec8);
@@ -581,7 +587,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
     if (h + 1 < my_halves) {
       const int kv0 = 32 * (h + 1);
       if ((CAUSAL && kv0 + 31 > qc0) || kv0 + 32 > S) mask_half(s_nxt, kv0);
-      if (!CAUSAL && a.mask_kind != 0) user_mask_half(s_nxt, kv0);
+      if (MASKB || MASKS) user_mask_half(s_nxt, kv0);
       settle_half(s_nxt, p_nxt, exp_half(s_nxt, p_nxt));
     }
   };
@@ -650,7 +656,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
     qk_half(sC, half_base(0));
     if (2 * kt0 + 1 < my_halves) qk_half(sB, half_base(1));
     if ((CAUSAL && kb + 31 > qc0) || kb + 32 > S) mask_half(sC, kb);
-    if (!CAUSAL && a.mask_kind != 0) user_mask_half(sC, kb);
+    if (MASKB || MASKS) user_mask_half(sC, kb);
     // first half of a row: the maximum is formed directly (what the lazy rule arrives at after exponentials against
     // -1e30, with nothing to rescale yet); a fully hidden half keeps -1e30 and gives zeros
     m_use = fmaxf(m_use, row_max(sC));
@@ -843,13 +849,13 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
   }  // part
 }
 
-template <typename TR, bool CAUSAL, bool PAGED, bool SPLIT, bool MASKB = false>
+template <typename TR, bool CAUSAL, bool PAGED, bool SPLIT, MaskForm MASK = kNoMask>
 int launch_v(const KArgs& a, dim3 grid, hipStream_t stream) {
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  const hipError_t granted = grant_dynamic_lds((const void*)prefill128_kernel<TR, CAUSAL, PAGED, SPLIT, MASKB>, LDS_BYTES, state, done);
+  const hipError_t granted = grant_dynamic_lds((const void*)prefill128_kernel<TR, CAUSAL, PAGED, SPLIT, MASK>, LDS_BYTES, state, done);
   if (granted != hipSuccess) return (int)granted;
-  hipLaunchKernelGGL((prefill128_kernel<TR, CAUSAL, PAGED, SPLIT, MASKB>), grid, dim3(NW * 64), LDS_BYTES, stream, a);
+  hipLaunchKernelGGL((prefill128_kernel<TR, CAUSAL, PAGED, SPLIT, MASK>), grid, dim3(NW * 64), LDS_BYTES, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -857,7 +863,10 @@ template <typename TR, bool CAUSAL>
 int launch_k(const KArgs& a, dim3 grid, hipStream_t stream) {
   if (a.kv_splits > 1) return launch_v<TR, CAUSAL, false, true>(a, grid, stream);  // (the host never splits a paged call)
   if constexpr (!CAUSAL)
-    if (bool_mask_streams_ok(a)) return launch_v<TR, false, false, false, true>(a, grid, stream);
+    if (a.mask_kind != 0) {
+      if (bool_mask_streams_ok(a)) return launch_v<TR, false, false, false, kStreamed>(a, grid, stream);
+      return a.block_table ? launch_v<TR, false, true, false, kStepped>(a, grid, stream) : launch_v<TR, false, false, false, kStepped>(a, grid, stream);
+    }
   return a.block_table ? launch_v<TR, CAUSAL, true, false>(a, grid, stream) : launch_v<TR, CAUSAL, false, false>(a, grid, stream);
 }
 

@@ -441,7 +441,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill64_kernel(KArgs a) {
   auto user_mask_half = [&](f32x16& s, int kv0) __attribute__((always_inline)) {
     int qi = qw0 + lq;
     qi = qi < a.L ? qi : a.L - 1;
-    apply_attn_mask<T>(a, s, b * a.ms[0] + h * a.ms[1] + qi * a.ms[2], kv0, lh, S, 1.f / a.scale);
+    apply_attn_mask<T>(a, s, b * a.ms[0] + h * a.ms[1] + qi * a.ms[2], kv0, lh, S);
   };
 
   auto row_max = [&](const f32x16& s) __attribute__((always_inline)) {

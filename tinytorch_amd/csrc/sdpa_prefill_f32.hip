@@ -113,9 +113,9 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
   for (int i = 0; i < DBLK; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) oacc[i][r] = 0.f;
-  const float c = a.scale * kLog2e;
+  const float c = MASKED ? scores_unit(a) : a.scale * kLog2e;
   const float lazy = kLazyExp / c;
-  float m_use = -1e30f;
+  float m_use = MASKED ? -FLT_MAX : -1e30f;
   float mc = m_use * c;
   float l_run = 0.f;
 
@@ -190,11 +190,9 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
   const int v_lane = 4 * lh * V_PITCH + lq;        // floats; + (8*(t/4) + t%4) * V_PITCH + 32*db
 
   long long mrow = 0;
-  float inv_scale = 0.f;
   if (MASKED) {
     const int qi = qw0 + lq;
     mrow = b * a.ms[0] + h * a.ms[1] + (qi < a.L ? qi : a.L - 1) * a.ms[2];
-    inv_scale = 1.f / a.scale;
   }
 
   if (KEYS) {
@@ -243,7 +241,7 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
 #pragma unroll
       for (int r = 0; r < 16; r++) s[r] = s0[r] + s1[r];
 
-      if (MASKED) apply_attn_mask<float>(a, s, mask, inv_scale);
+      if (MASKED) apply_attn_mask<float>(a, s, mask);
 
       // ---- mask the diagonal / ragged tile -----------------------------------------------------------------------------
       if ((CAUSAL && kv0 + BN - 1 > pos_lo + coff) || (kv0 + BN > S)) {
@@ -275,7 +273,7 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
       float psum = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        s[r] = fast_exp2(fmaf(s[r], c, -mc));
+        s[r] = fast_exp2(MASKED ? (s[r] - m_use) * c : fmaf(s[r], c, -mc));
         psum += s[r];
       }
       l_run += psum;

@@ -381,9 +381,10 @@ bool backward_on_mfma(const ttsdpa_backward_params* p) {
   return pick_backward_route(p) != TTSDPA_ROUTE_NONE && (backward_mfma_ok(p, true) || backward_f32_ok(p, true));
 }
 
-size_t backward_stats_bytes(const ttsdpa_backward_params* p) {
-  return (size_t)p->fwd.B * p->fwd.Hq * p->fwd.L * 2 * sizeof(float);
-}
+// The rows' statistics: (statistic, delta) pairs, then log_sums where the kernels keep one (BwdArgs).
+size_t backward_rows(const ttsdpa_backward_params* p) { return (size_t)p->fwd.B * p->fwd.Hq * p->fwd.L; }
+bool backward_log_sums(const ttsdpa_backward_params* p) { return p->fwd.mask_kind != TTSDPA_MASK_NONE || !backward_on_mfma(p); }
+size_t backward_stats_bytes(const ttsdpa_backward_params* p) { return backward_rows(p) * (backward_log_sums(p) ? 3 : 2) * sizeof(float); }
 
 // Scratch layout: the statistics, then (matrix-core pairs with a split query stream) the partial dk / dv, 256-byte aligned.
 int dkv_splits_of(const ttsdpa_backward_params* p, bool* dealt = nullptr) {
@@ -659,6 +660,7 @@ int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t wor
   const size_t need = backward_scratch_bytes(p);
   if (need > 0 && (!workspace || workspace_bytes < need || !ptr_aligned(workspace, 16))) return TTSDPA_ERR_WORKSPACE;
   a.stats = (float*)workspace;
+  a.log_sums = backward_log_sums(p) ? a.stats + 2 * backward_rows(p) : nullptr;
   a.dkv_splits = dkv_splits_of(p, &a.dkv_dealt);
   a.partial = a.dkv_splits > 1 ? (float*)((char*)workspace + backward_partial_offset(p)) : nullptr;
   a.dq_splits = dq_splits_of(p, &a.dq_dealt);
