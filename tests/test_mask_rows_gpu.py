@@ -127,3 +127,34 @@ def test_backward_far_values(shape, D, dtype):
     B, Hq, Hkv, L, S = shape
     q, k, v, g = operands(sum(shape) + D, B, Hq, Hkv, L, S, D, dtype)
     check_backward(q, k, v, g, additive(L, S, dtype), dtype)
+
+
+@pytest.mark.parametrize("kind", ["bool", "add"])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("D", [64, 80, 128, 90])
+@pytest.mark.parametrize("shape", BACKWARD_SHAPES, ids=str)
+def test_backward_hidden_rows(shape, D, dtype, kind):
+    """The forward's own output (NaN in such rows) goes back in: dq is 0 there, dk and dv hold the other rows' sums."""
+    print("backward, hidden rows", shape, D, dtype, kind, flush=True)
+    B, Hq, Hkv, L, S = shape
+    q, k, v, g = operands(sum(shape) + D, B, Hq, Hkv, L, S, D, dtype)
+    seen = torch.rand(L, S, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda") < 0.6
+    seen[:, S // 2] = True
+    seen[3::7] = False
+    seen[L - 1] = False
+    mask = seen if kind == "bool" else torch.zeros(L, S, device="cuda", dtype=DT[dtype]).masked_fill(~seen, -math.inf)
+    assert tt.sdpAttention(q, k, v, attnMask=mask)[:, :, 3::7].isnan().all()
+    dq = check_backward(q, k, v, g, mask, dtype)[0]
+    assert torch.count_nonzero(dq[:, :, 3::7]).item() == 0
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("S", [203, 204])
+def test_backward_hidden_rows_beside_key_counts(S, dtype):
+    B, H, L, D = 3, 4, 70, 64
+    q, k, v, g = operands(6, B, H, H, L, S, D, dtype)
+    lens = torch.tensor([S, 66, 1], device="cuda", dtype=torch.int32)
+    seen = torch.rand(L, S, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda") < 0.6
+    seen[5], seen[6, :66] = False, False
+    _, dk, dv = check_backward(q, k, v, g, seen, dtype, lens)
+    assert torch.count_nonzero(dk[1, :, 66:]).item() == 0 and torch.count_nonzero(dv[2, :, 1:]).item() == 0

@@ -377,8 +377,8 @@ __global__ __launch_bounds__(256, 2) void backward_dq_mfma_kernel(BwdArgs a) {
     // a row whose keys are all hidden (possible with an attnMask): dq = 0, and a statistic that gives it weight 0 below
     const bool seen = l_tot > 0.f;
     if (lh == 0) {
-      *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_use * c + __log2f(l_tot) : 1e30f, delta);
-      if (MASKED) store_masked_stat(a, row_id, seen, m_use, l_tot);
+      if (MASKED) store_masked_stat(a, row_id, seen, m_use, l_tot, delta);
+      else *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_use * c + __log2f(l_tot) : 1e30f, delta);
     }
     const float w = seen ? f.scale / l_tot : 0.f;
     T* dqp = (T*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];

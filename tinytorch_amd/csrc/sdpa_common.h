@@ -428,9 +428,10 @@ __device__ __forceinline__ void store_dq_partial(const BwdArgs& a, int piece, lo
 }
 
 // A row's statistics in a call with an attnMask (matrix-core pairs); a row whose keys are all hidden gets a maximum and a
-// logarithm that give it weight 0 in the dk/dv kernel.
-__device__ __forceinline__ void store_masked_stat(const BwdArgs& a, long long row_id, bool seen, float m, float l) {
-  a.stats[2 * row_id] = seen ? m : FLT_MAX;
+// logarithm that give it weight 0 in the dk/dv kernel, and a delta of 0: its own is NaN (the forward's output there), which 0
+// times would leave in dk.
+__device__ __forceinline__ void store_masked_stat(const BwdArgs& a, long long row_id, bool seen, float m, float l, float delta) {
+  *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m : FLT_MAX, seen ? delta : 0.f);
   a.log_sums[row_id] = seen ? __log2f(l) : 1e30f;
 }
 
@@ -478,7 +479,7 @@ __global__ __launch_bounds__(256) void backward_dq_merge_kernel(BwdArgs a, long 
   for (int e = 0; e < 4; e++) x[e] = seen ? x[e] * w : 0.f;
   *out = __builtin_convertvector(x, vec4t);
   if (d == 0) {
-    if (f.mask_kind != 0) store_masked_stat(a, row_id, seen, m, l);
+    if (f.mask_kind != 0) store_masked_stat(a, row_id, seen, m, l, a.stats[2 * row_id + 1]);
     else a.stats[2 * row_id] = seen ? m + __log2f(l) : 1e30f;
   }
 }
