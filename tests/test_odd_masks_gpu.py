@@ -46,3 +46,60 @@ def test_strided_mask_and_key_counts(dtype):
         exp = oracle.sdpa_f32(host[0][b:b + 1], host[1][b:b + 1, :, :n], host[2][b:b + 1, :, :n],
                               mask=np.ascontiguousarray(m.T[:, :n]).astype(np.uint8))
         assert np.abs(to_host_f32(out[b:b + 1]) - exp).max() <= TOL[dtype], b
+
+
+def _against_64_bits(out, host, mask):
+    """Relative error (2-norm), and the share of results that are not the 64-bit result rounded once."""
+    q, k, v = (torch.from_numpy(t).double().cuda() for t in host)
+    G = q.shape[1] // k.shape[1]
+    k, v = k.repeat_interleave(G, 1), v.repeat_interleave(G, 1)
+    s = torch.matmul(q, k.transpose(-1, -2).contiguous()) / q.shape[-1] ** 0.5
+    s = s.masked_fill(~mask, -float("inf")) if mask.dtype == torch.bool else s + mask.double()
+    ref = torch.matmul(torch.softmax(s, -1), v)
+    return ((out.double() - ref).norm() / ref.norm()).item(), (out != ref.to(out.dtype)).double().mean().item()
+
+
+@pytest.mark.parametrize("kind", ["bool", "add"])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("L,S,D", [(37, 197, 64), (197, 197, 64), (130, 333, 32), (101, 901, 80), (70, 333, 128), (33, 335, 96), (37, 203, 192),
+                                   (64, 333, 256)])
+@pytest.mark.parametrize("steep", [False, True])
+def test_probabilities_are_fp32(L, S, D, dtype, kind, steep):
+    """16-bit calls of the general route: as close to the 64-bit result as the vector-ALU kernel, whose probabilities are fp32
+    (bf16 ones, 2^-9 each, leave four results of ten off by a rounding).  steep: scores spread over some 20, and the key
+    with the most weight holds zeros, so that the result is that of the small probabilities."""
+    B, Hq, Hkv = 2, 4, 2
+    print("fp32 probabilities", L, S, D, dtype, kind, steep, flush=True)
+    host, dev = make_inputs(8950 + S, B, Hq, Hkv, L, S, D, dtype, 2.0 if steep else 1.0)
+    rng = np.random.default_rng(S)
+    m = rng.random((L, S)) > 0.3
+    m[:, S // 2] = True
+    md = torch.from_numpy(m).cuda()
+    if kind == "add":
+        md = torch.from_numpy(rng.standard_normal((L, S)).astype(np.float32)).cuda().to(dev[0].dtype)
+    if steep:
+        md = md.clone()
+        md[:, 3] = True if kind == "bool" else 12.0
+        host[2][:, :, 3] = 0
+        dev[2][:, :, 3] = 0
+    got, vec = call("forward", *dev, mask=md), call("general", *dev, mask=md)
+    assert got[0] == 0 and vec[0] == 0
+    err, off = _against_64_bits(got[1], host, md)
+    err0, off0 = _against_64_bits(vec[1], host, md)
+    # sums of S fp32 terms in another order: 2^-24 sqrt(S) against a rounding of 2^-12 (fp16) at most changes the result's rounding once in 2^-12 / that
+    assert err <= err0 * 1.001 and off <= off0 * 1.1 + 2e-3, (err, err0, off, off0)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("S", [197, 901])
+def test_infinite_values(S, dtype):
+    """Infinities and NaN in V (the last key's row among them) come out where the vector-ALU kernel has them."""
+    host, dev = make_inputs(8990, 2, 4, 4, 37, S, 64, dtype)
+    q, k, v = dev
+    m = torch.from_numpy(np.random.default_rng(1).random((37, S)) > 0.3).cuda()
+    m[:, [5, 70, S - 1]] = True
+    v[0, 0, 5, 3], v[0, 1, S - 1, 4], v[1, 0, 70, 7], v[1, 2, 5, :] = float("inf"), -float("inf"), float("nan"), 60000.0
+    got, vec = call("forward", q, k, v, mask=m), call("general", q, k, v, mask=m)
+    assert got[0] == 0 and vec[0] == 0
+    assert torch.equal(got[1].isnan(), vec[1].isnan()) and torch.equal(got[1].isinf(), vec[1].isinf())
+    assert torch.isinf(got[1]).any() and torch.equal(torch.sign(got[1][got[1].isinf()]), torch.sign(vec[1][vec[1].isinf()]))

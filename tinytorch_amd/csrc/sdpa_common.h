@@ -33,6 +33,7 @@ struct KArgs {
   // tile_split_merge_kernel or prefill_split_merge_kernel combines them.  kv_splits <= 1: no split.
   int kv_splits, kv_chunk;
   float* ws;
+  int full_p;  // 4-wavefront prefill kernel with an attnMask: probabilities reach the matrix cores with all their fp32 bits
   int mask_vec4;  // keys are contiguous in the mask and groups of 4 keys starting at a multiple of 4 are naturally aligned
   // Pipelined prefill kernels under a causal mask: 0 = a workgroup takes a row tile and its mirror (equal work for all),
   // 1 = one row tile per workgroup, longest first (launches whose pairs would leave CUs without a workgroup).
@@ -94,6 +95,20 @@ struct BF16 {
   static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
+  static constexpr int kParts = 3;  // parts that hold an fp32 number
+  // the leading bits of eight numbers, which are left with the rest (exactly)
+  static __device__ __forceinline__ vec8 take_part(f32x8& x) {
+    u32x4 w;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float x0 = x[2 * i], x1 = x[2 * i + 1];
+      const uint32_t a = __builtin_bit_cast(uint32_t, x0), b = __builtin_bit_cast(uint32_t, x1);
+      w[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);  // their upper halves
+      x[2 * i] = x0 - __builtin_bit_cast(float, a & 0xffff0000u);
+      x[2 * i + 1] = x1 - __builtin_bit_cast(float, b & 0xffff0000u);
+    }
+    return __builtin_bit_cast(vec8, w);
+  }
   // fp32 value of the low / high 16-bit half of a packed pair
   static __device__ __forceinline__ float lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
   static __device__ __forceinline__ float hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
@@ -108,6 +123,18 @@ struct F16 {
   }
   static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+  static constexpr int kParts = 2;  // to 2^-22 of it
+  static __device__ __forceinline__ vec8 take_part(f32x8& x) {
+    vec8 y;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const auto w = __builtin_amdgcn_cvt_pkrtz(x[2 * i], x[2 * i + 1]);  // (towards zero)
+      y[2 * i] = w[0], y[2 * i + 1] = w[1];
+      x[2 * i] = fmaf(-1.f, (float)w[0], x[2 * i]);
+      x[2 * i + 1] = fmaf(-1.f, (float)w[1], x[2 * i + 1]);
+    }
+    return y;
   }
   static __device__ __forceinline__ float lo(uint32_t w) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu));

@@ -28,6 +28,8 @@
 // Grouped-query attention: kv head = query head / (Hq/Hkv), resolved in the kernel; the workgroup order puts the
 // query heads and row tiles that share a KV head on the same XCD so its L2 holds that K/V once.
 
+#include <type_traits>
+
 #include "sdpa_common.h"
 
 namespace ttsdpa {
@@ -46,7 +48,7 @@ struct PrefillLds {
   static constexpr int K_PITCH = D + 8;   // elements; rows 16 B apart in bank space: 32 rows x b128 conflict-free
   static constexpr int V_PITCH = D + 32;  // elements; rows 64 B apart in bank space: 4 rows x 64 B conflict-free
   static constexpr int STAGE = BN * (K_PITCH + V_PITCH);  // elements per stage
-  static constexpr int BYTES = 2 * STAGE * 2;
+  static constexpr int BYTES = 2 * STAGE * 2 + 2 * 4 * 4;  // ... and FULLP's flags: [stage][wavefront]
 };
 
 // One MFMA A operand of V^T from a row-major V tile: lane l (column d = d0 + l%32, half h = l/32) receives the
@@ -63,10 +65,19 @@ __device__ __forceinline__ vec8 v_operand(const void* lane_base, int byte_off_lo
 }
 
 // MASKED: an attnMask is applied (a variant of its own: the mask addressing costs registers the other variants keep).
+// FULLP (with MASKED): the probabilities are fp32 in P.V too, for the calls of the general route, whose arithmetic is fp32.  A
+// probability goes to the matrix cores in parts (take_part): three in bf16, which hold its 24 bits; two in fp16, which hold it
+// to 2^-22 of itself or, fp16's range being short, 2^-35 of the row's largest: there the exponentials carry a factor of 2^10
+// (it cancels when the row is normalised), and their sums may reach 2^15 only.  The first parts are accumulated for all of
+// the tile, then the others, with V read again (all parts of an operand at a time cost 100 registers and spilled).  Infinities
+// and NaN in V meet the first part only: times a part that is 0 they would be NaN where the probability gives infinity; the
+// wavefronts look for them in what they bring to LDS, and a tile that has some loses them between the two passes.  Error
+// against 64 bits: the vector-ALU kernel's (tests/test_odd_masks_gpu.py).  16 x 12 heads x 197 rows, head_dim 64, fp16, key
+// padding: 16.1 us with 16-bit probabilities, 18.0 so, 124 on the vector ALUs; 8 x 12 x 777 x 80: 71, 86, 1294.
 // PAD: the tensors' head_dim a.D is a multiple of 8 below D.  The 16-byte chunks of a row beyond a.D are taken as zeros
 // (Q and K: they add nothing to a score; V: columns of the output that are not stored), everything else is the
 // kernel for head_dim D.  The reference takes any head size (src/Function/FuncNNLayer.h:231-236).
-template <typename TR, int D, bool CAUSAL, bool MASKED, bool PAD>
+template <typename TR, int D, bool CAUSAL, bool MASKED, bool PAD, bool FULLP>
 __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a) {
   typedef typename TR::elem T;
   typedef typename TR::vec8 vec8;
@@ -75,6 +86,8 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   constexpr int KSTEPS = D / 16;           // MFMAs along head_dim for S^T
   constexpr int DBLK = D / 32;             // 32-row blocks of O^T
   constexpr int NLD = (BN * D / 8) / 256;  // 16-byte chunks per thread per tile, for K and for V
+  constexpr bool SHIFT = FULLP && __is_same(T, _Float16);
+  constexpr float kMostSum = SHIFT ? 32768.f : kSumLimit;
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* smem = (T*)smem_raw;
@@ -140,7 +153,9 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   const float c = MASKED ? scores_unit(a) : a.scale * kLog2e;
   float m_use = MASKED ? -FLT_MAX : -1e30f;  // maximum the exponentials are taken against; finite: no inf - inf
   float mc = m_use * c;
-  auto weight = [&](float s) __attribute__((always_inline)) { return fast_exp2(MASKED ? (s - m_use) * c : fmaf(s, c, -mc)); };
+  auto weight = [&](float s) __attribute__((always_inline)) {
+    return fast_exp2(SHIFT ? fmaf(s - m_use, c, 10.f) : MASKED ? (s - m_use) * c : fmaf(s, c, -mc));
+  };
   float l_run = 0.f;     // this lane's share of the running row sum
 
   int S = a.S;  // keys of this batch entry: all of them, or the filled prefix of a cache / the unpadded length
@@ -205,16 +220,19 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
         kst[i] = *(const u32x4*)(kt + koff[i]);
         vst[i] = *(const u32x4*)(vt + voff[i]);
       }
-    } else {  // ragged last tile: rows past the end re-read the last valid row (masked later)
+    } else {  // ragged last tile: rows past the end re-read the last valid row (masked later; FULLP: zeros for V)
 #pragma unroll
       for (int i = 0; i < NLD; i++) {
         int row = lrow[i];
         row = kv0 + row < S ? row : S - 1 - kv0;
         kst[i] = *(const u32x4*)(ktile + row * a.ks[2] + 8 * gcol[i]);
-        vst[i] = *(const u32x4*)(vtile + row * a.vs[2] + 8 * gcol[i]);
+        if (FULLP) vst[i] = u32x4{0u, 0u, 0u, 0u};
+        if (!FULLP || kv0 + lrow[i] < S) vst[i] = *(const u32x4*)(vtile + row * a.vs[2] + 8 * gcol[i]);
       }
     }
   };
+  constexpr uint32_t kExponent = __is_same(T, _Float16) ? 0x7c007c00u : 0x7f807f80u;  // of two values: all ones in infinities and NaN
+  int* vflags = (int*)(smem + 2 * Lds::STAGE);
   auto store_tile = [&](int stage) {
     T* Ks = smem + stage * Lds::STAGE;
     T* Vs = Ks + BN * K_PITCH;
@@ -223,6 +241,15 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
       const u32x4 zero = {0u, 0u, 0u, 0u};
       *(u32x4*)(Ks + lrow[i] * K_PITCH + 8 * lcol[i]) = cval[i] ? kst[i] : zero;
       *(u32x4*)(Vs + lrow[i] * V_PITCH + 8 * lcol[i]) = cval[i] ? vst[i] : zero;
+    }
+    if constexpr (FULLP) {
+      uint32_t odd = 0;  // the exponent's lowest bit added: a carry into the sign's place where it is all ones
+#pragma unroll
+      for (int i = 0; i < NLD; i++)
+#pragma unroll
+        for (int w = 0; w < 4; w++) odd |= ((vst[i][w] & 0x7fff7fffu) + (kExponent & -kExponent & 0xffffu) * 0x10001u) & 0x80008000u;
+      const bool any = __builtin_amdgcn_ballot_w64(odd != 0) != 0;
+      if (lane == 0) vflags[4 * stage + wave] = any;
     }
   };
 
@@ -259,7 +286,9 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
       if (jt + 2 < jt1) load_tile(kv0 + 2 * BN);
     }
 
-    if (qw0 < a.L && (!CAUSAL || kv0 <= pos_hi + coff)) {  // else: no rows here, or the whole tile is above the diagonal
+    const bool live = qw0 < a.L && (!CAUSAL || kv0 <= pos_hi + coff);  // else: no rows here, or the whole tile is above the diagonal
+    f32x16 pr[2];
+    if (live) {
       const T* Ks = smem + cur * Lds::STAGE;
       const T* Vs = Ks + BN * K_PITCH;
 
@@ -299,7 +328,6 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
       }
       // ---- online softmax with a lazily raised maximum ---------------------------------------------------------------
       float psum = 0.f;
-      f32x16 pr[2];
 #pragma unroll
       for (int blk = 0; blk < 2; blk++)
 #pragma unroll
@@ -307,7 +335,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
           pr[blk][r] = weight(sacc[blk][r]);
           psum += pr[blk][r];
         }
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(psum <= kSumLimit)) != 0, 0)) {  // some row of the wavefront outgrew its maximum
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(psum <= kMostSum)) != 0, 0)) {  // some row of the wavefront outgrew its maximum
         float mloc = sacc[0][0];
 #pragma unroll
         for (int blk = 0; blk < 2; blk++)
@@ -341,7 +369,13 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
         f32x8 x;
 #pragma unroll
         for (int i = 0; i < 8; i++) x[i] = pr[t >> 1][8 * (t & 1) + i];
-        pb[t] = __builtin_convertvector(x, vec8);
+        if constexpr (FULLP) {
+          pb[t] = TR::take_part(x);
+#pragma unroll
+          for (int i = 0; i < 8; i++) pr[t >> 1][8 * (t & 1) + i] = x[i];
+        } else {
+          pb[t] = __builtin_convertvector(x, vec8);
+        }
       }
 
       // ---- O^T += V^T . P^T ---------------------------------------------------------------------------------------------
@@ -352,6 +386,37 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
         for (int t = 0; t < 4; t++) {
           vec8 va = v_operand<vec8>(vl, ((16 * t) * V_PITCH + 32 * db) * 2, ((16 * t + 8) * V_PITCH + 32 * db) * 2);
           oacc[db] = TR::mfma32(va, pb[t], oacc[db]);
+        }
+      }
+    }
+    if constexpr (FULLP) {  // what the first parts left of the probabilities
+      T* Vs = smem + cur * Lds::STAGE + BN * K_PITCH;
+      const int* flags = vflags + 4 * cur;
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(flags[0] | flags[1] | flags[2] | flags[3]) != 0, 0)) {
+        __syncthreads();
+        for (int e = tid; e < BN * D; e += 256) {
+          T* at = Vs + e / D * V_PITCH + e % D;
+          if (!__builtin_isfinite((float)*at)) *at = (T)0.f;
+        }
+        __syncthreads();
+      }
+      if (live) {
+        const T* vl = Vs + v_lane;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          f32x8 x;
+#pragma unroll
+          for (int i = 0; i < 8; i++) x[i] = pr[t >> 1][8 * (t & 1) + i];
+          vec8 part[TR::kParts - 1];
+#pragma unroll
+          for (int j = 0; j + 2 < TR::kParts; j++) part[j] = TR::take_part(x);
+          part[TR::kParts - 2] = __builtin_convertvector(x, vec8);
+#pragma unroll
+          for (int db = 0; db < DBLK; db++) {
+            vec8 va = v_operand<vec8>(vl, ((16 * t) * V_PITCH + 32 * db) * 2, ((16 * t + 8) * V_PITCH + 32 * db) * 2);
+#pragma unroll
+            for (int j = TR::kParts - 2; j >= 0; j--) oacc[db] = TR::mfma32(va, part[j], oacc[db]);
+          }
         }
       }
     }
@@ -392,13 +457,13 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   }
 }
 
-template <typename TR, int D, bool CAUSAL, bool MASKED, bool PAD>
+template <typename TR, int D, bool CAUSAL, bool MASKED, bool PAD, bool FULLP = false>
 int launch_prefill_k(const KArgs& a, dim3 grid, hipStream_t stream) {
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  const hipError_t granted = grant_dynamic_lds((const void*)prefill_kernel<TR, D, CAUSAL, MASKED, PAD>, PrefillLds<D>::BYTES, state, done);
+  const hipError_t granted = grant_dynamic_lds((const void*)prefill_kernel<TR, D, CAUSAL, MASKED, PAD, FULLP>, PrefillLds<D>::BYTES, state, done);
   if (granted != hipSuccess) return (int)granted;
-  hipLaunchKernelGGL((prefill_kernel<TR, D, CAUSAL, MASKED, PAD>), grid, dim3(256), PrefillLds<D>::BYTES, stream, a);
+  hipLaunchKernelGGL((prefill_kernel<TR, D, CAUSAL, MASKED, PAD, FULLP>), grid, dim3(256), PrefillLds<D>::BYTES, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -408,7 +473,8 @@ int launch_prefill_t(const KArgs& a, hipStream_t stream) {
   if (PAD && (a.D % 8 != 0 || a.D >= D || a.D < 8)) return (int)hipErrorInvalidValue;
   long long nwg = (long long)a.B * a.Hq * ((a.L + BM - 1) / BM) * (a.kv_splits > 1 ? a.kv_splits : 1);
   dim3 grid((unsigned)nwg);
-  if (a.mask_kind != 0) return launch_prefill_k<TR, D, false, true, PAD>(a, grid, stream);  // exclusive with causal (validated)
+  if (a.mask_kind != 0)  // exclusive with causal (validated)
+    return a.full_p ? launch_prefill_k<TR, D, false, true, PAD, true>(a, grid, stream) : launch_prefill_k<TR, D, false, true, PAD>(a, grid, stream);
   return a.causal ? launch_prefill_k<TR, D, true, false, PAD>(a, grid, stream) : launch_prefill_k<TR, D, false, false, PAD>(a, grid, stream);
 }
 

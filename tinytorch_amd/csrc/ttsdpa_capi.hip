@@ -64,7 +64,7 @@ int validate(const ttsdpa_params* p, KArgs* a) {
   }
   if (p->mask_kind == TTSDPA_MASK_ADD && !ptr_aligned(p->mask, esz)) return TTSDPA_ERR_STRIDE;
   a->mask_vec4 = mask_vec4_ok(p) ? 1 : 0;
-  a->single_tiles = 0;
+  a->single_tiles = 0, a->full_p = 0;
   a->pack_L = 0, a->kv_splits = 1, a->kv_chunk = 0, a->ws = nullptr;
   if (p->kv_len && !ptr_aligned(p->kv_len, 4)) return TTSDPA_ERR_STRIDE;
   a->kv_len = p->kv_len;
@@ -564,6 +564,7 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
         check_grid((long long)a.B * a.Hkv * pl.splits) == TTSDPA_OK)
       return launch_decode(a, p->dtype, workspace, (hipStream_t)stream);
   }
+  a.full_p = p->mask_kind != TTSDPA_MASK_NONE && !simple_mask_ok(p);  // (any_mask: the general route's calls, its arithmetic)
   auto launch = [&](const KArgs& k) {
     return p->dtype == TTSDPA_F32 ? launch_prefill_f32(k, (hipStream_t)stream) : launch_prefill(k, p->dtype, (hipStream_t)stream);
   };
