@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import TOL, call, make_inputs, to_device, to_host_f32
+from gpu_util import TOL, backward_call, call, make_inputs, to_device, to_host_f32
 
 pytestmark = pytest.mark.gpu
 
@@ -103,3 +103,43 @@ def test_infinite_values(S, dtype):
     assert got[0] == 0 and vec[0] == 0
     assert torch.equal(got[1].isnan(), vec[1].isnan()) and torch.equal(got[1].isinf(), vec[1].isinf())
     assert torch.isinf(got[1]).any() and torch.equal(torch.sign(got[1][got[1].isinf()]), torch.sign(vec[1][vec[1].isinf()]))
+
+
+def _gradients_64(host, go, md):
+    q, k, v = (torch.from_numpy(t).double().cuda() for t in host)
+    G, g = q.shape[1] // k.shape[1], go.double()
+    kk, vv = k.repeat_interleave(G, 1), v.repeat_interleave(G, 1)
+    s = torch.matmul(q, kk.transpose(-1, -2).contiguous()) / q.shape[-1] ** 0.5
+    p = torch.softmax(s.masked_fill(~md, -float("inf")) if md.dtype == torch.bool else s + md.double(), -1)
+    return p, q, kk, vv, g, (lambda t: t.view(t.shape[0], -1, G, *t.shape[2:]).sum(2))
+
+
+@pytest.mark.parametrize("kind", ["bool", "add"])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,D", [(2, 4, 2, 37, 197, 64), (1, 1, 1, 33, 65, 32), (4, 16, 16, 260, 333, 64), (1, 4, 2, 130, 901, 80),
+                                            (1, 4, 1, 70, 333, 128), (4, 16, 8, 140, 203, 120)])
+@pytest.mark.parametrize("size", [1.0, 1e-6, 3e3])
+def test_gradients_are_fp32(B, Hq, Hkv, L, S, D, dtype, kind, size):
+    """16-bit calls of the general route: P and dS are fp32, so that an upstream gradient of any size of the type gives the 64-bit
+    result rounded once (16-bit dS: off by several roundings, lost to zero below 1e-7 in fp16 and infinite beyond 65504)."""
+    print("fp32 gradients", B, Hq, Hkv, L, S, D, dtype, kind, size, flush=True)
+    host, dev = make_inputs(8970 + S, B, Hq, Hkv, L, S, D, dtype)
+    rng = np.random.default_rng(S)
+    m = rng.random((L, S)) > 0.3
+    m[:, S // 2] = True
+    md = torch.from_numpy(m).cuda() if kind == "bool" else torch.from_numpy(rng.standard_normal((L, S)).astype(np.float32)).cuda().to(dev[0].dtype)
+    go = (torch.from_numpy(rng.standard_normal((B, Hq, L, D)).astype(np.float32)).cuda() * size).to(dev[0].dtype)
+    rc, out = call("forward", *dev, mask=md)
+    assert rc == 0
+    rc, grads = backward_call(*dev, out, go, mask=md)
+    assert rc == 0
+    p, q, kk, vv, g, group = _gradients_64(host, go, md)
+    # delta is dout . out with the forward's rounded output, as the backward is defined
+    ds = p * (torch.matmul(g, vv.transpose(-1, -2).contiguous()) - (g * out.double()).sum(-1, keepdim=True)) / D ** 0.5
+    refs = (torch.matmul(ds, kk), group(torch.matmul(ds.transpose(-1, -2).contiguous(), q)), group(torch.matmul(p.transpose(-1, -2).contiguous(), g)))
+    for name, got, ref in zip(("dq", "dk", "dv"), grads, refs):
+        assert torch.isfinite(got).all(), name
+        # one rounding of the result, and sums of fp32 terms in another order: a rounding in a hundred may go the other way
+        want = ref.to(got.dtype)
+        assert (got != want).double().mean().item() <= 0.01, name
+        assert ((got.double() - ref).norm() / ref.norm()).item() <= 1.001 * ((want.double() - ref).norm() / ref.norm()).item() + 1e-7, name

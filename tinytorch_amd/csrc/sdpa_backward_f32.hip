@@ -1,4 +1,4 @@
-// Attention backward for fp32 tensors on the gfx950 fp32 matrix cores (v_mfma_f32_32x32x2_f32: full fp32 products and
+// Attention backward in fp32 on the gfx950 fp32 matrix cores (v_mfma_f32_32x32x2_f32: full fp32 products and
 // sums), head_dim 64 or 128, optional causal mask (either alignment) or attnMask, per-batch key counts, grouped heads.
 // fp32 is the reference's default dtype.  The reference has no attention backward (reference
 // src/Function/FuncNNLayer.h:267 is NOT_IMPLEMENTED); this is the chain rule through its forward chain matmul -> scale -> bias -> softmax -> matmul
@@ -27,6 +27,12 @@
 // stage of LDS of its own, and add their sums through LDS: a stream of a few tiles is one or two long, without the second
 // launch and the records of a split (4 heads x 128 x 64: dq 10.9 + 4.3 us in four splits, dk/dv 11.7 + 3.9).
 // No atomics: a fixed summation order, reproducible results.
+// E, the tensors' element type: fp32, or with an attnMask fp16 / bf16 as well, for the calls that only their mask's layout keeps
+// off the 16-bit pair: the general route's arithmetic is fp32, and P and dS rounded to 16 bits (dS beyond fp16's range
+// altogether, where gradients are large) would not be.  16-bit rows become fp32 on their way into LDS and registers.  16 x 12 heads x 197
+// rows, head_dim 64, fp16, key padding: 149 us, 324 on the vector ALUs (46 on the 16-bit pair); 8 x 12 x 777 x 128 1390, 5245 (340).
+
+#include <type_traits>
 
 #include "sdpa_common.h"
 
@@ -45,6 +51,9 @@ struct BwdF32Lds {
   static constexpr int STAGE = 2 * TILE + 3 * BT;     // two tiles and, in kernel 2, (statistic, delta) and log_sums per query row
   static constexpr int BYTES = 2 * STAGE * 4;         // double-buffered
 };
+
+template <typename E>
+using Row4 = E __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x16 zero16() {
   f32x16 x;
@@ -68,15 +77,15 @@ __device__ __forceinline__ f32x16 score_product(const float* xrow, const float (
   return s0;
 }
 
-// This lane's half (lh) of a row of D floats, 16 bytes at a time; the row holds `have` floats (a multiple of 4, at most
+// This lane's half (lh) of a row of D elements, four at a time; the row holds `have` elements (a multiple of 4, at most
 // D), the rest reads as zeros.
-template <int D>
-__device__ __forceinline__ void load_half_row(const float* row, int lh, float (&reg)[D / 2], int have) {
-  const float* p = row + lh * (D / 2);
+template <int D, typename E>
+__device__ __forceinline__ void load_half_row(const E* row, int lh, float (&reg)[D / 2], int have) {
+  const E* p = row + lh * (D / 2);
 #pragma unroll
   for (int i = 0; i < D / 8; i++) {
     f32x4 t = {0.f, 0.f, 0.f, 0.f};
-    if (lh * (D / 2) + 4 * i < have) t = *(const f32x4*)(p + 4 * i);
+    if (lh * (D / 2) + 4 * i < have) t = __builtin_convertvector(*(const Row4<E>*)(p + 4 * i), f32x4);
 #pragma unroll
     for (int e = 0; e < 4; e++) reg[4 * i + e] = t[e];
   }
@@ -87,7 +96,7 @@ __device__ __forceinline__ void load_half_row(const float* row, int lh, float (&
 // PAD (both kernels): the tensors' head_dim f.D is a multiple of 4 below D.  The 16-byte chunks of a row beyond it are
 // taken as zeros (q, k: nothing added to a score; dout, v: nothing added to dP or delta; gradient columns beyond f.D are
 // not stored, records of splits hold f.D of them); everything else is the kernel for head_dim D.
-template <int D, bool CAUSAL, bool MASKED, bool PAD, bool DEAL>
+template <typename E, int D, bool CAUSAL, bool MASKED, bool PAD, bool DEAL>
 __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32_kernel(BwdArgs a) {
   typedef BwdF32Lds<D> Lds;
   constexpr int PITCH = Lds::PITCH, DBLK = D / 32;
@@ -116,8 +125,8 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
   const int q0 = rt * ROWS, qw0 = DEAL ? q0 : q0 + wave * 32;
   const bool wave_live = qw0 < f.L;
 
-  const float* kp = (const float*)f.k + b * f.ks[0] + hk * f.ks[1];
-  const float* vp = (const float*)f.v + b * f.vs[0] + hk * f.vs[1];
+  const E* kp = (const E*)f.k + b * f.ks[0] + hk * f.ks[1];
+  const E* vp = (const E*)f.v + b * f.vs[0] + hk * f.vs[1];
 
   // ---- this lane's query row: halves of q and dout as B operands, delta = dout . out --------------------------------------
   float qreg[D / 2], greg[D / 2];
@@ -125,14 +134,14 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
   {
     int row = qw0 + lq;
     row = row < f.L ? row : f.L - 1;
-    load_half_row<D>((const float*)f.q + b * f.qs[0] + h * f.qs[1] + row * f.qs[2], lh, qreg, have);
-    load_half_row<D>((const float*)a.dout + b * a.dos[0] + h * a.dos[1] + row * a.dos[2], lh, greg, have);
-    const float* orow = (const float*)f.out + b * f.os[0] + h * f.os[1] + row * f.os[2] + lh * (D / 2);
+    load_half_row<D>((const E*)f.q + b * f.qs[0] + h * f.qs[1] + row * f.qs[2], lh, qreg, have);
+    load_half_row<D>((const E*)a.dout + b * a.dos[0] + h * a.dos[1] + row * a.dos[2], lh, greg, have);
+    const E* orow = (const E*)f.out + b * f.os[0] + h * f.os[1] + row * f.os[2] + lh * (D / 2);
     float part = 0.f;
 #pragma unroll
     for (int i = 0; i < D / 8; i++) {
       if (PAD && lh * (D / 2) + 4 * i >= have) continue;
-      const f32x4 o = *(const f32x4*)(orow + 4 * i);
+      const f32x4 o = __builtin_convertvector(*(const Row4<E>*)(orow + 4 * i), f32x4);
 #pragma unroll
       for (int e = 0; e < 4; e++) part = fmaf(o[e], greg[4 * i + e], part);
     }
@@ -151,8 +160,8 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
     if (a.dq_splits > 1) return;  // the merge kernel writes the zeros
     const int qi = qw0 + lq;
     if (qi < f.L) {
-      float* dqp = (float*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
-      for (int d = 4 * lh; d < have; d += 8) *(f32x4*)(dqp + d) = (f32x4){0.f, 0.f, 0.f, 0.f};
+      E* dqp = (E*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
+      for (int d = 4 * lh; d < have; d += 8) *(Row4<E>*)(dqp + d) = __builtin_convertvector((f32x4){0.f, 0.f, 0.f, 0.f}, Row4<E>);
     }
     return;
   }
@@ -167,7 +176,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
   const int t0 = (int)((long long)ntiles_kv * piece / a.dq_splits), t1 = (int)((long long)ntiles_kv * (piece + 1) / a.dq_splits);
 
   // ---- global -> register -> LDS staging of one K/V tile (thread t moves 16-byte chunks t, t+256, ...) ----------------------
-  f32x4 kst[NLD], vst[NLD];
+  Row4<E> kst[NLD], vst[NLD];
   int lrow[NLD], lcol[NLD], gcol[NLD];
   bool cval[NLD];  // PAD: the chunk lies inside the tensors' rows; the others are loaded from the row's first chunk instead
                    // (the loads stay unconditional) and reach LDS as zeros
@@ -184,8 +193,8 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
     for (int i = 0; i < NLD; i++) {
       int key = kv0 + lrow[i];
       key = key < S ? key : S - 1;  // rows past the end re-read the last valid row (hidden below)
-      kst[i] = *(const f32x4*)(kp + key * f.ks[2] + 4 * gcol[i]);
-      vst[i] = *(const f32x4*)(vp + key * f.vs[2] + 4 * gcol[i]);
+      kst[i] = *(const Row4<E>*)(kp + key * f.ks[2] + 4 * gcol[i]);
+      vst[i] = *(const Row4<E>*)(vp + key * f.vs[2] + 4 * gcol[i]);
     }
   };
   auto store_tile = [&](int stage) {
@@ -195,8 +204,8 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
     for (int i = 0; i < NLD; i++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {  // rows are not 16-byte aligned
-        Ks[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? kst[i][e] : 0.f;
-        Vs[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? vst[i][e] : 0.f;
+        Ks[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? (float)kst[i][e] : 0.f;
+        Vs[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? (float)vst[i][e] : 0.f;
       }
   };
   const int s_lane = lq * PITCH + lh * (D / 2);  // score products: row l%32, this lane's half of head_dim
@@ -233,7 +242,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
         int qi = qw0 + lq;
         qi = qi < f.L ? qi : f.L - 1;
         const long long mrow = b * f.ms[0] + h * f.ms[1] + qi * f.ms[2];
-        apply_attn_mask<float>(f, s, load_attn_mask<float>(f, mrow, kv0, lh, S));
+        apply_attn_mask<E>(f, s, load_attn_mask<E>(f, mrow, kv0, lh, S));
       }
       if ((CAUSAL && kv0 + BT - 1 > qw0 + coff) || kv0 + BT > S) {
         const int qi = qw0 + lq + coff;
@@ -308,7 +317,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
         else *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_all * c + __log2f(l_all) : 1e30f, delta);
       }
       const float w = seen ? f.scale / l_all : 0.f;
-      float* dqp = (float*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
+      E* dqp = (E*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
 #pragma unroll
       for (int db = 0; db < DBLK; db++) {
         const int d = 32 * db + 8 * wave + 4 * lh;
@@ -318,7 +327,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
           const float* at = smem_bwd_f32 + (16 * db + 4 * wave + e) * 64 + lane;
           x[e] = seen ? (((at[0] + at[D * 32]) + at[2 * D * 32]) + at[3 * D * 32]) * w : 0.f;
         }
-        if (!PAD || d < have) *(f32x4*)(dqp + d) = x;
+        if (!PAD || d < have) *(Row4<E>*)(dqp + d) = __builtin_convertvector(x, Row4<E>);
       }
     }
     return;
@@ -337,7 +346,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
       else *(float2*)(a.stats + 2 * row_id) = make_float2(seen ? m_use * c + __log2f(l_tot) : 1e30f, delta);
     }
     const float w = seen ? f.scale / l_tot : 0.f;
-    float* dqp = (float*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
+    E* dqp = (E*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2];
 #pragma unroll
     for (int db = 0; db < DBLK; db++)
 #pragma unroll
@@ -346,7 +355,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
 #pragma unroll
         for (int i = 0; i < 4; i++) x[i] = seen ? dqacc[db][4 * rg + i] * w : 0.f;
         if (PAD && 32 * db + 8 * rg + 4 * lh >= have) continue;
-        *(f32x4*)(dqp + 32 * db + 8 * rg + 4 * lh) = x;
+        *(Row4<E>*)(dqp + 32 * db + 8 * rg + 4 * lh) = __builtin_convertvector(x, Row4<E>);
       }
   }
 }
@@ -354,7 +363,7 @@ __global__ __launch_bounds__(256, (D > 64 || DEAL ? 1 : 2)) void backward_dq_f32
 // ---- kernel 2: dk, dv -----------------------------------------------------------------------------------------------
 // MASKED reads one mask value per score (a key is a lane column here, the mask's rows run across registers); with its
 // addressing the head_dim-64 variant no longer fits two wavefronts per SIMD either.
-template <int D, bool CAUSAL, bool MASKED, bool PAD, bool DEAL>
+template <typename E, int D, bool CAUSAL, bool MASKED, bool PAD, bool DEAL>
 __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backward_dkv_f32_kernel(BwdArgs a) {
   typedef BwdF32Lds<D> Lds;
   constexpr int PITCH = Lds::PITCH, DBLK = D / 32;
@@ -380,19 +389,27 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
   const int k0 = kb * ROWS, kw0 = DEAL ? k0 : k0 + wave * 32;
   const int S = keys_of_batch(f, b);
   const int key = kw0 + lq;
-  float* dkp = (float*)a.dk + b * a.dks[0] + hk * a.dks[1] + key * a.dks[2];
-  float* dvp = (float*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + key * a.dvs[2];
-  if (nsplit > 1) {  // partial sums: dense [split][dk | dv][B][Hkv][S][D]
+  E* dkp = (E*)a.dk + b * a.dks[0] + hk * a.dks[1] + key * a.dks[2];
+  E* dvp = (E*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + key * a.dvs[2];
+  float *dk_part = nullptr, *dv_part = nullptr;
+  if (nsplit > 1) {  // partial sums: dense [split][dk | dv][B][Hkv][S][D], fp32
     const long long plane = (long long)f.B * f.Hkv * f.S * have;
-    dkp = a.partial + 2 * split * plane + (((long long)b * f.Hkv + hk) * f.S + key) * have;
-    dvp = dkp + plane;
+    dk_part = a.partial + 2 * split * plane + (((long long)b * f.Hkv + hk) * f.S + key) * have;
+    dv_part = dk_part + plane;
+    if constexpr (std::is_same<E, float>::value) dkp = dk_part, dvp = dv_part;
   }
+  auto put = [&](int d, f32x4 dk, f32x4 dv) __attribute__((always_inline)) {
+    if (!std::is_same<E, float>::value && nsplit > 1) {
+      *(f32x4*)(dk_part + d) = dk;
+      *(f32x4*)(dv_part + d) = dv;
+    } else {
+      *(Row4<E>*)(dkp + d) = __builtin_convertvector(dk, Row4<E>);
+      *(Row4<E>*)(dvp + d) = __builtin_convertvector(dv, Row4<E>);
+    }
+  };
   if (k0 >= S) {  // keys no query row attends to (at or beyond the batch entry's key count): zeros
     if (key < f.S)
-      for (int d = 4 * lh; d < have; d += 8) {
-        *(f32x4*)(dkp + d) = (f32x4){0.f, 0.f, 0.f, 0.f};
-        *(f32x4*)(dvp + d) = (f32x4){0.f, 0.f, 0.f, 0.f};
-      }
+      for (int d = 4 * lh; d < have; d += 8) put(d, (f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f});
     return;
   }
   const bool wave_live = kw0 < S;
@@ -402,8 +419,8 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
   float kreg[D / 2], vreg[D / 2];
   {
     const int row = key < S ? key : S - 1;
-    load_half_row<D>((const float*)f.k + b * f.ks[0] + hk * f.ks[1] + row * f.ks[2], lh, kreg, have);
-    load_half_row<D>((const float*)f.v + b * f.vs[0] + hk * f.vs[1] + row * f.vs[2], lh, vreg, have);
+    load_half_row<D>((const E*)f.k + b * f.ks[0] + hk * f.ks[1] + row * f.ks[2], lh, kreg, have);
+    load_half_row<D>((const E*)f.v + b * f.vs[0] + hk * f.vs[1] + row * f.vs[2], lh, vreg, have);
   }
   f32x16 dkacc[DBLK], dvacc[DBLK];
 #pragma unroll
@@ -422,7 +439,7 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
   const bool walk_up = dkv_walks_up(a, CAUSAL);  // every second round of an XCD's workgroups (sdpa_common.h)
   auto tile_of = [&](int idx) __attribute__((always_inline)) { return walk_up ? it0 + idx / f.G : ntq - 1 - idx / f.G; };
 
-  f32x4 qst[NLD], gst[NLD];
+  Row4<E> qst[NLD], gst[NLD];
   float2 sst = make_float2(0.f, 0.f);
   float slog = 0.f;
   int lrow[NLD], lcol[NLD], gcol[NLD];
@@ -438,14 +455,14 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
   auto load_tile = [&](int idx) {
     const int h = hk * f.G + idx % f.G;
     const int i0 = tile_of(idx) * BT;
-    const float* qp = (const float*)f.q + b * f.qs[0] + h * f.qs[1];
-    const float* gp = (const float*)a.dout + b * a.dos[0] + h * a.dos[1];
+    const E* qp = (const E*)f.q + b * f.qs[0] + h * f.qs[1];
+    const E* gp = (const E*)a.dout + b * a.dos[0] + h * a.dos[1];
 #pragma unroll
     for (int i = 0; i < NLD; i++) {
       int row = i0 + lrow[i];
       row = row < f.L ? row : f.L - 1;  // rows past the end re-read the last valid row (their weight is forced to 0)
-      qst[i] = *(const f32x4*)(qp + row * f.qs[2] + 4 * gcol[i]);
-      gst[i] = *(const f32x4*)(gp + row * a.dos[2] + 4 * gcol[i]);
+      qst[i] = *(const Row4<E>*)(qp + row * f.qs[2] + 4 * gcol[i]);
+      gst[i] = *(const Row4<E>*)(gp + row * a.dos[2] + 4 * gcol[i]);
     }
     if ((DEAL ? lane : tid) < BT) {
       const int row = i0 + (DEAL ? lane : tid);
@@ -461,8 +478,8 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
     for (int i = 0; i < NLD; i++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        Qs[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? qst[i][e] : 0.f;
-        Gs[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? gst[i][e] : 0.f;
+        Qs[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? (float)qst[i][e] : 0.f;
+        Gs[lrow[i] * PITCH + 4 * lcol[i] + e] = cval[i] ? (float)gst[i][e] : 0.f;
       }
     if ((DEAL ? lane : tid) < BT) {
       *(float2*)(Gs + Lds::TILE + 2 * (DEAL ? lane : tid)) = sst;
@@ -523,7 +540,7 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
             if (f.mask_kind == 1) {
               bias = ((const uint8_t*)f.mask)[at] == 0 ? -INFINITY : 0.f;
             } else {
-              bias = ((const float*)f.mask)[at];
+              bias = (float)((const E*)f.mask)[at];
             }
           }
           // with an attnMask: the score as the dq kernel has it; a hidden key weighs nothing, whatever its k and v hold
@@ -582,8 +599,7 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
           y[e] = ((v4[0] + v4[2 * D * 32]) + v4[4 * D * 32]) + v4[6 * D * 32];
         }
         if (PAD && d >= have) continue;
-        *(f32x4*)(dkp + d) = x;
-        *(f32x4*)(dvp + d) = y;
+        put(d, x, y);
       }
     }
     return;
@@ -598,66 +614,72 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
 #pragma unroll
         for (int i = 0; i < 4; i++) x[i] = dkacc[db][4 * rg + i] * f.scale, y[i] = dvacc[db][4 * rg + i];
         if (PAD && 32 * db + 8 * rg + 4 * lh >= have) continue;
-        *(f32x4*)(dkp + 32 * db + 8 * rg + 4 * lh) = x;
-        *(f32x4*)(dvp + 32 * db + 8 * rg + 4 * lh) = y;
+        put(32 * db + 8 * rg + 4 * lh, x, y);
       }
   }
 }
 
-template <int D, bool CAUSAL, bool MASKED, bool PAD, bool DEAL>
+template <typename E, int D, bool CAUSAL, bool MASKED, bool PAD, bool DEAL>
 int launch_dq(const BwdArgs& a, hipStream_t stream) {
   constexpr int rows = DEAL ? 32 : BM, lds = (DEAL ? 4 : 2) * BwdF32Lds<D>::STAGE * 4;
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  const hipError_t e = grant_dynamic_lds((const void*)backward_dq_f32_kernel<D, CAUSAL, MASKED, PAD, DEAL>, lds, state, done);
+  const hipError_t e = grant_dynamic_lds((const void*)backward_dq_f32_kernel<E, D, CAUSAL, MASKED, PAD, DEAL>, lds, state, done);
   if (e != hipSuccess) return (int)e;
   const long long g = (long long)a.f.B * a.f.Hq * ((a.f.L + rows - 1) / rows) * a.dq_splits;
-  hipLaunchKernelGGL((backward_dq_f32_kernel<D, CAUSAL, MASKED, PAD, DEAL>), dim3((unsigned)g), dim3(256), lds, stream, a);
+  hipLaunchKernelGGL((backward_dq_f32_kernel<E, D, CAUSAL, MASKED, PAD, DEAL>), dim3((unsigned)g), dim3(256), lds, stream, a);
   return (int)hipGetLastError();
 }
 
-template <int D, bool CAUSAL, bool MASKED, bool PAD, bool DEAL>
+template <typename E, int D, bool CAUSAL, bool MASKED, bool PAD, bool DEAL>
 int launch_dkv(const BwdArgs& a, hipStream_t stream) {
   constexpr int rows = DEAL ? 32 : BM, lds = (DEAL ? 4 : 2) * BwdF32Lds<D>::STAGE * 4;
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  const hipError_t e = grant_dynamic_lds((const void*)backward_dkv_f32_kernel<D, CAUSAL, MASKED, PAD, DEAL>, lds, state, done);
+  const hipError_t e = grant_dynamic_lds((const void*)backward_dkv_f32_kernel<E, D, CAUSAL, MASKED, PAD, DEAL>, lds, state, done);
   if (e != hipSuccess) return (int)e;
   const long long g = (long long)a.f.B * a.f.Hkv * ((a.f.S + rows - 1) / rows) * a.dkv_splits;
-  hipLaunchKernelGGL((backward_dkv_f32_kernel<D, CAUSAL, MASKED, PAD, DEAL>), dim3((unsigned)g), dim3(256), lds, stream, a);
+  hipLaunchKernelGGL((backward_dkv_f32_kernel<E, D, CAUSAL, MASKED, PAD, DEAL>), dim3((unsigned)g), dim3(256), lds, stream, a);
   return (int)hipGetLastError();
 }
 
-template <int D, bool CAUSAL, bool MASKED, bool PAD>
+template <typename E, int D, bool CAUSAL, bool MASKED, bool PAD>
 int launch_k(const BwdArgs& args, hipStream_t stream) {
   BwdArgs a = args;
   // the callers keep to this (rows are read in 16-byte chunks)
   if (PAD && (a.f.D % 4 != 0 || a.f.D >= D || a.f.D < 4)) return (int)hipErrorInvalidValue;
   static int round_cache[kMaxDevices];
-  a.dkv_round = CAUSAL && !a.dkv_dealt ? dkv_round_of((const void*)backward_dkv_f32_kernel<D, CAUSAL, MASKED, PAD, false>, 256, BwdF32Lds<D>::BYTES, round_cache) : 0;
-  int rc = a.dq_dealt ? launch_dq<D, CAUSAL, MASKED, PAD, true>(a, stream) : launch_dq<D, CAUSAL, MASKED, PAD, false>(a, stream);
+  a.dkv_round = CAUSAL && !a.dkv_dealt ? dkv_round_of((const void*)backward_dkv_f32_kernel<E, D, CAUSAL, MASKED, PAD, false>, 256, BwdF32Lds<D>::BYTES, round_cache) : 0;
+  int rc = a.dq_dealt ? launch_dq<E, D, CAUSAL, MASKED, PAD, true>(a, stream) : launch_dq<E, D, CAUSAL, MASKED, PAD, false>(a, stream);
   if (rc != 0) return rc;
   if (a.dq_splits > 1) {
-    rc = launch_backward_dq_merge<float>(a, stream);
+    rc = launch_backward_dq_merge<E>(a, stream);
     if (rc != 0) return rc;
   }
-  rc = a.dkv_dealt ? launch_dkv<D, CAUSAL, MASKED, PAD, true>(a, stream) : launch_dkv<D, CAUSAL, MASKED, PAD, false>(a, stream);
-  return rc != 0 || a.dkv_splits == 1 ? rc : launch_backward_dkv_sum<float>(a, stream);
+  rc = a.dkv_dealt ? launch_dkv<E, D, CAUSAL, MASKED, PAD, true>(a, stream) : launch_dkv<E, D, CAUSAL, MASKED, PAD, false>(a, stream);
+  return rc != 0 || a.dkv_splits == 1 ? rc : launch_backward_dkv_sum<E>(a, stream);
 }
 
-template <int D, bool PAD>
+template <typename E, int D, bool PAD>
 int launch_d(const BwdArgs& a, hipStream_t stream) {
-  if (a.f.mask_kind != 0) return launch_k<D, false, true, PAD>(a, stream);  // exclusive with causal (validated by the caller, as the reference asserts)
-  return a.f.causal ? launch_k<D, true, false, PAD>(a, stream) : launch_k<D, false, false, PAD>(a, stream);
+  if (a.f.mask_kind != 0) return launch_k<E, D, false, true, PAD>(a, stream);  // exclusive with causal (validated by the caller, as the reference asserts)
+  if constexpr (std::is_same<E, float>::value)
+    return a.f.causal ? launch_k<E, D, true, false, PAD>(a, stream) : launch_k<E, D, false, false, PAD>(a, stream);
+  return (int)hipErrorInvalidValue;  // (16-bit tensors come here for their masks only)
+}
+
+template <typename E>
+int launch_e(const BwdArgs& a, hipStream_t stream) {
+  if (a.f.D == 128) return launch_d<E, 128, false>(a, stream);
+  if (a.f.D == 64) return launch_d<E, 64, false>(a, stream);
+  // any other multiple of 4 up to 128: the kernels of the next size up, the missing columns as zeros
+  return a.f.D < 64 ? launch_d<E, 64, true>(a, stream) : launch_d<E, 128, true>(a, stream);
 }
 
 }  // namespace
 
-int launch_backward_f32(const BwdArgs& a, hipStream_t stream) {
-  if (a.f.D == 128) return launch_d<128, false>(a, stream);
-  if (a.f.D == 64) return launch_d<64, false>(a, stream);
-  // any other multiple of 4 up to 128: the kernels of the next size up, the missing columns as zeros
-  return a.f.D < 64 ? launch_d<64, true>(a, stream) : launch_d<128, true>(a, stream);
+int launch_backward_f32(const BwdArgs& a, int dtype, hipStream_t stream) {
+  return dtype == 0 ? launch_e<float>(a, stream) : dtype == 1 ? launch_e<_Float16>(a, stream) : launch_e<__bf16>(a, stream);
 }
 
 }  // namespace ttsdpa

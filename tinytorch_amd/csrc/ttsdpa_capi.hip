@@ -106,7 +106,7 @@ bool fast_layout_ok(const ttsdpa_params* p, bool masks_ok = false, bool pages_ok
 // What the MFMA routes take: attnMasks readable four keys at a time (aligned groups, whole groups only).  The kernels
 // themselves apply any attnMask: any_mask = true in the tests below admits the others, which the general route hands
 // to them (a general-route call of 16 x 12 heads x 197 rows, head_dim 64, fp16, with a key-padding mask: 124 us on the
-// vector ALUs, 16 us there).
+// vector ALUs, 18 us there).
 bool simple_mask_ok(const ttsdpa_params* p, bool any_mask = false) {
   return any_mask || p->mask_kind == TTSDPA_MASK_NONE || (mask_vec4_ok(p) && p->S % 4 == 0 && !p->kv_len);
 }
@@ -376,9 +376,14 @@ int pick_backward_route(const ttsdpa_backward_params* p) {
   return backward_mfma_ok(p) || backward_f32_ok(p) ? TTSDPA_ROUTE_PREFILL : TTSDPA_ROUTE_GENERAL;
 }
 
-// The matrix-core pairs run the call: the MFMA route, and of the general route what only its attnMask keeps off it.
+// The matrix-core pairs run the call: the MFMA route, and of the general route what only its attnMask keeps off it (16-bit tensors
+// then on the fp32 pair: that route's arithmetic is fp32).
 bool backward_on_mfma(const ttsdpa_backward_params* p) {
   return pick_backward_route(p) != TTSDPA_ROUTE_NONE && (backward_mfma_ok(p, true) || backward_f32_ok(p, true));
+}
+
+bool backward_on_f32_pair(const ttsdpa_backward_params* p) {
+  return backward_on_mfma(p) && (p->fwd.dtype == TTSDPA_F32 || !simple_mask_ok(&p->fwd));
 }
 
 // The rows' statistics: (statistic, delta) pairs, then log_sums where the kernels keep one (BwdArgs).
@@ -395,7 +400,7 @@ int dkv_splits_of(const ttsdpa_backward_params* p, bool* dealt = nullptr) {
   if (!backward_on_mfma(p)) return 1;
   const int groups = f->dtype != TTSDPA_F32 && f->D == 128 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
   const int per_cu = f->D <= 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
-  return backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, groups, per_cu, f->dtype == TTSDPA_F32, dealt);
+  return backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, groups, per_cu, backward_on_f32_pair(p), dealt);
 }
 // ... then (matrix-core pairs whose dq kernel splits its key ranges) the partial dq records, 256-byte aligned.
 int dq_splits_of(const ttsdpa_backward_params* p, bool* dealt = nullptr) {
@@ -404,8 +409,9 @@ int dq_splits_of(const ttsdpa_backward_params* p, bool* dealt = nullptr) {
   if (!dealt) dealt = &unused;
   *dealt = false;
   if (!backward_on_mfma(p)) return 1;
-  const int slots = f->dtype == TTSDPA_F32 && f->D > 64 ? 256 : 512;
-  return backward_dq_splits(f->B, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, slots, f->dtype == TTSDPA_F32, dealt);
+  const bool f32 = backward_on_f32_pair(p);
+  const int slots = f32 && f->D > 64 ? 256 : 512;
+  return backward_dq_splits(f->B, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, slots, f32, dealt);
 }
 size_t backward_partial_offset(const ttsdpa_backward_params* p) { return (backward_stats_bytes(p) + 255) & ~(size_t)255; }
 size_t backward_dq_partial_offset(const ttsdpa_backward_params* p) {
@@ -669,7 +675,7 @@ int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t wor
   if (backward_on_mfma(p)) {
     const long long g1 = (long long)a.f.B * a.f.Hq * ((a.f.L + 127) / 128) * a.dq_splits, g2 = (long long)a.f.B * a.f.Hkv * ((a.f.S + 127) / 128);
     if (check_grid(g1) != TTSDPA_OK || check_grid(g2) != TTSDPA_OK) return TTSDPA_ERR_SHAPE;
-    if (p->fwd.dtype == TTSDPA_F32) return launch_backward_f32(a, (hipStream_t)stream);
+    if (backward_on_f32_pair(p)) return launch_backward_f32(a, p->fwd.dtype, (hipStream_t)stream);
     return launch_backward_mfma(a, p->fwd.dtype, (hipStream_t)stream);
   }
   {  // the vector-ALU pair: 64 rows per workgroup up to head_dim 128, 32 beyond
