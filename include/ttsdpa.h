@@ -88,6 +88,8 @@ enum ttsdpa_route {
  * {batch, head, query row, key}; an axis the mask does not have, or has with size 1, gets stride 0.  A dense
  * [L,S] mask is {0, 0, S, 1} (what ttsdpa_params_init fills), a per-batch key-padding mask [B,1,1,S] is {S, 0, 0, 1}.
  * scale multiplies q.k^T before the bias; the reference default is 1/sqrt(D).
+ * Rows that no key gives any weight, in every kernel: a batch entry without keys (S or kv_len of 0) gives zeros, the reference's
+ * empty contraction; a row that has keys, but all of them hidden by its attnMask or with scores of -inf, gives NaN, its softmax's 0 / 0.
  */
 typedef struct ttsdpa_params {
   uint32_t struct_size; /* sizeof(ttsdpa_params) */

@@ -596,7 +596,7 @@ int launch_decode(const KArgs& a, int dtype, void* workspace, hipStream_t stream
 
 // The records of a split launch of a pipelined prefill kernel -> out.  One thread per four elements of a row (eight rows per workgroup): the row's
 // splits up to its last visible key (a split wholly beyond the keys of a row tile wrote nothing), brought to their
-// common maximum, added in split order, normalised.  Rows of a batch entry without keys: zeros.
+// common maximum, added in split order, normalised.  Rows of a batch entry without keys: zeros (weightless rows: ttsdpa.h).
 template <typename T, int D>
 __global__ __launch_bounds__(256) void prefill_split_merge_kernel(KArgs a, long long nvec) {
   typedef T vec4t __attribute__((ext_vector_type(4)));
@@ -632,7 +632,7 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(KArgs a, long 
     const float2 lo = *(const float2*)(rec + s * step + d), hi = *(const float2*)(rec + s * step + d + 2);
     x[0] = fmaf(w, lo.x, x[0]), x[1] = fmaf(w, lo.y, x[1]), x[2] = fmaf(w, hi.x, x[2]), x[3] = fmaf(w, hi.y, x[3]);
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = n > 0 ? 1.f / l : 0.f;
 #pragma unroll
   for (int e = 0; e < 4; e++) x[e] *= inv;
   *(vec4t*)((T*)a.out + b * a.os[0] + h * a.os[1] + qi * a.os[2] + d) = __builtin_convertvector(x, vec4t);
@@ -648,10 +648,9 @@ int launch_prefill_split_merge(const KArgs& a, int dtype, hipStream_t stream) {
 }
 
 // The same for a split launch of the 4-wavefront kernels (16-bit and fp32), whose splits all write their records, of the kernel's
-// head_dim W >= a.D.  A row that sees no key although there are some: NaN, the unsplit kernels' and the reference's 0 / 0, or
-// with hidden_zero zeros.
+// head_dim W >= a.D.
 template <typename T>
-__global__ __launch_bounds__(256) void tile_split_merge_kernel(KArgs a, int W, int hidden_zero, long long nvec) {
+__global__ __launch_bounds__(256) void tile_split_merge_kernel(KArgs a, int W, long long nvec) {
   typedef T vec4t __attribute__((ext_vector_type(4)));
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= nvec) return;
@@ -677,14 +676,14 @@ __global__ __launch_bounds__(256) void tile_split_merge_kernel(KArgs a, int W, i
     x[0] = fmaf(w, lo.x, x[0]), x[1] = fmaf(w, lo.y, x[1]), x[2] = fmaf(w, hi.x, x[2]), x[3] = fmaf(w, hi.y, x[3]);
   }
   const bool empty = a.S == 0 || (a.kv_len && a.kv_len[b] <= 0);
-  const float inv = l > 0.f || !(empty || hidden_zero) ? 1.f / l : 0.f;
+  const float inv = empty ? 0.f : 1.f / l;
 #pragma unroll
   for (int e = 0; e < 4; e++) x[e] *= inv;
   *(vec4t*)((T*)a.out + b * a.os[0] + h * a.os[1] + qi * a.os[2] + d) = __builtin_convertvector(x, vec4t);
 }
 
 
-int launch_tile_merge(const KArgs& a, int dtype, int W, bool hidden_zero, hipStream_t stream);  // tile_split_merge_kernel (sdpa_prefill.hip)
+int launch_tile_merge(const KArgs& a, int dtype, int W, hipStream_t stream);  // tile_split_merge_kernel (sdpa_prefill.hip)
 int launch_zero(const KArgs& a, int dtype, hipStream_t stream);
 struct KvAppendArgs {
   void* kc;

@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
     if (splits == 1) {
       int xl = x / a.G, xg = x % a.G;
       T* op = (T*)a.out + b * a.os[0] + (hk * a.G + xg) * a.os[1] + xl * a.os[2];
-      if (!PAD || d < a.D) store_from_float(op + d, lsum > 0.f ? o / lsum : 0.f);  // no keys at all: zeros, as the reference's empty contraction
+      if (!PAD || d < a.D) store_from_float(op + d, S > 0 ? o / lsum : 0.f);  // no keys at all: zeros, as the reference's empty contraction
     } else {
       float* rec = ws + ((long long)blockIdx.x * rows + x) * (DD + 2);
       rec[d] = o;
@@ -362,7 +362,8 @@ __global__ __launch_bounds__(DD) void merge_kernel(KArgs a, int splits, const fl
   for (int s = 0; s < splits; s++) o = fmaf(weight[s], rec0[s * step + t], o);
   const int xl = x / a.G, xg = x % a.G;
   T* op = (T*)a.out + b * a.os[0] + (hk * a.G + xg) * a.os[1] + xl * a.os[2];
-  if (t < a.D) store_from_float(op + t, total > 0.f ? o / total : 0.f);  // (a.D < DD: the decode kernel's zero-column variant)
+  const bool empty = a.kv_len && a.kv_len[b] <= 0;  // (as the decode kernel has it)
+  if (t < a.D) store_from_float(op + t, empty ? 0.f : o / total);  // (a.D < DD: the decode kernel's zero-column variant)
 }
 
 template <typename TR, int DD, bool PAD>

@@ -500,12 +500,12 @@ int launch_prefill_d(const KArgs& a, hipStream_t stream) {
   return launch_prefill_t<TR, 256, true>(a, stream);
 }
 
-int launch_tile_merge(const KArgs& a, int dtype, int W, bool hidden_zero, hipStream_t stream) {
+int launch_tile_merge(const KArgs& a, int dtype, int W, hipStream_t stream) {
   const long long nvec = (long long)a.B * a.Hq * a.L * (a.D / 4);
   const dim3 grid((unsigned)((nvec + 255) / 256));
-  if (dtype == 0) hipLaunchKernelGGL((tile_split_merge_kernel<float>), grid, dim3(256), 0, stream, a, W, (int)hidden_zero, nvec);
-  else if (dtype == 1) hipLaunchKernelGGL((tile_split_merge_kernel<_Float16>), grid, dim3(256), 0, stream, a, W, (int)hidden_zero, nvec);
-  else hipLaunchKernelGGL((tile_split_merge_kernel<__bf16>), grid, dim3(256), 0, stream, a, W, (int)hidden_zero, nvec);
+  if (dtype == 0) hipLaunchKernelGGL((tile_split_merge_kernel<float>), grid, dim3(256), 0, stream, a, W, nvec);
+  else if (dtype == 1) hipLaunchKernelGGL((tile_split_merge_kernel<_Float16>), grid, dim3(256), 0, stream, a, W, nvec);
+  else hipLaunchKernelGGL((tile_split_merge_kernel<__bf16>), grid, dim3(256), 0, stream, a, W, nvec);
   return (int)hipGetLastError();
 }
 

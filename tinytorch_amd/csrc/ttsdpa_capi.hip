@@ -231,13 +231,6 @@ SplitPlan plan_prefill_splits(const ttsdpa_params* p, const KArgs& a /* after pa
                         f32 ? us * prefill_f32_tiles(whole) : 0);
 }
 
-// Calls of these sizes, one query head per KV head, without an attnMask, have always had zeros where a causal mask leaves a row
-// no key (their splits were merged by the decode path's kernel); others have NaN there.
-bool hidden_rows_zero(const ttsdpa_params* p, const KArgs& a) {
-  const long long wgs = (long long)a.B * a.Hq * ((a.L + 127) / 128);
-  return a.G == 1 && (a.D == 64 || a.D == 128) && p->mask_kind == TTSDPA_MASK_NONE && !pipelined_ok(p) && a.S >= 1024 && wgs < 512;
-}
-
 // Key splits for the pipelined kernels (head_dim 128 and 64): a call with a quarter as many 256-row tiles as the chip has CUs, or
 // fewer (a chunk of one sequence's rows against a long cache, a few heads of a tensor-parallel share), leaves most CUs
 // without work.  Its row tiles then share their keys among workgroups of `chunk` keys (a multiple of 256: four key
@@ -582,7 +575,7 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
     if ((rc = check_grid((long long)a.B * a.Hq * ((a.L + 127) / 128) * sp.splits)) != TTSDPA_OK) return rc;
     rc = launch(a);
     if (rc != 0) return rc;
-    return launch_tile_merge(a, p->dtype, tile_width(p->dtype, a.D), hidden_rows_zero(p, a), (hipStream_t)stream);
+    return launch_tile_merge(a, p->dtype, tile_width(p->dtype, a.D), (hipStream_t)stream);
   }
   return launch(a);
 }
