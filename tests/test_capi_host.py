@@ -1,6 +1,7 @@
 """Host-only checks of the C ABI (no GPU, no kernel launch): the library loads, exports every symbol that
 include/ttsdpa.h declares, lays out ttsdpa_params as the header says, validates arguments and picks routes."""
 import ctypes
+import time
 import os
 import re
 
@@ -391,3 +392,22 @@ def test_static_scratch_decode_refuses_what_does_not_fit():
     fp32.q = fp32.k = fp32.v = fp32.out = 0x1000
     assert lib.ttsdpa_decode_static(ctypes.byref(fp32), None) == _capi.ERR_UNSUPPORTED
     assert lib.ttsdpa_decode_static(None, None) == _capi.ERR_NULL
+
+
+def test_decode_plan_costs_the_same_at_any_size():
+    """Host time of a decode plan does not grow where few (batch, KV head) pairs would allow many splits of the keys."""
+    L = _capi.lib()
+
+    def cost(B, Hkv, S):
+        p = ctypes.byref(params(_capi.BF16, B, 4 * Hkv, Hkv, 1, S, 128))
+        best = 1e9
+        for _ in range(30):
+            t = time.perf_counter()
+            for _ in range(200):
+                L.ttsdpa_workspace_bytes(p)
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    # 300 pairs: at most two counts to look at; the others had up to 524 of them (2.0 against 0.45 us with the call's own cost in C)
+    most = max(cost(1, 1, 4096), cost(1, 1, 131072), cost(2, 1, 65536))
+    assert most <= 1.6 * cost(75, 4, 4096)

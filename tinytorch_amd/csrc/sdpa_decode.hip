@@ -401,19 +401,20 @@ DecodePlan plan_decode(const KArgs& a) {
   int max_splits = (a.S + 2 * round - 1) / (2 * round);
   if (pairs * max_splits < 128 && a.S > 2 * round) max_splits = (a.S + round - 1) / round;
   if (max_splits < 1) max_splits = 1;
+  if (max_splits > kMaxSplits) max_splits = kMaxSplits;
   // Two workgroups per CU or a few more: the count, up to four per CU, that fills its last round best (a CU takes in its
   // workgroups' keys at a rate of its own, so 2.25 per CU cost as much as 3: 24 sequences of 3000 keys on 4 KV heads, 96
-  // pairs, 37.7 us in 6 splits of the keys and 31 in 8), the smaller of two that are equally good.
-  int splits = 1;
+  // pairs, 37.7 us in 6 splits of the keys and 31 in 8), the smaller of two that are equally good.  Few pairs: as many as may be,
+  // without a look at counts beyond that (one pair: 524 of them, 1.5 us of host time in each of a call's three plans).
+  const long long first = (500 + pairs - 1) / pairs;
+  int splits = first < max_splits ? 1 : max_splits;
   double best = 0;
-  for (long long s = (500 + pairs - 1) / pairs; s == 1 || s * pairs <= 4 * 256; s++) {
+  for (long long s = first; first < max_splits && s <= max_splits && (s == 1 || s * pairs <= 4 * 256); s++) {
     const long long wgs = s * pairs, rounds = (wgs + 255) / 256;
     const double fill = (double)wgs / (double)(rounds * 256) - 0.01 * rounds;
     if (s > 1 && fill <= best) continue;
     best = fill, splits = (int)s;
   }
-  if (splits > max_splits) splits = max_splits;
-  if (splits > kMaxSplits) splits = kMaxSplits;
   int chunk = (a.S + splits - 1) / splits;
   chunk = (chunk + round - 1) / round * round;
   if (chunk < round) chunk = round;
