@@ -74,6 +74,18 @@ struct Scratch {
 };
 
 PyObject* none() { Py_RETURN_NONE; }
+PyObject* yes() { Py_RETURN_TRUE; }
+
+// While a call allocates and launches, other Python threads run: an allocation may wait for the device, a launch for room in
+// a full queue.
+class Unlocked {
+  PyThreadState* state_ = PyEval_SaveThread();
+
+ public:
+  Unlocked() = default;
+  Unlocked(const Unlocked&) = delete;
+  ~Unlocked() { PyEval_RestoreThread(state_); }
+};
 
 // C++ exceptions of torch (an allocation that fails) become its Python ones.
 template <typename F>
@@ -203,12 +215,17 @@ PyObject* sdp_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     ttsdpa_params p;
     if (!fill_params(&p, *q, *k, *v, causal_of(a[3], a[8]), a[4], a[6], a[7], a[9])) return none();
-    const Tensor out = empty_like_shape(q->sizes(), *q);
-    p.out = out.data_ptr();
-    const size_t bytes = ttsdpa_workspace_bytes(&p);
-    const Scratch ws(bytes, *q);
-    if (ttsdpa_forward(&p, ws.ptr, bytes, stream_of(*q)) != TTSDPA_OK) return none();
-    return THPVariable_Wrap(out);
+    Tensor out;
+    int rc;
+    {
+      const Unlocked others;
+      out = empty_like_shape(q->sizes(), *q);
+      p.out = out.data_ptr();
+      const size_t bytes = ttsdpa_workspace_bytes(&p);
+      const Scratch ws(bytes, *q);
+      rc = ttsdpa_forward(&p, ws.ptr, bytes, stream_of(*q));
+    }
+    return rc == TTSDPA_OK ? THPVariable_Wrap(out) : none();
   });
 }
 
@@ -228,16 +245,21 @@ PyObject* sdp_attention_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     bp.fwd = p;
     bp.fwd.out = o->data_ptr();
     strides3(bp.fwd.o_stride, *o);
-    // the gradients take their operand's layout (torch.empty_like) unless that leaves head_dim strided
-    Tensor gq = at::empty_like(*q), gk = at::empty_like(*k), gv = at::empty_like(*v);
-    if (gq.stride(-1) != 1 || gk.stride(-1) != 1 || gv.stride(-1) != 1)
-      gq = empty_like_shape(q->sizes(), *q), gk = empty_like_shape(k->sizes(), *k), gv = empty_like_shape(v->sizes(), *v);
-    bp.dout = g->data_ptr(), bp.dq = gq.data_ptr(), bp.dk = gk.data_ptr(), bp.dv = gv.data_ptr();
-    strides3(bp.dout_stride, *g), strides3(bp.dq_stride, gq), strides3(bp.dk_stride, gk), strides3(bp.dv_stride, gv);
-    const size_t bytes = ttsdpa_backward_workspace_bytes(&bp);
-    const Scratch ws(bytes, *q);
-    if (ttsdpa_backward(&bp, ws.ptr, bytes, stream_of(*q)) != TTSDPA_OK) return none();
-    return tuple_of({&gq, &gk, &gv});
+    Tensor gq, gk, gv;
+    int rc;
+    {
+      const Unlocked others;
+      // the gradients take their operand's layout (torch.empty_like) unless that leaves head_dim strided
+      gq = at::empty_like(*q), gk = at::empty_like(*k), gv = at::empty_like(*v);
+      if (gq.stride(-1) != 1 || gk.stride(-1) != 1 || gv.stride(-1) != 1)
+        gq = empty_like_shape(q->sizes(), *q), gk = empty_like_shape(k->sizes(), *k), gv = empty_like_shape(v->sizes(), *v);
+      bp.dout = g->data_ptr(), bp.dq = gq.data_ptr(), bp.dk = gk.data_ptr(), bp.dv = gv.data_ptr();
+      strides3(bp.dout_stride, *g), strides3(bp.dq_stride, gq), strides3(bp.dk_stride, gk), strides3(bp.dv_stride, gv);
+      const size_t bytes = ttsdpa_backward_workspace_bytes(&bp);
+      const Scratch ws(bytes, *q);
+      rc = ttsdpa_backward(&bp, ws.ptr, bytes, stream_of(*q));
+    }
+    return rc == TTSDPA_OK ? tuple_of({&gq, &gk, &gv}) : none();
   });
 }
 
@@ -283,12 +305,29 @@ PyObject* kv_cache_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
       p.page_size = (int32_t)kc->size(2);
       p.block_table_stride = (int32_t)table->stride(0);
     }
-    if (ttsdpa_kv_append(&p, stream_of(*kc)) != TTSDPA_OK) return none();
-    Py_RETURN_TRUE;
+    int rc;
+    {
+      const Unlocked others;
+      rc = ttsdpa_kv_append(&p, stream_of(*kc));
+    }
+    return rc == TTSDPA_OK ? yes() : none();
   });
 }
 
 // ---- row-wise ops ------------------------------------------------------------------------------------------------------
+
+// A new tensor of `like`'s type that `enqueue` (a status code, from its address) fills.
+template <typename F>
+PyObject* result_of(const Tensor& like, at::IntArrayRef shape, F&& enqueue) {
+  Tensor out;
+  int rc;
+  {
+    const Unlocked others;
+    out = empty_like_shape(shape, like);
+    rc = enqueue(out.data_ptr());
+  }
+  return rc == TTSDPA_OK ? THPVariable_Wrap(out) : none();
+}
 
 bool rowwise(const Tensor& t) { return dtype_of(t) >= 0 && t.dim() > 0 && on_current_gpu(t) && t.is_contiguous(); }
 
@@ -312,11 +351,10 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!rowwise(*x)) return none();
     const int64_t dim = x->size(-1);
     if (!is_shape_of(a[1], dim) || (w && (!same_kind(*w, *x) || w->dim() != 1 || w->size(0) != dim || !w->is_contiguous()))) return none();
-    const Tensor out = empty_like_shape(x->sizes(), *x);
-    if (ttfused_rms_norm(dtype_of(*x), x->data_ptr(), w ? w->data_ptr() : nullptr, out.data_ptr(), dim ? x->numel() / dim : 0, dim,
-                         (float)eps, stream_of(*x)) != TTSDPA_OK)
-      return none();
-    return THPVariable_Wrap(out);
+    return result_of(*x, x->sizes(), [&](void* out) {
+      return ttfused_rms_norm(dtype_of(*x), x->data_ptr(), w ? w->data_ptr() : nullptr, out, dim ? x->numel() / dim : 0, dim, (float)eps,
+                              stream_of(*x));
+    });
   });
 }
 
@@ -329,10 +367,13 @@ PyObject* fused_add_rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!rowwise(*x) || !same_kind(*r, *x) || r->sizes() != x->sizes() || !r->is_contiguous()) return none();
     const int64_t dim = x->size(-1);
     if (!same_kind(*w, *x) || w->dim() != 1 || w->size(0) != dim || !w->is_contiguous()) return none();
-    if (ttfused_add_rms_norm(dtype_of(*x), x->data_ptr(), r->data_ptr(), w->data_ptr(), dim ? x->numel() / dim : 0, dim, (float)eps,
-                             stream_of(*x)) != TTSDPA_OK)
-      return none();
-    Py_RETURN_TRUE;
+    int rc;
+    {
+      const Unlocked others;
+      rc = ttfused_add_rms_norm(dtype_of(*x), x->data_ptr(), r->data_ptr(), w->data_ptr(), dim ? x->numel() / dim : 0, dim, (float)eps,
+                                stream_of(*x));
+    }
+    return rc == TTSDPA_OK ? yes() : none();
   });
 }
 
@@ -345,9 +386,9 @@ PyObject* silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t d = x->size(-1) / 2;
     at::DimVector shape(x->sizes());
     shape.back() = d;
-    const Tensor out = empty_like_shape(shape, *x);
-    if (ttfused_silu_mul(dtype_of(*x), x->data_ptr(), out.data_ptr(), d ? x->numel() / (2 * d) : 0, d, stream_of(*x)) != TTSDPA_OK) return none();
-    return THPVariable_Wrap(out);
+    return result_of(*x, shape, [&](void* out) {
+      return ttfused_silu_mul(dtype_of(*x), x->data_ptr(), out, d ? x->numel() / (2 * d) : 0, d, stream_of(*x));
+    });
   });
 }
 
@@ -373,10 +414,9 @@ PyObject* softmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 3 || !(x = tensor(a[0]))) return none();
   return guarded([&]() -> PyObject* {
     if (!rowwise(*x) || !around_axis(*x, a[1], &outer, &dim, &inner)) return none();
-    const Tensor out = empty_like_shape(x->sizes(), *x);
-    if (ttfused_softmax(dtype_of(*x), x->data_ptr(), out.data_ptr(), outer, dim, inner, a[2] == Py_True, stream_of(*x)) != TTSDPA_OK)
-      return none();
-    return THPVariable_Wrap(out);
+    return result_of(*x, x->sizes(), [&](void* out) {
+      return ttfused_softmax(dtype_of(*x), x->data_ptr(), out, outer, dim, inner, a[2] == Py_True, stream_of(*x));
+    });
   });
 }
 
@@ -388,11 +428,9 @@ PyObject* softmax_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     if (!rowwise(*g) || !same_kind(*y, *g) || y->sizes() != g->sizes() || !y->is_contiguous() || !around_axis(*g, a[2], &outer, &dim, &inner))
       return none();
-    const Tensor out = empty_like_shape(g->sizes(), *g);
-    if (ttfused_softmax_backward(dtype_of(*g), g->data_ptr(), y->data_ptr(), out.data_ptr(), outer, dim, inner, a[3] == Py_True,
-                                 stream_of(*g)) != TTSDPA_OK)
-      return none();
-    return THPVariable_Wrap(out);
+    return result_of(*g, g->sizes(), [&](void* out) {
+      return ttfused_softmax_backward(dtype_of(*g), g->data_ptr(), y->data_ptr(), out, outer, dim, inner, a[3] == Py_True, stream_of(*g));
+    });
   });
 }
 
@@ -425,23 +463,13 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     at::DimVector shape(x->sizes());
     shape.back() = N;
-    const Tensor out = empty_like_shape(shape, *x);
-    const size_t bytes = ttlinear_matmul_workspace_bytes(dt, M, N, K, 0, 1);
-    const Scratch ws(bytes, *x);
-    if (ttlinear_matmul(dt, x->data_ptr(), w->data_ptr(), b ? b->data_ptr() : nullptr, out.data_ptr(), M, N, K, 0, 1, ldx, ld_of(*w), N,
-                        ws.ptr, bytes, stream_of(*x)) != TTSDPA_OK)
-      return none();
-    return THPVariable_Wrap(out);
+    return result_of(*x, shape, [&](void* out) {
+      const size_t bytes = ttlinear_matmul_workspace_bytes(dt, M, N, K, 0, 1);
+      const Scratch ws(bytes, *x);
+      return ttlinear_matmul(dt, x->data_ptr(), w->data_ptr(), b ? b->data_ptr() : nullptr, out, M, N, K, 0, 1, ldx, ld_of(*w), N, ws.ptr,
+                             bytes, stream_of(*x));
+    });
   });
-}
-
-// out = op(a) . op(b) + bias for matrices; a status code
-int product(const Tensor& x, const Tensor& y, bool ta, bool tb, const Tensor* bias, const Tensor& out, int64_t M, int64_t N, int64_t K) {
-  const int dt = dtype_of(x);
-  const size_t bytes = ttlinear_matmul_workspace_bytes(dt, M, N, K, ta, tb);
-  const Scratch ws(bytes, x);
-  return ttlinear_matmul(dt, x.data_ptr(), y.data_ptr(), bias ? bias->data_ptr() : nullptr, out.data_ptr(), M, N, K, ta, tb, ld_of(x), ld_of(y),
-                         N, ws.ptr, bytes, stream_of(x));
 }
 
 // (a, b, transA, transB, bias): matrices only, batches go through Python
@@ -455,9 +483,13 @@ PyObject* matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t M = x->size(ta ? 1 : 0), K = x->size(ta ? 0 : 1), N = y->size(tb ? 0 : 1);
     if (y->size(tb ? 1 : 0) != K || !bias_ok(bias, N, *x)) return none();
     const int64_t shape[2] = {M, N};
-    const Tensor out = empty_like_shape(shape, *x);
-    if (product(*x, *y, ta, tb, bias, out, M, N, K) != TTSDPA_OK) return none();
-    return THPVariable_Wrap(out);
+    return result_of(*x, shape, [&](void* out) {
+      const int dt = dtype_of(*x);
+      const size_t bytes = ttlinear_matmul_workspace_bytes(dt, M, N, K, ta, tb);
+      const Scratch ws(bytes, *x);
+      return ttlinear_matmul(dt, x->data_ptr(), y->data_ptr(), bias ? bias->data_ptr() : nullptr, out, M, N, K, ta, tb, ld_of(*x), ld_of(*y), N,
+                             ws.ptr, bytes, stream_of(*x));
+    });
   });
 }
 
@@ -480,18 +512,21 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     };
     int64_t M, Mx, ldg, ldx;
     if (!rows(*g, N, &M, &ldg) || !rows(*x, K, &Mx, &ldx) || M != Mx || M < 1) return none();
-    const Tensor gi = empty_like_shape(x->sizes(), *x), gw = empty_like_shape(w->sizes(), *w);
-    Tensor gb;
-    if (need_bias) {
-      const int64_t shape[1] = {N};
-      gb = empty_like_shape(shape, *x);
+    Tensor gi, gw, gb;
+    int rc;
+    {
+      const Unlocked others;
+      gi = empty_like_shape(x->sizes(), *x), gw = empty_like_shape(w->sizes(), *w);
+      if (need_bias) {
+        const int64_t shape[1] = {N};
+        gb = empty_like_shape(shape, *x);
+      }
+      const size_t bytes = ttlinear_backward_workspace_bytes(dt, M, N, K);
+      const Scratch ws(bytes, *x);
+      rc = ttlinear_backward(dt, g->data_ptr(), x->data_ptr(), w->data_ptr(), gi.data_ptr(), gw.data_ptr(), need_bias ? gb.data_ptr() : nullptr,
+                             M, N, K, ldg, ldx, ld_of(*w), ws.ptr, bytes, stream_of(*x));
     }
-    const size_t bytes = ttlinear_backward_workspace_bytes(dt, M, N, K);
-    const Scratch ws(bytes, *x);
-    if (ttlinear_backward(dt, g->data_ptr(), x->data_ptr(), w->data_ptr(), gi.data_ptr(), gw.data_ptr(), need_bias ? gb.data_ptr() : nullptr,
-                          M, N, K, ldg, ldx, ld_of(*w), ws.ptr, bytes, stream_of(*x)) != TTSDPA_OK)
-      return none();
-    return tuple_of({&gi, &gw, need_bias ? &gb : nullptr});
+    return rc == TTSDPA_OK ? tuple_of({&gi, &gw, need_bias ? &gb : nullptr}) : none();
   });
 }
 
