@@ -1178,6 +1178,8 @@ static LinArgs flags_args(int64_t M, int64_t N, int64_t K, int trans_a, int tran
 }
 
 // Room for the copies (where the product would be made on copies, or operands lie contraction-major) or the parts of a divided contraction.
+// The latter also where aligned operands would go another way: sizes do not say how rows are aligned, and unaligned ones go to the
+// streaming kernel.  (Some MB at most: only products of few tiles are divided.)
 size_t ttlinear_matmul_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const LinArgs g = flags_args(M, N, K, trans_a, trans_b);

@@ -62,14 +62,20 @@ Tensor empty_like_shape(at::IntArrayRef shape, const Tensor& like) {
 }
 
 // Device scratch of one call from torch's caching allocator: a buffer per call, so that the allocator orders reuse by
-// stream and a captured call keeps its scratch in the graph's pool.
+// stream and a captured call keeps its scratch in the graph's pool.  Where the device has no room for it the call goes on with
+// none: the C ABI runs it without (operands read in place, keys not divided) or says that it cannot.
 struct Scratch {
   Tensor t;
   void* ptr = nullptr;
-  Scratch(size_t bytes, const Tensor& like) {
-    if (bytes == 0) return;
-    t = at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(like.device()));
-    ptr = t.data_ptr();
+  size_t bytes = 0;
+  Scratch(size_t want, const Tensor& like) {
+    if (want == 0) return;
+    try {
+      t = at::empty({(int64_t)want}, at::TensorOptions().dtype(at::kByte).device(like.device()));
+    } catch (const c10::OutOfMemoryError&) {
+      return;
+    }
+    ptr = t.data_ptr(), bytes = want;
   }
 };
 
@@ -221,9 +227,8 @@ PyObject* sdp_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const Unlocked others;
       out = empty_like_shape(q->sizes(), *q);
       p.out = out.data_ptr();
-      const size_t bytes = ttsdpa_workspace_bytes(&p);
-      const Scratch ws(bytes, *q);
-      rc = ttsdpa_forward(&p, ws.ptr, bytes, stream_of(*q));
+      const Scratch ws(ttsdpa_workspace_bytes(&p), *q);
+      rc = ttsdpa_forward(&p, ws.ptr, ws.bytes, stream_of(*q));
     }
     return rc == TTSDPA_OK ? THPVariable_Wrap(out) : none();
   });
@@ -255,9 +260,8 @@ PyObject* sdp_attention_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         gq = empty_like_shape(q->sizes(), *q), gk = empty_like_shape(k->sizes(), *k), gv = empty_like_shape(v->sizes(), *v);
       bp.dout = g->data_ptr(), bp.dq = gq.data_ptr(), bp.dk = gk.data_ptr(), bp.dv = gv.data_ptr();
       strides3(bp.dout_stride, *g), strides3(bp.dq_stride, gq), strides3(bp.dk_stride, gk), strides3(bp.dv_stride, gv);
-      const size_t bytes = ttsdpa_backward_workspace_bytes(&bp);
-      const Scratch ws(bytes, *q);
-      rc = ttsdpa_backward(&bp, ws.ptr, bytes, stream_of(*q));
+      const Scratch ws(ttsdpa_backward_workspace_bytes(&bp), *q);
+      rc = ttsdpa_backward(&bp, ws.ptr, ws.bytes, stream_of(*q));
     }
     return rc == TTSDPA_OK ? tuple_of({&gq, &gk, &gv}) : none();
   });
@@ -464,10 +468,9 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::DimVector shape(x->sizes());
     shape.back() = N;
     return result_of(*x, shape, [&](void* out) {
-      const size_t bytes = ttlinear_matmul_workspace_bytes(dt, M, N, K, 0, 1);
-      const Scratch ws(bytes, *x);
+      const Scratch ws(ttlinear_matmul_workspace_bytes(dt, M, N, K, 0, 1), *x);
       return ttlinear_matmul(dt, x->data_ptr(), w->data_ptr(), b ? b->data_ptr() : nullptr, out, M, N, K, 0, 1, ldx, ld_of(*w), N, ws.ptr,
-                             bytes, stream_of(*x));
+                             ws.bytes, stream_of(*x));
     });
   });
 }
@@ -485,10 +488,9 @@ PyObject* matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t shape[2] = {M, N};
     return result_of(*x, shape, [&](void* out) {
       const int dt = dtype_of(*x);
-      const size_t bytes = ttlinear_matmul_workspace_bytes(dt, M, N, K, ta, tb);
-      const Scratch ws(bytes, *x);
+      const Scratch ws(ttlinear_matmul_workspace_bytes(dt, M, N, K, ta, tb), *x);
       return ttlinear_matmul(dt, x->data_ptr(), y->data_ptr(), bias ? bias->data_ptr() : nullptr, out, M, N, K, ta, tb, ld_of(*x), ld_of(*y), N,
-                             ws.ptr, bytes, stream_of(*x));
+                             ws.ptr, ws.bytes, stream_of(*x));
     });
   });
 }
@@ -521,10 +523,9 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t shape[1] = {N};
         gb = empty_like_shape(shape, *x);
       }
-      const size_t bytes = ttlinear_backward_workspace_bytes(dt, M, N, K);
-      const Scratch ws(bytes, *x);
+      const Scratch ws(ttlinear_backward_workspace_bytes(dt, M, N, K), *x);
       rc = ttlinear_backward(dt, g->data_ptr(), x->data_ptr(), w->data_ptr(), gi.data_ptr(), gw.data_ptr(), need_bias ? gb.data_ptr() : nullptr,
-                             M, N, K, ldg, ldx, ld_of(*w), ws.ptr, bytes, stream_of(*x));
+                             M, N, K, ldg, ldx, ld_of(*w), ws.ptr, ws.bytes, stream_of(*x));
     }
     return rc == TTSDPA_OK ? tuple_of({&gi, &gw, need_bias ? &gb : nullptr}) : none();
   });

@@ -27,6 +27,16 @@ def _workspace(device, nbytes):
     return torch.empty(max(int(nbytes), 16), dtype=torch.uint8, device=device)
 
 
+def _optional_workspace(device, nbytes):
+    """(scratch, its bytes) for a call that can do without: (None, 0) where none is wanted or the device has no room for it."""
+    if nbytes:
+        try:
+            return _workspace(device, nbytes), nbytes
+        except torch.OutOfMemoryError:
+            pass
+    return None, 0
+
+
 def _strides3(t):
     assert t.stride(-1) == 1 or t.size(-1) == 1
     return (t.stride(0), t.stride(1), t.stride(2))
@@ -135,9 +145,12 @@ def sdpAttention(query, key, value, isCausal=False, attnMask=None, dropoutP=0.0,
     L = _capi.lib()
     with torch.cuda.device(query.device):
         nbytes = L.ttsdpa_workspace_bytes(ctypes.byref(p))
-        ws = _workspace(query.device, nbytes) if nbytes else None
+        ws, have = _optional_workspace(query.device, nbytes)
         stream = torch.cuda.current_stream().cuda_stream
-        rc = L.ttsdpa_forward(ctypes.byref(p), ws.data_ptr() if ws is not None else None, nbytes, stream)
+        rc = L.ttsdpa_forward(ctypes.byref(p), ws.data_ptr() if ws is not None else None, have, stream)
+        if rc == _capi.ERR_WORKSPACE:  # a call that cannot do without
+            ws = _workspace(query.device, nbytes)
+            rc = L.ttsdpa_forward(ctypes.byref(p), ws.data_ptr(), nbytes, stream)
     if rc != 0:
         raise RuntimeError("ttsdpa_forward failed: %d (%s)" % (rc, _capi.status_string(rc)))
     return out
@@ -452,8 +465,7 @@ def matmul(a, b, transA=False, transB=False, bias=None):
     bs = bias.contiguous() if bias is not None else None
     out = torch.empty(batch + (M, N), dtype=a.dtype, device=a.device)
     L = _capi.lib()
-    nbytes = L.ttlinear_matmul_workspace_bytes(_DTYPES[a.dtype], M, N, K, int(transA), int(transB))
-    ws = _workspace(a.device, nbytes) if nbytes else None
+    ws, nbytes = _optional_workspace(a.device, L.ttlinear_matmul_workspace_bytes(_DTYPES[a.dtype], M, N, K, int(transA), int(transB)))
     lda = a.stride(-2) if a.shape[-2] > 1 else max(a.shape[-1], 1)
     ldb = b.stride(-2) if b.shape[-2] > 1 else max(b.shape[-1], 1)
     common = (_DTYPES[a.dtype], a.data_ptr(), b.data_ptr(), bs.data_ptr() if bs is not None else None, out.data_ptr(), M, N, K,
