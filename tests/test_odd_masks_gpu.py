@@ -66,7 +66,7 @@ def _against_64_bits(out, host, mask):
 @pytest.mark.parametrize("steep", [False, True])
 def test_probabilities_are_fp32(L, S, D, dtype, kind, steep):
     """16-bit calls of the general route: as close to the 64-bit result as the vector-ALU kernel, whose probabilities are fp32
-    (bf16 ones, 2^-9 each, leave four results of ten off by a rounding).  steep: scores spread over some 20, and the key
+    (16-bit ones leave four results of ten off by a rounding).  steep: scores spread over some 20, and the key
     with the most weight holds zeros, so that the result is that of the small probabilities."""
     B, Hq, Hkv = 2, 4, 2
     print("fp32 probabilities", L, S, D, dtype, kind, steep, flush=True)
@@ -143,3 +143,61 @@ def test_gradients_are_fp32(B, Hq, Hkv, L, S, D, dtype, kind, size):
         want = ref.to(got.dtype)
         assert (got != want).double().mean().item() <= 0.01, name
         assert ((got.double() - ref).norm() / ref.norm()).item() <= 1.001 * ((want.double() - ref).norm() / ref.norm()).item() + 1e-7, name
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("D", [64, 72, 128])
+@pytest.mark.parametrize("form", ["keys strided", "per head", "per entry and key"])
+def test_layouts(form, D, dtype):
+    """Views of one packed buffer, masks whose keys are strided or whose rows or heads are broadcast, grouped heads: output and gradients."""
+    B, Hq, Hkv, L, S = 2, 6, 2, 61, 147
+    print("layouts", form, D, dtype, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(21)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to({"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[dtype])
+    q = r(B, L, Hq, D + 8)[..., :D].transpose(1, 2)  # rows of wider rows, sequence outside the heads
+    kv = r(B, S, 2 * Hkv, D).transpose(1, 2)
+    k, v = kv[:, :Hkv], kv[:, Hkv:]
+    go = r(B, L, Hq, D).transpose(1, 2)
+    if form == "keys strided":
+        mask = (torch.rand(S, L, generator=g, device="cuda") < 0.7).t()
+        mask[:, 5] = True
+    elif form == "per head":
+        mask = r(Hq, 1, S)
+    else:
+        mask = r(B, 1, 1, 2 * S)[..., ::2]
+    rc, out = call("forward", q, k, v, mask=mask)
+    assert rc == 0
+    rc, grads = backward_call(q, k, v, out, go, mask=mask)
+    assert rc == 0
+    host = [t.float().cpu().numpy() for t in (q, k, v)]
+    p, qd, kk, vv, gd, group = _gradients_64(host, go, mask)
+    ref = torch.matmul(p, vv)
+    ds = p * (torch.matmul(gd, vv.transpose(-1, -2).contiguous()) - (gd * out.double()).sum(-1, keepdim=True)) / D ** 0.5
+    refs = (ref, torch.matmul(ds, kk), group(torch.matmul(ds.transpose(-1, -2).contiguous(), qd)), group(torch.matmul(p.transpose(-1, -2).contiguous(), gd)))
+    for name, got, want in zip(("out", "dq", "dk", "dv"), (out,) + tuple(grads), refs):
+        rounded = want.to(got.dtype).double()
+        # one rounding of the result (16-bit), and fp32 sums of some 150 products in another order
+        assert ((got.double() - want).norm() / want.norm()).item() <= 1.01 * ((rounded - want).norm() / want.norm()).item() + 2e-6, name
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("D", [64, 80])
+def test_pages(D, dtype):
+    """The same call on a paged cache, the pages scattered: bit for bit the contiguous one's result."""
+    B, H, L, S, page = 2, 4, 50, 256, 64
+    host, (q, k, v) = make_inputs(8995, B, H, H, L, S, D, dtype)
+    table = torch.tensor([[3, 0, 6, 1], [7, 2, 5, 4]], dtype=torch.int32, device="cuda")
+    pools = []
+    for t in (k, v):
+        pool = torch.zeros(8, H, page, D, dtype=t.dtype, device="cuda")
+        for b in range(B):
+            for i in range(4):
+                pool[table[b, i].item()] = t[b, :, page * i:page * (i + 1)]
+        pools.append(pool)
+    lens = torch.tensor([251, 130], dtype=torch.int32, device="cuda")
+    mask = torch.from_numpy(np.random.default_rng(3).random((L, S)) > 0.4).cuda()
+    mask[:, 0] = True
+    whole, paged = call("forward", q, k, v, mask=mask, kv_lens=lens), call("forward", q, *pools, mask=mask, kv_lens=lens, block_table=table)
+    assert whole[0] == 0 and paged[0] == 0 and torch.equal(whole[1], paged[1])
+    vec = call("general", q, k, v, mask=mask, kv_lens=lens)
+    assert (whole[1] != vec[1]).double().mean().item() <= 0.005  # (a rounding here and there)
