@@ -859,8 +859,7 @@ template <typename TR, bool CAUSAL>
 int launch_k(const KArgs& a, dim3 grid, hipStream_t stream) {
   if (a.kv_splits > 1) return a.block_table ? launch_v<TR, CAUSAL, true, true>(a, grid, stream) : launch_v<TR, CAUSAL, false, true>(a, grid, stream);
   if constexpr (!CAUSAL)
-    if (a.mask_kind != 0)  // the host sends only Bool masks the streams can apply (bool_mask_streams_ok)
-      return launch_v<TR, false, false, false, true>(a, grid, stream);
+    if (a.mask_kind != 0) return launch_v<TR, false, false, false, true>(a, grid, stream);
   return a.block_table ? launch_v<TR, CAUSAL, true, false>(a, grid, stream) : launch_v<TR, CAUSAL, false, false>(a, grid, stream);
 }
 
@@ -868,6 +867,8 @@ int launch_k(const KArgs& a, dim3 grid, hipStream_t stream) {
 
 int launch_prefill_d128(const KArgs& args, int dtype, hipStream_t stream) {
   KArgs a = args;
+  // the host sends no other masks here; one of those would be read as bytes that it does not hold, or left out
+  if (a.mask_kind != 0 && !bool_mask_streams_ok(a)) return (int)hipErrorInvalidValue;
   const int ntile = (a.L + BM - 1) / BM;
   long long nwg = (long long)a.B * a.Hq * (a.causal ? (ntile + 1) / 2 : ntile);
   // Mirror pairs are equal work, so a launch of them ends evenly only when the pairs fill whole rounds of the chip's 256

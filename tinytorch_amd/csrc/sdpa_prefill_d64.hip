@@ -782,10 +782,7 @@ int launch_v(const KArgs& a, dim3 grid, hipStream_t stream) {
 template <typename TR, bool CAUSAL>
 int launch_k(const KArgs& a, dim3 grid, hipStream_t stream) {
   if constexpr (!CAUSAL)
-    if (a.mask_kind != 0) {  // the host sends only Bool masks the streams can apply (bool_mask_streams_ok)
-      if (!bool_mask_streams_ok(a)) return (int)hipErrorInvalidValue;
-      return launch_v<TR, false, false, true>(a, grid, stream);
-    }
+    if (a.mask_kind != 0) return launch_v<TR, false, false, true>(a, grid, stream);
   return a.kv_splits > 1 ? launch_v<TR, CAUSAL, true>(a, grid, stream) : launch_v<TR, CAUSAL, false>(a, grid, stream);
 }
 
@@ -793,6 +790,8 @@ int launch_k(const KArgs& a, dim3 grid, hipStream_t stream) {
 
 int launch_prefill_d64(const KArgs& args, int dtype, hipStream_t stream) {
   KArgs a = args;
+  // the host sends no other masks here; one of those would be read as bytes that it does not hold, or left out
+  if (a.mask_kind != 0 && !bool_mask_streams_ok(a)) return (int)hipErrorInvalidValue;
   const int ntile = (a.L + BM - 1) / BM;
   long long nwg = (long long)a.B * a.Hq * (a.causal ? (ntile + 1) / 2 : ntile);
   // Mirror pairs are equal work, so a launch of them ends evenly only when the pairs fill whole rounds of the chip's 256
