@@ -83,10 +83,12 @@ __device__ __forceinline__ vec8 v_operand(const void* lane_base, int byte_off_lo
 // and the kind is known, which keeps registers.  The shape above, lengths 49 to 197: 17.3 -> 13.1 us (nothing hidden: 17.6 -> 14.3);
 // 30 x 16 x 513 x 64, bf16: 152 -> 106; 8 x 12 x 777 x 80: 94 -> 80; 16-bit probabilities, 16 x 12 x 512 x 32: 33.2 -> 18.6.
 // From head_dim 128 on it spills (8 x 12 x 777 x 128: 74.7, 68.0 without; 4 x 8 x 300 x 256: 37.5, 28.8).
+// SPLIT: a launch with divided keys, a variant of its own: as a run-time branch it made short launches without them slower (forward
+// and backward of 4 x 2 heads x 103 rows, head_dim 64, causal 24.1 us, 23.8 so).
 // PAD: the tensors' head_dim a.D is a multiple of 8 below D.  The 16-byte chunks of a row beyond a.D are taken as zeros
 // (Q and K: they add nothing to a score; V: columns of the output that are not stored), everything else is the
 // kernel for head_dim D.  The reference takes any head size (src/Function/FuncNNLayer.h:231-236).
-template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP>
+template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP, bool SPLIT>
 __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a) {
   typedef typename TR::elem T;
   typedef typename TR::vec8 vec8;
@@ -116,9 +118,8 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   const int inner = a.G * ntile;           // workgroups that share one (batch, kv head)
   const int npair = a.B * a.Hkv;
   int pair, in;
-  const int nsplit = a.kv_splits > 1 ? a.kv_splits : 1;
   int split = 0;    // key range of this workgroup (the only one unless the keys are split)
-  if (nsplit > 1) {
+  if (SPLIT) {
     if (!find_piece(a, BM, CAUSAL, &pair, &in, &split)) return;
   } else {
     const int n = blockIdx.x;
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
     int len = __builtin_amdgcn_readfirstlane(a.kv_len[b]);
     S = len < 0 ? 0 : (len < S ? len : S);
   }
-  if (S == 0 && nsplit == 1) {  // no keys: zeros, the reference's empty contraction
+  if (!SPLIT && S == 0) {  // no keys: zeros, the reference's empty contraction
     const int qi = qw0 + lq;
     if (qi < a.L) {
       T* op = (T*)a.out + b * a.os[0] + h * a.os[1] + qi * a.os[2];
@@ -197,7 +198,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   const int ntiles_kv = (last_key_of_rows(a, q0, BM, S) + BN) / BN;
   // tiles jt0 .. jt1-1 are this workgroup's: all of them, or those of its split (kv_chunk is a multiple of the tile)
   int jt0 = 0, jt1 = ntiles_kv;
-  if (nsplit > 1) {
+  if (SPLIT) {
     jt0 = split * (a.kv_chunk / BN);
     const int end = jt0 + a.kv_chunk / BN;
     jt1 = end < jt1 ? end : jt1;
@@ -468,7 +469,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   // ---- normalise and store ----------------------------------------------------------------------------------------------
   float l_tot = l_run + __shfl_xor(l_run, 32);
   const int qi = qw0 + lq;
-  if (nsplit > 1 && ntiles_kv * BN > a.kv_chunk) {  // a partial result (else the row tile's keys end in the first split: the output itself)
+  if (SPLIT && ntiles_kv * BN > a.kv_chunk) {  // a partial result (else the row tile's keys end in the first split: the output itself)
     store_split_record<D>(a, (long long)b * a.Hq + h, split, qw0, lane, oacc, m_use, l_tot);
     return;
   }
@@ -488,30 +489,38 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   }
 }
 
-template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP = false>
-int launch_prefill_k(const KArgs& a, dim3 grid, hipStream_t stream) {
+template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP, bool SPLIT>
+int launch_prefill_v(const KArgs& a, hipStream_t stream) {
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  const hipError_t granted = grant_dynamic_lds((const void*)prefill_kernel<TR, D, CAUSAL, MASK, PAD, FULLP>, PrefillLds<D>::BYTES, state, done);
+  const hipError_t granted = grant_dynamic_lds((const void*)prefill_kernel<TR, D, CAUSAL, MASK, PAD, FULLP, SPLIT>, PrefillLds<D>::BYTES, state, done);
   if (granted != hipSuccess) return (int)granted;
-  hipLaunchKernelGGL((prefill_kernel<TR, D, CAUSAL, MASK, PAD, FULLP>), grid, dim3(256), PrefillLds<D>::BYTES, stream, a);
+  const long long nwg = SPLIT ? split_grid(a, BM) : (long long)a.B * a.Hq * ((a.L + BM - 1) / BM);
+  hipLaunchKernelGGL((prefill_kernel<TR, D, CAUSAL, MASK, PAD, FULLP, SPLIT>), dim3((unsigned)nwg), dim3(256), PrefillLds<D>::BYTES, stream, a);
   return (int)hipGetLastError();
+}
+
+template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP = false>
+int launch_prefill_k(const KArgs& a, hipStream_t stream) {
+  return a.kv_splits > 1 ? launch_prefill_v<TR, D, CAUSAL, MASK, PAD, FULLP, true>(a, stream)
+                         : launch_prefill_v<TR, D, CAUSAL, MASK, PAD, FULLP, false>(a, stream);
 }
 
 template <typename TR, int D, bool PAD>
 int launch_prefill_t(const KArgs& a, hipStream_t stream) {
   // the callers keep to this (rows are read in 16-byte chunks)
   if (PAD && (a.D % 8 != 0 || a.D >= D || a.D < 8)) return (int)hipErrorInvalidValue;
-  const long long nwg = a.kv_splits > 1 ? split_grid(a, BM) : (long long)a.B * a.Hq * ((a.L + BM - 1) / BM);
-  dim3 grid((unsigned)nwg);
   if (a.mask_kind != 0)  // exclusive with causal (validated)
-    return a.mask_kind == 1 ? a.full_p ? launch_prefill_k<TR, D, false, 1, PAD, true>(a, grid, stream) : launch_prefill_k<TR, D, false, 1, PAD>(a, grid, stream)
-           : a.full_p       ? launch_prefill_k<TR, D, false, 2, PAD, true>(a, grid, stream)
-                            : launch_prefill_k<TR, D, false, 2, PAD>(a, grid, stream);
-  return a.causal ? launch_prefill_k<TR, D, true, 0, PAD>(a, grid, stream) : launch_prefill_k<TR, D, false, 0, PAD>(a, grid, stream);
+    return a.mask_kind == 1 ? a.full_p ? launch_prefill_k<TR, D, false, 1, PAD, true>(a, stream) : launch_prefill_k<TR, D, false, 1, PAD>(a, stream)
+           : a.full_p       ? launch_prefill_k<TR, D, false, 2, PAD, true>(a, stream)
+                            : launch_prefill_k<TR, D, false, 2, PAD>(a, stream);
+  return a.causal ? launch_prefill_k<TR, D, true, 0, PAD>(a, stream) : launch_prefill_k<TR, D, false, 0, PAD>(a, stream);
 }
 
 }  // namespace
+
+// The file is compiled twice, for the time that it takes: fp16 and what is common, and with TT_PREFILL_BF16 bf16.
+int launch_prefill_bf16(const KArgs& a, hipStream_t stream);
 
 template <typename TR>
 int launch_prefill_d(const KArgs& a, hipStream_t stream) {
@@ -533,6 +542,9 @@ int launch_prefill_d(const KArgs& a, hipStream_t stream) {
   return launch_prefill_t<TR, 256, true>(a, stream);
 }
 
+#ifdef TT_PREFILL_BF16
+int launch_prefill_bf16(const KArgs& a, hipStream_t stream) { return launch_prefill_d<BF16>(a, stream); }
+#else
 int launch_split_merge(const KArgs& a, int dtype, int W, int rows, hipStream_t stream) {
   const long long blocks = (long long)a.B * a.Hq * ((a.L + 31) / 32);
   if (blocks > 0x7fffffffLL) return (int)hipErrorInvalidValue;
@@ -544,7 +556,8 @@ int launch_split_merge(const KArgs& a, int dtype, int W, int rows, hipStream_t s
 }
 
 int launch_prefill(const KArgs& a, int dtype, hipStream_t stream) {
-  return dtype == 1 ? launch_prefill_d<F16>(a, stream) : launch_prefill_d<BF16>(a, stream);
+  return dtype == 1 ? launch_prefill_d<F16>(a, stream) : launch_prefill_bf16(a, stream);
 }
+#endif
 
 }  // namespace ttsdpa
