@@ -63,7 +63,11 @@ int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, v
  * forward's x [M,K] and w [N,K] (row strides ldg, ldx, ldw in elements)
  *   grad_x [M,K] = grad . w,   grad_w [N,K] = grad^T . x,   grad_b [N] = column sums of grad (NULL: not wanted),
  * all dense, sums in fp32, one rounding of each result.  M, N, K > 0.  workspace: ttlinear_backward_workspace_bytes() bytes of
- * device scratch, 256-byte aligned (TTSDPA_ERR_WORKSPACE with less).  Enqueues on `stream`. */
+ * device scratch, 256-byte aligned.  Much of it may be for copies of the operands, which are faster to multiply than operands read
+ * in place (bf16, 8192 x 6144 x 4096: 169 MB, the weight's gradient 340 us with its copies, 443 without).  With less the call
+ * runs without what does not fit, down to the column sums' parts, ttlinear_backward_least_workspace_bytes() (196 KB there);
+ * TTSDPA_ERR_WORKSPACE with less than that.  Enqueues on `stream`. */
+size_t ttlinear_backward_least_workspace_bytes(int dtype, int64_t M, int64_t N);
 size_t ttlinear_backward_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K);
 int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w, void* grad_x, void* grad_w, void* grad_b, int64_t M,
                       int64_t N, int64_t K, int64_t ldg, int64_t ldx, int64_t ldw, void* workspace, size_t workspace_bytes,

@@ -302,6 +302,11 @@ def test_linear_routes_and_validation():
     assert plan(_capi.BF16, -1, 64, 64)[0] == _capi.ERR_SHAPE
     assert plan(_capi.BF16, 64, 64, 64, ldx=32)[0] == _capi.ERR_STRIDE
     assert plan(_capi.BF16, 64, 64, 64, x=None)[0] == _capi.ERR_NULL
+    # the layer's backward: room for the column sums' parts is enough, less is refused
+    least = L.ttlinear_backward_least_workspace_bytes(_capi.BF16, 8192, 6144)
+    assert 0 < least < 1 << 20 < L.ttlinear_backward_workspace_bytes(_capi.BF16, 8192, 6144, 4096)
+    assert L.ttlinear_backward(_capi.BF16, *[FAKE] * 6, 8192, 6144, 4096, 6144, 4096, 4096, FAKE, least - 1, None) == _capi.ERR_WORKSPACE
+    assert L.ttlinear_backward(_capi.BF16, *[FAKE] * 6, 8192, 6144, 4096, 6144, 4096, 4096, None, 1 << 30, None) == _capi.ERR_WORKSPACE
     assert L.ttlinear_forward(_capi.BF16, None, None, None, None, 0, 64, 64, 64, 64, 64, None) == 0
     assert L.ttlinear_forward(_capi.BF16, FAKE, FAKE, None, None, 8, 64, 64, 64, 64, 64, None) == _capi.ERR_NULL
 

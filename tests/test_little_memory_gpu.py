@@ -76,6 +76,52 @@ def test_linear_backward(way):
         assert rel(a, b) <= REL
 
 
+def test_linear_backward_in_place():
+    """The weight's gradient is made on copies of its operands (75 MB): without room for them on operands as they lie.  Nor is there
+    room for what the call would be made of otherwise, an fp32 copy of grad."""
+    M, N, K = 2048, 9216, 4096
+    x, w, g = operands((M, K), (N, K), (M, N))
+    refs = (g.float() @ w.float(), g.float().t() @ x.float(), g.float().sum(0))
+    L = _capi.lib()
+    need, least = L.ttlinear_backward_workspace_bytes(_capi.BF16, M, N, K), L.ttlinear_backward_least_workspace_bytes(_capi.BF16, M, N)
+    assert need > 60 * MB and least < MB
+    torch.cuda.synchronize()
+    with room((M * K + N * K) * 2 + 16 * MB):
+        got = tt.linearBackward(g, x, w)
+    for a, b in zip(got, refs):
+        assert rel(a, b) <= REL
+    # any scratch between the two is enough
+    for nbytes in (least, need - 1):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        out = [torch.empty_like(t) for t in got]
+        rc = L.ttlinear_backward(_capi.BF16, g.data_ptr(), x.data_ptr(), w.data_ptr(), *[t.data_ptr() for t in out], M, N, K, N, K, K,
+                                 ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rc == 0
+        for a, b in zip(out, refs):
+            assert rel(a, b) <= REL
+
+
+@pytest.mark.parametrize("M,N,K,dtype", [(64, 500, 784, torch.float32), (1501, 1999, 2501, torch.float32), (300, 260, 4100, torch.bfloat16),
+                                         (4100, 65, 70, torch.float16)])
+def test_linear_backward_with_the_least(M, N, K, dtype):
+    """Products on the streaming kernel, of which the weight's would be divided, or made in one launch with the other."""
+    x, w, g = operands((M, K), (N, K), (M, N), dtype=dtype)
+    L = _capi.lib()
+    kind = {torch.float32: _capi.F32, torch.float16: _capi.F16, torch.bfloat16: _capi.BF16}[dtype]
+    least = L.ttlinear_backward_least_workspace_bytes(kind, M, N)
+    assert 0 < least <= L.ttlinear_backward_workspace_bytes(kind, M, N, K)
+    ws = torch.full((least + 4096,), 77, dtype=torch.uint8, device="cuda")
+    out = [torch.empty(s, dtype=dtype, device="cuda") for s in ((M, K), (N, K), (N,))]
+    rc = L.ttlinear_backward(kind, g.data_ptr(), x.data_ptr(), w.data_ptr(), *[t.data_ptr() for t in out], M, N, K, N, K, K, ws.data_ptr(),
+                             least, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0
+    assert bool((ws[least:] == 77).all())
+    for a, b in zip(out, (g.double() @ w.double(), g.double().t() @ x.double(), g.double().sum(0))):
+        assert rel(a, b) <= (1e-5 if dtype == torch.float32 else REL)
+
+
 def test_attention(way):
     B, H, L, S, D = 1, 16, 100, 8191, 128
     q, k, v = operands((B, H, L, D), (B, H, S, D), (B, H, S, D))

@@ -27,7 +27,7 @@ EXPORTS = [
     "ttfused_rms_norm", "ttfused_add_rms_norm", "ttfused_silu_mul", "ttfused_softmax", "ttfused_softmax_backward",
     # include/ttlinear.h
     "ttlinear_forward", "ttlinear_plan", "ttlinear_matmul", "ttlinear_matmul_batched", "ttlinear_matmul_workspace_bytes",
-    "ttlinear_backward", "ttlinear_backward_workspace_bytes",
+    "ttlinear_backward", "ttlinear_backward_workspace_bytes", "ttlinear_backward_least_workspace_bytes",
 ]
 LINEAR_ROUTE_NAMES = {0: "none", 1: "mfma", 2: "general"}
 
@@ -172,6 +172,8 @@ def lib():
         L.ttlinear_matmul_batched.restype = ctypes.c_int
         L.ttlinear_backward_workspace_bytes.argtypes = [ctypes.c_int, i64, i64, i64]
         L.ttlinear_backward_workspace_bytes.restype = ctypes.c_size_t
+        L.ttlinear_backward_least_workspace_bytes.argtypes = [ctypes.c_int, i64, i64]
+        L.ttlinear_backward_least_workspace_bytes.restype = ctypes.c_size_t
         L.ttlinear_backward.argtypes = [ctypes.c_int] + [vp] * 6 + [i64] * 6 + [vp, ctypes.c_size_t, vp]
         L.ttlinear_backward.restype = ctypes.c_int
         if L.ttsdpa_abi_version() != 7:

@@ -1396,6 +1396,10 @@ int ttlinear_matmul_batched(int dtype, const void* a, const void* b, const void*
 // Ranges of rows that a packed grad^T's column sums come in.
 static long long pack_ranges(long long kpad) { return (kpad + kPackRows - 1) / kPackRows; }
 
+size_t ttlinear_backward_least_workspace_bytes(int dtype, int64_t M, int64_t N) {
+  return M <= 0 || N <= 0 ? 0 : (size_t)colsum_ranges(M, N, dtype) * (size_t)N * sizeof(float);
+}
+
 size_t ttlinear_backward_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const LinArgs g = flags_args(N, K, M, 1, 0);
@@ -1403,7 +1407,7 @@ size_t ttlinear_backward_workspace_bytes(int dtype, int64_t M, int64_t N, int64_
   size_t gw = ttlinear_matmul_workspace_bytes(dtype, N, K, M, 1, 0);
   PackPlan p;
   if (choose(g, dtype, true, ~(size_t)0, &p) == Way::Packed) gw = p.bytes + (size_t)pack_ranges(p.kpad) * (size_t)N * sizeof(float);
-  const size_t gb = (size_t)colsum_ranges(M, N, dtype) * (size_t)N * sizeof(float);
+  const size_t gb = ttlinear_backward_least_workspace_bytes(dtype, M, N);
   const size_t pair = stream_pair_scratch(g, flags_args(M, K, N, 0, 0), dtype);
   size_t most = gi > gw ? gi : gw;  // one after the other on the same scratch
   if (pair > most) most = pair;
@@ -1420,7 +1424,7 @@ int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w,
   const size_t esz = dtype == TTSDPA_F32 ? 4 : 2;
   if (!aligned(grad, esz) || !aligned(x, esz) || !aligned(w, esz) || !aligned(grad_x, esz) || !aligned(grad_w, esz) || !aligned(grad_b, esz))
     return TTSDPA_ERR_STRIDE;
-  if (workspace_bytes < ttlinear_backward_workspace_bytes(dtype, M, N, K) || (workspace_bytes && (!workspace || !aligned(workspace, 256))))
+  if (workspace_bytes < ttlinear_backward_least_workspace_bytes(dtype, M, N) || !workspace || !aligned(workspace, 256))
     return TTSDPA_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   // grad_w [N,K] = grad^T . x, grad_x [M,K] = grad . w
@@ -1436,7 +1440,7 @@ int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w,
   const Way way_i = choose(gi, dtype, true, workspace_bytes, &pi, &us_i);
   const bool pair = way_w == Way::Stream && way_i == Way::Stream;
   if ((pair || (dtype == TTSDPA_F32 && stream_takes(gw, dtype) && stream_takes(gi, dtype))) &&
-      stream_pair_cost(gw, gi, dtype) < us_w + us_i + 5) {
+      stream_pair_cost(gw, gi, dtype) < us_w + us_i + 5 && stream_pair_scratch(gw, gi, dtype) <= workspace_bytes) {
     gw.rowsum = grad_b;
     return launch_stream_pair(gw, gi, dtype, s, workspace);
   }

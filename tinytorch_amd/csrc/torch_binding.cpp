@@ -63,19 +63,25 @@ Tensor empty_like_shape(at::IntArrayRef shape, const Tensor& like) {
 
 // Device scratch of one call from torch's caching allocator: a buffer per call, so that the allocator orders reuse by
 // stream and a captured call keeps its scratch in the graph's pool.  Where the device has no room for it the call goes on with
-// none: the C ABI runs it without (operands read in place, keys not divided) or says that it cannot.
+// the least it asks for, or none: the C ABI runs it without (operands read in place, keys not divided) or says that it cannot.
 struct Scratch {
   Tensor t;
   void* ptr = nullptr;
   size_t bytes = 0;
-  Scratch(size_t want, const Tensor& like) {
-    if (want == 0) return;
+  Scratch(size_t want, const Tensor& like, size_t least = 0) {
+    if (!take(want, like) && least < want) take(least, like);
+  }
+
+ private:
+  bool take(size_t want, const Tensor& like) {
+    if (want == 0) return true;
     try {
       t = at::empty({(int64_t)want}, at::TensorOptions().dtype(at::kByte).device(like.device()));
     } catch (const c10::OutOfMemoryError&) {
-      return;
+      return false;
     }
     ptr = t.data_ptr(), bytes = want;
+    return true;
   }
 };
 
@@ -523,7 +529,7 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t shape[1] = {N};
         gb = empty_like_shape(shape, *x);
       }
-      const Scratch ws(ttlinear_backward_workspace_bytes(dt, M, N, K), *x);
+      const Scratch ws(ttlinear_backward_workspace_bytes(dt, M, N, K), *x, ttlinear_backward_least_workspace_bytes(dt, M, N));
       rc = ttlinear_backward(dt, g->data_ptr(), x->data_ptr(), w->data_ptr(), gi.data_ptr(), gw.data_ptr(), need_bias ? gb.data_ptr() : nullptr,
                              M, N, K, ldg, ldx, ld_of(*w), ws.ptr, ws.bytes, stream_of(*x));
     }
