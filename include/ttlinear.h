@@ -59,6 +59,17 @@ int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, v
                     int trans_a, int trans_b, int64_t lda, int64_t ldb, int64_t ldo, void* workspace,
                     size_t workspace_bytes, void* stream);
 
+/* The output tiles that ttlinear_matmul makes a 16-bit product of dense, aligned operands on, given its workspace (rows x columns; OTHER:
+ * fp32, the streaming kernel, operands read contraction-major).  Estimates decide: the answer may change with the library. */
+enum ttlinear_tiles {
+  TTLINEAR_TILES_OTHER = 0,
+  TTLINEAR_TILES_128x128 = 1,
+  TTLINEAR_TILES_256x256 = 2,
+  TTLINEAR_TILES_128x256 = 3, /* where 256 x 256 would leave CUs idle */
+  TTLINEAR_TILES_MIXED = 4    /* whole rounds of 256 x 256, what is left as 128 x 256 */
+};
+int ttlinear_matmul_tiles(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b);
+
 /* FuncLinear::backward (reference src/Function/FuncNNLayer.h:20-33) in one call: from the upstream gradient grad [M,N], the
  * forward's x [M,K] and w [N,K] (row strides ldg, ldx, ldw in elements)
  *   grad_x [M,K] = grad . w,   grad_w [N,K] = grad^T . x,   grad_b [N] = column sums of grad (NULL: not wanted),

@@ -302,6 +302,10 @@ def test_linear_routes_and_validation():
     assert plan(_capi.BF16, -1, 64, 64)[0] == _capi.ERR_SHAPE
     assert plan(_capi.BF16, 64, 64, 64, ldx=32)[0] == _capi.ERR_STRIDE
     assert plan(_capi.BF16, 64, 64, 64, x=None)[0] == _capi.ERR_NULL
+    # the tiles of 16-bit products: a tile for every CU and more, and what is not on tiles
+    tiles = lambda *a: _capi.LINEAR_TILES_NAMES[L.ttlinear_matmul_tiles(*a)]
+    assert tiles(_capi.BF16, 8192, 8192, 8192, 0, 1) == tiles(_capi.F16, 8192, 8192, 8192, 0, 1) == "256x256"
+    assert tiles(_capi.F32, 8192, 8192, 8192, 0, 1) == tiles(_capi.BF16, 1, 4096, 4096, 0, 1) == tiles(_capi.BF16, 0, 64, 64, 0, 1) == "other"
     # the layer's backward: room for the column sums' parts is enough, less is refused
     least = L.ttlinear_backward_least_workspace_bytes(_capi.BF16, 8192, 6144)
     assert 0 < least < 1 << 20 < L.ttlinear_backward_workspace_bytes(_capi.BF16, 8192, 6144, 4096)

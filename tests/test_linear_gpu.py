@@ -280,11 +280,18 @@ def test_matmul_batched_against_oracle(dtype, case):
     assert err <= tol
 
 
+def tiles_of(M, N, K, dtype):
+    return _capi.LINEAR_TILES_NAMES[_capi.lib().ttlinear_matmul_tiles(_capi.BF16 if dtype == torch.bfloat16 else _capi.F16, M, N, K, 0, 1)]
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M,N,K", [(1999, 4096, 832), (2048, 4090, 1024), (1921, 3841, 1088), (1500, 5000, 896), (129, 32769, 960)])
+@pytest.mark.parametrize("M,N,K", [(1999, 4096, 832), (2048, 4090, 1024), (1921, 3841, 1088), (1500, 5000, 896),
+                                   (129, 32700, 2112), (2048, 4090, 2176), (1921, 3841, 2240), (1500, 5000, 2048)])
 def test_half_tiles(M, N, K, dtype):
-    """128 x 256 tiles (products whose 256 x 256 tiles would leave CUs idle): edges in both directions, 13 to 17 k-tiles over three
-    stages.  Bound: half a unit in the last place of the result's type for each element (fp32 sums: 2^-24 each, far below)."""
+    """128 x 256 tiles (products whose 256 x 256 tiles would leave CUs idle): edges in both directions, 13 to 17 and 32 to 35 k-tiles
+    over three stages.  The short ones are estimated 3 to 5 % faster so than on other tiles, the long ones 12 and more.  Bound: half a
+    unit in the last place of the result's type for each element (fp32 sums: 2^-24 each, far below)."""
+    assert tiles_of(M, N, K, dtype) == "128x256"
     g = torch.Generator(device="cuda").manual_seed(M + K)
     x, w = (torch.randn(n, K, generator=g, device="cuda").to(dtype) for n in (M, N))
     b = torch.randn(N, generator=g, device="cuda").to(dtype)
@@ -295,10 +302,13 @@ def test_half_tiles(M, N, K, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M,N,K", [(4200, 5000, 832), (4225, 4990, 896), (6144, 4095, 832), (1921, 12000, 960), (3001, 7400, 1024)])
+@pytest.mark.parametrize("M,N,K", [(4200, 5000, 832), (4225, 4990, 896), (6144, 4095, 832), (1921, 12000, 960), (3001, 7400, 1024),
+                                   (4200, 5000, 2112), (4225, 4990, 2176), (6144, 4095, 2240)])
 def test_mixed_tiles(M, N, K, dtype):
     """Whole rounds of 256 x 256 tiles, the rest in halves of 128 x 256: a last tile row whose second half is empty or has one row,
-    XCDs with fewer tiles than the others, up to half a round left over, 13 to 16 k-tiles.  Bound as for the halves alone."""
+    XCDs with fewer tiles than the others, up to half a round left over, 13 to 16 and 33 to 35 k-tiles (estimated 3 to 12 % faster so than
+    otherwise, the long ones 13 and more).  Bound as for the halves alone."""
+    assert tiles_of(M, N, K, dtype) == "mixed"
     g = torch.Generator(device="cuda").manual_seed(M + K)
     x, w = (torch.randn(n, K, generator=g, device="cuda").to(dtype) for n in (M, N))
     b = torch.randn(N, generator=g, device="cuda").to(dtype)

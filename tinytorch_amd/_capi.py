@@ -27,9 +27,11 @@ EXPORTS = [
     "ttfused_rms_norm", "ttfused_add_rms_norm", "ttfused_silu_mul", "ttfused_softmax", "ttfused_softmax_backward",
     # include/ttlinear.h
     "ttlinear_forward", "ttlinear_plan", "ttlinear_matmul", "ttlinear_matmul_batched", "ttlinear_matmul_workspace_bytes",
+    "ttlinear_matmul_tiles",
     "ttlinear_backward", "ttlinear_backward_workspace_bytes", "ttlinear_backward_least_workspace_bytes",
 ]
 LINEAR_ROUTE_NAMES = {0: "none", 1: "mfma", 2: "general"}
+LINEAR_TILES_NAMES = {0: "other", 1: "128x128", 2: "256x256", 3: "128x256", 4: "mixed"}
 
 
 class Params(ctypes.Structure):
@@ -163,6 +165,8 @@ def lib():
         L.ttlinear_plan.restype = ctypes.c_int
         L.ttlinear_matmul_workspace_bytes.argtypes = [ctypes.c_int, i64, i64, i64, ctypes.c_int, ctypes.c_int]
         L.ttlinear_matmul_workspace_bytes.restype = ctypes.c_size_t
+        L.ttlinear_matmul_tiles.argtypes = [ctypes.c_int, i64, i64, i64, ctypes.c_int, ctypes.c_int]
+        L.ttlinear_matmul_tiles.restype = ctypes.c_int
         L.ttlinear_matmul.argtypes = [ctypes.c_int, vp, vp, vp, vp, i64, i64, i64, ctypes.c_int, ctypes.c_int, i64, i64, i64,
                                       vp, ctypes.c_size_t, vp]
         L.ttlinear_matmul.restype = ctypes.c_int

@@ -684,10 +684,10 @@ __global__ __launch_bounds__(256, 1) void linear256_kernel(LinArgs a) {
   linear256_tile<TR, TM>(a, (long long)tm * TM, (long long)tn * 256);
 }
 
-// Large tiles in whole rounds of the CUs (an XCD has 32), what is left over in halves: a last round of large tiles that is half full or less
-// costs nearly as much as a full one of halves, which is shorter, and a half takes the place of a tile as soon as a CU is free.
-// Forward and both gradients, in us: 2048 x 4096 x 9216 551 -> 498, 5000 x 4096 x 3584 502 -> 442, 8192 x 4096 x 6144 1075 -> 1040 (the
-// weight's gradient alone, 384 tiles, of them).
+// Large tiles in whole rounds of the CUs (an XCD has 32), what is left over in halves: a last round of large tiles that is half full
+// or less takes nearly as long as a full one; in halves it is a full one, but of tiles half as long, and a half takes the place of a
+// tile as soon as a CU is free.  Forward and both gradients, in us, without and with it: 2048 x 4096 x 9216 518, 459; 5000 x 4096 x
+// 3584 475, 417; 8192 x 4096 x 6144 1025, 984 (there the weight's gradient alone is such a product: 384 tiles).
 constexpr int kCusOfXcd = 32;
 
 template <typename TR>
@@ -1075,8 +1075,8 @@ double small_tiles_cost(const LinArgs& a, int dtype, unsigned entries) {
   return 1 + cold + 1.2 * rounds + steps * (rounds > 1 ? 0.54 * (rounds - 1) + 0.3 + 0.24 * fill : 0.54 + 0.06 * fill);
 }
 // The hand-ordered kernel's 256 x 256 tiles, 16-bit, one to a CU: 9 us a round for its first loads and its output and 1.5 a k-step, in
-// a last round that is not full less, because the power is shared by fewer (1999 x 4096 x 14336, 128 tiles, 240 us; x 6144 x 4096, 192, 82; 4096 x 4096 x 4096, 256, 102; 4096 x 6144 x
-// 8192, 384, 318).
+// a last round that is not full less, because the power is shared by fewer (1999 x 4096 x 14336, 128 tiles, 240 us; x 6144 x 4096,
+// 192, 82; 4096 x 4096 x 4096, 256, 102; 4096 x 6144 x 8192, 384, 318).
 // Few k-steps do not hide a tile's first loads (2495 x 4876, 3 steps: 22 us; on the small tiles 16).
 double large_cold(const LinArgs& a) { return a.K < 1024 ? 5 * (2 - a.K / 512.0) : 0; }
 double large_tiles_cost(const LinArgs& a) {
@@ -1110,16 +1110,26 @@ double nt_cost(const LinArgs& a, int dtype, unsigned entries) {
   return mixed < us ? mixed : us;
 }
 
+// The tiles of a 16-bit product on rows of whole k-tiles: the cheapest by estimate.
+int tiles_of(const LinArgs& a) {
+  const double us = nt_cost(a, TTSDPA_BF16, 1);
+  if (large_tiles_cost(a) <= us) return TTLINEAR_TILES_256x256;
+  if (half_tiles_cost(a) <= us) return TTLINEAR_TILES_128x256;
+  if (mixed_tiles_cost(a) <= us) return TTLINEAR_TILES_MIXED;
+  return TTLINEAR_TILES_128x128;
+}
+
 template <typename TR>
 int launch_mfma(const LinArgs& a, hipStream_t stream) {
   // (four wavefronts with 128 x 128 each — accumulators in AGPRs, half the LDS operand reads — measured 2-10 % slower
   // than eight with 64 x 128: one wavefront per SIMD hides too little)
   if constexpr (!std::is_same<TR, F32>::value) {
-    const double us = nt_cost(a, TTSDPA_BF16, 1);  // the hand-ordered kernel's two tiles
-    if (large_tiles_cost(a) <= us) return launch_linear256<TR, 256>(a, stream);
-    if (half_tiles_cost(a) <= us) return launch_linear256<TR, 128>(a, stream);
-    if (mixed_tiles_cost(a) <= us) return launch_linear256_mixed<TR>(a, stream);
-    return launch_small_tiles<TR>(a, stream);
+    switch (tiles_of(a)) {
+      case TTLINEAR_TILES_256x256: return launch_linear256<TR, 256>(a, stream);  // the hand-ordered kernel
+      case TTLINEAR_TILES_128x256: return launch_linear256<TR, 128>(a, stream);
+      case TTLINEAR_TILES_MIXED: return launch_linear256_mixed<TR>(a, stream);
+      default: return launch_small_tiles<TR>(a, stream);
+    }
   } else {
     const long long big = ((a.M + 255) / 256) * ((a.N + 255) / 256);
     return big >= 256 ? launch_mfma_stages<TR, 256, 256, 4, 2, 2>(a, stream, 1) : launch_small_tiles<TR>(a, stream);
@@ -1296,6 +1306,15 @@ size_t ttlinear_matmul_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t 
   const bool packed = choose(g, dtype, true, ~(size_t)0, &p) == Way::Packed;
   const size_t parts = stream_scratch(g, dtype);
   return packed && p.bytes > parts ? p.bytes : parts;
+}
+
+int ttlinear_matmul_tiles(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
+  if ((dtype != TTSDPA_F16 && dtype != TTSDPA_BF16) || M <= 0 || N <= 0 || K <= 0) return TTLINEAR_TILES_OTHER;
+  LinArgs g = flags_args(M, N, K, trans_a, trans_b);
+  PackPlan p;
+  if (choose(g, dtype, true, ~(size_t)0, &p) != Way::Packed) return TTLINEAR_TILES_OTHER;
+  g.K = p.kpad, g.xt = g.wt = 0;
+  return tiles_of(g);
 }
 
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
