@@ -1,7 +1,7 @@
-"""Key splits of the pipelined prefill kernels (head_dim 128 and 64): calls with at most a quarter as many 256-row tiles as the chip
-has CUs (a chunk of rows against a long cache, a few heads) divide the keys of a row tile among workgroups, and the decode path's merge kernel combines their
-records.  ttsdpa_forward with its workspace takes that form; ttsdpa_prefill (no workspace) runs the same call unsplit:
-both against the oracle, and against each other.  The records are combined by the kernel file's own merge kernel."""
+"""Key splits of the pipelined prefill kernels (head_dim 128 and 64): calls with at most half as many 256-row tiles as the chip has
+CUs (a chunk of rows against a long cache, a few heads) divide the keys of a row tile among workgroups, and the prefill kernels'
+merge kernel (split_merge_kernel) combines their records.  ttsdpa_forward with its workspace takes that form; ttsdpa_prefill (no
+workspace) runs the same call unsplit: both against the oracle, and against each other."""
 import ctypes
 
 import numpy as np

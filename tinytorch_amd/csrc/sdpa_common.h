@@ -32,7 +32,7 @@ struct KArgs {
   int pack_L;
   // Split keys (prefill kernels): workgroup (.., split) covers keys split * kv_chunk .. + kv_chunk - 1 of its row tile and leaves a
   // record per row in ws (store_split_record) for split_merge_kernel, or the output itself where the row tile's keys end in the
-  // first split.  kv_splits <= 1: no split.
+  // first split (the pipelined kernel of head_dim 64: a record then too).  kv_splits <= 1: no split.
   int kv_splits, kv_chunk;
   float* ws;
   int full_p;  // 4-wavefront prefill kernel with an attnMask: probabilities reach the matrix cores with all their fp32 bits
@@ -613,7 +613,7 @@ __host__ __device__ inline int split_classes(const KArgs& a) { return pair_class
 // The piece of a split launch of a prefill kernel (row tiles of `rows` rows) that this workgroup takes.  A class's pieces start in
 // this order: every row tile's first split, longest row tile first, then every row tile's second one ... (those that run together
 // read the same keys), and without gaps: a workgroup with nothing to do among the others leaves CUs empty (workgroups go to the
-// parts of an XCD in turn: 2 heads on 1 of 8192 rows, head_dim 128, 68 us with gaps, 42 so).  False: nothing is left for this one.
+// parts of an XCD in turn: 2 heads on 1 of 8192 rows, head_dim 128, 68 us with gaps, 42 so; the merge takes 5 more).  False: nothing is left for this one.
 // in: the head in its group and the row tile (longest first under a causal mask).
 __device__ __forceinline__ bool find_piece(const KArgs& a, int rows, bool causal, int* pair, int* in, int* split) {
   const int gq = split_classes(a), ppc = a.B * a.Hkv / gq;

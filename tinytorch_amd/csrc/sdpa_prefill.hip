@@ -431,7 +431,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
     } else if (SKIP && MASK_AHEAD && jt + 1 < jt1) {
       load_mask(kv0 + BN);
     }
-        if constexpr (FULLP) {  // what the first parts left of the probabilities
+    if constexpr (FULLP) {  // what the first parts left of the probabilities
       T* Vs = smem + cur * Lds::STAGE + BN * K_PITCH;
       const int* flags = vflags + 4 * cur;
       if (__builtin_expect(__builtin_amdgcn_readfirstlane(flags[0] | flags[1] | flags[2] | flags[3]) != 0, 0)) {

@@ -321,7 +321,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
     if (kt0 + 2 < ntiles_kv) dma_v(kt0 + 2, 2);
   };
   issue_tiles(0);
-  // ---- Bool attnMask in the streams (kStreamed) -------------------------------------------------------------------------------
+  // ---- Bool attnMask in the streams (MASKB) ----------------------------------------------------------------------------------
   // Ring in LDS: two tiles of 2 KiB per wavefront behind the K/V stages.  Load i of a tile (two per tile) brings the 64-byte
   // segments of rows 16i .. 16i+15 of the wavefront, 16 bytes per lane: lane l the chunk l/16 of row 16i + l%16, which lands at
   // 1024 i + 16 l, i.e. chunk c of row q at 1024 (q/16) + 256 c + 16 (q%16).  A lane (row q, h = lane/32) needs dwords g = 0..3 of

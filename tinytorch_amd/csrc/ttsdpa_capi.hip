@@ -151,27 +151,33 @@ bool pipelined_ok(const ttsdpa_params* p) {
   return long_d128(p) && (p->mask_kind == TTSDPA_MASK_NONE || mask_streams_best(p));
 }
 
-// Shapes whose row tiles the pipelined kernels divide among workgroups by keys (plan_pipelined_splits): `units` 256-row
-// tiles in all, `keys` = what a row can see (under a top-left aligned causal mask no more than there are rows).
-bool split_shape(const ttsdpa_params* p, long long* units, long long* keys) {
-  *units = (long long)p->B * p->Hq * ((p->L + 255) / 256);
-  *keys = effective_causal(p) == TTSDPA_CAUSAL_TOP_LEFT && p->L < p->S ? p->L : p->S;
-  if (p->mask_kind != TTSDPA_MASK_NONE || *units > 128 || *keys < 2048) return false;
-  return *units <= 64 || (p->causal && *keys >= 4096);
+// 256-row tiles in all.
+long long row_tiles(const ttsdpa_params* p) { return (long long)p->B * p->Hq * ((p->L + 255) / 256); }
+
+// Keys that a row can see: under a top-left aligned causal mask no more than there are rows.
+long long visible_keys(const ttsdpa_params* p) {
+  return effective_causal(p) == TTSDPA_CAUSAL_TOP_LEFT && p->L < p->S ? p->L : p->S;
 }
 
-// The pipelined kernel at head_dim 64: no pages, and of attnMasks only Bool masks its streams can apply.  Against the 4-wavefront kernel (128-row tiles, keys
-// divided among workgroups when the heads are not grouped) it measured level or up to 30 % faster from 512 query rows
-// on; shorter calls take it when they fill half of the chip's CUs, or when their keys are split (16 heads x 256 rows on
-// 32768 keys: 0.56 ms on the 4-wavefront kernel, which cannot split grouped heads).
+// The pipelined kernel at head_dim 64: no pages, and of attnMasks only Bool masks its streams can apply.  Against the 4-wavefront
+// kernel (128-row tiles) it measured level or up to 30 % faster from 512 query rows on; shorter calls take it when they fill half of
+// the chip's CUs, or on many keys with up to 64 row tiles (causal: 128).  Both kernels divide the keys of these among workgroups; us
+// on the 4-wavefront kernel and on this one, rows by keys, no mask:
+//   130 x 512:    8 heads  9.2 and 11.1    32 heads 11.0 and 11.1    100 heads  11.7 and  11.6
+//   256 x 2048:   8       12.8     14.5    32       18.9     23.4    100        31.7      28.4
+//   400 x 4096:   8       20.5     20.8    32       31.0     28.7
+//   256 x 16384:  8       25.6     25.4    32       56.6     48.4    100       183.8     148.6
+// so that neither line is sharp: few heads on 2048 to 4096 keys lose up to a fifth here, 65 to 128 row tiles without a mask on 4096
+// keys or more up to a third there.
 bool pipelined64_ok(const ttsdpa_params* p) {
   if (p->D != 64 || p->L <= 128 || p->block_table) return false;
   if (p->mask_kind != TTSDPA_MASK_NONE && !mask_streams_best(p)) return false;
   if (!(p->k_stride[2] < (1 << 24) && p->v_stride[2] < (1 << 24) && p->q_stride[2] < (1 << 22))) return false;
   const long long tiles = (p->L + 255) / 256;
   if ((long long)p->B * p->Hq * (p->causal ? (tiles + 1) / 2 : tiles) >= 128) return true;
-  long long units, keys;
-  return p->L >= 512 || split_shape(p, &units, &keys);
+  if (p->L >= 512) return true;
+  const long long units = row_tiles(p), keys = visible_keys(p);
+  return p->mask_kind == TTSDPA_MASK_NONE && keys >= 2048 && (units <= 64 || (units <= 128 && p->causal && keys >= 4096));
 }
 
 // Few query rows per head against many keys on the 4-wavefront kernel: the G heads of a KV head share one row tile
@@ -201,12 +207,14 @@ struct SplitPlan {
   size_t ws_bytes;
 };
 
-// heads, L: with records of L rows each; share: of the keys, that a row sees on average; whole_us: of the unsplit call, where it does not follow from the rest; tile_us, tile: of one key tile; slots: workgroups that run side by side; step: a chunk is a multiple of it
+// heads, L: with records of L rows each; share: of the keys, that a row sees on average; tile_us, tile: of one key tile; slots:
+// workgroups that run side by side; step: a chunk is a multiple of it; whole_us: of the unsplit call, where it does not follow from
+// the rest
 SplitPlan cheapest_split(long long wgs, long long keys, long long heads, int L, int width, double share, double tile_us, int tile, int slots, int step,
                          double whole_us = 0) {
   SplitPlan best{1, 0, 0};
   double least = 0;
-  for (long long want = 1; want <= 64; want++) {  // 64: the merge kernels' limit
+  for (long long want = 1; want <= 64; want++) {  // (64: more have not been measured)
     long long chunk = (keys + want - 1) / want;
     chunk = (chunk + step - 1) / step * step;
     const long long n = (keys + chunk - 1) / chunk;
@@ -287,9 +295,8 @@ struct SplitCost {
 // 6000, 5392 and 4062 keys: 134 us whole, 128 with 68-tile pieces, 141 with 64, 151 with 32).
 SplitPlan plan_pipelined_splits(const ttsdpa_params* p) {
   SplitPlan s{1, 0, 0};
-  long long units, keys;
   if (p->dtype == TTSDPA_F32 || !(pipelined_ok(p) || pipelined64_ok(p)) || p->mask_kind != TTSDPA_MASK_NONE) return s;
-  split_shape(p, &units, &keys);
+  const long long units = row_tiles(p), keys = visible_keys(p);
   if (units > 128 || keys < 512) return s;
   const long long heads = (long long)p->B * p->Hq;
   const int ntile = (p->L + 255) / 256, causal = effective_causal(p);
