@@ -83,12 +83,14 @@ __device__ __forceinline__ vec8 v_operand(const void* lane_base, int byte_off_lo
 // and the kind is known, which keeps registers.  The shape above, lengths 49 to 197: 17.3 -> 13.1 us (nothing hidden: 17.6 -> 14.3);
 // 30 x 16 x 513 x 64, bf16: 152 -> 106; 8 x 12 x 777 x 80: 94 -> 80; 16-bit probabilities, 16 x 12 x 512 x 32: 33.2 -> 18.6.
 // From head_dim 128 on it spills (8 x 12 x 777 x 128: 74.7, 68.0 without; 4 x 8 x 300 x 256: 37.5, 28.8).
-// SPLIT: a launch with divided keys, a variant of its own: as a run-time branch it made short launches without them slower (forward
-// and backward of 4 x 2 heads x 103 rows, head_dim 64, causal 24.1 us, 23.8 so).
+// SPLIT: whether the keys are divided: 0 no, 1 yes, 2 told at run time.  Variants of their own where that is faster (as a run-time
+// branch: forward and backward of 4 x 2 heads x 103 rows, head_dim 64, causal 24.1 us, 23.8 so).  The additive masks' variants, the
+// Bool ones from head_dim 128 on and head_dim 256 lose by it: the compiler keeps more addresses in registers and spills (25 x 12
+// heads x 36 rows, head_dim 128, additive 12.3 us, 8.3 with the branch; 4 x 8 x 300 x 256, causal 25.4, 24.0).
 // PAD: the tensors' head_dim a.D is a multiple of 8 below D.  The 16-byte chunks of a row beyond a.D are taken as zeros
 // (Q and K: they add nothing to a score; V: columns of the output that are not stored), everything else is the
 // kernel for head_dim D.  The reference takes any head size (src/Function/FuncNNLayer.h:231-236).
-template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP, bool SPLIT>
+template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP, int SPLIT>
 __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a) {
   typedef typename TR::elem T;
   typedef typename TR::vec8 vec8;
@@ -118,8 +120,9 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   const int inner = a.G * ntile;           // workgroups that share one (batch, kv head)
   const int npair = a.B * a.Hkv;
   int pair, in;
-  int split = 0;    // key range of this workgroup (the only one unless the keys are split)
-  if (SPLIT) {
+  const bool divided = SPLIT == 1 || (SPLIT == 2 && a.kv_splits > 1);
+  int split = 0;    // key range of this workgroup (the only one unless the keys are divided)
+  if (divided) {
     if (!find_piece(a, BM, CAUSAL, &pair, &in, &split)) return;
   } else {
     const int n = blockIdx.x;
@@ -180,7 +183,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
     int len = __builtin_amdgcn_readfirstlane(a.kv_len[b]);
     S = len < 0 ? 0 : (len < S ? len : S);
   }
-  if (!SPLIT && S == 0) {  // no keys: zeros, the reference's empty contraction
+  if (S == 0 && !divided) {  // no keys: zeros, the reference's empty contraction
     const int qi = qw0 + lq;
     if (qi < a.L) {
       T* op = (T*)a.out + b * a.os[0] + h * a.os[1] + qi * a.os[2];
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   const int ntiles_kv = (last_key_of_rows(a, q0, BM, S) + BN) / BN;
   // tiles jt0 .. jt1-1 are this workgroup's: all of them, or those of its split (kv_chunk is a multiple of the tile)
   int jt0 = 0, jt1 = ntiles_kv;
-  if (SPLIT) {
+  if (divided) {
     jt0 = split * (a.kv_chunk / BN);
     const int end = jt0 + a.kv_chunk / BN;
     jt1 = end < jt1 ? end : jt1;
@@ -469,7 +472,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   // ---- normalise and store ----------------------------------------------------------------------------------------------
   float l_tot = l_run + __shfl_xor(l_run, 32);
   const int qi = qw0 + lq;
-  if (SPLIT && ntiles_kv * BN > a.kv_chunk) {  // a partial result (else the row tile's keys end in the first split: the output itself)
+  if (divided && ntiles_kv * BN > a.kv_chunk) {  // a partial result (else the row tile's keys end in the first split: the output itself)
     store_split_record<D>(a, (long long)b * a.Hq + h, split, qw0, lane, oacc, m_use, l_tot);
     return;
   }
@@ -489,21 +492,25 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void prefill_kernel(KArgs a
   }
 }
 
-template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP, bool SPLIT>
+template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP, int SPLIT>
 int launch_prefill_v(const KArgs& a, hipStream_t stream) {
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
   const hipError_t granted = grant_dynamic_lds((const void*)prefill_kernel<TR, D, CAUSAL, MASK, PAD, FULLP, SPLIT>, PrefillLds<D>::BYTES, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long nwg = SPLIT ? split_grid(a, BM) : (long long)a.B * a.Hq * ((a.L + BM - 1) / BM);
+  const long long nwg = a.kv_splits > 1 ? split_grid(a, BM) : (long long)a.B * a.Hq * ((a.L + BM - 1) / BM);
   hipLaunchKernelGGL((prefill_kernel<TR, D, CAUSAL, MASK, PAD, FULLP, SPLIT>), dim3((unsigned)nwg), dim3(256), PrefillLds<D>::BYTES, stream, a);
   return (int)hipGetLastError();
 }
 
 template <typename TR, int D, bool CAUSAL, int MASK, bool PAD, bool FULLP = false>
 int launch_prefill_k(const KArgs& a, hipStream_t stream) {
-  return a.kv_splits > 1 ? launch_prefill_v<TR, D, CAUSAL, MASK, PAD, FULLP, true>(a, stream)
-                         : launch_prefill_v<TR, D, CAUSAL, MASK, PAD, FULLP, false>(a, stream);
+  if constexpr (D > 192 || MASK == 2 || (MASK == 1 && D > 96)) {
+    return launch_prefill_v<TR, D, CAUSAL, MASK, PAD, FULLP, 2>(a, stream);
+  } else {
+    return a.kv_splits > 1 ? launch_prefill_v<TR, D, CAUSAL, MASK, PAD, FULLP, 1>(a, stream)
+                           : launch_prefill_v<TR, D, CAUSAL, MASK, PAD, FULLP, 0>(a, stream);
+  }
 }
 
 template <typename TR, int D, bool PAD>

@@ -44,12 +44,13 @@ struct F32Lds {
 // its weights are 0 (a tile whose V holds infinities or NaN is taken, 0 times those counts).  A tile is 2.7 us of matrix
 // instructions: 30 x 16 heads x 300 rows, head_dim 64, lengths 75 to 300 154 -> 110 us; 4 x 8 x 1001 100 -> 90, its longest
 // entry's tiles in a row.
-// SPLIT: a launch with divided keys, a variant of its own: as a run-time branch it made launches without them slower (64 heads x 2527
-// rows, head_dim 64, causal 489 us, 484 so).
+// SPLIT: whether the keys are divided among workgroups: 0 no, 1 yes, 2 told at run time.  Without a mask variants of their own: as a
+// run-time branch it made launches without divided keys slower (64 heads x 2527 rows, head_dim 64, causal 489 us, 484 so).  With a
+// mask the unsplit variant takes more registers than the one that asks (head_dim below 64, Bool: a wavefront a SIMD less).
 // PAD: the tensors' head_dim a.D is a multiple of 4 below D; the 16-byte chunks of a row beyond it are taken as zeros (Q
 // and K: nothing added to a score; V: output columns that are not stored).  The reference takes any head size
 // (src/Function/FuncNNLayer.h:231-236).
-template <int D, bool CAUSAL, int MASK, bool PAD, bool KEYS, bool SPLIT>
+template <int D, bool CAUSAL, int MASK, bool PAD, bool KEYS, int SPLIT>
 __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs a) {
   typedef F32Lds<D> Lds;
   constexpr int K_PITCH = Lds::K_PITCH, V_PITCH = Lds::V_PITCH;
@@ -77,8 +78,9 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
   const int npair = a.B * a.Hkv;
   int pair, in;
   static_assert(!(KEYS && SPLIT), "keys are divided among workgroups or among wavefronts");
-  int split = 0;  // key range of this workgroup (the only one unless the keys are split)
-  if (SPLIT) {
+  const bool divided = SPLIT == 1 || (SPLIT == 2 && a.kv_splits > 1);
+  int split = 0;  // key range of this workgroup (the only one unless the keys are divided)
+  if (divided) {
     if (!find_piece(a, ROWS, CAUSAL, &pair, &in, &split)) return;
   } else {
     const int n = blockIdx.x;
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
     int len = __builtin_amdgcn_readfirstlane(a.kv_len[b]);
     S = len < 0 ? 0 : (len < S ? len : S);
   }
-  if (!SPLIT && S == 0) {  // no keys: zeros, the reference's empty contraction
+  if (S == 0 && !divided) {  // no keys: zeros, the reference's empty contraction
     const int qi = qw0 + lq;
     if (qi < a.L) {
       float* op = (float*)a.out + b * a.os[0] + h * a.os[1] + qi * a.os[2];
@@ -149,7 +151,7 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
   const int ntiles_kv = (last_key_of_rows(a, q0, ROWS, S) + BN) / BN;
   // tiles jt0 .. jt1-1 are this workgroup's: all of them, or those of its split (kv_chunk is a multiple of the tile)
   int jt0 = 0, jt1 = ntiles_kv;
-  if (SPLIT) {
+  if (divided) {
     jt0 = split * (a.kv_chunk / BN);
     const int end = jt0 + a.kv_chunk / BN;
     jt1 = end < jt1 ? end : jt1;
@@ -353,7 +355,7 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
     }
     return;
   }
-  if (SPLIT && ntiles_kv * BN > a.kv_chunk) {  // a partial result (else the row tile's keys end in the first split: the output itself)
+  if (divided && ntiles_kv * BN > a.kv_chunk) {  // a partial result (else the row tile's keys end in the first split: the output itself)
     store_split_record<D>(a, (long long)b * a.Hq + h, split, qw0, lane, oacc, m_use, l_tot);
     return;
   }
@@ -372,14 +374,14 @@ __global__ __launch_bounds__(256, (KEYS ? 1 : 2)) void prefill_f32_kernel(KArgs 
   }
 }
 
-template <int D, bool CAUSAL, int MASK, bool PAD, bool KEYS, bool SPLIT>
+template <int D, bool CAUSAL, int MASK, bool PAD, bool KEYS, int SPLIT>
 int launch_f32_v(const KArgs& a, hipStream_t stream) {
   constexpr int lds = (KEYS ? 4 : 2) * F32Lds<D>::STAGE * 4, rows = KEYS ? 32 : BM;
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
   const hipError_t granted = grant_dynamic_lds((const void*)prefill_f32_kernel<D, CAUSAL, MASK, PAD, KEYS, SPLIT>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long nwg = SPLIT ? split_grid(a, rows) : (long long)a.B * a.Hq * ((a.L + rows - 1) / rows);
+  const long long nwg = a.kv_splits > 1 ? split_grid(a, rows) : (long long)a.B * a.Hq * ((a.L + rows - 1) / rows);
   if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL((prefill_f32_kernel<D, CAUSAL, MASK, PAD, KEYS, SPLIT>), dim3((unsigned)nwg), dim3(256), lds, stream, a);
   return (int)hipGetLastError();
@@ -408,8 +410,12 @@ bool keys_among_wavefronts(const KArgs& a, double* tiles_walked = nullptr) {
 
 template <int D, bool CAUSAL, int MASK, bool PAD>
 int launch_f32_k(const KArgs& a, hipStream_t stream) {
-  if (a.kv_splits > 1) return launch_f32_v<D, CAUSAL, MASK, PAD, false, true>(a, stream);
-  return keys_among_wavefronts(a) ? launch_f32_v<D, CAUSAL, MASK, PAD, true, false>(a, stream) : launch_f32_v<D, CAUSAL, MASK, PAD, false, false>(a, stream);
+  if (a.kv_splits <= 1 && keys_among_wavefronts(a)) return launch_f32_v<D, CAUSAL, MASK, PAD, true, 0>(a, stream);
+  if constexpr (MASK != 0) {
+    return launch_f32_v<D, CAUSAL, MASK, PAD, false, 2>(a, stream);
+  } else {
+    return a.kv_splits > 1 ? launch_f32_v<D, CAUSAL, MASK, PAD, false, 1>(a, stream) : launch_f32_v<D, CAUSAL, MASK, PAD, false, 0>(a, stream);
+  }
 }
 
 template <int D, bool PAD>
