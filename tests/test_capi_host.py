@@ -315,6 +315,18 @@ def test_linear_routes_and_validation():
     assert L.ttlinear_forward(_capi.BF16, FAKE, FAKE, None, None, 8, 64, 64, 64, 64, 64, None) == _capi.ERR_NULL
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_splits_of_short_prefill_calls(D):
+    # us whole and in pieces, head_dim 64 / 128: 17.0 / 23.5 and 13.0 / 18.6; 1 x 4096 in 8 pieces and in 16: 21.1 / 30.5 and 25.4 / 31.0
+    def splits(H, L):
+        p = params(_capi.BF16, 1, H, H, L, L, D)
+        return _capi.lib().ttsdpa_workspace_bytes(ctypes.byref(p)) // (H * ((L + 31) // 32) * 32 * (D + 2) * 4)
+
+    assert splits(2, 777) == 4
+    assert splits(1, 4096) == 8
+    assert splits(64, 1024) == 0   # 256 row tiles: whole
+
+
 def test_backward_params_layout_routes_and_validation():
     """struct ttsdpa_backward_params as the header lays it out; plan and validation of ttsdpa_backward without a GPU."""
     L = _capi.lib()

@@ -265,7 +265,9 @@ SplitPlan plan_prefill_splits(const ttsdpa_params* p, const KArgs& a /* after pa
 // row tiles of `tiles` key tiles).  Whole pieces fill rounds of the 256 CUs, the row tiles' last pieces what those leave free and
 // then rounds of their own.  A tile takes 1.4 us, 1.85 with every CU busy (power); a piece that is not all of its row tile leaves a
 // record, 133 KB, which all CUs write at about the same time and the merge kernel reads: 1 x 32 heads x 500 rows on 6000 keys in
-// 4 pieces 54 + 9 us, on 16000 127 + 9.
+// 4 pieces 54 + 9 us, on 16000 127 + 9.  Few records cost little beside the merge's launch: 2 heads x 777 rows, whole 23.5 us, in 4
+// pieces, 32 records, 18.6 (head_dim 64: 17.0, 13.0); 1 x 300 on 600 keys 19.9, 16.7.  Many cost what shorter pieces gain: 1 x 4096
+// in 8 pieces, 128 records, 30.5, in 16 31.0 (head_dim 64: 21.1, 25.4).
 struct SplitCost {
   double chunk, whole = 0, rests = 0, rest = 0, longest_rest = 0, records = 0;
   void add(double count, int tiles) {
@@ -283,7 +285,8 @@ struct SplitCost {
       tiles += left / 256 > longest ? left / 256 : longest;
     }
     const double busy = (whole * chunk + rest) / (256 * tiles);
-    return tiles * (1.4 + 0.45 * busy) + (records > 0 ? 12 + 0.03 * records : 0);
+    const double many = 12 + 0.035 * records, few = 6 + 0.1 * records;
+    return tiles * (1.4 + 0.45 * busy) + (records > 0 ? (few < many ? few : many) : 0);
   }
 };
 
