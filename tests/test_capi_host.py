@@ -315,10 +315,9 @@ def test_linear_routes_and_validation():
     assert L.ttlinear_forward(_capi.BF16, FAKE, FAKE, None, None, 8, 64, 64, 64, 64, 64, None) == _capi.ERR_NULL
 
 
-@pytest.mark.parametrize("D", [64, 128])
-def test_splits_of_short_prefill_calls(D):
-    # us whole and in pieces, head_dim 64 / 128: 17.0 / 23.5 and 13.0 / 18.6; 1 x 4096 in 8 pieces and in 16: 21.1 / 30.5 and 25.4 / 31.0
-    def splits(H, L):
+def test_splits_of_short_prefill_calls():
+    # us whole and in pieces: 2 heads x 777 rows 23.5 and 18.6; 1 x 4096 in 8 pieces 30.5, in 16 31.0
+    def splits(H, L, D=128):
         p = params(_capi.BF16, 1, H, H, L, L, D)
         return _capi.lib().ttsdpa_workspace_bytes(ctypes.byref(p)) // (H * ((L + 31) // 32) * 32 * (D + 2) * 4)
 
