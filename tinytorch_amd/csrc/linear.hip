@@ -1,9 +1,10 @@
 // The linear layer y = x . w^T + bias on gfx950 (reference: op::matmul(input, weight, false, true, bias) behind
 // function::linear, src/Function/FuncNNLayer.h:14-19; device GEMM src/Operation/OpLinalgCuda.cuh:239-293).
 //
-// linear_mfma_kernel (fp16 / bf16 on v_mfma_f32_32x32x16, fp32 on v_mfma_f32_32x32x2 with full fp32 products): a workgroup of 8 wavefronts owns a 256 x 256 tile of the output and walks K in
-// steps of 128 bytes (64 or 32 elements).  Both operands have K contiguous ("NT"), which is the layout v_mfma_f32_32x32x16 wants for both inputs:
-// a lane supplies 8 consecutive k of one row, so operand fragments are plain 16-byte LDS reads, no transposes.
+// linear_mfma_kernel (fp16 / bf16 on v_mfma_f32_32x32x16, fp32 on v_mfma_f32_32x32x2 with full fp32 products): a workgroup of 8
+// wavefronts owns a 256 x 256 tile of the output and walks K in steps of 128 bytes (64 or 32 elements).  Both operands have K
+// contiguous ("NT"), which is the layout v_mfma_f32_32x32x16 wants for both inputs: a lane supplies 8 consecutive k of one row, so
+// operand fragments are plain 16-byte LDS reads, no transposes.
 //   global -> LDS   global_load_lds_dwordx4, two (or four) stages, of 64 KB for this tile (x tile 256 x 64, w tile 256 x 64); the 16-byte chunks
 //                   of a 128-byte LDS row are XOR-swizzled with half the row number so that the 32 rows a fragment read
 //                   touches spread over the banks; the loads for tile t+2 are requested while tile t's last k-step

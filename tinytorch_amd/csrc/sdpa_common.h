@@ -317,8 +317,8 @@ struct BwdArgs {
 
 // Splits of a backward launch that would leave half of the chip idle with `n`: its workgroups walk their streams tile by tile,
 // tile_us each, however few they are.  The number, up to 16, whose longest stream, second launch and partial records (record_us
-// for each split, written and read at 2 TB/s, in fp32, whose tiles hide half of it, 4) take least by estimate: bf16 2 x 4 heads on 1 x 199 rows, head_dim 128: whole backward 50 -> 37 us;
-// fp32 8 heads on 1 x 2000 x 2000, head_dim 64: 665 -> 257.
+// for each split, written and read at 2 TB/s, in fp32, whose tiles hide half of it, 4) take least by estimate: bf16 2 x 4 heads on
+// 1 x 199 rows, head_dim 128: whole backward 50 -> 37 us; fp32 8 heads on 1 x 2000 x 2000, head_dim 64: 665 -> 257.
 inline int cheapest_backward_splits(int n, long long wgs, long long tiles, long long slots, double tile_us, double record_us) {
   if (wgs * n * 2 > slots) return n;
   auto us = [&](int k) {
@@ -613,7 +613,8 @@ __host__ __device__ inline int split_classes(const KArgs& a) { return pair_class
 // The piece of a split launch of a prefill kernel (row tiles of `rows` rows) that this workgroup takes.  A class's pieces start in
 // this order: every row tile's first split, longest row tile first, then every row tile's second one ... (those that run together
 // read the same keys), and without gaps: a workgroup with nothing to do among the others leaves CUs empty (workgroups go to the
-// parts of an XCD in turn: 2 heads on 1 of 8192 rows, head_dim 128, 68 us with gaps, 42 so; the merge takes 5 more).  False: nothing is left for this one.
+// parts of an XCD in turn: 2 heads on 1 of 8192 rows, head_dim 128, 68 us with gaps, 42 so; the merge takes 5 more).
+// False: nothing is left for this one.
 // in: the head in its group and the row tile (longest first under a causal mask).
 __device__ __forceinline__ bool find_piece(const KArgs& a, int rows, bool causal, int* pair, int* in, int* split) {
   const int gq = split_classes(a), ppc = a.B * a.Hkv / gq;
