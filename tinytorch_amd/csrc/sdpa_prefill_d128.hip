@@ -760,6 +760,10 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill128_kernel(KArgs a) {
       dma_wait_and_sync(keep);                                                                           \
       j++;                                                                                               \
     }
+    // Where the loop lies in the code, 16 bytes into a line, and what follows it.  Where earlier code happened to put it, 8 bytes in,
+    // calls of any length were slower: 2 x 4 heads x 565 rows 19.75 us, 19.63 so; 1 x 32 x 1500 37.85, 37.64; 2 x 8 x 300 15.20, 15.12;
+    // 3 x 16 x 1100 32.43, 32.14 (at a line's start 2 x 8 x 300 15.30).
+    if constexpr (CAUSAL && !PAGED && !SPLIT) asm volatile(".p2align 6\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
     for (;;) {
       TT_P128_TILE(0)
       TT_P128_TILE(1)
