@@ -323,6 +323,72 @@ SplitPlan plan_pipelined_splits(const ttsdpa_params* p) {
   return s;
 }
 
+// ---- short sequences (sdpa_short.hip) -----------------------------------------------------------------------------------
+// Calls whose other kernels are a wavefront's chain of a few tiles on part of the chip.  Which way is shorter follows from estimates,
+// each fitted to 128 calls of its element type and head_dim (64, or 128 for those above it): 1 to 4 sequences, 2 to 64 query heads,
+// groups of 1, 2 and 4, 64 to 1024 rows on as many keys, causal or not, us.  They miss by 8 to 10 % on average and by a third at
+// worst, mostly where a second workgroup shares a CU, so that more of those ask for a wider margin.
+struct ShortShape {
+  int rows, keys;         // units of 16
+  double heads, kv, avg;  // query heads and KV heads of all sequences; key units that a row unit sees on average
+  bool causal, f32, wide;
+  int group, L;
+  ShortShape(const ttsdpa_params* p) {
+    const int c = effective_causal(p);
+    rows = (p->L + 15) / 16, keys = ((c == TTSDPA_CAUSAL_TOP_LEFT && p->L < p->S ? p->L : p->S) + 15) / 16;
+    heads = (double)p->B * p->Hq, kv = (double)p->B * p->Hkv, group = p->Hq / p->Hkv, L = p->L;
+    causal = c != TTSDPA_CAUSAL_NONE, f32 = p->dtype == TTSDPA_F32, wide = p->D > 64;
+    const double tri = 0.5 * ((rows < keys ? rows : keys) - 1);
+    avg = !causal ? keys : keys - tri;
+  }
+  // what the workgroups beyond the first on each CU add, in key units (row units)
+  static double more(double wgs, double each) { return wgs > 256 ? (ceil(wgs / 256) - 1) * each : 0; }
+  double least_margin() const { return heads * rows > 256 ? 0.8 : 0.92; }
+
+  double forward_us() const {
+    static const double fit[2][2][3] = {{{4.2, 0.57, 0.11}, {4.2, 1.2, 0.23}}, {{3.9, 1.7, 0.25}, {5.3, 2.8, 0.58}}};
+    const double* c = fit[f32][wide];
+    return c[0] + c[1] * ((keys + 7) / 8) + c[2] * more(heads * rows, avg);
+  }
+  // of the other kernels: 16-bit ones by 64-key tiles, up to eight in a row (more are divided); fp32 ones by the tiles of 32 that their
+  // own rule for dealing them out finds
+  double other_forward_us(double f32_tiles) const {
+    const int tiles = (keys + 3) / 4;
+    const double work = heads * ((L + 127) / 128) * tiles * (causal ? 0.6 : 1.0) / 512, row = tiles < 8 ? tiles : 8;
+    if (f32) return wide ? 5.8 + 2.96 * f32_tiles : 4.0 + 2.3 * f32_tiles;
+    return wide ? 4.8 + 1.47 * row + 0.33 * work + (L > 128 ? 1.5 : 0) : 4.1 + 1.05 * row + 0.48 * work;
+  }
+  // workgroups that share a dk / dv workgroup's units: as many as have a CU, each with a unit for its wavefronts
+  int splits() const {
+    const double wgs = kv * keys;
+    const int most = (group * rows + 7) / 8, room = wgs < 256 ? (int)(256 / wgs) : 1, n = most < room ? most : room;
+    return n < 1 ? 1 : n > 16 ? 16 : n;
+  }
+  double backward_us(bool joint) const {
+    static const double two[2][2][6] = {{{9.6, 1.2, 0.28, 1.3, 0.16, 3.8}, {11.9, 2.5, 0.68, 2.2, 0.30, 4.4}},
+                                        {{11.8, 2.8, 0.74, 2.7, 0.34, 4.3}, {16.8, 5.8, 1.5, 5.2, 0.58, 4.9}}};
+    static const double one[2][2][6] = {{{7.6, 0.163, 0.062, 0.31, 0.71, 3.8}, {10.3, 0.258, 0.132, 0.54, 1.07, 5.1}},
+                                        {{10.7, 0.37, 0.134, 0.46, 1.57, 5.4}, {}}};
+    const int n = splits(), turns = ((group * rows + n - 1) / n + 7) / 8;
+    const double per_key = heads * rows * avg / (kv * keys * n);  // units of a dk / dv workgroup on average
+    const double q = more(heads * rows, avg), k = more(kv * keys * n, per_key), sum = n > 1 ? 1 : 0;
+    if (!joint) {
+      const double* c = two[f32][wide];
+      return c[0] + c[1] * ((keys + 7) / 8) + c[2] * q + c[3] * turns + c[4] * k + c[5] * sum;
+    }
+    if (f32 && wide) return 1e9;  // (its registers do not hold both roles)
+    const double* c = one[f32][wide];
+    const double stats = heads * rows * keys * keys * (causal ? 1.0 / 3 : 1.0) / 256;  // score products for the statistics
+    return c[0] + c[1] * turns * keys + c[2] * stats + c[3] * q + c[4] * k + c[5] * sum;
+  }
+};
+
+// Calls the kernels take, of a length that the estimates are for.
+bool short_ok(const ttsdpa_params* p) {
+  return p->mask_kind == TTSDPA_MASK_NONE && !p->block_table && p->D <= 128 && p->L >= 16 && p->S >= 16 && p->L <= 1024 && p->S <= 1024 &&
+         p->L <= 2 * p->S && p->S <= 2 * p->L && (long long)p->B * p->Hq <= 1024;
+}
+
 bool prefill_ok(const ttsdpa_params* p, bool any_mask = false) {
   if (f32_prefill_ok(p, any_mask)) return true;
   // any attnMask at head_dim 128 with more than 128 rows; else those that can be read four keys at a time
@@ -351,6 +417,13 @@ bool decode_ok(const ttsdpa_params* p) {
 bool f32_decode_ok(const ttsdpa_params* p) {
   return f32_prefill_ok(p) && p->mask_kind == TTSDPA_MASK_NONE && effective_causal(p) != TTSDPA_CAUSAL_TOP_LEFT &&
          (long long)p->L * (p->Hq / p->Hkv) <= kDecodeMaxRows;
+}
+
+// ... where that is the shortest way forward (of a call of the prefill route).
+bool short_forward_best(const ttsdpa_params* p, const KArgs& a) {
+  if (!short_ok(p) || pack_heads_ok(p) || !prefill_ok(p)) return false;
+  const ShortShape s(p);
+  return s.forward_us() < s.least_margin() * s.other_forward_us(s.f32 ? prefill_f32_tiles(a) : 0);
 }
 
 int pick_route(const ttsdpa_params* p) {
@@ -475,6 +548,42 @@ size_t backward_dq_partial_offset(const ttsdpa_backward_params* p) {
   const size_t end = backward_partial_offset(p) + (size_t)n * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float);
   return (end + 255) & ~(size_t)255;
 }
+// Estimated time of a call on the matrix-core pairs, by the longest stream of each kernel.
+double pair_backward_us(const ttsdpa_backward_params* p) {
+  const ttsdpa_params* f = &p->fwd;
+  const ShortShape s(f);
+  if (!s.f32) {
+    const int tiles = (s.keys + 3) / 4, stream = s.group * ((f->L + 31) / 32);
+    const double work = s.heads * ((f->L + 127) / 128) * tiles * (s.causal ? 0.6 : 1.0) / 512, row = tiles < 8 ? tiles : 8, st = stream < 32 ? stream : 32;
+    return s.wide ? 16.6 + 2.2 * row + 6.9 * work + 0.37 * st : 11.6 + 1.7 * row + 4.3 * work + 0.27 * st;
+  }
+  bool dealt;
+  auto us = [&](int n, double wgs, int tiles, double slots, double tile_us) {
+    if (dealt) return ((tiles + 3) / 4 + 0.5) * tile_us;
+    const double rounds = (s.causal ? 0.6 : 1.0) * wgs * n / slots;
+    return (tiles + n - 1) / n * tile_us * (rounds > 1 ? rounds : 1) + (n > 1 ? 4.5 : 0);
+  };
+  const int nk = dkv_splits_of(p, &dealt);
+  const double dkv = us(nk, s.kv * ((f->S + 127) / 128), s.group * ((f->L + 31) / 32), s.wide ? 256 : 512, s.wide ? 10 : 5);
+  const int nq = dq_splits_of(p, &dealt);
+  const double dq = us(nq, s.heads * ((f->L + 127) / 128), (f->S + 31) / 32, s.wide ? 256 : 512, s.wide ? 8 : 4);
+  return s.wide ? 18.5 + 0.54 * dq + 1.08 * dkv : 5.5 + 1.5 * dq + 1.0 * dkv;
+}
+
+// The short sequences' backward: splits of its dk / dv workgroups, 0 where the pairs are the shorter way.
+int short_backward_splits(const ttsdpa_backward_params* p, bool* joint = nullptr) {
+  const ttsdpa_params* f = &p->fwd;
+  if (!short_ok(f) || !(backward_mfma_ok(p) || backward_f32_ok(p))) return 0;
+  const ShortShape s(f);
+  const double one = s.backward_us(true), two = s.backward_us(false);
+  if (joint) *joint = one < two;
+  return (one < two ? one : two) < s.least_margin() * pair_backward_us(p) ? s.splits() : 0;
+}
+size_t short_backward_bytes(const ttsdpa_backward_params* p, int splits) {
+  return backward_partial_offset(p) + (splits > 1 ? (size_t)splits * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float) : 0);
+}
+
+// of the pairs
 size_t backward_scratch_bytes(const ttsdpa_backward_params* p) {
   const int n = dkv_splits_of(p), nq = dq_splits_of(p);
   if (nq > 1)
@@ -599,6 +708,7 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
   if (p->B == 0 || p->L == 0) return TTSDPA_OK;
   if (!prefill_ok(p, any_mask)) return TTSDPA_ERR_UNSUPPORTED;
   if ((rc = check_grid((long long)a.B * a.Hq * ((a.L + 127) / 128))) != TTSDPA_OK) return rc;
+  if (short_forward_best(p, a)) return launch_short_forward(a, p->dtype, (hipStream_t)stream);
   // head_dim 128 with enough rows to fill 256-row workgroups takes the software-pipelined kernel (its tile loads
   // address 64 rows with 32-bit byte offsets)
   if (p->dtype != TTSDPA_F32 && pipelined_ok(p)) {
@@ -710,7 +820,10 @@ int ttsdpa_backward_plan(const ttsdpa_backward_params* p, int* route) {
 size_t ttsdpa_backward_workspace_bytes(const ttsdpa_backward_params* p) {
   BwdArgs a;
   if (validate_backward(p, &a) != TTSDPA_OK) return 0;
-  return backward_scratch_bytes(p);
+  const size_t pairs = backward_scratch_bytes(p);
+  const int n = short_backward_splits(p);
+  const size_t own = n > 0 ? short_backward_bytes(p, n) : 0;
+  return own > pairs ? own : pairs;
 }
 
 int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t workspace_bytes, void* stream) {
@@ -723,6 +836,12 @@ int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t wor
   if (need > 0 && (!workspace || workspace_bytes < need || !ptr_aligned(workspace, 16))) return TTSDPA_ERR_WORKSPACE;
   a.stats = (float*)workspace;
   a.log_sums = backward_log_sums(p) ? a.stats + 2 * backward_rows(p) : nullptr;
+  bool joint = false;
+  const int n = short_backward_splits(p, &joint);
+  if (n > 0 && workspace_bytes >= short_backward_bytes(p, n)) {  // (less scratch than the query asks for: the pairs)
+    a.dkv_splits = n, a.partial = n > 1 ? (float*)((char*)workspace + backward_partial_offset(p)) : nullptr;
+    return launch_short_backward(a, p->fwd.dtype, joint, (hipStream_t)stream);
+  }
   a.dkv_splits = dkv_splits_of(p, &a.dkv_dealt);
   a.partial = a.dkv_splits > 1 ? (float*)((char*)workspace + backward_partial_offset(p)) : nullptr;
   a.dq_splits = dq_splits_of(p, &a.dq_dealt);
