@@ -582,6 +582,8 @@ int launch_prefill_d128(const KArgs& a, int dtype, hipStream_t stream);  // 256-
 int launch_prefill_d64(const KArgs& a, int dtype, hipStream_t stream);   // the same at head_dim 64 (no attnMask, no pages)
 int launch_prefill_f32(const KArgs& a, hipStream_t stream);              // fp32 tensors on the fp32 matrix cores; head_dim 64 or 128
 double prefill_f32_tiles(const KArgs& a);  // key tiles (of 32) that an unsplit launch takes one after the other
+int heads_rows(const KArgs& a, int dtype);                                     // whether, and how, launch_heads is the way for a call
+int launch_heads(const KArgs& a, int dtype, hipStream_t stream);            // with an attnMask, up to 256 keys, 16-bit tensors (sdpa_heads.hip)
 int launch_short_forward(const KArgs& a, int dtype, hipStream_t stream);    // short sequences, any element type (sdpa_short.hip)
 int launch_short_backward(const BwdArgs& a, int dtype, bool joint, hipStream_t stream);  // joint: in one launch
 int launch_decode(const KArgs& a, int dtype, void* workspace, hipStream_t stream);

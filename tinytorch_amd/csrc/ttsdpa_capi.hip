@@ -708,6 +708,8 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
   if (p->B == 0 || p->L == 0) return TTSDPA_OK;
   if (!prefill_ok(p, any_mask)) return TTSDPA_ERR_UNSUPPORTED;
   if ((rc = check_grid((long long)a.B * a.Hq * ((a.L + 127) / 128))) != TTSDPA_OK) return rc;
+  a.full_p = p->mask_kind != TTSDPA_MASK_NONE && !long_d128(p) && !simple_mask_ok(p);  // (any_mask: the general route's calls, its arithmetic)
+  if (heads_rows(a, p->dtype) > 0) return launch_heads(a, p->dtype, (hipStream_t)stream);
   if (short_forward_best(p, a)) return launch_short_forward(a, p->dtype, (hipStream_t)stream);
   // head_dim 128 with enough rows to fill 256-row workgroups takes the software-pipelined kernel (its tile loads
   // address 64 rows with 32-bit byte offsets)
@@ -735,7 +737,6 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
         check_grid((long long)a.B * a.Hkv * pl.splits) == TTSDPA_OK)
       return launch_decode(a, p->dtype, workspace, (hipStream_t)stream);
   }
-  a.full_p = p->mask_kind != TTSDPA_MASK_NONE && !long_d128(p) && !simple_mask_ok(p);  // (any_mask: the general route's calls, its arithmetic)
   auto launch = [&](const KArgs& k) {
     return p->dtype == TTSDPA_F32 ? launch_prefill_f32(k, (hipStream_t)stream) : launch_prefill(k, p->dtype, (hipStream_t)stream);
   };
