@@ -109,8 +109,14 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane & 31, lh = lane >> 5;
 
-  int tm, tn;
-  if (!tile_of_block<TM, TN>(a, blockIdx.x >> 3, &tm, &tn)) return;
+  int tm, tn, split = 0, slot = blockIdx.x >> 3, step0 = 0, ntk = (int)(a.K / BK);
+  if (TM == 128 && TN == 128 && a.part) {  // the contraction is divided: all tiles of the first share of it, of the second, ...
+    const int per = (((int)a.M + TM - 1) / TM * (((int)a.N + TN - 1) / TN) + 7) / 8;
+    split = slot / per, slot %= per;
+    step0 = ntk * split / a.splits;  // (few steps and shares: launch_packed)
+    ntk = ntk * (split + 1) / a.splits - step0;
+  }
+  if (!tile_of_block<TM, TN>(a, slot, &tm, &tn)) return;
   const long long m0 = (long long)tm * TM, n0 = (long long)tn * TN;
 
   // ---- global -> LDS: wavefront w moves rows (TM/8)w .. of the x tile and (TN/8)w .. of the w tile, 8 rows (1 KB) per instruction
@@ -125,8 +131,8 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
     const long long r = row < lim ? row : lim;
     return (unsigned)((r * ld + G::KPC * chunk) * ESZ);
   };
-  const char* xbase = (const char*)((const T*)a.x + (long long)blockIdx.y * a.bsx + m0 * a.ldx);
-  const char* wbase = (const char*)((const T*)a.w + (long long)blockIdx.y * a.bsw + n0 * a.ldw);
+  const char* xbase = (const char*)((const T*)a.x + (long long)blockIdx.y * a.bsx + m0 * a.ldx) + (long long)step0 * ROWB;
+  const char* wbase = (const char*)((const T*)a.w + (long long)blockIdx.y * a.bsw + n0 * a.ldw) + (long long)step0 * ROWB;
   const unsigned smem_addr = (unsigned)(unsigned long)(lds_void_t*)smem;
   // issued as asm so that the compiler does not treat it as an LDS store it must order every later LDS read behind
   // (the lane's full address goes in a register pair: a scalar base operand is not always kept in scalar registers by
@@ -164,7 +170,7 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const long long n = n0 + (TN / WN) * wn + 32 * i + 8 * (r >> 2) + 4 * lh + (r & 3);
-      const float b = (a.bias && n < a.N) ? (float)((const T*)a.bias)[n] : 0.f;
+      const float b = (a.bias && !a.part && n < a.N) ? (float)((const T*)a.bias)[n] : 0.f;
 #pragma unroll
       for (int j = 0; j < MJ; j++) acc[i][j][r] = b;
     }
@@ -190,7 +196,6 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
 
   // Past the last tile it is requested again, into stages that nothing reads any more: the number of loads in flight behind
   // every wait is the same.
-  const int ntk = (int)(a.K / BK);
   if (ntk > 0) {
 #pragma unroll
     for (int t = 0; t < ST; t++) dma_tile(t < ntk ? t : ntk - 1, t);
@@ -226,6 +231,41 @@ __global__ __launch_bounds__(WN * WM * 64, 1) void linear_mfma_kernel(LinArgs a)
     // accumulators lie, took 56 us for a 4095 x 4095 x 64 product's rows of odd length, 25 so): 16-byte chunk c of row r at slot c ^ (r % chunks).
     constexpr int CH = TN * ESZ / 16;  // chunks of a row
     __builtin_amdgcn_s_barrier();      // every wavefront has taken its last operands
+    if (a.part) {  // fp32 sums of this share of the contraction, rows of 512 bytes
+#pragma unroll
+      for (int j = 0; j < MJ; j++) {
+        const int row = (TM / WM) * wm + 32 * j + lq;
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+          for (int rg = 0; rg < 4; rg++) {
+            const int c = (TN / WN) / 4 * wn + 8 * i + 2 * rg + lh;
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * rg + e];
+            *(f32x4*)(smem + row * TN * 4 + 16 * (c ^ (row & 31))) = v;
+          }
+      }
+      __syncthreads();
+      float* part = a.part + split * (a.M * a.N + a.M);
+#pragma unroll
+      for (int it = 0; it < TM * 32 / (NW * 64); it++) {
+        const int row = NW * 2 * it + tid / 32, c = tid % 32;
+        const u32x4 v = *(const u32x4*)(smem + row * TN * 4 + 16 * (c ^ (row & 31)));
+        const long long m = m0 + row, n = n0 + 4 * c;
+        if (m >= a.M) continue;
+        float* dst = part + m * a.N + n;
+        if (n + 4 <= a.N) {
+          *(loose16*)dst = v;
+        } else {
+          const f32x4 o = __builtin_bit_cast(f32x4, v);
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            if (n + e < a.N) dst[e] = o[e];
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < MJ; j++) {
       const int row = (TM / WM) * wm + 32 * j + lq;
@@ -987,7 +1027,7 @@ int launch_mfma_stages(const LinArgs& a, hipStream_t stream, unsigned entries) {
   static bool done[kMaxDevices];
   const hipError_t granted = grant_dynamic_lds((const void*)linear_mfma_kernel<TR, TM, TN, WN, WM, ST>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long nwg = blocks_of_tiles(a, TM, TN);
+  const long long nwg = blocks_of_tiles(a, TM, TN) * a.splits;
   if (nwg > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
   hipLaunchKernelGGL((linear_mfma_kernel<TR, TM, TN, WN, WM, ST>), dim3((unsigned)nwg, entries), dim3(WN * WM * 64), lds, stream, a);
   return (int)hipGetLastError();
@@ -999,6 +1039,12 @@ bool tile_per_cu(const LinArgs& a, unsigned entries) { return ((a.M + 127) / 128
 template <typename TR>
 int launch_small_tiles(const LinArgs& a, hipStream_t stream, unsigned entries = 1) {
   return tile_per_cu(a, entries) ? launch_mfma_stages<TR, 128, 128, 4, 2, 4>(a, stream, entries) : launch_mfma_stages<TR, 128, 128, 4, 2, 2>(a, stream, entries);
+}
+
+// ... with the contraction divided (a.splits, a.part)
+template <typename TR>
+int launch_divided(const LinArgs& a, hipStream_t stream) {
+  return launch_mfma_stages<TR, 128, 128, 4, 2, 4>(a, stream, 1);
 }
 
 template <typename TR, int T_, bool XT, bool WT>
@@ -1101,6 +1147,22 @@ double mixed_tiles_cost(const LinArgs& a) {
   return 9 * rounds + 6 + large_cold(a) + a.K / 64.0 * (1.5 * rounds + 0.62 + 0.24 * (2 * left) / kCusOfXcd);
 }
 
+// 128 x 128 tiles whose contraction is divided among S workgroups each, one to a CU at most: a launch more, and the shares' fp32 sums
+// written and read at 5 TB/s.  What leaves most CUs idle otherwise, or goes to the streaming kernel, which takes in the operands of
+// smaller tiles: 288 x 2048 x 6592, 48 tiles, 34.7 there -> 22.9 in 5 shares; 200 x 4096 x 14336, 64, 74 -> 48 in 4; 720 x 1536 x 4736,
+// 72, 43 -> 24 in 3 (2: 26.6; 5, more than a round: 27.3); fp32 119 x 3072 x 9152, 24, 108 -> 75 in 10.  (Four wavefronts of 64 x 64
+// instead of eight of 64 x 32, fewer LDS reads: 3 to 8 % slower in every such call.)
+double divided_cost(const LinArgs& a, int dtype, int S) {
+  const long long tiles = ((a.M + 127) / 128) * ((a.N + 127) / 128);
+  if ((tiles + 7) / 8 * S > kCusOfXcd) return 1e30;  // (an XCD's: 826 x 1536 x 4160, 84 tiles in 3 shares, 33 on some, 36 us; 28 by this)
+  const double esz = dtype == TTSDPA_F32 ? 4 : 2, sums = 5.5 + 8.0 * S * a.M * a.N / 5e6;
+  LinArgs share = a;
+  share.K = (long long)((a.K * esz / 128 + S - 1) / S) * (long long)(128 / esz);
+  const double work = small_tiles_cost(share, dtype, S), read = 2.2 + esz * (a.M + a.N) * a.K / 4.2e6;  // weights from memory: 69 x 6208 x 5440 29.5
+  return (work > read ? work : read) + sums;
+}
+size_t divided_bytes(const LinArgs& a, int S) { return S > 1 ? ((size_t)S * (size_t)(a.M * a.N + a.M) * sizeof(float) + 255) / 256 * 256 : 0; }
+
 // x . w^T on rows of whole k-tiles
 double nt_cost(const LinArgs& a, int dtype, unsigned entries) {
   double us = small_tiles_cost(a, dtype, entries);
@@ -1193,14 +1255,16 @@ static bool in_place_ok(const LinArgs& g, int dtype) {
 
 // x . w^T on the tiled kernels, with copies of the operands whose layout they do not take (contraction-major, rows that are
 // not whole k-tiles, unaligned) in scratch: what the copies need and what the product is estimated to take with them.
+// And the shares of its contraction, where that is divided (S > 1), whose sums lie behind the copies.
 struct PackPlan {
   bool ok, x, w;
   long long kpad;
-  size_t xbytes, bytes;
+  size_t xbytes, copies, bytes;
+  int S;
   double us;
 };
 
-static PackPlan plan_pack(const LinArgs& g, int dtype) {
+static PackPlan plan_pack(const LinArgs& g, int dtype, size_t room) {
   const long long esz = dtype == TTSDPA_F32 ? 4 : 2, bk = ROWB / esz, kpc = 16 / esz;
   PackPlan p{};
   p.kpad = (g.K + bk - 1) / bk * bk;
@@ -1213,10 +1277,19 @@ static PackPlan plan_pack(const LinArgs& g, int dtype) {
   if (!p.ok) return p;
   auto bytes = [&](long long rows) { return ((size_t)rows * (size_t)p.kpad * (size_t)esz + 255) / 256 * 256; };
   p.xbytes = p.x ? bytes(g.M) : 0;
-  p.bytes = p.xbytes + (p.w ? bytes(g.N) : 0);
+  p.copies = p.bytes = p.xbytes + (p.w ? bytes(g.N) : 0);
   LinArgs nt = g;
   nt.K = p.kpad, nt.xt = nt.wt = 0;
-  p.us = nt_cost(nt, dtype, 1) + (double)p.bytes * 2 / 5e6 + 5.5 * (p.x + p.w);  // read and written at 5 TB/s; a launch each, and the next one's wait
+  const double whole = nt_cost(nt, dtype, 1);
+  double us = whole;
+  p.S = 1;
+  const bool may = p.copies == 0 || g.xt || g.wt;  // (copies for the alignment's sake alone: 804 x 1983 x 5329 64 us, undivided 57)
+  for (int S = 2; may && S <= 16 && p.kpad / bk >= 4 * S; S++) {
+    const double divided = divided_cost(nt, dtype, S);
+    if (divided < us && divided < 0.9 * whole && p.copies + divided_bytes(nt, S) <= room) us = divided, p.S = S;
+  }
+  p.bytes += divided_bytes(nt, p.S);
+  p.us = us + (double)p.copies * 2 / 5e6 + 5.5 * (p.x + p.w);  // read and written at 5 TB/s; a launch each, and the next one's wait
   // (262 x 866 x 2545: 6.5 and 5.0 us beside 5.2 MB's 1)
   return p;
 }
@@ -1242,6 +1315,11 @@ static int launch_packed(const LinArgs& g, const PackPlan& p, int dtype, hipStre
     if (rc != 0) return rc;
     nt.w = scratch + p.xbytes, nt.ldw = p.kpad;
   }
+  if (p.S > 1) {
+    nt.splits = p.S, nt.part = (float*)(scratch + p.copies);
+    const int rc = dtype == TTSDPA_F32 ? launch_divided<F32>(nt, s) : dtype == TTSDPA_F16 ? launch_divided<F16>(nt, s) : launch_divided<BF16>(nt, s);
+    return rc != 0 ? rc : launch_linear_merge(nt, dtype, s);
+  }
   return dtype == TTSDPA_F32 ? launch_mfma<F32>(nt, s) : dtype == TTSDPA_F16 ? launch_mfma<F16>(nt, s) : launch_mfma<BF16>(nt, s);
 }
 
@@ -1254,8 +1332,12 @@ static Way choose(const LinArgs& g, int dtype, bool scratch, size_t scratch_byte
   auto take = [&](Way w, double cost) {
     if (cost < best) way = w, best = cost;
   };
-  *p = plan_pack(g, dtype);
-  if (p->ok && p->bytes <= (scratch ? scratch_bytes : 0)) take(Way::Packed, p->us);
+  *p = plan_pack(g, dtype, scratch ? scratch_bytes : 0);
+  // (margins for divided contractions: the estimates miss by a tenth, 719 x 1024 x 2688 15.8 us on the streaming kernel, 16.8
+  // divided; those of the ways that read contraction-major operands as they lie by more, the input gradient of 231 x 19072 x 3072 17
+  // us shorter so than divided with its copies)
+  const double us_packed = p->S == 1 ? p->us : p->copies > 0 ? p->us / 0.75 : p->us / 0.9;
+  if (p->ok && p->bytes <= (scratch ? scratch_bytes : 0)) take(Way::Packed, us_packed);
   if (in_place_ok(g, dtype)) take(Way::InPlace, in_place_cost(g, dtype, 1));
   if (stream_takes(g, dtype)) take(Way::Stream, stream_cost(g, dtype, 1, scratch));
   if (us) *us = best;
@@ -1315,7 +1397,7 @@ int ttlinear_matmul_tiles(int dtype, int64_t M, int64_t N, int64_t K, int trans_
   PackPlan p;
   if (choose(g, dtype, true, ~(size_t)0, &p) != Way::Packed) return TTLINEAR_TILES_OTHER;
   g.K = p.kpad, g.xt = g.wt = 0;
-  return tiles_of(g);
+  return p.S > 1 ? TTLINEAR_TILES_128x128 : tiles_of(g);
 }
 
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,

@@ -28,6 +28,8 @@ bool stream_takes(const LinArgs& a, int dtype);                             // s
 double stream_cost(const LinArgs& a, int dtype, unsigned entries, bool may_split);  // estimated microseconds
 size_t stream_scratch(const LinArgs& a, int dtype);                         // bytes that let it divide the contraction
 int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, unsigned entries = 1, void* scratch = nullptr, size_t scratch_bytes = 0);
+// out = bias + the sums of a.splits shares of a product in a.part (and the row sums)
+int launch_linear_merge(const LinArgs& a, int dtype, hipStream_t stream);
 // a layer's two backward products in one launch (gw: both operands k-major; gi: w k-major), each in the kernel's range
 double stream_pair_cost(const LinArgs& gw, const LinArgs& gi, int dtype);
 size_t stream_pair_scratch(const LinArgs& gw, const LinArgs& gi, int dtype);

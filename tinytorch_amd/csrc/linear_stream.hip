@@ -346,20 +346,29 @@ __device__ __forceinline__ void stream_tile(const LinArgs& a, char* smem, int bl
   }
 }
 
-// out = bias + the sum of the splits' partial products, and the same of the row sums.
-template <typename T>
+// out = bias + the sum of the splits' partial products, and the same of the row sums.  I: integers that hold an index into a split.
+template <typename T, typename I>
 __global__ __launch_bounds__(256) void linear_merge_kernel(LinArgs a) {
+  typedef float loose4 __attribute__((ext_vector_type(4), aligned(4)));  // (a split begins at any element)
+  typedef T out4 __attribute__((ext_vector_type(4)));
   const long long total = a.M * a.N + a.M;
   const long long per = a.rowsum ? total : a.M * a.N;
+  const bool fours = ((a.N | a.ldo) & 3) == 0;
+  const bool whole = ((uintptr_t)a.out & (4 * sizeof(T) - 1)) == 0;
   for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4; i < per; i += (long long)gridDim.x * 1024) {
-    if (i + 4 <= a.M * a.N && (a.N & 3) == 0 && (a.ldo & 3) == 0 && (total & 3) == 0) {
-      f32x4 v = *(const f32x4*)(a.part + i);
+    if (i + 4 <= a.M * a.N && fours) {
+      f32x4 v = *(const loose4*)(a.part + i);
 #pragma unroll 4
-      for (int s = 1; s < a.splits; s++) v += *(const f32x4*)(a.part + s * total + i);
-      const long long m = i / a.N, n = i % a.N;
-      T* dst = (T*)a.out + m * a.ldo + n;
+      for (int s = 1; s < a.splits; s++) v += (f32x4)*(const loose4*)(a.part + s * total + i);
+      const I m = (I)i / (I)a.N, n = (I)i - m * (I)a.N;
+      if (a.bias)
 #pragma unroll
-      for (int e = 0; e < 4; e++) store_from_float(dst + e, v[e] + (a.bias ? load_as_float((const T*)a.bias + n + e) : 0.f));
+        for (int e = 0; e < 4; e++) v[e] += load_as_float((const T*)a.bias + n + e);
+      T* dst = (T*)a.out + (long long)m * a.ldo + n;
+      if (whole) *(out4*)dst = __builtin_convertvector(v, out4);
+      else
+#pragma unroll
+        for (int e = 0; e < 4; e++) store_from_float(dst + e, v[e]);
     } else {
       for (long long k = i; k < i + 4 && k < per; k++) {
         float v = 0.f;
@@ -375,13 +384,19 @@ __global__ __launch_bounds__(256) void linear_merge_kernel(LinArgs a) {
 template <typename T>
 int launch_merge(const LinArgs& a, hipStream_t stream) {
   const long long groups = (a.M * a.N + a.M + 1023) / 1024;
-  hipLaunchKernelGGL((linear_merge_kernel<T>), dim3((unsigned)(groups < 2048 ? groups : 2048)), dim3(256), 0, stream, a);
+  const dim3 grid((unsigned)(groups < 2048 ? groups : 2048));
+  if (a.M * a.N + a.M < 0x7fffffffLL) hipLaunchKernelGGL((linear_merge_kernel<T, uint32_t>), grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((linear_merge_kernel<T, long long>), grid, dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
 
-int launch_merge_type(const LinArgs& a, int dtype, hipStream_t stream) {
+}  // namespace
+
+int launch_linear_merge(const LinArgs& a, int dtype, hipStream_t stream) {
   return dtype == 0 ? launch_merge<float>(a, stream) : dtype == 1 ? launch_merge<_Float16>(a, stream) : launch_merge<__bf16>(a, stream);
 }
+
+namespace {
 
 // Wavefronts and units in flight of each by the tile's size in blocks of 16: eight with a ring of as many units as their registers
 // hold; on the largest tile four, which have twice the registers (eight measure the same, and spill).
@@ -447,7 +462,8 @@ namespace {
 // measurements (MI355X, 16-bit unless said): 3 us of launch, latency and the meeting of the partial sums (2 more on the
 // largest tile: a wavefront's sums are 16 KB); then, for each round of the 256 CUs, half a microsecond and the operands of
 // a tile at the 65 GB/s that a CU takes in (it measured 60-75 over all shapes that the L2s hold or that are read once: when
-// both operands are larger, all tiles together take theirs in at 8 TB/s, 1636 x 3775 x 2025 100 us; 16-bit k-major operands come in pieces of
+// both operands are larger, all tiles together take theirs in at 8 TB/s, 1636 x 3775 x 2025 100 us, with k-major operands at
+// 10, 205 x 4096 x 25472 160; 16-bit k-major operands come in pieces of
 // 32*R bytes, which costs 2.6, 1.6 and 1.1 times that), or the tile's products where those take longer (fp32: 0.45 TFLOP/s
 // of a CU's 0.61 on the largest tile while a CU has one, 0.36 with more, 0.3 on the others).  With S > 1 another launch and the partial products written and
 // read.
@@ -464,7 +480,7 @@ double stream_us(const LinArgs& a, int esz, int R, int S, double entries) {
   const double rate = esz == 2 ? 4e6 : R < 4 ? 0.3e6 : rounds > 1.5 ? 0.36e6 : 0.45e6, flops = 2 * tm * tn * k;
   const double per = bytes / 65e3 > flops / rate ? bytes / 65e3 : flops / rate;
   const double few = (double)(a.M < a.N ? a.M : a.N) * a.K * esz, all = (double)(a.M + a.N) * a.K * esz;
-  const double missed = few > 2e6 && all > 8e6 ? tiles * bytes / 8e6 : 0;
+  const double missed = few > 2e6 && all > 8e6 ? tiles * bytes / (esz == 2 && (a.xt || a.wt) ? 10e6 : 8e6) : 0;
   // 16-bit: the next tile's first loads and the last one's output do not overlap (tiles of 64 rows: 72 of k into 960 x 7552, 7 rounds
   // 38 us, 752 into 1906 x 2088, 3.9: 32; of 32: 327 into 310 x 4245, 5.2: 17.6, 262 k-major into 2545 x 866, 8.8: 27)
   // (two workgroups of 32 rows share a CU: two rounds are one)
@@ -554,7 +570,7 @@ int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, unsigned e
     case 1: rc = launch_type<F16>(a, p.R, stream, entries); break;
     default: rc = launch_type<BF16>(a, p.R, stream, entries);
   }
-  return rc != 0 || p.S == 1 ? rc : launch_merge_type(a, dtype, stream);
+  return rc != 0 || p.S == 1 ? rc : launch_linear_merge(a, dtype, stream);
 }
 
 double stream_pair_cost(const LinArgs& gw, const LinArgs& gi, int dtype) {
@@ -575,7 +591,7 @@ int launch_stream_pair(const LinArgs& gw_, const LinArgs& gi, int dtype, hipStre
     case 1: rc = launch_pair_type<F16>(gw, gi, p.gw.R, p.gi.R, stream); break;
     default: rc = launch_pair_type<BF16>(gw, gi, p.gw.R, p.gi.R, stream);
   }
-  return rc != 0 || p.gw.S == 1 ? rc : launch_merge_type(gw, dtype, stream);
+  return rc != 0 || p.gw.S == 1 ? rc : launch_linear_merge(gw, dtype, stream);
 }
 
 }  // namespace ttsdpa
