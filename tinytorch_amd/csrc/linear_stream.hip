@@ -411,6 +411,14 @@ __global__ __launch_bounds__(64 * Shape<R>::W, Shape<R>::W / 4) void linear_stre
   stream_tile<TR, XT, WT, R, R, Shape<R>::W, Shape<R>::P, XT && WT>(a, smem, blockIdx.x, blockIdx.y);  // row sums: a weight's gradient
 }
 
+// Few rows of x (one tile of them) against a weight that 32 x 32 tiles cut into more pieces than there are CUs, up to twice as many: tiles
+// of as many of its rows as make one round (few_rows_tile).
+template <typename TR, int MB, int NB, int P>
+__global__ __launch_bounds__(512, 2) void linear_rows_kernel(LinArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  stream_tile<TR, false, false, MB, NB, 8, P, false>(a, smem, blockIdx.x, blockIdx.y);
+}
+
 // Both products of a linear layer's backward in one launch, the first `split` workgroups those of the weight's gradient
 // (grad^T . x, with grad's column sums: the bias's gradient), the others those of the input's (grad . w).
 template <typename TR, int RW, int RI>
@@ -436,6 +444,18 @@ int launch_kernel(const LinArgs& a, hipStream_t stream, unsigned entries) {
   if (granted != hipSuccess) return (int)granted;
   if (blocks_of<R>(a) > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
   hipLaunchKernelGGL((linear_stream_kernel<TR, XT, WT, R>), dim3((unsigned)blocks_of<R>(a), entries), dim3(64 * Shape<R>::W), lds, stream, a);
+  return (int)hipGetLastError();
+}
+
+template <typename TR, int MB, int NB, int P>
+int launch_rows_kernel(const LinArgs& a, hipStream_t stream) {
+  static hipError_t state[kMaxDevices];
+  static bool done[kMaxDevices];
+  constexpr int lds = StreamLds<TR, false, false, MB, NB, 8>::BYTES;
+  const hipError_t granted = grant_dynamic_lds((const void*)linear_rows_kernel<TR, MB, NB, P>, lds, state, done);
+  if (granted != hipSuccess) return (int)granted;
+  const long long tiles = ((a.M + 16 * MB - 1) / (16 * MB)) * ((a.N + 16 * NB - 1) / (16 * NB));
+  hipLaunchKernelGGL((linear_rows_kernel<TR, MB, NB, P>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), lds, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -510,6 +530,23 @@ StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split
   return best;
 }
 
+// The tile for up to 32 rows of x where 32 x 32 ones would be taken, 16-bit x . w^T.  Those of one to two rounds of the 256 CUs last as
+// long as two; us on them and so:
+//   24 rows x 8704, K 1024, 2048, 4096    8.4, 14.2, 23.5 -> 7.1, 11.6, 18.6 (32 x 48)      x 12288    9.0, 14.8, 23.7 -> 8.1, 14.0, 19.2
+//   6 x 8448                              7.9, 13.0, 21.1 -> 6.7 (32 x 48), 10.5 (16 x 64), 17.3 (16 x 16: four times the workgroups, no remainder)
+//   6 x 16384                             9.1, 15.1, 32.0 -> 9.3, 14.9 (16 x 64), 26.1 (16 x 16)
+// and a weight of more than 200 MB, with up to eight rows of up to 4096, streams best in small pieces: 1 x 28672 x 4096 43.2 -> 40.7
+// (16 x 28672 x 4096 and 3 x 20480 x 3072 the same; 6 x 28544 x 5120 55.6 in 32 x 32 tiles, 59.1 so).
+enum class Tile { Square, Square16, Rows32x48, Rows16x64 };
+Tile few_rows_tile(const LinArgs& a) {
+  if (a.xt || a.wt || a.M > 32) return Tile::Square;
+  const long long tiles = (a.N + 31) / 32;
+  if (a.M <= 8 && a.K <= 4096 && a.N * a.K > 100000000ll) return Tile::Square16;
+  if (tiles <= 256 || tiles > 512) return Tile::Square;
+  if (a.M > 16 || a.K < 1536) return a.N <= 48 * 256 ? Tile::Rows32x48 : Tile::Square;
+  return a.K <= 2560 ? Tile::Rows16x64 : Tile::Square16;
+}
+
 size_t part_bytes(const LinArgs& a, int S) { return S > 1 ? (size_t)S * (size_t)(a.M * a.N + a.M) * sizeof(float) : 0; }
 
 template <typename TR, bool XT, bool WT>
@@ -565,6 +602,14 @@ int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, unsigned e
   a.splits = p.S;
   a.part = p.S > 1 ? (float*)scratch : nullptr;
   int rc;
+  if (dtype != 0 && entries == 1 && p.S == 1 && p.R == 2) {
+    switch (few_rows_tile(a)) {
+      case Tile::Square16: p.R = 1; break;
+      case Tile::Rows32x48: return dtype == 1 ? launch_rows_kernel<F16, 2, 3, 2>(a, stream) : launch_rows_kernel<BF16, 2, 3, 2>(a, stream);
+      case Tile::Rows16x64: return dtype == 1 ? launch_rows_kernel<F16, 1, 4, 4>(a, stream) : launch_rows_kernel<BF16, 1, 4, 4>(a, stream);
+      default: break;
+    }
+  }
   switch (dtype) {
     case 0: rc = launch_type<F32>(a, p.R, stream, entries); break;
     case 1: rc = launch_type<F16>(a, p.R, stream, entries); break;
