@@ -1284,7 +1284,9 @@ static PackPlan plan_pack(const LinArgs& g, int dtype, size_t room) {
   double us = whole;
   p.S = 1;
   const bool may = p.copies == 0 || g.xt || g.wt;  // (copies for the alignment's sake alone: 804 x 1983 x 5329 64 us, undivided 57)
-  for (int S = 2; may && S <= 16 && p.kpad / bk >= 4 * S; S++) {
+  // fp32: no fewer shares than the streaming kernel has chains of sums, where that takes the call
+  const int least = dtype == TTSDPA_F32 && stream_takes(g, dtype) ? stream_chains(g, dtype, true) : 2;
+  for (int S = least > 2 ? least : 2; may && S <= 16 && p.kpad / bk >= 4 * S; S++) {
     const double divided = divided_cost(nt, dtype, S);
     if (divided < us && divided < 0.9 * whole && p.copies + divided_bytes(nt, S) <= room) us = divided, p.S = S;
   }
@@ -1337,7 +1339,8 @@ static Way choose(const LinArgs& g, int dtype, bool scratch, size_t scratch_byte
   // divided; those of the ways that read contraction-major operands as they lie by more, the input gradient of 231 x 19072 x 3072 17
   // us shorter so than divided with its copies)
   const double us_packed = p->S == 1 ? p->us : p->copies > 0 ? p->us / 0.75 : p->us / 0.9;
-  if (p->ok && p->bytes <= (scratch ? scratch_bytes : 0)) take(Way::Packed, us_packed);
+  const bool behind = p->S > 1 && dtype == TTSDPA_F32 && stream_takes(g, dtype) && stream_call_cost(g, dtype, scratch) < us_packed;
+  if (p->ok && p->bytes <= (scratch ? scratch_bytes : 0) && !behind) take(Way::Packed, us_packed);
   if (in_place_ok(g, dtype)) take(Way::InPlace, in_place_cost(g, dtype, 1));
   if (stream_takes(g, dtype)) take(Way::Stream, stream_cost(g, dtype, 1, scratch));
   if (us) *us = best;

@@ -26,6 +26,8 @@ struct LinArgs {
 // linear_stream.hip: products whose wavefronts divide the contraction among themselves, for any alignment of the operands.
 bool stream_takes(const LinArgs& a, int dtype);                             // sizes and strides are in its range
 double stream_cost(const LinArgs& a, int dtype, unsigned entries, bool may_split);  // estimated microseconds
+double stream_call_cost(const LinArgs& a, int dtype, bool may_split);        // of the plan that a call has
+int stream_chains(const LinArgs& a, int dtype, bool may_split);              // chains that it adds a contraction up in
 size_t stream_scratch(const LinArgs& a, int dtype);                         // bytes that let it divide the contraction
 int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, unsigned entries = 1, void* scratch = nullptr, size_t scratch_bytes = 0);
 // out = bias + the sums of a.splits shares of a product in a.part (and the row sums)

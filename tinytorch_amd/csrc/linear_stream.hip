@@ -490,10 +490,13 @@ namespace {
 //   measured / this: 1000^3 on 16, 32, 64: 25 / 26, 12 / 13, 9.5 / 9.4; 24 x 2048 x 5632: 7.4 / 9, 10.5 / 13, 19 / 21;
 //   64 x 4096 x 4096: 17 / 20, 11 / 12, 21 / 22; fp32 1000^3: 42 / 43, 30 / 32, 25 / 24; both k-major, 500 x 500 x 8192:
 //   88 / 90, 29 / 29, 40 / 40
-double stream_us(const LinArgs& a, int esz, int R, int S, double entries) {
+// whole: fp32's largest tiles are bound by the matrix cores, so that the 8 of 264 that make a second round take as long as it (62 x 16896
+// x 3072, 138 us; 130 x 3072 x 8448 182, divided among more 95).  A call's own plan goes by this; which way a product runs goes by the other, for the tiled kernels, which
+// would then be taken for more calls, add up the contraction in fewer and longer chains.
+double stream_us(const LinArgs& a, int esz, int R, int S, double entries, bool whole = false) {
   const double tm = 16 * R, tn = 16 * R;
   const double tiles = (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)) * entries * S;
-  const double rounds = tiles > 256 ? tiles / 256 : 1;
+  const double rounds = tiles <= 256 ? 1 : whole && R == 4 ? ceil(tiles / 256) : tiles / 256;
   const double narrow = esz == 4 ? 1 : R == 1 ? 2.6 : R == 2 ? 1.6 : 1.1;
   const double k = (double)a.K / S;
   const double bytes = ((a.M < tm ? a.M : tm) * (a.xt ? narrow : 1) + (a.N < tn ? a.N : tn) * (a.wt ? narrow : 1)) * k * esz;
@@ -515,7 +518,8 @@ struct StreamPlan {
   int R, S;
   double us;
 };
-StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split, int least = 1, int most = 4) {
+constexpr int wavefronts(int R) { return R == 4 ? Shape<4>::W : Shape<1>::W; }  // of a workgroup
+StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split, int least = 1, int most = 4, bool whole = false, int chains = 0) {
   StreamPlan best{0, 1, 0};
   for (int R = least; R <= most; R *= 2) {
     if ((a.xt && a.M < 16 * R) || (a.wt && a.N < 16 * R)) break;
@@ -523,7 +527,8 @@ StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split
     // 5120 x 34944: 87 us in 64-row tiles, 69 in 32-row ones; 12 x 4096 x 28672 54 and 45)
     if (R == 4 && R > least && (a.M <= 32 || a.N <= 32)) break;
     for (int S = 1; S <= 32 && (S == 1 || (may_split && a.K >= 512 * S)); S *= 2) {
-      const double t = stream_us(a, esz, R, S, entries);
+      if (wavefronts(R) * S < chains) continue;
+      const double t = stream_us(a, esz, R, S, entries, whole);
       if (!best.R || t < best.us) best = {R, S, t};
     }
   }
@@ -592,13 +597,27 @@ double stream_cost(const LinArgs& a, int dtype, unsigned entries, bool may_split
   return plan_stream(a, dtype == 0 ? 4 : 2, entries, may_split).us;
 }
 
-size_t stream_scratch(const LinArgs& a, int dtype) { return part_bytes(a, plan_stream(a, dtype == 0 ? 4 : 2, 1, true).S); }
+// The plan of a call.  fp32: by whole rounds, with as many chains of sums (wavefronts and shares) as the other estimate's plan has.
+static StreamPlan plan_call(const LinArgs& a, int dtype, double entries, bool may_split) {
+  const StreamPlan p = plan_stream(a, dtype == 0 ? 4 : 2, entries, may_split);
+  if (dtype != 0 || p.R == 0) return p;
+  const StreamPlan q = plan_stream(a, 4, entries, may_split, 1, 4, true, wavefronts(p.R) * p.S);
+  return q.us < 0.9 * stream_us(a, 4, p.R, p.S, entries, true) ? q : p;
+}
+
+int stream_chains(const LinArgs& a, int dtype, bool may_split) {
+  const StreamPlan p = plan_stream(a, dtype == 0 ? 4 : 2, 1, may_split);
+  return p.R == 0 ? 1 : wavefronts(p.R) * p.S;
+}
+
+size_t stream_scratch(const LinArgs& a, int dtype) { return part_bytes(a, plan_call(a, dtype, 1, true).S); }
+
+double stream_call_cost(const LinArgs& a, int dtype, bool may_split) { return plan_call(a, dtype, 1, may_split).us; }
 
 int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, unsigned entries, void* scratch, size_t scratch_bytes) {
-  const int esz = dtype == 0 ? 4 : 2;
   LinArgs a = args;
-  StreamPlan p = plan_stream(a, esz, entries, entries == 1 && scratch);
-  if (part_bytes(a, p.S) > scratch_bytes) p = plan_stream(a, esz, entries, false);
+  StreamPlan p = plan_call(a, dtype, entries, entries == 1 && scratch);
+  if (part_bytes(a, p.S) > scratch_bytes) p = plan_call(a, dtype, entries, false);
   a.splits = p.S;
   a.part = p.S > 1 ? (float*)scratch : nullptr;
   int rc;
