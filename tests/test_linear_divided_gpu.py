@@ -77,3 +77,13 @@ def test_less_scratch(dtype, M, N, K):
         assert rc == 0
         _close(out, x, w.t(), b)
         assert (ws[size:] == 77).all()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(256, 4096, 2048), (257, 4096, 2048), (448, 4672, 1537), (512, 4096, 1536), (513, 4096, 1536), (220, 4608, 3072),
+                                   (865, 1024, 3328), (64, 16448, 1600)])
+def test_rounds_of_64_rows(dtype, M, N, K):
+    """Both sides of 256 and 512 tiles of 64 x 64, where the streaming kernel's estimate counts in whole rounds."""
+    print("rounds", dtype, M, N, K, flush=True)
+    x, w, b = _operands(M, N, K, dtype)
+    _close(tt.linear(x, w, b), x, w.t(), b)
