@@ -1,5 +1,6 @@
 """Gradients of a layer over few rows, against float64: a contraction of one to eight units of the streaming kernel's tiles, whose
-workgroups take as many tiles as leave no wavefront idle (csrc/linear_stream.hip, tile_wavefronts), with a last workgroup not full of them."""
+workgroups take as many tiles as leave no wavefront idle (csrc/linear_stream.hip, tile_wavefronts), with a last workgroup not full of
+them; and large tiles of short contractions."""
 import pytest
 import torch
 
@@ -33,6 +34,20 @@ def test_backward(dtype, M, N, K):
     _close(gx, go, w)
     _close(gw, go.t(), x)
     _close(gb.view(1, N), torch.ones(1, M, device="cuda"), go)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(1, 128, 4096), (16, 2048, 2048), (17, 4001, 1111), (31, 3000, 1000), (32, 2047, 1536), (33, 2048, 2048), (64, 1023, 2049),
+                                   (65, 2048, 1024), (128, 1536, 1535), (129, 3071, 257), (255, 1500, 2000), (256, 2048, 1536), (257, 2048, 1536)])
+def test_large_tiles(dtype, M, N, K):
+    """128 x 128 tiles of the weight's gradient (csrc/linear_outer.hip): units of the contraction and remainders of them, last tiles that
+    are moved back, unaligned rows; both with the bias's gradient and through matmul with a bias."""
+    test_backward(dtype, M, N, K)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b, c = (torch.randn(*s, generator=g, device="cuda").to(_TYPES[dtype]) for s in ((M, N + 1), (M, K + 3), (K,)))
+    got = tt.matmul(a[:, 1:], b[:, 3:], True, False, c)
+    one = torch.ones(N, 1, device="cuda", dtype=a.dtype)
+    _close(got, torch.cat((a[:, 1:].t(), one), 1), torch.cat((b[:, 3:], c.view(1, K)), 0))
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16"])

@@ -1326,7 +1326,7 @@ static int launch_packed(const LinArgs& g, const PackPlan& p, int dtype, hipStre
 }
 
 // How a product runs: the cheapest by estimate of the ways that take it.
-enum class Way { General, Stream, InPlace, Packed };
+enum class Way { General, Stream, InPlace, Packed, Outer };
 
 static Way choose(const LinArgs& g, int dtype, bool scratch, size_t scratch_bytes, PackPlan* p, double* us = nullptr) {
   Way way = Way::General;
@@ -1343,6 +1343,8 @@ static Way choose(const LinArgs& g, int dtype, bool scratch, size_t scratch_byte
   if (p->ok && p->bytes <= (scratch ? scratch_bytes : 0) && !behind) take(Way::Packed, us_packed);
   if (in_place_ok(g, dtype)) take(Way::InPlace, in_place_cost(g, dtype, 1));
   if (stream_takes(g, dtype)) take(Way::Stream, stream_cost(g, dtype, 1, scratch));
+  // (row sums, where wanted, come with the product, as on the streaming kernel; the tiled kernels need launches for them)
+  if (outer_takes(g, dtype)) take(Way::Outer, outer_cost(g, dtype) - (g.rowsum && way != Way::Stream ? 4 : 0));
   if (us) *us = best;
   return way;
 }
@@ -1353,6 +1355,7 @@ static int product(const LinArgs& g, int dtype, void* scratch, size_t scratch_by
     case Way::Stream: return launch_stream(g, dtype, s, 1, scratch, scratch_bytes);
     case Way::InPlace: return dtype == TTSDPA_F16 ? launch_mfma_t<F16>(g, s) : launch_mfma_t<BF16>(g, s);
     case Way::Packed: return launch_packed(g, p, dtype, s, (char*)scratch, nullptr);
+    case Way::Outer: return launch_outer(g, dtype, s);
     default: break;
   }
   switch (dtype) {
@@ -1534,6 +1537,7 @@ int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w,
   hipStream_t s = (hipStream_t)stream;
   // grad_w [N,K] = grad^T . x, grad_x [M,K] = grad . w
   LinArgs gw{grad, x, nullptr, grad_w, N, K, M, ldg, ldx, K, 1, 1};
+  gw.rowsum = grad_b;
   const LinArgs gi{grad, w, nullptr, grad_x, M, K, N, ldg, ldw, K, 0, 1};
   // Small layers: both products, and the column sums with the weight's, in one launch.  Where the two would be launched
   // on the streaming kernel anyway and the launches saved (5 us, the column sums' among them) are worth more than what
@@ -1543,18 +1547,17 @@ int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w,
   double us_w, us_i;
   const Way way_w = choose(gw, dtype, true, workspace_bytes, &pw, &us_w);
   const Way way_i = choose(gi, dtype, true, workspace_bytes, &pi, &us_i);
-  const bool pair = way_w == Way::Stream && way_i == Way::Stream;
+  // Against a launch each, the weight's gradient in 128 x 128 tiles: 16-bit 20 x 1024 x 1024 5.1 us in one, 7.5 in two, 20 x 2048 x 1024 9.7
+  // and 8.4; 120 rows 7.8 and 8.7, 12.9 and 12.3.
+  const bool pair = (way_w == Way::Stream || way_w == Way::Outer) && way_i == Way::Stream && stream_takes(gw, dtype);
   if ((pair || (dtype == TTSDPA_F32 && stream_takes(gw, dtype) && stream_takes(gi, dtype))) &&
-      stream_pair_cost(gw, gi, dtype) < us_w + us_i + 5 && stream_pair_scratch(gw, gi, dtype) <= workspace_bytes) {
-    gw.rowsum = grad_b;
+      stream_pair_cost(gw, gi, dtype) < (way_w == Way::Outer ? outer_cost(gw, dtype) - 0.2 : us_w + 5) + us_i && stream_pair_scratch(gw, gi, dtype) <= workspace_bytes)
     return launch_stream_pair(gw, gi, dtype, s, workspace);
-  }
   int rc = product(gi, dtype, workspace, workspace_bytes, s);
   if (rc != 0) return rc;
-  if (way_w == Way::Stream) {
-    gw.rowsum = grad_b;
-    return launch_stream(gw, dtype, s, 1, workspace, workspace_bytes);
-  }
+  if (way_w == Way::Stream) return launch_stream(gw, dtype, s, 1, workspace, workspace_bytes);
+  if (way_w == Way::Outer) return launch_outer(gw, dtype, s);
+  gw.rowsum = nullptr;  // a launch of its own, or with the copies
   const long long sums = pack_ranges(pw.kpad);
   if (way_w == Way::Packed && pw.x && workspace_bytes >= pw.bytes + (size_t)sums * (size_t)N * sizeof(float)) {
     // the column sums come with the transposed copy

@@ -37,4 +37,9 @@ double stream_pair_cost(const LinArgs& gw, const LinArgs& gi, int dtype);
 size_t stream_pair_scratch(const LinArgs& gw, const LinArgs& gi, int dtype);
 int launch_stream_pair(const LinArgs& gw, const LinArgs& gi, int dtype, hipStream_t stream, void* scratch);
 
+// linear_outer.hip: both operands k-major, a short contraction (and the row sums, as above).
+bool outer_takes(const LinArgs& a, int dtype);
+double outer_cost(const LinArgs& a, int dtype);  // estimated microseconds
+int launch_outer(const LinArgs& a, int dtype, hipStream_t stream);
+
 }  // namespace ttsdpa

@@ -515,6 +515,19 @@ int launch_pair_kernel(const LinArgs& gw, const LinArgs& gi, hipStream_t stream)
 
 namespace {
 
+constexpr int wavefronts(int R) { return R == 4 ? Shape<4>::W : Shape<1>::W; }  // of a workgroup
+
+// Wavefronts that share a tile where a workgroup has several tiles; 0: it has one.
+int waves_of_tile(const LinArgs& a, int esz, int R) {
+  const int G = a.xt && a.wt ? tile_wavefronts(a.K, 128 / esz, wavefronts(R), 1) : wavefronts(R);
+  return G < wavefronts(R) ? G : 0;
+}
+
+double rounds_of(const LinArgs& a, long long tm, long long tn, double entries) {
+  const double tiles = (double)((a.M + tm - 1) / tm) * (double)((a.N + tn - 1) / tn) * entries;
+  return tiles > 256 ? tiles / 256 : 1;
+}
+
 // Microseconds of a product on tiles of 16*R rows of x by 16*R of w, its contraction divided among S workgroups per tile, from
 // measurements (MI355X, 16-bit unless said): 3 us of launch, latency and the meeting of the partial sums (2 more on the
 // largest tile: a wavefront's sums are 16 KB); then, for each round of the 256 CUs, half a microsecond and the operands of
@@ -530,7 +543,16 @@ namespace {
 // whole: fp32's largest tiles are bound by the matrix cores, so that the 8 of 264 that make a second round take as long as it (62 x 16896
 // x 3072, 138 us; 130 x 3072 x 8448 182, divided among more 95).  A call's own plan goes by this; which way a product runs goes by the other, for the tiled kernels, which
 // would then be taken for more calls, add up the contraction in fewer and longer chains.
+// Several tiles to a workgroup (a weight's gradient of few rows), 16-bit: by its wavefronts with work, 1024 of which run at once; tiles of
+// 16, 32 and 64 rows take 0.9, 1.9 and 7.7 us for each 1024 more: in 32 x 32 tiles 20 x 2048 x 2048 9.8 us, 120 x 2048 x 1024
+// 6.9, 250 x 2048 x 1024 12.9, 24 x 11264 x 2048 42.  fp32, whose products bound it, takes what the rounds say but for single units on the largest
+// tiles: 20 x 9000 x 3000 66 us in 32 x 32 ones, 98 in 64 x 64.
 double stream_us(const LinArgs& a, int esz, int R, int S, double entries, bool whole = false) {
+  if (esz == 4 && R == 4 && S == 1 && waves_of_tile(a, esz, R) == 1) return 5 + 3 * rounds_of(a, 64, 64, entries);
+  if (const int G = esz == 2 && S == 1 ? waves_of_tile(a, esz, R) : 0) {
+    const double tiles = (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)) * entries, waves = tiles * G / 1024;
+    return 3 + (waves <= 1 && R < 4 ? 0.5 : waves * (R == 1 ? 0.9 : R == 2 ? 1.9 : 7.7));
+  }
   const double tm = 16 * R, tn = 16 * R;
   const double tiles = (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)) * entries * S;
   // (16-bit x . w^T, 64 rows: a second round lasts as long as the first, however few its tiles: 720 x 1536 x 1536, 288 tiles, 18.2 us, on the
@@ -557,7 +579,6 @@ struct StreamPlan {
   int R, S;
   double us;
 };
-constexpr int wavefronts(int R) { return R == 4 ? Shape<4>::W : Shape<1>::W; }  // of a workgroup
 StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split, int least = 1, int most = 4, bool whole = false, int chains = 0) {
   StreamPlan best{0, 1, 0};
   for (int R = least; R <= most; R *= 2) {
@@ -618,7 +639,13 @@ struct PairPlan {
   StreamPlan gw, gi;
 };
 PairPlan plan_pair(const LinArgs& gw, const LinArgs& gi, int esz) {
-  const PairPlan few{plan_stream(gw, esz, 1, true, 1, 2), plan_stream(gi, esz, 1, false, 1, 2)};
+  PairPlan few{plan_stream(gw, esz, 1, true, 1, 2), plan_stream(gi, esz, 1, false, 1, 2)};
+  // one round of the CUs with both, if that only takes larger tiles of the other (16-bit; 60 x 777 x 1001 10.8 -> 6.1, 60 x 512 x 1024 6.5 -> 5.0)
+  auto tiles = [](const LinArgs& a, int R) { return ((a.M + 16 * R - 1) / (16 * R)) * ((a.N + 16 * R - 1) / (16 * R)); };
+  if (const int G = esz == 2 && few.gw.S == 1 && few.gw.R == 2 && few.gi.R == 1 && gi.N >= 32 ? waves_of_tile(gw, esz, 2) : 0) {
+    const long long blocks = tiles(gw, 2) * G / wavefronts(2);
+    if (blocks + tiles(gi, 1) > 256 && blocks + tiles(gi, 2) <= 256) few.gi = {2, 1, stream_us(gi, esz, 2, 1, 1)};
+  }
   const PairPlan many{plan_stream(gw, esz, 1, true, 4, 4), plan_stream(gi, esz, 1, false, 4, 4)};
   return many.gw.R && many.gi.R && many.gw.us + many.gi.us < few.gw.us + few.gi.us ? many : few;
 }
