@@ -32,6 +32,17 @@ def test_few_rows(M, N, K, dtype):
     _close(tt.linear(x, w, b), x, w.t(), b)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 4100, 2048), (16, 8192, 2048), (5, 8191, 1001), (17, 8193, 1024), (32, 11264, 2048), (31, 16384, 1000), (20, 16385, 1024), (33, 11200, 4096),
+    (48, 17281, 3000), (40, 11201, 4095), (49, 11200, 4096)])
+def test_few_rows_contraction_major(M, N, K, dtype):
+    print("rows, k-major", M, N, K, dtype, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w, b = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((M, K), (K, N), (N,)))
+    _close(tt.matmul(x, w, False, False, b), x, w, b)
+
+
 def test_views():
     """Rows that begin at odd elements, and an output with rows longer than the product's."""
     g = torch.Generator(device="cuda").manual_seed(3)

@@ -439,11 +439,11 @@ __global__ __launch_bounds__(64 * Shape<R>::W, Shape<R>::W / 4) void linear_stre
 }
 
 // Few rows of x (one tile of them) against a weight that 32 x 32 tiles cut into more pieces than there are CUs, up to twice as many: tiles
-// of as many of its rows as make one round (few_rows_tile).
-template <typename TR, int MB, int NB, int P>
+// of as many of its rows as make one round; and rows that leave much of a square tile idle (few_rows_tile).
+template <typename TR, bool WT, int MB, int NB, int P>
 __global__ __launch_bounds__(512, 2) void linear_rows_kernel(LinArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  stream_tile<TR, false, false, MB, NB, 8, P, false>(a, smem, blockIdx.x, blockIdx.y);
+  stream_tile<TR, false, WT, MB, NB, 8, P, false>(a, smem, blockIdx.x, blockIdx.y);
 }
 
 // Both products of a linear layer's backward in one launch, the first `split` workgroups those of the weight's gradient
@@ -482,15 +482,15 @@ int launch_kernel(const LinArgs& a, hipStream_t stream, unsigned entries) {
   return (int)hipGetLastError();
 }
 
-template <typename TR, int MB, int NB, int P>
+template <typename TR, bool WT, int MB, int NB, int P>
 int launch_rows_kernel(const LinArgs& a, hipStream_t stream) {
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
-  constexpr int lds = StreamLds<TR, false, false, MB, NB, 8>::BYTES;
-  const hipError_t granted = grant_dynamic_lds((const void*)linear_rows_kernel<TR, MB, NB, P>, lds, state, done);
+  constexpr int lds = StreamLds<TR, false, WT, MB, NB, 8>::BYTES;
+  const hipError_t granted = grant_dynamic_lds((const void*)linear_rows_kernel<TR, WT, MB, NB, P>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
   const long long tiles = ((a.M + 16 * MB - 1) / (16 * MB)) * ((a.N + 16 * NB - 1) / (16 * NB));
-  hipLaunchKernelGGL((linear_rows_kernel<TR, MB, NB, P>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), lds, stream, a);
+  hipLaunchKernelGGL((linear_rows_kernel<TR, WT, MB, NB, P>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(512), lds, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -602,14 +602,34 @@ StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split
 //   6 x 16384                             9.1, 15.1, 32.0 -> 9.3, 14.9 (16 x 64), 26.1 (16 x 16)
 // and a weight of more than 200 MB, with up to eight rows of up to 4096, streams best in small pieces: 1 x 28672 x 4096 43.2 -> 40.7
 // (16 x 28672 x 4096 and 3 x 20480 x 3072 the same; 6 x 28544 x 5120 55.6 in 32 x 32 tiles, 59.1 so).
-enum class Tile { Square, Square16, Rows32x48, Rows16x64 };
-Tile few_rows_tile(const LinArgs& a) {
-  if (a.xt || a.wt || a.M > 32) return Tile::Square;
+// k-major w (a layer's input gradient), us, rows x columns x contraction: up to 16 rows in 16 x 32 tiles, 16 x 8192 x 2048 12.6 -> 11.0 (5 x 7839 x 731
+// 6.4 -> 7.2, hence the least contraction); 32 x 64 ones where 32 x 32 make one to two rounds, 30 x 11264 x 4096 38 -> 28, 8 x 10880 x 5760 40
+// -> 30; 33 to 48 rows in 48 x 64 tiles of eight wavefronts instead of 64 x 64 of four, 42 x 11200 x 4096 28 -> 23, 37 x 17280 x 5120 58 -> 54.
+enum class Tile { Square, Square16, Rows32x48, Rows16x64, Rows16x32, Rows32x64, Rows48x64 };
+Tile few_rows_tile(const LinArgs& a, int R) {
+  if (a.wt && !a.xt) {
+    if (R == 4) return a.M > 32 && a.M <= 48 ? Tile::Rows48x64 : Tile::Square;
+    const long long pieces = (a.N + 31) / 32;
+    if (a.M > 32 || pieces > 512) return Tile::Square;
+    return pieces > 256 ? Tile::Rows32x64 : a.M <= 16 && a.K >= 1200 ? Tile::Rows16x32 : Tile::Square;
+  }
+  if (a.xt || a.M > 32 || R != 2) return Tile::Square;
   const long long tiles = (a.N + 31) / 32;
   if (a.M <= 8 && a.K <= 4096 && a.N * a.K > 100000000ll) return Tile::Square16;
   if (tiles <= 256 || tiles > 512) return Tile::Square;
   if (a.M > 16 || a.K < 1536) return a.N <= 48 * 256 ? Tile::Rows32x48 : Tile::Square;
   return a.K <= 2560 ? Tile::Rows16x64 : Tile::Square16;
+}
+
+template <typename TR>
+int launch_rows_type(const LinArgs& a, Tile tile, hipStream_t stream) {
+  switch (tile) {
+    case Tile::Rows32x48: return launch_rows_kernel<TR, false, 2, 3, 2>(a, stream);
+    case Tile::Rows16x64: return launch_rows_kernel<TR, false, 1, 4, 4>(a, stream);
+    case Tile::Rows16x32: return launch_rows_kernel<TR, true, 1, 2, 4>(a, stream);
+    case Tile::Rows32x64: return launch_rows_kernel<TR, true, 2, 4, 2>(a, stream);
+    default: return launch_rows_kernel<TR, true, 3, 4, 1>(a, stream);
+  }
 }
 
 size_t part_bytes(const LinArgs& a, int S) { return S > 1 ? (size_t)S * (size_t)(a.M * a.N + a.M) * sizeof(float) : 0; }
@@ -687,13 +707,10 @@ int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, unsigned e
   a.splits = p.S;
   a.part = p.S > 1 ? (float*)scratch : nullptr;
   int rc;
-  if (dtype != 0 && entries == 1 && p.S == 1 && p.R == 2) {
-    switch (few_rows_tile(a)) {
-      case Tile::Square16: p.R = 1; break;
-      case Tile::Rows32x48: return dtype == 1 ? launch_rows_kernel<F16, 2, 3, 2>(a, stream) : launch_rows_kernel<BF16, 2, 3, 2>(a, stream);
-      case Tile::Rows16x64: return dtype == 1 ? launch_rows_kernel<F16, 1, 4, 4>(a, stream) : launch_rows_kernel<BF16, 1, 4, 4>(a, stream);
-      default: break;
-    }
+  if (dtype != 0 && entries == 1 && p.S == 1 && p.R >= 2) {
+    const Tile tile = few_rows_tile(a, p.R);
+    if (tile == Tile::Square16) p.R = 1;
+    else if (tile != Tile::Square) return dtype == 1 ? launch_rows_type<F16>(a, tile, stream) : launch_rows_type<BF16>(a, tile, stream);
   }
   switch (dtype) {
     case 0: rc = launch_type<F32>(a, p.R, stream, entries); break;
