@@ -1147,14 +1147,14 @@ double mixed_tiles_cost(const LinArgs& a) {
   return 9 * rounds + 6 + large_cold(a) + a.K / 64.0 * (1.5 * rounds + 0.62 + 0.24 * (2 * left) / kCusOfXcd);
 }
 
-// 128 x 128 tiles whose contraction is divided among S workgroups each, one to a CU at most: a launch more, and the shares' fp32 sums
+// 128 x 128 tiles whose contraction is divided among S workgroups each, one to a CU (of an XCD's: 826 x 1536 x 4160, 84 tiles in 3 shares, 33
+// on some, 36 us; 28 by this) at most: a launch more, and the shares' fp32 sums
 // written and read at 5 TB/s.  What leaves most CUs idle otherwise, or goes to the streaming kernel, which takes in the operands of
 // smaller tiles: 288 x 2048 x 6592, 48 tiles, 34.7 there -> 22.9 in 5 shares; 200 x 4096 x 14336, 64, 74 -> 48 in 4; 720 x 1536 x 4736,
-// 72, 43 -> 24 in 3 (2: 26.6; 5, more than a round: 27.3); fp32 119 x 3072 x 9152, 24, 108 -> 75 in 10.  (Four wavefronts of 64 x 64
-// instead of eight of 64 x 32, fewer LDS reads: 3 to 8 % slower in every such call.)
+// 72, 43 -> 24 in 3 (2: 26.6; 5, more than a round: 27.3).  fp32: only what the streaming kernel does not take, contraction-major
+// operands of fewer than 16 rows.  (Four wavefronts of 64 x 64 instead of eight of 64 x 32, fewer LDS reads: 3 to 8 % slower in every
+// such call.)
 double divided_cost(const LinArgs& a, int dtype, int S) {
-  const long long tiles = ((a.M + 127) / 128) * ((a.N + 127) / 128);
-  if ((tiles + 7) / 8 * S > kCusOfXcd) return 1e30;  // (an XCD's: 826 x 1536 x 4160, 84 tiles in 3 shares, 33 on some, 36 us; 28 by this)
   const double esz = dtype == TTSDPA_F32 ? 4 : 2, sums = 5.5 + 8.0 * S * a.M * a.N / 5e6;
   LinArgs share = a;
   share.K = (long long)((a.K * esz / 128 + S - 1) / S) * (long long)(128 / esz);
@@ -1211,16 +1211,16 @@ double in_place_cost(const LinArgs& a, int dtype, unsigned entries) {
   return (1.3 + (1.7 + a.K / 64.0 * 0.6) * (tiles > 256 ? tiles / 256 : 1)) * (a.wt && !a.xt ? 1.1 : 1);
 }
 
-bool streams(const LinArgs& a, int dtype, unsigned entries = 1, bool may_split = false) {
-  return stream_takes(a, dtype) && stream_cost(a, dtype, entries, may_split) < in_place_cost(a, dtype, entries);
+bool streams(const LinArgs& a, int dtype, unsigned entries) {
+  return stream_takes(a, dtype) && plan_stream(a, dtype, entries, false).us < in_place_cost(a, dtype, entries);
 }
 
 // What the tiled kernels' layout does not allow: the streaming kernel, or where one of its operands is too narrow for that (a
 // k-major operand of fewer than 16 rows, an empty contraction) the vector ALUs.
 template <typename T>
-int launch_general_linear(const LinArgs& a, hipStream_t stream, unsigned entries = 1, void* scratch = nullptr, size_t scratch_bytes = 0) {
+int launch_general_linear(const LinArgs& a, hipStream_t stream, unsigned entries = 1) {
   const int dtype = sizeof(T) == 4 ? TTSDPA_F32 : std::is_same<T, _Float16>::value ? TTSDPA_F16 : TTSDPA_BF16;
-  if (stream_takes(a, dtype)) return launch_stream(a, dtype, stream, entries, scratch, scratch_bytes);
+  if (stream_takes(a, dtype)) return launch_stream(a, dtype, stream, plan_stream(a, dtype, entries, false), entries);
   dim3 grid((unsigned)((a.N + 63) / 64), (unsigned)((a.M + 63) / 64), entries);
   hipLaunchKernelGGL((linear_general_kernel<T>), grid, dim3(256), 0, stream, a);
   return (int)hipGetLastError();
@@ -1264,7 +1264,8 @@ struct PackPlan {
   double us;
 };
 
-static PackPlan plan_pack(const LinArgs& g, int dtype, size_t room) {
+// beat: what another way of the product is estimated to take.
+static PackPlan plan_pack(const LinArgs& g, int dtype, size_t room, double beat) {
   const long long esz = dtype == TTSDPA_F32 ? 4 : 2, bk = ROWB / esz, kpc = 16 / esz;
   PackPlan p{};
   p.kpad = (g.K + bk - 1) / bk * bk;
@@ -1283,10 +1284,13 @@ static PackPlan plan_pack(const LinArgs& g, int dtype, size_t room) {
   const double whole = nt_cost(nt, dtype, 1);
   double us = whole;
   p.S = 1;
-  const bool may = p.copies == 0 || g.xt || g.wt;  // (copies for the alignment's sake alone: 804 x 1983 x 5329 64 us, undivided 57)
-  // fp32: no fewer shares than the streaming kernel has chains of sums, where that takes the call
-  const int least = dtype == TTSDPA_F32 && stream_takes(g, dtype) ? stream_chains(g, dtype, true) : 2;
-  for (int S = least > 2 ? least : 2; may && S <= 16 && p.kpad / bk >= 4 * S; S++) {
+  // (copies for the alignment's sake alone: 804 x 1983 x 5329 64 us, undivided 57; fp32 that the streaming kernel takes: that adds a
+  // contraction up in more and shorter chains)
+  // And not worth a look where two shares' sums and the operands read once take longer than another way, at choose()'s margin.
+  const bool may = (p.copies == 0 || g.xt || g.wt) && !(dtype == TTSDPA_F32 && stream_takes(g, dtype)) &&
+                   7.7 + (double)esz * (double)(g.M + g.N) * (double)g.K / 4.2e6 + 16.0 * (double)g.M * (double)g.N / 5e6 < 0.9 * beat;
+  const long long most = kCusOfXcd / ((((g.M + 127) / 128) * ((g.N + 127) / 128) + 7) / 8);  // a workgroup to a CU
+  for (int S = 2; may && S <= 16 && S <= most && p.kpad / bk >= 4 * S; S++) {
     const double divided = divided_cost(nt, dtype, S);
     if (divided < us && divided < 0.9 * whole && p.copies + divided_bytes(nt, S) <= room) us = divided, p.S = S;
   }
@@ -1327,42 +1331,50 @@ static int launch_packed(const LinArgs& g, const PackPlan& p, int dtype, hipStre
 
 // How a product runs: the cheapest by estimate of the ways that take it.
 enum class Way { General, Stream, InPlace, Packed, Outer };
-
-static Way choose(const LinArgs& g, int dtype, bool scratch, size_t scratch_bytes, PackPlan* p, double* us = nullptr) {
+struct Choice {
   Way way = Way::General;
-  double best = 1e30;
+  double us = 1e30;
+  PackPlan pack;
+  StreamPlan stream{0, 1, 0};  // where the kernel takes the product
+};
+
+static Choice choose(const LinArgs& g, int dtype, bool scratch, size_t scratch_bytes) {
+  Choice c;
   auto take = [&](Way w, double cost) {
-    if (cost < best) way = w, best = cost;
+    if (cost < c.us) c.way = w, c.us = cost;
   };
-  *p = plan_pack(g, dtype, scratch ? scratch_bytes : 0);
+  if (in_place_ok(g, dtype)) take(Way::InPlace, in_place_cost(g, dtype, 1));
+  if (stream_takes(g, dtype)) {
+    c.stream = plan_stream(g, dtype, 1, scratch);
+    take(Way::Stream, c.stream.us);
+  }
+  c.pack = plan_pack(g, dtype, scratch ? scratch_bytes : 0, c.us);
   // (margins for divided contractions: the estimates miss by a tenth, 719 x 1024 x 2688 15.8 us on the streaming kernel, 16.8
   // divided; those of the ways that read contraction-major operands as they lie by more, the input gradient of 231 x 19072 x 3072 17
   // us shorter so than divided with its copies)
-  const double us_packed = p->S == 1 ? p->us : p->copies > 0 ? p->us / 0.75 : p->us / 0.9;
-  const bool behind = p->S > 1 && dtype == TTSDPA_F32 && stream_takes(g, dtype) && stream_call_cost(g, dtype, scratch) < us_packed;
-  if (p->ok && p->bytes <= (scratch ? scratch_bytes : 0) && !behind) take(Way::Packed, us_packed);
-  if (in_place_ok(g, dtype)) take(Way::InPlace, in_place_cost(g, dtype, 1));
-  if (stream_takes(g, dtype)) take(Way::Stream, stream_cost(g, dtype, 1, scratch));
+  if (c.pack.ok && c.pack.bytes <= (scratch ? scratch_bytes : 0)) take(Way::Packed, c.pack.S == 1 ? c.pack.us : c.pack.us / (c.pack.copies > 0 ? 0.75 : 0.9));
   // (row sums, where wanted, come with the product, as on the streaming kernel; the tiled kernels need launches for them)
-  if (outer_takes(g, dtype)) take(Way::Outer, outer_cost(g, dtype) - (g.rowsum && way != Way::Stream ? 4 : 0));
-  if (us) *us = best;
-  return way;
+  if (outer_takes(g, dtype)) take(Way::Outer, outer_cost(g, dtype) - (g.rowsum && c.way != Way::Stream ? 4 : 0));
+  return c;
 }
 
-static int product(const LinArgs& g, int dtype, void* scratch, size_t scratch_bytes, hipStream_t s) {
-  PackPlan p;
-  switch (choose(g, dtype, scratch, scratch_bytes, &p)) {
-    case Way::Stream: return launch_stream(g, dtype, s, 1, scratch, scratch_bytes);
+static int run(const LinArgs& g, const Choice& c, int dtype, void* scratch, size_t scratch_bytes, hipStream_t s) {
+  switch (c.way) {
+    case Way::Stream: return launch_stream(g, dtype, s, c.stream, 1, scratch, scratch_bytes);
     case Way::InPlace: return dtype == TTSDPA_F16 ? launch_mfma_t<F16>(g, s) : launch_mfma_t<BF16>(g, s);
-    case Way::Packed: return launch_packed(g, p, dtype, s, (char*)scratch, nullptr);
+    case Way::Packed: return launch_packed(g, c.pack, dtype, s, (char*)scratch, nullptr);
     case Way::Outer: return launch_outer(g, dtype, s);
     default: break;
   }
   switch (dtype) {
-    case TTSDPA_F32: return launch_general_linear<float>(g, s, 1, scratch, scratch_bytes);
-    case TTSDPA_F16: return launch_general_linear<_Float16>(g, s, 1, scratch, scratch_bytes);
-    default: return launch_general_linear<__bf16>(g, s, 1, scratch, scratch_bytes);
+    case TTSDPA_F32: return launch_general_linear<float>(g, s);
+    case TTSDPA_F16: return launch_general_linear<_Float16>(g, s);
+    default: return launch_general_linear<__bf16>(g, s);
   }
+}
+
+static int product(const LinArgs& g, int dtype, void* scratch, size_t scratch_bytes, hipStream_t s) {
+  return run(g, choose(g, dtype, scratch, scratch_bytes), dtype, scratch, scratch_bytes, s);
 }
 
 // x . w^T + bias; scratch (optional): lets the streaming kernel divide the contraction among workgroups, and holds copies
@@ -1388,22 +1400,25 @@ static LinArgs flags_args(int64_t M, int64_t N, int64_t K, int trans_a, int tran
 // Room for the copies (where the product would be made on copies, or operands lie contraction-major) or the parts of a divided contraction.
 // The latter also where aligned operands would go another way: sizes do not say how rows are aligned, and unaligned ones go to the
 // streaming kernel.  (Some MB at most: only products of few tiles are divided.)
+static size_t scratch_of(const LinArgs& g, const Choice& c, int dtype, size_t behind_copies = 0) {
+  const size_t parts = stream_part_bytes(g, plan_stream_call(g, dtype, 1, true, c.stream));
+  const size_t packed = c.way == Way::Packed ? c.pack.bytes + behind_copies : 0;
+  return packed > parts ? packed : parts;
+}
+
 size_t ttlinear_matmul_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const LinArgs g = flags_args(M, N, K, trans_a, trans_b);
-  PackPlan p;
-  const bool packed = choose(g, dtype, true, ~(size_t)0, &p) == Way::Packed;
-  const size_t parts = stream_scratch(g, dtype);
-  return packed && p.bytes > parts ? p.bytes : parts;
+  return scratch_of(g, choose(g, dtype, true, ~(size_t)0), dtype);
 }
 
 int ttlinear_matmul_tiles(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
   if ((dtype != TTSDPA_F16 && dtype != TTSDPA_BF16) || M <= 0 || N <= 0 || K <= 0) return TTLINEAR_TILES_OTHER;
   LinArgs g = flags_args(M, N, K, trans_a, trans_b);
-  PackPlan p;
-  if (choose(g, dtype, true, ~(size_t)0, &p) != Way::Packed) return TTLINEAR_TILES_OTHER;
-  g.K = p.kpad, g.xt = g.wt = 0;
-  return p.S > 1 ? TTLINEAR_TILES_128x128 : tiles_of(g);
+  const Choice c = choose(g, dtype, true, ~(size_t)0);
+  if (c.way != Way::Packed) return TTLINEAR_TILES_OTHER;
+  g.K = c.pack.kpad, g.xt = g.wt = 0;
+  return c.pack.S > 1 ? TTLINEAR_TILES_128x128 : tiles_of(g);
 }
 
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
@@ -1508,18 +1523,45 @@ size_t ttlinear_backward_least_workspace_bytes(int dtype, int64_t M, int64_t N) 
   return M <= 0 || N <= 0 ? 0 : (size_t)colsum_ranges(M, N, dtype) * (size_t)N * sizeof(float);
 }
 
+// The two products of a layer's backward, and whether they run in one launch.
+struct BackwardPlan {
+  Choice w, i;
+  PairPlan pair;
+  bool paired, joint;  // pair is filled in; and is the way
+};
+
+// Small layers: both products, and the column sums with the weight's, in one launch.  Where the two would be launched
+// on the streaming kernel anyway and the launches saved (5 us, the column sums' among them) are worth more than what
+// the common workgroup size may cost (64 x 784 x 500 fp32: 10 us in two launches and 5 for the column sums); fp32, which
+// the products bound, wherever it is estimated faster (1501 x 1999 x 2501: 322 us, on tiles with copies 381).
+static BackwardPlan plan_backward(const LinArgs& gw, const LinArgs& gi, int dtype, size_t workspace_bytes) {
+  BackwardPlan p;
+  p.w = choose(gw, dtype, true, workspace_bytes);
+  p.i = choose(gi, dtype, true, workspace_bytes);
+  const bool takes = stream_takes(gw, dtype) && stream_takes(gi, dtype);
+  const bool streams = (p.w.way == Way::Stream || p.w.way == Way::Outer) && p.i.way == Way::Stream;
+  p.joint = p.paired = takes && (streams || dtype == TTSDPA_F32);
+  if (!p.paired) return p;
+  p.pair = plan_stream_pair(gw, gi, dtype);
+  // Against a launch each, the weight's gradient in 128 x 128 tiles: 16-bit 20 x 1024 x 1024 5.1 us in one, 7.5 in two, 20 x 2048 x 1024 9.7
+  // and 8.4; 120 rows 7.8 and 8.7, 12.9 and 12.3.
+  p.joint = p.pair.us() < (p.w.way == Way::Outer ? outer_cost(gw, dtype) - 0.2 : p.w.us + 5) + p.i.us && stream_part_bytes(gw, p.pair.gw) <= workspace_bytes;
+  return p;
+}
+
 size_t ttlinear_backward_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const LinArgs g = flags_args(N, K, M, 1, 0);
-  const size_t gi = ttlinear_matmul_workspace_bytes(dtype, M, K, N, 0, 0);
-  size_t gw = ttlinear_matmul_workspace_bytes(dtype, N, K, M, 1, 0);
-  PackPlan p;
-  if (choose(g, dtype, true, ~(size_t)0, &p) == Way::Packed) gw = p.bytes + (size_t)pack_ranges(p.kpad) * (size_t)N * sizeof(float);
-  const size_t gb = ttlinear_backward_least_workspace_bytes(dtype, M, N);
-  const size_t pair = stream_pair_scratch(g, flags_args(M, K, N, 0, 0), dtype);
-  size_t most = gi > gw ? gi : gw;  // one after the other on the same scratch
-  if (pair > most) most = pair;
-  return most > gb ? most : gb;
+  const LinArgs gw = flags_args(N, K, M, 1, 0), gi = flags_args(M, K, N, 0, 0);
+  const BackwardPlan p = plan_backward(gw, gi, dtype, ~(size_t)0);
+  // one after the other on the same scratch; sizes do not say how rows are aligned (above)
+  const size_t of_i = scratch_of(gi, p.i, dtype), of_w = scratch_of(gw, p.w, dtype, (size_t)pack_ranges(p.w.pack.kpad) * (size_t)N * sizeof(float));
+  const size_t of_b = ttlinear_backward_least_workspace_bytes(dtype, M, N);
+  size_t most = of_i > of_w ? of_i : of_w;
+  if (stream_takes(gw, dtype) && stream_takes(gi, dtype)) {
+    const size_t of_pair = stream_part_bytes(gw, (p.paired ? p.pair : plan_stream_pair(gw, gi, dtype)).gw);
+    if (of_pair > most) most = of_pair;
+  }
+  return most > of_b ? most : of_b;
 }
 
 int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w, void* grad_x, void* grad_w, void* grad_b, int64_t M,
@@ -1539,27 +1581,15 @@ int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w,
   LinArgs gw{grad, x, nullptr, grad_w, N, K, M, ldg, ldx, K, 1, 1};
   gw.rowsum = grad_b;
   const LinArgs gi{grad, w, nullptr, grad_x, M, K, N, ldg, ldw, K, 0, 1};
-  // Small layers: both products, and the column sums with the weight's, in one launch.  Where the two would be launched
-  // on the streaming kernel anyway and the launches saved (5 us, the column sums' among them) are worth more than what
-  // the common workgroup size may cost (64 x 784 x 500 fp32: 10 us in two launches and 5 for the column sums); fp32, which
-  // the products bound, wherever it is estimated faster (1501 x 1999 x 2501: 322 us, on tiles with copies 381).
-  PackPlan pw, pi;
-  double us_w, us_i;
-  const Way way_w = choose(gw, dtype, true, workspace_bytes, &pw, &us_w);
-  const Way way_i = choose(gi, dtype, true, workspace_bytes, &pi, &us_i);
-  // Against a launch each, the weight's gradient in 128 x 128 tiles: 16-bit 20 x 1024 x 1024 5.1 us in one, 7.5 in two, 20 x 2048 x 1024 9.7
-  // and 8.4; 120 rows 7.8 and 8.7, 12.9 and 12.3.
-  const bool pair = (way_w == Way::Stream || way_w == Way::Outer) && way_i == Way::Stream && stream_takes(gw, dtype);
-  if ((pair || (dtype == TTSDPA_F32 && stream_takes(gw, dtype) && stream_takes(gi, dtype))) &&
-      stream_pair_cost(gw, gi, dtype) < (way_w == Way::Outer ? outer_cost(gw, dtype) - 0.2 : us_w + 5) + us_i && stream_pair_scratch(gw, gi, dtype) <= workspace_bytes)
-    return launch_stream_pair(gw, gi, dtype, s, workspace);
-  int rc = product(gi, dtype, workspace, workspace_bytes, s);
+  const BackwardPlan p = plan_backward(gw, gi, dtype, workspace_bytes);
+  if (p.joint) return launch_stream_pair(gw, gi, dtype, s, p.pair, workspace);
+  int rc = run(gi, p.i, dtype, workspace, workspace_bytes, s);
   if (rc != 0) return rc;
-  if (way_w == Way::Stream) return launch_stream(gw, dtype, s, 1, workspace, workspace_bytes);
-  if (way_w == Way::Outer) return launch_outer(gw, dtype, s);
+  if (p.w.way == Way::Stream || p.w.way == Way::Outer) return run(gw, p.w, dtype, workspace, workspace_bytes, s);
   gw.rowsum = nullptr;  // a launch of its own, or with the copies
+  const PackPlan& pw = p.w.pack;
   const long long sums = pack_ranges(pw.kpad);
-  if (way_w == Way::Packed && pw.x && workspace_bytes >= pw.bytes + (size_t)sums * (size_t)N * sizeof(float)) {
+  if (p.w.way == Way::Packed && pw.x && workspace_bytes >= pw.bytes + (size_t)sums * (size_t)N * sizeof(float)) {
     // the column sums come with the transposed copy
     float* part = grad_b ? (float*)((char*)workspace + pw.bytes) : nullptr;
     rc = launch_packed(gw, pw, dtype, s, (char*)workspace, part);
@@ -1570,7 +1600,7 @@ int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w,
       default: return launch_colsum_merge<__bf16>(part, (int)sums, N, grad_b, s);
     }
   }
-  rc = product(gw, dtype, workspace, workspace_bytes, s);
+  rc = run(gw, p.w, dtype, workspace, workspace_bytes, s);
   if (rc != 0 || !grad_b) return rc;
   const int ranges = colsum_ranges(M, N, dtype);
   switch (dtype) {

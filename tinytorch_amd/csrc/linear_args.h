@@ -21,21 +21,31 @@ struct LinArgs {
   void* rowsum = nullptr;
   int splits = 1;
   float* part = nullptr;
+  int tile_waves = 0;  // linear_stream.hip: wavefronts that share a tile (0: a workgroup's all)
 };
 
 // linear_stream.hip: products whose wavefronts divide the contraction among themselves, for any alignment of the operands.
-bool stream_takes(const LinArgs& a, int dtype);                             // sizes and strides are in its range
-double stream_cost(const LinArgs& a, int dtype, unsigned entries, bool may_split);  // estimated microseconds
-double stream_call_cost(const LinArgs& a, int dtype, bool may_split);        // of the plan that a call has
-int stream_chains(const LinArgs& a, int dtype, bool may_split);              // chains that it adds a contraction up in
-size_t stream_scratch(const LinArgs& a, int dtype);                         // bytes that let it divide the contraction
-int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, unsigned entries = 1, void* scratch = nullptr, size_t scratch_bytes = 0);
+// A plan: tiles of 16 R rows of either operand, the contraction divided among S workgroups, estimated microseconds.  Planning is host
+// time of every call, so that a call's plan is made once and handed on.
+struct StreamPlan {
+  int R, S;
+  double us;
+};
+bool stream_takes(const LinArgs& a, int dtype);                                               // sizes and strides are in its range
+StreamPlan plan_stream(const LinArgs& a, int dtype, unsigned entries, bool may_split);        // the estimate that chooses a product's way
+StreamPlan plan_stream_call(const LinArgs& a, int dtype, unsigned entries, bool may_split, const StreamPlan& p);  // what a call with that plan runs on
+size_t stream_part_bytes(const LinArgs& a, const StreamPlan& call);                           // scratch for its shares
+int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, const StreamPlan& p, unsigned entries = 1, void* scratch = nullptr,
+                  size_t scratch_bytes = 0);
 // out = bias + the sums of a.splits shares of a product in a.part (and the row sums)
 int launch_linear_merge(const LinArgs& a, int dtype, hipStream_t stream);
 // a layer's two backward products in one launch (gw: both operands k-major; gi: w k-major), each in the kernel's range
-double stream_pair_cost(const LinArgs& gw, const LinArgs& gi, int dtype);
-size_t stream_pair_scratch(const LinArgs& gw, const LinArgs& gi, int dtype);
-int launch_stream_pair(const LinArgs& gw, const LinArgs& gi, int dtype, hipStream_t stream, void* scratch);
+struct PairPlan {
+  StreamPlan gw, gi;
+  double us() const { return gw.us + gi.us - 3; }  // one launch
+};
+PairPlan plan_stream_pair(const LinArgs& gw, const LinArgs& gi, int dtype);
+int launch_stream_pair(const LinArgs& gw, const LinArgs& gi, int dtype, hipStream_t stream, const PairPlan& p, void* scratch);
 
 // linear_outer.hip: both operands k-major, a short contraction (and the row sums, as above).
 bool outer_takes(const LinArgs& a, int dtype);

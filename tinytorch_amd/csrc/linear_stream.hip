@@ -575,11 +575,7 @@ double stream_us(const LinArgs& a, int esz, int R, int S, double entries, bool w
 
 // The cheapest tile (rows in blocks of 16: 1, 2 or 4, as far as a k-major operand has them; R = 0: none) and, when the caller
 // has scratch for partial products, division of the contraction (no less than 512 of it per workgroup).
-struct StreamPlan {
-  int R, S;
-  double us;
-};
-StreamPlan plan_stream(const LinArgs& a, int esz, double entries, bool may_split, int least = 1, int most = 4, bool whole = false, int chains = 0) {
+StreamPlan plan_tiles(const LinArgs& a, int esz, double entries, bool may_split, int least = 1, int most = 4, bool whole = false, int chains = 0) {
   StreamPlan best{0, 1, 0};
   for (int R = least; R <= most; R *= 2) {
     if ((a.xt && a.M < 16 * R) || (a.wt && a.N < 16 * R)) break;
@@ -655,55 +651,44 @@ int launch_pair_type(const LinArgs& gw, const LinArgs& gi, int RW, int RI, hipSt
 }
 
 // Tiles of the two products of a layer's backward: one workgroup size, so both of 64 rows or both of fewer.
-struct PairPlan {
-  StreamPlan gw, gi;
-};
 PairPlan plan_pair(const LinArgs& gw, const LinArgs& gi, int esz) {
-  PairPlan few{plan_stream(gw, esz, 1, true, 1, 2), plan_stream(gi, esz, 1, false, 1, 2)};
+  PairPlan few{plan_tiles(gw, esz, 1, true, 1, 2), plan_tiles(gi, esz, 1, false, 1, 2)};
   // one round of the CUs with both, if that only takes larger tiles of the other (16-bit; 60 x 777 x 1001 10.8 -> 6.1, 60 x 512 x 1024 6.5 -> 5.0)
   auto tiles = [](const LinArgs& a, int R) { return ((a.M + 16 * R - 1) / (16 * R)) * ((a.N + 16 * R - 1) / (16 * R)); };
   if (const int G = esz == 2 && few.gw.S == 1 && few.gw.R == 2 && few.gi.R == 1 && gi.N >= 32 ? waves_of_tile(gw, esz, 2) : 0) {
     const long long blocks = tiles(gw, 2) * G / wavefronts(2);
     if (blocks + tiles(gi, 1) > 256 && blocks + tiles(gi, 2) <= 256) few.gi = {2, 1, stream_us(gi, esz, 2, 1, 1)};
   }
-  const PairPlan many{plan_stream(gw, esz, 1, true, 4, 4), plan_stream(gi, esz, 1, false, 4, 4)};
+  const PairPlan many{plan_tiles(gw, esz, 1, true, 4, 4), plan_tiles(gi, esz, 1, false, 4, 4)};
   return many.gw.R && many.gi.R && many.gw.us + many.gi.us < few.gw.us + few.gi.us ? many : few;
 }
 
 }  // namespace
 
 bool stream_takes(const LinArgs& a, int dtype) {
-  // a tile's rows and a unit's k-rows are addressed with 32-bit byte offsets
+  // a tile's rows and a unit's k-rows are addressed with 32-bit byte offsets; a k-major operand has a tile's rows at least
   const long long ld_max = 1ll << 24;
-  if (a.K < 1 || a.K > 0x3fffffffLL || a.ldx >= ld_max || a.ldw >= ld_max) return false;
-  return plan_stream(a, dtype == 0 ? 4 : 2, 1, false).R > 0;
+  return a.K >= 1 && a.K <= 0x3fffffffLL && a.ldx < ld_max && a.ldw < ld_max && (!a.xt || a.M >= 16) && (!a.wt || a.N >= 16);
 }
 
-double stream_cost(const LinArgs& a, int dtype, unsigned entries, bool may_split) {
-  return plan_stream(a, dtype == 0 ? 4 : 2, entries, may_split).us;
+StreamPlan plan_stream(const LinArgs& a, int dtype, unsigned entries, bool may_split) {
+  return plan_tiles(a, dtype == 0 ? 4 : 2, entries, may_split);
 }
 
-// The plan of a call.  fp32: by whole rounds, with as many chains of sums (wavefronts and shares) as the other estimate's plan has.
-static StreamPlan plan_call(const LinArgs& a, int dtype, double entries, bool may_split) {
-  const StreamPlan p = plan_stream(a, dtype == 0 ? 4 : 2, entries, may_split);
-  if (dtype != 0 || p.R == 0) return p;
-  const StreamPlan q = plan_stream(a, 4, entries, may_split, 1, 4, true, wavefronts(p.R) * p.S);
+// fp32: by whole rounds, which count on the largest tiles, with as many chains of sums (wavefronts and shares) as the other estimate's
+// plan has.
+StreamPlan plan_stream_call(const LinArgs& a, int dtype, unsigned entries, bool may_split, const StreamPlan& p) {
+  if (dtype != 0 || p.R != 4) return p;
+  const StreamPlan q = plan_tiles(a, 4, entries, may_split, 1, 4, true, wavefronts(p.R) * p.S);
   return q.us < 0.9 * stream_us(a, 4, p.R, p.S, entries, true) ? q : p;
 }
 
-int stream_chains(const LinArgs& a, int dtype, bool may_split) {
-  const StreamPlan p = plan_stream(a, dtype == 0 ? 4 : 2, 1, may_split);
-  return p.R == 0 ? 1 : wavefronts(p.R) * p.S;
-}
+size_t stream_part_bytes(const LinArgs& a, const StreamPlan& call) { return part_bytes(a, call.S); }
 
-size_t stream_scratch(const LinArgs& a, int dtype) { return part_bytes(a, plan_call(a, dtype, 1, true).S); }
-
-double stream_call_cost(const LinArgs& a, int dtype, bool may_split) { return plan_call(a, dtype, 1, may_split).us; }
-
-int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, unsigned entries, void* scratch, size_t scratch_bytes) {
+int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, const StreamPlan& chosen, unsigned entries, void* scratch, size_t scratch_bytes) {
   LinArgs a = args;
-  StreamPlan p = plan_call(a, dtype, entries, entries == 1 && scratch);
-  if (part_bytes(a, p.S) > scratch_bytes) p = plan_call(a, dtype, entries, false);
+  StreamPlan p = plan_stream_call(a, dtype, entries, entries == 1 && scratch, chosen);
+  if (part_bytes(a, p.S) > scratch_bytes) p = plan_stream_call(a, dtype, entries, false, plan_stream(a, dtype, entries, false));
   a.splits = p.S;
   a.part = p.S > 1 ? (float*)scratch : nullptr;
   int rc;
@@ -720,15 +705,9 @@ int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, unsigned e
   return rc != 0 || p.S == 1 ? rc : launch_linear_merge(a, dtype, stream);
 }
 
-double stream_pair_cost(const LinArgs& gw, const LinArgs& gi, int dtype) {
-  const PairPlan p = plan_pair(gw, gi, dtype == 0 ? 4 : 2);
-  return p.gw.us + p.gi.us - 3;  // one launch
-}
+PairPlan plan_stream_pair(const LinArgs& gw, const LinArgs& gi, int dtype) { return plan_pair(gw, gi, dtype == 0 ? 4 : 2); }
 
-size_t stream_pair_scratch(const LinArgs& gw, const LinArgs& gi, int dtype) { return part_bytes(gw, plan_pair(gw, gi, dtype == 0 ? 4 : 2).gw.S); }
-
-int launch_stream_pair(const LinArgs& gw_, const LinArgs& gi, int dtype, hipStream_t stream, void* scratch) {
-  const PairPlan p = plan_pair(gw_, gi, dtype == 0 ? 4 : 2);
+int launch_stream_pair(const LinArgs& gw_, const LinArgs& gi, int dtype, hipStream_t stream, const PairPlan& p, void* scratch) {
   LinArgs gw = gw_;
   gw.splits = p.gw.S;
   gw.part = p.gw.S > 1 ? (float*)scratch : nullptr;
