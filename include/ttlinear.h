@@ -70,6 +70,26 @@ enum ttlinear_tiles {
 };
 int ttlinear_matmul_tiles(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b);
 
+/* The kernel and the tiles that a product of dense, aligned operands runs on, given its workspace.  Launches nothing and needs no GPU;
+ * as above the answer may change with the library. */
+enum ttlinear_way {
+  TTLINEAR_WAY_GENERAL = 0,  /* the vector ALUs */
+  TTLINEAR_WAY_STREAM = 1,   /* small tiles whose wavefronts divide the contraction among themselves */
+  TTLINEAR_WAY_IN_PLACE = 2, /* large tiles of contraction-major operands read as they lie */
+  TTLINEAR_WAY_TILED = 3,    /* large tiles, of copies where the layout asks for them */
+  TTLINEAR_WAY_OUTER = 4     /* 128 x 128 tiles of a short contraction, both operands contraction-major */
+};
+typedef struct ttlinear_kernel_info {
+  int32_t way;                      /* enum ttlinear_way */
+  int32_t tile_rows, tile_columns;  /* STREAM: rows and columns of the output in a tile; 0 otherwise (ttlinear_matmul_tiles) */
+  int32_t tiles_per_workgroup;      /* STREAM; 1 otherwise */
+  int32_t shares;                   /* workgroups among which a tile's contraction is divided */
+} ttlinear_kernel_info;
+int ttlinear_matmul_kernel(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, ttlinear_kernel_info* info);
+/* The same of ttlinear_backward's two products, and whether they run in one launch. */
+int ttlinear_backward_kernels(int dtype, int64_t M, int64_t N, int64_t K, int with_bias, ttlinear_kernel_info* of_weight,
+                              ttlinear_kernel_info* of_input, int* one_launch);
+
 /* FuncLinear::backward (reference src/Function/FuncNNLayer.h:20-33) in one call: from the upstream gradient grad [M,N], the
  * forward's x [M,K] and w [N,K] (row strides ldg, ldx, ldw in elements)
  *   grad_x [M,K] = grad . w,   grad_w [N,K] = grad^T . x,   grad_b [N] = column sums of grad (NULL: not wanted),

@@ -137,6 +137,17 @@ void ttsdpa_params_init(ttsdpa_params* p, int dtype, int B, int Hq, int Hkv, int
  * needs no GPU.  Plays the role of the reference's shape checks before a device op (src/Operation/OpLinalg.cpp:62-89). */
 int ttsdpa_plan(const ttsdpa_params* p, int* route);
 
+/* Within a route, the kernels for short sequences that *p (ttsdpa_backward_kernel: with that much scratch) runs on, or OTHER: the
+ * route's kernels for long ones.  Estimates decide: the answer may change with the library.  Launches nothing and needs no GPU. */
+enum ttsdpa_kernel_kind {
+  TTSDPA_KERNEL_OTHER = 0,
+  TTSDPA_KERNEL_SHORT = 1,       /* 16 rows or keys a workgroup; backward: dq, then dk and dv */
+  TTSDPA_KERNEL_SHORT_JOINT = 2, /* backward: all gradients in one launch */
+  TTSDPA_KERNEL_HEADS_16 = 3,    /* with an attnMask, a head's K and V in LDS at once; 16 rows a wavefront */
+  TTSDPA_KERNEL_HEADS_32 = 4     /* 32 */
+};
+int ttsdpa_kernel(const ttsdpa_params* p, int* kind);
+
 /* Bytes of device scratch ttsdpa_forward / ttsdpa_decode use for *p (0 for calls that need none): the split-KV
  * partials of the decode route, and of calls on the prefill route whose keys are divided among workgroups (few query
  * rows, or few 256-row tiles of head_dim 128 against many keys).
@@ -206,6 +217,7 @@ void ttsdpa_backward_params_init(ttsdpa_backward_params* p, int dtype, int B, in
  * arithmetic: the vector-ALU kernels, or, where only an attnMask keeps the call off the MFMA route, the kernels on the fp32
  * matrix cores; TTSDPA_ROUTE_NONE = nothing to compute.  Needs no GPU. */
 int ttsdpa_backward_plan(const ttsdpa_backward_params* p, int* route);
+int ttsdpa_backward_kernel(const ttsdpa_backward_params* p, size_t workspace_bytes, int* kind);
 size_t ttsdpa_backward_workspace_bytes(const ttsdpa_backward_params* p);
 int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t workspace_bytes, void* stream);
 

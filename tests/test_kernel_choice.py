@@ -1,0 +1,67 @@
+"""Which kernel a call runs on, as the host's queries answer without a GPU: sizes on either side of the rules that choose among kernels,
+with what both sides measured on an MI355X."""
+import ctypes
+
+import pytest
+
+from tinytorch_amd import _capi
+
+F32, F16, BF16 = _capi.F32, _capi.F16, _capi.BF16
+FAKE = 1 << 30  # an aligned address that nothing reads
+
+
+def attention(dtype, B, Hq, Hkv, L, S, D, causal=False, mask=None, back=False):
+    """Parameter block of dense tensors; mask: "keys" (Bool, one row for all), "bool" or "add" (a row each)."""
+    bp = _capi.BackwardParams()
+    _capi.lib().ttsdpa_backward_params_init(ctypes.byref(bp), dtype, B, Hq, Hkv, L, S, D)
+    p = bp.fwd
+    p.q = p.k = p.v = p.out = bp.dout = bp.dq = bp.dk = bp.dv = FAKE
+    p.causal = _capi.CAUSAL_TOP_LEFT if causal else _capi.CAUSAL_NONE
+    if mask:
+        p.mask, p.mask_kind = FAKE, _capi.MASK_ADD if mask == "add" else _capi.MASK_BOOL
+        for i, x in enumerate((S, 0, 0, 1) if mask == "keys" else (0, L * S, S, 1)):
+            p.mask_stride[i] = x
+    return bp if back else p
+
+
+def test_queries_refuse_what_the_calls_refuse():
+    L = _capi.lib()
+    i, k = _capi.LinearKernelInfo(), ctypes.c_int(-1)
+    assert L.ttlinear_matmul_kernel(7, 64, 64, 64, 0, 1, ctypes.byref(i)) == _capi.ERR_DTYPE
+    assert L.ttlinear_matmul_kernel(BF16, 64, 0, 64, 0, 1, ctypes.byref(i)) == _capi.ERR_SHAPE
+    assert L.ttlinear_matmul_kernel(BF16, 64, 64, 64, 0, 1, None) == _capi.ERR_NULL
+    assert L.ttlinear_backward_kernels(BF16, 64, 64, 64, 1, ctypes.byref(i), None, ctypes.byref(k)) == _capi.ERR_NULL
+    p = attention(BF16, 1, 3, 2, 64, 64, 64)
+    assert L.ttsdpa_kernel(ctypes.byref(p), ctypes.byref(k)) == _capi.ERR_SHAPE
+    bp = attention(BF16, 1, 2, 2, 64, 64, 64, back=True)
+    bp.dout = None
+    assert L.ttsdpa_backward_kernel(ctypes.byref(bp), 1 << 20, ctypes.byref(k)) == _capi.ERR_NULL
+
+
+def test_ways_of_products():
+    assert _capi.linear_kernel(BF16, 8192, 6144, 4096)[0] == "tiled"
+    assert _capi.linear_kernel(BF16, 24, 2048, 5632) == ("stream", (16, 16), 1, 1)
+    assert _capi.linear_kernel(BF16, 288, 2048, 6592) == ("tiled", (0, 0), 1, 5)     # divided
+    assert _capi.linear_kernel(F16, 4096, 4096, 16, 1, 0)[0] == "outer"              # a weight's gradient of 16 rows
+    assert _capi.linear_kernel(F32, 6, 768, 28672, 1, 1) == ("tiled", (0, 0), 1, 16)  # too narrow for the streaming kernel
+    assert _capi.linear_kernel(F32, 3, 50, 70, 1, 0)[0] in ("general", "tiled")
+    assert _capi.linear_backward_kernels(BF16, 8192, 4096, 4096)[2] is False
+    assert _capi.linear_backward_kernels(F32, 64, 500, 784)[2] is True
+
+
+# (the calls that the streaming kernel takes in fp32 add a contraction up in its chains)
+@pytest.mark.parametrize("M,N,K", [(119, 3072, 9152), (300, 1021, 3200), (64, 512, 16384)])
+def test_fp32_products_are_not_divided_into_longer_chains(M, N, K):
+    assert _capi.linear_kernel(F32, M, N, K)[0] == "stream"
+
+
+def test_kernels_of_short_sequences():
+    assert _capi.kernel(attention(F32, 1, 4, 4, 128, 128, 64, causal=True)) == "short"
+    assert _capi.backward_kernel(attention(F32, 1, 4, 4, 128, 128, 64, causal=True, back=True)) == "short_joint"
+    assert _capi.kernel(attention(BF16, 2, 32, 8, 4096, 4096, 128, causal=True)) == "other"
+    assert _capi.kernel(attention(F16, 16, 12, 12, 197, 197, 64, mask="keys")) == "heads_32"
+    assert _capi.kernel(attention(F16, 1, 8, 8, 94, 94, 64, mask="keys")) == "heads_16"
+    assert _capi.kernel(attention(F32, 1, 8, 8, 94, 94, 64, mask="keys")) == "other"
+    bp = attention(BF16, 3, 4, 2, 100, 160, 64, causal=True, back=True)  # less scratch than asked for: the other kernels
+    need = _capi.lib().ttsdpa_backward_workspace_bytes(ctypes.byref(bp))
+    assert _capi.backward_kernel(bp) != "other" and _capi.backward_kernel(bp, need - 1) == "other"

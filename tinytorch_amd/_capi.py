@@ -20,17 +20,19 @@ STATIC_SCRATCH_BYTES = 2 << 20
 
 EXPORTS = [
     "ttsdpa_abi_version", "ttsdpa_status_string", "ttsdpa_params_init", "ttsdpa_plan", "ttsdpa_workspace_bytes",
-    "ttsdpa_forward", "ttsdpa_prefill", "ttsdpa_decode", "ttsdpa_decode_static", "ttsdpa_general",
+    "ttsdpa_kernel", "ttsdpa_backward_kernel", "ttsdpa_forward", "ttsdpa_prefill", "ttsdpa_decode", "ttsdpa_decode_static", "ttsdpa_general",
     "ttsdpa_kv_append_params_init", "ttsdpa_kv_append",
     "ttsdpa_backward_params_init", "ttsdpa_backward_plan", "ttsdpa_backward_workspace_bytes", "ttsdpa_backward",
     # include/ttfused.h
     "ttfused_rms_norm", "ttfused_add_rms_norm", "ttfused_silu_mul", "ttfused_softmax", "ttfused_softmax_backward",
     # include/ttlinear.h
     "ttlinear_forward", "ttlinear_plan", "ttlinear_matmul", "ttlinear_matmul_batched", "ttlinear_matmul_workspace_bytes",
-    "ttlinear_matmul_tiles",
+    "ttlinear_matmul_tiles", "ttlinear_matmul_kernel", "ttlinear_backward_kernels",
     "ttlinear_backward", "ttlinear_backward_workspace_bytes", "ttlinear_backward_least_workspace_bytes",
 ]
 LINEAR_ROUTE_NAMES = {0: "none", 1: "mfma", 2: "general"}
+LINEAR_WAY_NAMES = {0: "general", 1: "stream", 2: "in_place", 3: "tiled", 4: "outer"}
+KERNEL_NAMES = {0: "other", 1: "short", 2: "short_joint", 3: "heads_16", 4: "heads_32"}
 LINEAR_TILES_NAMES = {0: "other", 1: "128x128", 2: "256x256", 3: "128x256", 4: "mixed"}
 
 
@@ -101,6 +103,12 @@ class KvAppendParams(ctypes.Structure):
     ]
 
 
+class LinearKernelInfo(ctypes.Structure):
+    """struct ttlinear_kernel_info"""
+    _fields_ = [("way", ctypes.c_int32), ("tile_rows", ctypes.c_int32), ("tile_columns", ctypes.c_int32),
+                ("tiles_per_workgroup", ctypes.c_int32), ("shares", ctypes.c_int32)]
+
+
 _lib = None
 
 
@@ -123,6 +131,8 @@ def lib():
         L.ttsdpa_params_init.restype = None
         L.ttsdpa_plan.argtypes = [P, ctypes.POINTER(ctypes.c_int)]
         L.ttsdpa_plan.restype = ctypes.c_int
+        L.ttsdpa_kernel.argtypes = [P, ctypes.POINTER(ctypes.c_int)]
+        L.ttsdpa_kernel.restype = ctypes.c_int
         L.ttsdpa_workspace_bytes.argtypes = [P]
         L.ttsdpa_workspace_bytes.restype = ctypes.c_size_t
         L.ttsdpa_forward.argtypes = [P, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
@@ -144,6 +154,8 @@ def lib():
         L.ttsdpa_backward_params_init.restype = None
         L.ttsdpa_backward_plan.argtypes = [BP, ctypes.POINTER(ctypes.c_int)]
         L.ttsdpa_backward_plan.restype = ctypes.c_int
+        L.ttsdpa_backward_kernel.argtypes = [BP, ctypes.c_size_t, ctypes.POINTER(ctypes.c_int)]
+        L.ttsdpa_backward_kernel.restype = ctypes.c_int
         L.ttsdpa_backward_workspace_bytes.argtypes = [BP]
         L.ttsdpa_backward_workspace_bytes.restype = ctypes.c_size_t
         L.ttsdpa_backward.argtypes = [BP, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
@@ -167,6 +179,11 @@ def lib():
         L.ttlinear_matmul_workspace_bytes.restype = ctypes.c_size_t
         L.ttlinear_matmul_tiles.argtypes = [ctypes.c_int, i64, i64, i64, ctypes.c_int, ctypes.c_int]
         L.ttlinear_matmul_tiles.restype = ctypes.c_int
+        IP = ctypes.POINTER(LinearKernelInfo)
+        L.ttlinear_matmul_kernel.argtypes = [ctypes.c_int, i64, i64, i64, ctypes.c_int, ctypes.c_int, IP]
+        L.ttlinear_matmul_kernel.restype = ctypes.c_int
+        L.ttlinear_backward_kernels.argtypes = [ctypes.c_int, i64, i64, i64, ctypes.c_int, IP, IP, ctypes.POINTER(ctypes.c_int)]
+        L.ttlinear_backward_kernels.restype = ctypes.c_int
         L.ttlinear_matmul.argtypes = [ctypes.c_int, vp, vp, vp, vp, i64, i64, i64, ctypes.c_int, ctypes.c_int, i64, i64, i64,
                                       vp, ctypes.c_size_t, vp]
         L.ttlinear_matmul.restype = ctypes.c_int
@@ -201,3 +218,36 @@ def plan(p):
     r = ctypes.c_int(-1)
     rc = lib().ttsdpa_plan(ctypes.byref(p), ctypes.byref(r))
     return rc, r.value
+
+
+def linear_kernel(dtype, M, N, K, trans_a=0, trans_b=1):
+    """(way, (rows, columns of a tile), tiles of a workgroup, shares of the contraction) that ttlinear_matmul runs a product on."""
+    i = LinearKernelInfo()
+    assert lib().ttlinear_matmul_kernel(dtype, M, N, K, trans_a, trans_b, ctypes.byref(i)) == OK
+    return _info(i)
+
+
+def linear_backward_kernels(dtype, M, N, K, with_bias=True):
+    """The same of a layer's weight and input gradients, and whether they run in one launch."""
+    w, i, one = LinearKernelInfo(), LinearKernelInfo(), ctypes.c_int(-1)
+    assert lib().ttlinear_backward_kernels(dtype, M, N, K, int(with_bias), ctypes.byref(w), ctypes.byref(i), ctypes.byref(one)) == OK
+    return _info(w), _info(i), bool(one.value)
+
+
+def _info(i):
+    return LINEAR_WAY_NAMES[i.way], (i.tile_rows, i.tile_columns), i.tiles_per_workgroup, i.shares
+
+
+def kernel(p):
+    """The kernel for short sequences that ttsdpa_forward runs a call on, or "other"."""
+    k = ctypes.c_int(-1)
+    assert lib().ttsdpa_kernel(ctypes.byref(p), ctypes.byref(k)) == OK
+    return KERNEL_NAMES[k.value]
+
+
+def backward_kernel(p, workspace_bytes=None):
+    """The same of ttsdpa_backward, with the scratch it asks for unless said otherwise."""
+    k = ctypes.c_int(-1)
+    n = lib().ttsdpa_backward_workspace_bytes(ctypes.byref(p)) if workspace_bytes is None else workspace_bytes
+    assert lib().ttsdpa_backward_kernel(ctypes.byref(p), n, ctypes.byref(k)) == OK
+    return KERNEL_NAMES[k.value]

@@ -1330,7 +1330,13 @@ static int launch_packed(const LinArgs& g, const PackPlan& p, int dtype, hipStre
 }
 
 // How a product runs: the cheapest by estimate of the ways that take it.
-enum class Way { General, Stream, InPlace, Packed, Outer };
+enum class Way {
+  General = TTLINEAR_WAY_GENERAL,
+  Stream = TTLINEAR_WAY_STREAM,
+  InPlace = TTLINEAR_WAY_IN_PLACE,
+  Packed = TTLINEAR_WAY_TILED,
+  Outer = TTLINEAR_WAY_OUTER
+};
 struct Choice {
   Way way = Way::General;
   double us = 1e30;
@@ -1419,6 +1425,24 @@ int ttlinear_matmul_tiles(int dtype, int64_t M, int64_t N, int64_t K, int trans_
   if (c.way != Way::Packed) return TTLINEAR_TILES_OTHER;
   g.K = c.pack.kpad, g.xt = g.wt = 0;
   return c.pack.S > 1 ? TTLINEAR_TILES_128x128 : tiles_of(g);
+}
+
+static ttlinear_kernel_info info_of(const LinArgs& g, const Choice& c, int dtype) {
+  ttlinear_kernel_info info{(int32_t)c.way, 0, 0, 1, 1};
+  if (c.way == Way::Packed) info.shares = c.pack.S;
+  if (c.way != Way::Stream) return info;
+  const StreamPlan call = plan_stream_call(g, dtype, 1, true, c.stream);
+  const StreamTiles t = stream_tiles(g, dtype, 1, call);
+  return {TTLINEAR_WAY_STREAM, t.rows, t.columns, t.per_workgroup, call.S};
+}
+
+int ttlinear_matmul_kernel(int dtype, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, ttlinear_kernel_info* info) {
+  if (!info) return TTSDPA_ERR_NULL;
+  if (dtype != TTSDPA_F32 && dtype != TTSDPA_F16 && dtype != TTSDPA_BF16) return TTSDPA_ERR_DTYPE;
+  if (M <= 0 || N <= 0 || K <= 0) return TTSDPA_ERR_SHAPE;
+  const LinArgs g = flags_args(M, N, K, trans_a, trans_b);
+  *info = info_of(g, choose(g, dtype, true, ~(size_t)0), dtype);
+  return TTSDPA_OK;
 }
 
 int ttlinear_matmul(int dtype, const void* a, const void* b, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
@@ -1562,6 +1586,26 @@ size_t ttlinear_backward_workspace_bytes(int dtype, int64_t M, int64_t N, int64_
     if (of_pair > most) most = of_pair;
   }
   return most > of_b ? most : of_b;
+}
+
+int ttlinear_backward_kernels(int dtype, int64_t M, int64_t N, int64_t K, int with_bias, ttlinear_kernel_info* of_weight,
+                              ttlinear_kernel_info* of_input, int* one_launch) {
+  if (!of_weight || !of_input || !one_launch) return TTSDPA_ERR_NULL;
+  if (dtype != TTSDPA_F32 && dtype != TTSDPA_F16 && dtype != TTSDPA_BF16) return TTSDPA_ERR_DTYPE;
+  if (M <= 0 || N <= 0 || K <= 0) return TTSDPA_ERR_SHAPE;
+  LinArgs gw = flags_args(N, K, M, 1, 0);
+  int sum;  // (never written: whether the row sums are wanted decides)
+  gw.rowsum = with_bias ? &sum : nullptr;
+  const LinArgs gi = flags_args(M, K, N, 0, 0);
+  const BackwardPlan p = plan_backward(gw, gi, dtype, ~(size_t)0);
+  *one_launch = p.joint;
+  *of_weight = info_of(gw, p.w, dtype), *of_input = info_of(gi, p.i, dtype);
+  if (p.joint) {
+    const StreamTiles w = stream_tiles(gw, dtype, 1, p.pair.gw);
+    *of_weight = {TTLINEAR_WAY_STREAM, w.rows, w.columns, w.per_workgroup, p.pair.gw.S};
+    *of_input = {TTLINEAR_WAY_STREAM, 16 * p.pair.gi.R, 16 * p.pair.gi.R, 1, 1};
+  }
+  return TTSDPA_OK;
 }
 
 int ttlinear_backward(int dtype, const void* grad, const void* x, const void* w, void* grad_x, void* grad_w, void* grad_b, int64_t M,

@@ -35,6 +35,10 @@ bool stream_takes(const LinArgs& a, int dtype);                                 
 StreamPlan plan_stream(const LinArgs& a, int dtype, unsigned entries, bool may_split);        // the estimate that chooses a product's way
 StreamPlan plan_stream_call(const LinArgs& a, int dtype, unsigned entries, bool may_split, const StreamPlan& p);  // what a call with that plan runs on
 size_t stream_part_bytes(const LinArgs& a, const StreamPlan& call);                           // scratch for its shares
+struct StreamTiles {
+  int rows, columns, per_workgroup;  // of the output in a tile; tiles of a workgroup
+};
+StreamTiles stream_tiles(const LinArgs& a, int dtype, unsigned entries, const StreamPlan& call);
 int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, const StreamPlan& p, unsigned entries = 1, void* scratch = nullptr,
                   size_t scratch_bytes = 0);
 // out = bias + the sums of a.splits shares of a product in a.part (and the row sums)

@@ -617,6 +617,11 @@ Tile few_rows_tile(const LinArgs& a, int R) {
   return a.K <= 2560 ? Tile::Rows16x64 : Tile::Square16;
 }
 
+// The tile of a call
+Tile tile_of_call(const LinArgs& a, int dtype, unsigned entries, const StreamPlan& p) {
+  return dtype != 0 && entries == 1 && p.S == 1 && p.R >= 2 ? few_rows_tile(a, p.R) : Tile::Square;
+}
+
 template <typename TR>
 int launch_rows_type(const LinArgs& a, Tile tile, hipStream_t stream) {
   switch (tile) {
@@ -685,6 +690,20 @@ StreamPlan plan_stream_call(const LinArgs& a, int dtype, unsigned entries, bool 
 
 size_t stream_part_bytes(const LinArgs& a, const StreamPlan& call) { return part_bytes(a, call.S); }
 
+StreamTiles stream_tiles(const LinArgs& a, int dtype, unsigned entries, const StreamPlan& call) {
+  switch (tile_of_call(a, dtype, entries, call)) {
+    case Tile::Square16: return {16, 16, 1};
+    case Tile::Rows32x48: return {32, 48, 1};
+    case Tile::Rows16x64: return {16, 64, 1};
+    case Tile::Rows16x32: return {16, 32, 1};
+    case Tile::Rows32x64: return {32, 64, 1};
+    case Tile::Rows48x64: return {48, 64, 1};
+    default: break;
+  }
+  const int W = wavefronts(call.R);
+  return {16 * call.R, 16 * call.R, a.xt && a.wt ? W / tile_wavefronts(a.K, dtype == 0 ? 32 : 64, W, call.S) : 1};
+}
+
 int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, const StreamPlan& chosen, unsigned entries, void* scratch, size_t scratch_bytes) {
   LinArgs a = args;
   StreamPlan p = plan_stream_call(a, dtype, entries, entries == 1 && scratch, chosen);
@@ -692,11 +711,9 @@ int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, const Stre
   a.splits = p.S;
   a.part = p.S > 1 ? (float*)scratch : nullptr;
   int rc;
-  if (dtype != 0 && entries == 1 && p.S == 1 && p.R >= 2) {
-    const Tile tile = few_rows_tile(a, p.R);
-    if (tile == Tile::Square16) p.R = 1;
-    else if (tile != Tile::Square) return dtype == 1 ? launch_rows_type<F16>(a, tile, stream) : launch_rows_type<BF16>(a, tile, stream);
-  }
+  const Tile tile = tile_of_call(a, dtype, entries, p);
+  if (tile == Tile::Square16) p.R = 1;
+  else if (tile != Tile::Square) return dtype == 1 ? launch_rows_type<F16>(a, tile, stream) : launch_rows_type<BF16>(a, tile, stream);
   switch (dtype) {
     case 0: rc = launch_type<F32>(a, p.R, stream, entries); break;
     case 1: rc = launch_type<F16>(a, p.R, stream, entries); break;

@@ -583,6 +583,12 @@ size_t short_backward_bytes(const ttsdpa_backward_params* p, int splits) {
   return backward_partial_offset(p) + (splits > 1 ? (size_t)splits * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float) : 0);
 }
 
+// ... with that much scratch (less than the query asks for: the pairs).
+int short_backward_taken(const ttsdpa_backward_params* p, size_t workspace_bytes, bool* joint) {
+  const int n = short_backward_splits(p, joint);
+  return n > 0 && workspace_bytes >= short_backward_bytes(p, n) ? n : 0;
+}
+
 // of the pairs
 size_t backward_scratch_bytes(const ttsdpa_backward_params* p) {
   const int n = dkv_splits_of(p), nq = dq_splits_of(p);
@@ -700,6 +706,16 @@ int ttsdpa_general(const ttsdpa_params* p, void* stream) {
   return launch_general(a, p->dtype, (hipStream_t)stream);
 }
 
+// Which of the kernels for short sequences a call of the prefill route (or of the general one whose masks the matrix-core kernels
+// apply) runs on.
+static int short_kernel_of(const ttsdpa_params* p, const KArgs& a) {
+  const int rows = heads_rows(a, p->dtype);
+  if (rows > 0) return rows == 16 ? TTSDPA_KERNEL_HEADS_16 : TTSDPA_KERNEL_HEADS_32;
+  return short_forward_best(p, a) ? TTSDPA_KERNEL_SHORT : TTSDPA_KERNEL_OTHER;
+}
+// masked calls of the general route: fp32 probabilities
+static int full_probabilities(const ttsdpa_params* p) { return p->mask_kind != TTSDPA_MASK_NONE && !long_d128(p) && !simple_mask_ok(p); }
+
 // ttsdpa_prefill with optional scratch: with it, a short-L call may divide its keys among workgroups.
 static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspace_bytes, void* stream, bool any_mask = false) {
   KArgs a;
@@ -708,9 +724,10 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
   if (p->B == 0 || p->L == 0) return TTSDPA_OK;
   if (!prefill_ok(p, any_mask)) return TTSDPA_ERR_UNSUPPORTED;
   if ((rc = check_grid((long long)a.B * a.Hq * ((a.L + 127) / 128))) != TTSDPA_OK) return rc;
-  a.full_p = p->mask_kind != TTSDPA_MASK_NONE && !long_d128(p) && !simple_mask_ok(p);  // (any_mask: the general route's calls, its arithmetic)
-  if (heads_rows(a, p->dtype) > 0) return launch_heads(a, p->dtype, (hipStream_t)stream);
-  if (short_forward_best(p, a)) return launch_short_forward(a, p->dtype, (hipStream_t)stream);
+  a.full_p = full_probabilities(p);  // (any_mask: the general route's calls, its arithmetic)
+  const int kind = short_kernel_of(p, a);
+  if (kind == TTSDPA_KERNEL_SHORT) return launch_short_forward(a, p->dtype, (hipStream_t)stream);
+  if (kind != TTSDPA_KERNEL_OTHER) return launch_heads(a, p->dtype, (hipStream_t)stream);
   // head_dim 128 with enough rows to fill 256-row workgroups takes the software-pipelined kernel (its tile loads
   // address 64 rows with 32-bit byte offsets)
   if (p->dtype != TTSDPA_F32 && pipelined_ok(p)) {
@@ -800,6 +817,17 @@ int ttsdpa_forward(const ttsdpa_params* p, void* workspace, size_t workspace_byt
   return ttsdpa_general(p, stream);
 }
 
+int ttsdpa_kernel(const ttsdpa_params* p, int* kind) {
+  KArgs a;
+  const int rc = validate(p, &a);
+  if (rc != TTSDPA_OK) return rc;
+  const int route = pick_route(p);
+  a.full_p = full_probabilities(p);
+  const bool prefill = route == TTSDPA_ROUTE_PREFILL || (route == TTSDPA_ROUTE_GENERAL && p->mask_kind != TTSDPA_MASK_NONE && prefill_ok(p, true));
+  if (kind) *kind = prefill ? short_kernel_of(p, a) : TTSDPA_KERNEL_OTHER;
+  return TTSDPA_OK;
+}
+
 void ttsdpa_backward_params_init(ttsdpa_backward_params* p, int dtype, int B, int Hq, int Hkv, int L, int S, int D) {
   memset(p, 0, sizeof(*p));
   p->struct_size = sizeof(*p);
@@ -815,6 +843,16 @@ int ttsdpa_backward_plan(const ttsdpa_backward_params* p, int* route) {
   int rc = validate_backward(p, &a);
   if (rc != TTSDPA_OK) return rc;
   if (route) *route = pick_backward_route(p);
+  return TTSDPA_OK;
+}
+
+int ttsdpa_backward_kernel(const ttsdpa_backward_params* p, size_t workspace_bytes, int* kind) {
+  BwdArgs a;
+  const int rc = validate_backward(p, &a);
+  if (rc != TTSDPA_OK) return rc;
+  bool joint = false;
+  const int n = pick_backward_route(p) == TTSDPA_ROUTE_NONE ? 0 : short_backward_taken(p, workspace_bytes, &joint);
+  if (kind) *kind = n == 0 ? TTSDPA_KERNEL_OTHER : joint ? TTSDPA_KERNEL_SHORT_JOINT : TTSDPA_KERNEL_SHORT;
   return TTSDPA_OK;
 }
 
@@ -838,8 +876,8 @@ int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t wor
   a.stats = (float*)workspace;
   a.log_sums = backward_log_sums(p) ? a.stats + 2 * backward_rows(p) : nullptr;
   bool joint = false;
-  const int n = short_backward_splits(p, &joint);
-  if (n > 0 && workspace_bytes >= short_backward_bytes(p, n)) {  // (less scratch than the query asks for: the pairs)
+  const int n = short_backward_taken(p, workspace_bytes, &joint);
+  if (n > 0) {
     a.dkv_splits = n, a.partial = n > 1 ? (float*)((char*)workspace + backward_partial_offset(p)) : nullptr;
     return launch_short_backward(a, p->fwd.dtype, joint, (hipStream_t)stream);
   }
