@@ -65,3 +65,19 @@ def test_kernels_of_short_sequences():
     bp = attention(BF16, 3, 4, 2, 100, 160, 64, causal=True, back=True)  # less scratch than asked for: the other kernels
     need = _capi.lib().ttsdpa_backward_workspace_bytes(ctypes.byref(bp))
     assert _capi.backward_kernel(bp) != "other" and _capi.backward_kernel(bp, need - 1) == "other"
+
+
+@pytest.mark.parametrize("dtype,M,N,K,tile,tiles", [
+    # backward of a layer, us, a tile of the weight's gradient to a workgroup / several
+    (BF16, 24, 128, 192, 16, 1),     # 3.7 / 4.5: all tiles of both products run side by side
+    (F16, 34, 128, 128, 16, 1),      # 3.7 / 4.5
+    (BF16, 97, 320, 232, 32, 1),     # 4.2 / 5.0 (16 x 16): a round of larger ones
+    (F32, 24, 512, 320, 32, 1),      # 5.4 / 7.7: fp32's share a CU in pairs
+    (F32, 20, 40, 3328, 32, 1),      # 5.5 / 7.3
+    (F32, 72, 576, 320, 32, 2),      # 6.7 / 6.0
+    (F32, 64, 500, 784, 32, 4),      # more than a round
+    (F32, 19, 2048, 2048, 32, 8),    # 55 / 21
+])
+def test_tiles_of_a_weights_gradient(dtype, M, N, K, tile, tiles):
+    of_weight, _, one = _capi.linear_backward_kernels(dtype, M, N, K)
+    assert one and of_weight == ("stream", (tile, tile), tiles, 1)

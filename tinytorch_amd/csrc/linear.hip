@@ -1601,7 +1601,7 @@ int ttlinear_backward_kernels(int dtype, int64_t M, int64_t N, int64_t K, int wi
   *one_launch = p.joint;
   *of_weight = info_of(gw, p.w, dtype), *of_input = info_of(gi, p.i, dtype);
   if (p.joint) {
-    const StreamTiles w = stream_tiles(gw, dtype, 1, p.pair.gw);
+    const StreamTiles w = stream_tiles(gw, dtype, 1, p.pair.gw, &gi, p.pair.gi.R);
     *of_weight = {TTLINEAR_WAY_STREAM, w.rows, w.columns, w.per_workgroup, p.pair.gw.S};
     *of_input = {TTLINEAR_WAY_STREAM, 16 * p.pair.gi.R, 16 * p.pair.gi.R, 1, 1};
   }

@@ -38,7 +38,8 @@ size_t stream_part_bytes(const LinArgs& a, const StreamPlan& call);             
 struct StreamTiles {
   int rows, columns, per_workgroup;  // of the output in a tile; tiles of a workgroup
 };
-StreamTiles stream_tiles(const LinArgs& a, int dtype, unsigned entries, const StreamPlan& call);
+// other, RI: another product in the launch, on tiles of 16 RI rows
+StreamTiles stream_tiles(const LinArgs& a, int dtype, unsigned entries, const StreamPlan& call, const LinArgs* other = nullptr, int RI = 0);
 int launch_stream(const LinArgs& a, int dtype, hipStream_t stream, const StreamPlan& p, unsigned entries = 1, void* scratch = nullptr,
                   size_t scratch_bytes = 0);
 // out = bias + the sums of a.splits shares of a product in a.part (and the row sums)

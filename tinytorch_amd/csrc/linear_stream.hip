@@ -180,20 +180,10 @@ struct StreamLds {
   static constexpr int BYTES = W * (STAGE > SUMS ? STAGE : SUMS);
 };
 
-// Wavefronts of a tile where both operands are k-major (a weight's gradient): as many of the W as a short contraction has units, the
-// workgroup's others take tiles of their own (GROUP: there are others).
-__host__ __device__ inline int tile_wavefronts(long long K, int KU, int W, int splits) {
-  int g = 1;
-  while (g < W && (long long)g * KU < K) g *= 2;
-  return splits > 1 ? W : g;
-}
-
 // One tile of the product: workgroup `block` of those of entry `entry`.  ROWSUM: the workgroups of the first column of tiles
 // also write a.rowsum[m] = sum_k x(m,k) (a product with ones that rides along in the matrix pipe).
 //
-// Tiles of a short contraction beside each other (tile_wavefronts; a wavefront each before, the workgroup's others idle), backward of a
-// layer, us: fp32 20 x 9000 x 3000 264 -> 155, 32 x 4096 x 1024 42.6 -> 21.7, 128 x 2048 x 2048 44.7 -> 37.9, 64 x 500 x 784 8.7 -> 8.3; 16-bit
-// 48 x 777 x 1001 13.3 -> 11.0.
+// GROUP: a.tile_waves of the workgroup's wavefronts share a tile, the others have tiles of their own (waves_of_call).
 template <typename TR, bool XT, bool WT, int MB, int NB, int W, int P, bool ROWSUM, bool GROUP = false>
 __device__ __forceinline__ void stream_tile(const LinArgs& a, char* smem, int block, int entry) {
   typedef Operand<TR, XT, MB> OX;
@@ -204,7 +194,7 @@ __device__ __forceinline__ void stream_tile(const LinArgs& a, char* smem, int bl
   constexpr int TM = 16 * MB, TN = 16 * NB, KU = OX::KU;
   const int lane = threadIdx.x & 63;
   const int wg_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = GROUP ? tile_wavefronts(a.K, KU, W, a.splits) : W;                                        // wavefronts of a tile
+  const int G = GROUP ? a.tile_waves : W;  // wavefronts of a tile
   const int wave = GROUP ? wg_wave & (G - 1) : wg_wave, first_wave = wg_wave - wave, per_block = GROUP ? W / G : 1;  // tiles of a workgroup
 
   // workgroup -> tile: an XCD (workgroup i runs on XCD i % 8) takes a contiguous band of tiles, rows of x fastest, so that
@@ -456,27 +446,27 @@ __global__ __launch_bounds__(64 * Shape<RW>::W, Shape<RW>::W / 4) void linear_st
   else stream_tile<TR, false, true, RI, RI, Shape<RI>::W, Shape<RI>::P, false>(gi, smem, blockIdx.x - split, 0);
 }
 
-template <typename TR, int R>
+template <int R>
 int tiles_of_block(const LinArgs& a) {
-  return a.xt && a.wt ? Shape<R>::W / tile_wavefronts(a.K, 8 * Step<TR>::KV, Shape<R>::W, a.splits) : 1;
+  return a.tile_waves ? Shape<R>::W / a.tile_waves : 1;
 }
 
-template <typename TR, int R>
+template <int R>
 long long blocks_of(const LinArgs& a) {
-  const long long tiles = ((a.M + 16 * R - 1) / (16 * R)) * ((a.N + 16 * R - 1) / (16 * R)), per_block = tiles_of_block<TR, R>(a);
+  const long long tiles = ((a.M + 16 * R - 1) / (16 * R)) * ((a.N + 16 * R - 1) / (16 * R)), per_block = tiles_of_block<R>(a);
   return ((tiles + per_block - 1) / per_block + 7) / 8 * 8 * a.splits;
 }
 
 template <typename TR, bool XT, bool WT, int R, bool GROUP = false>
 int launch_kernel(const LinArgs& a, hipStream_t stream, unsigned entries) {
   if constexpr (XT && WT && !GROUP)
-    if (tiles_of_block<TR, R>(a) > 1) return launch_kernel<TR, XT, WT, R, true>(a, stream, entries);
+    if (tiles_of_block<R>(a) > 1) return launch_kernel<TR, XT, WT, R, true>(a, stream, entries);
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
   constexpr int lds = StreamLds<TR, XT, WT, R, R, Shape<R>::W>::BYTES + (XT && WT ? Shape<R>::W * 16 * R * 4 : 0);
   const hipError_t granted = grant_dynamic_lds((const void*)linear_stream_kernel<TR, XT, WT, R, GROUP>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long blocks = blocks_of<TR, R>(a);
+  const long long blocks = blocks_of<R>(a);
   if (blocks > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
   hipLaunchKernelGGL((linear_stream_kernel<TR, XT, WT, R, GROUP>), dim3((unsigned)blocks, entries), dim3(64 * Shape<R>::W), lds, stream, a);
   return (int)hipGetLastError();
@@ -497,7 +487,7 @@ int launch_rows_kernel(const LinArgs& a, hipStream_t stream) {
 template <typename TR, int RW, int RI, bool GROUP = false>
 int launch_pair_kernel(const LinArgs& gw, const LinArgs& gi, hipStream_t stream) {
   if constexpr (!GROUP)
-    if (tiles_of_block<TR, RW>(gw) > 1) return launch_pair_kernel<TR, RW, RI, true>(gw, gi, stream);
+    if (tiles_of_block<RW>(gw) > 1) return launch_pair_kernel<TR, RW, RI, true>(gw, gi, stream);
   static hipError_t state[kMaxDevices];
   static bool done[kMaxDevices];
   constexpr int W = Shape<RW>::W;
@@ -505,7 +495,7 @@ int launch_pair_kernel(const LinArgs& gw, const LinArgs& gi, hipStream_t stream)
   constexpr int lds = lds_w > lds_i ? lds_w : lds_i;
   const hipError_t granted = grant_dynamic_lds((const void*)linear_stream_pair_kernel<TR, RW, RI, GROUP>, lds, state, done);
   if (granted != hipSuccess) return (int)granted;
-  const long long split = blocks_of<TR, RW>(gw), all = split + blocks_of<TR, RI>(gi);
+  const long long split = blocks_of<RW>(gw), all = split + blocks_of<RI>(gi);
   if (all > 0x3fffffffLL) return TTSDPA_ERR_SHAPE;
   hipLaunchKernelGGL((linear_stream_pair_kernel<TR, RW, RI, GROUP>), dim3((unsigned)all), dim3(64 * W), lds, stream, gw, gi, (int)split);
   return (int)hipGetLastError();
@@ -517,10 +507,28 @@ namespace {
 
 constexpr int wavefronts(int R) { return R == 4 ? Shape<4>::W : Shape<1>::W; }  // of a workgroup
 
-// Wavefronts that share a tile where a workgroup has several tiles; 0: it has one.
+// Wavefronts that a tile has work for where both operands are k-major (a weight's gradient) and a short contraction has fewer units
+// than a workgroup wavefronts; 0: for all.
 int waves_of_tile(const LinArgs& a, int esz, int R) {
-  const int G = a.xt && a.wt ? tile_wavefronts(a.K, 128 / esz, wavefronts(R), 1) : wavefronts(R);
+  if (!a.xt || !a.wt) return 0;
+  int G = 1;
+  while (G < wavefronts(R) && (long long)G * (128 / esz) < a.K) G *= 2;
   return G < wavefronts(R) ? G : 0;
+}
+
+double tiles_of(const LinArgs& a, int R) { return (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)); }
+
+// Wavefronts that share a tile of a call (others, RI: tiles and size of another product in the launch).  A workgroup takes as many tiles
+// as leave none of its wavefronts idle; backward of a layer, us, a tile to a workgroup -> so: fp32 19 x 2048 x 2048 55 -> 21; 16-bit 62 x 1024 x
+// 1024 13.4 -> 8.2.  But where all tiles run side by side there is nothing to gain, and those of a workgroup wait for each other: 16-bit layers of up to 256 tiles 4.2 us a tile to a workgroup, 4.5 in groups; fp32
+// 24 x 512 x 320 5.4 and 7.7, whose 32 x 32 tiles share a CU in pairs, where one unit is all their work or the other product's tiles are of
+// that size too (20 x 40 x 3328, 312 tiles, 5.5 and 7.3; 72 x 576 x 320, 280 tiles of three units and 16-row ones, 6.7 and 6.0).
+int waves_of_call(const LinArgs& a, int esz, int R, int S, double entries, double others, int RI) {
+  const int W = wavefronts(R), G = S > 1 ? 0 : waves_of_tile(a, esz, R);
+  if (G == 0) return W;
+  const double tiles = 8 * ceil(tiles_of(a, R) / 8) * entries;
+  const bool pairs = esz == 4 && R == 2 && (RI == 2 || (G == 1 && tiles <= 256));
+  return tiles + 8 * ceil(others / 8) <= (pairs ? 512 : 256) ? W : G;
 }
 
 double rounds_of(const LinArgs& a, long long tm, long long tn, double entries) {
@@ -550,11 +558,11 @@ double rounds_of(const LinArgs& a, long long tm, long long tn, double entries) {
 double stream_us(const LinArgs& a, int esz, int R, int S, double entries, bool whole = false) {
   if (esz == 4 && R == 4 && S == 1 && waves_of_tile(a, esz, R) == 1) return 5 + 3 * rounds_of(a, 64, 64, entries);
   if (const int G = esz == 2 && S == 1 ? waves_of_tile(a, esz, R) : 0) {
-    const double tiles = (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)) * entries, waves = tiles * G / 1024;
+    const double tiles = tiles_of(a, R) * entries, waves = tiles * G / 1024;
     return 3 + (waves <= 1 && R < 4 ? 0.5 : waves * (R == 1 ? 0.9 : R == 2 ? 1.9 : 7.7));
   }
   const double tm = 16 * R, tn = 16 * R;
-  const double tiles = (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)) * entries * S;
+  const double tiles = tiles_of(a, R) * entries * S;
   // (16-bit x . w^T, 64 rows: a second round lasts as long as the first, however few its tiles: 720 x 1536 x 1536, 288 tiles, 18.2 us, on the
   // tiled kernel 14.8; k-major operands bound such calls otherwise)
   const double rounds = tiles <= 256 ? 1 : whole && R == 4 ? ceil(tiles / 256) : esz == 2 && R == 4 && !a.xt && !a.wt && tiles < 512 ? 2 : tiles / 256;
@@ -659,10 +667,14 @@ int launch_pair_type(const LinArgs& gw, const LinArgs& gi, int RW, int RI, hipSt
 PairPlan plan_pair(const LinArgs& gw, const LinArgs& gi, int esz) {
   PairPlan few{plan_tiles(gw, esz, 1, true, 1, 2), plan_tiles(gi, esz, 1, false, 1, 2)};
   // one round of the CUs with both, if that only takes larger tiles of the other (16-bit; 60 x 777 x 1001 10.8 -> 6.1, 60 x 512 x 1024 6.5 -> 5.0)
-  auto tiles = [](const LinArgs& a, int R) { return ((a.M + 16 * R - 1) / (16 * R)) * ((a.N + 16 * R - 1) / (16 * R)); };
   if (const int G = esz == 2 && few.gw.S == 1 && few.gw.R == 2 && few.gi.R == 1 && gi.N >= 32 ? waves_of_tile(gw, esz, 2) : 0) {
-    const long long blocks = tiles(gw, 2) * G / wavefronts(2);
-    if (blocks + tiles(gi, 1) > 256 && blocks + tiles(gi, 2) <= 256) few.gi = {2, 1, stream_us(gi, esz, 2, 1, 1)};
+    const double blocks = floor(tiles_of(gw, 2) * G / wavefronts(2));
+    if (blocks + tiles_of(gi, 1) > 256 && blocks + tiles_of(gi, 2) <= 256) few.gi = {2, 1, stream_us(gi, esz, 2, 1, 1)};
+  }
+  // and a round with a tile of the weight's gradient to a workgroup, if larger ones of it make that (97 x 320 x 232 5.0 -> 4.2)
+  if (esz == 2 && few.gw.S == 1 && few.gw.R == 1 && gw.M >= 32 && gw.N >= 32 && waves_of_tile(gw, esz, 1) > 0) {
+    const double of_i = tiles_of(gi, few.gi.R);
+    if (tiles_of(gw, 1) + of_i > 256 && tiles_of(gw, 2) + of_i <= 240) few.gw.R = 2;
   }
   const PairPlan many{plan_tiles(gw, esz, 1, true, 4, 4), plan_tiles(gi, esz, 1, false, 4, 4)};
   return many.gw.R && many.gi.R && many.gw.us + many.gi.us < few.gw.us + few.gi.us ? many : few;
@@ -690,7 +702,7 @@ StreamPlan plan_stream_call(const LinArgs& a, int dtype, unsigned entries, bool 
 
 size_t stream_part_bytes(const LinArgs& a, const StreamPlan& call) { return part_bytes(a, call.S); }
 
-StreamTiles stream_tiles(const LinArgs& a, int dtype, unsigned entries, const StreamPlan& call) {
+StreamTiles stream_tiles(const LinArgs& a, int dtype, unsigned entries, const StreamPlan& call, const LinArgs* other, int RI) {
   switch (tile_of_call(a, dtype, entries, call)) {
     case Tile::Square16: return {16, 16, 1};
     case Tile::Rows32x48: return {32, 48, 1};
@@ -700,8 +712,7 @@ StreamTiles stream_tiles(const LinArgs& a, int dtype, unsigned entries, const St
     case Tile::Rows48x64: return {48, 64, 1};
     default: break;
   }
-  const int W = wavefronts(call.R);
-  return {16 * call.R, 16 * call.R, a.xt && a.wt ? W / tile_wavefronts(a.K, dtype == 0 ? 32 : 64, W, call.S) : 1};
+  return {16 * call.R, 16 * call.R, wavefronts(call.R) / waves_of_call(a, dtype == 0 ? 4 : 2, call.R, call.S, entries, other ? tiles_of(*other, RI) : 0, RI)};
 }
 
 int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, const StreamPlan& chosen, unsigned entries, void* scratch, size_t scratch_bytes) {
@@ -710,6 +721,7 @@ int launch_stream(const LinArgs& args, int dtype, hipStream_t stream, const Stre
   if (part_bytes(a, p.S) > scratch_bytes) p = plan_stream_call(a, dtype, entries, false, plan_stream(a, dtype, entries, false));
   a.splits = p.S;
   a.part = p.S > 1 ? (float*)scratch : nullptr;
+  a.tile_waves = waves_of_call(a, dtype == 0 ? 4 : 2, p.R, p.S, entries, 0, 0);
   int rc;
   const Tile tile = tile_of_call(a, dtype, entries, p);
   if (tile == Tile::Square16) p.R = 1;
@@ -728,6 +740,7 @@ int launch_stream_pair(const LinArgs& gw_, const LinArgs& gi, int dtype, hipStre
   LinArgs gw = gw_;
   gw.splits = p.gw.S;
   gw.part = p.gw.S > 1 ? (float*)scratch : nullptr;
+  gw.tile_waves = waves_of_call(gw, dtype == 0 ? 4 : 2, p.gw.R, p.gw.S, 1, tiles_of(gi, p.gi.R), p.gi.R);
   int rc;
   switch (dtype) {
     case 0: rc = launch_pair_type<F32>(gw, gi, p.gw.R, p.gi.R, stream); break;
