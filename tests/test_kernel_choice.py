@@ -81,3 +81,17 @@ def test_kernels_of_short_sequences():
 def test_tiles_of_a_weights_gradient(dtype, M, N, K, tile, tiles):
     of_weight, _, one = _capi.linear_backward_kernels(dtype, M, N, K)
     assert one and of_weight == ("stream", (tile, tile), tiles, 1)
+
+
+@pytest.mark.parametrize("M,N,K,way", [
+    # us in one round of 64 x 64 tiles on the streaming kernel / divided among workgroups
+    (539, 1600, 2432, "stream"),   # 14.1 / 18.1
+    (444, 1920, 2624, "stream"),   # 14.4 / 18.0
+    (865, 1024, 3328, "stream"),   # 17.6 / 19.4
+    (288, 2048, 6592, "tiled"),    # 29.2 / 22.9
+    (414, 2176, 9984, "tiled"),    # 49.0 / 36.8
+])
+def test_divided_where_one_round_of_small_tiles_is_longer(M, N, K, way):
+    for dtype in (F16, BF16):
+        kernel = _capi.linear_kernel(dtype, M, N, K)
+        assert kernel[0] == way and (kernel[3] > 1) == (way == "tiled")

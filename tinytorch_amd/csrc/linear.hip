@@ -1286,9 +1286,9 @@ static PackPlan plan_pack(const LinArgs& g, int dtype, size_t room, double beat)
   p.S = 1;
   // (copies for the alignment's sake alone: 804 x 1983 x 5329 64 us, undivided 57; fp32 that the streaming kernel takes: that adds a
   // contraction up in more and shorter chains)
-  // And not worth a look where two shares' sums and the operands read once take longer than another way, at choose()'s margin.
+  // And not worth a look where two shares' sums and the operands read once take longer than another way, at choose()'s margins.
   const bool may = (p.copies == 0 || g.xt || g.wt) && !(dtype == TTSDPA_F32 && stream_takes(g, dtype)) &&
-                   7.7 + (double)esz * (double)(g.M + g.N) * (double)g.K / 4.2e6 + 16.0 * (double)g.M * (double)g.N / 5e6 < 0.9 * beat;
+                   7.7 + (double)esz * (double)(g.M + g.N) * (double)g.K / 4.2e6 + 16.0 * (double)g.M * (double)g.N / 5e6 < 1.03 * beat;
   const long long most = kCusOfXcd / ((((g.M + 127) / 128) * ((g.N + 127) / 128) + 7) / 8);  // a workgroup to a CU
   for (int S = 2; may && S <= 16 && S <= most && p.kpad / bk >= 4 * S; S++) {
     const double divided = divided_cost(nt, dtype, S);
@@ -1355,10 +1355,12 @@ static Choice choose(const LinArgs& g, int dtype, bool scratch, size_t scratch_b
     take(Way::Stream, c.stream.us);
   }
   c.pack = plan_pack(g, dtype, scratch ? scratch_bytes : 0, c.us);
-  // (margins for divided contractions: the estimates miss by a tenth, 719 x 1024 x 2688 15.8 us on the streaming kernel, 16.8
-  // divided; those of the ways that read contraction-major operands as they lie by more, the input gradient of 231 x 19072 x 3072 17
-  // us shorter so than divided with its copies)
-  if (c.pack.ok && c.pack.bytes <= (scratch ? scratch_bytes : 0)) take(Way::Packed, c.pack.S == 1 ? c.pack.us : c.pack.us / (c.pack.copies > 0 ? 0.75 : 0.9));
+  // (margins for divided contractions: the estimates of the ways that read contraction-major operands as they lie miss by more, the
+  // input gradient of 231 x 19072 x 3072 17 us shorter so than divided with its copies; those of the streaming kernel's small tiles and
+  // shares by a tenth, of its large tiles less)
+  const bool sure = c.way == Way::Stream && c.stream.R == 4 && c.stream.S == 1;
+  if (c.pack.ok && c.pack.bytes <= (scratch ? scratch_bytes : 0))
+    take(Way::Packed, c.pack.S == 1 ? c.pack.us : c.pack.us / (c.pack.copies > 0 ? 0.75 : sure ? 1.03 : 0.9));
   // (row sums, where wanted, come with the product, as on the streaming kernel; the tiled kernels need launches for them)
   if (outer_takes(g, dtype)) take(Way::Outer, outer_cost(g, dtype) - (g.rowsum && c.way != Way::Stream ? 4 : 0));
   return c;

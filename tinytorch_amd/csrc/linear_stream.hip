@@ -572,7 +572,10 @@ double stream_us(const LinArgs& a, int esz, int R, int S, double entries, bool w
   const double rate = esz == 2 ? 4e6 : R < 4 ? 0.3e6 : rounds > 1.5 ? 0.36e6 : 0.45e6, flops = 2 * tm * tn * k;
   const double per = bytes / 65e3 > flops / rate ? bytes / 65e3 : flops / rate;
   const double few = (double)(a.M < a.N ? a.M : a.N) * a.K * esz, all = (double)(a.M + a.N) * a.K * esz;
-  const double missed = few > 2e6 && all > 8e6 ? tiles * bytes / (esz == 2 && (a.xt || a.wt) ? 10e6 : 8e6) : 0;
+  // (one round of tiles on rows of whole lines: they go along the contraction together, and the L2s hold what they are at: 539 x 1600 x 2432
+  // 14.1 us, 22.5 by the rate; rows across lines up to 1.4 times that)
+  const bool together = esz == 2 && S == 1 && !a.xt && !a.wt && tiles <= 256 && (a.ldx | a.ldw) % 64 == 0;
+  const double missed = few > 2e6 && all > 8e6 && !together ? tiles * bytes / (esz == 2 && (a.xt || a.wt) ? 10e6 : 8e6) : 0;
   // 16-bit: the next tile's first loads and the last one's output do not overlap (tiles of 64 rows: 72 of k into 960 x 7552, 7 rounds
   // 38 us, 752 into 1906 x 2088, 3.9: 32; of 32: 327 into 310 x 4245, 5.2: 17.6, 262 k-major into 2545 x 866, 8.8: 27)
   // (two workgroups of 32 rows share a CU: two rounds are one)
