@@ -95,3 +95,12 @@ def test_divided_where_one_round_of_small_tiles_is_longer(M, N, K, way):
     for dtype in (F16, BF16):
         kernel = _capi.linear_kernel(dtype, M, N, K)
         assert kernel[0] == way and (kernel[3] > 1) == (way == "tiled")
+
+
+def test_whole_rounds_of_shares():
+    for dtype in (F16, BF16):
+        # us in one share and two: 32.7 and 35.2, 29.4 and 32.5
+        assert _capi.linear_kernel(dtype, 54, 18688, 3072)[3] == 1
+        assert _capi.linear_kernel(dtype, 276, 3864, 2800)[3] == 1
+        # 44 tiles in four shares and eight, a round and a half: 16.8 and 21.1
+        assert _capi.linear_kernel(dtype, 112, 1408, 8448)[3] == 4

@@ -564,8 +564,10 @@ double stream_us(const LinArgs& a, int esz, int R, int S, double entries, bool w
   const double tm = 16 * R, tn = 16 * R;
   const double tiles = tiles_of(a, R) * entries * S;
   // (16-bit x . w^T, 64 rows: a second round lasts as long as the first, however few its tiles: 720 x 1536 x 1536, 288 tiles, 18.2 us, on the
-  // tiled kernel 14.8; k-major operands bound such calls otherwise)
-  const double rounds = tiles <= 256 ? 1 : whole && R == 4 ? ceil(tiles / 256) : esz == 2 && R == 4 && !a.xt && !a.wt && tiles < 512 ? 2 : tiles / 256;
+  // tiled kernel 14.8; k-major operands bound such calls otherwise.  The shares of such calls are counted so too, lest two of them look
+  // shorter: 54 x 18688 x 3072, 292 tiles, 32.7, in two shares 35.2)
+  const bool whole_rounds = R == 4 && (whole || (esz == 2 && !a.xt && !a.wt && (tiles < 512 || (tiles > 256 * S && tiles < 512 * S))));
+  const double rounds = tiles <= 256 ? 1 : whole_rounds ? ceil(tiles / 256) : tiles / 256;
   const double narrow = esz == 4 ? 1 : R == 1 ? 2.6 : R == 2 ? 1.6 : 1.1;
   const double k = (double)a.K / S;
   const double bytes = ((a.M < tm ? a.M : tm) * (a.xt ? narrow : 1) + (a.N < tn ? a.N : tn) * (a.wt ? narrow : 1)) * k * esz;
