@@ -104,3 +104,26 @@ def test_whole_rounds_of_shares():
         assert _capi.linear_kernel(dtype, 276, 3864, 2800)[3] == 1
         # 44 tiles in four shares and eight, a round and a half: 16.8 and 21.1
         assert _capi.linear_kernel(dtype, 112, 1408, 8448)[3] == 4
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    # us in 32 x 32 tiles / the smaller ones that were taken
+    (1, 28672, 4096, (16, 16)),    # 45.1 / 42.5
+    (8, 32000, 4096, (16, 16)),    # 55.3 / 48.7
+    (6, 44032, 2560, (32, 32)),    # 0.91 of the speed in 16 x 16 ones
+    (8, 50304, 3072, (32, 32)),    # 59.1 / 61.1
+    (9, 28672, 4096, (32, 32)),
+    (14, 15360, 5120, (32, 32)),   # 29.3 / 34.2
+    (11, 16000, 3072, (32, 32)),   # 21.2 / 24.2
+    (14, 10000, 3072, (32, 48)),   # of 16 x 16, 32 x 48 and 16 x 64 tiles the shortest, by 14 and 12 %
+    (14, 10000, 4096, (16, 16)),
+    (14, 10000, 2048, (16, 64)),
+    (14, 16384, 2048, (16, 64)),
+    (24, 8704, 4096, (32, 48)),
+    (24, 12352, 4096, (32, 32)),
+    (8, 8192, 4096, (32, 32)),
+])
+def test_tiles_of_few_rows(M, N, K, tile):
+    for dtype in (F16, BF16):
+        kernel = _capi.linear_kernel(dtype, M, N, K)
+        assert kernel[0] == "stream" and kernel[1] == tile

@@ -605,12 +605,16 @@ StreamPlan plan_tiles(const LinArgs& a, int esz, double entries, bool may_split,
 }
 
 // The tile for up to 32 rows of x where 32 x 32 ones would be taken, 16-bit x . w^T.  Those of one to two rounds of the 256 CUs last as
-// long as two; us on them and so:
-//   24 rows x 8704, K 1024, 2048, 4096    8.4, 14.2, 23.5 -> 7.1, 11.6, 18.6 (32 x 48)      x 12288    9.0, 14.8, 23.7 -> 8.1, 14.0, 19.2
-//   6 x 8448                              7.9, 13.0, 21.1 -> 6.7 (32 x 48), 10.5 (16 x 64), 17.3 (16 x 16: four times the workgroups, no remainder)
-//   6 x 16384                             9.1, 15.1, 32.0 -> 9.3, 14.9 (16 x 64), 26.1 (16 x 16)
-// and a weight of more than 200 MB, with up to eight rows of up to 4096, streams best in small pieces: 1 x 28672 x 4096 43.2 -> 40.7
-// (16 x 28672 x 4096 and 3 x 20480 x 3072 the same; 6 x 28544 x 5120 55.6 in 32 x 32 tiles, 59.1 so).
+// long as two.  A tile's eight wavefronts take its units of 64 of K in turn, with four on their way in 16-row tiles: those go by
+// whole rings (K 1536, 2048, 3584, 4096, 6144, 8192, or a few units more), while a ring of one or two at the end costs what the smaller tile
+// gained.  Times of 32 x 32 tiles over those of others, weights from memory, geometric means of 6500 products by K and tiles:
+//   257 to 384 tiles    up to 16 rows, whole rings    K < 2560  16 x 64 1.14 to 1.24, 32 x 48 1.02 to 1.18    beyond  16 x 16 1.11 to 1.23
+//                       others                        32 x 48 1.07 to 1.31 (16 x 16 1.0 to 1.17, K 1024 0.9)
+//   385 to 512          up to 16 rows, whole rings    K < 2560  16 x 64 1.05 to 1.14    beyond  up to 8  16 x 16 1.01 to 1.12, more  16 x 64 1.02 to 1.10
+//                       others                        16 x 16 0.82 to 0.98, 16 x 64 0.95 to 1.08, 32 x 48 0.75
+//   more, 200 MB        up to 8 rows, whole rings     16 x 16 1.00 to 1.08 (28672 x 4096 1.06, 32000 x 4096 1.14)
+//                       others                        16 x 16 K 1024 0.75 to 0.85, 2560 0.91, 3072 0.97, 5120 0.98
+//   24 rows x 8704, K 1024, 2048, 4096    8.4, 14.2, 23.5 us -> 7.1, 11.6, 18.6 (32 x 48)
 // k-major w (a layer's input gradient), us, rows x columns x contraction: up to 16 rows in 16 x 32 tiles, 16 x 8192 x 2048 12.6 -> 11.0 (5 x 7839 x 731
 // 6.4 -> 7.2, hence the least contraction); 32 x 64 ones where 32 x 32 make one to two rounds, 30 x 11264 x 4096 38 -> 28, 8 x 10880 x 5760 40
 // -> 30; 33 to 48 rows in 48 x 64 tiles of eight wavefronts instead of 64 x 64 of four, 42 x 11200 x 4096 28 -> 23, 37 x 17280 x 5120 58 -> 54.
@@ -624,10 +628,15 @@ Tile few_rows_tile(const LinArgs& a, int R) {
   }
   if (a.xt || a.M > 32 || R != 2) return Tile::Square;
   const long long tiles = (a.N + 31) / 32;
-  if (a.M <= 8 && a.K <= 4096 && a.N * a.K > 100000000ll) return Tile::Square16;
-  if (tiles <= 256 || tiles > 512) return Tile::Square;
-  if (a.M > 16 || a.K < 1536) return a.N <= 48 * 256 ? Tile::Rows32x48 : Tile::Square;
-  return a.K <= 2560 ? Tile::Rows16x64 : Tile::Square16;
+  const int units = (int)((a.K + 63) / 64), rest = units & 31;  // beyond whole rings of all wavefronts
+  const bool whole_rings = rest == 0 || rest >= 22 || (rest <= 4 && units > 64);
+  if (tiles > 512) return a.M <= 8 && whole_rings && a.K > 1400 && a.N * a.K > 100000000ll ? Tile::Square16 : Tile::Square;
+  if (tiles <= 256) return Tile::Square;
+  if (a.M <= 16 && a.K >= 1536) {
+    if (a.K < 2560 && (whole_rings || tiles > 384)) return Tile::Rows16x64;
+    if (whole_rings) return tiles > 384 && a.M > 8 ? Tile::Rows16x64 : Tile::Square16;
+  }
+  return tiles <= 384 ? Tile::Rows32x48 : Tile::Square;  // (a round of 32 x 48)
 }
 
 // The tile of a call
