@@ -127,3 +127,19 @@ def test_tiles_of_few_rows(M, N, K, tile):
     for dtype in (F16, BF16):
         kernel = _capi.linear_kernel(dtype, M, N, K)
         assert kernel[0] == "stream" and kernel[1] == tile
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    # us in 32 x 32 tiles / 16 x 32 ones, of a contraction-major weight
+    (16, 8192, 2048, (16, 32)),   # 12.6 / 11.0
+    (12, 7928, 2744, (32, 32)),   # 14.4 / 15.3: six units a wavefront
+    (8, 5179, 3064, (32, 32)),    # 14.5 / 15.3
+    (16, 5179, 3064, (32, 32)),   # 15.2 / 16.1
+    (14, 6144, 4096, (16, 32)),
+    (16, 8192, 1100, (32, 32)),
+    (30, 11264, 4096, (32, 64)),
+])
+def test_tiles_of_few_rows_contraction_major(M, N, K, tile):
+    for dtype in (F16, BF16):
+        kernel = _capi.linear_kernel(dtype, M, N, K, 0, 0)
+        assert kernel[0] == "stream" and kernel[1] == tile

@@ -616,7 +616,8 @@ StreamPlan plan_tiles(const LinArgs& a, int esz, double entries, bool may_split,
 //                       others                        16 x 16 K 1024 0.75 to 0.85, 2560 0.91, 3072 0.97, 5120 0.98
 //   24 rows x 8704, K 1024, 2048, 4096    8.4, 14.2, 23.5 us -> 7.1, 11.6, 18.6 (32 x 48)
 // k-major w (a layer's input gradient), us, rows x columns x contraction: up to 16 rows in 16 x 32 tiles, 16 x 8192 x 2048 12.6 -> 11.0 (5 x 7839 x 731
-// 6.4 -> 7.2, hence the least contraction); 32 x 64 ones where 32 x 32 make one to two rounds, 30 x 11264 x 4096 38 -> 28, 8 x 10880 x 5760 40
+// 6.4 -> 7.2, hence the least contraction; 5850 products by units of a wavefront: 3 and 4 1.10, 5 1.03, 8, 12 and 16 1.03 to 1.04, 6 0.98, 7 1.02 with
+// a tenth of them 0.95 to 0.97, 10 and 14 1.00); 32 x 64 ones where 32 x 32 make one to two rounds, 30 x 11264 x 4096 38 -> 28, 8 x 10880 x 5760 40
 // -> 30; 33 to 48 rows in 48 x 64 tiles of eight wavefronts instead of 64 x 64 of four, 42 x 11200 x 4096 28 -> 23, 37 x 17280 x 5120 58 -> 54.
 enum class Tile { Square, Square16, Rows32x48, Rows16x64, Rows16x32, Rows32x64, Rows48x64 };
 Tile few_rows_tile(const LinArgs& a, int R) {
@@ -624,7 +625,9 @@ Tile few_rows_tile(const LinArgs& a, int R) {
     if (R == 4) return a.M > 32 && a.M <= 48 ? Tile::Rows48x64 : Tile::Square;
     const long long pieces = (a.N + 31) / 32;
     if (a.M > 32 || pieces > 512) return Tile::Square;
-    return pieces > 256 ? Tile::Rows32x64 : a.M <= 16 && a.K >= 1200 ? Tile::Rows16x32 : Tile::Square;
+    if (pieces > 256) return Tile::Rows32x64;
+    const int each = (int)((a.K + 511) / 512);  // units of a wavefront: rings of four
+    return a.M <= 16 && a.K >= 1200 && (each & 3) != 2 && each != 7 ? Tile::Rows16x32 : Tile::Square;
   }
   if (a.xt || a.M > 32 || R != 2) return Tile::Square;
   const long long tiles = (a.N + 31) / 32;
