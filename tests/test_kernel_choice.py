@@ -143,3 +143,26 @@ def test_tiles_of_few_rows_contraction_major(M, N, K, tile):
     for dtype in (F16, BF16):
         kernel = _capi.linear_kernel(dtype, M, N, K, 0, 0)
         assert kernel[0] == "stream" and kernel[1] == tile
+
+
+@pytest.mark.parametrize("mask,B,H,L,D,kernel", [
+    # us on the kernel for long sequences / on the one that holds a head's keys
+    ("keys", 38, 16, 60, 32, "other"),     # 6.2 / 7.8: more than two rounds of workgroups
+    ("keys", 43, 12, 22, 32, "other"),     # 5.4 / 6.7
+    ("keys", 39, 16, 24, 16, "other"),     # 5.5 / 6.6
+    ("keys", 39, 16, 23, 16, "heads_16"),  # 7.8 / 6.9: keys of no whole fours
+    ("keys", 8, 12, 60, 32, "heads_16"),
+    ("keys", 43, 12, 22, 64, "heads_16"),
+    ("keys", 16, 12, 197, 64, "heads_32"),
+    ("bool", 4, 8, 50, 32, "other"),       # 0.95 of the speed
+    ("bool", 4, 8, 30, 48, "heads_16"),    # 1.2
+    ("bool", 4, 8, 100, 32, "heads_16"),
+    ("bool", 4, 8, 50, 64, "heads_16"),
+    ("add", 8, 16, 128, 32, "other"),      # 6.5 / 7.7, its keys read four at a time
+    ("add", 8, 16, 130, 32, "heads_16"),   # 8.5 / 6.2 at 93
+    ("add", 46, 16, 20, 32, "heads_16"),   # 10.3 / 7.2
+    ("add", 8, 16, 128, 64, "heads_16"),
+])
+def test_masked_heads(mask, B, H, L, D, kernel):
+    for dtype in (F16, BF16):
+        assert _capi.kernel(attention(dtype, B, H, H, L, L, D, mask=mask)) == kernel

@@ -365,14 +365,18 @@ int launch_t(const KArgs& a, int rows, hipStream_t stream) {
 
 // Rows of a wavefront of the kernel for a call, 0: another kernel is the shorter way (or the only one).  a.full_p as the call has it.
 // 16 rows where the workgroups run side by side, at most two rounds of them of the shortest heads; 32, with half the LDS reads for
-// each product but nothing requested ahead, where more are needed and the mask is the keys' alone; head_dim 32 and below has tiles of
-// its own in the other kernel.  Against that kernel, us, key padding / additive [H, L, L]:
+// each product but nothing requested ahead, where more are needed and the mask is the keys' alone.  Against the other kernel, us, key
+// padding / additive [H, L, L]:
 //   8 heads x 94       7.0 ->  5.3              16 x 49 (bf16)          6.7 -> 5.7
 //   64 x 247 (bf16)   12.2 ->  8.3              64 x 217 (bf16)        15.8 -> 10.5
 //   128 x 136          8.4 ->  6.5              128 x 93 (bf16)        10.2 -> 6.8
 //   192 x 197         13.0 -> 12.0 (32 rows)    256 x 189              16.8 -> 16.8 (there; 19.6 here)
 //   256 x 137         11.7 ->  9.1 (32 rows)    384 x 104 (bf16)       10.1 -> 10.1 (there; 13.3 here)
 //   768 x 174         32.4 -> 26.9 (32 rows)    768 x 47 (bf16)        12.7 -> 10.6
+// head_dim 32 and below has tiles of its own in the other kernel.  Its time over this one's there, geometric means of 3800 calls: keys 1.05
+// to 1.2, but 0.82 with two rounds of workgroups at 32, or where it reads the mask four keys at a time; Bool rows 0.95 to 0.98 up to 64 rows (0.7 with two rounds), 1.02 to 1.07 beyond;
+// additive ones 1.06 to 1.4, but where it reads their keys four at a time 0.9 to 0.95 with more than 96 rows and 1024 units of 16 in all.  At 40
+// to 64 the same are 1.1 to 1.5 throughout, Bool rows up to 32 1.00 to 1.2.
 int heads_rows(const KArgs& a, int dtype) {
   if (dtype == 0 || a.D < 8 || a.D > W || a.D % 8 != 0 || a.S < 1 || a.S > 32 * kMostPairs || a.L < 16 || a.L > 256 || a.block_table ||
       a.pack_L || a.causal || a.mask_kind == 0)
@@ -381,8 +385,13 @@ int heads_rows(const KArgs& a, int dtype) {
   if (!keys_only && (a.ms[3] != 1 || a.S < 4 || a.kv_len)) return 0;  // (it reads such masks four keys at a time)
   const HeadsShape n(a, 1);
   const long long side = 256ll * (kMostWaves / n.waves);
-  if (n.wgs <= (n.waves <= 4 ? 2 : 1) * side && (keys_only || a.full_p || n.wgs * n.units < 2048)) return 16;
-  return keys_only && a.D > 32 ? 32 : 0;
+  const bool narrow = a.D <= 32;
+  bool best = n.wgs <= (n.waves <= 4 ? 2 : 1) * side;
+  if (keys_only) best = best && !(narrow && n.wgs >= 512 && (a.D == 32 || !a.full_p));
+  else if (a.mask_kind == 1) best = best && (!narrow || a.L > 64);
+  else if (narrow && !a.full_p) best = best && (a.L <= 96 || n.wgs * n.units < 1024);
+  if (best) return 16;
+  return keys_only && !narrow ? 32 : 0;
 }
 
 int launch_heads(const KArgs& a, int dtype, hipStream_t stream) {
