@@ -166,3 +166,20 @@ def test_tiles_of_few_rows_contraction_major(M, N, K, tile):
 def test_masked_heads(mask, B, H, L, D, kernel):
     for dtype in (F16, BF16):
         assert _capi.kernel(attention(dtype, B, H, H, L, L, D, mask=mask)) == kernel
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,D,kernel", [
+    # fp32, causal: us on the kernel for long sequences / on the short sequences' one
+    (1, 1, 1, 918, 128, "other"),   # 20.1 / 27.3
+    (1, 1, 1, 892, 64, "other"),    # 14.5 / 15.8
+    (2, 1, 1, 701, 64, "short"),    # 14.7 / 12.8
+    (8, 32, 8, 76, 64, "other"),    # 12.1 / 14.6
+    (4, 32, 4, 107, 128, "other"),  # 21.3 / 24.5
+    (8, 4, 1, 435, 128, "other"),   # 33.5 / 38.6
+    (4, 32, 8, 83, 64, "short"),    # 12.0 / 10.1
+    (4, 32, 4, 75, 128, "short"),   # 19.4 / 17.9
+    (1, 32, 8, 259, 128, "short"),  # 43.2 / 22.0
+    (1, 16, 2, 652, 128, "short"),  # 50.4 / 38.4
+])
+def test_fp32_forward_of_short_sequences(B, Hq, Hkv, L, D, kernel):
+    assert _capi.kernel(attention(F32, B, Hq, Hkv, L, L, D, causal=True)) == kernel

@@ -581,7 +581,8 @@ int launch_prefill(const KArgs& a, int dtype, hipStream_t stream);       // 128-
 int launch_prefill_d128(const KArgs& a, int dtype, hipStream_t stream);  // 256-row workgroups, pipelined; head_dim 128
 int launch_prefill_d64(const KArgs& a, int dtype, hipStream_t stream);   // the same at head_dim 64 (no attnMask, no pages)
 int launch_prefill_f32(const KArgs& a, hipStream_t stream);              // fp32 tensors on the fp32 matrix cores; head_dim 64 or 128
-double prefill_f32_tiles(const KArgs& a);  // key tiles (of 32) that an unsplit launch takes one after the other
+// key tiles (of 32) that an unsplit launch takes one after the other; dealt: its wavefronts share a row tile's
+double prefill_f32_tiles(const KArgs& a, bool* dealt = nullptr);
 int heads_rows(const KArgs& a, int dtype);                                     // whether, and how, launch_heads is the way for a call
 int launch_heads(const KArgs& a, int dtype, hipStream_t stream);            // with an attnMask, up to 256 keys, 16-bit tensors (sdpa_heads.hip)
 int launch_short_forward(const KArgs& a, int dtype, hipStream_t stream);    // short sequences, any element type (sdpa_short.hip)

@@ -429,9 +429,10 @@ int launch_f32_d(const KArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-double prefill_f32_tiles(const KArgs& a) {
+double prefill_f32_tiles(const KArgs& a, bool* dealt) {
   double tiles = 0;
-  keys_among_wavefronts(a, &tiles);
+  const bool among = keys_among_wavefronts(a, &tiles);
+  if (dealt) *dealt = among;
   return tiles;
 }
 

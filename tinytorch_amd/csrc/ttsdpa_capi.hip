@@ -350,6 +350,17 @@ struct ShortShape {
     const double* c = fit[f32][wide];
     return c[0] + c[1] * ((keys + 7) / 8) + c[2] * more(heads * rows, avg);
   }
+  // Whether an fp32 forward call is one of those that the two estimates get wrong: a single long head, which the other kernel divides (892
+  // rows 14.5 us, 15.8 here; 918 x 128 20.0 and 27.3), and causal ones of several rounds of workgroups, whose loads then bound this
+  // kernel and whose end the other one's wavefronts share (256 heads x 76 x 64 12.1 and 14.6; 128 x 107 x 128 21.3 and 24.5, 32 x 435 x 128
+  // 33.5 and 38.6): 17 of 448 drawn calls, none of the others lost.
+  bool forward_misses(const ttsdpa_params* p, double f32_tiles, bool dealt) const {
+    if (heads == 1) return rows > 52;
+    if (!wide) return heads * rows > 1024;
+    if (p->D <= 96 || !causal || heads * rows <= 512 || L > 512) return false;
+    const double other = dealt && heads * ((L + 31) / 32) > 256 ? 17 + 1.1 * f32_tiles : 6.5 + 4.1 * f32_tiles;
+    return forward_us() + more(heads * rows, 2.7) > other;
+  }
   // of the other kernels: 16-bit ones by 64-key tiles, up to eight in a row (more are divided); fp32 ones by the tiles of 32 that their
   // own rule for dealing them out finds
   double other_forward_us(double f32_tiles) const {
@@ -423,7 +434,9 @@ bool f32_decode_ok(const ttsdpa_params* p) {
 bool short_forward_best(const ttsdpa_params* p, const KArgs& a) {
   if (!short_ok(p) || pack_heads_ok(p) || !prefill_ok(p)) return false;
   const ShortShape s(p);
-  return s.forward_us() < s.least_margin() * s.other_forward_us(s.f32 ? prefill_f32_tiles(a) : 0);
+  bool dealt = false;
+  const double tiles = s.f32 ? prefill_f32_tiles(a, &dealt) : 0;
+  return s.forward_us() < s.least_margin() * s.other_forward_us(tiles) && !(s.f32 && s.forward_misses(p, tiles, dealt));
 }
 
 int pick_route(const ttsdpa_params* p) {
