@@ -183,3 +183,16 @@ def test_masked_heads(mask, B, H, L, D, kernel):
 ])
 def test_fp32_forward_of_short_sequences(B, Hq, Hkv, L, D, kernel):
     assert _capi.kernel(attention(F32, B, Hq, Hkv, L, L, D, causal=True)) == kernel
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,L,D,kernel", [
+    # causal, us on the kernels for long sequences / on the short sequences' one launch
+    (F32, 4, 64, 8, 64, 64, "other"),          # 34.9 / 45.6
+    (BF16, 4, 64, 8, 75, 64, "other"),         # 24.3 / 28.2
+    (BF16, 8, 16, 2, 65, 128, "other"),        # 29.2 / 32.3
+    (BF16, 2, 56, 8, 77, 128, "other"),        # 29.5 / 31.4
+    (BF16, 8, 8, 8, 72, 64, "short_joint"),    # 15.0 / 14.4
+    (BF16, 4, 16, 2, 124, 64, "short_joint"),  # 23.5 / 22.8
+])
+def test_backward_of_short_sequences_in_one_launch(dtype, B, Hq, Hkv, L, D, kernel):
+    assert _capi.backward_kernel(attention(dtype, B, Hq, Hkv, L, L, D, causal=True, back=True)) == kernel

@@ -590,7 +590,12 @@ int short_backward_splits(const ttsdpa_backward_params* p, bool* joint = nullptr
   const ShortShape s(f);
   const double one = s.backward_us(true), two = s.backward_us(false);
   if (joint) *joint = one < two;
-  return (one < two ? one : two) < s.least_margin() * pair_backward_us(p) ? s.splits() : 0;
+  // (the joint launch takes longer than its estimate by a tenth for each round of workgroups beyond the first: with more than three of
+  // them it lost up to 24 %, 256 heads x 64 x 64 fp32 34.9 us on the pairs, 45.6 here; bf16 x 75 24.3 and 28.2)
+  const double us = one < two ? one : two, pair = pair_backward_us(p), rounds = s.heads * s.rows / 256;
+  const bool padded = s.wide && f->D <= 96;  // (of 128 columns: less than the estimate, 64 heads x 111 x 80 18.0 us, 27.4 on the pairs)
+  if (one < two && rounds > 1 && !padded && us * (1 + 0.1 * (rounds - 1)) >= 0.85 * pair) return 0;
+  return us < s.least_margin() * pair ? s.splits() : 0;
 }
 size_t short_backward_bytes(const ttsdpa_backward_params* p, int splits) {
   return backward_partial_offset(p) + (splits > 1 ? (size_t)splits * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float) : 0);
