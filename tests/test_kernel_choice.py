@@ -180,6 +180,7 @@ def test_masked_heads(mask, B, H, L, D, kernel):
     (4, 32, 4, 75, 128, "short"),   # 19.4 / 17.9
     (1, 32, 8, 259, 128, "short"),  # 43.2 / 22.0
     (1, 16, 2, 652, 128, "short"),  # 50.4 / 38.4
+    (8, 4, 4, 328, 128, "short"),   # 32.7 / 27.1: a head to every KV head
 ])
 def test_fp32_forward_of_short_sequences(B, Hq, Hkv, L, D, kernel):
     assert _capi.kernel(attention(F32, B, Hq, Hkv, L, L, D, causal=True)) == kernel

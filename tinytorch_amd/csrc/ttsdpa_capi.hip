@@ -351,13 +351,13 @@ struct ShortShape {
     return c[0] + c[1] * ((keys + 7) / 8) + c[2] * more(heads * rows, avg);
   }
   // Whether an fp32 forward call is one of those that the two estimates get wrong: a single long head, which the other kernel divides (892
-  // rows 14.5 us, 15.8 here; 918 x 128 20.0 and 27.3), and causal ones of several rounds of workgroups, whose loads then bound this
+  // rows 14.5 us, 15.8 here; 918 x 128 20.0 and 27.3), and causal ones of several rounds of workgroups on shared KV heads, whose loads then bound this
   // kernel and whose end the other one's wavefronts share (256 heads x 76 x 64 12.1 and 14.6; 128 x 107 x 128 21.3 and 24.5, 32 x 435 x 128
-  // 33.5 and 38.6): 17 of 448 drawn calls, none of the others lost.
+  // 33.5 and 38.6; but 32 x 328 x 128, each with its own keys, 32.7 and 27.1).
   bool forward_misses(const ttsdpa_params* p, double f32_tiles, bool dealt) const {
     if (heads == 1) return rows > 52;
-    if (!wide) return heads * rows > 1024;
-    if (p->D <= 96 || !causal || heads * rows <= 512 || L > 512) return false;
+    if (!wide) return heads * rows > 1152;
+    if (p->D <= 96 || group == 1 || !causal || heads * rows <= 512 || L > 512) return false;
     const double other = dealt && heads * ((L + 31) / 32) > 256 ? 17 + 1.1 * f32_tiles : 6.5 + 4.1 * f32_tiles;
     return forward_us() + more(heads * rows, 2.7) > other;
   }
