@@ -363,8 +363,9 @@ __device__ __forceinline__ void stream_tile(const LinArgs& a, char* smem, int bl
   }
 }
 
-// out = bias + the sum of the splits' partial products, and the same of the row sums.  I: integers that hold an index into a split.
-template <typename T, typename I>
+// out = bias + the sum of the splits' partial products, and the same of the row sums.  An index into a split has 32 bits (plan_tiles; divided
+// tiles are few).
+template <typename T>
 __global__ __launch_bounds__(256) void linear_merge_kernel(LinArgs a) {
   typedef float loose4 __attribute__((ext_vector_type(4), aligned(4)));  // (a split begins at any element)
   typedef T out4 __attribute__((ext_vector_type(4)));
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(256) void linear_merge_kernel(LinArgs a) {
       f32x4 v = *(const loose4*)(a.part + i);
 #pragma unroll 4
       for (int s = 1; s < a.splits; s++) v += (f32x4)*(const loose4*)(a.part + s * total + i);
-      const I m = (I)i / (I)a.N, n = (I)i - m * (I)a.N;
+      const uint32_t m = (uint32_t)i / (uint32_t)a.N, n = (uint32_t)i - m * (uint32_t)a.N;
       if (a.bias)
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] += load_as_float((const T*)a.bias + n + e);
@@ -402,8 +403,8 @@ template <typename T>
 int launch_merge(const LinArgs& a, hipStream_t stream) {
   const long long groups = (a.M * a.N + a.M + 1023) / 1024;
   const dim3 grid((unsigned)(groups < 2048 ? groups : 2048));
-  if (a.M * a.N + a.M < 0x7fffffffLL) hipLaunchKernelGGL((linear_merge_kernel<T, uint32_t>), grid, dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL((linear_merge_kernel<T, long long>), grid, dim3(256), 0, stream, a);
+  if (a.M * a.N + a.M >= 0x7fffffffLL) return TTSDPA_ERR_SHAPE;  // (the plans keep to this)
+  hipLaunchKernelGGL((linear_merge_kernel<T>), grid, dim3(256), 0, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -519,8 +520,8 @@ int waves_of_tile(const LinArgs& a, int esz, int R) {
 double tiles_of(const LinArgs& a, int R) { return (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)); }
 
 // Wavefronts that share a tile of a call (others, RI: tiles and size of another product in the launch).  A workgroup takes as many tiles
-// as leave none of its wavefronts idle; backward of a layer, us, a tile to a workgroup -> so: fp32 19 x 2048 x 2048 55 -> 21; 16-bit 62 x 1024 x
-// 1024 13.4 -> 8.2.  But where all tiles run side by side there is nothing to gain, and those of a workgroup wait for each other: 16-bit layers of up to 256 tiles 4.2 us a tile to a workgroup, 4.5 in groups; fp32
+// as leave none of its wavefronts idle; backward of a layer, us, a tile to a workgroup -> so: fp32 19 x 2048 x 2048 54 -> 20; 16-bit 62 x 1024 x
+// 1024 13.5 -> 6.0.  But where all tiles run side by side there is nothing to gain, and those of a workgroup wait for each other: 16-bit layers of up to 256 tiles 4.2 us a tile to a workgroup, 4.5 in groups; fp32
 // 24 x 512 x 320 5.4 and 7.7, whose 32 x 32 tiles share a CU in pairs, where one unit is all their work or the other product's tiles are of
 // that size too (20 x 40 x 3328, 312 tiles, 5.5 and 7.3; 72 x 576 x 320, 280 tiles of three units and 16-row ones, 6.7 and 6.0).
 int waves_of_call(const LinArgs& a, int esz, int R, int S, double entries, double others, int RI) {
@@ -595,7 +596,7 @@ StreamPlan plan_tiles(const LinArgs& a, int esz, double entries, bool may_split,
     // half of a 64 square tile idle: its few workgroups stream a weight slower than the estimate, which has every round full (12 x
     // 5120 x 34944: 87 us in 64-row tiles, 69 in 32-row ones; 12 x 4096 x 28672 54 and 45)
     if (R == 4 && R > least && (a.M <= 32 || a.N <= 32)) break;
-    for (int S = 1; S <= 32 && (S == 1 || (may_split && a.K >= 512 * S)); S *= 2) {
+    for (int S = 1; S <= 32 && (S == 1 || (may_split && a.K >= 512 * S && a.M * a.N + a.M < 0x7fffffffLL)); S *= 2) {
       if (wavefronts(R) * S < chains) continue;
       const double t = stream_us(a, esz, R, S, entries, whole);
       if (!best.R || t < best.us) best = {R, S, t};
