@@ -107,3 +107,20 @@ def grad_err(got_dev, expect):
     assert y.shape == expect.shape
     assert np.isfinite(y).all(), "non-finite values in the GPU gradient"
     return float(np.abs(y.astype(np.float64) - expect.astype(np.float64)).max() / max(1.0, float(np.abs(expect).max())))
+
+
+_EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}
+CODE = {torch.float32: _capi.F32, torch.float16: _capi.F16, torch.bfloat16: _capi.BF16}
+
+
+def close_product(got, a, b, extra=None):
+    """got = a . b (+ extra): one rounding of the result and fp32 sums of K products, whose error grows at most with the sum of their
+    magnitudes (K * 2^-24 of it is never reached: sqrt(K) steps of random sign, times eight).  fp16 below its normal numbers (one
+    product of two small ones) is rounded to multiples of 2^-24: half of that."""
+    a, b = a.double(), b.double()
+    ref, mag = a @ b, a.abs() @ b.abs()
+    if extra is not None:
+        ref, mag = ref + extra.double(), mag + extra.double().abs()
+    bound = _EPS[got.dtype] * ref.abs() + 8 * a.shape[1] ** 0.5 * 2.0 ** -24 * mag + (2.0 ** -25 if got.dtype == torch.float16 else 1e-30)
+    worst = ((got.double() - ref).abs() / bound).max().item()
+    assert worst <= 1.0, worst

@@ -8,6 +8,8 @@ import pytest
 import torch
 
 import tinytorch_amd as tt
+from tinytorch_amd import _capi
+from tinytorch_amd.function import build_params
 
 pytestmark = pytest.mark.gpu
 
@@ -87,6 +89,7 @@ def test_heads(case, dtype):
     if kind == "counts":  # key counts beside the mask; the first key of every entry is visible
         lens = torch.randint(1, S + 1, (B,), generator=g, device="cuda", dtype=torch.int32)
     out = tt.sdpAttention(q, k, v, attnMask=mask, kvLens=lens)
+    assert _capi.kernel(build_params(q, k, v, out, False, mask, None, lens)) == ("heads_32" if B == 40 or B == 16 else "heads_16")
     ref = expected(q, k, v, mask, lens)
     err = ((out.double().cpu() - ref).norm() / ref.norm()).item()
     assert err <= REL[dtype], err
@@ -105,6 +108,7 @@ def test_rows_and_values_at_the_edge(B, H, L, dtype):
     mask[0, :, :, L - 3:] = False
     k[0, 0, L - 1] = math.nan
     out = tt.sdpAttention(q, k, v, attnMask=mask)
+    assert _capi.kernel(build_params(q, k, v, out, False, mask)) == ("heads_32" if B == 40 else "heads_16")
     ref = expected(q, k.nan_to_num(), v, mask, None)
     assert out[1].isnan().all()
     seen = torch.ones(B, dtype=torch.bool)
@@ -127,6 +131,7 @@ def test_lowest_value(dtype):
     mask = torch.zeros(4, 50, 50, device="cuda", dtype=DT[dtype])
     mask[:, 7] = torch.finfo(DT[dtype]).min
     out = tt.sdpAttention(q, k, v, attnMask=mask)
+    assert _capi.kernel(build_params(q, k, v, out, False, mask)) == "heads_16"
     assert out.isfinite().all()
     if dtype == "bf16":  # (fp16's lowest value leaves the scores their bits)
         mean = v.double().mean(2)

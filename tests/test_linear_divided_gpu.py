@@ -7,59 +7,60 @@ import pytest
 import torch
 
 import tinytorch_amd as tt
+from gpu_util import close_product
 from tinytorch_amd import _capi
 
 pytestmark = pytest.mark.gpu
 
 DT = {"f32": (torch.float32, 0), "f16": (torch.float16, 1), "bf16": (torch.bfloat16, 2)}
-_EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}
-
-
-def _close(got, a, b, extra=None):
-    """got = a . b (+ extra): one rounding of the result and fp32 sums of K products, whose error grows at most with the sum of
-    their magnitudes (K * 2^-24 of it is never reached: sqrt(K) steps of random sign, times eight)."""
-    a, b = a.double(), b.double()
-    ref, mag = a @ b, a.abs() @ b.abs()
-    if extra is not None:
-        ref, mag = ref + extra.double(), mag + extra.double().abs()
-    bound = _EPS[got.dtype] * ref.abs() + 8 * a.shape[1] ** 0.5 * 2.0 ** -24 * mag + 1e-30
-    worst = ((got.double() - ref).abs() / bound).max().item()
-    assert worst <= 1.0, worst
-
-
 def _operands(M, N, K, dtype, seed=0):
     g = torch.Generator(device="cuda").manual_seed(seed + M + N + K)
     return [torch.randn(*s, generator=g, device="cuda").to(DT[dtype][0]) for s in ((M, K), (N, K), (N,))]
 
 
-# tiles 24 to 112 in all, 2 to 10 shares; 103, 74 and 81 k-steps, which no number of shares here divides evenly
-SIZES = [("f16", 288, 2048, 6592), ("bf16", 720, 1536, 4736), ("bf16", 129, 4097, 10368), ("bf16", 200, 4094, 14336), ("f32", 119, 3072, 9152),
-         ("f32", 300, 1021, 3200), ("f16", 500, 2050, 5632), ("bf16", 978, 1024, 2688)]
+# tiles 48 to 72 in all; 103, 74 and 81 k-steps, which no number of shares here divides evenly
+SIZES = [("f16", 288, 2048, 6592, 5), ("bf16", 720, 1536, 4736, 3), ("bf16", 129, 4097, 10368, 3), ("bf16", 200, 4094, 14336, 4), ("f16", 500, 2050, 5632, 3)]
 
 
-@pytest.mark.parametrize("dtype,M,N,K", SIZES)
-def test_divided(dtype, M, N, K):
+@pytest.mark.parametrize("dtype,M,N,K,shares", SIZES)
+def test_divided(dtype, M, N, K, shares):
     print("divided", dtype, M, N, K, flush=True)
+    assert _capi.linear_kernel(DT[dtype][1], M, N, K) == ("tiled", (0, 0), 1, shares)
     x, w, b = _operands(M, N, K, dtype)
-    _close(tt.linear(x, w, b), x, w.t(), b)
+    close_product(tt.linear(x, w, b), x, w.t(), b)
     assert torch.equal(tt.linear(x, w, b), tt.linear(x, w, b))  # shares are added in one order
 
 
-@pytest.mark.parametrize("dtype,M,N,K", [("bf16", 407, 17920, 3072), ("f16", 574, 13824, 2048), ("bf16", 954, 10368, 1536)])
-def test_input_gradient(dtype, M, N, K):
+@pytest.mark.parametrize("trans_b", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(6, 768, 28672), (15, 3000, 16385), (1, 500, 4097)])
+def test_narrow_operand(M, N, K, trans_b):
+    """fp32 is divided where the streaming kernel does not take it: a contraction-major operand of fewer than 16 rows, whose copy (and
+    that of the other one) lies in the scratch before the sums."""
+    print("narrow", M, N, K, trans_b, flush=True)
+    kernel = _capi.linear_kernel(_capi.F32, M, N, K, 1, trans_b)
+    assert kernel[0] == "tiled" and kernel[3] > 1
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b, c = (torch.randn(*s, generator=g, device="cuda") for s in ((K, M), (N, K) if trans_b else (K, N), (N,)))
+    close_product(tt.matmul(a, b, True, bool(trans_b), c), a.t(), b.t() if trans_b else b, c)
+
+
+@pytest.mark.parametrize("dtype,M,N,K,shares", [("bf16", 535, 19072, 2048, 3), ("f16", 809, 16576, 1024, 4), ("bf16", 954, 10368, 1536, 2)])
+def test_input_gradient(dtype, M, N, K, shares):
     """grad . w with w contraction-major: the copy of w lies in the scratch before the sums."""
     print("gradient", dtype, M, N, K, flush=True)
+    assert _capi.linear_backward_kernels(DT[dtype][1], M, N, K)[1] == ("tiled", (0, 0), 1, shares)
     x, w, _ = _operands(M, N, K, dtype)
     go = _operands(M, N, N, dtype, 1)[0]
     gx, gw, gb = tt.linearBackward(go, x, w)
-    _close(gx, go, w)
-    _close(gw, go.t(), x)
-    _close(gb.view(1, N), torch.ones(1, M, device="cuda"), go)
+    close_product(gx, go, w)
+    close_product(gw, go.t(), x)
+    close_product(gb.view(1, N), torch.ones(1, M, device="cuda"), go)
 
 
-@pytest.mark.parametrize("dtype,M,N,K", [("bf16", 720, 1536, 4736), ("f32", 119, 3072, 9152)])
+@pytest.mark.parametrize("dtype,M,N,K", [("bf16", 720, 1536, 4736), ("f16", 288, 2048, 6592)])
 def test_less_scratch(dtype, M, N, K):
     """A caller with less than the sums need gets the same product another way; what lies behind its scratch stays as it was."""
+    assert _capi.linear_kernel(DT[dtype][1], M, N, K)[0] == "tiled"
     x, w, b = _operands(M, N, K, dtype)
     code = DT[dtype][1]
     L = _capi.lib()
@@ -75,7 +76,7 @@ def test_less_scratch(dtype, M, N, K):
         rc = L.ttlinear_matmul(code, p(x), p(w), p(b), p(out), i64(M), i64(N), i64(K), 0, 1, i64(K), i64(K), i64(N), p(ws), ctypes.c_size_t(size),
                                stream)
         assert rc == 0
-        _close(out, x, w.t(), b)
+        close_product(out, x, w.t(), b)
         assert (ws[size:] == 77).all()
 
 
@@ -86,4 +87,4 @@ def test_rounds_of_64_rows(dtype, M, N, K):
     """Both sides of 256 and 512 tiles of 64 x 64, where the streaming kernel's estimate counts in whole rounds."""
     print("rounds", dtype, M, N, K, flush=True)
     x, w, b = _operands(M, N, K, dtype)
-    _close(tt.linear(x, w, b), x, w.t(), b)
+    close_product(tt.linear(x, w, b), x, w.t(), b)

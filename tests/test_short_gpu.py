@@ -1,7 +1,7 @@
-"""Short sequences, forward and backward (csrc/sdpa_short.hip), against the chain matmul -> scale -> mask -> softmax -> matmul
+"""Short sequences, forward and backward (csrc/sdpa_short.hip; each case says which of its calls run there), against the chain matmul -> scale -> mask -> softmax -> matmul
 (reference src/Function/FuncNNLayer.h:237-265) and its gradients in 64 bits: sizes around the kernels' units of 16 rows and keys and
 their eight wavefronts, every element type, head sizes of 8 to 128, both causal alignments, key counts, grouped heads whose units are
-divided among workgroups, gradients in one launch (up to about 130 rows) and in two."""
+divided among workgroups, more workgroups than CUs, gradients in one launch and in two."""
 import ctypes
 import math
 
@@ -9,8 +9,8 @@ import pytest
 import torch
 
 import tinytorch_amd as tt
-from gpu_util import backward_call, call
 from tinytorch_amd import _capi, build_backward_params
+from tinytorch_amd.function import build_params
 
 pytestmark = pytest.mark.gpu
 
@@ -21,27 +21,34 @@ DT = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
 REL = {"f32": 3e-6, "f16": 2 ** -11 * 1.6, "bf16": 2 ** -8 * 1.6}
 
 CASES = [
-    # B, Hq, Hkv, L, S, D, causal ("br": bottom-right aligned), key counts
-    (1, 2, 2, 16, 16, 64, True, None),          # one unit
-    (1, 2, 1, 17, 31, 64, False, None),
-    (2, 2, 2, 31, 17, 128, True, None),         # rows past S see every key
-    (1, 4, 4, 64, 64, 64, True, None),
-    (1, 4, 4, 100, 100, 80, True, None),
-    (1, 3, 1, 127, 129, 128, False, None),      # eight units and one key
-    (1, 4, 4, 128, 128, 64, True, None),
-    (2, 8, 2, 129, 129, 64, True, None),        # nine units; groups of four heads divided
-    (1, 7, 1, 90, 90, 128, True, None),
-    (2, 4, 2, 150, 200, 96, "br", None),
-    (2, 2, 2, 200, 150, 64, "br", None),        # more rows than keys
-    (3, 4, 2, 100, 160, 64, "br", (160, 77, 101)),
-    (3, 2, 2, 120, 120, 128, False, (1, 120, 63)),
-    (4, 2, 1, 60, 70, 64, False, (70, 0, 16, 33)),  # an entry without keys
-    (1, 8, 2, 333, 333, 128, True, None),       # gradients in two launches and divided
-    (2, 2, 2, 500, 511, 64, False, None),
-    (1, 2, 1, 1000, 1000, 64, True, None),
-    (1, 2, 2, 48, 48, 8, True, None),
-    (1, 2, 2, 48, 40, 40, False, None),
-    (2, 16, 16, 260, 260, 64, True, None),      # more workgroups than CUs
+    # B, Hq, Hkv, L, S, D, causal ("br": bottom-right aligned), key counts; kernels of fp32 forward and backward, 16-bit forward and
+    # backward: s(hort; backward: dq, then dk and dv), j(oint: one launch), o(ther)
+    (1, 2, 2, 16, 16, 64, True, None, "sjoj"),          # one unit
+    (1, 2, 1, 17, 31, 64, False, None, "sjoj"),
+    (2, 2, 2, 31, 17, 128, True, None, "ossj"),         # rows past S see every key
+    (1, 4, 4, 64, 64, 64, True, None, "sjoj"),
+    (1, 4, 4, 100, 100, 80, True, None, "sssj"),
+    (1, 3, 1, 127, 129, 128, False, None, "sosj"),      # eight units and one key
+    (1, 4, 4, 128, 128, 64, True, None, "sjsj"),
+    (2, 8, 2, 129, 129, 64, True, None, "sjsj"),        # nine units; groups of four heads divided
+    (1, 7, 1, 90, 90, 128, True, None, "sssj"),
+    (2, 4, 2, 150, 200, 96, "br", None, "sosj"),
+    (2, 2, 2, 200, 150, 64, "br", None, "sjsj"),        # more rows than keys
+    (3, 4, 2, 100, 160, 64, "br", (160, 77, 101), "sjsj"),
+    (3, 2, 2, 120, 120, 128, False, (1, 120, 63), "sssj"),
+    (4, 2, 1, 60, 70, 64, False, (70, 0, 16, 33), "sjsj"),  # an entry without keys
+    (1, 8, 2, 333, 333, 128, True, None, "ssss"),       # gradients in two launches and divided
+    (2, 2, 2, 500, 511, 64, False, None, "soss"),
+    (1, 2, 1, 1000, 1000, 64, True, None, "soss"),
+    (1, 2, 2, 48, 48, 8, True, None, "sjoj"),
+    (1, 2, 2, 48, 40, 40, False, None, "sjoj"),
+    (2, 16, 16, 260, 260, 64, True, None, "sooo"),      # more workgroups than CUs, in each of the kernels
+    (2, 8, 8, 300, 300, 64, True, None, "ooso"),
+    (2, 8, 2, 333, 333, 64, True, None, "ooss"),
+    (8, 8, 8, 72, 72, 64, True, None, "oooj"),
+    (1, 16, 2, 330, 330, 64, True, None, "osss"),
+    (1, 32, 4, 130, 130, 64, True, None, "ojoj"),
+    (1, 64, 8, 70, 70, 128, True, None, "ossj"),
 ]
 
 
@@ -74,12 +81,16 @@ def rel_err(got, ref):
 @pytest.mark.parametrize("dtype", list(DT))
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "B%dH%dk%dL%dS%dD%d-%s-%s" % (c[:7] + ("all" if c[7] is None else "lens",)))
 def test_short(case, dtype):
-    B, Hq, Hkv, L, S, D, causal, lens = case
+    B, Hq, Hkv, L, S, D, causal, lens, kernels = case
     print("short", case, dtype, flush=True)
     q, k, v, go = operands(L + S + D, B, Hq, Hkv, L, S, D, dtype)
     n = torch.tensor(lens, dtype=torch.int32, device="cuda") if lens else None
     kw = dict(isCausal=bool(causal), kvLens=n, causalAlign="bottom-right" if causal == "br" else "top-left")
     out = tt.sdpAttention(q, k, v, **kw)
+    args = (bool(causal), None, None, n, kw["causalAlign"])
+    letter = {"short": "s", "short_joint": "j", "other": "o"}
+    ran = letter[_capi.kernel(build_params(q, k, v, out, *args))] + letter[_capi.backward_kernel(build_backward_params(q, k, v, out, go, q, k, v, *args))]
+    assert ran == (kernels[:2] if dtype == "f32" else kernels[2:])
     got = (out,) + tuple(tt.sdpAttentionBackward(go, q, k, v, out, **kw))
     for name, x, y in zip(("out", "dq", "dk", "dv"), got, expected(q, k, v, go, causal, lens)):
         assert rel_err(x, y) <= REL[dtype], (name, rel_err(x, y))
@@ -114,27 +125,26 @@ def test_nan_reaches_the_gradients(dtype):
     assert not dq[0, 0, :20].isnan().any() and not dq[0, 1].isnan().any() and not dk[0, 1].isnan().any()
 
 
-@pytest.mark.parametrize("L", [128, 300])
-def test_less_scratch(L):
-    """A caller whose scratch holds the pairs' needs only (4 x 8 heads on 2: the divided sums of the short way need more) gets the
-    same gradients; one byte of statistics less is refused."""
-    q, k, v, go = operands(9, 1, 8, 2, L, L, 128, "bf16")
-    out = tt.sdpAttention(q, k, v, isCausal=True)
-    ref = expected(q, k, v, go, True, None)[1:]
+def test_less_scratch():
+    """A caller whose scratch is less than the divided sums of the short way need, but enough for the kernels of long sequences, gets
+    the same gradients from those; with less it is refused."""
+    B, Hq, Hkv, L, S, D = 3, 4, 2, 100, 160, 64
+    lens = (160, 77, 101)
+    q, k, v, go = operands(9, B, Hq, Hkv, L, S, D, "bf16")
+    n = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out = tt.sdpAttention(q, k, v, isCausal=True, kvLens=n, causalAlign="bottom-right")
+    ref = expected(q, k, v, go, "br", lens)[1:]
     d = [torch.empty_like(x) for x in (q, k, v)]
-    p = build_backward_params(q, k, v, out, go, *d, True, None, None, None, "top-left")
-    need = _capi.lib().ttsdpa_backward_workspace_bytes(ctypes.byref(p))
+    p = build_backward_params(q, k, v, out, go, *d, True, None, None, n, "bottom-right")
+    need, least = _capi.lib().ttsdpa_backward_workspace_bytes(ctypes.byref(p)), 8 * B * Hq * L
+    assert need > 2 * least
     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    ran = 0
-    for size in (need, need // 2, need // 4, 8 * 8 * L - 1):
+    for size, kernel in ((need, "short_joint"), (need - 1, "other"), (least, "other")):
+        assert _capi.backward_kernel(p, size) == kernel
         for x in d:
             x.fill_(7)
-        rc = _capi.lib().ttsdpa_backward(ctypes.byref(p), ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(size), stream)
-        if rc == 0:
-            ran += 1
-            for x, y in zip(d, ref):
-                assert rel_err(x, y) <= REL["bf16"]
-        else:
-            assert rc == _capi.ERR_WORKSPACE
-    assert ran >= 1 and rc == _capi.ERR_WORKSPACE
+        assert _capi.lib().ttsdpa_backward(ctypes.byref(p), ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(size), stream) == 0
+        for x, y in zip(d, ref):
+            assert rel_err(x, y) <= REL["bf16"]
+    assert _capi.lib().ttsdpa_backward(ctypes.byref(p), ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(least - 1), stream) == _capi.ERR_WORKSPACE
