@@ -133,6 +133,7 @@ def test_tiles_of_few_rows(M, N, K, tile):
     # us in 32 x 32 tiles / 16 x 32 ones, of a contraction-major weight
     (16, 8192, 2048, (16, 32)),   # 12.6 / 11.0
     (12, 7928, 2744, (32, 32)),   # 14.4 / 15.3: six units a wavefront
+    (4, 4911, 3321, (16, 32)),    # 15.9 / 13.7
     (8, 5179, 3064, (32, 32)),    # 14.5 / 15.3
     (16, 5179, 3064, (32, 32)),   # 15.2 / 16.1
     (14, 6144, 4096, (16, 32)),

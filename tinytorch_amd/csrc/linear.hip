@@ -1147,13 +1147,12 @@ double mixed_tiles_cost(const LinArgs& a) {
   return 9 * rounds + 6 + large_cold(a) + a.K / 64.0 * (1.5 * rounds + 0.62 + 0.24 * (2 * left) / kCusOfXcd);
 }
 
-// 128 x 128 tiles whose contraction is divided among S workgroups each, one to a CU (of an XCD's: 826 x 1536 x 4160, 84 tiles in 3 shares, 33
-// on some, 36 us; 28 by this) at most: a launch more, and the shares' fp32 sums
-// written and read at 5 TB/s.  What leaves most CUs idle otherwise, or goes to the streaming kernel, which takes in the operands of
-// smaller tiles: 288 x 2048 x 6592, 48 tiles, 34.7 there -> 22.9 in 5 shares; 200 x 4096 x 14336, 64, 74 -> 48 in 4; 720 x 1536 x 4736,
-// 72, 43 -> 24 in 3 (2: 26.6; 5, more than a round: 27.3).  fp32: only what the streaming kernel does not take, contraction-major
-// operands of fewer than 16 rows (6 x 768 x 28672 1740 -> 133).  (Four wavefronts of 64 x 64 instead of eight of 64 x 32, fewer LDS reads: 3 to 8 % slower in every
-// such call.)
+// 128 x 128 tiles whose contraction is divided among S workgroups each, one to a CU (of an XCD's: 826 x 1536 x 4160, 84 tiles in 3 shares,
+// 33 on some, 36 us; 28 by this) at most: a launch more, and the shares' fp32 sums written and read at 5 TB/s.  What leaves most CUs
+// idle otherwise, or goes to the streaming kernel, which takes in the operands of smaller tiles: 288 x 2048 x 6592, 48 tiles, 34.7 there
+// -> 22.9 in 5 shares; 200 x 4096 x 14336, 64, 74 -> 48 in 4; 720 x 1536 x 4736, 72, 43 -> 24 in 3 (2: 26.6; 5, more than a round: 27.3).
+// fp32: only what the streaming kernel does not take, contraction-major operands of fewer than 16 rows (6 x 768 x 28672 1740 -> 133).
+// (Four wavefronts of 64 x 64 instead of eight of 64 x 32, fewer LDS reads: 3 to 8 % slower in every such call.)
 double divided_cost(const LinArgs& a, int dtype, int S) {
   const double esz = dtype == TTSDPA_F32 ? 4 : 2, sums = 5.5 + 8.0 * S * a.M * a.N / 5e6;
   LinArgs share = a;

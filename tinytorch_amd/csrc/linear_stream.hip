@@ -520,10 +520,11 @@ int waves_of_tile(const LinArgs& a, int esz, int R) {
 double tiles_of(const LinArgs& a, int R) { return (double)((a.M + 16 * R - 1) / (16 * R)) * (double)((a.N + 16 * R - 1) / (16 * R)); }
 
 // Wavefronts that share a tile of a call (others, RI: tiles and size of another product in the launch).  A workgroup takes as many tiles
-// as leave none of its wavefronts idle; backward of a layer, us, a tile to a workgroup -> so: fp32 19 x 2048 x 2048 54 -> 20; 16-bit 62 x 1024 x
-// 1024 13.5 -> 6.0.  But where all tiles run side by side there is nothing to gain, and those of a workgroup wait for each other: 16-bit layers of up to 256 tiles 4.2 us a tile to a workgroup, 4.5 in groups; fp32
-// 24 x 512 x 320 5.4 and 7.7, whose 32 x 32 tiles share a CU in pairs, where one unit is all their work or the other product's tiles are of
-// that size too (20 x 40 x 3328, 312 tiles, 5.5 and 7.3; 72 x 576 x 320, 280 tiles of three units and 16-row ones, 6.7 and 6.0).
+// as leave none of its wavefronts idle; backward of a layer, us, a tile to a workgroup -> so: fp32 19 x 2048 x 2048 54 -> 20; 16-bit 62 x
+// 1024 x 1024 13.5 -> 6.0.  But where all tiles run side by side there is nothing to gain, and those of a workgroup wait for each other:
+// 16-bit layers of up to 256 tiles 4.2 us a tile to a workgroup, 4.5 in groups; fp32 24 x 512 x 320 5.4 and 7.7, whose 32 x 32 tiles
+// share a CU in pairs, where one unit is all their work or the other product's tiles are of that size too (20 x 40 x 3328, 312 tiles, 5.5 and
+// 7.3; 72 x 576 x 320, 280 tiles of three units and 16-row ones, 6.8 and 6.1).
 int waves_of_call(const LinArgs& a, int esz, int R, int S, double entries, double others, int RI) {
   const int W = wavefronts(R), G = S > 1 ? 0 : waves_of_tile(a, esz, R);
   if (G == 0) return W;
@@ -617,8 +618,8 @@ StreamPlan plan_tiles(const LinArgs& a, int esz, double entries, bool may_split,
 //                       others                        16 x 16 K 1024 0.75 to 0.85, 2560 0.91, 3072 0.97, 5120 0.98
 //   24 rows x 8704, K 1024, 2048, 4096    8.4, 14.2, 23.5 us -> 7.1, 11.6, 18.6 (32 x 48)
 // k-major w (a layer's input gradient), us, rows x columns x contraction: up to 16 rows in 16 x 32 tiles, 16 x 8192 x 2048 12.6 -> 11.0 (5 x 7839 x 731
-// 6.4 -> 7.2, hence the least contraction; 5850 products by units of a wavefront: 3 and 4 1.10, 5 1.03, 8, 12 and 16 1.03 to 1.04, 6 0.98, 7 1.02 with
-// a tenth of them 0.95 to 0.97, 10 and 14 1.00); 32 x 64 ones where 32 x 32 make one to two rounds, 30 x 11264 x 4096 38 -> 28, 8 x 10880 x 5760 40
+// 6.4 -> 7.2, hence the least contraction; 5850 products by units of a wavefront: 3 and 4 1.10, 8, 12 and 16 1.03 to 1.04, other odd ones 1.02, 6
+// 0.98, 10 and 14 1.00); 32 x 64 ones where 32 x 32 make one to two rounds, 30 x 11264 x 4096 38 -> 28, 8 x 10880 x 5760 40
 // -> 30; 33 to 48 rows in 48 x 64 tiles of eight wavefronts instead of 64 x 64 of four, 42 x 11200 x 4096 28 -> 23, 37 x 17280 x 5120 58 -> 54.
 enum class Tile { Square, Square16, Rows32x48, Rows16x64, Rows16x32, Rows32x64, Rows48x64 };
 Tile few_rows_tile(const LinArgs& a, int R) {
@@ -628,7 +629,7 @@ Tile few_rows_tile(const LinArgs& a, int R) {
     if (a.M > 32 || pieces > 512) return Tile::Square;
     if (pieces > 256) return Tile::Rows32x64;
     const int each = (int)((a.K + 511) / 512);  // units of a wavefront: rings of four
-    return a.M <= 16 && a.K >= 1200 && (each & 3) != 2 && each != 7 ? Tile::Rows16x32 : Tile::Square;
+    return a.M <= 16 && a.K >= 1200 && (each & 3) != 2 ? Tile::Rows16x32 : Tile::Square;
   }
   if (a.xt || a.M > 32 || R != 2) return Tile::Square;
   const long long tiles = (a.N + 31) / 32;
