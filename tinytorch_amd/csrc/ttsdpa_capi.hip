@@ -532,59 +532,48 @@ size_t backward_rows(const ttsdpa_backward_params* p) { return (size_t)p->fwd.B 
 bool backward_log_sums(const ttsdpa_backward_params* p) { return p->fwd.mask_kind != TTSDPA_MASK_NONE || !backward_on_mfma(p); }
 size_t backward_stats_bytes(const ttsdpa_backward_params* p) { return backward_rows(p) * (backward_log_sums(p) ? 3 : 2) * sizeof(float); }
 
-// Scratch layout: the statistics, then (matrix-core pairs with a split query stream) the partial dk / dv, 256-byte aligned.
-int dkv_splits_of(const ttsdpa_backward_params* p, bool* dealt = nullptr) {
-  const ttsdpa_params* f = &p->fwd;
-  bool unused;
-  if (!dealt) dealt = &unused;
-  *dealt = false;
-  if (!backward_on_mfma(p)) return 1;
-  const int groups = f->dtype != TTSDPA_F32 && f->D == 128 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
-  const int per_cu = f->D <= 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
-  return backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, groups, per_cu, backward_on_f32_pair(p), dealt);
-}
-// ... then (matrix-core pairs whose dq kernel splits its key ranges) the partial dq records, 256-byte aligned.
-int dq_splits_of(const ttsdpa_backward_params* p, bool* dealt = nullptr) {
-  const ttsdpa_params* f = &p->fwd;
-  bool unused;
-  if (!dealt) dealt = &unused;
-  *dealt = false;
-  if (!backward_on_mfma(p)) return 1;
-  const bool f32 = backward_on_f32_pair(p);
-  const int slots = f32 && f->D > 64 ? 256 : 512;
-  return backward_dq_splits(f->B, f->Hq, f->L, f->S, f->D, effective_causal(f) != TTSDPA_CAUSAL_NONE, slots, f32, dealt);
-}
+// How the matrix-core pairs divide a call (made once for a call): the dk / dv kernel's query streams and the dq kernel's key ranges.
+struct PairSplits {
+  int dkv = 1, dq = 1;
+  bool dkv_dealt = false, dq_dealt = false;
+  PairSplits(const ttsdpa_backward_params* p) {
+    const ttsdpa_params* f = &p->fwd;
+    if (!backward_on_mfma(p)) return;
+    const bool f32 = backward_on_f32_pair(p), causal = effective_causal(f) != TTSDPA_CAUSAL_NONE;
+    const int groups = f->dtype != TTSDPA_F32 && f->D == 128 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
+    const int per_cu = f->D <= 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
+    dkv = backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, causal, groups, per_cu, f32, &dkv_dealt);
+    dq = backward_dq_splits(f->B, f->Hq, f->L, f->S, f->D, causal, f32 && f->D > 64 ? 256 : 512, f32, &dq_dealt);
+  }
+};
+
+// Scratch layout: the statistics, then (a split query stream) the partial dk / dv, then (split key ranges) the partial dq records,
+// each 256-byte aligned.
 size_t backward_partial_offset(const ttsdpa_backward_params* p) { return (backward_stats_bytes(p) + 255) & ~(size_t)255; }
-size_t backward_dq_partial_offset(const ttsdpa_backward_params* p) {
-  const int n = dkv_splits_of(p);
-  if (n == 1) return backward_partial_offset(p);
-  const size_t end = backward_partial_offset(p) + (size_t)n * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float);
+size_t backward_dq_partial_offset(const ttsdpa_backward_params* p, const PairSplits& n) {
+  if (n.dkv == 1) return backward_partial_offset(p);
+  const size_t end = backward_partial_offset(p) + (size_t)n.dkv * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float);
   return (end + 255) & ~(size_t)255;
 }
 // Estimated time of a call on the matrix-core pairs, by the longest stream of each kernel.
-double pair_backward_us(const ttsdpa_backward_params* p) {
-  const ttsdpa_params* f = &p->fwd;
-  const ShortShape s(f);
+double pair_backward_us(const ttsdpa_params* f, const ShortShape& s, const PairSplits& n) {
   if (!s.f32) {
     const int tiles = (s.keys + 3) / 4, stream = s.group * ((f->L + 31) / 32);
     const double work = s.heads * ((f->L + 127) / 128) * tiles * (s.causal ? 0.6 : 1.0) / 512, row = tiles < 8 ? tiles : 8, st = stream < 32 ? stream : 32;
     return s.wide ? 16.6 + 2.2 * row + 6.9 * work + 0.37 * st : 11.6 + 1.7 * row + 4.3 * work + 0.27 * st;
   }
-  bool dealt;
-  auto us = [&](int n, double wgs, int tiles, double slots, double tile_us) {
+  auto us = [&](int n, bool dealt, double wgs, int tiles, double slots, double tile_us) {
     if (dealt) return ((tiles + 3) / 4 + 0.5) * tile_us;
     const double rounds = (s.causal ? 0.6 : 1.0) * wgs * n / slots;
     return (tiles + n - 1) / n * tile_us * (rounds > 1 ? rounds : 1) + (n > 1 ? 4.5 : 0);
   };
-  const int nk = dkv_splits_of(p, &dealt);
-  const double dkv = us(nk, s.kv * ((f->S + 127) / 128), s.group * ((f->L + 31) / 32), s.wide ? 256 : 512, s.wide ? 10 : 5);
-  const int nq = dq_splits_of(p, &dealt);
-  const double dq = us(nq, s.heads * ((f->L + 127) / 128), (f->S + 31) / 32, s.wide ? 256 : 512, s.wide ? 8 : 4);
+  const double dkv = us(n.dkv, n.dkv_dealt, s.kv * ((f->S + 127) / 128), s.group * ((f->L + 31) / 32), s.wide ? 256 : 512, s.wide ? 10 : 5);
+  const double dq = us(n.dq, n.dq_dealt, s.heads * ((f->L + 127) / 128), (f->S + 31) / 32, s.wide ? 256 : 512, s.wide ? 8 : 4);
   return s.wide ? 18.5 + 0.54 * dq + 1.08 * dkv : 5.5 + 1.5 * dq + 1.0 * dkv;
 }
 
 // The short sequences' backward: splits of its dk / dv workgroups, 0 where the pairs are the shorter way.
-int short_backward_splits(const ttsdpa_backward_params* p, bool* joint = nullptr) {
+int short_backward_splits(const ttsdpa_backward_params* p, const PairSplits& n, bool* joint = nullptr) {
   const ttsdpa_params* f = &p->fwd;
   if (!short_ok(f) || !(backward_mfma_ok(p) || backward_f32_ok(p))) return 0;
   const ShortShape s(f);
@@ -592,7 +581,7 @@ int short_backward_splits(const ttsdpa_backward_params* p, bool* joint = nullptr
   if (joint) *joint = one < two;
   // (the joint launch takes longer than its estimate by a tenth for each round of workgroups beyond the first: with more than three of
   // them it lost up to 24 %, 256 heads x 64 x 64 fp32 34.9 us on the pairs, 45.6 here; bf16 x 75 24.3 and 28.2)
-  const double us = one < two ? one : two, pair = pair_backward_us(p), rounds = s.heads * s.rows / 256;
+  const double us = one < two ? one : two, pair = pair_backward_us(f, s, n), rounds = s.heads * s.rows / 256;
   const bool padded = s.wide && f->D <= 96;  // (of 128 columns: less than the estimate, 64 heads x 111 x 80 18.0 us, 27.4 on the pairs)
   if (one < two && rounds > 1 && !padded && us * (1 + 0.1 * (rounds - 1)) >= 0.85 * pair) return 0;
   return us < s.least_margin() * pair ? s.splits() : 0;
@@ -602,18 +591,17 @@ size_t short_backward_bytes(const ttsdpa_backward_params* p, int splits) {
 }
 
 // ... with that much scratch (less than the query asks for: the pairs).
-int short_backward_taken(const ttsdpa_backward_params* p, size_t workspace_bytes, bool* joint) {
-  const int n = short_backward_splits(p, joint);
+int short_backward_taken(const ttsdpa_backward_params* p, const PairSplits& pair, size_t workspace_bytes, bool* joint) {
+  const int n = short_backward_splits(p, pair, joint);
   return n > 0 && workspace_bytes >= short_backward_bytes(p, n) ? n : 0;
 }
 
 // of the pairs
-size_t backward_scratch_bytes(const ttsdpa_backward_params* p) {
-  const int n = dkv_splits_of(p), nq = dq_splits_of(p);
-  if (nq > 1)
-    return backward_dq_partial_offset(p) + (size_t)nq * p->fwd.B * p->fwd.Hq * p->fwd.L * (p->fwd.D + 2) * sizeof(float);
-  if (n == 1) return backward_stats_bytes(p);
-  return backward_partial_offset(p) + (size_t)n * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float);
+size_t backward_scratch_bytes(const ttsdpa_backward_params* p, const PairSplits& n) {
+  if (n.dq > 1)
+    return backward_dq_partial_offset(p, n) + (size_t)n.dq * p->fwd.B * p->fwd.Hq * p->fwd.L * (p->fwd.D + 2) * sizeof(float);
+  if (n.dkv == 1) return backward_stats_bytes(p);
+  return backward_partial_offset(p) + (size_t)n.dkv * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float);
 }
 
 int check_grid(long long nwg) { return nwg > 0x7fffffffLL ? TTSDPA_ERR_SHAPE : TTSDPA_OK; }
@@ -869,7 +857,7 @@ int ttsdpa_backward_kernel(const ttsdpa_backward_params* p, size_t workspace_byt
   const int rc = validate_backward(p, &a);
   if (rc != TTSDPA_OK) return rc;
   bool joint = false;
-  const int n = pick_backward_route(p) == TTSDPA_ROUTE_NONE ? 0 : short_backward_taken(p, workspace_bytes, &joint);
+  const int n = pick_backward_route(p) == TTSDPA_ROUTE_NONE ? 0 : short_backward_taken(p, PairSplits(p), workspace_bytes, &joint);
   if (kind) *kind = n == 0 ? TTSDPA_KERNEL_OTHER : joint ? TTSDPA_KERNEL_SHORT_JOINT : TTSDPA_KERNEL_SHORT;
   return TTSDPA_OK;
 }
@@ -877,8 +865,9 @@ int ttsdpa_backward_kernel(const ttsdpa_backward_params* p, size_t workspace_byt
 size_t ttsdpa_backward_workspace_bytes(const ttsdpa_backward_params* p) {
   BwdArgs a;
   if (validate_backward(p, &a) != TTSDPA_OK) return 0;
-  const size_t pairs = backward_scratch_bytes(p);
-  const int n = short_backward_splits(p);
+  const PairSplits pair(p);
+  const size_t pairs = backward_scratch_bytes(p, pair);
+  const int n = short_backward_splits(p, pair);
   const size_t own = n > 0 ? short_backward_bytes(p, n) : 0;
   return own > pairs ? own : pairs;
 }
@@ -889,20 +878,21 @@ int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t wor
   if (rc != TTSDPA_OK) return rc;
   const int route = pick_backward_route(p);
   if (route == TTSDPA_ROUTE_NONE) return TTSDPA_OK;
-  const size_t need = backward_scratch_bytes(p);
+  const PairSplits pair(p);
+  const size_t need = backward_scratch_bytes(p, pair);
   if (need > 0 && (!workspace || workspace_bytes < need || !ptr_aligned(workspace, 16))) return TTSDPA_ERR_WORKSPACE;
   a.stats = (float*)workspace;
   a.log_sums = backward_log_sums(p) ? a.stats + 2 * backward_rows(p) : nullptr;
   bool joint = false;
-  const int n = short_backward_taken(p, workspace_bytes, &joint);
+  const int n = short_backward_taken(p, pair, workspace_bytes, &joint);
   if (n > 0) {
     a.dkv_splits = n, a.partial = n > 1 ? (float*)((char*)workspace + backward_partial_offset(p)) : nullptr;
     return launch_short_backward(a, p->fwd.dtype, joint, (hipStream_t)stream);
   }
-  a.dkv_splits = dkv_splits_of(p, &a.dkv_dealt);
+  a.dkv_splits = pair.dkv, a.dkv_dealt = pair.dkv_dealt;
   a.partial = a.dkv_splits > 1 ? (float*)((char*)workspace + backward_partial_offset(p)) : nullptr;
-  a.dq_splits = dq_splits_of(p, &a.dq_dealt);
-  a.dq_partial = a.dq_splits > 1 ? (float*)((char*)workspace + backward_dq_partial_offset(p)) : nullptr;
+  a.dq_splits = pair.dq, a.dq_dealt = pair.dq_dealt;
+  a.dq_partial = a.dq_splits > 1 ? (float*)((char*)workspace + backward_dq_partial_offset(p, pair)) : nullptr;
   if (backward_on_mfma(p)) {
     const long long g1 = (long long)a.f.B * a.f.Hq * ((a.f.L + 127) / 128) * a.dq_splits, g2 = (long long)a.f.B * a.f.Hkv * ((a.f.S + 127) / 128);
     if (check_grid(g1) != TTSDPA_OK || check_grid(g2) != TTSDPA_OK) return TTSDPA_ERR_SHAPE;
