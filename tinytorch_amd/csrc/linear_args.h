@@ -20,8 +20,8 @@ struct LinArgs {
   // among `splits` workgroups per tile, whose sums go to part ([splits][M*N + M] floats) to be added by another kernel
   void* rowsum = nullptr;
   int splits = 1;
-  float* part = nullptr;
   int tile_waves = 0;  // linear_stream.hip: wavefronts that share a tile (0: a workgroup's all)
+  float* part = nullptr;
 };
 
 // linear_stream.hip: products whose wavefronts divide the contraction among themselves, for any alignment of the operands.
