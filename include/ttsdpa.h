@@ -137,14 +137,15 @@ void ttsdpa_params_init(ttsdpa_params* p, int dtype, int B, int Hq, int Hkv, int
  * needs no GPU.  Plays the role of the reference's shape checks before a device op (src/Operation/OpLinalg.cpp:62-89). */
 int ttsdpa_plan(const ttsdpa_params* p, int* route);
 
-/* Within a route, the kernels for short sequences that *p (ttsdpa_backward_kernel: with that much scratch) runs on, or OTHER: the
- * route's kernels for long ones.  Estimates decide: the answer may change with the library.  Launches nothing and needs no GPU. */
+/* Within a route, the kernels for short or unevenly long calls that *p (ttsdpa_backward_kernel: with that much scratch) runs on, or
+ * OTHER: the route's kernels for long ones.  Estimates decide: the answer may change with the library.  Launches nothing and needs no GPU. */
 enum ttsdpa_kernel_kind {
   TTSDPA_KERNEL_OTHER = 0,
   TTSDPA_KERNEL_SHORT = 1,       /* 16 rows or keys a workgroup; backward: dq, then dk and dv */
   TTSDPA_KERNEL_SHORT_JOINT = 2, /* backward: all gradients in one launch */
   TTSDPA_KERNEL_HEADS_16 = 3,    /* with an attnMask, a head's K and V in LDS at once; 16 rows a wavefront */
-  TTSDPA_KERNEL_HEADS_32 = 4     /* 32 */
+  TTSDPA_KERNEL_HEADS_32 = 4,    /* 32 */
+  TTSDPA_KERNEL_DEALT = 5        /* 128 rows a workgroup, their keys dealt out to two groups of wavefronts */
 };
 int ttsdpa_kernel(const ttsdpa_params* p, int* kind);
 

@@ -32,7 +32,7 @@ EXPORTS = [
 ]
 LINEAR_ROUTE_NAMES = {0: "none", 1: "mfma", 2: "general"}
 LINEAR_WAY_NAMES = {0: "general", 1: "stream", 2: "in_place", 3: "tiled", 4: "outer"}
-KERNEL_NAMES = {0: "other", 1: "short", 2: "short_joint", 3: "heads_16", 4: "heads_32"}
+KERNEL_NAMES = {0: "other", 1: "short", 2: "short_joint", 3: "heads_16", 4: "heads_32", 5: "dealt"}
 LINEAR_TILES_NAMES = {0: "other", 1: "128x128", 2: "256x256", 3: "128x256", 4: "mixed"}
 
 

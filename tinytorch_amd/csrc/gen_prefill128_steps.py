@@ -27,6 +27,9 @@ key is visible iff kvs + 8*(n/4) + n%4 <= rl: two more instructions per score, a
 select).  The second form serves the one or two tiles of a wavefront's row group that touch the diagonal; it sits out
 of line, in subsection 1 of the kernel's section, so that the steady state falls through without a taken branch.
 
+The dealt kernel (sdpa_prefill_dealt.hip) has rings of two tiles, four halves, for K and for V: TT_P128_DSTEP_..._N<n> takes the
+half in place n (V; K two places on).
+
 Calls with a Bool attnMask have a third form of the plain step, TT_P128_MSTEP_... (TT_P64_MSTEP_...): a score's probability is
 kept iff its mask byte is set (a compare on one byte of a register through SDWA and a select: two more instructions per
 score).  A lane's 16 mask bytes of a 32-key half are four dwords (keys 8g + 4*(lane/32) .. +3 of the lane's query row, g = 0..3) in
@@ -63,13 +66,13 @@ def vr(lo, n=1):
     return "v%d" % lo if n == 1 else "v[%d:%d]" % (lo, lo + n - 1)
 
 
-def fetch(G):
-    """LDS operand request of slot G of the 4-tile body into its ring place."""
-    G %= BODY
+def fetch(G, stages=4):
+    """LDS operand request of slot G of the body (a tile per stage) into its ring place."""
+    G %= BODY * stages // 4
     u, kind, s = G // (2 * NS), (G // NS) % 2, G % NS
     i, r = s >> 1, RING0 + 4 * (G % RING)
     if s % 2 == 0:  # K rows of half `kind` of tile u+1, k-step i
-        off = ((u + 1) & 3) * STAGE + kind * 32 * ROW
+        off = ((u + 1) % stages) * STAGE + kind * 32 * ROW
         return ["ds_read_b128 %s, %s offset:%d" % (vr(r, 4), vr(KADDR0 + i), off)]
     t, db = i // NDB, i % NDB  # V^T of half `kind` of tile u, keys 16t..16t+15, head_dim block db
     off = u * STAGE + kind * 32 * ROW + 16 * t * ROW
@@ -82,7 +85,7 @@ def pending_after(G):
     return sum(len(fetch(g)) for g in range(G + 1, G + PD))
 
 
-def step(u, kind, elem, masked=False, bmask=False):
+def step(u, kind, elem, masked=False, bmask=False, stages=4):
     mfma = "v_mfma_f32_32x32x16_%s" % elem
     cvt = "v_cvt_pk_%s_f32" % elem
     G0 = 2 * NS * u + NS * kind
@@ -132,7 +135,7 @@ def step(u, kind, elem, masked=False, bmask=False):
         else:
             i = n // 2
             out.append("%s %%[o%d], %s, %s, %%[o%d]" % (mfma, i % NDB, vr(r, 4), vr(p_cur + 4 * (i // NDB), 4), i % NDB))
-        out += fetch(G + PD)  # directly behind the matrix instruction: measured 0.7% faster than behind the vector work
+        out += fetch(G + PD, stages)  # directly behind the matrix instruction: measured 0.7% faster than behind the vector work
         for q in range(SPS * n, SPS * (n + 1)):
             out += vector_work(q)
     if not masked:
@@ -181,7 +184,7 @@ def main():
     lab = ".Ltt_%s" % NAME.lower()
     print("// Generated by gen_prefill128_steps.py%s; do not edit.  Instruction streams of the pipelined prefill kernel's" % ("" if head_dim == 128 else " %d" % head_dim))
     print("// steady state: TT_%s_STEP_<elem>_U<tile of the unrolled body>_K<step of the tile> (with the causal variant out of" % NAME)
-    print("// line), TT_%s_PSTEP_... the plain step alone." % NAME)
+    print("// line), TT_%s_PSTEP_... the plain step alone; TT_%s_DSTEP_<elem>_N<half>, TT_%s_DPSTEP_...: the same on rings of four halves." % (NAME, NAME, NAME))
     print()
     emit("TT_%s_PREFETCH" % NAME, prefetch())
     for elem in ("bf16", "f16"):
@@ -194,6 +197,12 @@ def main():
                 emit("TT_%s_STEP_%s_U%d_K%d" % (NAME, elem.upper(), u, kind), both)
                 emit("TT_%s_PSTEP_%s_U%d_K%d" % (NAME, elem.upper(), u, kind), step(u, kind, elem))  # calls without a causal mask
                 emit("TT_%s_MSTEP_%s_U%d_K%d" % (NAME, elem.upper(), u, kind), step(u, kind, elem, bmask=True))  # Bool attnMask
+        for n in range(4):  # the dealt kernel's ring of four halves
+            u, kind = n // 2, n % 2
+            both = (["s_cmp_eq_u32 %[mk], 0", "s_cbranch_scc0 %s_m%%=" % lab] + step(u, kind, elem, stages=2) + ["%s_e%%=:" % lab, ".subsection 1", "%s_m%%=:" % lab]
+                    + step(u, kind, elem, True, stages=2) + ["s_branch %s_e%%=" % lab, ".subsection 0"])
+            emit("TT_%s_DSTEP_%s_N%d" % (NAME, elem.upper(), n), both)
+            emit("TT_%s_DPSTEP_%s_N%d" % (NAME, elem.upper(), n), step(u, kind, elem, stages=2))
     emit("TT_%s_MDMA" % NAME, mask_dma())
     # before the first step of a workgroup (tile index a multiple of 4: ring place 0): the half it takes, half 1 of that tile
     # (waited for at once: the first tile's own loads go to the same ring place)

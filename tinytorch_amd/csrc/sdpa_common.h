@@ -66,6 +66,7 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -580,6 +581,7 @@ int launch_general(const KArgs& a, int dtype, hipStream_t stream);
 int launch_prefill(const KArgs& a, int dtype, hipStream_t stream);       // 128-row workgroups; head_dim 64 or 128
 int launch_prefill_d128(const KArgs& a, int dtype, hipStream_t stream);  // 256-row workgroups, pipelined; head_dim 128
 int launch_prefill_d64(const KArgs& a, int dtype, hipStream_t stream);   // the same at head_dim 64 (no attnMask, no pages)
+int launch_prefill_dealt(const KArgs& a, int dtype, hipStream_t stream);  // 128-row workgroups, keys dealt out to two groups of wavefronts; head_dim 128 or 64
 int launch_prefill_f32(const KArgs& a, hipStream_t stream);              // fp32 tensors on the fp32 matrix cores; head_dim 64 or 128
 // key tiles (of 32) that an unsplit launch takes one after the other; dealt: its wavefronts share a row tile's
 double prefill_f32_tiles(const KArgs& a, bool* dealt = nullptr);

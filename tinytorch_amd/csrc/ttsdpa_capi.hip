@@ -245,7 +245,7 @@ int tile_width(int dtype, int D) {
 // 18 -> 12 us, 2 x 8 x 927 rows, head_dim 80, 128 workgroups 37 -> 33).
 SplitPlan plan_prefill_splits(const ttsdpa_params* p, const KArgs& a /* after packing */) {
   const bool f32 = p->dtype == TTSDPA_F32;
-  if (!f32 && pipelined_ok(p)) return SplitPlan{1, 0, 0};
+  if (!f32 && (pipelined_ok(p) || pipelined64_ok(p))) return SplitPlan{1, 0, 0};
   const int W = tile_width(p->dtype, a.D);
   const long long heads = (long long)a.B * a.Hq, wgs = heads * ((a.L + 127) / 128);
   const double us = f32 ? (W == 64 ? 2.7 : 4.6) : W <= 64 ? 1.8 : W <= 128 ? 2.2 : 4.0;
@@ -277,14 +277,17 @@ struct SplitCost {
     if (last > longest_rest) longest_rest = last;
     if (tiles > chunk) records += count * (pieces + (last > 0));
   }
-  double us() const {
+  double longest() const {  // a CU's tiles
     const double rounds = ceil(whole / 256), room = 256 * rounds - whole, left = rest - room * chunk;
     double tiles = rounds * chunk;
     if (rests > room) {  // the longest of them go first: lengths taken to be spread evenly, or all the same
       const double spread = 2 * rest / rests * (1 - room / rests), longest = spread < longest_rest ? spread : longest_rest;
       tiles += left / 256 > longest ? left / 256 : longest;
     }
-    const double busy = (whole * chunk + rest) / (256 * tiles);
+    return tiles;
+  }
+  double us() const {
+    const double tiles = longest(), busy = (whole * chunk + rest) / (256 * tiles);
     const double many = 12 + 0.035 * records, few = 6 + 0.1 * records;
     return tiles * (1.4 + 0.45 * busy) + (records > 0 ? (few < many ? few : many) : 0);
   }
@@ -321,6 +324,92 @@ SplitPlan plan_pipelined_splits(const ttsdpa_params* p) {
   if (s.splits < 2) return SplitPlan{1, 0, 0};
   s.ws_bytes = split_record_bytes(heads, p->L, s.splits, p->D);
   return s;
+}
+
+// ---- 256 rows to a workgroup, or 128 with the keys dealt out (sdpa_prefill_dealt.hip) ------------------------------------------
+// What a launch of either kernel takes, us, from the lengths of its row tiles (in 64 keys: a tile of the one, a step of both groups of
+// the other).  Fitted to 600 calls (1 to 8 sequences, 1 to 64 query heads, 129 to 8192 rows on as many keys or a chunk's on up to 16384,
+// paged or not, causal or not); they miss by 4 to 7 % on average.  A workgroup costs `start` lengths beside its own (its launch, the
+// first loads, the output), which shows where a CU has several; a length costs `each`, and `busy` more where all CUs are at work (power).
+struct PipelinedCost {
+  double base, each, busy, start;              // undivided launches
+  double split_base, split_each, split_busy, split_more, record;  // divided keys: with the merge's launch; per round beyond the first; per record
+};
+constexpr PipelinedCost kRows256[2] = {{7.2, 0.74, 0.30, 6, 11.2, 0.63, 0.33, 0.0, 0.027}, {8.9, 1.02, 0.58, 7, 14.9, 0.60, 0.83, 8.2, 0.039}};
+constexpr PipelinedCost kRows128[2] = {{6.6, 0.47, 0.09, 10, 8.2, 0.53, 0.0, 1.9, 0.027}, {7.6, 0.68, 0.20, 9, 11.8, 0.69, 0.17, 4.0, 0.026}};
+
+// Row tiles of `rows` rows, longest first: length of the t-th, and of all.
+struct RowTiles {
+  int rows, ntile, S, offset, L;
+  bool causal;
+  long long heads, sum = 0;
+  RowTiles(const ttsdpa_params* p, int rows_) : rows(rows_), ntile((p->L + rows_ - 1) / rows_), S(p->S), L(p->L), heads((long long)p->B * p->Hq) {
+    const int c = effective_causal(p);
+    causal = c != TTSDPA_CAUSAL_NONE, offset = c == TTSDPA_CAUSAL_BOTTOM_RIGHT && S > L ? S - L : 0;
+    if (!causal) sum = heads * ntile * length(0);
+    else
+      for (int t = 0; t < ntile; t++) sum += heads * length(t);
+  }
+  int length(int t) const {
+    long long last = S;
+    if (causal) {
+      const long long end = (long long)rows * (ntile - t), v = (end < L ? end : L) + offset;
+      last = v < last ? v : last;
+    }
+    return (int)((last + 63) / 64);
+  }
+  double whole_us(const PipelinedCost& c) const {
+    const long long n = heads * ntile, rounds = (n + 255) / 256, pairs = heads * ((ntile + 1) / 2), pair_rounds = (pairs + 255) / 256;
+    double longest = length(0);
+    if (n > 256) {
+      if (!causal) longest = rounds * longest + (rounds - 1) * c.start;
+      else if (rows == 256 && ntile > 1 && pairs >= 256 && pairs * 10 >= pair_rounds * 256 * 9)  // mirrored pairs (launch_prefill_d128)
+        longest = pair_rounds * (longest + length(ntile - 1) + c.start) - c.start;
+      else {
+        // the CU with the shortest of the first 256 takes the next one
+        const double next = n <= 512 ? length((int)(255 / heads)) + length((int)(256 / heads)) + c.start
+                                     : sum / 256.0 + 0.5 * length(ntile - 1) + c.start * (n / 256.0 - 1);
+        longest = next > longest ? next : longest;
+      }
+    }
+    return c.base + c.each * longest + c.busy * sum / 256.0;
+  }
+  // with pieces of `chunk` (64 keys); 0: none that is shorter than the longest row tile
+  double split_us(const PipelinedCost& c, int chunk) const {
+    SplitCost s{(double)chunk};
+    for (int t = ntile - 1; t >= 0; t--) s.add((double)heads, length(t));
+    const double pieces = (s.whole + s.rests) / 256 - 1;
+    return c.split_base + c.split_each * s.longest() + c.split_busy * (s.whole * chunk + s.rest) / 256 + (pieces > 0 ? c.split_more * pieces : 0) + c.record * s.records;
+  }
+};
+
+// The call's way through the pipelined kernels: which of them, and the division of its keys.  dealt: the kernel of 128-row workgroups, with
+// the number of pieces that is shortest there, where that is shorter by these estimates: 2 x 8 x 756 rows, head_dim 128, causal 24.3 -> 16.5
+// us, 16 x 1327 34.4 -> 22.9, 32 x 1539 41 -> 33, 6 x 32 x 326 on 3781 keys, paged, 162 -> 126; head_dim 64, 4 x 8 x 727 18.1 -> 12.8.  Where
+// row tiles fill the chip evenly its keys cost more (2 x 32 x 4096, no mask, 454 and 511): a barrier for 32 of them.
+struct PipelinedPlan {
+  bool dealt;
+  SplitPlan split;
+};
+PipelinedPlan plan_pipelined(const ttsdpa_params* p, bool divided = true, double* us = nullptr) {
+  PipelinedPlan plan{false, divided ? plan_pipelined_splits(p) : SplitPlan{1, 0, 0}};
+  if (p->dtype == TTSDPA_F32 || p->mask_kind != TTSDPA_MASK_NONE || !(pipelined_ok(p) || pipelined64_ok(p)) || p->S < 1) return plan;
+  const RowTiles wide(p, 256), narrow(p, 128);
+  const PipelinedCost &c256 = kRows256[p->D == 128], &c128 = kRows128[p->D == 128];
+  double least = plan.split.splits > 1 ? wide.split_us(c256, plan.split.chunk / 64) : wide.whole_us(c256);
+  const double whole = narrow.whole_us(c128);
+  // (sequences of unlike lengths: the estimates take them all for the longest, which is too much for a divided launch)
+  if (whole < (p->kv_len && p->B > 1 ? 0.9 : 0.95) * least) least = whole, plan.dealt = true, plan.split = SplitPlan{1, 0, 0};
+  const int longest = narrow.length(0);
+  for (int n = 2; divided && n <= 16 && narrow.heads * narrow.ntile * n <= 1024; n++) {
+    const int chunk = ((longest + n - 1) / n + 3) & ~3;
+    if ((longest + chunk - 1) / chunk < n) continue;  // the same as fewer
+    const double t = narrow.split_us(c128, chunk);
+    if (t < (plan.dealt ? 1.0 : 0.95) * least)
+      least = t, plan.dealt = true, plan.split = SplitPlan{n, 64 * chunk, split_record_bytes(narrow.heads, p->L, n, p->D)};
+  }
+  if (us) *us = least;
+  return plan;
 }
 
 // ---- short sequences (sdpa_short.hip) -----------------------------------------------------------------------------------
@@ -436,7 +525,9 @@ bool short_forward_best(const ttsdpa_params* p, const KArgs& a) {
   const ShortShape s(p);
   bool dealt = false;
   const double tiles = s.f32 ? prefill_f32_tiles(a, &dealt) : 0;
-  return s.forward_us() < s.least_margin() * s.other_forward_us(tiles) && !(s.f32 && s.forward_misses(p, tiles, dealt));
+  if (s.forward_us() >= s.least_margin() * s.other_forward_us(tiles) || (s.f32 && s.forward_misses(p, tiles, dealt))) return false;
+  double pipelined = 0;
+  return s.f32 || !plan_pipelined(p, true, &pipelined).dealt || s.forward_us() < pipelined;
 }
 
 int pick_route(const ttsdpa_params* p) {
@@ -696,7 +787,7 @@ size_t ttsdpa_workspace_bytes(const ttsdpa_params* p) {
     if (pack_heads_ok(p)) pack_heads(&a);
     size_t split = plan_prefill_splits(p, a).ws_bytes;
     need = split > need ? split : need;
-    split = plan_pipelined_splits(p).ws_bytes;
+    split = plan_pipelined(p).split.ws_bytes;
     need = split > need ? split : need;
   }
   return need;
@@ -736,23 +827,18 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
   if (kind != TTSDPA_KERNEL_OTHER) return launch_heads(a, p->dtype, (hipStream_t)stream);
   // head_dim 128 with enough rows to fill 256-row workgroups takes the software-pipelined kernel (its tile loads
   // address 64 rows with 32-bit byte offsets)
-  if (p->dtype != TTSDPA_F32 && pipelined_ok(p)) {
-    const SplitPlan sp = plan_pipelined_splits(p);
-    if (sp.splits > 1 && workspace && workspace_bytes >= sp.ws_bytes && ptr_aligned(workspace, 16)) {
-      a.kv_splits = sp.splits, a.kv_chunk = sp.chunk, a.ws = (float*)workspace;
-      if ((rc = check_grid((long long)a.B * a.Hq * ((a.L + 255) / 256 + 8) * sp.splits)) != TTSDPA_OK) return rc;
-      return launch_prefill_d128(a, p->dtype, (hipStream_t)stream);  // the kernel and the merge of its records
-    }
-    a.kv_splits = 1, a.kv_chunk = 0, a.ws = nullptr;
-    return launch_prefill_d128(a, p->dtype, (hipStream_t)stream);
-  }
-  if (p->dtype != TTSDPA_F32 && pipelined64_ok(p)) {
-    const SplitPlan sp = plan_pipelined_splits(p);
-    if (sp.splits > 1 && workspace && workspace_bytes >= sp.ws_bytes && ptr_aligned(workspace, 16))
-      a.kv_splits = sp.splits, a.kv_chunk = sp.chunk, a.ws = (float*)workspace;
-    else
+  if (p->dtype != TTSDPA_F32 && (pipelined_ok(p) || pipelined64_ok(p))) {
+    PipelinedPlan plan = plan_pipelined(p);
+    if (plan.split.splits > 1 && !(workspace && workspace_bytes >= plan.split.ws_bytes && ptr_aligned(workspace, 16))) plan = plan_pipelined(p, false);
+    if (plan.split.splits > 1) {
+      a.kv_splits = plan.split.splits, a.kv_chunk = plan.split.chunk, a.ws = (float*)workspace;
+      if ((rc = check_grid((long long)a.B * a.Hq * ((a.L + (plan.dealt ? 127 : 255)) / (plan.dealt ? 128 : 256) + 8) * a.kv_splits)) != TTSDPA_OK) return rc;
+    } else {
       a.kv_splits = 1, a.kv_chunk = 0, a.ws = nullptr;
-    return launch_prefill_d64(a, p->dtype, (hipStream_t)stream);  // with splits: the kernel and the merge of its records
+    }
+    // with splits: the kernel and the merge of its records
+    if (plan.dealt) return launch_prefill_dealt(a, p->dtype, (hipStream_t)stream);
+    return p->D == 128 ? launch_prefill_d128(a, p->dtype, (hipStream_t)stream) : launch_prefill_d64(a, p->dtype, (hipStream_t)stream);
   }
   if (f32_decode_ok(p)) {
     const DecodePlan pl = plan_decode(a);
@@ -830,7 +916,9 @@ int ttsdpa_kernel(const ttsdpa_params* p, int* kind) {
   const int route = pick_route(p);
   a.full_p = full_probabilities(p);
   const bool prefill = route == TTSDPA_ROUTE_PREFILL || (route == TTSDPA_ROUTE_GENERAL && p->mask_kind != TTSDPA_MASK_NONE && prefill_ok(p, true));
-  if (kind) *kind = prefill ? short_kernel_of(p, a) : TTSDPA_KERNEL_OTHER;
+  int k = prefill ? short_kernel_of(p, a) : TTSDPA_KERNEL_OTHER;
+  if (prefill && k == TTSDPA_KERNEL_OTHER && plan_pipelined(p).dealt) k = TTSDPA_KERNEL_DEALT;
+  if (kind) *kind = k;
   return TTSDPA_OK;
 }
 
