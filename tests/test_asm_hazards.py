@@ -12,7 +12,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "tinytorch_amd", "csrc")
-SOURCES = ["sdpa_prefill_d128.hip", "sdpa_prefill_d64.hip", "sdpa_prefill_dealt.hip", "sdpa_backward_mfma.hip", "linear.hip"]
+SOURCES = ["sdpa_prefill_d128.hip", "sdpa_prefill_d64.hip", "sdpa_prefill_dealt.hip", "sdpa_backward_mfma.hip", "sdpa_backward_d128.hip", "linear.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 

@@ -1,4 +1,4 @@
-"""The generated instruction streams kept in the tree (prefill128_steps.inc, prefill64_steps.inc, linear256_loop.inc,
+"""The generated instruction streams kept in the tree (prefill128_steps.inc, prefill64_steps.inc, backward128_steps.inc, linear256_loop.inc,
 linear128_loop.inc) are what their generators write today: an edit to a generator without a regeneration would otherwise ship a stale kernel
 silently.  CPU only."""
 import os
@@ -14,6 +14,7 @@ CSRC = os.path.join(ROOT, "tinytorch_amd", "csrc")
 @pytest.mark.parametrize("generator, args, inc", [
     ("gen_prefill128_steps.py", [], "prefill128_steps.inc"),
     ("gen_prefill128_steps.py", ["64"], "prefill64_steps.inc"),
+    ("gen_backward128_steps.py", [], "backward128_steps.inc"),
     ("gen_linear256_loop.py", [], "linear256_loop.inc"),
     ("gen_linear256_loop.py", ["128"], "linear128_loop.inc"),
 ])

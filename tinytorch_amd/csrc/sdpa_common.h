@@ -518,6 +518,7 @@ int launch_backward_dq_merge(const BwdArgs& a, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 int launch_backward_general(const BwdArgs& a, int dtype, hipStream_t stream);
+int launch_backward_dq_d128(const BwdArgs& a, bool bf16, hipStream_t stream);  // its dq kernel at head_dim 128 without an attnMask
 int launch_backward_mfma(const BwdArgs& a, int dtype, hipStream_t stream);  // fp16/bf16, head_dim 64 or 128
 int launch_backward_f32(const BwdArgs& a, int dtype, hipStream_t stream);   // on the fp32 matrix cores, head_dim 64 or 128: fp32, and fp16/bf16 with an attnMask
 
