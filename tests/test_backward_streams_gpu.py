@@ -1,4 +1,4 @@
-"""The 16-bit backward pair's streams (sdpa_backward_d128.hip): key counts around its tiles of 32 and
+"""The 16-bit backward pair's streams and splits (sdpa_backward_d128.hip, backward_splits_16bit): key counts around its tiles of 32 and
 its two steps at a time, row tiles whose wavefronts end at different tiles, maxima that rise on the way, and numbers of splits
 that are no power of two over more workgroups than run side by side.  All three gradients against float64."""
 import ctypes
@@ -74,3 +74,11 @@ def test_dq_stream(case, dtype):
 def test_maxima_that_rise(dtype):
     """Scores with a standard deviation of 7: the running maximum is raised within the streams."""
     check((1, 8, 4, 1100, 1100, True, TL), dtype, 128, mul=0.8 * (1024 / 128) ** 0.25, rel=2.0)  # (dS differs from its sum's terms by more)
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("case", [(4, 56, 8, 383, 383, True, TL), (4, 32, 4, 909, 909, True, TL), (2, 32, 8, 700, 700, True, TL)],
+                         ids=lambda c: "B%dH%dk%dL%dS%d-c%d-%s" % c)
+def test_splits_of_a_key_block_walk_alike(case, D):
+    """Causal calls of a multiple of eight (batch, KV head) pairs, whose workgroups walk their tiles in alternating directions."""
+    check(case, "bf16", D)

@@ -436,7 +436,7 @@ __global__ __launch_bounds__(256, (D > 64 || MASKED || DEAL ? 1 : 2)) void backw
   if (CAUSAL) it0 = (k0 - coff > 0 ? k0 - coff : 0) / BT;
   const int nt = ntq > it0 ? ntq - it0 : 0;
   const int total = f.G * nt;
-  const bool walk_up = dkv_walks_up(a, CAUSAL);  // every second round of an XCD's workgroups (sdpa_common.h)
+  const bool walk_up = dkv_walks_up(a, CAUSAL, wg);  // every second round of an XCD's workgroups (sdpa_common.h)
   auto tile_of = [&](int idx) __attribute__((always_inline)) { return walk_up ? it0 + idx / f.G : ntq - 1 - idx / f.G; };
 
   Row4<E> qst[NLD], gst[NLD];

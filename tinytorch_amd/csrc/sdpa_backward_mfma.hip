@@ -466,7 +466,7 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dkv_mfma_kerne
   if (CAUSAL) it0 = (k0 - coff > 0 ? k0 - coff : 0) / BQ;
   const int nt = ntq > it0 ? ntq - it0 : 0;
   const int total = f.G * nt;
-  const bool walk_up = dkv_walks_up(a, CAUSAL);  // every second round of an XCD's workgroups (sdpa_common.h)
+  const bool walk_up = dkv_walks_up(a, CAUSAL, wg);  // every second round of an XCD's workgroups (sdpa_common.h)
   auto tile_of = [&](int idx) __attribute__((always_inline)) { return walk_up ? it0 + idx / f.G : ntq - 1 - idx / f.G; };
 
   u32x4 qst[NLD], gst[NLD];
@@ -721,7 +721,7 @@ __global__ __launch_bounds__(512, 1) void backward_dkv128_kernel(BwdArgs a) {
   const int nt = ntq > it0 ? ntq - it0 : 0;
   const int total = split < f.G * nt ? (f.G * nt - split + nsplit - 1) / nsplit : 0;
   const int niter = (total + 1) / 2;  // iterations of either group (the second may have one entry less)
-  const bool walk_up = dkv_walks_up(a, CAUSAL);  // every second round of an XCD's workgroups (sdpa_common.h)
+  const bool walk_up = dkv_walks_up(a, CAUSAL, wg);  // every second round of an XCD's workgroups (sdpa_common.h)
   auto tile_of = [&](int entry) __attribute__((always_inline)) { return walk_up ? it0 + entry / f.G : ntq - 1 - entry / f.G; };
 
   // wavefront gw of a group brings rows 8gw .. 8gw+7 of the Q tile and of the dout tile (two loads each) into the

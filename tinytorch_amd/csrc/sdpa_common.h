@@ -387,6 +387,53 @@ inline int backward_dq_splits(int B, int Hq, int L, int S, int D, bool causal, i
   return *dealt ? 1 : n;
 }
 
+// Splits of the 16-bit pair's kernels at head_dim 64 and 128 without an attnMask.  A launch of n splits takes, us, `launch` + a tile's time
+// times the longest chain of tiles that a place for a workgroup runs, + (n > 1) the second launch and the partial records at `per_mb`.
+// Fitted to 480 calls of 1 to 8 sequences, 1 to 64 heads, 100 to 4096 rows with the number of either kernel forced to 1 .. 8
+// (the estimates' differences miss by 4 to 8 % of the call's time; the numbers they choose give 1 % less than the best ones).
+// Records cost more than an uneven end: 4 x 8 heads x 1545 rows, head_dim 128, causal, dq in 4 splits 192 us, whole 143 (whole backward).
+struct BackwardCost {
+  double start, tile_us, launch, per_mb;  // start: what a workgroup costs beside its tiles, in tiles, where another one has its place before
+};
+inline int backward_splits_16bit(const BackwardCost& c, bool of_keys, int B, int Hq, int Hkv, int L, int S, int D, bool causal, int offset) {
+  const int slots = of_keys && D == 128 ? 256 : 512;  // workgroups side by side
+  const int group = of_keys ? Hq / Hkv : 1, halves = of_keys && D == 128 ? 2 : 1;  // heads of a stream; wavefront groups that share it
+  const int nblk = ((of_keys ? S : L) + 127) / 128;
+  const long long heads = (long long)B * (of_keys ? Hkv : Hq);
+  auto tiles = [&](int t) {  // of the t-th longest block
+    if (!causal) return group * (((of_keys ? L : S) + 31) / 32);
+    if (of_keys) {
+      const int first = 128 * t - offset > 0 ? (128 * t - offset) / 32 : 0, all = (L + 31) / 32;
+      return first < all ? group * (all - first) : 0;
+    }
+    const int row = 128 * (nblk - t) < L ? 128 * (nblk - t) : L, last = row + offset < S ? row + offset : S;
+    return (last + 31) / 32;
+  };
+  double sum = 0;
+  for (int t = 0; t < nblk; t++) sum += tiles(t);
+  auto us = [&](int n) {
+    const double per = n * halves;
+    const long long wgs = heads * nblk * n, each = heads * n;
+    double chain = ceil(tiles(0) / per);
+    if (wgs > slots) {
+      double next;
+      if (!causal) next = (wgs + slots - 1) / slots * (chain + c.start) - c.start;
+      else if (wgs <= 2 * slots) next = ceil(tiles((int)((slots - 1) / each)) / per) + ceil(tiles((int)(slots / each)) / per) + c.start;
+      else next = heads * sum / halves / slots + 0.5 * tiles(nblk - 1) / per + c.start * ((double)wgs / slots - 1);
+      chain = next > chain ? next : chain;
+    }
+    const double record_mb = of_keys ? 8e-6 * n * heads * S * D : 4e-6 * n * heads * L * (D + 2);
+    return c.tile_us * chain + (n > 1 ? c.launch + c.per_mb * record_mb : 0);
+  };
+  int best = 1;
+  double least = us(1);
+  for (int n = 2; n <= 16; n++) {
+    const double t = us(n);
+    if (t < 0.95 * least) best = n, least = t;
+  }
+  return best;
+}
+
 // Workgroup id of a dk/dv launch with split query streams -> (key-block workgroup n, split).  The hardware hands
 // workgroup id to XCD id % 8 and map_workgroup places n by n % 8: the splits of eight consecutive n follow each other in
 // groups of eight, so that n % 8 == id % 8 and the order (longest key blocks first) is kept.
@@ -555,8 +602,9 @@ __device__ __forceinline__ void pin_accumulator(f32x16& acc) {
 // second round (all arrive at the last tile together); walking down, each would be alone with its position and fetch
 // its tiles from memory itself.  The third round starts together again: rounds alternate.  (bf16 head_dim 128, B2 32q/8kv
 // 4096 x 4096: 458 -> 240 MB read per launch of the dk/dv kernel.)
-__device__ __forceinline__ bool dkv_walks_up(const BwdArgs& a, bool causal) {
-  return causal && a.dkv_round > 0 && ((a.f.B * a.f.Hkv) & 7) == 0 && (((int)(blockIdx.x >> 3) / a.dkv_round) & 1) != 0;
+// The splits of a key block walk alike, whatever round each is in: wg, its place without splits.
+__device__ __forceinline__ bool dkv_walks_up(const BwdArgs& a, bool causal, int wg) {
+  return causal && a.dkv_round > 0 && ((a.f.B * a.f.Hkv) & 7) == 0 && (((wg >> 3) * a.dkv_splits / a.dkv_round) & 1) != 0;
 }
 
 // Workgroups of `kernel` that fit one CU, times the CUs of an XCD: the dkv_round of a launch (looked up once per device).

@@ -624,6 +624,8 @@ bool backward_log_sums(const ttsdpa_backward_params* p) { return p->fwd.mask_kin
 size_t backward_stats_bytes(const ttsdpa_backward_params* p) { return backward_rows(p) * (backward_log_sums(p) ? 3 : 2) * sizeof(float); }
 
 // How the matrix-core pairs divide a call (made once for a call): the dk / dv kernel's query streams and the dq kernel's key ranges.
+struct PairSplits;
+int short_backward_splits(const ttsdpa_backward_params* p, const PairSplits& n, bool* joint = nullptr);
 struct PairSplits {
   int dkv = 1, dq = 1;
   bool dkv_dealt = false, dq_dealt = false;
@@ -631,6 +633,14 @@ struct PairSplits {
     const ttsdpa_params* f = &p->fwd;
     if (!backward_on_mfma(p)) return;
     const bool f32 = backward_on_f32_pair(p), causal = effective_causal(f) != TTSDPA_CAUSAL_NONE;
+    if (f->dtype != TTSDPA_F32 && f->mask_kind == TTSDPA_MASK_NONE && (f->D == 64 || f->D == 128)) {
+      static constexpr BackwardCost kDq[2] = {{0, 0.59, 3.6, 0.47}, {4.5, 0.53, 2.9, 0.37}}, kDkv[2] = {{0, 0.95, 2.5, 0.40}, {0, 1.75, 1.8, 0.41}};
+      if (short_backward_splits(p, *this) > 0) return;  // (whole: with less scratch than those kernels ask for)
+      const int more = f->S > f->L ? f->S - f->L : 0, offset = effective_causal(f) == TTSDPA_CAUSAL_BOTTOM_RIGHT ? more : 0;
+      dq = backward_splits_16bit(kDq[f->D == 128], false, f->B, f->Hq, f->Hkv, f->L, f->S, f->D, causal, more);
+      dkv = backward_splits_16bit(kDkv[f->D == 128], true, f->B, f->Hq, f->Hkv, f->L, f->S, f->D, causal, offset);
+      return;
+    }
     const int groups = f->dtype != TTSDPA_F32 && f->D == 128 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
     const int per_cu = f->D <= 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
     dkv = backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, causal, groups, per_cu, f32, &dkv_dealt);
@@ -664,7 +674,7 @@ double pair_backward_us(const ttsdpa_params* f, const ShortShape& s, const PairS
 }
 
 // The short sequences' backward: splits of its dk / dv workgroups, 0 where the pairs are the shorter way.
-int short_backward_splits(const ttsdpa_backward_params* p, const PairSplits& n, bool* joint = nullptr) {
+int short_backward_splits(const ttsdpa_backward_params* p, const PairSplits& n, bool* joint) {
   const ttsdpa_params* f = &p->fwd;
   if (!short_ok(f) || !(backward_mfma_ok(p) || backward_f32_ok(p))) return 0;
   const ShortShape s(f);
