@@ -856,8 +856,9 @@ struct DecodePlan {
   int chunk;       // keys per split (multiple of the per-wave key block)
   int rows;        // query rows handled together per KV head: L * G
   size_t ws_bytes; // workspace: per (batch, kv head, split): rows * (D + 2) floats
+  int waves;  // wavefronts of a workgroup: 4, or 8 (up to 8 query rows)
 };
-DecodePlan plan_decode(const KArgs& a);
+DecodePlan plan_decode(const KArgs& a, bool f32);
 
 constexpr int kDecodeMaxRows = 16;  // L * (Hq/Hkv) handled by one MFMA row block
 

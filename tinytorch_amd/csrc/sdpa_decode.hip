@@ -26,7 +26,6 @@ namespace ttsdpa {
 namespace {
 
 constexpr int KB = 32;       // keys per wavefront block
-constexpr int NWAVE = 4;
 
 // What the kernel needs to know about the element type: 16 bytes of it as an MFMA operand, and as floats.
 template <typename TR>
@@ -73,6 +72,39 @@ __device__ __forceinline__ float row16_sum(float x) {
   return x;
 }
 
+// Sums of N values of a lane over the lanes of its chunk (lane % CH): a swap of two registers' halves (of their rows of 16 lanes) and one
+// addition fold two values into one register, so that four (CH = 32: two) values end in one, each in its own rows: value
+// phase_value + 4 i (2 i) in element i.  (As 2 shuffles through LDS for each value, 64 a wavefront, this took 0.7 us.)
+__device__ __forceinline__ float fold32(float a, float b) {
+  const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+  const int lo = t[0], hi = t[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+__device__ __forceinline__ float fold16(float a, float b) {
+  const auto t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+  const int lo = t[0], hi = t[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+template <int CH>
+__device__ __forceinline__ int phase_value(int lane) {
+  return CH < 32 ? (lane >> 5) + 2 * ((lane >> 4) & 1) : lane >> 5;
+}
+template <int CH, int N>
+__device__ __forceinline__ void add_phases(float* x) {
+  static_assert(CH == 8 || CH == 16 || CH == 32, "");
+  if constexpr (CH == 32) {
+#pragma unroll
+    for (int i = 0; i < N / 2; i++) x[i] = fold32(x[2 * i], x[2 * i + 1]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N / 4; i++) {
+      float t = fold16(fold32(x[4 * i], x[4 * i + 1]), fold32(x[4 * i + 2], x[4 * i + 3]));
+      if constexpr (CH == 8) t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x128, 0xf, 0xf, false));  // row_ror:8
+      x[i] = t;
+    }
+  }
+}
+
 // Make this wavefront's LDS writes visible to its own later reads and keep the compiler from reordering across.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -86,8 +118,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 // PAD: the tensors' head_dim a.D is a multiple of 8 below DD.  The 16-byte chunks of a row beyond it read as zeros (q, k)
 // or are left out of the output (v: the lanes of those chunks fetch the row's first chunk instead, so that the loads stay
 // unconditional); the split records keep the pitch DD + 2.
-template <typename TR, int R, int DD, bool PAGED, bool PAD>
-__global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int chunk, float* __restrict__ ws) {
+template <typename TR, int R, int DD, bool PAGED, bool PAD, int NWAVE>
+__global__ __launch_bounds__(64 * NWAVE, 2) void decode_kernel(KArgs a, int splits, int chunk, float* __restrict__ ws) {
   typedef typename Dec<TR>::elem T;
   typedef typename Dec<TR>::chunk chunk_t;
   constexpr int E = 16 / sizeof(T);  // elements of a 16-byte chunk
@@ -274,20 +306,13 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
   // ---- wavefront totals: sums over the 16 key lanes; accumulators over the key phases ------------------------------------
 #pragma unroll
   for (int r = 0; r < R; r++) l_run[r] = row16_sum(l_run[r]);
+  add_phases<CH, NR * E>(&acc[0][0]);
+  if (CH > 8 || (lane & 8) == 0) {
 #pragma unroll
-  for (int x = 0; x < NR; x++)
-#pragma unroll
-    for (int i = 0; i < E; i++) {
-      float t = acc[x][i];
-#pragma unroll
-      for (int off = CH; off < 64; off *= 2) t += __shfl_xor(t, off);
-      acc[x][i] = t;
+    for (int i = 0; i < NR * E / (CH < 32 ? 4 : 2); i++) {
+      const int v = phase_value<CH>(lane) + (CH < 32 ? 4 : 2) * i;  // of the lane's chunk
+      Om[wave][v / E][E * vc + v % E] = (&acc[0][0])[i];
     }
-  if (vph == 0) {
-#pragma unroll
-    for (int x = 0; x < NR; x++)
-#pragma unroll
-      for (int i = 0; i < E; i++) Om[wave][x][E * vc + i] = acc[x][i];
   }
   if (l16 == 0) {
 #pragma unroll
@@ -298,8 +323,8 @@ __global__ __launch_bounds__(256, 2) void decode_kernel(KArgs a, int splits, int
   }
   __syncthreads();
 
-  // ---- merge the four wavefronts; thread t handles (row slot, dim) pairs ------------------------------------------------------
-  for (int e = tid; e < NR * DD; e += 256) {
+  // ---- merge the wavefronts; thread t handles (row slot, dim) pairs ------------------------------------------------------
+  for (int e = tid; e < NR * DD; e += 64 * NWAVE) {
     int x = e / DD, d = e % DD;  // row slot x holds query row x (slot index == query row index)
     if (x >= rows) continue;
     float mx = Om[0][x][DD];
@@ -366,23 +391,27 @@ __global__ __launch_bounds__(DD) void merge_kernel(KArgs a, int splits, const fl
   if (t < a.D) store_from_float(op + t, empty ? 0.f : o / total);  // (a.D < DD: the decode kernel's zero-column variant)
 }
 
+template <typename TR, int R, int DD, bool PAD, int NWAVE>
+void launch_decode_w(const KArgs& a, const DecodePlan& pl, float* ws, hipStream_t stream) {
+  const dim3 grid((unsigned)((long long)a.B * a.Hkv * pl.splits)), block(64 * NWAVE);
+  if (a.block_table) hipLaunchKernelGGL((decode_kernel<TR, R, DD, true, PAD, NWAVE>), grid, block, 0, stream, a, pl.splits, pl.chunk, ws);
+  else hipLaunchKernelGGL((decode_kernel<TR, R, DD, false, PAD, NWAVE>), grid, block, 0, stream, a, pl.splits, pl.chunk, ws);
+}
+template <typename TR, int R, int DD, bool PAD>
+void launch_decode_r(const KArgs& a, const DecodePlan& pl, float* ws, hipStream_t stream) {
+  if constexpr (R <= 2)
+    if (pl.waves == 8) return launch_decode_w<TR, R, DD, PAD, 8>(a, pl, ws, stream);
+  launch_decode_w<TR, R, DD, PAD, 4>(a, pl, ws, stream);
+}
 template <typename TR, int DD, bool PAD>
 int launch_decode_t(const KArgs& a, const DecodePlan& pl, float* ws, hipStream_t stream) {
   typedef typename Dec<TR>::elem T;
-  dim3 grid((unsigned)((long long)a.B * a.Hkv * pl.splits)), block(256);
-  int R = (pl.rows + 3) / 4;
-#define TT_DECODE(R_)                                                                                                      \
-  if (a.block_table)                                                                                                       \
-    hipLaunchKernelGGL((decode_kernel<TR, R_, DD, true, PAD>), grid, block, 0, stream, a, pl.splits, pl.chunk, ws);       \
-  else                                                                                                                     \
-    hipLaunchKernelGGL((decode_kernel<TR, R_, DD, false, PAD>), grid, block, 0, stream, a, pl.splits, pl.chunk, ws)
-  switch (R) {
-    case 1: TT_DECODE(1); break;
-    case 2: TT_DECODE(2); break;
-    case 3: TT_DECODE(3); break;
-    default: TT_DECODE(4); break;
+  switch ((pl.rows + 3) / 4) {
+    case 1: launch_decode_r<TR, 1, DD, PAD>(a, pl, ws, stream); break;
+    case 2: launch_decode_r<TR, 2, DD, PAD>(a, pl, ws, stream); break;
+    case 3: launch_decode_r<TR, 3, DD, PAD>(a, pl, ws, stream); break;
+    default: launch_decode_r<TR, 4, DD, PAD>(a, pl, ws, stream); break;
   }
-#undef TT_DECODE
   int rc = (int)hipGetLastError();
   if (rc != 0 || pl.splits == 1) return rc;
   hipLaunchKernelGGL((merge_kernel<T, DD>), dim3((unsigned)((long long)a.B * a.Hkv * pl.rows)), dim3(DD), 0, stream, a, pl.splits, ws);
@@ -391,10 +420,11 @@ int launch_decode_t(const KArgs& a, const DecodePlan& pl, float* ws, hipStream_t
 
 }  // namespace
 
-DecodePlan plan_decode(const KArgs& a) {
+DecodePlan plan_decode(const KArgs& a, bool f32) {
   DecodePlan p;
   p.rows = a.L * a.G;
-  const int round = NWAVE * KB;
+  const int round = 4 * KB;
+  p.waves = 4;
   long long pairs = (long long)a.B * a.Hkv;
   // two blocks of keys per wavefront at least, or one where that leaves most of the CUs idle (1 sequence of 1500 keys, 8 KV heads
   // 11.2 -> 9.5 us, 2 of 324, one KV head 12.2 -> 10.3; not for a single chunk: the merge costs more)
@@ -420,6 +450,25 @@ DecodePlan plan_decode(const KArgs& a) {
   if (chunk < round) chunk = round;
   splits = (a.S + chunk - 1) / chunk;
   if (splits < 1) splits = 1;
+  // A workgroup of four or eight wavefronts for all of a sequence's keys, in one launch, where that is shorter than the split and its
+  // merge: us for a turn of the wavefronts (32 keys each), the merge's launch, a CU's further workgroups (four wavefronts of them: each, and
+  // for a turn), and twice the wavefronts, by head_dim, element type and rows; fitted to 400 calls of 1 to 1500 (sequence, KV head)
+  // pairs on 128 to 4096 keys (9 to 15 % off; a turn is the vector ALUs' P.V for the most part: requesting the next turn's keys ahead gave
+  // nothing).  A cache is taken to be filled to nine tenths.  24 x 8 pairs on up to 1024 keys 13.3 -> 9.5 us, 12 x 8 on 178 of 1024 9.6 -> 6.4;
+  // 12 x 1 on 1024 stay split, 8.2 and 14.2.  Not beyond the keys it was fitted on, where memory's rate is all that counts: 64 x 8 on 8192 316
+  // us with four wavefronts and 323 with eight.
+  static constexpr double fit[2][2][2][5] = {{{{1.2, 3.6, 0.40, 0, 0.8}, {1.25, 3.0, 1.5, 0, 0.4}}, {{1.95, 3.6, 0, 0.80, 1.35}, {2.5, 4.8, 2.2, 0, 1.8}}},
+                                             {{{2.0, 3.7, 0, 0.68, 1.15}, {2.15, 3.5, 1.5, 0.62, 1.2}}, {{3.8, 4.3, 1.3, 0.86, 2.6}, {4.7, 4.5, 0.93, 1.55, 2.6}}}};
+  if (p.rows <= 8 && a.S <= 4096) {
+    const double* f = fit[a.D > 64][f32][p.rows > 4];
+    const double keys = a.kv_len ? 0.9 * a.S : a.S, fixed = 2.5 + 1e-7 * pairs * keys * a.D * (f32 ? 8 : 4);  // (0.1 us for a MB)
+    auto us = [&](int waves, int n) {
+      const double further = (double)((pairs * n + 255) / 256 - 1) * waves / 4, turns = ceil(ceil(keys / n) / (KB * waves));
+      return fixed + f[0] * turns + (n > 1 ? f[1] : 0) + (f[2] + f[3] * turns) * further + (waves > 4 ? f[4] : 0);
+    };
+    const double split = us(4, splits), four = us(4, 1), eight = us(8, 1);
+    if ((four < eight ? four : eight) < 0.95 * split) splits = 1, chunk = (a.S + round - 1) / round * round, p.waves = eight < four ? 8 : 4;
+  }
   p.splits = splits;
   p.chunk = chunk;
   p.ws_bytes = splits > 1 ? (size_t)pairs * splits * p.rows * ((a.D <= 64 ? 64 : 128) + 2) * sizeof(float) : 0;  // the kernel's head_dim: 64 or 128
@@ -442,7 +491,7 @@ int launch_decode_d(const KArgs& a, const DecodePlan& pl, float* ws, hipStream_t
 }  // namespace
 
 int launch_decode(const KArgs& a, int dtype, void* workspace, hipStream_t stream) {
-  const DecodePlan pl = plan_decode(a);
+  const DecodePlan pl = plan_decode(a, dtype == 0);
   switch (dtype) {
     case 0: return launch_decode_d<F32>(a, pl, (float*)workspace, stream);
     case 1: return launch_decode_d<F16>(a, pl, (float*)workspace, stream);

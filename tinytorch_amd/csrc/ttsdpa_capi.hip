@@ -787,11 +787,11 @@ size_t ttsdpa_workspace_bytes(const ttsdpa_params* p) {
   if (validate(p, &a) != TTSDPA_OK) return 0;
   if (p->B == 0 || p->L == 0 || p->S == 0) return 0;
   // enough for ttsdpa_forward's route and for an explicit ttsdpa_decode of the same call
-  size_t need = decode_ok(p) ? plan_decode(a).ws_bytes : 0;
+  size_t need = decode_ok(p) ? plan_decode(a, p->dtype == TTSDPA_F32).ws_bytes : 0;
   const int route = pick_route(p);
   if (route == TTSDPA_ROUTE_PREFILL || (route == TTSDPA_ROUTE_GENERAL && p->mask_kind != TTSDPA_MASK_NONE && prefill_ok(p, true))) {
     if (f32_decode_ok(p)) {
-      const size_t decode = plan_decode(a).ws_bytes;
+      const size_t decode = plan_decode(a, p->dtype == TTSDPA_F32).ws_bytes;
       need = decode > need ? decode : need;
     }
     if (pack_heads_ok(p)) pack_heads(&a);
@@ -851,7 +851,7 @@ static int prefill_impl(const ttsdpa_params* p, void* workspace, size_t workspac
     return p->D == 128 ? launch_prefill_d128(a, p->dtype, (hipStream_t)stream) : launch_prefill_d64(a, p->dtype, (hipStream_t)stream);
   }
   if (f32_decode_ok(p)) {
-    const DecodePlan pl = plan_decode(a);
+    const DecodePlan pl = plan_decode(a, p->dtype == TTSDPA_F32);
     if ((pl.ws_bytes == 0 || (workspace && workspace_bytes >= pl.ws_bytes && ptr_aligned(workspace, 16))) &&
         check_grid((long long)a.B * a.Hkv * pl.splits) == TTSDPA_OK)
       return launch_decode(a, p->dtype, workspace, (hipStream_t)stream);
@@ -880,7 +880,7 @@ int ttsdpa_decode(const ttsdpa_params* p, void* workspace, size_t workspace_byte
   if (rc != TTSDPA_OK) return rc;
   if (p->B == 0 || p->L == 0) return TTSDPA_OK;
   if (!decode_ok(p)) return TTSDPA_ERR_UNSUPPORTED;
-  DecodePlan pl = plan_decode(a);
+  DecodePlan pl = plan_decode(a, p->dtype == TTSDPA_F32);
   if (pl.ws_bytes > 0 && (!workspace || workspace_bytes < pl.ws_bytes || !ptr_aligned(workspace, 16)))
     return TTSDPA_ERR_WORKSPACE;
   if ((rc = check_grid((long long)a.B * a.Hkv * pl.splits)) != TTSDPA_OK) return rc;
@@ -893,7 +893,7 @@ int ttsdpa_decode_static(const ttsdpa_params* p, void* stream) {
   if (rc != TTSDPA_OK) return rc;
   if (p->B == 0 || p->L == 0) return TTSDPA_OK;
   if (!decode_ok(p)) return TTSDPA_ERR_UNSUPPORTED;
-  const DecodePlan pl = plan_decode(a);
+  const DecodePlan pl = plan_decode(a, p->dtype == TTSDPA_F32);
   if (pl.ws_bytes > kStaticScratchBytes) return TTSDPA_ERR_STATIC_SCRATCH;
   if ((rc = check_grid((long long)a.B * a.Hkv * pl.splits)) != TTSDPA_OK) return rc;
   void* ws = nullptr;
