@@ -364,7 +364,8 @@ struct RowTiles {
     if (n > 256) {
       if (!causal) longest = rounds * longest + (rounds - 1) * c.start;
       else if (rows == 256 && ntile > 1 && pairs >= 256 && pairs * 10 >= pair_rounds * 256 * 9)  // mirrored pairs (launch_prefill_d128)
-        longest = pair_rounds * (longest + length(ntile - 1) + c.start) - c.start;
+        longest = ntile % 2 == 0 ? pair_rounds * (longest + length(ntile - 1) + c.start) - c.start
+                                 : sum / 256.0 + c.start * (pairs / 256.0 - 1) + 0.25 * longest;  // (the middle ones are single)
       else {
         // the CU with the shortest of the first 256 takes the next one
         const double next = n <= 512 ? length((int)(255 / heads)) + length((int)(256 / heads)) + c.start
