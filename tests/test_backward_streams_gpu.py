@@ -1,5 +1,5 @@
 """The 16-bit backward pair's streams and splits (sdpa_backward_d128.hip, backward_splits_16bit): key counts around its tiles of 32 and
-its two steps at a time, row tiles whose wavefronts end at different tiles, maxima that rise on the way, and numbers of splits
+its two steps at a time, query streams of few tiles, row tiles whose wavefronts end at different tiles, maxima that rise on the way, and numbers of splits
 that are no power of two over more workgroups than run side by side.  All three gradients against float64."""
 import ctypes
 
@@ -68,6 +68,16 @@ TL, BR = "top-left", "bottom-right"
 ], ids=lambda c: "B%dH%dk%dL%dS%d-c%d-%s" % c)
 def test_dq_stream(case, dtype):
     check(case, dtype, 128)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("Hq,Hkv", [(6, 2), (5, 5), (7, 1)])
+@pytest.mark.parametrize("L", [33, 64, 96, 160, 193])
+def test_dkv_stream_of_few_tiles(L, Hq, Hkv, dtype):
+    """Fewer tiles than the ring's stages, none for the second group of wavefronts, one left over, a ragged one at either end; key
+    blocks that do not end with the keys."""
+    check((1, Hq, Hkv, L, 1230, False, TL), dtype, 128)
+    check((1, Hq, Hkv, L, 1230, True, BR), dtype, 128)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])

@@ -24,6 +24,18 @@ Register plan of a lane (fixed, named in the statements' constraints by the kern
 Named operands: o0-o3 the dq accumulators (read-write), ps the lane's sum of the step's probabilities (out), c = scale*log2(e)
 (scalar register), mc = maximum*c, dl = delta of the lane's row.
 
+dk/dv, a tile of 32 query rows against the wavefront's 32 keys (K in registers), 32 slots:
+    0 .. 7    S = Q . K^T, a chain of dependent products
+    8 .. 15   dP - delta = dout . V^T - delta (the chain's first accumulator)      P = exp2(S c - lse) from slot 9
+    16 .. 23  dv^T += dout^T . P                                                                      dS = (dP - delta) P from slot 18
+    24 .. 31  dk^T += Q^T . dS
+    Fixed registers: v[136:139] transposed, v[140:143] row operand addresses
+    v[144:151]  lse of rows, quads 0 and 1 (2 and 3 lie in v[152:159] before P does)     v[152:159] P in pairs of 16 bits
+    v[160:175]  dP (then dS)      v[176:191]  S (then P)      v[192:223]  K, 8 k-steps x 4 registers      v[224:255]  operand ring
+    Named: o0-o3 dk, o4-o7 dv (read-write), c = scale*log2(e), vb = the wavefront's V rows from the stage's start, st = the stage's start,
+    adv = the next stage's from there, more = whether the step has asked for a tile (scalar registers).  One stream for all stages: with one
+    each, a workgroup's first steps waited for their instructions (of 36 to 90 us on 165 to 480 rows, 2 to 5).
+
 LDS: a tile is 8 groups of 4 rows of 256 bytes, a group every GROUP bytes (the 16 bytes between them spread the banks); chunk c of
 16 bytes of row i of a group sits at slot c ^ 4i.
 """
@@ -120,6 +132,105 @@ def dq_step(u, elem):
     return out
 
 
+# ---- dk/dv -----------------------------------------------------------------------------------------------------------------
+KV_SLOTS = 32
+KTR, KR, KL, KPB, KD, KS, KK = 136, 140, 144, 152, 160, 176, 192
+# operands of a step in the order of their use: the slots' counts
+KV_OPS = [1] * 8 + [2] * 8 + [1] * 16
+KV_ENTRIES = sum(KV_OPS)  # a multiple of RING: the same registers in every step
+
+
+# All reads of the step's tile have arrived, and so has the next tile (what was asked for last, %[more], may still be on its way: five
+# loads of a wavefront); the next tile's first operands follow.
+KV_BARRIER, KV_NEXT = 28, {28: 2, 29: 3, 30: 5, 31: 6}
+KV_SYNC = ["s_cmp_lg_u32 %[more], 0", "s_cbranch_scc1 1f", "s_waitcnt vmcnt(0)", "1:", "s_waitcnt vmcnt(5) lgkmcnt(0)", "s_barrier"]
+
+
+def kv_row(r, address, ks, base):
+    return "ds_read_b128 %s, %s offset:%d" % (vr(r, 4), vr(address), base + 32 * (ks & 1))
+
+
+def kv_fetch(e):
+    """Requests of entry e of a step (entries behind the last are the next one's: the addresses have moved on by then)."""
+    e %= KV_ENTRIES
+    r = RING0 + 4 * (e % RING)
+    if e < 8:
+        return [kv_row(r, KR + e // 2, e, 0)]
+    if e < 24:
+        ks, of_v = (e - 8) // 2, (e - 8) % 2
+        if not of_v:
+            return [kv_row(r, KR + ks // 2, ks, TILE)]
+        return ["v_add_u32 v%d, %%[vb], v%d" % (r, KR + ks // 2), kv_row(r, r, ks, 0)]  # (the address in a register of the operand)
+    t, db = (e - 24) % 8 // NDB, e % NDB
+    tile = TILE if e < 32 else 0
+    return ["ds_read_b64_tr_b16 %s, %s offset:%d" % (vr(r + 2 * ld, 2), vr(KTR + db), tile + (4 * t + 2 * ld) * GROUP) for ld in range(2)]
+
+
+def kv_statistics():
+    """Requests of the row statistics, by slot: lse's four quads, -delta into dP's accumulator (their address in one of its registers)."""
+    at, adr = 2 * TILE, KD + 12
+    lse = ["ds_read_b128 %s, v%d offset:%d" % (vr(r, 4), adr, at + 32 * q) for q, r in enumerate((KL, KL + 4, KPB, KPB + 4))]
+    delta = ["ds_read_b128 %s, v%d offset:%d" % (vr(KD + 4 * q, 4), adr, at + 128 + 32 * q) for q in range(4)]
+    address = ["v_mbcnt_lo_u32_b32 v%d, -1, 0" % adr, "v_bfe_u32 v%d, v%d, 5, 1" % (adr, adr), "v_lshl_add_u32 v%d, v%d, 4, %%[st]" % (adr, adr)]
+    return {1: address + lse[:1], 2: lse[1:2], 3: lse[2:], 4: delta[:1], 5: delta[1:2], 6: delta[2:]}
+
+
+def kv_vector_work(elem):
+    """The vector instructions of the slots."""
+    cvt = "v_cvt_pk_%s_f32" % elem
+    lse = [KL, KPB]
+    fma = lambda n: "v_fma_f32 %s, %s, %%[c], -%s" % (vr(KS + n), vr(KS + n), vr(lse[n // 8] + n % 8))
+    exp = lambda n: "v_exp_f32 %s, %s" % (vr(KS + n), vr(KS + n))
+    mul = lambda n: "v_mul_f32 %s, %s, %s" % (vr(KD + n), vr(KD + n), vr(KS + n))
+    pack = lambda to, frm, j: "%s %s, %s, %s" % (cvt, vr(to + j), vr(frm + 2 * j), vr(frm + 2 * j + 1))
+    p, ds = lambda j: pack(KPB, KS, j), lambda j: pack(KD, KD, j)
+    first = sum(([fma(2 * n), fma(2 * n + 1), exp(n)] for n in range(8)), []) + [exp(8)] + [p(j) for j in range(4)]
+    second = [exp(9), exp(10), p(4), exp(11), exp(12), p(5), exp(13), exp(14), p(6), exp(15), mul(0), mul(1), p(7)]
+    third = [mul(2), mul(3), ds(0), mul(4), mul(5), ds(1), mul(6), mul(7), ds(2), mul(8), mul(9), ds(3)]
+    third += [mul(10), mul(11), ds(4), mul(12), mul(13), ds(5), mul(14), mul(15), ds(6), ds(7)]
+    out = [[] for _ in range(KV_SLOTS)]
+    for lo, work, slots in ((9, first, 6), (15, second, 4), (19, third, 4)):
+        out[lo:lo + slots] = spread(work, slots)
+    advance = lambda r: "v_add_u32 v%d, %%[adv], v%d" % (r, r)  # to the next stage, behind their last use in this one
+    out[24], out[25] = [advance(KR), advance(KR + 1)], [advance(KR + 2), advance(KR + 3)]
+    out[26], out[27] = [advance(KTR), advance(KTR + 1)], [advance(KTR + 2), advance(KTR + 3)]
+    return out
+
+
+def kv_step(elem):
+    mfma = "v_mfma_f32_32x32x16_%s" % elem
+    work, stat = kv_vector_work(elem), kv_statistics()
+    # LDS requests in their order, those of the first PD entries from the step before
+    order = [("e", e) for e in range(PD) for r in kv_fetch(e)]
+    out, used, asked = [], 0, PD
+    for s in range(KV_SLOTS):
+        entries = range(used, used + KV_OPS[s])
+        used += KV_OPS[s]
+        needed = [("e", e) for e in entries] + ([("s", t) for t in range(1, 7)] if s == 8 else [])
+        last = max(i for i, o in enumerate(order) if o in needed)
+        out.append("s_waitcnt lgkmcnt(%d)" % min(15, len(order) - 1 - last))
+        ring = [vr(RING0 + 4 * (e % RING), 4) for e in entries]
+        if s < 8:
+            out.append("%s %s, %s, %s, %s" % (mfma, vr(KS, 16), ring[0], vr(KK + 4 * s, 4), "0" if s == 0 else vr(KS, 16)))
+        elif s < 16:
+            out.append("%s %s, %s, %s, %s" % (mfma, vr(KD, 16), ring[0], ring[1], vr(KD, 16)))
+        else:
+            db, t, of_k = s % NDB, s % 8 // NDB, s >= 24
+            out.append("%s %%[o%d], %s, %s, %%[o%d]" % (mfma, db if of_k else 4 + db, ring[0], vr((KD if of_k else KPB) + 4 * t, 4), db if of_k else 4 + db))
+        if s == KV_BARRIER:
+            out += KV_SYNC
+        while asked < (used + PD if s < 26 else KV_ENTRIES + KV_NEXT.get(s, 0)):
+            lines = kv_fetch(asked)
+            out += lines
+            order += [("e", asked)] * sum("ds_read" in x for x in lines)
+            asked += 1
+        out += stat.get(s, [])
+        order += [("s", s)] * sum("ds_read" in x for x in stat.get(s, []))
+        out += work[s]
+    assert asked == KV_ENTRIES + PD == KV_ENTRIES + KV_NEXT[31] and KV_ENTRIES % RING == 0
+    return out
+
+
 def emit(name, lines):
     print("#define %s \\" % name)
     print(" \\\n".join('  "%s\\n\\t"' % l for l in lines))
@@ -128,13 +239,16 @@ def emit(name, lines):
 
 def main():
     print("// Generated by gen_backward128_steps.py; do not edit.  Instruction streams of the head_dim-128 attention backward:")
-    print("// TT_B128_DQ_<elem>_U<tile of the unrolled body>.")
+    print("// TT_B128_DQ_<elem>_U<tile of the unrolled body>, TT_B128_DKV_<elem>.")
     print()
     for u in range(STAGES):  # the first requests of a step, where the step before was not a stream
         emit("TT_B128_DQ_PREFETCH_U%d" % u, sum((dq_fetch(DQ_SLOTS * u + g) for g in range(PD)), []))
     for elem in ("bf16", "f16"):
         for u in range(STAGES):
             emit("TT_B128_DQ_%s_U%d" % (elem.upper(), u), dq_step(u, elem))
+    emit("TT_B128_DKV_PREFETCH", sum((kv_fetch(e) for e in range(PD)), []))
+    for elem in ("bf16", "f16"):
+        emit("TT_B128_DKV_%s" % elem.upper(), kv_step(elem))
 
 
 if __name__ == "__main__":

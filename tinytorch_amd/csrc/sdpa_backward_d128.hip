@@ -1,7 +1,7 @@
-// Attention backward for fp16 / bf16, head_dim 128, without an attnMask, on gfx950 matrix cores: dq and the row statistics
-// (sdpa_backward_mfma.hip has the mathematics and the other half).
+// Attention backward for fp16 / bf16, head_dim 128, without an attnMask, on gfx950 matrix cores (sdpa_backward_mfma.hip has
+// the mathematics).
 //
-// A workgroup owns 128 query rows of one (batch, query head), a wavefront 32 of them (Q and dout in registers); keys stream in tiles
+// dq and the row statistics: a workgroup owns 128 query rows of one (batch, query head), a wavefront 32 of them (Q and dout in registers); keys stream in tiles
 // of 32.  Per tile a wavefront forms S^T = K.Q^T and dP^T = V.dout^T, turns them into P and dS on the vector ALU and accumulates dq^T +=
 // K^T.dS^T: 24 matrix instructions (768 cycles) and 88 vector ones, 16 of them exponentials (about 550 cycles of issue, beside 16 for every
 // matrix instruction).  In the compiler's order the three followed each other, the wavefronts of a SIMD hardly overlapping: 3250 cycles
@@ -13,6 +13,12 @@
 // K and V come by direct global->LDS loads, four stages each (K of tiles i-1, i, i+1 and, on its way, i+2): a tile is eight groups of
 // four 256-byte rows, 1040 bytes apart, chunk c of 16 bytes of row i of a group at slot c ^ 4i, so that one copy serves the
 // row-major reads and the transposed ones without bank conflicts and both take four address registers.
+
+// dk and dv: a workgroup owns 128 keys.  A tile of 32 query rows costs a wavefront 32 matrix instructions (1024 cycles), 80 vector ones
+// and 44 KB of LDS operands, a SIMD's two wavefronts the LDS's whole 2050 cycles; here everything of a tile is one stream, a step, with its
+// operands requested into the register ring 6 ahead (the next tile's first before the step ends) and all that is not a matrix
+// instruction spread between those.  Same call: 620 -> 566 us in the first launches, the matrix pipe 55 % busy at 1.73 GHz
+// (45 % at 1.87 in the compiler's order), 545 -> 520 among others once the chip is warm: power again.
 
 #include "backward128_steps.inc"  // hand-ordered instruction streams (gen_backward128_steps.py)
 #include "sdpa_common.h"
@@ -353,10 +359,10 @@ __global__ __launch_bounds__(256, 2) void backward_dq128_kernel(BwdArgs a) {
   if (qi >= f.L) return;
   const long long row_id = ((long long)b * f.Hq + h) * f.L + qi;
   if (a.dq_splits > 1) {
-    store_dq_partial<D>(a, piece, row_id, half, dqacc, m_use * c, l_tot, delta);
+    store_dq_partial<D>(a, piece, row_id, half, dqacc, m_use * c, l_tot, -delta);
     return;
   }
-  if (half == 0) *(float2*)(a.stats + 2 * row_id) = make_float2(m_use * c + __log2f(l_tot), delta);
+  if (half == 0) *(float2*)(a.stats + 2 * row_id) = make_float2(m_use * c + __log2f(l_tot), -delta);  // -delta: see the dk/dv kernel
   const float w = f.scale / l_tot;
   T* dqp = (T*)a.dq + b * a.dqs[0] + h * a.dqs[1] + qi * a.dqs[2] + 4 * half;
 #pragma unroll
@@ -370,6 +376,319 @@ __global__ __launch_bounds__(256, 2) void backward_dq128_kernel(BwdArgs a) {
     }
 }
 
+// ---- dk, dv ----------------------------------------------------------------------------------------------------------------
+// A workgroup owns 128 keys of a (batch, KV head), a wavefront 32 of them (K in registers, V in LDS): the 32-row tiles of the query
+// heads that see them stream past.  Eight wavefronts in two groups of four: both groups own the same keys and take alternate tiles, each
+// with its own ring of three stages, and the second's gradients join the first's at the end — under a causal mask the first key block
+// sees every row of every head of its group, the longest workgroup of the launch.
+constexpr int KV_STAGES = 3, KV_STAGE_BYTES = 2 * TILE_BYTES + 256;  // Q, dout, lse and delta of 32 rows
+constexpr int V_BYTES = 4 * TILE_BYTES;
+constexpr int KV_LDS = V_BYTES + 2 * KV_STAGES * KV_STAGE_BYTES;
+static_assert(KV_LDS >= 2 * 128 * 64 * 4, "the sum of one gradient needs 64 KiB");
+
+__device__ __forceinline__ int ceil_div(int a, int b) { return a > 0 ? (a + b - 1) / b : 0; }
+
+template <typename TR, bool CAUSAL>
+__global__ __launch_bounds__(512, 2) void backward_dkv128_kernel(BwdArgs a) {
+  typedef typename TR::elem T;
+  typedef typename TR::vec8 vec8;
+  typedef __attribute__((address_space(3))) vec8 lds_vec8;
+  typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+  constexpr bool kIsBf16 = __is_same(T, __bf16);
+  const KArgs& f = a.f;
+
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const unsigned smem_addr = (unsigned)(unsigned long)(lds_void*)smem;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave >> 2, gw = wave & 3;  // group, wavefront of it
+  const int lq = lane & 31, lh = lane >> 5;
+
+  const int nkb = (f.S + BM - 1) / BM;
+  const int nsplit = a.dkv_splits;
+  int wg, split;  // this workgroup takes entries split, split + nsplit, ... of key-block workgroup wg
+  split_of_workgroup(blockIdx.x, nsplit, f.B * f.Hkv, &wg, &split);
+  int pair, kb;
+  map_workgroup(wg, f.B * f.Hkv, nkb, &pair, &kb);
+  const int hk = pair % f.Hkv, b = pair / f.Hkv;
+  const int k0 = kb * BM, kw0 = k0 + gw * 32;
+  const int S = keys_of_batch(f, b);  // rows of dk / dv from here to f.S are written as zeros
+  if (k0 >= S) {
+    if (grp == 0) zero_key_rows<TR, D>(a, split, b, hk, kw0 + lq, lh);
+    return;
+  }
+  const int coff = CAUSAL ? causal_offset(f, S) : 0;
+
+  // (asm: the compiler would make every LDS read wait for all loads that store there)
+  auto dma16 = [&](const char* sbase, unsigned voff, unsigned lds_addr) __attribute__((always_inline)) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
+  };
+  auto dma4 = [&](const char* sbase, unsigned voff, unsigned lds_addr) __attribute__((always_inline)) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
+  };
+
+  // ---- V into LDS (wavefront w brings rows 16w .. 16w+15), this wavefront's K into registers -------------------------------------------
+  {
+    const char* vb = (const char*)((const T*)f.v + b * f.vs[0] + hk * f.vs[1] + (long long)k0 * f.vs[2]);
+    const unsigned ch = (unsigned)((lane & 15) ^ (4 * (lane >> 4)));
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const int row = 16 * wave + 4 * g + (lane >> 4);
+      const int rowc = k0 + row < S ? row : S - 1 - k0;  // rows past the end re-read the last key (never stored)
+      dma16(vb, ((unsigned)rowc * (unsigned)f.vs[2] + 8u * ch) * 2u, smem_addr + (4 * wave + g) * GROUP_BYTES);
+    }
+  }
+  u32x32 kv;  // k-step ks in elements 4ks .. 4ks+3
+  {
+    int row = kw0 + lq;
+    row = row < S ? row : S - 1;
+    const T* kr = (const T*)f.k + b * f.ks[0] + hk * f.ks[1] + row * f.ks[2] + 8 * lh;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ks++) {
+      const u32x4 k4 = *(const u32x4*)(kr + 16 * ks);
+#pragma unroll
+      for (int i = 0; i < 4; i++) kv[4 * ks + i] = k4[i];
+    }
+  }
+
+  // Query tiles it0 .. ntq-1 of each of the G heads see keys of this workgroup.  They are taken from the last tile down (or
+  // up: dkv_walks_up), the heads of a tile one after the other: every key block of a (batch, KV head) then starts at the same tile and
+  // walks in step with the others (one further down the causal triangle just stops earlier), so the tile one workgroup
+  // fetches from HBM is in the XCD's L2 for the others.  This workgroup's entries are split, split + nsplit, ... of that
+  // list; entry idx of ITS list belongs to group idx % 2.
+  const int ntq = (f.L + 31) / 32;
+  int it0 = 0;
+  if (CAUSAL) it0 = (k0 - coff > 0 ? k0 - coff : 0) / 32;
+  const int nt = ntq > it0 ? ntq - it0 : 0;
+  const int total = split < f.G * nt ? (f.G * nt - split + nsplit - 1) / nsplit : 0;
+  const int niter = (total + 1) / 2;  // iterations of either group (the second may have one entry less)
+  const bool walk_up = dkv_walks_up(a, CAUSAL, wg);
+  // wavefront gw of a group brings rows 8gw .. 8gw+7 (two groups of four) of the Q tile and of the dout tile into the group's ring, and
+  // the statistics (all four the same): lse of the 32 rows, then -delta, where the sums of dP - delta start
+  const unsigned ring_addr = smem_addr + V_BYTES + grp * KV_STAGES * KV_STAGE_BYTES;
+  const unsigned chunk = (unsigned)((lane & 15) ^ (4 * (lane >> 4)));
+  const u32x2 offs = {((unsigned)(lane >> 4) * (unsigned)f.qs[2] + 8u * chunk) * 2u, ((unsigned)(lane >> 4) * (unsigned)a.dos[2] + 8u * chunk) * 2u};
+  // what the next request is for: entry, head of the group, first row, and where this wavefront's part begins
+  int next = grp, next_head = (split + nsplit * grp) % f.G, next_row = 32 * (walk_up ? it0 + (split + nsplit * grp) / f.G : ntq - 1 - (split + nsplit * grp) / f.G);
+  const int dir = walk_up ? 32 : -32, step_head = 2 * nsplit % f.G, step_row = 2 * nsplit / f.G * dir;
+  const long long head0 = (long long)b * f.Hq + hk * f.G + next_head;
+  const char* q_next = (const char*)((const T*)f.q + b * f.qs[0] + (hk * f.G + next_head) * f.qs[1] + (long long)(next_row + 8 * gw) * f.qs[2]);
+  const char* g_next = (const char*)((const T*)a.dout + b * a.dos[0] + (hk * f.G + next_head) * a.dos[1] + (long long)(next_row + 8 * gw) * a.dos[2]);
+  const char* s_next = (const char*)(a.stats + 2 * (head0 * f.L + next_row));
+  const long long q_step = 2 * (step_head * f.qs[1] + step_row * f.qs[2]), q_wrap = 2 * (dir * f.qs[2] - f.G * f.qs[1]);
+  const long long g_step = 2 * (step_head * a.dos[1] + step_row * a.dos[2]), g_wrap = 2 * (dir * a.dos[2] - f.G * a.dos[1]);
+  const long long s_step = 8 * ((long long)step_head * f.L + step_row), s_wrap = 8 * (dir - (long long)f.G * f.L);
+  auto dma_next = [&](int stage) __attribute__((always_inline)) {
+    const bool more = next < total;
+    if (more) {
+      const unsigned at = ring_addr + stage * KV_STAGE_BYTES, mine = at + 2 * gw * GROUP_BYTES;
+      int ln;  // the lane number anew: nothing derived from it lives through the loop
+      asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+      if (__builtin_expect(next_row + 32 <= f.L, 1)) {
+        dma16(q_next, offs[0], mine);
+        dma16(g_next, offs[1], mine + TILE_BYTES);
+        dma16(q_next + 8 * f.qs[2], offs[0], mine + GROUP_BYTES);
+        dma16(g_next + 8 * a.dos[2], offs[1], mine + TILE_BYTES + GROUP_BYTES);
+        dma4(s_next, (unsigned)(2 * (ln & 31) + (ln >> 5)) * 4u, at + 2 * TILE_BYTES);
+      } else {  // rows past the end re-read the last row (weight forced to 0)
+        const unsigned ch = (unsigned)((ln & 15) ^ (4 * (ln >> 4)));
+        const char *qb = q_next - 16 * gw * f.qs[2], *gb = g_next - 16 * gw * a.dos[2];
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+          const int row = 8 * gw + 4 * g + (ln >> 4), rowc = next_row + row < f.L ? row : f.L - 1 - next_row;
+          dma16(qb, ((unsigned)rowc * (unsigned)f.qs[2] + 8u * ch) * 2u, mine + g * GROUP_BYTES);
+          dma16(gb, ((unsigned)rowc * (unsigned)a.dos[2] + 8u * ch) * 2u, mine + TILE_BYTES + g * GROUP_BYTES);
+        }
+        const int row = ln & 31, rowc = next_row + row < f.L ? row : f.L - 1 - next_row;
+        dma4(s_next, (unsigned)(2 * rowc + (ln >> 5)) * 4u, at + 2 * TILE_BYTES);
+      }
+    }
+    const bool wrap = next_head + step_head >= f.G;
+    next += 2;
+    next_head += step_head - (wrap ? f.G : 0), next_row += step_row + (wrap ? dir : 0);
+    q_next += q_step + (wrap ? q_wrap : 0), g_next += g_step + (wrap ? g_wrap : 0), s_next += s_step + (wrap ? s_wrap : 0);
+    return more;
+  };
+  int row_now = next_row;  // first rows of the tiles of this iteration and the next
+  dma_next(0);
+  int row_next = next_row;
+  dma_next(1);
+
+  // Iterations j0 .. j1-1 take the stream: tiles that hide nothing from the wavefront's keys.
+  int j0 = niter, j1 = niter;
+  if (kw0 + 32 <= S) {
+    int lo = it0, hi = f.L / 32;  // first such tile and the one behind the last
+    if (CAUSAL) {
+      const int first = ceil_div(kw0 + 31 - coff, 32);
+      lo = first > lo ? first : lo;
+    }
+    lo = lo < hi ? lo : hi;
+    const int e0 = f.G * (walk_up ? lo - it0 : ntq - hi), e1 = f.G * (walk_up ? hi - it0 : ntq - lo);
+    j0 = ceil_div(ceil_div(e0 - split, nsplit) - grp, 2);
+    j1 = ceil_div(ceil_div(e1 - split, nsplit) - grp, 2);
+    j0 = __builtin_amdgcn_readfirstlane(j0 < niter ? j0 : niter), j1 = __builtin_amdgcn_readfirstlane(j1 < niter ? j1 : niter);
+  }
+
+  f32x16 dkacc[DBLK], dvacc[DBLK];
+#pragma unroll
+  for (int i = 0; i < DBLK; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) dkacc[i][r] = 0.f, dvacc[i][r] = 0.f;
+  const float c = f.scale * kLog2e;
+  const float c_s = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, c)));
+  u32x4 row_addr, tr_addr;
+  operand_offsets(lane, row_addr, tr_addr);
+#pragma unroll
+  for (int i = 0; i < 4; i++) row_addr[i] += ring_addr, tr_addr[i] += ring_addr;
+  const unsigned v_from_ring = (unsigned)__builtin_amdgcn_readfirstlane((int)(smem_addr + gw * TILE_BYTES - ring_addr));
+
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+
+  // every wavefront is through with its reads, and the next tile is in place (what was asked for last may still be on its way)
+  auto sync = [&](bool more) __attribute__((always_inline)) {
+    if (more) asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // General form of iteration j.  The operand addresses are the ring's current stage's.
+  auto slow_step = [&](int j, int stage) __attribute__((always_inline)) {
+    const int i0 = row_now;
+    row_now = row_next, row_next = next_row;
+    const bool more = dma_next(stage == 0 ? 2 : stage - 1);
+    const unsigned at_stage = stage * KV_STAGE_BYTES;
+    const int idx = 2 * j + grp;
+    if (idx < total) {
+      int ln;
+      asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+      const int lh = ln >> 5;
+      const unsigned st = ring_addr + at_stage + 2 * TILE_BYTES + 16 * lh;
+      f32x16 s, d;
+#pragma unroll
+      for (int rg = 0; rg < 4; rg++) {
+        const f32x4 minus_delta = *(lds_f32x4*)(st + 128 + 32 * rg);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[4 * rg + e] = 0.f, d[4 * rg + e] = minus_delta[e];
+      }
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ks++) {
+        u32x4 w;
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[i] = kv[4 * ks + i];
+        s = TR::mfma32(*(lds_vec8*)(row_addr[ks >> 1] + 32 * (ks & 1)), __builtin_bit_cast(vec8, w), s);
+      }
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ks++)
+        d = TR::mfma32(*(lds_vec8*)(row_addr[ks >> 1] + TILE_BYTES + 32 * (ks & 1)), *(lds_vec8*)(row_addr[ks >> 1] + (v_from_ring - at_stage) + 32 * (ks & 1)), d);
+#pragma unroll
+      for (int rg = 0; rg < 4; rg++) {
+        const f32x4 lse = *(lds_f32x4*)(st + 32 * rg);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int r = 4 * rg + e;
+          s[r] = fast_exp2(fmaf(s[r], c, -lse[e]));
+          d[r] *= s[r];
+        }
+      }
+      // (a wavefront whose keys no row of the tile sees runs it with every weight 0)
+      if ((CAUSAL && kw0 + 31 > i0 + coff) || kw0 + 32 > S || i0 + 32 > f.L) {
+        const int key = kw0 + (ln & 31);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int qrow = i0 + 8 * (r >> 2) + 4 * lh + (r & 3);
+          const bool hidden = (key >= S) | (qrow >= f.L) | (CAUSAL && key > qrow + coff);
+          s[r] = hidden ? 0.f : s[r], d[r] = hidden ? 0.f : d[r];
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        f32x8 x, y;
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = s[8 * t + i], y[i] = d[8 * t + i];
+        const vec8 p = __builtin_convertvector(x, vec8), ds = __builtin_convertvector(y, vec8);
+#pragma unroll
+        for (int db = 0; db < DBLK; db++) {
+          const unsigned at = tr_addr[db] + 4 * t * GROUP_BYTES;
+          const s16x4 glo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + TILE_BYTES));
+          const s16x4 ghi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + TILE_BYTES + 2 * GROUP_BYTES));
+          const s16x4 qlo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
+          const s16x4 qhi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 2 * GROUP_BYTES));
+          dvacc[db] = TR::mfma32(__builtin_bit_cast(vec8, (s16x8)__builtin_shufflevector(glo, ghi, 0, 1, 2, 3, 4, 5, 6, 7)), p, dvacc[db]);
+          dkacc[db] = TR::mfma32(__builtin_bit_cast(vec8, (s16x8)__builtin_shufflevector(qlo, qhi, 0, 1, 2, 3, 4, 5, 6, 7)), ds, dkacc[db]);
+        }
+      }
+    }
+    const unsigned advance = stage == 2 ? 0u - 2 * KV_STAGE_BYTES : KV_STAGE_BYTES;
+#pragma unroll
+    for (int i = 0; i < 4; i++) row_addr[i] += advance, tr_addr[i] += advance;
+    sync(more);
+  };
+
+  int j = 0, stage = 0;
+#pragma nounroll
+  for (int turn = 0; turn < 2; turn++) {
+    for (const int end = turn == 0 ? j0 : niter; j < end; j++) {
+      slow_step(j, stage);
+      stage = stage == 2 ? 0 : stage + 1;
+    }
+    if (j >= j1) continue;
+    u32x32 ring;
+    f32x16 tmp[3];
+#pragma unroll
+    for (int i = 0; i < 32; i++) ring[i] = 0u;
+    asm volatile(TT_B128_DKV_PREFETCH : "+{v[224:255]}"(ring) : "{v[140:143]}"(row_addr) : "memory");
+#define TT_DKV_RUN(TXT)                                                                                                        \
+  asm volatile(TXT                                                                                                            \
+               : [o0] "+v"(dkacc[0]), [o1] "+v"(dkacc[1]), [o2] "+v"(dkacc[2]), [o3] "+v"(dkacc[3]), [o4] "+v"(dvacc[0]),       \
+                 [o5] "+v"(dvacc[1]), [o6] "+v"(dvacc[2]), [o7] "+v"(dvacc[3]), "+{v[224:255]}"(ring), "=&{v[144:159]}"(tmp[0]), \
+                 "=&{v[160:175]}"(tmp[1]), "=&{v[176:191]}"(tmp[2]), "+{v[140:143]}"(row_addr), "+{v[136:139]}"(tr_addr)       \
+               : [c] "s"(c_s), [vb] "s"(v_from_ring - at_stage), [st] "s"(ring_addr + at_stage), [adv] "s"(advance),           \
+                 [more] "s"(more), "{v[192:223]}"(kv), "{v[132:133]}"(offs)                                                    \
+               : "memory", "scc")
+    do {
+      row_now = row_next, row_next = next_row;
+      const int more = __builtin_amdgcn_readfirstlane((int)dma_next(stage == 0 ? 2 : stage - 1));
+      const unsigned at_stage = stage * KV_STAGE_BYTES, advance = stage == 2 ? 0u - 2 * KV_STAGE_BYTES : KV_STAGE_BYTES;
+      if constexpr (kIsBf16) TT_DKV_RUN(TT_B128_DKV_BF16);
+      else TT_DKV_RUN(TT_B128_DKV_F16);
+      stage = stage == 2 ? 0 : stage + 1;
+    } while (++j < j1);
+#undef TT_DKV_RUN
+    // the ring's last requests land, and the last matrix instructions end, before the compiler's code goes on with the registers
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15" : "+{v[224:255]}"(ring), "+v"(dkacc[0]), "+v"(dkacc[1]), "+v"(dkacc[2]), "+v"(dkacc[3]),
+                 "+v"(dvacc[0]), "+v"(dvacc[1]), "+v"(dvacc[2]), "+v"(dvacc[3]) : : "memory");
+  }
+
+  // ---- the second group's gradients join the first's, one (64 KiB of fp32) at a time -------------------------------------------------
+  int ln;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+  float* red = (float*)smem;
+  const int slot = gw * 64 + ln;
+#pragma unroll
+  for (int which = 0; which < 2; which++) {
+    f32x16* acc = which == 0 ? dkacc : dvacc;
+    if (grp == 1) {
+#pragma unroll
+      for (int db = 0; db < DBLK; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) red[(db * 16 + r) * 256 + slot] = acc[db][r];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int db = 0; db < DBLK; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[db][r] += red[(db * 16 + r) * 256 + slot];
+    }
+    __syncthreads();
+  }
+  if (grp == 0) store_key_grads<TR, D>(a, split, b, hk, kw0 + (ln & 31), ln >> 5, dkacc, dvacc, f.scale);
+}
+
 template <typename TR, bool CAUSAL>
 int launch_dq(const BwdArgs& a, hipStream_t stream) {
   static hipError_t state[kMaxDevices];
@@ -381,11 +700,30 @@ int launch_dq(const BwdArgs& a, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
+template <typename TR, bool CAUSAL>
+int launch_dkv(const BwdArgs& args, hipStream_t stream) {
+  BwdArgs a = args;
+  static hipError_t state[kMaxDevices];
+  static bool done[kMaxDevices];
+  const hipError_t granted = grant_dynamic_lds((const void*)backward_dkv128_kernel<TR, CAUSAL>, KV_LDS, state, done);
+  if (granted != hipSuccess) return (int)granted;
+  static int round_cache[kMaxDevices];
+  a.dkv_round = CAUSAL ? dkv_round_of((const void*)backward_dkv128_kernel<TR, CAUSAL>, 512, KV_LDS, round_cache) : 0;
+  const long long grid = (long long)a.f.B * a.f.Hkv * ((a.f.S + BM - 1) / BM) * a.dkv_splits;
+  hipLaunchKernelGGL((backward_dkv128_kernel<TR, CAUSAL>), dim3((unsigned)grid), dim3(512), KV_LDS, stream, a);
+  return (int)hipGetLastError();
+}
+
 }  // namespace
 
 int launch_backward_dq_d128(const BwdArgs& a, bool bf16, hipStream_t stream) {
   if (bf16) return a.f.causal ? launch_dq<BF16, true>(a, stream) : launch_dq<BF16, false>(a, stream);
   return a.f.causal ? launch_dq<F16, true>(a, stream) : launch_dq<F16, false>(a, stream);
+}
+
+int launch_backward_dkv_d128(const BwdArgs& a, bool bf16, hipStream_t stream) {
+  if (bf16) return a.f.causal ? launch_dkv<BF16, true>(a, stream) : launch_dkv<BF16, false>(a, stream);
+  return a.f.causal ? launch_dkv<F16, true>(a, stream) : launch_dkv<F16, false>(a, stream);
 }
 
 }  // namespace ttsdpa

@@ -11,19 +11,19 @@
 //      and streams the keys in tiles of 64 (32 at head_dim 128) like the forward kernel: S^T = K.Q^T, an online softmax with a lazily
 //      raised maximum (so lse_i needs no pass of its own), dP^T = V.dout^T, dS^T, dq^T += K^T.dS^T.  At the end
 //      dq = scale/l * accumulator, and (lse_i, delta_i) go to scratch for the second kernel.
-//   2. backward_dkv_mfma_kernel (head_dim 64) / backward_dkv128_kernel (head_dim 128) — a workgroup owns 128 keys of
+//   2. backward_dkv_mfma_kernel — a workgroup owns 128 keys of
 //      one (batch, kv head), a wavefront 32 of them, and streams the query rows of every head of the group in tiles
 //      of 32: S = Q.K^T, P from lse, dP = dout.V^T, dS, dv^T += dout^T.P, dk^T += Q^T.dS.
+// head_dim 128 without an attnMask takes sdpa_backward_d128.hip's forms of both.
 // Both compute 32 x 32 score blocks with v_mfma_f32_32x32x16 whose accumulator layout (lane = column, registers = rows)
 // is the B operand of the following product, so P and dS go from registers to the matrix cores without touching LDS;
 // the register-staged tiles are kept in LDS twice where both a row-major operand and a transposed one
-// (ds_read_b64_tr_b16) are read from them, each copy with the row pitch that makes its reads conflict-free; the
-// head_dim-128 dk/dv kernel keeps one swizzled copy instead (see there).
+// (ds_read_b64_tr_b16) are read from them, each copy with the row pitch that makes its reads conflict-free.
 // Seven matrix products in all, against five in the textbook count (the scores are computed in both kernels).
-// When a call has too few key blocks to fill and balance the chip, the query stream of a key block is dealt out to 2-4
+// When a call has too few key blocks to fill and balance the chip, the query stream of a key block is dealt out to several
 // workgroups of kernel 2, which leave fp32 partial sums in scratch, and backward_dkv_sum_kernel (sdpa_common.h) adds
-// them in a fixed order.  Likewise kernel 1: with fewer than 512 query blocks the key range of a block is dealt out to
-// 2-8 workgroups, whose unnormalised fp32 sums and (maximum, sum of exponentials) backward_dq_merge_kernel combines.
+// them in a fixed order.  Likewise kernel 1: the key range of a query block is dealt out to several workgroups, whose unnormalised
+// fp32 sums and (maximum, sum of exponentials) backward_dq_merge_kernel combines.  How many: backward_splits_16bit.
 
 #include "sdpa_common.h"
 
@@ -65,58 +65,6 @@ __device__ __forceinline__ vec8 transposed_operand(const void* lane_base, int by
   s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)((const char*)lane_base + byte_off_hi));
   s16x8 r = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_bit_cast(vec8, r);
-}
-
-// A lane's share of the dk / dv rows of key `key` (accumulator layout: registers 4rg .. 4rg+3 of block db are elements
-// 32db + 8rg + 4lh .. +3) goes to the gradient tensors, or — when the key block's query stream is split over several
-// workgroups — as fp32 to this split's partial sums, dense [split][dk | dv][B][Hkv][S][D].
-// PAD: the tensors' head_dim a.f.D is a multiple of 8 below D; only its columns are written.
-template <typename TR, int D, bool PAD = false>
-__device__ __forceinline__ void store_key_grads(const BwdArgs& a, int split, int b, int hk, int key, int lh,
-                                                const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32], float scale) {
-  typedef typename TR::elem T;
-  if (key >= a.f.S) return;
-  if (a.dkv_splits > 1) {
-    const int have = PAD ? a.f.D : D;
-    const long long plane = (long long)a.f.B * a.f.Hkv * a.f.S * have;
-    float* dkp = a.partial + 2 * split * plane + (((long long)b * a.f.Hkv + hk) * a.f.S + key) * have;
-#pragma unroll
-    for (int db = 0; db < D / 32; db++)
-#pragma unroll
-      for (int rg = 0; rg < 4; rg++) {
-        f32x4 x, y;
-#pragma unroll
-        for (int i = 0; i < 4; i++) x[i] = dkacc[db][4 * rg + i] * scale, y[i] = dvacc[db][4 * rg + i];
-        if (PAD && 32 * db + 8 * rg + 4 * lh >= have) continue;
-        *(f32x4*)(dkp + 32 * db + 8 * rg + 4 * lh) = x;
-        *(f32x4*)(dkp + plane + 32 * db + 8 * rg + 4 * lh) = y;
-      }
-    return;
-  }
-  T* dkp = (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + key * a.dks[2];
-  T* dvp = (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + key * a.dvs[2];
-#pragma unroll
-  for (int db = 0; db < D / 32; db++)
-#pragma unroll
-    for (int rg = 0; rg < 4; rg++) {
-      f32x4 x, y;
-#pragma unroll
-      for (int i = 0; i < 4; i++) x[i] = dkacc[db][4 * rg + i] * scale, y[i] = dvacc[db][4 * rg + i];
-      if (PAD && 32 * db + 8 * rg + 4 * lh >= a.f.D) continue;
-      *(typename TR::vec4*)(dkp + 32 * db + 8 * rg + 4 * lh) = __builtin_convertvector(x, typename TR::vec4);
-      *(typename TR::vec4*)(dvp + 32 * db + 8 * rg + 4 * lh) = __builtin_convertvector(y, typename TR::vec4);
-    }
-}
-
-// dk and dv rows of a key no query row attends to (at or beyond the batch entry's key count): zeros.
-template <typename TR, int D, bool PAD = false>
-__device__ __forceinline__ void zero_key_rows(const BwdArgs& a, int split, int b, int hk, int key, int lh) {
-  f32x16 zero[D / 32];
-#pragma unroll
-  for (int i = 0; i < D / 32; i++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) zero[i][r] = 0.f;
-  store_key_grads<TR, D, PAD>(a, split, b, hk, key, lh, zero, zero, 0.f);
 }
 
 template <typename vec8>
@@ -616,269 +564,6 @@ __global__ __launch_bounds__(256, (D > 64 ? 1 : 2)) void backward_dkv_mfma_kerne
   store_key_grads<TR, D, PAD>(a, split, b, hk, kw0 + lq, lh, dkacc, dvacc, f.scale);
 }
 
-// ---- kernel 2 for head_dim 128: the same products with the tiles brought in by direct global->LDS loads ----------------
-// With register-staged tiles the kernel above needs ~330 registers per lane at head_dim 128: one wavefront per SIMD,
-// whose vector work nothing overlaps.  Here the Q / dout tiles (and the workgroup's V rows, once) go from global memory
-// straight into LDS (global_load_lds_dwordx4: 64 lanes x 16 bytes = four 256-byte rows per instruction, unpadded), which
-// frees the staging registers and the V fragments: under 256 registers, two wavefronts per SIMD.  Rows are 16 chunks of
-// 16 bytes; chunk c of row r sits in slot c ^ f(r), f(r) = 4*(r%4) + (r/4)%4, which makes both the row-major operand
-// reads (ds_read_b128) and the transposed ones (ds_read_b64_tr_b16) conflict-free on one copy of a tile.
-//
-// Eight wavefronts in two groups of four: both groups own the same 128 keys and take alternate tiles of the query
-// stream, each with its own three-stage ring of tiles, and group 1's partial dk / dv are added to group 0's through
-// LDS at the end.  Under a causal mask the first key block of a KV head sees every query row of every head of the
-// group — the longest workgroup of the launch; two groups halve that critical path.
-namespace dkv128 {
-constexpr int D = 128;
-constexpr int ROW_BYTES = D * 2;
-constexpr int TILE_BYTES = BQ * ROW_BYTES;                // one 32-row tile of Q or dout
-constexpr int STAGE_BYTES = 2 * TILE_BYTES + 2 * BQ * 4;  // Q, dout, (lse2, delta) per row
-constexpr int NSTAGE = 3;
-constexpr int V_BYTES = BM * ROW_BYTES;                   // the workgroup's V rows
-constexpr int LDS_BYTES = V_BYTES + 2 * NSTAGE * STAGE_BYTES;
-static_assert(LDS_BYTES >= 2 * 128 * 64 * 4, "the reduction of one gradient needs 64 KiB");
-__device__ __forceinline__ int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
-}  // namespace dkv128
-
-typedef __attribute__((address_space(3))) void lds_void;
-
-template <typename TR, bool CAUSAL>
-__global__ __launch_bounds__(512, 1) void backward_dkv128_kernel(BwdArgs a) {
-  using namespace dkv128;
-  typedef typename TR::elem T;
-  typedef typename TR::vec8 vec8;
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  constexpr int KSTEPS = D / 16, DBLK = D / 32;
-  const KArgs& f = a.f;
-
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const unsigned smem_addr = (unsigned)(unsigned long)(lds_void*)smem;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int grp = wave >> 2, gw = wave & 3;  // group, wavefront inside the group
-  const int lq = lane & 31, lh = lane >> 5;
-
-  const int nkb = (f.S + BM - 1) / BM;
-  const int nsplit = a.dkv_splits;
-  int wg, split;  // this workgroup takes entries split, split + nsplit, ... of key-block workgroup wg
-  split_of_workgroup(blockIdx.x, nsplit, f.B * f.Hkv, &wg, &split);
-  int pair, kb;
-  map_workgroup(wg, f.B * f.Hkv, nkb, &pair, &kb);
-  const int hk = pair % f.Hkv, b = pair / f.Hkv;
-  const int k0 = kb * BM, kw0 = k0 + gw * 32;
-  const int S = keys_of_batch(f, b);  // rows of dk / dv from here to f.S are written as zeros
-  if (k0 >= S) {
-    if (grp == 0) zero_key_rows<TR, D>(a, split, b, hk, kw0 + lq, lh);
-    return;
-  }
-  const int coff = CAUSAL ? causal_offset(f, S) : 0;
-
-  // Issued as asm so that the compiler does not see stores to LDS (it would make every LDS read wait for all loads).
-  auto dma16 = [&](const char* sbase, unsigned voff, unsigned lds_addr) __attribute__((always_inline)) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
-  };
-  auto dma4 = [&](const char* sbase, unsigned voff, unsigned lds_addr) __attribute__((always_inline)) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
-  };
-  const int drow = lane >> 4, dslot = lane & 15;  // this lane's row and slot inside a 4-row group of a load
-
-  // ---- the workgroup's V rows into LDS (wavefront w brings rows 16w .. 16w+15), this wavefront's K rows into registers ----
-  {
-    const char* vb = (const char*)((const T*)f.v + b * f.vs[0] + hk * f.vs[1] + (long long)k0 * f.vs[2]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int row = 16 * wave + 4 * i + drow;
-      const int rowc = k0 + row < S ? row : S - 1 - k0;  // rows past the end re-read the last key (never stored)
-      const unsigned voff = ((unsigned)rowc * (unsigned)f.vs[2] + 8u * (unsigned)(dslot ^ swz(row))) * 2u;
-      dma16(vb, voff, smem_addr + (16 * wave + 4 * i) * ROW_BYTES);
-    }
-  }
-  vec8 kreg[KSTEPS];
-  {
-    int row = kw0 + lq;
-    row = row < S ? row : S - 1;
-    const T* kr = (const T*)f.k + b * f.ks[0] + hk * f.ks[1] + row * f.ks[2] + 8 * lh;
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) kreg[ks] = *(const vec8*)(kr + 16 * ks);
-  }
-  f32x16 dkacc[DBLK], dvacc[DBLK];
-#pragma unroll
-  for (int i = 0; i < DBLK; i++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) dkacc[i][r] = 0.f, dvacc[i][r] = 0.f;
-  const float c = f.scale * kLog2e;
-
-  // Query tiles it0 .. ntq-1 of each of the G heads see keys of this workgroup.  They are taken from the last tile down,
-  // the heads of a tile one after the other: every key block of a (batch, kv head) then starts at the same tile and walks
-  // in step with the others (a block further down the causal triangle just stops earlier), so the tile one workgroup
-  // fetches from HBM is in the XCD's L2 for the others.  This workgroup's entries are split, split + nsplit, ... of that
-  // list; entry idx of ITS list belongs to group idx % 2.
-  const int ntq = (f.L + BQ - 1) / BQ;
-  int it0 = 0;
-  if (CAUSAL) it0 = (k0 - coff > 0 ? k0 - coff : 0) / BQ;
-  const int nt = ntq > it0 ? ntq - it0 : 0;
-  const int total = split < f.G * nt ? (f.G * nt - split + nsplit - 1) / nsplit : 0;
-  const int niter = (total + 1) / 2;  // iterations of either group (the second may have one entry less)
-  const bool walk_up = dkv_walks_up(a, CAUSAL, wg);  // every second round of an XCD's workgroups (sdpa_common.h)
-  auto tile_of = [&](int entry) __attribute__((always_inline)) { return walk_up ? it0 + entry / f.G : ntq - 1 - entry / f.G; };
-
-  // wavefront gw of a group brings rows 8gw .. 8gw+7 of the Q tile and of the dout tile (two loads each) into the
-  // group's ring; its first wavefront the statistics as well
-  const unsigned ring_addr = smem_addr + V_BYTES + grp * NSTAGE * STAGE_BYTES;
-  auto dma_tile = [&](int idx, int stage) __attribute__((always_inline)) {
-    const int entry = split + nsplit * idx;
-    const int h = hk * f.G + entry % f.G;
-    const int i0 = tile_of(entry) * BQ;
-    const char* qb = (const char*)((const T*)f.q + b * f.qs[0] + h * f.qs[1] + (long long)i0 * f.qs[2]);
-    const char* gb = (const char*)((const T*)a.dout + b * a.dos[0] + h * a.dos[1] + (long long)i0 * a.dos[2]);
-    const unsigned at = ring_addr + stage * STAGE_BYTES;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      const int row = 8 * gw + 4 * i + drow;
-      const int rowc = i0 + row < f.L ? row : f.L - 1 - i0;  // rows past the end re-read the last row (weight forced to 0)
-      const unsigned chunk = (unsigned)(dslot ^ swz(row));
-      dma16(qb, ((unsigned)rowc * (unsigned)f.qs[2] + 8u * chunk) * 2u, at + (8 * gw + 4 * i) * ROW_BYTES);
-      dma16(gb, ((unsigned)rowc * (unsigned)a.dos[2] + 8u * chunk) * 2u, at + TILE_BYTES + (8 * gw + 4 * i) * ROW_BYTES);
-    }
-    if (gw == 0) {  // 32 rows x (lse2, delta): 64 floats, one per lane
-      const char* sb = (const char*)(a.stats + 2 * (((long long)b * f.Hq + h) * f.L + i0));
-      const int row = lane >> 1;
-      const int rowc = i0 + row < f.L ? row : f.L - 1 - i0;
-      dma4(sb, (unsigned)(2 * rowc + (lane & 1)) * 4u, at + 2 * TILE_BYTES);
-    }
-  };
-
-  // ---- LDS operand addresses (bytes inside a tile), loop-invariant ----------------------------------------------------
-  // row-major operand, k-step ks: row lq, chunk 2ks + lh  ->  lq*256 + 16*((2ks + lh) ^ f(lq)) = r_base ^ (32*ks)
-  const unsigned r_base = (unsigned)(lq * ROW_BYTES + 16 * (lh ^ swz(lq)));
-  // transposed operand (db, ld) of k-step t: this lane points at row 16t + 8ld + 4lh + s/4, elements
-  // 32db + 16*dhalf + 4*(s%4) .. +3 (s = lane%16, dhalf = (lane/16)%2) and receives X[16t + 8ld + 4lh + 0..3][32db + lq]
-  unsigned t_base[2];
-  {
-    const int s = lane & 15, dhalf = (lane >> 4) & 1;
-#pragma unroll
-    for (int ld = 0; ld < 2; ld++) {
-      const int row = 8 * ld + 4 * lh + (s >> 2);  // f(row) does not depend on t
-      const int c0 = 2 * dhalf + ((s & 3) >> 1);
-      t_base[ld] = (unsigned)(row * ROW_BYTES + 16 * (c0 ^ swz(row)) + 8 * (s & 1));  // ^ (64*db) selects the 32-column block
-    }
-  }
-  const char* vown = smem + 32 * gw * ROW_BYTES;
-  const char* ring = smem + V_BYTES + grp * NSTAGE * STAGE_BYTES;
-
-  // entries grp, grp + 2 of the list on their way, everything landed before the first use
-  if (grp < total) dma_tile(grp, 0);
-  if (grp + 2 < total) dma_tile(grp + 2, 1);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-
-  const int key = kw0 + lq;
-  int cur = 0;  // j % 3
-  for (int j = 0; j < niter; j++) {
-    const int idx = 2 * j + grp;
-    const int nxt2 = cur == 0 ? 2 : cur - 1;  // (j + 2) % 3: last read in iteration j-1, which a barrier ended
-    const bool more = idx + 4 < total;
-    if (more) dma_tile(idx + 4, nxt2);
-    if (idx < total) {
-      const int i0 = tile_of(split + nsplit * idx) * BQ;
-      const char* qt = ring + cur * STAGE_BYTES;
-      const char* gt = qt + TILE_BYTES;
-      const float* st = (const float*)(qt + 2 * TILE_BYTES);
-
-      f32x16 sacc, dpacc;
-#pragma unroll
-      for (int r = 0; r < 16; r++) sacc[r] = 0.f, dpacc[r] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ks++) sacc = TR::mfma32(*(const vec8*)(qt + (r_base ^ (unsigned)(32 * ks))), kreg[ks], sacc);
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ks++)
-        dpacc = TR::mfma32(*(const vec8*)(gt + (r_base ^ (unsigned)(32 * ks))), *(const vec8*)(vown + (r_base ^ (unsigned)(32 * ks))), dpacc);
-
-#pragma unroll
-      for (int rg = 0; rg < 4; rg++) {
-        const f32x4 s0 = *(const f32x4*)(st + 2 * (8 * rg + 4 * lh));      // (lse2, delta) of rows 8rg+4lh+0, +1
-        const f32x4 s1 = *(const f32x4*)(st + 2 * (8 * rg + 4 * lh) + 4);  // ... +2, +3
-        const float lse2[4] = {s0[0], s0[2], s1[0], s1[2]};
-        const float dl[4] = {s0[1], s0[3], s1[1], s1[3]};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int r = 4 * rg + e;
-          const float p = fast_exp2(fmaf(sacc[r], c, -lse2[e]));
-          sacc[r] = p;
-          dpacc[r] = p * (dpacc[r] - dl[e]);
-        }
-      }
-      // only tiles on or above the diagonal, the last key block and the last query tile hide anything; a wavefront whose
-      // keys no row of the tile sees runs the tile with every weight 0
-      if ((CAUSAL && kw0 + 31 > i0 + coff) || kw0 + 32 > S || i0 + BQ > f.L) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int qrow = i0 + 8 * (r >> 2) + 4 * lh + (r & 3);
-          if (key >= S || qrow >= f.L || (CAUSAL && key > qrow + coff)) sacc[r] = 0.f, dpacc[r] = 0.f;
-        }
-      }
-      vec8 pb[2], dsb[2];
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        pb[t] = regs_to_operand<vec8>(sacc, t);
-        dsb[t] = regs_to_operand<vec8>(dpacc, t);
-      }
-#pragma unroll
-      for (int db = 0; db < DBLK; db++)
-#pragma unroll
-        for (int t = 0; t < 2; t++) {
-          const unsigned lo = (t_base[0] ^ (unsigned)(64 * db)) + 16 * t * ROW_BYTES, hi = (t_base[1] ^ (unsigned)(64 * db)) + 16 * t * ROW_BYTES;
-          const s16x4 glo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(gt + lo));
-          const s16x4 ghi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(gt + hi));
-          const s16x4 qlo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(qt + lo));
-          const s16x4 qhi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(qt + hi));
-          dvacc[db] = TR::mfma32(__builtin_bit_cast(vec8, __builtin_shufflevector(glo, ghi, 0, 1, 2, 3, 4, 5, 6, 7)), pb[t], dvacc[db]);
-          dkacc[db] = TR::mfma32(__builtin_bit_cast(vec8, __builtin_shufflevector(qlo, qhi, 0, 1, 2, 3, 4, 5, 6, 7)), dsb[t], dkacc[db]);
-        }
-    }
-    // Entry idx + 2 must have landed before the next iteration; the loads of entry idx + 4, issued above, may stay in
-    // flight (four per wavefront, five for the one that also brings the statistics; they complete in issue order).
-    if (more) {
-      if (gw == 0) {
-        asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-      } else {
-        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      }
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    __syncthreads();
-    cur = cur == 2 ? 0 : cur + 1;
-  }
-
-  // ---- group 1's partial gradients join group 0's, one gradient (64 KiB of fp32) at a time ------------------------------
-  float* red = (float*)smem;
-  const int slot = gw * 64 + lane;
-#pragma unroll
-  for (int which = 0; which < 2; which++) {
-    f32x16* acc = which == 0 ? dkacc : dvacc;
-    if (grp == 1) {
-#pragma unroll
-      for (int db = 0; db < DBLK; db++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) red[(db * 16 + r) * 256 + slot] = acc[db][r];
-    }
-    __syncthreads();
-    if (grp == 0) {
-#pragma unroll
-      for (int db = 0; db < DBLK; db++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[db][r] += red[(db * 16 + r) * 256 + slot];
-    }
-    __syncthreads();
-  }
-
-  if (grp == 0) store_key_grads<TR, D>(a, split, b, hk, key, lh, dkacc, dvacc, f.scale);
-}
-
 template <typename TR, int D, bool CAUSAL, bool MASKED, bool PAD>
 int launch_k(const BwdArgs& args, hipStream_t stream) {
   BwdArgs a = args;
@@ -887,45 +572,35 @@ int launch_k(const BwdArgs& args, hipStream_t stream) {
   typedef BwdLds<D> Lds;
   // with an attnMask, head_dim 128 takes the register-staged dk/dv kernel: the mask's 16 values per tile do not fit the
   // 256 registers of the direct-to-LDS one
-  constexpr bool DMA = D == 128 && !MASKED && !PAD;
-  static hipError_t state1[kMaxDevices], state2[kMaxDevices];
-  static bool done1[kMaxDevices], done2[kMaxDevices];
-  hipError_t e = hipSuccess;
-  if constexpr (!DMA) {
-    e = grant_dynamic_lds((const void*)backward_dq_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>, DqTile<D>::BYTES, state1, done1);
-    if (e != hipSuccess) return (int)e;
-  }
-  if (DMA) {
-    e = grant_dynamic_lds((const void*)backward_dkv128_kernel<TR, CAUSAL>, dkv128::LDS_BYTES, state2, done2);
-  } else {
-    e = grant_dynamic_lds((const void*)backward_dkv_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>, Lds::KV_BYTES, state2, done2);
-  }
-  if (e != hipSuccess) return (int)e;
+  // (head_dim 128 with an attnMask takes the register-staged kernels here: the mask's 16 values per tile do not fit the 256 registers
+  // of the others)
+  constexpr bool STREAMS = D == 128 && !MASKED && !PAD;
   const long long g1 = (long long)a.f.B * a.f.Hq * ((a.f.L + BM - 1) / BM) * a.dq_splits;
   const long long g2 = (long long)a.f.B * a.f.Hkv * ((a.f.S + BM - 1) / BM) * a.dkv_splits;
-  static int round_cache[kMaxDevices];
-  a.dkv_round = !CAUSAL ? 0
-                : DMA   ? dkv_round_of((const void*)backward_dkv128_kernel<TR, CAUSAL>, 512, dkv128::LDS_BYTES, round_cache)
-                        : dkv_round_of((const void*)backward_dkv_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>, 256, Lds::KV_BYTES, round_cache);
-  if constexpr (DMA) {
-    const int rc = launch_backward_dq_d128(a, __is_same(TR, BF16), stream);
-    if (rc != 0) return rc;
+  int rc;
+  if constexpr (STREAMS) {
+    rc = launch_backward_dq_d128(a, __is_same(TR, BF16), stream);
   } else {
+    static hipError_t state1[kMaxDevices], state2[kMaxDevices];
+    static bool done1[kMaxDevices], done2[kMaxDevices];
+    rc = (int)grant_dynamic_lds((const void*)backward_dq_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>, DqTile<D>::BYTES, state1, done1);
+    if (rc != 0) return rc;
+    rc = (int)grant_dynamic_lds((const void*)backward_dkv_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>, BwdLds<D>::KV_BYTES, state2, done2);
+    if (rc != 0) return rc;
+    static int round_cache[kMaxDevices];
+    a.dkv_round = CAUSAL ? dkv_round_of((const void*)backward_dkv_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>, 256, BwdLds<D>::KV_BYTES, round_cache) : 0;
     hipLaunchKernelGGL((backward_dq_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>), dim3((unsigned)g1), dim3(256), DqTile<D>::BYTES, stream, a);
-    e = hipGetLastError();
-    if (e != hipSuccess) return (int)e;
+    rc = (int)hipGetLastError();
   }
-  if (a.dq_splits > 1) {
-    const int rc = launch_backward_dq_merge<typename TR::elem>(a, stream);
-    if (rc != 0) return rc;
-  }
-  if (DMA) {
-    hipLaunchKernelGGL((backward_dkv128_kernel<TR, CAUSAL>), dim3((unsigned)g2), dim3(512), dkv128::LDS_BYTES, stream, a);
+  if (rc == 0 && a.dq_splits > 1) rc = launch_backward_dq_merge<typename TR::elem>(a, stream);
+  if (rc != 0) return rc;
+  if constexpr (STREAMS) {
+    rc = launch_backward_dkv_d128(a, __is_same(TR, BF16), stream);
   } else {
-    hipLaunchKernelGGL((backward_dkv_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>), dim3((unsigned)g2), dim3(256), Lds::KV_BYTES, stream, a);
+    hipLaunchKernelGGL((backward_dkv_mfma_kernel<TR, D, CAUSAL, MASKED, PAD>), dim3((unsigned)g2), dim3(256), BwdLds<D>::KV_BYTES, stream, a);
+    rc = (int)hipGetLastError();
   }
-  e = hipGetLastError();
-  if (e != hipSuccess || a.dkv_splits == 1) return (int)e;
+  if (rc != 0 || a.dkv_splits == 1) return rc;
   return launch_backward_dkv_sum<typename TR::elem>(a, stream);
 }
 

@@ -565,8 +565,9 @@ int launch_backward_dq_merge(const BwdArgs& a, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 int launch_backward_general(const BwdArgs& a, int dtype, hipStream_t stream);
-int launch_backward_dq_d128(const BwdArgs& a, bool bf16, hipStream_t stream);  // its dq kernel at head_dim 128 without an attnMask
 int launch_backward_mfma(const BwdArgs& a, int dtype, hipStream_t stream);  // fp16/bf16, head_dim 64 or 128
+int launch_backward_dq_d128(const BwdArgs& a, bool bf16, hipStream_t stream);   // its kernels at head_dim 128 without an attnMask
+int launch_backward_dkv_d128(const BwdArgs& a, bool bf16, hipStream_t stream);
 int launch_backward_f32(const BwdArgs& a, int dtype, hipStream_t stream);   // on the fp32 matrix cores, head_dim 64 or 128: fp32, and fp16/bf16 with an attnMask
 
 // Workgroup n -> (pair, block) for npair (batch, head) pairs of nblk blocks each, block 0 the longest under a causal
@@ -592,6 +593,58 @@ __device__ __forceinline__ void map_workgroup(int n, int npair, int nblk, int* p
 template <bool PIN>
 __device__ __forceinline__ void pin_accumulator(f32x16& acc) {
   if constexpr (PIN) asm volatile("" : "+a"(acc));
+}
+
+// A lane's share of the dk / dv rows of key `key` (accumulator layout: registers 4rg .. 4rg+3 of block db are elements
+// 32db + 8rg + 4lh .. +3) goes to the gradient tensors, or — when the key block's query stream is split over several
+// workgroups — as fp32 to this split's partial sums, dense [split][dk | dv][B][Hkv][S][D].
+// PAD: the tensors' head_dim a.f.D is a multiple of 8 below D; only its columns are written.
+template <typename TR, int D, bool PAD = false>
+__device__ __forceinline__ void store_key_grads(const BwdArgs& a, int split, int b, int hk, int key, int lh,
+                                                const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32], float scale) {
+  typedef typename TR::elem T;
+  if (key >= a.f.S) return;
+  if (a.dkv_splits > 1) {
+    const int have = PAD ? a.f.D : D;
+    const long long plane = (long long)a.f.B * a.f.Hkv * a.f.S * have;
+    float* dkp = a.partial + 2 * split * plane + (((long long)b * a.f.Hkv + hk) * a.f.S + key) * have;
+#pragma unroll
+    for (int db = 0; db < D / 32; db++)
+#pragma unroll
+      for (int rg = 0; rg < 4; rg++) {
+        f32x4 x, y;
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = dkacc[db][4 * rg + i] * scale, y[i] = dvacc[db][4 * rg + i];
+        if (PAD && 32 * db + 8 * rg + 4 * lh >= have) continue;
+        *(f32x4*)(dkp + 32 * db + 8 * rg + 4 * lh) = x;
+        *(f32x4*)(dkp + plane + 32 * db + 8 * rg + 4 * lh) = y;
+      }
+    return;
+  }
+  T* dkp = (T*)a.dk + b * a.dks[0] + hk * a.dks[1] + key * a.dks[2];
+  T* dvp = (T*)a.dv + b * a.dvs[0] + hk * a.dvs[1] + key * a.dvs[2];
+#pragma unroll
+  for (int db = 0; db < D / 32; db++)
+#pragma unroll
+    for (int rg = 0; rg < 4; rg++) {
+      f32x4 x, y;
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[i] = dkacc[db][4 * rg + i] * scale, y[i] = dvacc[db][4 * rg + i];
+      if (PAD && 32 * db + 8 * rg + 4 * lh >= a.f.D) continue;
+      *(typename TR::vec4*)(dkp + 32 * db + 8 * rg + 4 * lh) = __builtin_convertvector(x, typename TR::vec4);
+      *(typename TR::vec4*)(dvp + 32 * db + 8 * rg + 4 * lh) = __builtin_convertvector(y, typename TR::vec4);
+    }
+}
+
+// dk and dv rows of a key no query row attends to (at or beyond the batch entry's key count): zeros.
+template <typename TR, int D, bool PAD = false>
+__device__ __forceinline__ void zero_key_rows(const BwdArgs& a, int split, int b, int hk, int key, int lh) {
+  f32x16 zero[D / 32];
+#pragma unroll
+  for (int i = 0; i < D / 32; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) zero[i][r] = 0.f;
+  store_key_grads<TR, D, PAD>(a, split, b, hk, key, lh, zero, zero, 0.f);
 }
 
 // Direction in which a dk/dv workgroup walks the query tiles it0 .. ntq-1 that see its key block.  The workgroups of an XCD
