@@ -29,10 +29,10 @@ dk/dv, a tile of 32 query rows against the wavefront's 32 keys (K in registers),
     8 .. 15   dP - delta = dout . V^T - delta (the chain's first accumulator)      P = exp2(S c - lse) from slot 9
     16 .. 23  dv^T += dout^T . P                                                                      dS = (dP - delta) P from slot 18
     24 .. 31  dk^T += Q^T . dS
-    Fixed registers: v[136:139] transposed, v[140:143] row operand addresses
+    Fixed registers: v[128:131] addresses of V's rows, v[136:139] transposed, v[140:143] row operand addresses
     v[144:151]  lse of rows, quads 0 and 1 (2 and 3 lie in v[152:159] before P does)     v[152:159] P in pairs of 16 bits
     v[160:175]  dP (then dS)      v[176:191]  S (then P)      v[192:223]  K, 8 k-steps x 4 registers      v[224:255]  operand ring
-    Named: o0-o3 dk, o4-o7 dv (read-write), c = scale*log2(e), vb = the wavefront's V rows from the stage's start, st = the stage's start,
+    Named: o0-o3 dk, o4-o7 dv (read-write), c = scale*log2(e), st = the stage's start,
     adv = the next stage's from there, more = whether the step has asked for a tile (scalar registers).  One stream for all stages: with one
     each, a workgroup's first steps waited for their instructions (of 36 to 90 us on 165 to 480 rows, 2 to 5).
 
@@ -134,7 +134,7 @@ def dq_step(u, elem):
 
 # ---- dk/dv -----------------------------------------------------------------------------------------------------------------
 KV_SLOTS = 32
-KTR, KR, KL, KPB, KD, KS, KK = 136, 140, 144, 152, 160, 176, 192
+KV, KTR, KR, KL, KPB, KD, KS, KK = 128, 136, 140, 144, 152, 160, 176, 192
 # operands of a step in the order of their use: the slots' counts
 KV_OPS = [1] * 8 + [2] * 8 + [1] * 16
 KV_ENTRIES = sum(KV_OPS)  # a multiple of RING: the same registers in every step
@@ -160,7 +160,7 @@ def kv_fetch(e):
         ks, of_v = (e - 8) // 2, (e - 8) % 2
         if not of_v:
             return [kv_row(r, KR + ks // 2, ks, TILE)]
-        return ["v_add_u32 v%d, %%[vb], v%d" % (r, KR + ks // 2), kv_row(r, r, ks, 0)]  # (the address in a register of the operand)
+        return [kv_row(r, KV + ks // 2, ks, 0)]
     t, db = (e - 24) % 8 // NDB, e % NDB
     tile = TILE if e < 32 else 0
     return ["ds_read_b64_tr_b16 %s, %s offset:%d" % (vr(r + 2 * ld, 2), vr(KTR + db), tile + (4 * t + 2 * ld) * GROUP) for ld in range(2)]

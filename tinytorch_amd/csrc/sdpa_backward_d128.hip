@@ -18,7 +18,8 @@
 // and 44 KB of LDS operands, a SIMD's two wavefronts the LDS's whole 2050 cycles; here everything of a tile is one stream, a step, with its
 // operands requested into the register ring 6 ahead (the next tile's first before the step ends) and all that is not a matrix
 // instruction spread between those.  Same call: 620 -> 566 us in the first launches, the matrix pipe 55 % busy at 1.73 GHz
-// (45 % at 1.87 in the compiler's order), 545 -> 520 among others once the chip is warm: power again.
+// (45 % at 1.87 in the compiler's order), 545 -> 520 among others once the chip is warm.  V's row addresses in four registers of
+// their own instead of eight additions a step: forward and backward of this call 1160 -> 1152 us.
 
 #include "backward128_steps.inc"  // hand-ordered instruction streams (gen_backward128_steps.py)
 #include "sdpa_common.h"
@@ -640,14 +641,17 @@ __global__ __launch_bounds__(512, 2) void backward_dkv128_kernel(BwdArgs a) {
     f32x16 tmp[3];
 #pragma unroll
     for (int i = 0; i < 32; i++) ring[i] = 0u;
+    u32x4 v_addr;
+#pragma unroll
+    for (int i = 0; i < 4; i++) v_addr[i] = row_addr[i] + (v_from_ring - stage * KV_STAGE_BYTES);
     asm volatile(TT_B128_DKV_PREFETCH : "+{v[224:255]}"(ring) : "{v[140:143]}"(row_addr) : "memory");
 #define TT_DKV_RUN(TXT)                                                                                                        \
   asm volatile(TXT                                                                                                            \
-               : [o0] "+v"(dkacc[0]), [o1] "+v"(dkacc[1]), [o2] "+v"(dkacc[2]), [o3] "+v"(dkacc[3]), [o4] "+v"(dvacc[0]),       \
-                 [o5] "+v"(dvacc[1]), [o6] "+v"(dvacc[2]), [o7] "+v"(dvacc[3]), "+{v[224:255]}"(ring), "=&{v[144:159]}"(tmp[0]), \
+               : [o0] "+{v[0:15]}"(dkacc[0]), [o1] "+{v[16:31]}"(dkacc[1]), [o2] "+{v[32:47]}"(dkacc[2]), [o3] "+{v[48:63]}"(dkacc[3]), [o4] "+{v[64:79]}"(dvacc[0]),       \
+                 [o5] "+{v[80:95]}"(dvacc[1]), [o6] "+{v[96:111]}"(dvacc[2]), [o7] "+{v[112:127]}"(dvacc[3]), "+{v[224:255]}"(ring), "=&{v[144:159]}"(tmp[0]), \
                  "=&{v[160:175]}"(tmp[1]), "=&{v[176:191]}"(tmp[2]), "+{v[140:143]}"(row_addr), "+{v[136:139]}"(tr_addr)       \
-               : [c] "s"(c_s), [vb] "s"(v_from_ring - at_stage), [st] "s"(ring_addr + at_stage), [adv] "s"(advance),           \
-                 [more] "s"(more), "{v[192:223]}"(kv), "{v[132:133]}"(offs)                                                    \
+               : [c] "s"(c_s), [st] "s"(ring_addr + at_stage), [adv] "s"(advance),           \
+                 [more] "s"(more), "{v[192:223]}"(kv), "{v[128:131]}"(v_addr), "{v[132:133]}"(offs)                                                    \
                : "memory", "scc")
     do {
       row_now = row_next, row_next = next_row;
