@@ -19,7 +19,8 @@
 // operands requested into the register ring 6 ahead (the next tile's first before the step ends) and all that is not a matrix
 // instruction spread between those.  Same call: 620 -> 566 us in the first launches, the matrix pipe 55 % busy at 1.73 GHz
 // (45 % at 1.87 in the compiler's order), 545 -> 520 among others once the chip is warm.  V's row addresses in four registers of
-// their own instead of eight additions a step: forward and backward of this call 1160 -> 1152 us.
+// their own instead of eight additions a step: forward and backward of this call 1160 -> 1152 us.  Without the compiler's wait for K in the loop (below)
+// -> 1089 (1139 with both as before, on that box).
 
 #include "backward128_steps.inc"  // hand-ordered instruction streams (gen_backward128_steps.py)
 #include "sdpa_common.h"
@@ -190,7 +191,9 @@ __global__ __launch_bounds__(256, 2) void backward_dq128_kernel(BwdArgs a) {
   u32x4 row_addr, tr_addr;
   operand_offsets(lane, row_addr, tr_addr);
 
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // (with the operands named the compiler's own wait for their loads lies here and not in the loop, where it would be one for the tile
+  // just asked for)
+  asm volatile("s_waitcnt vmcnt(0)" : "+v"(qv), "+v"(gv) : : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
@@ -545,7 +548,7 @@ __global__ __launch_bounds__(512, 2) void backward_dkv128_kernel(BwdArgs a) {
   for (int i = 0; i < 4; i++) row_addr[i] += ring_addr, tr_addr[i] += ring_addr;
   const unsigned v_from_ring = (unsigned)__builtin_amdgcn_readfirstlane((int)(smem_addr + gw * TILE_BYTES - ring_addr));
 
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(0)" : "+v"(kv) : : "memory");  // (named for the reason given in the dq kernel)
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
