@@ -124,12 +124,28 @@ __global__ __launch_bounds__(256, 2) void backward_dq128_kernel(BwdArgs a) {
   };
   const T* kp = (const T*)f.k + b * f.ks[0] + hk * f.ks[1];
   const T* vp = (const T*)f.v + b * f.vs[0] + hk * f.vs[1];
+  // f16: the lanes' offsets are formed for each tile from the lane number anew (a dozen instructions).  Kept, they were spilled, and a
+  // reload's wait in front of each request was one for the tiles in flight.  Forward and backward, 2 x 32 heads (8) x 4096 causal 1165 ->
+  // 1151 us, 4 x 8 x 1545 144.0 -> 141.4, 1 x 32 (4) x 2111 229.6 -> 225.8; 2 x 32 (8) x 2000 without a mask 626 -> 619.  bf16 keeps them:
+  // formed anew, causal 2 x 16 (8) x 1023 94.4 -> 95.9; without a mask 1 x 32 (8) x 4096 1025 -> 1016, but 1 x 28 (4) x 1311 159.5 -> 160.3.
+  constexpr bool kLaneKept = kIsBf16;
+  auto lane_now = [&]() __attribute__((always_inline)) {
+    int ln = lane;
+    if constexpr (!kLaneKept) asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+    return ln;
+  };
   const unsigned chunk = (unsigned)((lane & 15) ^ (4 * (lane >> 4)));
-  const unsigned koff = ((unsigned)(lane >> 4) * (unsigned)f.ks[2] + 8u * chunk) * 2u, voff = ((unsigned)(lane >> 4) * (unsigned)f.vs[2] + 8u * chunk) * 2u;
+  const unsigned koff_kept = ((unsigned)(lane >> 4) * (unsigned)f.ks[2] + 8u * chunk) * 2u, voff_kept = ((unsigned)(lane >> 4) * (unsigned)f.vs[2] + 8u * chunk) * 2u;
   auto dma_tile = [&](int i) __attribute__((always_inline)) {
     const int kv0 = first_key(i);
     const unsigned at = smem_addr + (i & 3) * TILE_BYTES + 2 * wave * GROUP_BYTES;
     if (__builtin_expect(kv0 + BN <= S, 1)) {
+      unsigned koff = koff_kept, voff = voff_kept;
+      if constexpr (!kLaneKept) {
+        const int ln = lane_now();
+        const unsigned ch = (unsigned)((ln & 15) ^ (4 * (ln >> 4)));
+        koff = ((unsigned)(ln >> 4) * (unsigned)f.ks[2] + 8u * ch) * 2u, voff = ((unsigned)(ln >> 4) * (unsigned)f.vs[2] + 8u * ch) * 2u;
+      }
 #pragma unroll
       for (int g = 0; g < 2; g++) {
         const int row = kv0 + 8 * wave + 4 * g;
@@ -139,10 +155,11 @@ __global__ __launch_bounds__(256, 2) void backward_dq128_kernel(BwdArgs a) {
     } else {  // rows past the end re-read the last key (hidden below)
 #pragma unroll
       for (int g = 0; g < 2; g++) {
-        int row = 8 * wave + 4 * g + (lane >> 4);
+        const int ln = lane_now();
+        int row = 8 * wave + 4 * g + (ln >> 4);
         asm volatile("" : "+v"(row));  // keeps this rarely taken path's address arithmetic inside the branch
         const int rowc = kv0 + row < S ? row : S - 1 - kv0;
-        const unsigned ch = (unsigned)((lane & 15) ^ (4 * (lane >> 4)));
+        const unsigned ch = (unsigned)((ln & 15) ^ (4 * (ln >> 4)));
         dma16((const char*)(kp + (long long)kv0 * f.ks[2]), ((unsigned)rowc * (unsigned)f.ks[2] + 8u * ch) * 2u, at + g * GROUP_BYTES);
         dma16((const char*)(vp + (long long)kv0 * f.vs[2]), ((unsigned)rowc * (unsigned)f.vs[2] + 8u * ch) * 2u, at + STAGES * TILE_BYTES + g * GROUP_BYTES);
       }
@@ -248,7 +265,7 @@ __global__ __launch_bounds__(256, 2) void backward_dq128_kernel(BwdArgs a) {
   };
   auto hide = [&](f32x16& s, int kv0) __attribute__((always_inline)) {
     if ((CAUSAL && kv0 + BN - 1 > qw0 + coff) || kv0 + BN > S) {
-      const int qi = qw0 + lq + coff;
+      const int ln = lane_now(), lh = ln >> 5, qi = qw0 + (ln & 31) + coff;
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const int key = kv0 + 8 * (r >> 2) + 4 * lh + (r & 3);
