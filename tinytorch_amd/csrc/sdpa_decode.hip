@@ -72,36 +72,37 @@ __device__ __forceinline__ float row16_sum(float x) {
   return x;
 }
 
-// Sums of N values of a lane over the lanes of its chunk (lane % CH): a swap of two registers' halves (of their rows of 16 lanes) and one
-// addition fold two values into one register, so that four (CH = 32: two) values end in one, each in its own rows: value
-// phase_value + 4 i (2 i) in element i.  (As 2 shuffles through LDS for each value, 64 a wavefront, this took 0.7 us.)
-__device__ __forceinline__ float fold32(float a, float b) {
-  const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
-  const int lo = t[0], hi = t[1];
-  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
-}
+// Sums of N values of a lane over the lanes of its chunk (lane % CH), neighbouring phases first: a swap of two registers' rows of 16 lanes (of
+// their halves) and one addition fold two values into one register, so that four (CH = 32: two) values end in one, each in its own rows:
+// value phase_value + 4 i (2 i) in element i.  (As 2 shuffles through LDS for each value, 64 a wavefront, this took 0.7 us.  Folding the
+// halves first, which saves the narrow rows three additions in four, adds in another order: results of 16 bits then differ in their last place.)
 __device__ __forceinline__ float fold16(float a, float b) {
   const auto t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
   const int lo = t[0], hi = t[1];
   return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
 }
+__device__ __forceinline__ float fold32(float a, float b) {
+  const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+  const int lo = t[0], hi = t[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
 template <int CH>
 __device__ __forceinline__ int phase_value(int lane) {
-  return CH < 32 ? (lane >> 5) + 2 * ((lane >> 4) & 1) : lane >> 5;
+  return CH < 32 ? lane >> 4 : lane >> 5;
 }
 template <int CH, int N>
 __device__ __forceinline__ void add_phases(float* x) {
   static_assert(CH == 8 || CH == 16 || CH == 32, "");
+  if constexpr (CH == 8) {
+#pragma unroll
+    for (int i = 0; i < N; i++) x[i] += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x[i]), 0x128, 0xf, 0xf, true));  // row_ror:8
+  }
   if constexpr (CH == 32) {
 #pragma unroll
     for (int i = 0; i < N / 2; i++) x[i] = fold32(x[2 * i], x[2 * i + 1]);
   } else {
 #pragma unroll
-    for (int i = 0; i < N / 4; i++) {
-      float t = fold16(fold32(x[4 * i], x[4 * i + 1]), fold32(x[4 * i + 2], x[4 * i + 3]));
-      if constexpr (CH == 8) t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x128, 0xf, 0xf, false));  // row_ror:8
-      x[i] = t;
-    }
+    for (int i = 0; i < N / 4; i++) x[i] = fold32(fold16(x[4 * i], x[4 * i + 1]), fold16(x[4 * i + 2], x[4 * i + 3]));
   }
 }
 
