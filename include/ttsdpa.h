@@ -149,6 +149,10 @@ enum ttsdpa_kernel_kind {
 };
 int ttsdpa_kernel(const ttsdpa_params* p, int* kind);
 
+/* How *p is divided with the scratch it asks for (estimates decide, as above): the pieces of the keys (1: undivided) and the wavefronts of
+ * a workgroup of the decode kernel (0: another kernel); in the backward the pieces of a key block's query stream and of a row block's keys. */
+int ttsdpa_division(const ttsdpa_params* p, int* key_pieces, int* wavefronts);
+
 /* Bytes of device scratch ttsdpa_forward / ttsdpa_decode use for *p (0 for calls that need none): the split-KV
  * partials of the decode route, and of calls on the prefill route whose keys are divided among workgroups (few query
  * rows, or few 256-row tiles of head_dim 128 against many keys).
@@ -219,6 +223,7 @@ void ttsdpa_backward_params_init(ttsdpa_backward_params* p, int dtype, int B, in
  * matrix cores; TTSDPA_ROUTE_NONE = nothing to compute.  Needs no GPU. */
 int ttsdpa_backward_plan(const ttsdpa_backward_params* p, int* route);
 int ttsdpa_backward_kernel(const ttsdpa_backward_params* p, size_t workspace_bytes, int* kind);
+int ttsdpa_backward_division(const ttsdpa_backward_params* p, int* query_pieces, int* key_pieces);
 size_t ttsdpa_backward_workspace_bytes(const ttsdpa_backward_params* p);
 int ttsdpa_backward(const ttsdpa_backward_params* p, void* workspace, size_t workspace_bytes, void* stream);
 

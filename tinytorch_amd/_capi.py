@@ -20,7 +20,7 @@ STATIC_SCRATCH_BYTES = 2 << 20
 
 EXPORTS = [
     "ttsdpa_abi_version", "ttsdpa_status_string", "ttsdpa_params_init", "ttsdpa_plan", "ttsdpa_workspace_bytes",
-    "ttsdpa_kernel", "ttsdpa_backward_kernel", "ttsdpa_forward", "ttsdpa_prefill", "ttsdpa_decode", "ttsdpa_decode_static", "ttsdpa_general",
+    "ttsdpa_kernel", "ttsdpa_backward_kernel", "ttsdpa_division", "ttsdpa_backward_division", "ttsdpa_forward", "ttsdpa_prefill", "ttsdpa_decode", "ttsdpa_decode_static", "ttsdpa_general",
     "ttsdpa_kv_append_params_init", "ttsdpa_kv_append",
     "ttsdpa_backward_params_init", "ttsdpa_backward_plan", "ttsdpa_backward_workspace_bytes", "ttsdpa_backward",
     # include/ttfused.h
@@ -160,6 +160,9 @@ def lib():
         L.ttsdpa_backward_workspace_bytes.restype = ctypes.c_size_t
         L.ttsdpa_backward.argtypes = [BP, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
         L.ttsdpa_backward.restype = ctypes.c_int
+        two = [ctypes.POINTER(ctypes.c_int)] * 2
+        L.ttsdpa_division.argtypes, L.ttsdpa_division.restype = [P] + two, ctypes.c_int
+        L.ttsdpa_backward_division.argtypes, L.ttsdpa_backward_division.restype = [BP] + two, ctypes.c_int
         vp, i64 = ctypes.c_void_p, ctypes.c_int64
         L.ttfused_rms_norm.argtypes = [ctypes.c_int, vp, vp, vp, i64, i64, ctypes.c_float, vp]
         L.ttfused_rms_norm.restype = ctypes.c_int
@@ -251,3 +254,17 @@ def backward_kernel(p, workspace_bytes=None):
     n = lib().ttsdpa_backward_workspace_bytes(ctypes.byref(p)) if workspace_bytes is None else workspace_bytes
     assert lib().ttsdpa_backward_kernel(ctypes.byref(p), n, ctypes.byref(k)) == OK
     return KERNEL_NAMES[k.value]
+
+
+def division(p):
+    """(pieces of the keys, wavefronts of a decode workgroup or 0) of a ttsdpa_forward call with the scratch it asks for."""
+    n, w = ctypes.c_int(-1), ctypes.c_int(-1)
+    assert lib().ttsdpa_division(ctypes.byref(p), ctypes.byref(n), ctypes.byref(w)) == OK
+    return n.value, w.value
+
+
+def backward_division(p):
+    """(pieces of a key block's query stream, pieces of a row block's keys) of a ttsdpa_backward call with the scratch it asks for."""
+    n, m = ctypes.c_int(-1), ctypes.c_int(-1)
+    assert lib().ttsdpa_backward_division(ctypes.byref(p), ctypes.byref(n), ctypes.byref(m)) == OK
+    return n.value, m.value

@@ -933,6 +933,30 @@ int ttsdpa_kernel(const ttsdpa_params* p, int* kind) {
   return TTSDPA_OK;
 }
 
+int ttsdpa_division(const ttsdpa_params* p, int* key_pieces, int* wavefronts) {
+  KArgs a;
+  const int rc = validate(p, &a);
+  if (rc != TTSDPA_OK) return rc;
+  int n = 1, w = 0;
+  const int route = pick_route(p);
+  a.full_p = full_probabilities(p);
+  const bool prefill = route == TTSDPA_ROUTE_PREFILL || (route == TTSDPA_ROUTE_GENERAL && p->mask_kind != TTSDPA_MASK_NONE && prefill_ok(p, true));
+  if (route == TTSDPA_ROUTE_DECODE || (prefill && f32_decode_ok(p))) {
+    const DecodePlan pl = plan_decode(a, p->dtype == TTSDPA_F32);
+    n = pl.splits, w = pl.waves;
+  } else if (prefill && short_kernel_of(p, a) == TTSDPA_KERNEL_OTHER) {
+    if (p->dtype != TTSDPA_F32 && (pipelined_ok(p) || pipelined64_ok(p))) {
+      n = plan_pipelined(p).split.splits;
+    } else {
+      if (pack_heads_ok(p)) pack_heads(&a);
+      n = plan_prefill_splits(p, a).splits;
+    }
+  }
+  if (key_pieces) *key_pieces = n;
+  if (wavefronts) *wavefronts = w;
+  return TTSDPA_OK;
+}
+
 void ttsdpa_backward_params_init(ttsdpa_backward_params* p, int dtype, int B, int Hq, int Hkv, int L, int S, int D) {
   memset(p, 0, sizeof(*p));
   p->struct_size = sizeof(*p);
@@ -958,6 +982,21 @@ int ttsdpa_backward_kernel(const ttsdpa_backward_params* p, size_t workspace_byt
   bool joint = false;
   const int n = pick_backward_route(p) == TTSDPA_ROUTE_NONE ? 0 : short_backward_taken(p, PairSplits(p), workspace_bytes, &joint);
   if (kind) *kind = n == 0 ? TTSDPA_KERNEL_OTHER : joint ? TTSDPA_KERNEL_SHORT_JOINT : TTSDPA_KERNEL_SHORT;
+  return TTSDPA_OK;
+}
+
+int ttsdpa_backward_division(const ttsdpa_backward_params* p, int* query_pieces, int* key_pieces) {
+  BwdArgs a;
+  const int rc = validate_backward(p, &a);
+  if (rc != TTSDPA_OK) return rc;
+  int n = 1, m = 1;
+  if (pick_backward_route(p) != TTSDPA_ROUTE_NONE) {
+    const PairSplits pair(p);
+    const int own = short_backward_splits(p, pair);
+    n = own > 0 ? own : pair.dkv, m = own > 0 ? 1 : pair.dq;
+  }
+  if (query_pieces) *query_pieces = n;
+  if (key_pieces) *key_pieces = m;
   return TTSDPA_OK;
 }
 
