@@ -47,3 +47,25 @@ def test_records_go_with_pieces(dtype, B, Hq, Hkv, L, S, D):
         assert (_capi.division(p)[0] > 1) == (scratch(p) > 0)
     bp = call(dtype, B, Hq, Hkv, L, S, D, back=True)
     assert (max(_capi.backward_division(bp)) > 1) == (scratch(bp) > 16 * B * Hq * L)
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,S,D,lens,one,waves", [
+    # us divided (or with four wavefronts) / in one launch (with eight), keys full, spread evenly and one long sequence among short ones
+    (BF16, 32, 32, 8, 4096, 128, True, False, 4),    # 92.6 / 89.9, 64.2 / 70.7, 46.1 / 62.3
+    (BF16, 32, 32, 8, 2048, 128, True, False, 4),    # 51.0 / 47.0, 35.7 / 37.2, 27.1 / 32.7
+    (F32, 32, 32, 8, 1024, 128, True, False, 4),     # 47.9 / 44.5, 34.7 / 36.5, 26.1 / 31.5
+    (BF16, 32, 32, 8, 1024, 128, True, True, 8),     # 29.4 / 24.8, 21.8 / 20.9, 17.1 / 17.6
+    (F16, 24, 32, 8, 1024, 64, True, True, 8),       # 16.2 / 13.1, 13.9 / 11.6, 11.4 / 9.9
+    (BF16, 32, 32, 8, 2048, 128, False, True, 8),    # 51.0 / 47.0
+    (BF16, 64, 64, 8, 1024, 128, False, True, 4),    # 51.0 / 54.5
+    (F16, 64, 64, 8, 4096, 64, False, True, 4),      # 93.2 / 94.3
+    (F32, 69, 4, 4, 434, 128, True, None, 4),        # 32.9 / 35.4
+    (BF16, 70, 16, 4, 1206, 80, True, False, 4),     # 35.8 / 41.7, 28.3 / 30.1, 16.5 / 19.3
+    (F32, 21, 8, 2, 284, 80, True, False, 4),        # 13.7 / 16.3, 11.6 / 12.1, 10.5 / 13.3
+])
+def test_decode_in_one_launch(dtype, B, Hq, Hkv, S, D, lens, one, waves):
+    """Where all keys of a sequence are one workgroup's, and of how many wavefronts: not where lengths may differ and the longest takes
+    longer than its pieces and their merge."""
+    pieces, w = _capi.division(call(dtype, B, Hq, Hkv, 1, S, D, lens=lens))
+    assert w == waves
+    assert one is None or (pieces == 1) == one

@@ -455,19 +455,27 @@ DecodePlan plan_decode(const KArgs& a, bool f32) {
   // merge: us for a turn of the wavefronts (32 keys each), the merge's launch, a CU's further workgroups (four wavefronts of them: each, and
   // for a turn), and twice the wavefronts, by head_dim, element type and rows; fitted to 400 calls of 1 to 1500 (sequence, KV head)
   // pairs on 128 to 4096 keys (9 to 15 % off; a turn is the vector ALUs' P.V for the most part: requesting the next turn's keys ahead gave
-  // nothing).  A cache is taken to be filled to nine tenths.  24 x 8 pairs on up to 1024 keys 13.3 -> 9.5 us, 12 x 8 on 178 of 1024 9.6 -> 6.4;
-  // 12 x 1 on 1024 stay split, 8.2 and 14.2.  Not beyond the keys it was fitted on, where memory's rate is all that counts: 64 x 8 on 8192 316
-  // us with four wavefronts and 323 with eight.
+  // nothing).  24 x 8 pairs on up to 1024 keys 13.3 -> 9.5 us, 12 x 8 on 178 of 1024 9.6 -> 6.4; 12 x 1 on 1024 stay split, 8.2 and 14.2.  Not
+  // beyond the keys it was fitted on, where memory's rate is all that counts: 64 x 8 on 8192 316 us with four wavefronts and 323 with eight.
+  // A cache is taken to be full: by nine tenths of its keys, a last turn was missed (fp32, 21 x 2 on 284, head_dim 80, 13.7 us divided, 16.3).
   static constexpr double fit[2][2][2][5] = {{{{1.2, 3.6, 0.40, 0, 0.8}, {1.25, 3.0, 1.5, 0, 0.4}}, {{1.95, 3.6, 0, 0.80, 1.35}, {2.5, 4.8, 2.2, 0, 1.8}}},
                                              {{{2.0, 3.7, 0, 0.68, 1.15}, {2.15, 3.5, 1.5, 0.62, 1.2}}, {{3.8, 4.3, 1.3, 0.86, 2.6}, {4.7, 4.5, 0.93, 1.55, 2.6}}}};
-  if (p.rows <= 8 && a.S <= 4096) {
+  // Sequences of unlike lengths: the longest one's chain lasts while the others' workgroups have ended, and a wavefront more does not shorten
+  // it (a CU takes in 35 KB of K and V a us).  Up to 256 KB of K the merge makes up for it in most batches (780 drawn ones of a third to all keys 0.99 to
+  // 2.2x, with a single long sequence among short ones of 60 keys 0.79 to 2.2x); beyond that their keys stay divided.
+  // bf16, head_dim 128, us divided and in one launch, lengths spread evenly / one long among short ones: 32 x 8 on 1024 21.8 and 20.9 / 17.1
+  // and 17.6, on 2048 35.7 and 37.2 / 27.1 and 32.7, on 4096 64.2 and 70.7 / 46.1 and 62.3; fp32 on 1024 34.7 and 36.5 / 26.1 and 31.5.
+  // Eight wavefronts only while a CU has one workgroup (up to head_dim 64: less than two): 64 x 8 on 1024 51.0 us with four, 54.5 with eight, a
+  // tenth full 12.2 and 13.0; 70 x 4 on 1206, head_dim 80, 35.8 divided and 41.7; 79 x 8, head_dim 64, on 1097 40.1 and 42.2.
+  const bool unlike = a.kv_len && a.B > 1;
+  if (p.rows <= 8 && a.S <= 4096 && (!unlike || (long long)a.S * a.D * (f32 ? 4 : 2) <= 256 << 10)) {
     const double* f = fit[a.D > 64][f32][p.rows > 4];
-    const double keys = a.kv_len ? 0.9 * a.S : a.S, fixed = 2.5 + 1e-7 * pairs * keys * a.D * (f32 ? 8 : 4);  // (0.1 us for a MB)
+    const double keys = a.S, fixed = 2.5 + 1e-7 * pairs * keys * a.D * (f32 ? 8 : 4);  // (0.1 us for a MB)
     auto us = [&](int waves, int n) {
       const double further = (double)((pairs * n + 255) / 256 - 1) * waves / 4, turns = ceil(ceil(keys / n) / (KB * waves));
       return fixed + f[0] * turns + (n > 1 ? f[1] : 0) + (f[2] + f[3] * turns) * further + (waves > 4 ? f[4] : 0);
     };
-    const double split = us(4, splits), four = us(4, 1), eight = us(8, 1);
+    const double split = us(4, splits), four = us(4, 1), eight = pairs <= (a.D > 64 ? 256 : 511) ? us(8, 1) : four;
     if ((four < eight ? four : eight) < 0.95 * split) splits = 1, chunk = (a.S + round - 1) / round * round, p.waves = eight < four ? 8 : 4;
   }
   p.splits = splits;
