@@ -1,5 +1,6 @@
 """How attention calls are divided, as the host's queries answer without a GPU."""
 import ctypes
+import time
 
 import pytest
 
@@ -69,3 +70,52 @@ def test_decode_in_one_launch(dtype, B, Hq, Hkv, S, D, lens, one, waves):
     pieces, w = _capi.division(call(dtype, B, Hq, Hkv, 1, S, D, lens=lens))
     assert w == waves
     assert one is None or (pieces == 1) == one
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,D,causal,kernel,pieces", [
+    # as summed up row tile by row tile
+    (2, 2, 2, 2489, 2489, 64, NONE, "other", 5),
+    (2, 2, 1, 6509, 6509, 128, NONE, "other", 2),
+    (5, 2, 2, 357, 2647, 64, NONE, "dealt", 6),
+    (1, 1, 1, 7821, 1760, 128, BR, "dealt", 4),
+    (3, 6, 6, 871, 5902, 64, BR, "dealt", 2),
+    (1, 10, 5, 7210, 7054, 128, TL, "dealt", 1),
+    (1, 3, 3, 1569, 1300, 128, TL, "dealt", 6),
+    (7, 1, 1, 3440, 3440, 64, BR, "other", 4),
+    (3, 3, 3, 4128, 4128, 64, BR, "dealt", 1),
+    (1, 9, 9, 231, 868, 64, BR, "other", 5),
+    (2, 4, 1, 8721, 8721, 64, BR, "dealt", 1),
+    (6, 2, 2, 2418, 2418, 128, TL, "dealt", 1),
+    (1, 22, 11, 806, 2578, 64, BR, "dealt", 1),
+    (4, 2, 2, 1231, 6702, 64, BR, "other", 6),
+    (1, 16, 16, 1112, 1112, 64, TL, "dealt", 1),
+    (7, 2, 1, 2722, 2722, 64, TL, "dealt", 1),
+    (1, 16, 4, 383, 866, 64, BR, "other", 3),
+    (2, 4, 1, 8980, 8980, 128, TL, "dealt", 1),
+    (1, 6, 3, 2290, 2290, 128, BR, "dealt", 3),
+    (1, 1, 1, 785, 2221, 128, BR, "dealt", 9),
+    (3, 2, 1, 1553, 1553, 128, BR, "dealt", 4),
+    (4, 1, 1, 1439, 1439, 64, NONE, "dealt", 3),
+    (2, 24, 6, 1341, 6526, 64, NONE, "dealt", 1),
+    (1, 1, 1, 1182, 1182, 128, TL, "dealt", 5),
+])
+def test_pieces_of_a_prompt(B, Hq, Hkv, L, S, D, causal, kernel, pieces):
+    """The row tiles' lengths in closed form: rows and keys that end anywhere, both alignments, more rows than keys."""
+    p = call(BF16, B, Hq, Hkv, L, S, D, causal)
+    assert (_capi.kernel(p), _capi.division(p)[0]) == (kernel, pieces)
+
+
+def test_planning_does_not_grow_with_the_rows():
+    """Host time of a scratch query for 16 to 64 times the rows (row tile by row tile 9 and 2 times as long)."""
+    def least(f, p):
+        ref, times = ctypes.byref(p), []
+        for _ in range(60):
+            t = time.perf_counter()
+            for _ in range(100):
+                f(ref)
+            times.append(time.perf_counter() - t)
+        return min(times)
+    L = _capi.lib()
+    f, g = L.ttsdpa_workspace_bytes, L.ttsdpa_backward_workspace_bytes
+    assert least(f, call(BF16, 1, 1, 1, 16384, 16384, 128, TL)) < 3 * least(f, call(BF16, 1, 1, 1, 1100, 1100, 128, TL))
+    assert least(g, call(BF16, 1, 1, 1, 65536, 65536, 128, TL, back=True)) < 1.5 * least(g, call(BF16, 1, 1, 1, 1100, 1100, 128, TL, back=True))

@@ -277,6 +277,21 @@ struct SplitCost {
     if (last > longest_rest) longest_rest = last;
     if (tiles > chunk) records += count * (pieces + (last > 0));
   }
+  // add(count, first + step * i), i = 0 .. n-1, of a step that divides the chunk: in pieces of p = chunk / step places, place i + first / step
+  // (first % step key tiles further: a rest, if not zero, even where a place is the first of its piece)
+  void add_series(double count, unsigned first, unsigned step, unsigned n) {
+    if (n < 1) return;
+    const unsigned c = (unsigned)chunk, p = c / step, lo = first / step, hi = lo + n, over = first % step;  // places lo .. hi-1
+    const unsigned q0 = lo / p, r0 = lo % p, q1 = hi / p, r1 = hi % p;
+    auto below = [&](double q, double r) { return p * (0.5 * q * (q - 1)) + q * r; };  // pieces before the places up to p q + r, added up
+    const double pieces = below(q1, r1) - below(q0, r0), sum = (double)n * first + step * (0.5 * n * (n - 1.0));
+    const double even = over ? 0 : (q1 + (r1 > 0)) - (q0 + (r0 > 0));  // places that end with a piece
+    const double longest = step * (double)(q1 > q0 ? p - 1 : r1 - 1) + over;
+    const unsigned undivided = first > c ? 0 : (c - first) / step + 1;
+    whole += count * pieces, rest += count * (sum - chunk * pieces), rests += count * (n - even);
+    if (longest > longest_rest) longest_rest = longest;
+    records += count * (pieces + (n - even) - (undivided < n ? undivided : n));
+  }
   double longest() const {  // a CU's tiles
     const double rounds = ceil(whole / 256), room = 256 * rounds - whole, left = rest - room * chunk;
     double tiles = rounds * chunk;
@@ -308,16 +323,15 @@ SplitPlan plan_pipelined_splits(const ttsdpa_params* p) {
   const int ntile = (p->L + 255) / 256, causal = effective_causal(p);
   const int offset = causal == TTSDPA_CAUSAL_BOTTOM_RIGHT && p->S > p->L ? p->S - p->L : 0;
   const int longest = (int)((keys + 63) / 64);
+  // row tiles that end before the keys do, each 256 keys behind the one above; the others see all keys
+  const long long ends = causal == TTSDPA_CAUSAL_NONE || p->S <= offset ? 0 : ((long long)p->S - offset - 1) / 256, rising = ends < ntile ? ends : ntile;
   double least = 0;
   for (int n = 1; n <= 64 && (n == 1 || units * n <= 1024); n++) {
     const int chunk = ((longest + n - 1) / n + 3) & ~3;
     if ((longest + chunk - 1) / chunk < n) continue;  // the same as fewer
     SplitCost cost{(double)chunk};
-    for (int t = 0; t < ntile; t++) {
-      long long last = p->S;
-      if (causal != TTSDPA_CAUSAL_NONE && 256ll * (t + 1) + offset < last) last = 256ll * (t + 1) + offset;
-      cost.add((double)heads, (int)((last + 63) / 64));
-    }
+    if (rising > 0) cost.add_series((double)heads, 4 + (unsigned)(offset + 63ll) / 64, 4, (unsigned)rising);
+    if (rising < ntile) cost.add((double)(heads * (ntile - rising)), (int)(((long long)p->S + 63) / 64));
     const double us = cost.us();
     if (n == 1 || us < 0.95 * least) least = us, s.splits = n, s.chunk = 64 * chunk;
   }
@@ -338,17 +352,25 @@ struct PipelinedCost {
 constexpr PipelinedCost kRows256[2] = {{7.2, 0.74, 0.30, 6, 11.2, 0.63, 0.33, 0.0, 0.027}, {8.9, 1.02, 0.58, 7, 14.9, 0.60, 0.83, 8.2, 0.039}};
 constexpr PipelinedCost kRows128[2] = {{6.6, 0.47, 0.09, 10, 8.2, 0.53, 0.0, 1.9, 0.027}, {7.6, 0.68, 0.20, 9, 11.8, 0.69, 0.17, 4.0, 0.026}};
 
-// Row tiles of `rows` rows, longest first: length of the t-th, and of all.
+// Row tiles of `rows` rows (256, 128), longest first: length of the t-th, and of all.  Under a causal mask their lengths rise from the last one by rows /
+// 64 up to that of all keys; the first one may have fewer rows.  Sums over them are closed forms: tile by tile, a plan of one head on
+// 16384 rows took 9.6 us of the host's time.
+template <int rows>
 struct RowTiles {
-  int rows, ntile, S, offset, L;
+  int ntile, S, offset, L;
   bool causal;
-  long long heads, sum = 0;
-  RowTiles(const ttsdpa_params* p, int rows_) : rows(rows_), ntile((p->L + rows_ - 1) / rows_), S(p->S), L(p->L), heads((long long)p->B * p->Hq) {
+  long long heads, rising = 0, first = 0, sum = 0;  // rising: whole tiles that end before the keys do, the shortest `first` long
+  explicit RowTiles(const ttsdpa_params* p) : ntile((p->L + rows - 1) / rows), S(p->S), L(p->L), heads((long long)p->B * p->Hq) {
     const int c = effective_causal(p);
     causal = c != TTSDPA_CAUSAL_NONE, offset = c == TTSDPA_CAUSAL_BOTTOM_RIGHT && S > L ? S - L : 0;
-    if (!causal) sum = heads * ntile * length(0);
-    else
-      for (int t = 0; t < ntile; t++) sum += heads * length(t);
+    const long long all = ((long long)S + 63) / 64;
+    if (!causal) {
+      sum = heads * ntile * all;
+      return;
+    }
+    const long long ends = S > offset ? ((long long)S - offset - 1) / rows : 0;
+    rising = ends < ntile - 1 ? ends : ntile - 1, first = rows / 64 + ((long long)offset + 63) / 64;
+    sum = heads * (rising * first + rows / 64 * (rising * (rising - 1) / 2) + (ntile - 1 - rising) * all + length(0));
   }
   int length(int t) const {
     long long last = S;
@@ -368,7 +390,7 @@ struct RowTiles {
                                  : sum / 256.0 + c.start * (pairs / 256.0 - 1) + 0.25 * longest;  // (the middle ones are single)
       else {
         // the CU with the shortest of the first 256 takes the next one
-        const double next = n <= 512 ? length((int)(255 / heads)) + length((int)(256 / heads)) + c.start
+        const double next = n <= 512 ? length(255 / (int)heads) + length(256 / (int)heads) + c.start
                                      : sum / 256.0 + 0.5 * length(ntile - 1) + c.start * (n / 256.0 - 1);
         longest = next > longest ? next : longest;
       }
@@ -378,7 +400,13 @@ struct RowTiles {
   // with pieces of `chunk` (64 keys); 0: none that is shorter than the longest row tile
   double split_us(const PipelinedCost& c, int chunk) const {
     SplitCost s{(double)chunk};
-    for (int t = ntile - 1; t >= 0; t--) s.add((double)heads, length(t));
+    if (!causal) {
+      s.add((double)(heads * ntile), length(0));
+    } else {
+      s.add_series((double)heads, (unsigned)first, rows / 64, (unsigned)rising);
+      if (rising < ntile - 1) s.add((double)(heads * (ntile - 1 - rising)), (int)(((long long)S + 63) / 64));
+      s.add((double)heads, length(0));
+    }
     const double pieces = (s.whole + s.rests) / 256 - 1;
     return c.split_base + c.split_each * s.longest() + c.split_busy * (s.whole * chunk + s.rest) / 256 + (pieces > 0 ? c.split_more * pieces : 0) + c.record * s.records;
   }
@@ -395,18 +423,24 @@ struct PipelinedPlan {
 PipelinedPlan plan_pipelined(const ttsdpa_params* p, bool divided = true, double* us = nullptr) {
   PipelinedPlan plan{false, divided ? plan_pipelined_splits(p) : SplitPlan{1, 0, 0}};
   if (p->dtype == TTSDPA_F32 || p->mask_kind != TTSDPA_MASK_NONE || !(pipelined_ok(p) || pipelined64_ok(p)) || p->S < 1) return plan;
-  const RowTiles wide(p, 256), narrow(p, 128);
+  const RowTiles<256> wide(p);
+  const RowTiles<128> narrow(p);
   const PipelinedCost &c256 = kRows256[p->D == 128], &c128 = kRows128[p->D == 128];
   double least = plan.split.splits > 1 ? wide.split_us(c256, plan.split.chunk / 64) : wide.whole_us(c256);
   const double whole = narrow.whole_us(c128);
   // (sequences of unlike lengths: the estimates take them all for the longest, which is too much for a divided launch)
   if (whole < (p->kv_len && p->B > 1 ? 0.9 : 0.95) * least) least = whole, plan.dealt = true, plan.split = SplitPlan{1, 0, 0};
   const int longest = narrow.length(0);
+  // least of any division: a CU has its share of all lengths, and a whole piece; a row tile is a piece or more
+  const double even = narrow.sum / 256.0, rounds = narrow.heads * narrow.ntile / 256.0 - 1;
+  const double further = c128.split_busy * even + (rounds > 0 ? c128.split_more * rounds : 0);
   for (int n = 2; divided && n <= 16 && narrow.heads * narrow.ntile * n <= 1024; n++) {
     const int chunk = ((longest + n - 1) / n + 3) & ~3;
     if ((longest + chunk - 1) / chunk < n) continue;  // the same as fewer
+    const double most = (plan.dealt ? 1.0 : 0.95) * least;
+    if (c128.split_base + c128.split_each * (even > chunk ? even : chunk) + further > 1.001 * most) continue;
     const double t = narrow.split_us(c128, chunk);
-    if (t < (plan.dealt ? 1.0 : 0.95) * least)
+    if (t < most)
       least = t, plan.dealt = true, plan.split = SplitPlan{n, 64 * chunk, split_record_bytes(narrow.heads, p->L, n, p->D)};
   }
   if (us) *us = least;
@@ -630,13 +664,16 @@ int short_backward_splits(const ttsdpa_backward_params* p, const PairSplits& n, 
 struct PairSplits {
   int dkv = 1, dq = 1;
   bool dkv_dealt = false, dq_dealt = false;
+  int own = -1;  // 16-bit calls: the answer of short_backward_splits, found on the way
+  bool own_joint = false;
   PairSplits(const ttsdpa_backward_params* p) {
     const ttsdpa_params* f = &p->fwd;
     if (!backward_on_mfma(p)) return;
     const bool f32 = backward_on_f32_pair(p), causal = effective_causal(f) != TTSDPA_CAUSAL_NONE;
     if (f->dtype != TTSDPA_F32 && f->mask_kind == TTSDPA_MASK_NONE && (f->D == 64 || f->D == 128)) {
       static constexpr BackwardCost kDq[2] = {{0, 0.59, 3.6, 0.47}, {4.5, 0.53, 2.9, 0.37}}, kDkv[2] = {{0, 0.95, 2.5, 0.40}, {0, 1.75, 1.8, 0.41}};
-      if (short_backward_splits(p, *this) > 0) return;  // (whole: with less scratch than those kernels ask for)
+      own = short_backward_splits(p, *this, &own_joint);
+      if (own > 0) return;  // (whole: with less scratch than those kernels ask for)
       const int more = f->S > f->L ? f->S - f->L : 0, offset = effective_causal(f) == TTSDPA_CAUSAL_BOTTOM_RIGHT ? more : 0;
       dq = backward_splits_16bit(kDq[f->D == 128], false, f->B, f->Hq, f->Hkv, f->L, f->S, f->D, causal, more);
       dkv = backward_splits_16bit(kDkv[f->D == 128], true, f->B, f->Hq, f->Hkv, f->L, f->S, f->D, causal, offset);
@@ -676,6 +713,10 @@ double pair_backward_us(const ttsdpa_params* f, const ShortShape& s, const PairS
 
 // The short sequences' backward: splits of its dk / dv workgroups, 0 where the pairs are the shorter way.
 int short_backward_splits(const ttsdpa_backward_params* p, const PairSplits& n, bool* joint) {
+  if (n.own >= 0) {
+    if (joint) *joint = n.own_joint;
+    return n.own;
+  }
   const ttsdpa_params* f = &p->fwd;
   if (!short_ok(f) || !(backward_mfma_ok(p) || backward_f32_ok(p))) return 0;
   const ShortShape s(f);
