@@ -119,3 +119,17 @@ def test_planning_does_not_grow_with_the_rows():
     f, g = L.ttsdpa_workspace_bytes, L.ttsdpa_backward_workspace_bytes
     assert least(f, call(BF16, 1, 1, 1, 16384, 16384, 128, TL)) < 3 * least(f, call(BF16, 1, 1, 1, 1100, 1100, 128, TL))
     assert least(g, call(BF16, 1, 1, 1, 65536, 65536, 128, TL, back=True)) < 1.5 * least(g, call(BF16, 1, 1, 1, 1100, 1100, 128, TL, back=True))
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,D", [
+    # us with the row blocks' keys counted as if all were seen / counted as they are
+    (1, 4, 4, 130, 817, 64),       # 26.3 / 18.5
+    (2, 4, 2, 187, 1230, 64),      # 33.0 / 24.5
+    (1, 8, 4, 1776, 6154, 64),     # 78.2 / 78.2
+    (2, 8, 4, 174, 1758, 128),     # 38.3 / 29.7
+    (1, 32, 8, 300, 4000, 128),    # 73 / 62
+    (4, 1, 1, 1401, 17781, 128),   # 75.1 / 68.5
+])
+def test_row_blocks_of_a_top_left_mask_see_as_many_keys_as_rows(dtype, B, Hq, Hkv, L, S, D):
+    assert _capi.backward_division(call(dtype, B, Hq, Hkv, L, S, D, TL, back=True))[1] == _capi.backward_division(call(dtype, B, Hq, Hkv, L, L, D, TL, back=True))[1]

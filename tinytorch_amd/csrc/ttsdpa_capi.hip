@@ -674,8 +674,8 @@ struct PairSplits {
       static constexpr BackwardCost kDq[2] = {{0, 0.59, 3.6, 0.47}, {4.5, 0.53, 2.9, 0.37}}, kDkv[2] = {{0, 0.95, 2.5, 0.40}, {0, 1.75, 1.8, 0.41}};
       own = short_backward_splits(p, *this, &own_joint);
       if (own > 0) return;  // (whole: with less scratch than those kernels ask for)
-      const int more = f->S > f->L ? f->S - f->L : 0, offset = effective_causal(f) == TTSDPA_CAUSAL_BOTTOM_RIGHT ? more : 0;
-      dq = backward_splits_16bit(kDq[f->D == 128], false, f->B, f->Hq, f->Hkv, f->L, f->S, f->D, causal, more);
+      const int offset = effective_causal(f) == TTSDPA_CAUSAL_BOTTOM_RIGHT && f->S > f->L ? f->S - f->L : 0;
+      dq = backward_splits_16bit(kDq[f->D == 128], false, f->B, f->Hq, f->Hkv, f->L, f->S, f->D, causal, offset);
       dkv = backward_splits_16bit(kDkv[f->D == 128], true, f->B, f->Hq, f->Hkv, f->L, f->S, f->D, causal, offset);
       return;
     }
