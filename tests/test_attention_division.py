@@ -133,3 +133,17 @@ def test_planning_does_not_grow_with_the_rows():
 ])
 def test_row_blocks_of_a_top_left_mask_see_as_many_keys_as_rows(dtype, B, Hq, Hkv, L, S, D):
     assert _capi.backward_division(call(dtype, B, Hq, Hkv, L, S, D, TL, back=True))[1] == _capi.backward_division(call(dtype, B, Hq, Hkv, L, L, D, TL, back=True))[1]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,D,causal,pieces", [
+    (1, 16, 2, 1031, 1031, 64, BR, (14, 3)),       # us with dk / dv in 8 pieces 71.3, in 14 58.5
+    (1, 32, 8, 4528, 111, 128, BR, (15, 1)),       # 128.9, 105.4
+    (2, 2, 1, 421, 6630, 128, NONE, (1, 14)),      # dq in 8 75.3, in 14 71.1
+    (1, 8, 8, 263, 4859, 64, BR, (1, 8)),          # in 14 52.4, in 8 49.4
+    (4, 2, 1, 424, 3598, 64, BR, (2, 8)),          # in 10 57.5, in 8 54.4
+    (4, 64, 8, 211, 1711, 64, TL, (3, 1)),         # dk / dv whole 85, in three pieces, of whose records most are zeros, 67
+    (2, 64, 8, 841, 7870, 128, TL, (1, 1)),        # 217, in two pieces 248: more than the caches hold
+])
+def test_pieces_of_long_streams(B, Hq, Hkv, L, S, D, causal, pieces):
+    for dtype in (F16, BF16):
+        assert _capi.backward_division(call(dtype, B, Hq, Hkv, L, S, D, causal, back=True)) == pieces

@@ -392,8 +392,15 @@ inline int backward_dq_splits(int B, int Hq, int L, int S, int D, bool causal, i
 // Fitted to 480 calls of 1 to 8 sequences, 1 to 64 heads, 100 to 4096 rows with the number of either kernel forced to 1 .. 8
 // (the estimates' differences miss by 4 to 8 % of the call's time; the numbers they choose give 1 % less than the best ones).
 // Records cost more than an uneven end: 4 x 8 heads x 1545 rows, head_dim 128, causal, dq in 4 splits 192 us, whole 143 (whole backward).
+// Up to 16 pieces, where few blocks have long streams: 70 drawn calls of 9 to 16 pieces take 2 % more than with their best number, with
+// 8 instead 6 % more (1 x 16 heads (2) x 1031, head_dim 64, dk/dv in 8 71 us, in 14 59); but dq at head_dim 64, in up to 16 instead of 8, lost 5 %
+// (1 x 8 x 263 rows on 4859 keys in 14 52.4 us, in 8 49.4; 4 x 2 (1) x 424 on 3598 in 10 57.5, in 8 54.4).
+// Records of keys that no row sees are zeros and cost half, while all records are `cached` MB or less (80 top-left causal calls on 2 to 12 times
+// as many keys as rows: 4 % from their best, 1.5 % so; 4 x 64 heads (8) x 211 rows on 1711 keys, head_dim 64, dk/dv whole 85 us, in 3 pieces 67;
+// beyond that not: 2 x 64 (8) x 841 on 7870, head_dim 128, whole 217, in two pieces, 259 MB, 248).
 struct BackwardCost {
   double start, tile_us, launch, per_mb;  // start: what a workgroup costs beside its tiles, in tiles, where another one has its place before
+  double cached = 0;
 };
 inline int backward_splits_16bit(const BackwardCost& c, bool of_keys, int B, int Hq, int Hkv, int L, int S, int D, bool causal, int offset) {
   const int slots = of_keys && D == 128 ? 256 : 512;  // workgroups side by side
@@ -428,8 +435,13 @@ inline int backward_splits_16bit(const BackwardCost& c, bool of_keys, int B, int
   const int longest = tiles(0);
   const long long blocks = heads * nblk;
   const double mb_each = of_keys ? 8e-6 * heads * S * D : 4e-6 * heads * L * (D + 2);  // records of a piece
+  const long long end = (((long long)L + offset + 127) & ~127ll), seen = causal && end < S ? end : S;
+  auto record_us = [&](int n) {
+    const double mb = n * mb_each;
+    return c.launch + c.per_mb * (mb <= c.cached ? mb * (seen + S) / (2.0 * S) : mb);
+  };
   auto us = [&](int n, double most) {  // (`most` or more: it is not less)
-    const double per = n * halves, more = n > 1 ? c.launch + c.per_mb * (n * mb_each) : 0;
+    const double per = n * halves, more = n > 1 ? record_us(n) : 0;
     const long long wgs = blocks * n;
     double chain = ceil(longest / per);
     if (n > 1 && c.tile_us * chain + more >= most) return most;
@@ -450,9 +462,10 @@ inline int backward_splits_16bit(const BackwardCost& c, bool of_keys, int B, int
   int best = 1;
   double least = us(1, 0);
   const double even = heads * sum / halves / slots;
-  for (int n = 2; n <= 16; n++) {
+  const int most = of_keys || D == 128 ? 16 : 8;
+  for (int n = 2; n <= most; n++) {
     // (in more than two rounds a place's chain is its share of all tiles at least, and more pieces only leave more records)
-    if (blocks * n > 2 * slots && c.tile_us * even + c.launch + c.per_mb * (n * mb_each) > 0.951 * least) break;
+    if (blocks * n > 2 * slots && c.tile_us * even + record_us(n) > 0.951 * least) break;
     const double t = us(n, 0.95 * least);
     if (t < 0.95 * least) best = n, least = t;
   }

@@ -671,7 +671,7 @@ struct PairSplits {
     if (!backward_on_mfma(p)) return;
     const bool f32 = backward_on_f32_pair(p), causal = effective_causal(f) != TTSDPA_CAUSAL_NONE;
     if (f->dtype != TTSDPA_F32 && f->mask_kind == TTSDPA_MASK_NONE && (f->D == 64 || f->D == 128)) {
-      static constexpr BackwardCost kDq[2] = {{0, 0.59, 3.6, 0.47}, {4.5, 0.53, 2.9, 0.37}}, kDkv[2] = {{0, 0.95, 2.5, 0.40}, {0, 1.75, 1.8, 0.41}};
+      static constexpr BackwardCost kDq[2] = {{0, 0.59, 3.6, 0.47}, {4.5, 0.53, 2.9, 0.37}}, kDkv[2] = {{0, 0.95, 2.5, 0.40, 120}, {0, 1.75, 1.8, 0.41, 80}};
       own = short_backward_splits(p, *this, &own_joint);
       if (own > 0) return;  // (whole: with less scratch than those kernels ask for)
       const int offset = effective_causal(f) == TTSDPA_CAUSAL_BOTTOM_RIGHT && f->S > f->L ? f->S - f->L : 0;
