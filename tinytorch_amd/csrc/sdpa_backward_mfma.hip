@@ -569,9 +569,6 @@ int launch_k(const BwdArgs& args, hipStream_t stream) {
   BwdArgs a = args;
   // the callers keep to this (rows are read in 16-byte chunks)
   if (PAD && (a.f.D % 8 != 0 || a.f.D >= D || a.f.D < 8)) return (int)hipErrorInvalidValue;
-  typedef BwdLds<D> Lds;
-  // with an attnMask, head_dim 128 takes the register-staged dk/dv kernel: the mask's 16 values per tile do not fit the
-  // 256 registers of the direct-to-LDS one
   // (head_dim 128 with an attnMask takes the register-staged kernels here: the mask's 16 values per tile do not fit the 256 registers
   // of the others)
   constexpr bool STREAMS = D == 128 && !MASKED && !PAD;

@@ -340,38 +340,31 @@ inline bool backward_tiles_dealt(int n, long long narrow, long long tiles, doubl
   return dealt < 0.8 * split;  // (a margin: one wavefront per SIMD hides less; 4 x 64 heads on 8 x 251 x 128 at 0.91: 313 us against 297)
 }
 
-// Workgroups that share a key block in the matrix-core dk/dv kernels (1: none, the kernel writes dk / dv itself).
+// Workgroups that share a key block in the matrix-core dk/dv kernels (1: none, the kernel writes dk / dv itself): fp32, calls with an attnMask, and
+// 16-bit head sizes other than 64 and 128 (those, without a mask: backward_splits_16bit).
 // A dk/dv workgroup owns 128 keys and about one runs per CU at a time; under a causal mask its length varies
 // 1 : (number of key blocks), and below about four workgroups per CU the longest ones set the time.  Without a causal
-// mask all are equally long and splitting only serves to give every CU one (splitting 256 equal workgroups further
-// measured 1 % slower, 13-20 % with an attnMask).  A split must still get a few tiles.  `groups`: wavefront groups
-// that already share a key block inside a workgroup (2 in the 16-bit head_dim-128 kernel, where splitting 512
-// workgroups of a causal call further measured 4 % slower, 256 of them 7-21 % faster).
-// `per_cu`: workgroups of the kernel that fit a CU (2 at head_dim 64 without an attnMask, else 1): head_dim 64, 256 equal
-// workgroups without a causal mask: two splits +28 %; causal with 512: four splits instead of two -2 to -5 %.
-inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, int D, bool causal, int groups, int per_cu, bool f32, bool* dealt) {
-  const long long wgs = (long long)B * Hkv * ((S + 127) / 128) * groups;
-  const long long tiles = (long long)(Hq / Hkv) * ((L + 31) / 32) / groups;  // the longest query stream, in 32-row tiles
-  // causal: two rounds of the workgroups a CU holds at a time (one for the 8-wavefront head_dim-128 kernel, whose two
-  // groups make `wgs` count double, and for the fp32 head_dim-128 kernel; two at head_dim 64).  fp32 head_dim 128, 512
-  // workgroups (B2 32q/8kv 4096 x 4096): splitting them in two measured the same time, 60 % more bytes read and a
-  // third kernel for the partial sums; 256 of them (2048 x 2048) two splits 76.5, four 74.1 TFLOP/s.
-  const long long enough = causal ? 512LL * per_cu * groups : 256 * per_cu;
+// mask all are equally long and splitting only serves to give every CU one (256 equal workgroups with an attnMask split further: 13-20 %
+// slower).  A split must still get a few tiles.  `per_cu`: workgroups of the kernel that fit a CU (2 up to head_dim 64 without an attnMask, else 1).
+inline int backward_dkv_splits(int B, int Hkv, int Hq, int L, int S, int D, bool causal, int per_cu, bool f32, bool* dealt) {
+  const long long wgs = (long long)B * Hkv * ((S + 127) / 128);
+  const long long tiles = (long long)(Hq / Hkv) * ((L + 31) / 32);  // the longest query stream, in 32-row tiles
+  // causal: two rounds of the workgroups a CU holds at a time.  fp32 head_dim 128, 512 workgroups (B2 32q/8kv 4096 x 4096): splitting
+  // them in two measured the same time, 60 % more bytes read and a third kernel for the partial sums; 256 of them (2048 x 2048) two
+  // splits 76.5, four 74.1 TFLOP/s.
+  const long long enough = causal ? 512LL * per_cu : 256 * per_cu;
   int n = 1;
   while (n < 4 && wgs * n < enough && tiles >= 16 * n && (D == 64 || D == 128)) n *= 2;  // (measured for these two sizes)
   const double record_us = (double)B * Hkv * S * D * 16 / (f32 ? 4e6 : 2e6), tile_us = f32 ? (D <= 64 ? 5.0 : 10.0) : D <= 64 ? 1.15 : 2.0;
-  n = cheapest_backward_splits(n, wgs / groups, tiles, 256 * per_cu, tile_us, record_us);
+  n = cheapest_backward_splits(n, wgs, tiles, 256 * per_cu, tile_us, record_us);
   *dealt = f32 && backward_tiles_dealt(n, (long long)B * Hkv * ((S + 31) / 32), tiles, tile_us, record_us);
   return *dealt ? 1 : n;
 }
 
 // Workgroups that share a 128-row query block in the matrix-core dq kernels (1: none, the kernel writes dq itself).
-// Two of its workgroups fit a CU (512 at a time on the chip).  A launch of fewer is split: that gives every slot a
-// workgroup, and under a causal mask, where their lengths vary 1 : (number of row blocks) and they start longest first,
-// a second round to end evenly
-// (bf16 head_dim 128, one batch entry: 8 heads 4096 x 4096 causal +26 %, 32 heads 512 x 8192 +46 %, 8 heads 2048 x 2048
-// without a mask +22 %; 512 causal workgroups split in two measured 5 % slower: the partial records cost more than the
-// uneven end).  A split must still get a few hundred keys.
+// The same calls.  A launch of fewer workgroups than the chip holds is split: that gives every slot a workgroup, and under a causal mask,
+// where their lengths vary 1 : (number of row blocks) and they start longest first, a second round to end evenly.  A split must still get
+// a few hundred keys.
 // `slots`: workgroups of the kernel the chip holds at a time (512; 256 for the fp32 kernel at head_dim 128).
 inline int backward_dq_splits(int B, int Hq, int L, int S, int D, bool causal, int slots, bool f32, bool* dealt) {
   *dealt = false;
@@ -770,9 +763,10 @@ __device__ __forceinline__ bool find_piece(const KArgs& a, int rows, bool causal
   const int ntile = (a.L + rows - 1) / rows;
   const bool alike = !a.kv_len || a.B == 1;
   const int own = alike ? 1 : ppc, same = alike ? a.G * ppc : a.G;  // pairs of unlike lengths one by one, else all together
-  // every split has all row tiles, or is beyond the keys: the caller returns; and launches of the 4-wavefront kernels that fit the
-  // CUs in one go, or nearly with one row tile a head, which gaps do not slow (3 heads x 136 rows on 1115 keys, ragged: 10.2 us with
-  // the search below, 8.6 so; 9 x 8 heads x 16 rows on 10495, 792 pieces, 36.2 and 35.0; 8 x 4 x 512 on 5000 35.5 and 37.6)
+  // every split has all row tiles, or is beyond the keys: the caller returns; and launches of 128-row workgroups that fit the
+  // CUs in one go, or nearly with one row tile a head, which gaps do not slow (the 4-wavefront kernels: 3 heads x 136 rows on 1115 keys, ragged, 10.2
+  // us with the search below, 8.6 so; 9 x 8 heads x 16 rows on 10495, 792 pieces, 36.2 and 35.0; 8 x 4 x 512 on 5000 35.5 and 37.6; the
+  // kernel with dealt keys: 60 drawn calls 2 % faster so, -1 to 5)
   const bool few = rows <= 128 && a.B * a.Hkv * a.G * ntile * a.kv_splits <= (ntile == 1 ? 1024 : 256);
   if (few || (alike && (!causal || a.pack_L))) {
     const int same = a.G * ppc;

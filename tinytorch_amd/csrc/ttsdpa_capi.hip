@@ -679,9 +679,8 @@ struct PairSplits {
       dkv = backward_splits_16bit(kDkv[f->D == 128], true, f->B, f->Hq, f->Hkv, f->L, f->S, f->D, causal, offset);
       return;
     }
-    const int groups = f->dtype != TTSDPA_F32 && f->D == 128 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
     const int per_cu = f->D <= 64 && f->mask_kind == TTSDPA_MASK_NONE ? 2 : 1;
-    dkv = backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, causal, groups, per_cu, f32, &dkv_dealt);
+    dkv = backward_dkv_splits(f->B, f->Hkv, f->Hq, f->L, f->S, f->D, causal, per_cu, f32, &dkv_dealt);
     dq = backward_dq_splits(f->B, f->Hq, f->L, f->S, f->D, causal, f32 && f->D > 64 ? 256 : 512, f32, &dq_dealt);
   }
 };
@@ -694,7 +693,9 @@ size_t backward_dq_partial_offset(const ttsdpa_backward_params* p, const PairSpl
   const size_t end = backward_partial_offset(p) + (size_t)n.dkv * 2 * p->fwd.B * p->fwd.Hkv * p->fwd.S * p->fwd.D * sizeof(float);
   return (end + 255) & ~(size_t)255;
 }
-// Estimated time of a call on the matrix-core pairs, by the longest stream of each kernel.
+// Estimated time of a call on the matrix-core pairs, by the longest stream of each kernel.  (16-bit: fitted to the head_dim-128 pair as the compiler
+// orders it and to its splits of then; of 104 drawn calls that go to the short sequences' kernels by it, the pair of now is shorter for one, 45.2 us and
+// 48.0, 1 x 4 heads (2) x 592 on 760, head_dim 128.)
 double pair_backward_us(const ttsdpa_params* f, const ShortShape& s, const PairSplits& n) {
   if (!s.f32) {
     const int tiles = (s.keys + 3) / 4, stream = s.group * ((f->L + 31) / 32);
