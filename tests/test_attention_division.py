@@ -147,3 +147,39 @@ def test_row_blocks_of_a_top_left_mask_see_as_many_keys_as_rows(dtype, B, Hq, Hk
 def test_pieces_of_long_streams(B, Hq, Hkv, L, S, D, causal, pieces):
     for dtype in (F16, BF16):
         assert _capi.backward_division(call(dtype, B, Hq, Hkv, L, S, D, causal, back=True)) == pieces
+
+
+# ---- what the GPU tests' cases are meant for: held here, where the estimates are ---------------------------------------------------------------
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("B,Hq,Hkv,L,S,causal,lens,divided", [
+    (1, 4, 2, 700, 5000, BR, False, True), (1, 4, 2, 1100, 3000, BR, False, True),
+    (3, 4, 2, 700, 3000, BR, True, True),                                             # (there in pages)
+    (1, 16, 4, 650, 650, TL, False, False), (4, 8, 8, 514, 545, NONE, True, False)])  # weightless rows; key counts
+def test_dealt_cases(B, Hq, Hkv, L, S, causal, lens, divided, dtype, D):
+    """test_prefill_dealt_gpu.py: the rows said to be divided are, and the test of infinities beyond the diagonal runs on that kernel."""
+    p = call(dtype, B, Hq, Hkv, L, S, D, causal, lens)
+    assert _capi.kernel(p) == "dealt" and (_capi.division(p)[0] > 1) == divided
+
+
+def test_backward_cases():
+    """test_backward_streams_gpu.py: divided key ranges; query streams in a number of pieces that is no power of two, over more workgroups than
+    run side by side; whole ones too."""
+    def pieces(*a, D=128, causal=NONE):
+        bp = call(BF16, *a, D, causal, back=True)
+        assert _capi.backward_kernel(bp) == "other"
+        return _capi.backward_division(bp)
+    assert pieces(2, 2, 1, 129, 2111)[1] > 1 and pieces(1, 8, 4, 200, 1500, causal=BR)[1] > 1
+    few = [pieces(1, Hq, Hkv, L, 1230, causal=c) for Hq, Hkv in ((6, 2), (5, 5), (7, 1)) for L in (33, 64, 96, 160, 193) for c in (NONE, BR)]
+    assert any(n > 1 and m > 1 for n, m in few) and any(n == 1 and m > 1 for n, m in few)
+    walks = [pieces(*a, D=D, causal=TL)[0] for D in (128, 64) for a in ((4, 56, 8, 383, 383), (4, 32, 4, 909, 909), (2, 32, 8, 700, 700))]
+    assert all(n > 1 for n in walks) and any(n & (n - 1) for n in walks)
+
+
+def test_decode_cases():
+    """test_decode_one_launch_gpu.py: workgroups of eight wavefronts for every type and head size there, and calls that stay divided."""
+    for D, dtype in ((128, BF16), (64, F16), (80, BF16), (128, F32), (64, F32)):
+        assert _capi.division(call(dtype, 2, 10, 2, 1, 256, D)) == (1, 8)
+    assert _capi.division(call(F32, 2, 6, 2, 1, 257, 128)) == (3, 4) and _capi.division(call(BF16, 2, 16, 2, 1, 289, 128)) == (3, 4)
+    for D, dtype in ((128, BF16), (64, F16), (64, F32)):
+        assert _capi.division(call(dtype, 24, 16, 8, 1, 1000, D, lens=True)) == (1, 8)
