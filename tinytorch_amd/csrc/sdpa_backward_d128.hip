@@ -124,11 +124,12 @@ __global__ __launch_bounds__(256, 2) void backward_dq128_kernel(BwdArgs a) {
   };
   const T* kp = (const T*)f.k + b * f.ks[0] + hk * f.ks[1];
   const T* vp = (const T*)f.v + b * f.vs[0] + hk * f.vs[1];
-  // f16: the lanes' offsets are formed for each tile from the lane number anew (a dozen instructions).  Kept, they were spilled, and a
-  // reload's wait in front of each request was one for the tiles in flight.  Forward and backward, 2 x 32 heads (8) x 4096 causal 1165 ->
-  // 1151 us, 4 x 8 x 1545 144.0 -> 141.4, 1 x 32 (4) x 2111 229.6 -> 225.8; 2 x 32 (8) x 2000 without a mask 626 -> 619.  bf16 keeps them:
-  // formed anew, causal 2 x 16 (8) x 1023 94.4 -> 95.9; without a mask 1 x 32 (8) x 4096 1025 -> 1016, but 1 x 28 (4) x 1311 159.5 -> 160.3.
-  constexpr bool kLaneKept = kIsBf16;
+  // The lanes' offsets are formed for each tile from the lane number anew (a dozen instructions), but for bf16 under a causal mask.  Kept, they were
+  // spilled, and a reload's wait in front of each request was one for the tiles in flight.  Forward and backward, f16, 2 x 32 heads (8) x 4096 causal
+  // 1165 -> 1151 us, 4 x 8 x 1545 144.0 -> 141.4, 1 x 32 (4) x 2111 229.6 -> 225.8; 2 x 32 (8) x 2000 without a mask 626 -> 619.  bf16 without a mask, twelve
+  // calls of 512 to 4096 rows, 1.7 % (1 x 32 (8) x 700 80.0 -> 77.3, 4 x 32 (8) x 1024 310.8 -> 304.9, 2 x 32 (8) x 4096 2052 -> 2040; 1 x 28 (4) x 1311 161.3 ->
+  // 162.9, 2 x 7 (1) x 3000 333.0 -> 337.1).  bf16 causal spills nothing and keeps them: formed anew, 2 x 16 (8) x 1023 94.4 -> 95.9.
+  constexpr bool kLaneKept = kIsBf16 && CAUSAL;
   auto lane_now = [&]() __attribute__((always_inline)) {
     int ln = lane;
     if constexpr (!kLaneKept) asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
