@@ -7,8 +7,9 @@
 // matrix instruction).  In the compiler's order the three followed each other, the wavefronts of a SIMD hardly overlapping: 3250 cycles
 // a tile of two wavefronts, the matrix pipe 44 % busy at 1.99 GHz.  Here a step is a stream of hand-ordered instructions
 // (gen_backward128_steps.py) over three tiles: scores and dP of tile i+1 and dq of tile i-1 on the matrix pipe, the vector work of
-// tile i between them.  2 x 32 heads (8) x 4096 x 4096, causal: 420 -> 378 us, the matrix pipe 58 % busy and the clock down at 1.69 GHz: as
-// in the forward kernel, power is what bounds it now.
+// tile i between them.  2 x 32 heads (8) x 4096 x 4096, causal: 420 -> 378 us, the matrix pipe 58 % busy and the clock down at 1.69 GHz.
+// Two things bound both kernels: the clock, which falls with the power of the operands' bits (on zeros dq takes 262 us of 370, dk/dv 361 of
+// 480), and the instructions that a step still has beside its matrix ones: a compiler-made wait taken out of the loops gave 4.6 % (below).
 //
 // K and V come by direct global->LDS loads, four stages each (K of tiles i-1, i, i+1 and, on its way, i+2): a tile is eight groups of
 // four 256-byte rows, 1040 bytes apart, chunk c of 16 bytes of row i of a group at slot c ^ 4i, so that one copy serves the

@@ -2,7 +2,7 @@
 // query heads sharing the KV head, instead of the reference's GEMM -> scale -> softmax -> GEMM chain over a
 // materialised score tensor (reference src/Function/FuncNNLayer.h:237-265).
 //
-// Work split.  Grid = splits x Hkv x B workgroups of 4 wavefronts.  A split is a contiguous range of keys; its
+// Work split.  Grid = splits x Hkv x B workgroups of 4 wavefronts, or of 8 up to 8 rows (plan_decode).  A split is a contiguous range of keys; its
 // wavefronts take 32-key blocks round-robin.  All query rows that read this KV head — the L * (Hq/Hkv) rows
 // (l, g), at most 16 — are handled together, so the cache is streamed once for the whole group.
 //
@@ -16,7 +16,7 @@
 //           l/C, l/C + 64/C, ... (one 16-byte load per key, a wavefront load instruction covers 64/C whole V rows =
 //           1 KiB contiguous); the probabilities
 //           travel from the score lanes to the value lanes through a per-wavefront LDS patch.
-// Each wavefront ends with (max, sum, acc) per row; the workgroup merges its four, then either writes the final
+// Each wavefront ends with (max, sum, acc) per row; the workgroup merges its four or eight, then either writes the final
 // output (splits == 1) or a partial (max, sum, acc) record that merge_kernel combines by log-sum-exp.
 
 #include "sdpa_common.h"
